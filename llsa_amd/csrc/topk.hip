@@ -1,10 +1,16 @@
 // Block selection: dense coarsest-level top-k and parent-guided fine top-k.
 //
-// The kernels score one tile of 16 pooled queries against 16-key tiles with the bf16 MFMA,
-// park the scores of the 16 rows in LDS and then let each wave select the T best entries of
-// "its" rows: by radix selection when a row fits in LDS, by repeated wave-wide arg-max over
-// chunks otherwise.  The order is total -- higher score first, equal scores by smaller key
-// index -- so the result does not depend on how the work is split.
+// A tile of 16 pooled queries is scored against 16-key tiles with the bf16 MFMA in the S^T orientation: lane l gets the
+// scores of query l%16, so a query's scores live in the registers of four lanes (l, l^16, l^32, l^48) and never leave
+// them.  All sixteen rows of a wave are selected side by side: bisection narrows every row down to a few more than its T
+// best keys -- a compare and an add-with-carry per score and step and two lane swaps per step for the row's count --, and
+// those are ranked among each other in LDS.  (One row per wave at a time, spread over the 64 lanes with a ballot and a
+// scalar population count per score, issues about three times the instructions per row and step, half of them on the one
+// scalar unit.  Bisecting down to exactly T keys takes 20 to 30 steps instead of 2 to 5: the T-th and the next best key of
+// the worst of sixteen rows agree in most of their bits.)
+//
+// The order is total -- higher score first, equal scores by smaller key index -- so the result does not depend on how the
+// work is split.
 #include "llsa_device.h"
 #include "llsa_host.h"
 #include "../../include/llsa_hip.h"
@@ -12,318 +18,642 @@
 namespace llsa {
 
 constexpr int kMaxT = 64;        // largest supported top-k
-constexpr int kChunk = 512;      // keys scored per pass of the dense kernel
 constexpr int kMaxCand = 512;    // candidates per parent in the sparse kernel (T2 * 16)
-constexpr int kNoIdx = 0x7fffffff;
 
-// Removes the T best entries of `row[0..npos)` (a wave's private LDS row) one by one.
-// Lane `lane` only ever touches positions congruent to it mod 64, so no barrier is
-// needed between iterations.  Taken entries are overwritten with NaN, which never
-// compares greater or equal.  Winners are written by lane 0.
-template <typename IdxFn>
-__device__ __forceinline__ void wave_topk_row(float* row, int npos, int T, IdxFn gidx_of, float* win_val,
-                                              int* win_idx) {
-    const int lane = threadIdx.x & (kWave - 1);
-    for (int t = 0; t < T; t++) {
-        float bv = -INFINITY;
-        int bi = kNoIdx, bp = -1;
-        for (int pos = lane; pos < npos; pos += kWave) {
-            const float v = row[pos];
-            const int gi = gidx_of(pos);
-            if (v > bv || (v == bv && gi < bi)) {
-                bv = v;
-                bi = gi;
-                bp = pos;
-            }
-        }
-        float wv = bv;
-        int wi = bi;
+// Unsigned integers that sort like the floats; 0 is kept for empty slots (a NaN becomes 1, below every number).
+__device__ __forceinline__ unsigned ordered_key(float f) {
+    const unsigned b = __float_as_uint(f);
+    const unsigned k = (b & 0x80000000u) ? ~b : (b | 0x80000000u);
+    return (f != f || k == 0u) ? 1u : k;
+}
+// Score rounded to bf16 and key index in one integer: the larger is the better key, equal scores by smaller index, and no
+// two keys of a row are equal.  For indices below 2^16 - 1 (a NaN sorts below every number, by index as well).
+constexpr int kMaxPackedKeys = 65535;
+__device__ __forceinline__ unsigned packed_key(float f, int idx) {
+    return (ordered_key(rn_bf16(f)) & 0xFFFF0000u) | (unsigned)(0xFFFF - idx);
+}
+// Any score, any index: the same order in 64 bits.
+__device__ __forceinline__ unsigned long long wide_key(unsigned score_key, int idx) {
+    return ((unsigned long long)score_key << 32) | (unsigned)(0x7FFFFFFF - idx);
+}
+
+// sum / largest / smallest over the four lanes that share a query
+__device__ __forceinline__ int quad_sum_i(int v) {
+    u32x2 a = __builtin_amdgcn_permlane16_swap((unsigned)v, (unsigned)v, false, false);
+    const unsigned w = a[0] + a[1];
+    u32x2 b = __builtin_amdgcn_permlane32_swap(w, w, false, false);
+    return (int)(b[0] + b[1]);
+}
+__device__ __forceinline__ unsigned quad_max_u(unsigned v) {
+    u32x2 a = __builtin_amdgcn_permlane16_swap(v, v, false, false);
+    const unsigned w = max(a[0], a[1]);
+    u32x2 b = __builtin_amdgcn_permlane32_swap(w, w, false, false);
+    return max(b[0], b[1]);
+}
+__device__ __forceinline__ unsigned quad_min_u(unsigned v) { return ~quad_max_u(~v); }
+__device__ __forceinline__ unsigned long long quad_max_u(unsigned long long v) {
+    const unsigned hi = quad_max_u((unsigned)(v >> 32));
+    const unsigned lo = quad_max_u((unsigned)(v >> 32) == hi ? (unsigned)v : 0u);
+    return ((unsigned long long)hi << 32) | lo;
+}
+
+// S^T tiles: rows = 16 keys starting at row_of(a) * kD elements into `keys`, columns = the wave's 16 queries (bq).  Lane l
+// gets the scores of query l%16 against keys 4*(l/16) .. +3 of tile a.  No branch around the loads, so that they are all in
+// flight together: the caller clamps the rows of tiles that do not exist and drops their scores.
+template <int TILES, typename RowOf>
+__device__ __forceinline__ void score_tiles(f32x4 (&s)[TILES], const bf16* keys, RowOf row_of, const bf16x8 bq[2], int lane) {
+    constexpr int kBatch = TILES < 8 ? TILES : 8;
+    const int at = (lane & 15) * kD + (lane >> 4) * 8;
 #pragma unroll
-        for (int off = 32; off >= 1; off >>= 1) {
-            const float ov = __shfl_xor(wv, off);
-            const int oi = __shfl_xor(wi, off);
-            if (ov > wv || (ov == wv && oi < wi)) {
-                wv = ov;
-                wi = oi;
-            }
+    for (int a0 = 0; a0 < TILES; a0 += kBatch) {
+        bf16x8 k[kBatch][2];
+#pragma unroll
+        for (int a = 0; a < kBatch; a++) {
+            const bf16* p = keys + (int64_t)row_of(a0 + a) * kD + at;
+            k[a][0] = ld16(p);
+            k[a][1] = ld16(p + 32);
         }
-        if (bp >= 0 && bi == wi && bv == wv) row[bp] = __builtin_nanf("");
-        if (lane == 0) {
-            win_val[t] = (wi == kNoIdx) ? __builtin_nanf("") : wv;
-            win_idx[t] = wi;
+#pragma unroll
+        for (int a = 0; a < kBatch; a++) {
+            f32x4 z = {0.f, 0.f, 0.f, 0.f};
+            s[a0 + a] = mfma_bf16(k[a][1], bq[1], mfma_bf16(k[a][0], bq[0], z));
         }
     }
 }
 
-// S^T tile: rows = 16 keys starting at krow, columns = the wave's 16 queries (bq).
-// Lane l gets the scores of query l%16 against keys 4*(l/16) .. +3 of the tile.
-__device__ __forceinline__ f32x4 score_tile(const bf16* krow, const bf16x8 bq[2]) {
-    const int lane = threadIdx.x & (kWave - 1);
-    const bf16* p = krow + (lane & 15) * kD + (lane >> 4) * 8;
-    f32x4 acc = {0.f, 0.f, 0.f, 0.f};
-    acc = mfma_bf16(ld16(p), bq[0], acc);
-    acc = mfma_bf16(ld16(p + 32), bq[1], acc);
-    return acc;
+// What the W waves of a workgroup that hold parts of the same sixteen rows use to add their counts; W = 1 needs none of it.
+template <int W>
+struct RowShare {
+    int part[2][W][16];
+};
+template <int W>
+__device__ __forceinline__ int rows_sum(int v, RowShare<W>* sh, int& turn, int wave, int lane) {
+    v = quad_sum_i(v);
+    if (W > 1) {
+        // (two buffers in turn: a wave that is through the barrier may write the next counts while another still reads these)
+        if (lane < 16) sh->part[turn][wave][lane] = v;
+        __syncthreads();
+        v = 0;
+#pragma unroll
+        for (int w = 0; w < W; w++) v += sh->part[turn][w][lane & 15];
+        turn ^= 1;
+    }
+    return v;
 }
 
-__global__ __launch_bounds__(256) void topk_dense_kernel(const bf16* __restrict__ pq, const bf16* __restrict__ pk,
-                                                         int* __restrict__ out, int n, int T, int round_scores) {
-    __shared__ float sc[16][kMaxT + kChunk + 1];
-    __shared__ int carry_idx[16][kMaxT];
-    __shared__ float win_val[16][kMaxT];
-    __shared__ int win_idx[16][kMaxT];
+// A key near the middle of the scores of two keys (it need not lie between them: a NaN, an overflow).
+__device__ __forceinline__ float key_score(unsigned k) { return __uint_as_float((k & 0x80000000u) ? (k ^ 0x80000000u) : ~k); }
+__device__ __forceinline__ unsigned middle_key(unsigned a, unsigned b) { return ordered_key(0.5f * (key_score(a) + key_score(b))); }
+__device__ __forceinline__ unsigned long long middle_key(unsigned long long a, unsigned long long b) {
+    return (unsigned long long)middle_key((unsigned)(a >> 32), (unsigned)(b >> 32)) << 32;
+}
 
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+// A threshold that leaves a few more than the T best keys of every row: count(key >= t) is at least T and at most T + kSpare,
+// or t is a key so often repeated that no threshold comes closer.  key[0..E): this lane's keys of its row (0: empty).  lo: a lower bound with
+// count(key >= lo) >= T; top: the row's largest key.  T may differ from row to row (it is the same in a row's lanes).  Returns
+// t; n_ge: the count at t.  The rows of a wave (of all W waves) run until the last one is decided.
+// The first steps halve the interval of scores, not of keys: half of all keys between 0.01 and 16 belong to scores below 0.4.
+constexpr int kSpare = 8, kScoreSteps = 10;
+template <int E, int W, typename Key>
+__device__ __forceinline__ Key row_threshold(const Key (&key)[E], int T, Key lo, Key top, RowShare<W>* sh, int& turn, int wave, int lane,
+                                             int& n_ge) {
+    Key mid = lo, hi = top + 1;                               // (top is below the largest integer: an index part is never all ones)
+    bool open = true;
+    n_ge = 0;
+    for (int step = 0;; step++) {
+        int c = 0;
+#pragma unroll
+        for (int i = 0; i < E; i++) c += (key[i] >= mid) ? 1 : 0;
+        c = rows_sum<W>(c, sh, turn, wave, lane);
+        if (open) {
+            if (c >= T) {
+                lo = mid;
+                n_ge = c;
+            } else {
+                hi = mid;
+            }
+            open = n_ge > T + kSpare && hi - lo > 1;
+        }
+        if (__ballot(open) == 0) return lo;
+        const Key half = lo + ((hi - lo) >> 1), of_score = middle_key(lo, hi);
+        mid = !open ? lo : (step < kScoreSteps && of_score > lo && of_score < hi) ? of_score : half;
+    }
+}
+
+// The T best of a row's m (>= T) keys in LDS, in order: a key's rank is the number of larger ones, 64 * W threads for sixteen rows.
+// keys[row][slot]: wide keys, no two of a row equal.  index_of(low word) is what goes to out + row * out_stride + rank.
+constexpr int kWin = kMaxT + kSpare, kWinStride = kWin + 1;       // (odd: the rows start in different banks; what is no winner goes to the last place)
+template <int W, typename IndexOf>
+__device__ __forceinline__ void write_winners(unsigned long long (*keys)[kWinStride], const int* n_keys, int T, int* out, int64_t out_stride, int tid,
+                                              IndexOf index_of) {
+    constexpr int kSub = 4 * W;                   // threads per row
+    const int row = tid / kSub, sub = tid % kSub, m = min(n_keys[row], kWin);
+    for (int j0 = sub; j0 < m; j0 += 4 * kSub) {
+        unsigned long long own[4];
+        int rank[4];
+#pragma unroll
+        for (int u = 0; u < 4; u++) {
+            own[u] = keys[row][min(j0 + u * kSub, m - 1)];
+            rank[u] = 0;
+        }
+#pragma unroll 4
+        for (int j = 0; j < m; j++) {
+            const unsigned long long o = keys[row][j];
+#pragma unroll
+            for (int u = 0; u < 4; u++) rank[u] += o > own[u] ? 1 : 0;
+        }
+#pragma unroll
+        for (int u = 0; u < 4; u++)
+            if (j0 + u * kSub < m && rank[u] < T) out[row * out_stride + rank[u]] = index_of((unsigned)own[u]);
+    }
+}
+__device__ __forceinline__ int wide_index(unsigned low) { return 0x7FFFFFFF - (int)low; }
+
+// t again, in a way the compiler cannot see through (slot is a small non-negative number out of LDS): the comparisons that
+// counted the winners are made a second time when they are written, instead of being kept as dozens of lane masks, for which
+// the scalar registers do not suffice.
+template <typename Key>
+__device__ __forceinline__ Key compare_again(Key t, int slot) { return t + (Key)((unsigned)slot >> 31); }
+
+// A lower bound of the T-th best key of every row (0 < bound): the keys are cut into disjoint groups, and the smallest of
+// the groups' largest keys has at least as many keys at or above it as there are groups.  tiles: key tiles there are (tile a * W +
+// wave is in registers 4 a ..); no group may be without any.
+template <int TPW, int W>
+__device__ __forceinline__ unsigned row_bound(const unsigned (&key)[4 * TPW], int tiles, int T, unsigned& top, RowShare<W>* sh, int& turn,
+                                              int wave, int lane) {
+    constexpr int kFew = TPW < 4 ? TPW : 4;                   // groups per lane: kFew large ones, or one per tile
+    unsigned tile_max[TPW], few[kFew];
+    unsigned least = 0xFFFFFFFFu, least_few = 0xFFFFFFFFu;
+    top = 0;
+#pragma unroll
+    for (int g = 0; g < kFew; g++) few[g] = 0;
+#pragma unroll
+    for (int a = 0; a < TPW; a++) {
+        tile_max[a] = max(max(key[4 * a], key[4 * a + 1]), max(key[4 * a + 2], key[4 * a + 3]));
+        least = min(least, tile_max[a]);
+        few[a % kFew] = max(few[a % kFew], tile_max[a]);
+    }
+#pragma unroll
+    for (int g = 0; g < kFew; g++) {
+        top = max(top, few[g]);
+        least_few = min(least_few, few[g]);
+    }
+    unsigned lo = (T <= 4 * W * kFew && tiles >= W * kFew) ? least_few : (T <= 4 * W * TPW && tiles == W * TPW) ? least : 0u;
+    top = quad_max_u(top);
+    lo = quad_min_u(lo);
+    if (W > 1) {
+        if (lane < 16) {
+            sh->part[0][wave][lane] = (int)top;
+            sh->part[1][wave][lane] = (int)lo;
+        }
+        __syncthreads();
+#pragma unroll
+        for (int w = 0; w < W; w++) {
+            top = max(top, (unsigned)sh->part[0][w][lane & 15]);
+            lo = min(lo, (unsigned)sh->part[1][w][lane & 15]);
+        }
+        __syncthreads();
+        turn = 0;
+    }
+    return max(lo, 1u);
+}
+
+constexpr int kRegMaxN = 1024;        // keys per row the register kernel takes: 4 waves x 16 tiles
+
+// Dense selection for n <= kRegMaxN: 16 query rows per workgroup, four waves that take every fourth key tile each.
+// PACK: scores rounded to bf16, score and index in one 32-bit key; otherwise fp32 scores with a second bisection over the
+// index where scores are equal.  Latency decides here (a few hundred workgroups of a few thousand cycles each); with
+// one row per wave and a ballot per score it took 17 us at n = 256, 24 rows of heads, and 44 us at n = 1024, 6.
+template <int TPW, int W, bool PACK>
+__global__ __launch_bounds__(64 * W) void topk_dense_kernel(const bf16* __restrict__ pq, const bf16* __restrict__ pk, int* __restrict__ out,
+                                                         int n, int T) {
+    constexpr int E = 4 * TPW;
+    __shared__ RowShare<W> share;
+    __shared__ unsigned long long win[16][kWinStride];
+    __shared__ int n_win[16];
+    const int tid = threadIdx.x, lane = tid & 63, wave = W == 1 ? 0 : __builtin_amdgcn_readfirstlane(tid >> 6), quad = lane >> 4, r = lane & 15;
     const int bh = blockIdx.y, q0 = blockIdx.x * 16;
     const bf16* pqb = pq + ((int64_t)bh * n + q0) * kD;
     const bf16* pkb = pk + (int64_t)bh * n * kD;
-
+    if (tid < 16) n_win[tid] = 0;
     bf16x8 bq[2];
-    bq[0] = ld16(pqb + (lane & 15) * kD + (lane >> 4) * 8);
-    bq[1] = ld16(pqb + (lane & 15) * kD + (lane >> 4) * 8 + 32);
-
-    for (int i = tid; i < 16 * T; i += 256) {
-        sc[i / T][i % T] = __builtin_nanf("");
-        carry_idx[i / T][i % T] = kNoIdx;
+    bq[0] = ld16(pqb + r * kD + quad * 8);
+    bq[1] = ld16(pqb + r * kD + quad * 8 + 32);
+    unsigned key[E];
+    f32x4 s[TPW];
+    score_tiles<TPW>(s, pkb, [=](int a) { return min(a * W + wave, n / 16 - 1) * 16; }, bq, lane);
+#pragma unroll
+    for (int a = 0; a < TPW; a++) {
+        const int tile = a * W + wave;
+#pragma unroll
+        for (int e = 0; e < 4; e++) {
+            const unsigned k = PACK ? packed_key(s[a][e], tile * 16 + 4 * quad + e) : ordered_key(s[a][e]);
+            key[4 * a + e] = tile < n / 16 ? k : 0u;
+        }
+    }
+    int turn = 0, n_ge;
+    unsigned top;
+    const unsigned lo = row_bound<TPW, W>(key, n / 16, T, top, &share, turn, wave, lane);
+    const unsigned t = row_threshold<E, W>(key, T, lo, top, &share, turn, wave, lane, n_ge);
+    if (!PACK) {                                              // of the keys equal to t, the ones at the smallest indices are taken
+        // (the same in all waves: counts are the workgroup's)
+        const bool tie = n_ge > T + kSpare;
+        if (__ballot(tie) != 0) {
+            int above = 0;
+#pragma unroll
+            for (int i = 0; i < E; i++) above += (key[i] > t) ? 1 : 0;
+            above = rows_sum<W>(above, &share, turn, wave, lane);
+            int a0 = -1, a1 = n - 1;                          // count(equal, index <= a0) < T - above <= count(equal, index <= a1)
+            while (__ballot(tie && a1 - a0 > 1) != 0) {
+                const int mid = a0 + ((a1 - a0) >> 1);
+                const unsigned te = compare_again(t, a1);
+                int c = 0;
+#pragma unroll
+                for (int i = 0; i < E; i++) c += (key[i] == te && ((i >> 2) * W + wave) * 16 + 4 * quad + (i & 3) <= mid) ? 1 : 0;
+                c = rows_sum<W>(c, &share, turn, wave, lane);
+                if (a1 - a0 > 1) {
+                    if (c >= T - above) a1 = mid;
+                    else a0 = mid;
+                }
+            }
+            if (tie) {
+#pragma unroll
+                for (int i = 0; i < E; i++) key[i] = (key[i] == t && ((i >> 2) * W + wave) * 16 + 4 * quad + (i & 3) > a1) ? 0u : key[i];
+            }
+        }
+    }
+    // winners to LDS, in any order (their keys are unique)
+    int mine = 0;
+#pragma unroll
+    for (int i = 0; i < E; i++) mine += key[i] >= t ? 1 : 0;
+    __syncthreads();                                          // (n_win is cleared)
+    int slot = mine > 0 ? atomicAdd(&n_win[r], mine) : 0;
+    const unsigned t2 = compare_again(t, slot);
+#pragma unroll
+    for (int i = 0; i < E; i++) {
+        const bool on = key[i] >= t2;
+        win[r][on ? min(slot, kWin) : kWin] = wide_key(PACK ? key[i] & 0xFFFF0000u : key[i], ((i >> 2) * W + wave) * 16 + 4 * quad + (i & 3));
+        slot += on ? 1 : 0;
     }
     __syncthreads();
+    write_winners<W>(win, n_win, T, out + ((int64_t)bh * n + q0) * T, T, tid, wide_index);
+}
 
-    for (int base = 0; base < n; base += kChunk) {
-        const int len = min(kChunk, n - base);
-        for (int tile = wave; tile < len / 16; tile += 4) {
-            f32x4 s = score_tile(pkb + (int64_t)(base + tile * 16) * kD, bq);
+// Dense selection for longer rows: the keys stream by, and only those that can still be among a row's T best are kept.
+// A wave owns sixteen rows (PARTS = 1: four waves of a workgroup = 64 rows, which share the key tiles through LDS) or a
+// quarter of the keys of sixteen rows (PARTS = 4, for grids too small to fill the chip otherwise).  Every row has a buffer
+// of kBuf keys in LDS and a threshold; a tile whose scores all lie below their rows' thresholds costs a handful of
+// instructions, the others append what passes.  When a buffer is nearly full the wave cuts all sixteen back to little more
+// than their T best, which also raises the thresholds.  In a stream of random order about T ln(n / T) keys of a row pass.
+// Key: the 32-bit packed key (scores rounded to bf16, n <= kMaxPackedKeys) or the 64-bit wide key.
+// (A T-step arg-max over chunks of 512 keys per row took 1480 us for 8 x 4096 rows of 4096 keys, T = 8.)
+constexpr int kBuf = 128, kBufFull = kBuf - 16;   // a tile adds at most 16 keys to a row
+constexpr int kStreamWaves = 4;
+constexpr int kStageKeys = 64;                    // keys per LDS buffer (one tile per wave)
+
+template <typename Key>
+struct StreamKey;
+template <>
+struct StreamKey<unsigned> {
+    static __device__ __forceinline__ unsigned make(float s, int idx, bool) { return packed_key(s, idx); }
+    static __device__ __forceinline__ unsigned long long wide(unsigned k) { return wide_key(k & 0xFFFF0000u, 0xFFFF - (int)(k & 0xFFFFu)); }
+    // a score below this cannot make a key of at least t: one bf16 step below t's score
+    static __device__ __forceinline__ unsigned score_bits(unsigned t) { return t & 0xFFFF0000u; }
+};
+template <>
+struct StreamKey<unsigned long long> {
+    static __device__ __forceinline__ unsigned long long make(float s, int idx, bool round) {
+        return wide_key(ordered_key(round ? rn_bf16(s) : s), idx);
+    }
+    static __device__ __forceinline__ unsigned long long wide(unsigned long long k) { return k; }
+    static __device__ __forceinline__ unsigned score_bits(unsigned long long t) { return (unsigned)(t >> 32) & 0xFFFF0000u; }
+};
+// The largest float that is certainly below (or rounds below) the score of key bits `k` (its low 16 bits are zero).
+__device__ __forceinline__ float score_floor(unsigned k) {
+    if (k < 0x00020000u) return -INFINITY;
+    k -= 0x00010000u;                                         // one bf16 step down
+    const unsigned b = (k & 0x80000000u) ? (k ^ 0x80000000u) : ~k;
+    const float f = __uint_as_float(b);
+    return (f != f) ? -INFINITY : f;
+}
+
+template <typename Key, int PARTS>
+__global__ __launch_bounds__(64 * kStreamWaves) void topk_stream_kernel(const bf16* __restrict__ pq, const bf16* __restrict__ pk,
+                                                                        int* __restrict__ out, int n, int T, int round_scores) {
+    constexpr int kE = kBuf / 4;                              // keys of a row's buffer per lane
+    // a wave's buffers; at the end a row tile's winners take their place
+    constexpr int kKeys = 16 * (kBuf + 1), kWide = 16 * kWinStride, kPer = sizeof(Key) == 8 ? kKeys : (kKeys + 1) / 2 > kWide ? (kKeys + 1) / 2 : kWide;
+    __shared__ unsigned long long space[kStreamWaves][kPer];
+    __shared__ int cnt[kStreamWaves][16];
+    __shared__ int n_win[kStreamWaves / PARTS][16];
+    __shared__ RowShare<PARTS> share;
+    __shared__ __align__(16) bf16 stage[PARTS == 1 ? 2 : 1][PARTS == 1 ? kStageKeys * kD : 8];
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), quad = lane >> 4, r = lane & 15;
+    const int part = PARTS == 1 ? 0 : wave, rowt = PARTS == 1 ? wave : 0;
+    const int bh = blockIdx.y, q0 = blockIdx.x * (PARTS == 1 ? 64 : 16) + rowt * 16;      // n is a multiple of 64 where PARTS == 1
+    const bf16* pqb = pq + ((int64_t)bh * n + q0) * kD;
+    const bf16* pkb = pk + (int64_t)bh * n * kD;
+    if (lane < 16) cnt[wave][lane] = 0;
+    if (lane < 16 && part == 0) n_win[rowt][lane] = 0;
+    bf16x8 bq[2];
+    bq[0] = ld16(pqb + r * kD + quad * 8);
+    bq[1] = ld16(pqb + r * kD + quad * 8 + 32);
+    Key tau = 1;                                              // keys below it are not among the row's T best
+    float low = -INFINITY;                                    // scores below it do not make such a key
+    Key (*const my)[kBuf + 1] = reinterpret_cast<Key (*)[kBuf + 1]>(space[wave]);
+    unsigned long long (*const win)[kWinStride] = reinterpret_cast<unsigned long long (*)[kWinStride]>(space[rowt]);
+    auto settle = [&]() __attribute__((always_inline)) {      // LDS of this wave: all writes land before what follows reads
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+    };
+    settle();
+
+    // cuts every row's buffer back to its T best keys
+    auto cut = [&]() __attribute__((always_inline)) {
+        settle();
+        const int have = cnt[wave][r];
+        Key key[kE], top = 0;
+#pragma unroll
+        for (int i = 0; i < kE; i++) {
+            const int at = i * 4 + quad;
+            key[i] = at < have ? my[r][at] : (Key)0;
+            top = key[i] > top ? key[i] : top;
+        }
+        top = quad_max_u(top);
+        int turn = 0, n_ge;
+        // (a row that has fewer than T keys keeps them all)
+        const Key t = row_threshold<kE, 1, Key>(key, min(T, have), tau, top > tau ? top : tau, (RowShare<1>*)nullptr, turn, 0, lane, n_ge);
+        int mine = 0;
+#pragma unroll
+        for (int i = 0; i < kE; i++) mine += key[i] >= t ? 1 : 0;
+        settle();
+        if (lane < 16) cnt[wave][lane] = 0;
+        settle();
+        int slot = mine > 0 ? atomicAdd(&cnt[wave][r], mine) : 0;
+        const Key t2 = compare_again(t, slot);
+#pragma unroll
+        for (int i = 0; i < kE; i++)
+            if (key[i] >= t2) my[r][min(slot++, kBuf)] = key[i];
+        if (have >= T) {
+            tau = t;
+            low = score_floor(StreamKey<Key>::score_bits(t));
+        }
+        settle();
+    };
+    auto take = [&](const f32x4 s, int key0) __attribute__((always_inline)) {      // the scores of one key tile
+        // (a NaN passes the test -- it has to be able to fill a row that has nothing better)
+        const bool any = !(fmaxf(fmaxf(s[0], s[1]), fmaxf(s[2], s[3])) < low);
+        if (__ballot(any) == 0) return;
+        Key k[4];
+        int mine = 0;
+#pragma unroll
+        for (int e = 0; e < 4; e++) {
+            k[e] = StreamKey<Key>::make(s[e], key0 + 4 * quad + e, round_scores != 0);
+            mine += k[e] >= tau ? 1 : 0;
+        }
+        int slot = 0;
+        if (mine > 0) {
+            slot = atomicAdd(&cnt[wave][r], mine);
+            const int full = slot + mine;
 #pragma unroll
             for (int e = 0; e < 4; e++)
-                sc[lane & 15][T + tile * 16 + 4 * (lane >> 4) + e] = round_scores ? rn_bf16(s[e]) : s[e];
+                if (k[e] >= tau) my[r][min(slot++, kBuf)] = k[e];
+            slot = full;
         }
-        __syncthreads();
-        for (int row = wave; row < 16; row += 4) {
-            const int* ci = carry_idx[row];
-            wave_topk_row(
-                sc[row], T + len, T, [=](int pos) { return pos < T ? ci[pos] : base + pos - T; }, win_val[row],
-                win_idx[row]);
-        }
-        __syncthreads();
-        for (int i = tid; i < 16 * T; i += 256) {
-            sc[i / T][i % T] = win_val[i / T][i % T];
-            carry_idx[i / T][i % T] = win_idx[i / T][i % T];
-        }
-        __syncthreads();
-    }
-    for (int i = tid; i < 16 * T; i += 256) out[((int64_t)bh * n + q0 + i / T) * T + i % T] = win_idx[i / T][i % T];
-}
+        if (__ballot(slot > kBufFull) != 0) cut();
+    };
 
-// ---------------------------------------------------------------------------------------
-// Radix selection.  Scores are mapped to unsigned integers that sort like the floats; the
-// T-th largest is found one bit at a time from the top with a wave-wide count per bit
-// (a compare, a ballot and a scalar popcount per entry, no cross-lane data movement), then
-// everything above it -- plus as many entries equal to it as are still needed, smallest
-// index first -- is compacted and put in final order by rank counting among the T winners.
-// ---------------------------------------------------------------------------------------
-__device__ __forceinline__ unsigned ordered_bits(float f) {
-    if (f != f) return 0u;                                    // NaN sorts below everything
-    const unsigned b = __float_as_uint(f);
-    return (b & 0x80000000u) ? ~b : (b | 0x80000000u);
-}
-
-// u[0..npos): ordered scores of one row (LDS); gidx_of(pos): global index of a position.
-// Each lane keeps its E entries (positions lane, lane + 64, ...) in registers, so a bit step is
-// E compares + ballots + scalar popcounts with no memory access.
-// sel_u / sel_i: 64 entries of LDS scratch each.  out[0..T): result, global memory.
-// low_bit: the keys' bits below it are known to be zero (16 for scores rounded to bf16) and are not
-// looked at; idx_bits: the global indices are below 2^idx_bits (the tie pass starts there).
-template <int E, typename IdxFn>
-__device__ __forceinline__ void wave_topk_radix(const unsigned* u, int npos, int T, IdxFn gidx_of, unsigned* sel_u,
-                                                int* sel_i, int* out, int lane, int low_bit, int idx_bits) {
-    unsigned uk[E];
-    unsigned gk[E];
-    bool ok[E];
+    if (PARTS == 1) {
+        // key tiles through LDS, 64 keys per buffer, in the order the lanes read them (R tile: 16-byte unit
+        // chunk * 16 + row), so each is fetched once per workgroup; the next buffer's copy runs during this one's work
+        auto fetch = [&](int c) __attribute__((always_inline)) {
+            const bf16* src = pkb + ((int64_t)c * kStageKeys + wave * 16 + r) * kD + quad * 8;
+            copy16_global_to_lds(src, &stage[c & 1][wave * kTile]);
+            copy16_global_to_lds(src + 32, &stage[c & 1][wave * kTile + 512]);
+        };
+        const int n_chunks = n / kStageKeys;
+        fetch(0);
+        for (int c = 0; c < n_chunks; c++) {
+            wait_vm0();
+            __syncthreads();                                  // everybody's part has landed, and the other buffer is free
+            bf16x8 ka[4][2];
 #pragma unroll
-    for (int e = 0; e < E; e++) {
-        const int pos = lane + e * kWave;
-        ok[e] = pos < npos;
-        uk[e] = ok[e] ? u[pos] : 0u;
-        gk[e] = ok[e] ? (unsigned)gidx_of(pos) : 0xFFFFFFFFu;
-    }
-    // Invalid slots hold key 0 and never equal `want` (its current bit is set), so the bit loop
-    // needs no validity mask.  `match` counts the entries that agree with the decided bits; once
-    // it equals the number still to take, all of them are winners and the remaining bits need
-    // not be looked at (tau = prefix with zero low bits then selects exactly those).
-    unsigned prefix = 0;
-    int remaining = T, match = npos;
-    for (int bit = 31; bit >= low_bit && match != remaining; bit--) {
-        const unsigned msk = (bit == 31) ? 0x80000000u : ((0xFFFFFFFFu << (bit + 1)) | (1u << bit));
-        const unsigned want = prefix | (1u << bit);
-        int cnt1 = 0;
-#pragma unroll
-        for (int e = 0; e < E; e++) cnt1 += __popcll(__ballot((uk[e] & msk) == want));
-        if (cnt1 >= remaining) {
-            prefix = want;
-            match = cnt1;
-        } else {
-            remaining -= cnt1;
-            match -= cnt1;
-        }
-    }
-    const unsigned tau = prefix;                              // the T-th largest score
-    int n_eq = 0;
-#pragma unroll
-    for (int e = 0; e < E; e++) n_eq += __popcll(__ballot(ok[e] && uk[e] == tau));
-    unsigned idx_thr = 0xFFFFFFFFu;
-    if (n_eq > remaining) {                                   // ties at the threshold: keep the smallest indices
-        unsigned p2 = 0;
-        int rem2 = remaining;
-        for (int bit = idx_bits - 1; bit >= 0; bit--) {
-            const unsigned msk = (0xFFFFFFFFu << (bit + 1)) | (1u << bit);
-            int cnt0 = 0;
-#pragma unroll
-            for (int e = 0; e < E; e++) cnt0 += __popcll(__ballot(ok[e] && uk[e] == tau && (gk[e] & msk) == p2));
-            if (cnt0 < rem2) {
-                rem2 -= cnt0;
-                p2 |= (1u << bit);
+            for (int a = 0; a < 4; a++) {
+                ka[a][0] = lds_ld16(&stage[c & 1][a * kTile + lane * 8]);
+                ka[a][1] = lds_ld16(&stage[c & 1][a * kTile + 512 + lane * 8]);
+            }
+            wait_all_mem();
+            if (c + 1 < n_chunks) fetch(c + 1);
+#pragma unroll 1
+            for (int a = 0; a < 4; a += 2) {
+                f32x4 z = {0.f, 0.f, 0.f, 0.f};
+                const bf16x8 k0 = a ? ka[2][0] : ka[0][0], k1 = a ? ka[2][1] : ka[0][1];
+                const bf16x8 k2 = a ? ka[3][0] : ka[1][0], k3 = a ? ka[3][1] : ka[1][1];
+                const f32x4 s0 = mfma_bf16(k1, bq[1], mfma_bf16(k0, bq[0], z)), s1 = mfma_bf16(k3, bq[1], mfma_bf16(k2, bq[0], z));
+                take(s0, c * kStageKeys + a * 16);
+                take(s1, c * kStageKeys + a * 16 + 16);
             }
         }
-        idx_thr = p2;
-    }
-    if (lane < T) {
-        sel_u[lane] = 0u;
-        sel_i[lane] = kNoIdx;
-    }
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    int base_slot = 0;
-#pragma unroll
-    for (int e = 0; e < E; e++) {
-        const bool sel = ok[e] && (uk[e] > tau || (uk[e] == tau && gk[e] <= idx_thr));
-        const unsigned long long m = __ballot(sel);
-        const int slot = base_slot + __popcll(m & ((1ull << lane) - 1ull));
-        if (sel && slot < T) {
-            sel_u[slot] = uk[e];
-            sel_i[slot] = (int)gk[e];
+    } else {
+        const int tiles = n / 16, per = (tiles + PARTS - 1) / PARTS, lo = min(part * per, tiles), hi = min(lo + per, tiles);
+        const bf16* p = pkb + r * kD + quad * 8;
+        bf16x8 k0 = zero8(), k1 = zero8();
+        if (lo < hi) {
+            k0 = ld16(p + (int64_t)lo * 16 * kD);
+            k1 = ld16(p + (int64_t)lo * 16 * kD + 32);
         }
-        base_slot += __popcll(m);
-    }
-    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    {   // final order by rank counting among the T winners: winner j sits in lane j and is handed round with readlane
-        const unsigned mu = sel_u[lane];
-        const int mi = sel_i[lane];
-        int rank = 0;
-        for (int j = 0; j < T; j++) {
-            const unsigned ou = (unsigned)__builtin_amdgcn_readlane((int)mu, j);
-            const int oi = __builtin_amdgcn_readlane(mi, j);
-            rank += (ou > mu || (ou == mu && (oi < mi || (oi == mi && j < lane)))) ? 1 : 0;
+        for (int t = lo; t < hi; t++) {
+            const bf16* nx = p + (int64_t)min(t + 1, hi - 1) * 16 * kD;
+            const bf16x8 n0 = ld16(nx), n1 = ld16(nx + 32);
+            f32x4 z = {0.f, 0.f, 0.f, 0.f};
+            take(mfma_bf16(k1, bq[1], mfma_bf16(k0, bq[0], z)), t * 16);
+            k0 = n0;
+            k1 = n1;
         }
-        if (lane < T) out[rank] = mi;
     }
-    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-}
-
-// entries per lane as a compile-time bound: 1, 2, 4, 8 or 16
-template <typename IdxFn>
-__device__ __forceinline__ void wave_topk_radix_any(const unsigned* u, int npos, int T, IdxFn gidx_of, unsigned* sel_u,
-                                                    int* sel_i, int* out, int lane, int low_bit, int idx_bits) {
-    if (npos <= 64) wave_topk_radix<1>(u, npos, T, gidx_of, sel_u, sel_i, out, lane, low_bit, idx_bits);
-    else if (npos <= 128) wave_topk_radix<2>(u, npos, T, gidx_of, sel_u, sel_i, out, lane, low_bit, idx_bits);
-    else if (npos <= 256) wave_topk_radix<4>(u, npos, T, gidx_of, sel_u, sel_i, out, lane, low_bit, idx_bits);
-    else if (npos <= 512) wave_topk_radix<8>(u, npos, T, gidx_of, sel_u, sel_i, out, lane, low_bit, idx_bits);
-    else wave_topk_radix<16>(u, npos, T, gidx_of, sel_u, sel_i, out, lane, low_bit, idx_bits);
-}
-
-constexpr int kRadixMaxN = 1024;      // keys per row the radix kernels keep in LDS
-
-// dense selection for n <= kRadixMaxN: 16 query rows per workgroup, all n keys scored into LDS
-// (16 waves: one row each, so the 16 selections run side by side instead of four deep)
-__global__ __launch_bounds__(1024) void topk_dense_radix_kernel(const bf16* __restrict__ pq, const bf16* __restrict__ pk,
-                                                                int* __restrict__ out, int n, int T, int round_scores) {
-    HIP_DYNAMIC_SHARED(unsigned, su)                          // [16][n + 1]
-    __shared__ unsigned sel_u[16][kWave];
-    __shared__ int sel_i[16][kWave];
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const int bh = blockIdx.y, q0 = blockIdx.x * 16;
-    const int stride = n + 1;
-    const bf16* pqb = pq + ((int64_t)bh * n + q0) * kD;
-    const bf16* pkb = pk + (int64_t)bh * n * kD;
-    bf16x8 bq[2];
-    bq[0] = ld16(pqb + (lane & 15) * kD + (lane >> 4) * 8);
-    bq[1] = ld16(pqb + (lane & 15) * kD + (lane >> 4) * 8 + 32);
-    for (int tile = wave; tile < n / 16; tile += 16) {
-        f32x4 s = score_tile(pkb + (int64_t)tile * 16 * kD, bq);
+    cut();
+    // at most T + kSpare keys are left in this wave's buffer of every row (all of its keys if it saw fewer)
+    const int have = cnt[wave][r];
+    Key key[kWin / 4], top = 0;
 #pragma unroll
-        for (int e = 0; e < 4; e++)
-            // (a score rounded to bf16 has 16 constant low key bits -- ones when negative; cleared, the
-            // selection below need not look at them)
-            su[(lane & 15) * stride + tile * 16 + 4 * (lane >> 4) + e] =
-                round_scores ? (ordered_bits(rn_bf16(s[e])) & 0xFFFF0000u) : ordered_bits(s[e]);
+    for (int i = 0; i < kWin / 4; i++) {
+        const int at = i * 4 + quad;
+        key[i] = at < have ? my[r][at] : (Key)0;
+        top = key[i] > top ? key[i] : top;
     }
+    Key t = 1;
+    if (PARTS > 1) {                                          // little more than the T best of the parts' keys
+        __shared__ Key tops[PARTS][16];
+        top = quad_max_u(top);
+        if (lane < 16) tops[wave][lane] = top;
+        __syncthreads();
+        for (int w = 0; w < PARTS; w++) top = tops[w][r] > top ? tops[w][r] : top;
+        int turn = 0, n_ge;
+        t = row_threshold<kWin / 4, PARTS, Key>(key, T, (Key)1, top, &share, turn, wave, lane, n_ge);
+    }
+    int mine = 0;
+#pragma unroll
+    for (int i = 0; i < kWin / 4; i++) mine += key[i] >= t ? 1 : 0;
     __syncthreads();
-    for (int row = wave; row < 16; row += 16)
-        wave_topk_radix_any(
-            su + row * stride, n, T, [](int pos) { return pos; }, sel_u[wave], sel_i[wave],
-            out + ((int64_t)bh * n + q0 + row) * T, lane, round_scores ? 16 : 0, 32 - __builtin_clz(n - 1));
+    int slot = mine > 0 ? atomicAdd(&n_win[rowt][r], mine) : 0;
+    const Key t2 = compare_again(t, slot);
+#pragma unroll
+    for (int i = 0; i < kWin / 4; i++)
+        if (key[i] >= t2) win[r][min(slot++, kWin)] = StreamKey<Key>::wide(key[i]);
+    __syncthreads();
+    int* o = out + ((int64_t)bh * n + q0) * T;
+    if (PARTS == 1) write_winners<1>(win, n_win[rowt], T, o, T, lane, wide_index);
+    else write_winners<kStreamWaves>(win, n_win[0], T, o, T, tid, wide_index);
 }
 
-constexpr int kSparseWaves = 8;       // two rows per wave: four workgroups fit a CU and the grid is one round
-// pq_par != nullptr: the parents are selected here first -- row G of the level above (N1/16 tokens, at most
-// kCascadeMaxParents) against all of its keys, scores rounded to bf16, top T2 as topk_dense_radix_kernel does it -- and
-// written to par_out; otherwise they are read from pidx.
-__global__ __launch_bounds__(64 * kSparseWaves) void topk_sparse_kernel(const bf16* __restrict__ pq, const bf16* __restrict__ pk,
-                                                           const int* __restrict__ pidx, int* __restrict__ out, int N1,
-                                                           int T, int T2, const bf16* __restrict__ pq_par,
-                                                           const bf16* __restrict__ pk_par, int* __restrict__ par_out) {
-    __shared__ unsigned su[16][kMaxCand + 1];
-    __shared__ int cand[kMaxCand];
-    __shared__ unsigned sel_u[16][kWave];
-    __shared__ int sel_i[16][kWave];
-    __shared__ int par[kMaxCand / 16];
-    static_assert(16 * (kMaxCand + 1) >= kRadixMaxN, "the parents' scores borrow the candidates' score rows");
-
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const int bh = blockIdx.y, G = blockIdx.x;
-    const int N2 = N1 / kBlk, C = T2 * kBlk;
+// Parent-guided selection: 16 sibling rows per workgroup against the 16 * T2 tokens under their parent's T2 blocks, W waves
+// (1 up to T2 = 16, 2 beyond: 64 keys a lane).  The parents are sorted by index first, so that of equal scores the one at the
+// smaller position wins, as it must.
+// P > 0: the parents are selected here first -- row G of the level above (N1/16 tokens, at most 16 P W) against all of its
+// keys, scores rounded to bf16, top T2 as topk_dense_kernel does it -- and written to par_out; otherwise they are read from pidx.
+// (One row per wave and 512 threads a workgroup took 25 us for 768 groups of 16 rows, T = T2 = 16, and 123 us for 6144.)
+constexpr int kCascadeMaxParents = 256;           // P * W <= 16
+template <int TPW, int W, int P>
+__global__ __launch_bounds__(64 * W) void topk_sparse_kernel(const bf16* __restrict__ pq, const bf16* __restrict__ pk,
+                                                             const int* __restrict__ pidx, int* __restrict__ out, int N1, int T, int T2,
+                                                             const bf16* __restrict__ pq_par, const bf16* __restrict__ pk_par,
+                                                             int* __restrict__ par_out) {
+    constexpr int E = 4 * TPW;
+    __shared__ RowShare<W> share;
+    __shared__ unsigned long long win[16][kWinStride];
+    __shared__ int n_win[16];
+    __shared__ int par[kMaxCand / 16], par_sorted[W][kMaxCand / 16], n_par;
+    const int tid = threadIdx.x, lane = tid & 63, wave = W == 1 ? 0 : __builtin_amdgcn_readfirstlane(tid >> 6), quad = lane >> 4, r = lane & 15;
+    const int lid = xcd_logical_id();                         // (neighbouring groups have parents in common: one L2)
+    const int bh = lid / (int)gridDim.x, G = lid % (int)gridDim.x;
+    const int N2 = N1 / kBlk;
     const bf16* pqb = pq + ((int64_t)bh * N1 + G * kBlk) * kD;
     const bf16* pkb = pk + (int64_t)bh * N1 * kD;
+    bf16x8 bq[2];
+    bq[0] = ld16(pqb + r * kD + quad * 8);
+    bq[1] = ld16(pqb + r * kD + quad * 8 + 32);
+    if (tid < 16) n_win[tid] = 0;
+    if (tid == 16) n_par = 0;
 
-    if (pq_par != nullptr) {
-        unsigned* su_par = &su[0][0];
-        const bf16* qt = pq_par + ((int64_t)bh * N2 + (G & ~15)) * kD;     // the tile of 16 rows that holds row G
+    if constexpr (P > 0) {
+        // every column of the score tiles is the parent row G, so all sixteen "rows" decide alike; row 0's lanes write
+        const bf16* qt = pq_par + ((int64_t)bh * N2 + G) * kD;
         bf16x8 bp[2];
-        bp[0] = ld16(qt + (lane & 15) * kD + (lane >> 4) * 8);
-        bp[1] = ld16(qt + (lane & 15) * kD + (lane >> 4) * 8 + 32);
-        for (int tile = wave; tile < N2 / 16; tile += kSparseWaves) {
-            f32x4 s = score_tile(pk_par + ((int64_t)bh * N2 + tile * 16) * kD, bp);
-            if ((lane & 15) == (G & 15)) {
+        bp[0] = ld16(qt + quad * 8);
+        bp[1] = ld16(qt + quad * 8 + 32);
+        unsigned key[4 * P], top;
+        f32x4 sp[P];
+        int turn = 0, n_ge;
+        score_tiles<P>(sp, pk_par + (int64_t)bh * N2 * kD, [=](int a) { return min(a * W + wave, N2 / 16 - 1) * 16; }, bp, lane);
 #pragma unroll
-                for (int e = 0; e < 4; e++) su_par[tile * 16 + 4 * (lane >> 4) + e] = ordered_bits(rn_bf16(s[e])) & 0xFFFF0000u;
+        for (int a = 0; a < P; a++)
+#pragma unroll
+            for (int e = 0; e < 4; e++) {
+                const int tile = a * W + wave;
+                key[4 * a + e] = tile * 16 < N2 ? packed_key(sp[a][e], tile * 16 + 4 * quad + e) : 0u;
+            }
+        const unsigned lo = row_bound<P, W>(key, N2 / 16, T2, top, &share, turn, wave, lane);
+        const unsigned t = row_threshold<4 * P, W>(key, T2, lo, top, &share, turn, wave, lane, n_ge);
+        int mine = 0;
+#pragma unroll
+        for (int i = 0; i < 4 * P; i++) mine += key[i] >= t ? 1 : 0;
+        __syncthreads();                                      // (n_par is cleared)
+        int slot = (r == 0 && mine > 0) ? atomicAdd(&n_par, mine) : 0;
+        const unsigned t2 = compare_again(t, slot);
+        if (r == 0) {
+#pragma unroll
+            for (int i = 0; i < 4 * P; i++) {
+                const bool on = key[i] >= t2;
+                win[0][on ? min(slot, kWin) : kWin] = key[i];
+                slot += on ? 1 : 0;
             }
         }
         __syncthreads();
-        if (wave == 0)
-            wave_topk_radix_any(
-                su_par, N2, T2, [](int pos) { return pos; }, sel_u[0], sel_i[0], par, lane, 16, 32 - __builtin_clz(N2 - 1));
-        __syncthreads();
-        if (tid < T2) par_out[((int64_t)bh * N2 + G) * T2 + tid] = par[tid];
+        const unsigned own = (unsigned)win[0][lane];          // (at most 32 + kSpare keys, one a lane, handed round with readlane)
+        const int m = __builtin_amdgcn_readfirstlane(n_ge);
+        int rank = 0;
+        for (int j = 0; j < m; j++) rank += (unsigned)__builtin_amdgcn_readlane((int)own, j) > own ? 1 : 0;
+        const int idx = 0xFFFF - (int)(own & 0xFFFFu);
+        if (wave == 0 && lane < m && rank < T2) {
+            par[rank] = idx;
+            par_out[((int64_t)bh * N2 + G) * T2 + rank] = idx;
+        }
     } else {
         if (tid < T2) par[tid] = clampi(pidx[((int64_t)bh * N2 + G) * T2 + tid], 0, N2 - 1);
-        __syncthreads();
     }
-    for (int i = tid; i < C; i += 64 * kSparseWaves) cand[i] = par[i / kBlk] * kBlk + (i % kBlk);
-    bf16x8 bq[2];
-    bq[0] = ld16(pqb + (lane & 15) * kD + (lane >> 4) * 8);
-    bq[1] = ld16(pqb + (lane & 15) * kD + (lane >> 4) * 8 + 32);
     __syncthreads();
+    {   // by index, every wave for itself; the clamp keeps what a lane without a parent reads out of use
+        const int own = par[min(lane, T2 - 1)];
+        int rank = 0;
+        for (int j = 0; j < T2; j++) {
+            const int o = __builtin_amdgcn_readlane(own, j);
+            rank += (o < own || (o == own && j < lane)) ? 1 : 0;
+        }
+        if (lane < T2) par_sorted[wave][rank] = own;
+    }
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    const int mine_par = par_sorted[wave][min(lane, T2 - 1)];
 
-    for (int a = wave; a < T2; a += kSparseWaves) {
-        f32x4 s = score_tile(pkb + (int64_t)cand[a * kBlk] * kD, bq);
+    // position of key i of this lane: tile (i / 4) * W + wave, token 4 * quad + i % 4 of it
+    unsigned key[E];
+    int blk[TPW];                                             // (wave-uniform: scalar registers)
 #pragma unroll
-        for (int e = 0; e < 4; e++) su[lane & 15][a * kBlk + 4 * (lane >> 4) + e] = ordered_bits(s[e]);
+    for (int a = 0; a < TPW; a++) blk[a] = __builtin_amdgcn_readlane(mine_par, min(a * W + wave, T2 - 1)) * kBlk;
+    f32x4 s[TPW];
+    score_tiles<TPW>(s, pkb, [&](int a) { return blk[a]; }, bq, lane);
+#pragma unroll
+    for (int a = 0; a < TPW; a++)
+#pragma unroll
+        for (int e = 0; e < 4; e++) key[4 * a + e] = a * W + wave < T2 ? ordered_key(s[a][e]) : 0u;
+    int turn = 0, n_ge;
+    unsigned top;
+    const unsigned lo = row_bound<TPW, W>(key, T2, T, top, &share, turn, wave, lane);
+    const unsigned t = row_threshold<E, W>(key, T, lo, top, &share, turn, wave, lane, n_ge);
+    const bool tie = n_ge > T + kSpare;
+    if (__ballot(tie) != 0) {                                 // of the keys equal to t, the ones at the smallest positions are taken
+        int above = 0;
+#pragma unroll
+        for (int i = 0; i < E; i++) above += (key[i] > t) ? 1 : 0;
+        above = rows_sum<W>(above, &share, turn, wave, lane);
+        int a0 = -1, a1 = T2 * kBlk - 1;
+        while (__ballot(tie && a1 - a0 > 1) != 0) {
+            const int mid = a0 + ((a1 - a0) >> 1);
+            const unsigned te = compare_again(t, a1);
+            int c = 0;
+#pragma unroll
+            for (int i = 0; i < E; i++) c += (key[i] == te && ((i >> 2) * W + wave) * 16 + 4 * quad + (i & 3) <= mid) ? 1 : 0;
+            c = rows_sum<W>(c, &share, turn, wave, lane);
+            if (a1 - a0 > 1) {
+                if (c >= T - above) a1 = mid;
+                else a0 = mid;
+            }
+        }
+        if (tie) {
+#pragma unroll
+            for (int i = 0; i < E; i++) key[i] = (key[i] == t && ((i >> 2) * W + wave) * 16 + 4 * quad + (i & 3) > a1) ? 0u : key[i];
+        }
+    }
+    int mine = 0;
+#pragma unroll
+    for (int i = 0; i < E; i++) mine += key[i] >= t ? 1 : 0;
+    int slot = mine > 0 ? atomicAdd(&n_win[r], mine) : 0;
+    const unsigned t2 = compare_again(t, slot);
+#pragma unroll
+    for (int a = 0; a < TPW; a++) {
+        const int base = (a * W + wave) * kBlk + 4 * quad;   // position: unique also where a caller's list names a parent twice
+#pragma unroll
+        for (int e = 0; e < 4; e++) {
+            const bool on = key[4 * a + e] >= t2;
+            win[r][on ? min(slot, kWin) : kWin] = wide_key(key[4 * a + e], base + e);
+            slot += on ? 1 : 0;
+        }
     }
     __syncthreads();
-    for (int row = wave; row < 16; row += kSparseWaves)
-        wave_topk_radix_any(
-            su[row], C, T, [&](int pos) { return cand[pos]; }, sel_u[wave], sel_i[wave],
-            out + ((int64_t)bh * N1 + G * kBlk + row) * T, lane, 0, 32 - __builtin_clz(N1 - 1));
+    write_winners<W>(win, n_win, T, out + ((int64_t)bh * N1 + G * kBlk) * T, T, tid, [&](unsigned low) {
+        const int pos = wide_index(low);
+        return par_sorted[wave][pos / kBlk] * kBlk + pos % kBlk;
+    });
 }
 
 }  // namespace llsa
@@ -336,18 +666,57 @@ extern "C" int llsa_topk_dense(const void* pq, const void* pk, int32_t* out_idx,
     LLSA_REQUIRE(B > 0 && H > 0 && n > 0 && n % 16 == 0, "topk_dense: n=%d must be a positive multiple of 16", n);
     LLSA_REQUIRE(T >= 1 && T <= kMaxT && T <= n, "topk_dense: need 1 <= T <= min(%d, n=%d), got %d", kMaxT, n, T);
     LLSA_REQUIRE(aligned16(pq) && aligned16(pk), "topk_dense: inputs must be 16-byte aligned");
-    if (n <= kRadixMaxN) {
-        const int lds = (int)sizeof(unsigned) * 16 * (n + 1);
-        if (lds > 60 * 1024) {
-            hipError_t e = hipFuncSetAttribute((const void*)topk_dense_radix_kernel, hipFuncAttributeMaxDynamicSharedMemorySize, lds);
-            if (e != hipSuccess) return fail(-101, "topk_dense: cannot raise dynamic LDS to %d bytes: %s", lds, hipGetErrorString(e));
-        }
-        hipLaunchKernelGGL(topk_dense_radix_kernel, dim3(n / 16, B * H), dim3(1024), sizeof(unsigned) * 16 * (n + 1),
-                           (hipStream_t)stream, (const bf16*)pq, (const bf16*)pk, out_idx, n, T, round_scores);
-    } else
-        hipLaunchKernelGGL(topk_dense_kernel, dim3(n / 16, B * H), dim3(256), 0, (hipStream_t)stream, (const bf16*)pq,
-                           (const bf16*)pk, out_idx, n, T, round_scores);
+    const hipStream_t st = (hipStream_t)stream;
+    const bf16 *q = (const bf16*)pq, *k = (const bf16*)pk;
+    if (n <= kRegMaxN) {
+        const dim3 grid(n / 16, B * H);
+#define LLSA_DENSE(TPW, W)                                                                                                               \
+    do {                                                                                                                                 \
+        if (round_scores)                                                                                                                \
+            hipLaunchKernelGGL(HIP_KERNEL_NAME(topk_dense_kernel<TPW, W, true>), grid, dim3(64 * W), 0, st, q, k, out_idx, n, T);        \
+        else hipLaunchKernelGGL(HIP_KERNEL_NAME(topk_dense_kernel<TPW, W, false>), grid, dim3(64 * W), 0, st, q, k, out_idx, n, T);      \
+    } while (0)
+        if (n <= 64) LLSA_DENSE(4, 1);
+        else if (n <= 128) LLSA_DENSE(2, 4);
+        else if (n <= 256) LLSA_DENSE(4, 4);
+        else if (n <= 512) LLSA_DENSE(8, 4);
+        else LLSA_DENSE(16, 4);
+#undef LLSA_DENSE
+    } else {
+        // one wave per sixteen rows while that fills the chip twice over (1024 SIMDs), four waves with a quarter of the keys each below
+        const bool wide = !round_scores || n > kMaxPackedKeys;
+        const bool whole = n % 64 == 0 && (int64_t)n / 16 * B * H >= 2048;
+        const dim3 grid(whole ? n / 64 : n / 16, B * H), block(64 * kStreamWaves);
+        if (whole && !wide) hipLaunchKernelGGL(HIP_KERNEL_NAME(topk_stream_kernel<unsigned, 1>), grid, block, 0, st, q, k, out_idx, n, T, round_scores);
+        else if (whole) hipLaunchKernelGGL(HIP_KERNEL_NAME(topk_stream_kernel<unsigned long long, 1>), grid, block, 0, st, q, k, out_idx, n, T, round_scores);
+        else if (!wide) hipLaunchKernelGGL(HIP_KERNEL_NAME(topk_stream_kernel<unsigned, 4>), grid, block, 0, st, q, k, out_idx, n, T, round_scores);
+        else hipLaunchKernelGGL(HIP_KERNEL_NAME(topk_stream_kernel<unsigned long long, 4>), grid, block, 0, st, q, k, out_idx, n, T, round_scores);
+    }
     return launch_status("topk_dense");
+}
+
+static void launch_sparse(const bf16* pq, const bf16* pk, const int* pidx, int* out, int B, int H, int N1, int T, int T2, const bf16* pq_par,
+                          const bf16* pk_par, int* par_out, hipStream_t st) {
+    const dim3 grid(N1 / 16, B * H);
+#define LLSA_SPARSE_P(TPW, W, P) \
+    hipLaunchKernelGGL(HIP_KERNEL_NAME(topk_sparse_kernel<TPW, W, P>), grid, dim3(64 * W), 0, st, pq, pk, pidx, out, N1, T, T2, pq_par, pk_par, par_out)
+#define LLSA_SPARSE(TPW, W)                                    \
+    do {                                                       \
+        if (pq_par == nullptr) LLSA_SPARSE_P(TPW, W, 0);       \
+        else if (N1 / 16 <= 64) LLSA_SPARSE_P(TPW, W, 4 / W);  \
+        else LLSA_SPARSE_P(TPW, W, 16 / W);                    \
+    } while (0)
+    // few groups: four waves each, for the shorter chain of steps; many (2 waves per SIMD): as few as hold the keys, for fewer instructions
+    const bool few = (int64_t)N1 / 16 * B * H < 2048;
+    if (T2 <= 4) LLSA_SPARSE(4, 1);
+    else if (T2 <= 8 && few) LLSA_SPARSE(2, 4);
+    else if (T2 <= 8) LLSA_SPARSE(8, 1);
+    else if (T2 <= 16 && few) LLSA_SPARSE(4, 4);
+    else if (T2 <= 16) LLSA_SPARSE(16, 1);
+    else if (few) LLSA_SPARSE(8, 4);
+    else LLSA_SPARSE(16, 2);
+#undef LLSA_SPARSE
+#undef LLSA_SPARSE_P
 }
 
 extern "C" int llsa_topk_sparse(const void* pq, const void* pk, const int32_t* parent_idx, int32_t* out_idx, int B, int H,
@@ -357,14 +726,11 @@ extern "C" int llsa_topk_sparse(const void* pq, const void* pk, const int32_t* p
     LLSA_REQUIRE(T2 >= 1 && T2 * 16 <= kMaxCand && T2 <= N1 / 16, "topk_sparse: need 1 <= T2 <= min(%d, N1/16), got %d", kMaxCand / 16, T2);
     LLSA_REQUIRE(T >= 1 && T <= kMaxT && T <= T2 * 16, "topk_sparse: need 1 <= T <= min(%d, 16*T2), got %d", kMaxT, T);
     LLSA_REQUIRE(aligned16(pq) && aligned16(pk), "topk_sparse: inputs must be 16-byte aligned");
-    hipLaunchKernelGGL(topk_sparse_kernel, dim3(N1 / 16, B * H), dim3(64 * kSparseWaves), 0, (hipStream_t)stream, (const bf16*)pq,
-                       (const bf16*)pk, parent_idx, out_idx, N1, T, T2, (const bf16*)nullptr, (const bf16*)nullptr, (int*)nullptr);
+    launch_sparse((const bf16*)pq, (const bf16*)pk, parent_idx, out_idx, B, H, N1, T, T2, nullptr, nullptr, nullptr, (hipStream_t)stream);
     return launch_status("topk_sparse");
 }
 
-// (a workgroup selects its parent row on one wave: beyond a few hundred parent tokens the separate dense kernel,
-// sixteen rows per workgroup side by side, is faster -- 277 vs 120 + 43 us at 1024)
-constexpr int kCascadeMaxParents = 256;
+// (a wave selects its parent row sixteen times over: beyond a few hundred parent tokens the separate dense kernel is faster)
 extern "C" int llsa_topk_cascade_max_parents(void) { return kCascadeMaxParents; }
 
 extern "C" int llsa_topk_cascade(const void* pq_parent, const void* pk_parent, int32_t* parent_out, const void* pq, const void* pk,
@@ -376,7 +742,7 @@ extern "C" int llsa_topk_cascade(const void* pq_parent, const void* pk_parent, i
     LLSA_REQUIRE(T2 >= 1 && T2 * 16 <= kMaxCand && T2 <= N1 / 16, "topk_cascade: need 1 <= T2 <= min(%d, N1/16), got %d", kMaxCand / 16, T2);
     LLSA_REQUIRE(T >= 1 && T <= kMaxT && T <= T2 * 16, "topk_cascade: need 1 <= T <= min(%d, 16*T2), got %d", kMaxT, T);
     LLSA_REQUIRE(aligned16(pq) && aligned16(pk) && aligned16(pq_parent) && aligned16(pk_parent), "topk_cascade: inputs must be 16-byte aligned");
-    hipLaunchKernelGGL(topk_sparse_kernel, dim3(N1 / 16, B * H), dim3(64 * kSparseWaves), 0, (hipStream_t)stream, (const bf16*)pq,
-                       (const bf16*)pk, (const int*)nullptr, out_idx, N1, T, T2, (const bf16*)pq_parent, (const bf16*)pk_parent, parent_out);
+    launch_sparse((const bf16*)pq, (const bf16*)pk, nullptr, out_idx, B, H, N1, T, T2, (const bf16*)pq_parent, (const bf16*)pk_parent, parent_out,
+                  (hipStream_t)stream);
     return launch_status("topk_cascade");
 }

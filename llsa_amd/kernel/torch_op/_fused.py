@@ -203,8 +203,9 @@ class LlsaFused(Function):
         # Selection, coarse to fine: a dense top-k over the coarsest level's tokens (each of them is a block of the level
         # below), then level by level among the blocks under the parent's selection.
         first = L - 1               # the first parent-guided selection still to do
-        if L >= 2 and n[L] <= lib.topk_cascade_max_parents():
-            # the dense selection rides in the workgroups of the first parent-guided one: one launch less
+        if L >= 2 and n[L] <= lib.topk_cascade_max_parents() and (n[L] <= 64 or B * H * n[L] < 2048):
+            # the dense selection rides in the workgroups of the first parent-guided one: one launch less (more than 64
+            # parent tokens in a large grid: sixteen rows a wave side by side in a launch of their own are cheaper)
             _check(lib, lib.topk_cascade(at(lay.pq, L), at(lay.pk, L), pi(lay.sel[L - 1]), at(lay.pq, L - 1), at(lay.pk, L - 1),
                                          pi(lay.sel[L - 2]), B, H, n[L - 1], topks[L - 2], topks[L - 1], stream), "topk_cascade")
             first = L - 2
