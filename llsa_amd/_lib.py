@@ -7,11 +7,16 @@ implementation in this package.
 from __future__ import annotations
 
 import ctypes as C
+import importlib.machinery
+import importlib.util
 import os
 from typing import Optional
 
+import torch                                                # (the host module links against it)
+
 HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(HERE, "lib", "libllsa_hip.so")
+HOST_PATH = os.path.join(HERE, "lib", "_llsa_host.so")
 
 c_void_p, c_int, c_int32, c_int64, c_float = C.c_void_p, C.c_int, C.c_int32, C.c_int64, C.c_float
 
@@ -109,6 +114,26 @@ class LlsaError(RuntimeError):
     pass
 
 
+_HOST = None
+
+
+def host_module():
+    """The native host side of the fused operators (csrc/host/operators.cpp)."""
+    global _HOST
+    if _HOST is None:
+        if not os.path.exists(HOST_PATH):
+            raise ImportError(f"{HOST_PATH} not found: build it first (python -m llsa_amd.build)")
+        loader = importlib.machinery.ExtensionFileLoader("_llsa_host", HOST_PATH)
+        mod = importlib.util.module_from_spec(importlib.util.spec_from_file_location("_llsa_host", HOST_PATH, loader=loader))
+        loader.exec_module(mod)
+        if mod.abi_version != ABI_VERSION:
+            raise ImportError(f"{HOST_PATH} was built for ABI version {mod.abi_version}, this package needs {ABI_VERSION}: rebuild it "
+                              "(python -m llsa_amd.build)")
+        mod.set_library_error(LlsaError)
+        _HOST = mod
+    return _HOST
+
+
 class Lib:
     """A loaded libllsa shared object with typed entry points."""
 
@@ -128,6 +153,8 @@ class Lib:
         if self.version() != ABI_VERSION:      # a library built from other sources than this binding describes
             raise ImportError(f"{path} has ABI version {self.version()}, this package needs {ABI_VERSION}: rebuild it "
                               "(python -m llsa_amd.build)")
+        self.host = host_module()
+        self.host_library = self.host.Library({n: C.cast(getattr(self.cdll, n), c_void_p).value for n in _SIGNATURES}, device_library)
 
     def check(self, rc: int, what: str):
         if rc != 0:

@@ -1,0 +1,631 @@
+// The host side of the fused operators (llsa_l1 / l2 / l3 / lk) and of the token permutation: argument checks, one arena
+// per call, the sequence of C-ABI calls of include/llsa_hip.h, and the autograd nodes.
+//
+//     forward   pool_pyramid_fwd (q, k, v: pooled rows, RoPE, operand tiles) [+ deeper levels]
+//               topk_dense / topk_cascade [+ topk_sparse ...]
+//               attn_fwd
+//               transpose_indices_multi  (second stream beside the attention kernel at the long sequences)
+//     backward  attn_bwd with fold_pooled = 1  (dq, dk, dv complete, rotated back) [+ rmsnorm_bwd]
+//
+// Native because at the short sequences a step is bound by its host side: at B=1, H=6, N=1024 the kernels of a forward
+// take about 20 us and those of a forward + backward 70, while the same sequence issued from Python took 33 and 100 to
+// 180 (a backward written in Python also has to win the interpreter lock on the autograd thread).
+//
+// The library's entry points are called through the table of addresses its ctypes binding (llsa_amd/_lib.py) passes in, so
+// that this file works on whatever build of the library the binding has loaded.
+#include <torch/csrc/Exceptions.h>
+#include <torch/csrc/autograd/function.h>
+#include <torch/csrc/autograd/functions/utils.h>
+#include <torch/csrc/autograd/saved_variable.h>
+#include <torch/csrc/autograd/variable.h>
+#include <torch/csrc/utils/pybind.h>
+#include <torch/extension.h>
+#include <c10/hip/HIPStream.h>
+#include <hip/hip_runtime_api.h>
+
+#include <array>
+#include <mutex>
+#include <optional>
+#include <string>
+#include <vector>
+
+#include "../../../include/llsa_hip.h"
+
+namespace {
+
+namespace py = pybind11;
+using at::Tensor;
+using torch::autograd::Node;
+using torch::autograd::SavedVariable;
+using torch::autograd::variable_list;
+
+// ---------------------------------------------------------------------------------------
+// errors: which Python exception, and its text
+// ---------------------------------------------------------------------------------------
+struct Failure {
+    enum Kind { kValue, kNotImplemented, kRuntime, kLibrary } kind;
+    std::string text;
+};
+PyObject* g_library_error = nullptr;      // llsa_amd._lib.LlsaError
+
+[[noreturn]] void fail(Failure::Kind kind, std::string text) { throw Failure{kind, std::move(text)}; }
+
+void set_python_error(const Failure& f) {                 // with the interpreter lock held
+    PyObject* type = f.kind == Failure::kValue            ? PyExc_ValueError
+                     : f.kind == Failure::kNotImplemented ? PyExc_NotImplementedError
+                     : f.kind == Failure::kLibrary && g_library_error != nullptr ? g_library_error
+                                                          : PyExc_RuntimeError;
+    PyErr_SetString(type, f.text.c_str());
+}
+
+template <typename Fn>
+auto without_interpreter(Fn fn) {
+    std::optional<Failure> failure;
+    {
+        py::gil_scoped_release release;
+        try {
+            return fn();
+        } catch (const Failure& f) {
+            failure = f;
+        }
+    }
+    set_python_error(*failure);
+    throw py::error_already_set();
+}
+// the same on a thread of the autograd engine, which does not hold the lock
+template <typename Fn>
+auto in_engine(Fn fn) {
+    try {
+        return fn();
+    } catch (const Failure& f) {
+        py::gil_scoped_acquire acquire;
+        set_python_error(f);
+        python_error e;
+        e.persist();
+        throw e;
+    }
+}
+
+// ---------------------------------------------------------------------------------------
+// the library
+// ---------------------------------------------------------------------------------------
+struct Library {
+    decltype(&llsa_last_error_string) last_error_string;
+    decltype(&llsa_pool_pyramid_fwd) pool_pyramid_fwd;
+    decltype(&llsa_topk_dense) topk_dense;
+    decltype(&llsa_topk_sparse) topk_sparse;
+    decltype(&llsa_topk_cascade) topk_cascade;
+    decltype(&llsa_topk_cascade_max_parents) topk_cascade_max_parents;
+    decltype(&llsa_attn_fwd) attn_fwd;
+    decltype(&llsa_transpose_indices_multi) transpose_indices_multi;
+    decltype(&llsa_work_list_len) work_list_len;
+    decltype(&llsa_fine_chunk) fine_chunk;
+    decltype(&llsa_attn_bwd_workspace_bytes) attn_bwd_workspace_bytes;
+    decltype(&llsa_attn_bwd) attn_bwd;
+    decltype(&llsa_rmsnorm_bwd_partials) rmsnorm_bwd_partials;
+    decltype(&llsa_rmsnorm_bwd) rmsnorm_bwd;
+    decltype(&llsa_gather_rows) gather_rows;
+    bool device;                          // false: the CPU emulation build the tests install
+
+    Library(const std::map<std::string, uintptr_t>& at_, bool device_) : device(device_) {
+        auto get = [&](const char* name, auto& fn) { fn = reinterpret_cast<std::decay_t<decltype(fn)>>(at_.at(name)); };
+        get("llsa_last_error_string", last_error_string);
+        get("llsa_pool_pyramid_fwd", pool_pyramid_fwd);
+        get("llsa_topk_dense", topk_dense);
+        get("llsa_topk_sparse", topk_sparse);
+        get("llsa_topk_cascade", topk_cascade);
+        get("llsa_topk_cascade_max_parents", topk_cascade_max_parents);
+        get("llsa_attn_fwd", attn_fwd);
+        get("llsa_transpose_indices_multi", transpose_indices_multi);
+        get("llsa_work_list_len", work_list_len);
+        get("llsa_fine_chunk", fine_chunk);
+        get("llsa_attn_bwd_workspace_bytes", attn_bwd_workspace_bytes);
+        get("llsa_attn_bwd", attn_bwd);
+        get("llsa_rmsnorm_bwd_partials", rmsnorm_bwd_partials);
+        get("llsa_rmsnorm_bwd", rmsnorm_bwd);
+        get("llsa_gather_rows", gather_rows);
+    }
+    void check(int rc, const char* what) const {
+        if (rc != 0) fail(Failure::kLibrary, std::string(what) + " failed (" + std::to_string(rc) + "): " + last_error_string());
+    }
+    void on_device(const Tensor& t) const {
+        if (device && !t.is_cuda())
+            fail(Failure::kRuntime, "llsa_amd runs on an AMD GPU only (got a CPU tensor); there is no CPU implementation");
+    }
+    void* stream(const Tensor& t) const {
+        return device ? static_cast<void*>(c10::hip::getCurrentHIPStream(t.device().index()).stream()) : nullptr;
+    }
+};
+
+std::string text_of(at::IntArrayRef v) {
+    std::string s = "(";
+    for (size_t i = 0; i < v.size(); i++) s += (i ? ", " : "") + std::to_string(v[i]);
+    return s + ")";
+}
+
+bool strides_multiple(at::IntArrayRef st, int64_t m) {
+    for (size_t i = 0; i + 1 < st.size(); i++)
+        if (st[i] % m != 0) return false;
+    return true;
+}
+// last stride 1 and every row 16-byte aligned: what the kernels' 16-byte loads need
+bool rows_ok(const Tensor& t) {
+    return t.stride(-1) == 1 && reinterpret_cast<uintptr_t>(t.data_ptr()) % 16 == 0 && strides_multiple(t.strides(), 8);
+}
+Tensor as_rows(const Tensor& t) { return rows_ok(t) ? t : t.contiguous(); }
+
+int64_t align_up(int64_t n, int64_t a) { return (n + a - 1) / a * a; }
+
+// ---------------------------------------------------------------------------------------
+// The second stream of a device, and the two events that tie it to the caller's.  The events are a thread's own: a wait
+// refers to the last record before it in issue order, so a thread may record them again in its next call.
+// ---------------------------------------------------------------------------------------
+struct SideStream {
+    hipEvent_t ready = nullptr, done = nullptr;
+    explicit SideStream() {
+        if (hipEventCreateWithFlags(&ready, hipEventDisableTiming) != hipSuccess || hipEventCreateWithFlags(&done, hipEventDisableTiming) != hipSuccess)
+            fail(Failure::kRuntime, "llsa_amd: cannot create an event");
+    }
+};
+constexpr int kMaxDevices = 64;
+hipStream_t side_stream(int device) {
+    static std::mutex mutex;
+    static std::array<hipStream_t, kMaxDevices> streams{};
+    std::lock_guard<std::mutex> lock(mutex);
+    if (streams.at(device) == nullptr) streams.at(device) = c10::hip::getStreamFromPool(false, static_cast<c10::DeviceIndex>(device)).stream();
+    return streams[device];
+}
+SideStream& side_events(int device) {
+    static thread_local std::array<std::unique_ptr<SideStream>, kMaxDevices> events;
+    if (!events.at(device)) events.at(device) = std::make_unique<SideStream>();
+    return *events[device];
+}
+void hip_check(hipError_t e) {
+    if (e != hipSuccess) fail(Failure::kRuntime, std::string("llsa_amd: ") + hipGetErrorString(e));
+}
+
+// ---------------------------------------------------------------------------------------
+// Where everything the forward produces lives: one arena (bytes), every section contiguous (B*H, ...) and 256-byte aligned.
+// Level 0 is the tokens themselves, level l = 1..L the pooled levels (n[l] = N / 16^l tokens each).
+// ---------------------------------------------------------------------------------------
+constexpr int kL = LLSA_MAX_LEVELS;
+struct Layout {
+    int64_t n[kL + 2];
+    int L, chunk;
+    int32_t topk[kL];
+    int64_t pq[kL + 1], pk[kL + 1], pv[kL + 1];             // pooled rows, index = level
+    int64_t qr, kr, vr = -1, vt;                            // operand tiles of the tokens
+    int64_t pkr[kL + 1], pvr[kL + 1], pvt[kL + 1];          // and of the pooled levels
+    int64_t sel[kL], off[kL], flat[kL], inv[kL], work = -1; // sel[0]: fine blocks per query block, sel[l]: blocks of level l per group of 16^(l+1) queries
+    int64_t lse, bytes;
+    int64_t dpk[kL + 1], dpv[kL + 1], ws, ws_bytes = 0, bwd_bytes;       // the backward's arena
+
+    Layout(const Library& lib, int64_t B, int64_t H, int64_t N, const std::vector<int64_t>& topks, bool grad) {
+        const int64_t BH = B * H;
+        L = static_cast<int>(topks.size());
+        n[0] = N;
+        for (int l = 1; l < L + 2; l++) n[l] = n[l - 1] / 16;
+        for (int l = 0; l < L; l++) topk[l] = static_cast<int32_t>(topks[l]);
+        int64_t o = 0;
+        auto take = [&](int64_t per_bh, bool on = true) -> int64_t {
+            if (!on) return -1;
+            const int64_t at = o;
+            o = align_up(o + BH * std::max<int64_t>(per_bh, 0), 256);      // (a topk below 1 is the library's to reject)
+            return at;
+        };
+        for (int l = 1; l <= L; l++) pq[l] = take(n[l] * 128);
+        for (int l = 1; l <= L; l++) pk[l] = take(n[l] * 128);
+        for (int l = 1; l <= L; l++) pv[l] = take(n[l] * 128);
+        qr = take(n[1] * 2048);
+        kr = take(n[1] * 2048);
+        vr = take(n[1] * 2048, grad);
+        vt = take(n[1] * 2048);
+        for (int l = 1; l <= L; l++) {
+            pkr[l] = take(n[l + 1] * 2048);
+            pvr[l] = take(n[l + 1] * 2048, grad);
+            pvt[l] = take(n[l + 1] * 2048);
+        }
+        for (int l = 0; l < L; l++) sel[l] = take(4 * n[l + 1] * topk[l]);
+        lse = take(4 * N);
+        chunk = lib.fine_chunk(static_cast<int>(N));
+        if (grad) {
+            for (int l = 0; l < L; l++) {
+                off[l] = take(4 * (n[l + 1] + 1));
+                flat[l] = take(4 * n[l + 1] * topk[l]);
+                inv[l] = take(4 * n[l + 1] * topk[l], l > 0);
+            }
+            work = take(4 * lib.work_list_len(static_cast<int>(n[1]), static_cast<int>(n[1]), topk[0], chunk));
+        }
+        bytes = o;
+        o = 0;
+        if (grad) {
+            ws_bytes = lib.attn_bwd_workspace_bytes(static_cast<int>(B), static_cast<int>(H), static_cast<int>(N), topk, L);
+            for (int l = 1; l <= L; l++) {
+                dpk[l] = take(n[l] * 128);
+                dpv[l] = take(n[l] * 128);
+            }
+        }
+        ws = o;
+        bwd_bytes = o + ws_bytes;
+    }
+};
+
+// ---------------------------------------------------------------------------------------
+// backward node
+// ---------------------------------------------------------------------------------------
+struct LlsaBackward : public Node {
+    std::shared_ptr<Library> lib;
+    std::optional<Layout> lay;
+    int64_t B, H, N;
+    std::array<int64_t, 4> sq, sk, sv;
+    double eps;
+    bool has_gq = false, has_gk = false;
+    at::ScalarType type_gq = at::kFloat, type_gk = at::kFloat;
+    Tensor arena;                                            // nobody else sees it
+    SavedVariable o, freq, gq, gk, q, k;
+    bool released = false;
+
+    std::string name() const override { return "LlsaBackward"; }
+    void release_variables() override {
+        std::lock_guard<std::mutex> lock(mutex_);
+        released = true;
+        arena.reset();
+        for (SavedVariable* s : {&o, &freq, &gq, &gk, &q, &k}) s->reset_data();
+    }
+    variable_list apply(variable_list&& grads) override {
+        std::lock_guard<std::mutex> lock(mutex_);
+        return in_engine([&] { return run(grads[0]); });
+    }
+    variable_list run(const Tensor& grad_out) {
+        if (released) fail(Failure::kRuntime, torch::autograd::ERR_BACKWARD_TWICE);
+        at::AutoDispatchBelowADInplaceOrView below;
+        const Tensor out = o.unpack(shared_from_this());
+        c10::OptionalDeviceGuard guard(lib->device ? std::optional<at::Device>(out.device()) : std::nullopt);
+        const Tensor d = as_rows(grad_out.defined() ? grad_out : at::zeros_like(out));
+        const Tensor fr = freq.unpack(), wq = gq.unpack(), wk = gk.unpack();
+        const auto opts = out.options();
+        const std::array<int64_t, 4> shape{B, H, N, 64};
+        auto like = [&](const std::array<int64_t, 4>& st) {  // gradients have the layout of their primals when the 8-byte stores allow it
+            return strides_multiple(st, 4) && st[3] == 1 ? at::empty_strided(shape, st, opts) : at::empty(shape, opts);
+        };
+        Tensor dq = like(sq), dk = like(sk), dv = like(sv);
+        const Tensor W = at::empty({lay->bwd_bytes}, opts.dtype(at::kByte));
+        char* const a0 = static_cast<char*>(arena.data_ptr());
+        char* const w0 = static_cast<char*>(W.data_ptr());
+        const Layout& y = *lay;
+        llsa_attn_bwd_args a{};
+        a.dout = d.data_ptr(); a.sdob = d.stride(0); a.sdoh = d.stride(1); a.sdon = d.stride(2);
+        a.o = out.data_ptr(); a.sob = out.stride(0); a.soh = out.stride(1); a.son = out.stride(2);
+        a.lse = reinterpret_cast<const float*>(a0 + y.lse);
+        a.qr = a0 + y.qr; a.kr = a0 + y.kr; a.vr = a0 + y.vr;
+        auto ints = [&](int64_t at) { return reinterpret_cast<const int32_t*>(a0 + at); };
+        a.idx = ints(y.sel[0]); a.off = ints(y.off[0]); a.flat = ints(y.flat[0]); a.work = ints(y.work);
+        a.dq = dq.data_ptr(); a.sdqb = dq.stride(0); a.sdqh = dq.stride(1); a.sdqn = dq.stride(2);
+        a.dk = dk.data_ptr(); a.sdkb = dk.stride(0); a.sdkh = dk.stride(1); a.sdkn = dk.stride(2);
+        a.dv = dv.data_ptr(); a.sdvb = dv.stride(0); a.sdvh = dv.stride(1); a.sdvn = dv.stride(2);
+        float w = 1.f;
+        for (int l = 1; l <= y.L; l++) {
+            llsa_bwd_level& lv = a.lvl[l - 1];
+            w *= 16.f;
+            lv.kr = a0 + y.pkr[l]; lv.vr = a0 + y.pvr[l];
+            lv.dk = w0 + y.dpk[l]; lv.dv = w0 + y.dpv[l];
+            // llsa_l1 keeps the reference's quirk: its pooled path is differentiated with weight 1
+            // (sparse_attention_res_1.py:388-389) although the forward uses token_weight
+            lv.w = w; lv.gw = y.L == 1 ? 1.f : w;
+            if (l < y.L) {
+                lv.sel = ints(y.sel[l]); lv.off = ints(y.off[l]); lv.inv = ints(y.inv[l]); lv.T = y.topk[l];
+            }
+        }
+        a.workspace = w0 + y.ws; a.workspace_bytes = y.ws_bytes;
+        if (fr.defined()) a.freq_dq = a.freq_dk = fr.data_ptr();
+        a.B = static_cast<int32_t>(B); a.H = static_cast<int32_t>(H); a.N = static_cast<int32_t>(N); a.T = y.topk[0]; a.levels = y.L;
+        a.fold_pooled = 1;
+        void* const stream = lib->stream(out);
+        lib->check(lib->attn_bwd(&a, stream), "attn_bwd");
+        Tensor dgq, dgk;
+        if (wq.defined() || wk.defined()) {                  // back through the qk-norm, in place on dq / dk
+            const auto f32 = opts.dtype(at::kFloat);
+            const Tensor P = at::empty({lib->rmsnorm_bwd_partials(a.B, a.H, a.N)}, f32);
+            auto norm = [&](const Tensor& gamma, const Tensor& x, Tensor& dx, at::ScalarType type) {
+                Tensor dg = at::empty({64}, f32);
+                lib->check(lib->rmsnorm_bwd(dx.data_ptr(), dx.strides().data(), x.data_ptr(), x.strides().data(), gamma.data_ptr<float>(),
+                                            static_cast<float>(eps), dx.data_ptr(), dx.strides().data(), dg.data_ptr<float>(), P.data_ptr<float>(),
+                                            a.B, a.H, a.N, stream),
+                           "rmsnorm_bwd");
+                return dg.to(type);
+            };
+            if (wq.defined()) dgq = norm(wq, q.unpack(), dq, type_gq);
+            if (wk.defined()) dgk = norm(wk, k.unpack(), dk, type_gk);
+        }
+        variable_list r{dq, dk, dv};
+        if (has_gq) r.push_back(dgq);
+        if (has_gk) r.push_back(dgk);
+        return r;
+    }
+};
+
+bool wants_grad(const std::optional<Tensor>& t) { return t.has_value() && t->requires_grad(); }
+
+// forward(q, k, v, topks, block_size, freq, gamma_q, gamma_k, eps) -> o
+//
+// topks: one entry per pooled level, (topk1, topk2, ...): the fine blocks a query block keeps, then the blocks of
+// pooled level 1, 2, ... its ancestor groups keep; one entry is llsa_l1, two are llsa_l2.
+// gamma_q / gamma_k ((64,) or none): RMS-normalise q / k over the head dimension first (the qk-norm of the reference's
+// attention processor), inside the pooling pass; they receive gradients.
+Tensor attend(const std::shared_ptr<Library>& lib, const Tensor& q_in, const Tensor& k_in, const Tensor& v_in, std::vector<int64_t> topks,
+              int64_t block_size, const std::optional<Tensor>& freq_in, const std::optional<Tensor>& gq_in, const std::optional<Tensor>& gk_in,
+              double eps) {
+    if (block_size != 16) fail(Failure::kNotImplemented, "block_size must be 16");
+    for (const Tensor* t : {&q_in, &k_in, &v_in}) {
+        lib->on_device(*t);
+        if (t->scalar_type() != at::kBFloat16)
+            fail(Failure::kNotImplemented, "llsa_amd attention kernels are bf16 only (got torch." + std::string(
+                     t->scalar_type() == at::kFloat ? "float32" : t->scalar_type() == at::kHalf ? "float16" : c10::toString(t->scalar_type())) + ")");
+    }
+    if (q_in.dim() != 4 || q_in.size(3) != 64) fail(Failure::kNotImplemented, "llsa_amd attention kernels need (B,H,N,64) tensors (got " + text_of(q_in.sizes()) + ")");
+    if (k_in.sizes() != q_in.sizes() || v_in.sizes() != q_in.sizes()) fail(Failure::kValue, "self-attention only: q, k, v must have the same shape");
+    const int64_t B = q_in.size(0), H = q_in.size(1), N = q_in.size(2);
+    const int L = static_cast<int>(topks.size());
+    if (L < 1 || L > kL) fail(Failure::kValue, "1 to " + std::to_string(kL) + " pooled levels (got " + std::to_string(L) + ")");
+    int64_t mult = 64, per = 16;
+    for (int l = 0; l < L; l++) mult *= 16;
+    if (N % mult != 0)
+        fail(Failure::kValue, "llsa_l" + std::to_string(L) + " needs a token count that is a multiple of " + std::to_string(mult) + " (got " + std::to_string(N) + ")");
+    for (int l = 0; l < L; l++, per *= 16) topks[l] = std::min(topks[l], N / per);
+
+    const bool grad = at::GradMode::is_enabled() && (q_in.requires_grad() || k_in.requires_grad() || v_in.requires_grad() || wants_grad(gq_in) || wants_grad(gk_in));
+    Tensor o;
+    std::shared_ptr<LlsaBackward> node;
+    {
+        at::AutoDispatchBelowADInplaceOrView below;
+        c10::OptionalDeviceGuard guard(lib->device ? std::optional<at::Device>(q_in.device()) : std::nullopt);
+        Tensor freq, gq, gk;
+        if (freq_in.has_value()) {
+            if (freq_in->scalar_type() != at::kBFloat16 || freq_in->dim() != 2 || freq_in->size(0) != N || freq_in->size(1) != 64)
+                fail(Failure::kValue, "rope table must be bf16 (N, 64)");
+            freq = freq_in->contiguous();
+        }
+        const Tensor q = as_rows(q_in), k = as_rows(k_in), v = as_rows(v_in);
+        if (gq_in.has_value()) gq = gq_in->to(q.device(), at::kFloat).contiguous();
+        if (gk_in.has_value()) gk = gk_in->to(q.device(), at::kFloat).contiguous();
+        for (const Tensor* g : {&gq, &gk})
+            if (g->defined() && g->numel() != 64) fail(Failure::kValue, "qk-norm weights must have 64 entries");
+        const Layout y(*lib, B, H, N, topks, grad);
+        const int64_t* n = y.n;
+        const Tensor arena = at::empty({y.bytes}, q.options().dtype(at::kByte));
+        o = strides_multiple(q.strides(), 4) ? at::empty_like(q) : at::empty(q.sizes(), q.options());
+        char* const a0 = static_cast<char*>(arena.data_ptr());
+        auto pa = [&](int64_t at) -> void* { return at < 0 ? nullptr : a0 + at; };
+        auto ints = [&](int64_t at) { return static_cast<int32_t*>(pa(at)); };
+        auto lev = [&](const int64_t* list, int l) -> void* { return l <= L ? pa(list[l]) : nullptr; };      // section of pooled level l (none beyond the last)
+        void* const stream = lib->stream(q);
+        const int b = static_cast<int>(B), h = static_cast<int>(H);
+
+        // The pyramid.  One pass over q, k, v gives the rows of levels 1 and 2 and the tiles of levels 0, 1, 2; every
+        // further pass starts from the rows of level 2p and gives rows and tiles of levels 2p + 1 and 2p + 2.
+        llsa_pool_item it[3];
+        for (int l0 = 0; l0 < L; l0 += 2) {
+            for (int i = 0; i < 3; i++) {                    // q, k, v
+                llsa_pool_item& p = it[i];
+                p = llsa_pool_item{};
+                const int64_t* rows = i == 0 ? y.pq : i == 1 ? y.pk : y.pv;
+                p.n = static_cast<int32_t>(n[l0]);
+                p.y1 = lev(rows, l0 + 1);
+                p.y2 = lev(rows, l0 + 2);
+                if (l0 == 0) {
+                    const Tensor& x = i == 0 ? q : i == 1 ? k : v;
+                    p.x = x.data_ptr(); p.sxb = x.stride(0); p.sxh = x.stride(1); p.sxn = x.stride(2);
+                    p.rope = i < 2 && freq.defined();
+                    p.xr = pa(i == 0 ? y.qr : i == 1 ? y.kr : y.vr);
+                    if (i == 2) p.xt = pa(y.vt);
+                    const Tensor& g = i == 0 ? gq : gk;
+                    if (i < 2 && g.defined()) {
+                        p.gamma = g.data_ptr<float>();
+                        p.eps = static_cast<float>(eps);
+                    }
+                } else {
+                    p.x = pa(rows[l0]); p.sxb = H * n[l0] * 64; p.sxh = n[l0] * 64; p.sxn = 64;
+                }
+                if (i == 1) {
+                    p.y1r = lev(y.pkr, l0 + 1);
+                    p.y2r = lev(y.pkr, l0 + 2);
+                }
+                if (i == 2) {
+                    p.y1r = lev(y.pvr, l0 + 1); p.y1t = lev(y.pvt, l0 + 1);
+                    p.y2r = lev(y.pvr, l0 + 2); p.y2t = lev(y.pvt, l0 + 2);
+                }
+            }
+            lib->check(lib->pool_pyramid_fwd(it, 3, l0 == 0 && freq.defined() ? freq.data_ptr() : nullptr, b, h, stream), "pool_pyramid");
+        }
+
+        // Selection, coarse to fine: a dense top-k over the coarsest level's tokens (each of them is a block of the level
+        // below), then level by level among the blocks under the parent's selection.
+        int first = L - 1;               // the first parent-guided selection still to do
+        if (L >= 2 && n[L] <= lib->topk_cascade_max_parents() && (n[L] <= 64 || B * H * n[L] < 2048)) {
+            // the dense selection rides in the workgroups of the first parent-guided one: one launch less (more than 64
+            // parent tokens in a large grid: sixteen rows a wave side by side in a launch of their own are cheaper)
+            lib->check(lib->topk_cascade(pa(y.pq[L]), pa(y.pk[L]), ints(y.sel[L - 1]), pa(y.pq[L - 1]), pa(y.pk[L - 1]), ints(y.sel[L - 2]), b, h,
+                                         static_cast<int>(n[L - 1]), y.topk[L - 2], y.topk[L - 1], stream),
+                       "topk_cascade");
+            first = L - 2;
+        } else {
+            lib->check(lib->topk_dense(pa(y.pq[L]), pa(y.pk[L]), ints(y.sel[L - 1]), b, h, static_cast<int>(n[L]), y.topk[L - 1], 1, stream),
+                       "gen_sparse_indices");
+        }
+        for (int l = first; l > 0; l--)
+            lib->check(lib->topk_sparse(pa(y.pq[l]), pa(y.pk[l]), ints(y.sel[l]), ints(y.sel[l - 1]), b, h, static_cast<int>(n[l]), y.topk[l - 1],
+                                        y.topk[l], stream),
+                       "compute_topk_indices_sparse");
+
+        // The lists of the backward (the transposed selections of all levels).  Up to 2^14 tokens a (b,h)'s bitmap of
+        // (key block, query block) fits LDS and one launch of one workgroup per (b,h) and level does everything, sorted as
+        // it goes, behind the attention kernel on the same stream (on a second stream, beside the backward's dQ kernel, the
+        // two event edges cost more than the overlap saves: 0.373 against 0.358 ms a step at B=2, H=6, N=16384).  Beyond
+        // that the lists take several kernels per level, which run on a second stream beside the attention kernel: the
+        // attention kernel is issued first (the GPU is waiting for it), and an event recorded before it lets the second
+        // stream start as soon as the selection is done.  With few tokens over all heads the event calls cost more than the
+        // overlap saves: everything then goes to the one stream.
+        const bool beside = grad && lib->device && n[1] * n[1] > (int64_t(1) << 20) && B * H * N >= (int64_t(1) << 17);
+        const int dev = beside ? q.device().index() : 0;
+        if (beside) hip_check(hipEventRecord(side_events(dev).ready, static_cast<hipStream_t>(stream)));
+
+        llsa_attn_fwd_args f{};
+        f.qr = pa(y.qr); f.kr = pa(y.kr); f.vt = pa(y.vt); f.idx = ints(y.sel[0]);
+        f.o = o.data_ptr(); f.sob = o.stride(0); f.soh = o.stride(1); f.son = o.stride(2);
+        f.lse = static_cast<float*>(pa(y.lse));
+        f.B = b; f.H = h; f.N = static_cast<int32_t>(N); f.T = y.topk[0]; f.levels = L;
+        float w = 1.f;
+        for (int l = 1; l <= L; l++) {
+            llsa_fwd_level& lv = f.lvl[l - 1];
+            w *= 16.f;
+            lv.kr = pa(y.pkr[l]); lv.vt = pa(y.pvt[l]); lv.w = w;
+            if (l < L) {
+                lv.sel = ints(y.sel[l]);
+                lv.T = y.topk[l];
+            }
+        }
+        lib->check(lib->attn_fwd(&f, stream), "attn_fwd");
+
+        if (grad) {
+            llsa_transpose_job jobs[kL];
+            for (int l = 0; l < L; l++) {
+                const int32_t m = static_cast<int32_t>(n[l + 1]);
+                jobs[l] = llsa_transpose_job{ints(y.sel[l]), ints(y.off[l]), ints(y.flat[l]), l == 0 ? ints(y.work) : nullptr, l == 0 ? nullptr : ints(y.inv[l]),
+                                             m, m, y.topk[l], l == 0 ? y.chunk : 1};
+            }
+            void* lists = stream;
+            if (beside) {
+                lists = side_stream(dev);
+                hip_check(hipStreamWaitEvent(static_cast<hipStream_t>(lists), side_events(dev).ready, 0));       // (the arena is older than the selection, so this covers it too)
+            }
+            lib->check(lib->transpose_indices_multi(jobs, L, b, h, lists), "transpose_indices");
+            if (beside) {                                    // (and the arena is not handed out again before the second stream is done)
+                hip_check(hipEventRecord(side_events(dev).done, static_cast<hipStream_t>(lists)));
+                hip_check(hipStreamWaitEvent(static_cast<hipStream_t>(stream), side_events(dev).done, 0));
+            }
+            node = std::shared_ptr<LlsaBackward>(new LlsaBackward, torch::autograd::deleteNode);
+            node->lib = lib;
+            node->lay = y;
+            node->B = B; node->H = H; node->N = N;
+            for (int i = 0; i < 4; i++) {
+                node->sq[i] = q.stride(i);
+                node->sk[i] = k.stride(i);
+                node->sv[i] = v.stride(i);
+            }
+            node->eps = eps;
+            node->arena = arena;
+            node->freq = SavedVariable(freq, false);
+            if (gq.defined()) {                              // (q and k themselves are needed again only by the backward of the qk-norm)
+                node->has_gq = true;
+                node->type_gq = gq_in->scalar_type();
+                node->gq = SavedVariable(gq.is_same(*gq_in) ? *gq_in : gq, false);
+                node->q = SavedVariable(q.is_same(q_in) ? q_in : q, false);
+            }
+            if (gk.defined()) {
+                node->has_gk = true;
+                node->type_gk = gk_in->scalar_type();
+                node->gk = SavedVariable(gk.is_same(*gk_in) ? *gk_in : gk, false);
+                node->k = SavedVariable(k.is_same(k_in) ? k_in : k, false);
+            }
+        }
+    }
+    if (node) {
+        variable_list inputs{q_in, k_in, v_in};
+        if (node->has_gq) inputs.push_back(*gq_in);
+        if (node->has_gk) inputs.push_back(*gk_in);
+        node->set_next_edges(torch::autograd::collect_next_edges(inputs));
+        torch::autograd::set_history(o, node);
+        node->o = SavedVariable(o, true);
+    }
+    return o;
+}
+
+// The blocks the forward that produced `out` chose, finest first: int32 views of the arena its autograd node holds.
+std::vector<Tensor> selection(const Tensor& out) {
+    auto* node = dynamic_cast<LlsaBackward*>(out.grad_fn().get());
+    if (node == nullptr) fail(Failure::kValue, "not an output of a fused operator that records its backward");
+    if (node->released) fail(Failure::kRuntime, torch::autograd::ERR_BACKWARD_TWICE);
+    const Layout& y = *node->lay;
+    std::vector<Tensor> r;
+    for (int l = 0; l < y.L; l++) {
+        const int64_t count = node->B * node->H * y.n[l + 1] * y.topk[l];
+        r.push_back(node->arena.narrow(0, y.sel[l], 4 * count).view(at::kInt).view({node->B, node->H, y.n[l + 1], y.topk[l]}));
+    }
+    return r;
+}
+
+// ---------------------------------------------------------------------------------------
+// token permutation
+// ---------------------------------------------------------------------------------------
+Tensor gather(const Library& lib, const Tensor& x_in, const Tensor& index_in) {
+    if (x_in.dim() != 3) fail(Failure::kValue, "gather_tokens expects (B, N, C)");
+    lib.on_device(x_in);
+    lib.on_device(index_in);
+    at::AutoDispatchBelowADInplaceOrView below;
+    c10::OptionalDeviceGuard guard(lib.device ? std::optional<at::Device>(x_in.device()) : std::nullopt);
+    const int64_t B = x_in.size(0), N = x_in.size(1), C = x_in.size(2), es = x_in.element_size();
+    if (C * es % 16 != 0) fail(Failure::kNotImplemented, "rows of " + std::to_string(C * es) + " bytes: a multiple of 16 is needed");
+    const bool in_place = x_in.stride(2) == 1 && x_in.stride(1) == C && x_in.stride(0) * es % 16 == 0 && reinterpret_cast<uintptr_t>(x_in.data_ptr()) % 16 == 0;
+    const Tensor x = in_place ? x_in : x_in.contiguous();
+    const Tensor index = index_in.scalar_type() == at::kInt && index_in.is_contiguous() ? index_in : index_in.to(at::kInt).contiguous();
+    const int64_t n_out = index.numel();
+    Tensor y = at::empty({B, n_out, C}, x.options());
+    if (B == 0 || n_out == 0) return y;
+    lib.check(lib.gather_rows(x.data_ptr(), y.data_ptr(), static_cast<const int32_t*>(index.data_ptr()), static_cast<int>(B), static_cast<int>(n_out),
+                              static_cast<int>(N), static_cast<int>(C * es), x.stride(0) * es, y.stride(0) * es, lib.stream(x)),
+              "gather_tokens");
+    return y;
+}
+
+struct PermuteBackward : public Node {
+    std::shared_ptr<Library> lib;
+    SavedVariable inv;
+    std::string name() const override { return "PermuteTokensBackward"; }
+    void release_variables() override {
+        std::lock_guard<std::mutex> lock(mutex_);
+        inv.reset_data();
+        released = true;
+    }
+    bool released = false;
+    variable_list apply(variable_list&& grads) override {
+        std::lock_guard<std::mutex> lock(mutex_);
+        return in_engine([&]() -> variable_list {
+            if (released) fail(Failure::kRuntime, torch::autograd::ERR_BACKWARD_TWICE);
+            if (!grads[0].defined()) return {Tensor()};
+            return {gather(*lib, grads[0], inv.unpack())};
+        });
+    }
+};
+
+Tensor permute(const std::shared_ptr<Library>& lib, const Tensor& x, const Tensor& perm, const Tensor& inv) {
+    Tensor y = gather(*lib, x, perm);
+    if (at::GradMode::is_enabled() && x.requires_grad()) {
+        auto node = std::shared_ptr<PermuteBackward>(new PermuteBackward, torch::autograd::deleteNode);
+        node->lib = lib;
+        node->inv = SavedVariable(inv, false);
+        node->set_next_edges(torch::autograd::collect_next_edges(x));
+        torch::autograd::set_history(y, node);
+    }
+    return y;
+}
+
+}  // namespace
+
+PYBIND11_MODULE(_llsa_host, m) {
+    m.doc() = "host side of llsa_amd's fused operators";
+    py::class_<Library, std::shared_ptr<Library>>(m, "Library").def(py::init<const std::map<std::string, uintptr_t>&, bool>());
+    m.def("set_library_error", [](py::object type) { g_library_error = type.release().ptr(); });
+    m.attr("abi_version") = LLSA_ABI_VERSION;
+    m.def("attend", torch::wrap_pybind_function([](const std::shared_ptr<Library>& lib, const Tensor& q, const Tensor& k, const Tensor& v,
+                                                   const std::vector<int64_t>& topks, int64_t block_size, const std::optional<Tensor>& freq,
+                                                   const std::optional<Tensor>& gq, const std::optional<Tensor>& gk, double eps) {
+        return without_interpreter([&] { return attend(lib, q, k, v, topks, block_size, freq, gq, gk, eps); });
+    }));
+    m.def("selection", torch::wrap_pybind_function([](const Tensor& out) { return without_interpreter([&] { return selection(out); }); }));
+    m.def("gather", torch::wrap_pybind_function([](const std::shared_ptr<Library>& lib, const Tensor& x, const Tensor& index) {
+        return without_interpreter([&] { return gather(*lib, x, index); });
+    }));
+    m.def("permute", torch::wrap_pybind_function([](const std::shared_ptr<Library>& lib, const Tensor& x, const Tensor& perm, const Tensor& inv) {
+        return without_interpreter([&] { return permute(lib, x, perm, inv); });
+    }));
+}

@@ -19,7 +19,7 @@ import torch
 from torch.autograd import Function
 
 from ..hip.mean_pool import mean_pool1d
-from ._fused import LlsaFused
+from ._fused import attend
 from ..hip.sparse_attention_res_1 import sparse_indices_attn_res_fwd, sparse_indices_attn_res_scatter_bwd_v2
 from ..hip.topk import gen_sparse_indices
 
@@ -50,8 +50,7 @@ flash_sparse_residual_attention_l1_op = FlashSparseResidualAttentionL1.apply
 
 def llsa_l1(q, k, v, topk=8, block_size=16, rope=None, qk_norm=None):
     """flash_sparse_attention_res_1.py:41-47."""
-    gq, gk, eps = qk_norm if qk_norm is not None else (None, None, 0.0)
-    return LlsaFused.apply(q, k, v, (topk,), block_size, rope, gq, gk, eps)
+    return attend(q, k, v, (int(topk),), block_size, rope, qk_norm)
 
 
 def llsa_l1_unfused(q, k, v, topk=8, block_size=16):

@@ -10,7 +10,7 @@ import torch
 from torch.autograd import Function
 
 from ..hip.mean_pool import mean_pool1d
-from ._fused import LlsaFused
+from ._fused import attend
 from ..hip.sparse_attention_res_2 import (sparse_indices_attn_res_2_2_fwd,
                                           sparse_indices_attn_res_scatter_2_2_bwd_v2)
 from ..hip.topk import compute_topk_indices_sparse, gen_sparse_indices
@@ -48,8 +48,7 @@ flash_sparse_residual_attention_l2_op = FlashSparseResidualAttentionL2.apply
 
 def llsa_l2(q, k, v, topk1=8, topk2=8, block_size=16, rope=None, qk_norm=None):
     """flash_sparse_attention_res_2.py:48-59."""
-    gq, gk, eps = qk_norm if qk_norm is not None else (None, None, 0.0)
-    return LlsaFused.apply(q, k, v, (topk1, topk2), block_size, rope, gq, gk, eps)
+    return attend(q, k, v, (int(topk1), int(topk2)), block_size, rope, qk_norm)
 
 
 def llsa_lk(q, k, v, topks, block_size=16, rope=None, qk_norm=None):
@@ -60,8 +59,7 @@ def llsa_lk(q, k, v, topks, block_size=16, rope=None, qk_norm=None):
     level, parent-guided selection level by level down to the fine blocks, and every query reads topk1 fine blocks,
     16 topk_(l+1) tokens of pooled level l < k with weight 16^l, and all N/16^k tokens of level k with weight 16^k.
     N must be a multiple of 64 * 16^k."""
-    gq, gk, eps = qk_norm if qk_norm is not None else (None, None, 0.0)
-    return LlsaFused.apply(q, k, v, tuple(int(t) for t in topks), block_size, rope, gq, gk, eps)
+    return attend(q, k, v, tuple(int(t) for t in topks), block_size, rope, qk_norm)
 
 
 def llsa_l3(q, k, v, topk1=8, topk2=8, topk3=8, block_size=16, rope=None, qk_norm=None):
