@@ -181,24 +181,32 @@ __device__ __forceinline__ Key compare_again(Key t, int slot) { return t + (Key)
 template <int TPW, int W>
 __device__ __forceinline__ unsigned row_bound(const unsigned (&key)[4 * TPW], int tiles, int T, unsigned& top, RowShare<W>* sh, int& turn,
                                               int wave, int lane) {
-    constexpr int kFew = TPW < 4 ? TPW : 4;                   // groups per lane: kFew large ones, or one per tile
+    constexpr int kFew = TPW < 4 ? TPW : 4;                   // groups per lane: all its keys, kFew groups, or one per tile
     unsigned tile_max[TPW], few[kFew];
-    unsigned least = 0xFFFFFFFFu, least_few = 0xFFFFFFFFu;
-    top = 0;
 #pragma unroll
     for (int g = 0; g < kFew; g++) few[g] = 0;
 #pragma unroll
     for (int a = 0; a < TPW; a++) {
         tile_max[a] = max(max(key[4 * a], key[4 * a + 1]), max(key[4 * a + 2], key[4 * a + 3]));
-        least = min(least, tile_max[a]);
         few[a % kFew] = max(few[a % kFew], tile_max[a]);
     }
+    top = 0;
 #pragma unroll
-    for (int g = 0; g < kFew; g++) {
-        top = max(top, few[g]);
-        least_few = min(least_few, few[g]);
+    for (int g = 0; g < kFew; g++) top = max(top, few[g]);
+    unsigned lo = top;                                        // the fewer groups the closer the bound
+    if (T > 4 * W || tiles < W) {
+        lo = 0xFFFFFFFFu;
+        if (T <= 4 * W * kFew && tiles >= W * kFew) {
+#pragma unroll
+            for (int g = 0; g < kFew; g++) lo = min(lo, few[g]);
+        } else if (T <= 4 * W * TPW && tiles == W * TPW) {
+#pragma unroll
+            for (int a = 0; a < TPW; a++) lo = min(lo, tile_max[a]);
+        } else {                                              // the row's smallest key
+#pragma unroll
+            for (int i = 0; i < 4 * TPW; i++) lo = key[i] != 0u ? min(lo, key[i]) : lo;
+        }
     }
-    unsigned lo = (T <= 4 * W * kFew && tiles >= W * kFew) ? least_few : (T <= 4 * W * TPW && tiles == W * TPW) ? least : 0u;
     top = quad_max_u(top);
     lo = quad_min_u(lo);
     if (W > 1) {
