@@ -247,8 +247,9 @@ int llsa_transpose_indices_multi(const llsa_transpose_job* jobs, int n_jobs, int
 int64_t llsa_work_list_len(int Mb, int Kb, int T, int chunk);
 /* Entries per work item of the fine level for a sequence of N tokens: 64 up to N = 16384, where a step is short and a long
  * item would end it alone, 256 beyond, where fewer items and fewer partial sums count for more (N = 65536: -2 %,
- * N = 262144: -3 % of the step).  Never more than LLSA_CHUNK_FINE_MAX.  No counterpart in the reference, which walks a key
- * block's whole list in one program (sparse_attention_res_1.py:300-322). */
+ * N = 262144: -3 % of the step); 16 up to N = 1024 and 32 up to 2048, where the whole pass is a few hundred waves and lasts
+ * as long as its longest item (6 x 1024 tokens, topk 8: 18 -> 10 us).  Never more than LLSA_CHUNK_FINE_MAX.  No
+ * counterpart in the reference, which walks a key block's whole list in one program (sparse_attention_res_1.py:300-322). */
 int llsa_fine_chunk(int N);
 #define LLSA_CHUNK_FINE_MAX 256
 

@@ -1240,7 +1240,7 @@ extern "C" int llsa_attn_bwd(const llsa_attn_bwd_args* a, void* stream) {
 
     const int stages = a->stages ? a->stages : (0x7fffffff & ~LLSA_BWD_NO_REDUCE);
     if (stages & LLSA_BWD_DQ) {
-        if (a->T <= kPairMaxTopk && N1 % 8 == 0)
+        if (a->T <= kPairMaxTopk && N1 % 8 == 0 && (int64_t)N1 / 8 * BH >= kPairMinGroups)
             hipLaunchKernelGGL(attn_dq_pair_kernel, dim3(N1 / 8, BH), dim3(256), 0, s, *a, delta, dor);
         else
             hipLaunchKernelGGL(attn_dq_kernel, dim3((N1 + 3) / 4, BH), dim3(256), 0, s, *a, delta, dor);

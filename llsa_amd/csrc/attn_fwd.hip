@@ -438,7 +438,7 @@ extern "C" int llsa_attn_fwd(const llsa_attn_fwd_args* a, void* stream) {
     LLSA_REQUIRE(aligned16(a->qr) && aligned16(a->kr) && aligned16(a->vt) && aligned16(a->o), "attn_fwd: tensors must be 16-byte aligned");
     LLSA_REQUIRE((a->sob % 4 == 0) && (a->soh % 4 == 0) && (a->son % 4 == 0), "attn_fwd: rows of o must be 8-byte aligned");
     const int N1 = a->N / 16;
-    if (a->T <= kPairMaxTopk && N1 % 8 == 0)
+    if (a->T <= kPairMaxTopk && N1 % 8 == 0 && (int64_t)N1 / 8 * a->B * a->H >= kPairMinGroups)
         hipLaunchKernelGGL(attn_fwd_pair_kernel, dim3(N1 / 8, a->B * a->H), dim3(256), 0, (hipStream_t)stream, *a);
     else
         hipLaunchKernelGGL(attn_fwd_kernel, dim3((N1 + 3) / 4, a->B * a->H), dim3(256), 0, (hipStream_t)stream, *a);

@@ -144,7 +144,7 @@ __device__ __forceinline__ bf16x4 rope_bwd4(bf16x4 o, bf16x4 f) {
 // ints at the end of a (b,h)'s work list (see transpose.hip) that the transpose of many entries uses as
 // histogram, then as cursors
 __host__ __device__ inline int work_tail_len(int Kb) { return (Kb + 3) & ~3; }
-__host__ __device__ inline int fine_chunk(int N) { return N > 16384 ? 256 : 64; }      // llsa_fine_chunk
+__host__ __device__ inline int fine_chunk(int N) { return N > 16384 ? 256 : N > 2048 ? 64 : N > 1024 ? 32 : 16; }      // llsa_fine_chunk
 
 constexpr int kGroup = 4;      // pooled blocks per LDS buffer in the query-side attention kernels (one per wave)
 
@@ -216,6 +216,9 @@ __device__ __forceinline__ SharedBlock shared_block(const SharedList& sl, const 
 // entries), indices clamped to [0, N1).  n_both is even (an odd common block out is listed once for each row).
 // A row that names a block twice shares nothing (n_both = 0).  `scratch`: kWave ints of LDS private to the wave.
 constexpr int kPairMaxTopk = 32;
+// Fewer groups of eight query blocks than CUs: one query block per wave then.  The chip has room for all of the waves either
+// way, and a wave of one block has half the serial chain (6 x 1024 tokens, topk 8: forward 8.7 -> 5.9 us, dQ 14.0 -> 8.5).
+constexpr int kPairMinGroups = 256;
 struct PairOrder {
     int mine;
     int n_both;
