@@ -638,11 +638,12 @@ __global__ __launch_bounds__(64 * kDenseWaves) void attn_kside_dense_kernel(KSid
     const int N1 = p.N / kBlk;
     // Workgroups that stream the same piece of the query range (one per group of units) get neighbouring logical ids,
     // which xcd_logical_id keeps on one XCD: the piece then comes out of that XCD's L2 for all but the first of them.
-    const int unit_groups = p.n_units / (kDenseWaves * UPW);
+    const int unit_groups = (p.n_units + kDenseWaves * UPW - 1) / (kDenseWaves * UPW);
     const int lid = xcd_logical_id();                          // grid: (unit_groups * chunks, BH)
     const int piece = (lid % (int)gridDim.x) / unit_groups;
     const int bh = lid / (int)gridDim.x;
-    const int unit0 = (((lid % (int)gridDim.x) % unit_groups) * kDenseWaves + wave) * UPW;   // + UPW <= n_units (the plan sees to it)
+    const int unit0 = (((lid % (int)gridDim.x) % unit_groups) * kDenseWaves + wave) * UPW;
+    const bool active = unit0 < p.n_units;                    // (n_units is a multiple of UPW; a wave past the end only moves tiles)
     const int start = piece * p.chunk_len;
     const int n_pairs = min(p.chunk_len, N1 - start) / 2;     // even: chunk_len and N1 are multiples of 4
     if (n_pairs <= 0) return;                                 // uniform over the workgroup
@@ -678,8 +679,9 @@ __global__ __launch_bounds__(64 * kDenseWaves) void attn_kside_dense_kernel(KSid
     bf16x8 bk[UPW][2], bv[UPW][2];
 #pragma unroll
     for (int j = 0; j < UPW; j++) {
-        const bf16* kp = p.kk + ((int64_t)bh * p.n_units + unit0 + j) * kTile + lane * 8;
-        const bf16* vp = p.vv + ((int64_t)bh * p.n_units + unit0 + j) * kTile + lane * 8;
+        const int unit = min(unit0 + j, p.n_units - 1);
+        const bf16* kp = p.kk + ((int64_t)bh * p.n_units + unit) * kTile + lane * 8;
+        const bf16* vp = p.vv + ((int64_t)bh * p.n_units + unit) * kTile + lane * 8;
         bk[j][0] = ld16(kp);
         bk[j][1] = ld16(kp + 512);
         bv[j][0] = ld16(vp);
@@ -720,6 +722,7 @@ __global__ __launch_bounds__(64 * kDenseWaves) void attn_kside_dense_kernel(KSid
         }
         deposit(t + 1, nxt);
         request(t + 3, nxt);
+        if (!active) return;
         float nl[2][4];
 #pragma unroll
         for (int u = 0; u < 2; u++)
@@ -755,6 +758,7 @@ __global__ __launch_bounds__(64 * kDenseWaves) void attn_kside_dense_kernel(KSid
         round(t, s1);
         round(t + 1, s0);
     }
+    if (!active) return;
 #pragma unroll
     for (int j = 0; j < UPW; j++) {
         f32x4* ps = part_slot(p.part, ((int64_t)piece * gridDim.y + bh) * p.n_units + unit0 + j);
@@ -1125,13 +1129,16 @@ static DensePlan dense_plan(int B, int H, int N, int levels) {
     const int n_units = d.n_tok / 16;
     // Q and dO are streamed n_units / (4 * upw) times (mostly out of an L2: see the kernel); four units per wave would
     // halve that again but leave one wave per SIMD, which measured slower (1.07 ms against 0.93 ms at N = 262144)
-    d.upw = (n_units % 8 == 0 && n_units >= 16) ? 2 : 1;
-    const int groups = max(1, n_units / (kDenseWaves * d.upw)) * B * H;   // workgroups per piece of the query range
+    d.upw = n_units >= 16 ? 2 : 1;
+    const int groups = (n_units + kDenseWaves * d.upw - 1) / (kDenseWaves * d.upw) * B * H;   // workgroups per piece of the query range
     // The query range is cut so that the workgroups fill the chip's resident slots (256 CUs x the workgroups the
-    // registers allow per CU) a whole number of times, three if there is that much work: a count just above a
-    // multiple of the slots leaves a last round in which a few workgroups run alone.
+    // registers allow per CU) a whole number of times: a count just above a multiple of the slots leaves a last round in
+    // which a few workgroups run alone.  Three times where the pieces are long even so, which evens out their progress
+    // (N = 262144: 862 us against 920 for once); once where they are short, for a third of the partial sums (N = 7168, 15
+    // heads: the reduction 13.6 -> 7.6 us, the pass itself the same).
     const int slots = 256 * (d.upw == 2 ? 2 : 3);
-    int chunks = 3 * slots / groups;
+    int chunks = slots / groups;
+    if (chunks < 1 || N1 / chunks > 256) chunks = 3 * slots / groups;
     if (chunks > N1 / 16) chunks = N1 / 16;
     if (chunks < 1) chunks = 1;
     int len = (N1 + chunks - 1) / chunks;
@@ -1357,7 +1364,7 @@ extern "C" int llsa_attn_bwd(const llsa_attn_bwd_args* a, void* stream) {
             rp.job[rp.n_jobs - 1].half_part = 1;
             return;
         }
-        const dim3 grid(p.n_units / (kDenseWaves * d.upw) * d.chunks, BH), block(64 * kDenseWaves);
+        const dim3 grid((p.n_units + kDenseWaves * d.upw - 1) / (kDenseWaves * d.upw) * d.chunks, BH), block(64 * kDenseWaves);
         if (d.upw == 2) hipLaunchKernelGGL(HIP_KERNEL_NAME(attn_kside_dense_kernel<2>), grid, block, 0, s, p);
         else hipLaunchKernelGGL(HIP_KERNEL_NAME(attn_kside_dense_kernel<1>), grid, block, 0, s, p);
         add_job(p, 1, p.n_units, d.chunks);
