@@ -230,13 +230,14 @@ __global__ __launch_bounds__(256) void attn_dq_kernel(llsa_attn_bwd_args a, floa
     dq_end(sd, a, b, h, g, lane);
 }
 
-// Two sibling query blocks per wave (topk <= kPairMaxTopk): the pooled blocks and the fine blocks both rows
+// Two sibling query blocks per wave (topk <= 32 R <= kPairMaxTopk): the pooled blocks and the fine blocks both rows
 // selected are read once -- from memory and, what weighs more here, from LDS, where every key block is read
 // three times (K rows, V rows, K transposed) -- and multiplied twice.  See pair_order for the walk.
+template <int R>
 __global__ __launch_bounds__(256, 3) void attn_dq_pair_kernel(llsa_attn_bwd_args a, float* __restrict__ delta,
                                                               bf16* __restrict__ dor) {
     __shared__ __align__(16) bf16 sh[2][kGroup][2 * kTile];
-    __shared__ int order[4][kWave];
+    __shared__ int order[4][R * kWave];
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int N1 = a.N / kBlk, T = a.T;
@@ -262,8 +263,7 @@ __global__ __launch_bounds__(256, 3) void attn_dq_pair_kernel(llsa_attn_bwd_args
         copy16_global_to_lds(vb + 512 + lane * 8, dst + kTile + 512);
     };
     issue_group(0);
-    const PairOrder po = pair_order(ip, T, N1, lane, order[wave]);
-    const int mine = po.mine;
+    const PairOrder<R> po = pair_order<R>(ip, T, N1, lane, order[wave]);
     const int steps_both = po.n_both / 2, steps_only = (T - po.n_both) / 2, n_steps = steps_both + 2 * steps_only;
 
     DqSide sd[2];
@@ -302,7 +302,7 @@ __global__ __launch_bounds__(256, 3) void attn_dq_pair_kernel(llsa_attn_bwd_args
         bf16* slot = priv + (t & 1) * (2 * kTile);
 #pragma unroll
         for (int j = 0; j < 2; j++) {
-            const int blk = __builtin_amdgcn_readlane(mine, 2 * t + j);
+            const int blk = po.entry(2 * t + j);
             const bf16* kb = kr + (int64_t)blk * kTile;
             const bf16* vb = vr + (int64_t)blk * kTile;
             copy16_global_to_lds(kb + lane * 8, slot + j * kTile);
@@ -1248,7 +1248,8 @@ extern "C" int llsa_attn_bwd(const llsa_attn_bwd_args* a, void* stream) {
     const int stages = a->stages ? a->stages : (0x7fffffff & ~LLSA_BWD_NO_REDUCE);
     if (stages & LLSA_BWD_DQ) {
         if (a->T <= kPairMaxTopk && N1 % 8 == 0 && (int64_t)N1 / 8 * BH >= kPairMinGroups)
-            hipLaunchKernelGGL(attn_dq_pair_kernel, dim3(N1 / 8, BH), dim3(256), 0, s, *a, delta, dor);
+            if (a->T <= 32) hipLaunchKernelGGL(HIP_KERNEL_NAME(attn_dq_pair_kernel<1>), dim3(N1 / 8, BH), dim3(256), 0, s, *a, delta, dor);
+            else hipLaunchKernelGGL(HIP_KERNEL_NAME(attn_dq_pair_kernel<2>), dim3(N1 / 8, BH), dim3(256), 0, s, *a, delta, dor);
         else
             hipLaunchKernelGGL(attn_dq_kernel, dim3((N1 + 3) / 4, BH), dim3(256), 0, s, *a, delta, dor);
     }

@@ -298,7 +298,7 @@ __global__ __launch_bounds__(256, 4) void attn_fwd_kernel(llsa_attn_fwd_args a) 
 }
 
 // ---------------------------------------------------------------------------------------
-// Two sibling query blocks per wave (topk <= 32).  Both walk the same pooled blocks, and on coherent inputs most
+// Two sibling query blocks per wave (topk <= 32 R, R = 1 or 2).  Both walk the same pooled blocks, and on coherent inputs most
 // of their fine blocks coincide, so every operand tile that both need is fetched once and multiplied twice: the
 // wave first sorts the two fine lists into [blocks both selected | only the first | only the second] and walks
 // that list in steps of NB blocks, a step of the first part feeding both soft-max states.  What bounds these
@@ -306,10 +306,11 @@ __global__ __launch_bounds__(256, 4) void attn_fwd_kernel(llsa_attn_fwd_args a) 
 // A row that names a block twice keeps the plain walk (nothing is shared).
 // ---------------------------------------------------------------------------------------
 
+template <int R>
 __global__ __launch_bounds__(256, 3) void attn_fwd_pair_kernel(llsa_attn_fwd_args a) {
     static_assert(NB == 2 && kGroup == 4, "the shared phase reads an LDS buffer of four blocks as two steps of two");
     __shared__ __align__(16) bf16 sh[2][kGroup][2 * kTile];
-    __shared__ int order[4][kWave];
+    __shared__ int order[4][R * kWave];
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int N1 = a.N / kBlk, T = a.T;
@@ -337,8 +338,7 @@ __global__ __launch_bounds__(256, 3) void attn_fwd_pair_kernel(llsa_attn_fwd_arg
     issue_group(0);
 
     // ---- the two fine lists, sorted into [both | only the first | only the second]; entry i ends in lane i
-    const PairOrder po = pair_order(ip, T, N1, lane, order[wave]);
-    const int mine = po.mine;
+    const PairOrder<R> po = pair_order<R>(ip, T, N1, lane, order[wave]);
     const int steps_both = po.n_both / NB, steps_only = (T - po.n_both) / NB, n_steps = steps_both + 2 * steps_only;
 
     bf16x8 bq[2][2];
@@ -380,7 +380,7 @@ __global__ __launch_bounds__(256, 3) void attn_fwd_pair_kernel(llsa_attn_fwd_arg
     auto describe = [=](int t, StepDesc& d) __attribute__((always_inline)) {
 #pragma unroll
         for (int j = 0; j < NB; j++) {
-            const int blk = __builtin_amdgcn_readlane(mine, NB * t + j);
+            const int blk = po.entry(NB * t + j);
             d.kb[j] = kr + (int64_t)blk * kTile;
             d.vtb[j] = vt + (int64_t)blk * kTile;
         }
@@ -439,7 +439,10 @@ extern "C" int llsa_attn_fwd(const llsa_attn_fwd_args* a, void* stream) {
     LLSA_REQUIRE((a->sob % 4 == 0) && (a->soh % 4 == 0) && (a->son % 4 == 0), "attn_fwd: rows of o must be 8-byte aligned");
     const int N1 = a->N / 16;
     if (a->T <= kPairMaxTopk && N1 % 8 == 0 && (int64_t)N1 / 8 * a->B * a->H >= kPairMinGroups)
-        hipLaunchKernelGGL(attn_fwd_pair_kernel, dim3(N1 / 8, a->B * a->H), dim3(256), 0, (hipStream_t)stream, *a);
+        if (a->T <= 32)
+            hipLaunchKernelGGL(HIP_KERNEL_NAME(attn_fwd_pair_kernel<1>), dim3(N1 / 8, a->B * a->H), dim3(256), 0, (hipStream_t)stream, *a);
+        else
+            hipLaunchKernelGGL(HIP_KERNEL_NAME(attn_fwd_pair_kernel<2>), dim3(N1 / 8, a->B * a->H), dim3(256), 0, (hipStream_t)stream, *a);
     else
         hipLaunchKernelGGL(attn_fwd_kernel, dim3((N1 + 3) / 4, a->B * a->H), dim3(256), 0, (hipStream_t)stream, *a);
     return launch_status("attn_fwd");

@@ -211,19 +211,28 @@ __device__ __forceinline__ SharedBlock shared_block(const SharedList& sl, const 
     return sb;
 }
 
-// The fine lists of two sibling query blocks (rows ip[0..T) and ip[T..2T), T <= kPairMaxTopk), sorted into
-// [blocks both rows name | only the first | only the second]: entry i of that order ends in lane i (2T - n_both
-// entries), indices clamped to [0, N1).  n_both is even (an odd common block out is listed once for each row).
-// A row that names a block twice shares nothing (n_both = 0).  `scratch`: kWave ints of LDS private to the wave.
-constexpr int kPairMaxTopk = 32;
-// Fewer groups of eight query blocks than CUs: one query block per wave then.  The chip has room for all of the waves either
-// way, and a wave of one block has half the serial chain (6 x 1024 tokens, topk 8: forward 8.7 -> 5.9 us, dQ 14.0 -> 8.5).
-constexpr int kPairMinGroups = 256;
+// The fine lists of two sibling query blocks (rows ip[0..T) and ip[T..2T), T <= 32 R), sorted into
+// [blocks both rows name | only the first | only the second]: entry i of that order ends in lane i % 64 of register i / 64
+// (2T - n_both entries), indices clamped to [0, N1).  n_both is even (an odd common block out is listed once for each row).
+// A row that names a block twice shares nothing (n_both = 0).  `scratch`: R * kWave ints of LDS private to the wave.
+constexpr int kPairMaxTopk = 64;
+// Fewer groups of eight query blocks than this: one query block per wave.  The chip then has room for all of the waves either way
+// (four workgroups of four single blocks or three of four pairs per CU), and a wave of one block has half the serial chain:
+// 6 x 1024 tokens, topk 8: forward 8.7 -> 5.9 us, dQ 14.0 -> 8.5; 6 x 8192, topk 16: step 147 -> 138 us; even at 8 x 8192.
+constexpr int kPairMinGroups = 512;
+template <int R>
 struct PairOrder {
-    int mine;
+    int mine[R];
     int n_both;
+    __device__ __forceinline__ int entry(int i) const {       // i is wave-uniform
+        const int v = __builtin_amdgcn_readlane(mine[0], i & (kWave - 1));
+        if (R == 1) return v;
+        const int o = __builtin_amdgcn_readlane(mine[R - 1], i & (kWave - 1));
+        return i < kWave ? v : o;
+    }
 };
-__device__ __forceinline__ PairOrder pair_order(const int* ip, int T, int N1, int lane, int* scratch) {
+template <int R>
+__device__ __forceinline__ PairOrder<R> pair_order(const int* ip, int T, int N1, int lane, int* scratch) {
     const int first = (lane < T) ? clampi(ip[lane], 0, N1 - 1) : -1 - lane;       // (distinct negative fillers)
     const int second = (lane < T) ? clampi(ip[T + lane], 0, N1 - 1) : -65 - lane;
     bool in_second = false, in_first = false, twice = false;
@@ -250,8 +259,9 @@ __device__ __forceinline__ PairOrder pair_order(const int* ip, int T, int N1, in
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
     __builtin_amdgcn_wave_barrier();
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-    PairOrder po;
-    po.mine = scratch[lane];
+    PairOrder<R> po;
+#pragma unroll
+    for (int k = 0; k < R; k++) po.mine[k] = scratch[k * kWave + lane];
     po.n_both = n_both;
     return po;
 }
