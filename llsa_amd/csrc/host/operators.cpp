@@ -98,6 +98,7 @@ struct Library {
     decltype(&llsa_topk_cascade_max_parents) topk_cascade_max_parents;
     decltype(&llsa_attn_fwd) attn_fwd;
     decltype(&llsa_transpose_indices_multi) transpose_indices_multi;
+    decltype(&llsa_transpose_one_launch) transpose_one_launch;
     decltype(&llsa_work_list_len) work_list_len;
     decltype(&llsa_fine_chunk) fine_chunk;
     decltype(&llsa_attn_bwd_workspace_bytes) attn_bwd_workspace_bytes;
@@ -117,6 +118,7 @@ struct Library {
         get("llsa_topk_cascade_max_parents", topk_cascade_max_parents);
         get("llsa_attn_fwd", attn_fwd);
         get("llsa_transpose_indices_multi", transpose_indices_multi);
+        get("llsa_transpose_one_launch", transpose_one_launch);
         get("llsa_work_list_len", work_list_len);
         get("llsa_fine_chunk", fine_chunk);
         get("llsa_attn_bwd_workspace_bytes", attn_bwd_workspace_bytes);
@@ -457,15 +459,13 @@ Tensor attend(const std::shared_ptr<Library>& lib, const Tensor& q_in, const Ten
                                         y.topk[l], stream),
                        "compute_topk_indices_sparse");
 
-        // The lists of the backward (the transposed selections of all levels).  Up to 2^14 tokens a (b,h)'s bitmap of
-        // (key block, query block) fits LDS and one launch of one workgroup per (b,h) and level does everything, sorted as
-        // it goes, behind the attention kernel on the same stream (on a second stream, beside the backward's dQ kernel, the
-        // two event edges cost more than the overlap saves: 0.373 against 0.358 ms a step at B=2, H=6, N=16384).  Beyond
-        // that the lists take several kernels per level, which run on a second stream beside the attention kernel: the
-        // attention kernel is issued first (the GPU is waiting for it), and an event recorded before it lets the second
-        // stream start as soon as the selection is done.  With few tokens over all heads the event calls cost more than the
-        // overlap saves: everything then goes to the one stream.
-        const bool beside = grad && lib->device && n[1] * n[1] > (int64_t(1) << 20) && B * H * N >= (int64_t(1) << 17);
+        // The lists of the backward (the transposed selections of all levels).  Where one launch makes them all they follow
+        // the attention kernel on the same stream; the several kernels per level of the longest sequences run on a second
+        // stream beside the attention kernel: the attention kernel is issued first (the GPU is waiting for it), and an
+        // event recorded before it lets the second stream start as soon as the selection is done.  With few tokens over all
+        // heads the event calls cost more than the overlap saves: everything then goes to the one stream.
+        const bool beside = grad && lib->device && B * H * N >= (int64_t(1) << 17) &&
+                            !lib->transpose_one_launch(static_cast<int>(n[1]), static_cast<int>(n[1]), y.topk[0], b, h);
         const int dev = beside ? q.device().index() : 0;
         if (beside) hip_check(hipEventRecord(side_events(dev).ready, static_cast<hipStream_t>(stream)));
 

@@ -65,15 +65,22 @@ __device__ __forceinline__ int offsets_and_work_list(CountFn count_of, StartFn s
     }
     __syncthreads();
     int run = incl - local, run_i = incl_i - l_items, run_s = incl_s - l_slots, run_m = incl_m - l_multi, run_l = incl_l - l_long;
-    int total_long = 0;
+    // (five LDS reads in flight together; the sums over the waves go by readlane)
+    int total_long = 0, tot[5];
+#pragma unroll
+    for (int k = 0; k < 5; k++) tot[k] = wave_tot[k * kTrWaves + (lane & (kTrWaves - 1))];
+#pragma unroll
     for (int w = 0; w < kTrWaves; w++) {
-        total_long += wave_tot[4 * kTrWaves + w];
-        if (w < wave) {
-            run += wave_tot[w];
-            run_i += wave_tot[kTrWaves + w];
-            run_s += wave_tot[2 * kTrWaves + w];
-            run_m += wave_tot[3 * kTrWaves + w];
-            run_l += wave_tot[4 * kTrWaves + w];
+        int o[5];
+#pragma unroll
+        for (int k = 0; k < 5; k++) o[k] = __builtin_amdgcn_readlane(tot[k], w);
+        total_long += o[4];
+        if (w < wave) {                                       // (uniform)
+            run += o[0];
+            run_i += o[1];
+            run_s += o[2];
+            run_m += o[3];
+            run_l += o[4];
         }
     }
     run_i += total_long;                                      // short items follow the long ones
@@ -194,97 +201,132 @@ __global__ __launch_bounds__(kTrThreads) void transpose_indices_kernel(const int
     // pos[n] is now the END of segment n; the segments are sorted by sort_segments_kernel
 }
 
-// The whole transpose of a small job in one workgroup and one pass, sorted as it is built: the workgroup keeps one
-// bitmap over the query blocks per key block in LDS (Kb rows of Mb bits; one word of padding per row keeps the rows
-// off each other's banks), every entry sets its bit, a key block's count is the population of its row, and its
-// segment is written by reading the row's bits back in order -- ascending query blocks with no scatter through
-// atomic cursors and no sorting pass afterwards; the inverse position of an entry is its segment's start plus the
-// bits below its own.  Several jobs (the selections of all levels of one operator call) share a launch:
-// blockIdx.y picks the job.  A job fits when its bitmaps do (tr_bitmap_lds_ints); bigger ones take the kernels above.
-// Writing the segments is the long phase (4-byte stores, every lane into a line of its own, which one CU's memory
-// pipeline takes a lane at a time): a job with many key blocks is given `parts` workgroups per (b,h), each of which
-// builds the same bitmaps, counts and starts for itself (cheap, and no word has to pass between workgroups) and writes
-// the segments of its share of the key blocks; the first of them also writes offsets and work list.
+// The transpose of all levels of one operator call in one launch, sorted as it is built.  A workgroup owns a range of key
+// blocks of one (b,h): it reads all entries, keeps one bitmap over the query blocks per key block of its range in LDS (one
+// word of padding per row keeps the rows off each other's banks), and counts the entries below its range -- which is
+// where its first segment starts, so that no word passes between workgroups.  A key block's count is the population of
+// its row, its segment is written by reading the row's bits back in order -- ascending query blocks with no scatter through
+// atomic cursors and no sorting pass afterwards; the inverse position of an entry is its segment's start plus the bits below
+// its own.  One more workgroup per (b,h) makes a histogram over all key blocks and from it offsets and work list.
+// Reading every entry once per range is cheap (4 a lane and load, from the L2), clearing and filling the bitmaps of
+// the whole matrix in every workgroup was not (two levels of 12 x 16384 tokens 15.9 us), and a range fits LDS where the
+// matrix does not.
 struct TrJob {
     const int* idx; int* offsets; int* flat; int* work; int* inv;
-    int Mb, Kb, T, chunk, work_stride, parts;
+    int Mb, Kb, T, chunk, work_stride;
+    int parts, rows;                                          // ranges per (b,h), key blocks per range
+    unsigned row_magic;                                       // entry i (of four, if `quads`) belongs to query block i * row_magic >> 32
+    int quads;                                                // T is a multiple of 4 and idx 16-byte aligned: entries are read four at a time
 };
 struct TrJobs {
     TrJob job[LLSA_MAX_LEVELS];
-    int max_parts;                                            // workgroups per (b,h) in the grid; job i uses the first job[i].parts
+    int n_jobs, wgs;                                          // workgroups per (b,h): job[i].parts + 1 for each job, one after the other
 };
-__host__ __device__ inline int64_t tr_bitmap_lds_ints(int Mb, int Kb) { return (int64_t)Kb * ((Mb + 31) / 32 + 1) + 5 * kTrWaves; }
-constexpr int64_t kTrBitmapMaxInts = 36 * 1024;               // 144 KB
+__host__ __device__ inline int tr_stride(int Mb) { return (Mb + 31) / 32 + 1; }
+
+// calls fn(key block, query block) for every entry of the (b,h), each in one thread
+template <typename Fn>
+__device__ __forceinline__ void tr_entries(const TrJob& jb, const int* __restrict__ idx, Fn fn) {
+    const int tid = threadIdx.x, n = jb.quads ? jb.Mb * jb.T / 4 : jb.Mb * jb.T;
+    constexpr int kBatch = 8;
+    auto query = [&](int i) { return jb.row_magic == 0 ? i : (int)(((unsigned long long)(unsigned)i * jb.row_magic) >> 32); };
+    if (jb.quads) {
+        for (int i0 = 0; i0 < n; i0 += kBatch * kTrThreads) {     // eight loads in flight per thread
+            i32x4 v[kBatch];
+#pragma unroll
+            for (int k = 0; k < kBatch; k++) v[k] = reinterpret_cast<const i32x4*>(idx)[min(i0 + k * kTrThreads + tid, n - 1)];
+#pragma unroll
+            for (int k = 0; k < kBatch; k++) {
+                const int i = i0 + k * kTrThreads + tid;
+                if (i < n) {
+                    const int q = query(i);
+#pragma unroll
+                    for (int e = 0; e < 4; e++) fn(clampi(v[k][e], 0, jb.Kb - 1), q, 4 * i + e);
+                }
+            }
+        }
+    } else {
+        for (int i = tid; i < n; i += kTrThreads) fn(clampi(idx[i], 0, jb.Kb - 1), query(i), i);
+    }
+}
 
 __global__ __launch_bounds__(kTrThreads) void transpose_bitmap_kernel(TrJobs jobs) {
     HIP_DYNAMIC_SHARED(int, smem)
-    const TrJob& jb = jobs.job[blockIdx.y];
-    const int part = blockIdx.x % jobs.max_parts, bh = blockIdx.x / jobs.max_parts;
-    if (part >= jb.parts) return;
-    const int Mb = jb.Mb, Kb = jb.Kb, T = jb.T;
-    const int words = (Mb + 31) / 32, stride = words + 1;
-    unsigned* bm = reinterpret_cast<unsigned*>(smem);         // [Kb][stride]
-    int* wave_tot = smem + Kb * stride;                       // 5 * kTrWaves
-    const int tid = threadIdx.x;
-    const int E = Mb * T;
+    __shared__ int wave_tot[5 * kTrWaves];
+    const int bh = blockIdx.x / jobs.wgs;
+    int part = blockIdx.x % jobs.wgs, ji = 0;
+    while (ji < jobs.n_jobs - 1 && part > jobs.job[ji].parts) part -= jobs.job[ji++].parts + 1;
+    const TrJob& jb = jobs.job[ji];
+    const int Mb = jb.Mb, Kb = jb.Kb, T = jb.T, E = Mb * T;
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int* idx = jb.idx + (int64_t)bh * E;
-    int* flat = jb.flat + (int64_t)bh * E;
-    int* offsets = jb.offsets + (int64_t)bh * (Kb + 1);
-    int* work = jb.work ? jb.work + (int64_t)bh * jb.work_stride : nullptr;
 
-    for (int i = tid; i < Kb * stride; i += kTrThreads) bm[i] = 0u;
+    if (part == jb.parts) {                                   // offsets and work list
+        for (int i = tid; i < Kb; i += kTrThreads) smem[i] = 0;
+        __syncthreads();
+        tr_entries(jb, idx, [&](int n, int, int) { atomicAdd(&smem[n], 1); });
+        __syncthreads();
+        offsets_and_work_list([&](int i) { return smem[i]; }, [](int, int) {}, wave_tot, jb.offsets + (int64_t)bh * (Kb + 1),
+                              jb.work ? jb.work + (int64_t)bh * jb.work_stride : nullptr, Kb, E, E, jb.chunk);
+        return;
+    }
+
+    const int words = (Mb + 31) / 32, stride = words + 1;
+    const int lo = part * jb.rows, nr = min(jb.rows, Kb - lo);       // > 0: the host leaves no range empty
+    unsigned* bm = reinterpret_cast<unsigned*>(smem);         // [nr][stride]
+    for (int i = tid; i < nr * stride; i += kTrThreads) bm[i] = 0u;
     __syncthreads();
-    constexpr int kBatch = 16;
-    for (int e0 = 0; e0 < E; e0 += kBatch * kTrThreads) {     // 16 loads in flight per thread
-        int v[kBatch];
-#pragma unroll
-        for (int k = 0; k < kBatch; k++) {
-            const int e = e0 + k * kTrThreads + tid;
-            v[k] = (e < E) ? idx[e] : -1;
+    int below = 0;
+    tr_entries(jb, idx, [&](int n, int q, int) {
+        const int r = n - lo;
+        below += r < 0 ? 1 : 0;
+        if ((unsigned)r < (unsigned)nr) {
+            atomicOr(&bm[r * stride + (q >> 5)], 1u << (q & 31));
+            atomicAdd(&bm[r * stride + words], 1u);           // the row's count, in its padding word
         }
+    });
+    below = wave_incl_scan(below, lane);
+    if (lane == kWave - 1) wave_tot[wave] = below;
+    __syncthreads();
+    int start = 0, tot = wave_tot[lane & (kTrWaves - 1)];     // (one LDS read; the sums over the waves go by readlane)
 #pragma unroll
-        for (int k = 0; k < kBatch; k++) {
-            const int e = e0 + k * kTrThreads + tid;
-            if (e < E) {
-                const int q = e / T;
-                atomicOr(&bm[clampi(v[k], 0, Kb - 1) * stride + (q >> 5)], 1u << (q & 31));
-            }
+    for (int w = 0; w < kTrWaves; w++) start += __builtin_amdgcn_readlane(tot, w);
+    {   // the rows' starts take the place of the counts (a range has at most kTrThreads rows)
+        const int c = tid < nr ? (int)bm[tid * stride + words] : 0;
+        const int incl = wave_incl_scan(c, lane);
+        if (lane == kWave - 1) wave_tot[kTrWaves + wave] = incl;
+        __syncthreads();
+        tot = wave_tot[kTrWaves + (lane & (kTrWaves - 1))];
+#pragma unroll
+        for (int w = 0; w < kTrWaves; w++) {
+            const int o = __builtin_amdgcn_readlane(tot, w);
+            start += w < wave ? o : 0;
         }
+        if (tid < nr) bm[tid * stride + words] = (unsigned)(start + incl - c);
     }
     __syncthreads();
-    // counts -> the padding word of each row; the scan then leaves the segment's start there
-    for (int n = tid; n < Kb; n += kTrThreads) {
-        int c = 0;
-        for (int w = 0; w < words; w++) c += __popc(bm[n * stride + w]);
-        bm[n * stride + words] = (unsigned)c;
-    }
-    __syncthreads();
-    offsets_and_work_list([&](int i) { return (int)bm[i * stride + words]; },
-                          [&](int i, int st) { bm[i * stride + words] = (unsigned)st; },      // the count gives way to the start
-                          wave_tot, offsets, work, Kb, E, E, jb.chunk, part == 0);
-    __syncthreads();                                          // (every row's start is in place)
     if (jb.inv != nullptr) {
         int* inv = jb.inv + (int64_t)bh * E;
-        for (int e = part * kTrThreads + tid; e < E; e += jb.parts * kTrThreads) {
-            const int q = e / T, n = clampi(idx[e], 0, Kb - 1);
-            const unsigned* row = bm + n * stride;
+        tr_entries(jb, idx, [&](int n, int q, int e) {
+            const int r = n - lo;
+            if ((unsigned)r >= (unsigned)nr) return;
+            const unsigned* row = bm + r * stride;
             int pos = (int)row[words];
             for (int w = 0; w < (q >> 5); w++) pos += __popc(row[w]);
-            pos += __popc(row[q >> 5] & ((1u << (q & 31)) - 1u));
-            inv[e] = pos;
-        }
+            inv[e] = pos + __popc(row[q >> 5] & ((1u << (q & 31)) - 1u));
+        });
     }
-    // The segments, ascending.  Eight neighbouring lanes share a key block's row, each with an eighth of its words: the lanes
-    // count their bits, a scan over the eight gives each its place in the segment, and each writes the query blocks of its
-    // own words.  (One lane per row made a wave walk as many rounds as its longest segment has entries, every round a 4-byte
-    // store per lane into a line of its own; this way a round writes eight segments, and a row of 16 entries takes 2 or 3.)
-    const int rows = (Kb + jb.parts - 1) / jb.parts, r1 = min(Kb, (part + 1) * rows);
+    // The segments, ascending.  Eight neighbouring lanes share a row, each with an eighth of its words: the lanes count their
+    // bits, a scan over the eight gives each its place in the segment, and each writes the query blocks of its own words.
+    // (Stores of 4 bytes, every lane into a line of its own: with one lane per row a wave walked as many rounds as its longest
+    // segment has entries.)
     const int sub = tid & 7, wps = (words + 7) / 8, w_lo = min(words, sub * wps), w_hi = min(words, w_lo + wps);
-    for (int n0 = part * rows; n0 < r1; n0 += kTrThreads / 8) {
-        const int n = n0 + (tid >> 3);
-        const unsigned* row = bm + min(n, Kb - 1) * stride;
+    int* flat = jb.flat + (int64_t)bh * E;
+    for (int r0 = 0; r0 < nr; r0 += kTrThreads / 8) {
+        const int r = r0 + (tid >> 3);
+        const unsigned* row = bm + min(r, nr - 1) * stride;
         int mine = 0;
-        if (n < r1)
+        if (r < nr)
             for (int w = w_lo; w < w_hi; w++) mine += __popc(row[w]);
         int incl = mine;                                      // (all lanes take part in the shuffles)
 #pragma unroll
@@ -292,7 +334,7 @@ __global__ __launch_bounds__(kTrThreads) void transpose_bitmap_kernel(TrJobs job
             const int o = __shfl_up(incl, d, 8);
             if (sub >= d) incl += o;
         }
-        if (n >= r1) continue;
+        if (r >= nr) continue;
         int out = (int)row[words] + incl - mine;
         for (int w = w_lo; w < w_hi; w++) {
             unsigned wd = row[w];
@@ -441,18 +483,39 @@ static int check_transpose_job(const int32_t* idx, const int32_t* offsets, const
     return 0;
 }
 
-// the jobs whose bitmaps fit LDS, all in one launch
+// Ranges of key blocks a job is cut into for transpose_bitmap_kernel, 0: too large for it.  At least so many that a range's bitmaps take
+// at most 64 KB of LDS, and towards half the CUs over all (b,h): every range reads all entries, which is what a range's workgroup
+// spends its time on beyond about four of them (with a workgroup for every CU two levels of 12 x 16384 tokens 15.3 us, so 12).
+// More than 65536 entries (65536 tokens at topk 16) take as long here as the several kernels for large jobs take
+// beside the attention kernel on another stream (131072 entries: step 928 against 923 us, 196608: 672 against 664).
+constexpr int kTrLdsInts = 16 * 1024;
+static int tr_parts(int Mb, int Kb, int T, int BH) {
+    const int64_t stride = tr_stride(Mb), E = (int64_t)Mb * T;
+    if (stride > kTrLdsInts || Kb > 2 * kTrLdsInts) return 0;
+    const int most_rows = (int)std::min<int64_t>(kTrLdsInts / stride, kTrThreads);
+    const int least = (Kb + most_rows - 1) / most_rows;
+    if (E > 1 << 16) return 0;
+    const int parts = std::max({least, std::min(std::max(128 / BH - 1, 4), Kb / 32), 1});
+    const int rows = (Kb + parts - 1) / parts;
+    return (Kb + rows - 1) / rows;                            // no empty range
+}
+
+// the jobs that are small enough, all in one launch
 static int launch_bitmap_jobs(TrJobs& jobs, int n_jobs, int B, int H, hipStream_t st) {
     int64_t ints = 0;
-    for (int i = 0; i < n_jobs; i++) ints = std::max(ints, tr_bitmap_lds_ints(jobs.job[i].Mb, jobs.job[i].Kb));
+    jobs.wgs = 0;
+    jobs.n_jobs = n_jobs;
+    for (int i = 0; i < n_jobs; i++) {
+        const TrJob& j = jobs.job[i];
+        ints = std::max<int64_t>(ints, std::max<int64_t>((int64_t)j.rows * tr_stride(j.Mb), j.Kb));
+        jobs.wgs += j.parts + 1;
+    }
     const size_t lds = sizeof(int) * (size_t)ints;
-    if (lds > 64 * 1024) {
+    if (lds > 60 * 1024) {
         hipError_t e = hipFuncSetAttribute((const void*)transpose_bitmap_kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
         if (e != hipSuccess) return fail(-101, "transpose_indices: cannot raise dynamic LDS to %zu bytes: %s", lds, hipGetErrorString(e));
     }
-    jobs.max_parts = 1;
-    for (int i = 0; i < n_jobs; i++) jobs.max_parts = std::max(jobs.max_parts, jobs.job[i].parts);
-    hipLaunchKernelGGL(transpose_bitmap_kernel, dim3(B * H * jobs.max_parts, n_jobs), dim3(kTrThreads), lds, st, jobs);
+    hipLaunchKernelGGL(transpose_bitmap_kernel, dim3(B * H * jobs.wgs), dim3(kTrThreads), lds, st, jobs);
     return launch_status("transpose_indices");
 }
 
@@ -499,32 +562,32 @@ static int transpose_general(const int32_t* idx, int32_t* offsets, int32_t* flat
     return launch_status("transpose_indices");
 }
 
+extern "C" int llsa_transpose_one_launch(int Mb, int Kb, int T, int B, int H) {
+    return Mb > 0 && Kb > 0 && T > 0 && B > 0 && H > 0 && tr_parts(Mb, Kb, T, B * H) > 0;
+}
+
 extern "C" int llsa_transpose_indices_multi(const llsa_transpose_job* jobs, int n_jobs, int B, int H, void* stream) {
     LLSA_REQUIRE(jobs != nullptr && n_jobs >= 1 && n_jobs <= LLSA_MAX_LEVELS, "transpose_indices: 1..%d jobs, got %d", LLSA_MAX_LEVELS, n_jobs);
-    // One launch when the bitmaps of every job fit.  Beside a job that is too large for that, a small job shares the
-    // launch of the small ones only while its bitmaps are light (32 KB): a workgroup that wants most of a CU's LDS waits
-    // for a CU to drain when it runs next to the large job's kernels -- or next to an attention kernel on another
-    // stream, which is where a caller with large jobs runs this (0.6 ms instead of 16 us for the level-1 selection of
-    // 262144 tokens beside the forward kernel) -- so such a job takes the kernels for large jobs too.
-    bool all_fit = true;
-    for (int i = 0; i < n_jobs; i++) {
-        const llsa_transpose_job& j = jobs[i];
-        const int rc = check_transpose_job(j.idx, j.offsets, j.flat, j.work, B, H, j.Mb, j.Kb, j.T, j.chunk);
-        if (rc != 0) return rc;
-        all_fit = all_fit && tr_bitmap_lds_ints(j.Mb, j.Kb) <= kTrBitmapMaxInts;
-    }
-    constexpr int64_t kLightInts = 8 * 1024;
     TrJobs small;
     int n_small = 0;
     for (int i = 0; i < n_jobs; i++) {
         const llsa_transpose_job& j = jobs[i];
-        const int chunk = j.chunk < 1 ? 1 : j.chunk;
-        if (tr_bitmap_lds_ints(j.Mb, j.Kb) <= (all_fit ? kTrBitmapMaxInts : kLightInts)) {
+        const int rc = check_transpose_job(j.idx, j.offsets, j.flat, j.work, B, H, j.Mb, j.Kb, j.T, j.chunk);
+        if (rc != 0) return rc;
+    }
+    for (int i = 0; i < n_jobs; i++) {
+        const llsa_transpose_job& j = jobs[i];
+        const int chunk = j.chunk < 1 ? 1 : j.chunk, parts = tr_parts(j.Mb, j.Kb, j.T, B * H);
+        if (parts > 0) {
             TrJob& t = small.job[n_small++];
             t.idx = j.idx; t.offsets = j.offsets; t.flat = j.flat; t.work = j.work; t.inv = j.inv;
             t.Mb = j.Mb; t.Kb = j.Kb; t.T = j.T; t.chunk = chunk;
             t.work_stride = j.work ? (int)llsa_work_list_len(j.Mb, j.Kb, j.T, chunk) : 0;
-            t.parts = std::min(8, std::max(1, j.Kb / 128));
+            t.parts = parts;
+            t.rows = (j.Kb + parts - 1) / parts;
+            t.quads = j.T % 4 == 0 && aligned16(j.idx);
+            const unsigned per = t.quads ? j.T / 4 : j.T;     // (i * ceil(2^32 / per) >> 32 is i / per while i * per < 2^32)
+            t.row_magic = per == 1 ? 0u : (unsigned)((((uint64_t)1 << 32) + per - 1) / per);
         } else {
             const int rc = transpose_general(j.idx, j.offsets, j.flat, j.work, j.inv, B, H, j.Mb, j.Kb, j.T, chunk, stream);
             if (rc != 0) return rc;
