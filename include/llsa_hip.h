@@ -238,9 +238,10 @@ int llsa_transpose_one_launch(int Mb, int Kb, int T, int B, int H);
  * (the reference walks each segment serially, sparse_attention_res_1.py:300-322).  `work` is
  * (B,H,llsa_work_list_len(Mb,Kb,T,chunk)) int32, 16-byte aligned; llsa_attn_bwd needs the
  * work list of idx with chunk = llsa_fine_chunk(N) (the pooled levels need none).  Per (b,h), in int32:
- *   [0] items, [1] partial-sum slots, [2] key blocks with more than one chunk, [3] 0
+ *   [0] items, [1] partial-sum slots, [2] key blocks with more than one chunk,
+ *   [3] items with more than chunk/2 entries
  *   [4 + 4i ..]              item i = {key block, first entry in flat, entries, partial-sum slot or -1};
- *                            items with more than chunk/2 entries come first
+ *                            the items with more than chunk/2 entries come first
  *   [4 + 4*max_items + 4j ..] j-th key block with more than one chunk = {key block, first slot, chunks, 0}
  *   then Kb ints (rounded up to a multiple of 4) that the transpose itself uses as scratch
  * with max_items = Mb*T/chunk + Kb; every key block has at least one item. */

@@ -115,7 +115,7 @@ __device__ __forceinline__ int offsets_and_work_list(CountFn count_of, StartFn s
         work[0] = run_i;                                      // (the last thread's short items end the list)
         work[1] = run_s;
         work[2] = run_m;
-        work[3] = 0;
+        work[3] = total_long;
     }
     (void)E_total;
     return run;                                               // the end of this thread's key blocks: the total for the last thread
@@ -125,7 +125,7 @@ __device__ __forceinline__ int offsets_and_work_list(CountFn count_of, StartFn s
 // `chunk` entries so that a popular key block does not serialise on one wave.  Per (b,h), all
 // records 4 ints (16-byte aligned when the list is, so that one load fetches a record):
 //   work[0] = number of items, work[1] = number of partial-sum slots, work[2] = number of key
-//   blocks with more than one chunk, work[3] unused,
+//   blocks with more than one chunk, work[3] = number of items with more than chunk/2 entries (they come first),
 //   work[4 + 4i ..]             item i = {key block n, first entry in flat, entries, partial-sum slot
 //                               or -1 when n has one chunk}      (items of one key block are adjacent),
 //   work[4 + 4 max_items + 4j ..] j-th key block with more than one chunk = {n, first slot, chunks, 0}.
