@@ -35,6 +35,8 @@ __device__ __forceinline__ f32x4 mfma_bf16(bf16x8 a, bf16x8 b, f32x4 c) {
 __device__ __forceinline__ bf16x8 ld16(const bf16* p) { return *reinterpret_cast<const bf16x8*>(p); }
 __device__ __forceinline__ bf16x4 ld8(const bf16* p) { return *reinterpret_cast<const bf16x4*>(p); }
 __device__ __forceinline__ void st16(bf16* p, bf16x8 v) { *reinterpret_cast<bf16x8*>(p) = v; }
+// the same without a claim to the caches: for data that is not read again before much else has passed through them
+__device__ __forceinline__ bf16x8 ld16_stream(const bf16* p) { return __builtin_nontemporal_load(reinterpret_cast<const bf16x8*>(p)); }
 __device__ __forceinline__ void st8(bf16* p, bf16x4 v) { *reinterpret_cast<bf16x4*>(p) = v; }
 
 __device__ __forceinline__ bf16x8 cat(bf16x4 lo, bf16x4 hi) {

@@ -57,33 +57,38 @@ struct PoolParams {
 // array.  A thread's registers hold 256-byte pieces of it that are 256 bytes apart from its
 // neighbours' (R) or 8-byte pieces scattered over a whole tile (T); stored straight from the
 // registers every store instruction would touch 64 different cache lines with 16 or 8 bytes
-// each.  They go through LDS instead and leave as full-width stores: thread t of the workgroup
-// writes the 16 bytes at (k * 128 + t) * 16 for k = 0..15.  The staging buffer holds the 16-byte
-// units of a block in tile order with their low index bits XOR-ed so that both sides spread over
-// the banks without padding: exactly 32 KB, five workgroups per CU.
-__device__ __forceinline__ int swz_r(int u, int blk) { return u ^ ((u >> 4) ^ (blk & 15)); }   // u = chunk * 16 + row
-__device__ __forceinline__ int swz_t(int u) { return u ^ (u >> 5); }                           // u = unit of the T tile
+// each.  They go through LDS instead, eight rows of every block at a time and every wave by itself: 8 KB hold the half
+// tiles of the wave's eight blocks, and a store instruction writes half a tile in whole 128- or 256-byte pieces.
+// The pass is bound by memory -- loads and stores each take about as long as the whole should (19 and 15 us of 48 for
+// 2 x 6 x 16384 tokens with RoPE) -- so what counts is that waves in different phases overlap: half tiles leave LDS
+// for sixteen waves per CU, and no barrier keeps the waves of a workgroup together.
+// Units (16 bytes) of a half tile in LDS: their low index bits are XOR-ed with bits of chunk and block, so that the threads'
+// writes and the linear reads both spread evenly over the banks without padding.
+__device__ __forceinline__ int swz_r(int u, int blk) { return u ^ (u >> 3) ^ ((blk & 1) << 3); }               // u = chunk * 8 + row % 8
+__device__ __forceinline__ int swz_t(int u, int blk) { return u ^ (u >> 4) ^ ((blk & 1) << 3); }               // u = (chunk / 2) * 16 + unit % 16
 
-__device__ __forceinline__ void stage_out(bf16* stage, bf16* tiles32k, int t, int n_valid_blocks, bool r_layout) {
-    __syncthreads();                              // the staging buffer is filled
+__device__ __forceinline__ void wave_settle() {   // LDS of this wave: what was written is there for what follows
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+}
+// half h of the tiles of the wave's blocks b0 .. b0 + 7 from `stage` (the wave's 8 KB) to the workgroup's 32 KB piece of the tile array
+template <bool R>
+__device__ __forceinline__ void stage_out(const bf16* stage, bf16* tiles32k, int lane, int b0, int n_valid_blocks, int h) {
+    wave_settle();
+    // unit l of a half tile: R: chunk l / 8, row 8 h + l % 8; T: channel tile l / 16, units 16 h + l % 16 of it
+    const int unit = R ? (lane >> 3) * 16 + h * 8 + (lane & 7) : (lane >> 4) * 32 + h * 16 + (lane & 15);
 #pragma unroll
-    for (int k = 0; k < 16; k++) {
-        if (k < n_valid_blocks) {
-            const int u = r_layout ? swz_r(t, k) : swz_t(t);
-            st16(tiles32k + (k * 128 + t) * 8, ld16(stage + (k * 128 + u) * 8));
-        }
-    }
-    __syncthreads();                              // and may be refilled
+    for (int k = 0; k < 8; k++)
+        if (b0 + k < n_valid_blocks)
+            st16(tiles32k + ((b0 + k) * 128 + unit) * 8, ld16(stage + (k * 64 + (R ? swz_r(lane, k) : swz_t(lane, k))) * 8));
+    wave_settle();                                // and may be refilled
 }
 
-// RMS normalisation of the thread's 16 rows (8 channels of each; the row's other channels are
+// RMS normalisation of eight of the thread's rows (8 channels of each; the row's other channels are
 // in the 7 neighbouring lanes): x <- bf16(x * rsqrt(mean(x^2) + eps) * gamma), in fp32.
-__device__ __forceinline__ void rms_norm_rows(bf16x8 xv[16], const float* gamma, float eps, int c) {
-    float g[8];
+__device__ __forceinline__ void rms_norm_rows(bf16x8* xv, const float (&g)[8], float eps) {
 #pragma unroll
-    for (int e = 0; e < 8; e++) g[e] = gamma[c * 8 + e];
-#pragma unroll
-    for (int i = 0; i < 16; i++) {
+    for (int i = 0; i < 8; i++) {
         float ss = 0.f;
 #pragma unroll
         for (int e = 0; e < 8; e++) ss += (float)xv[i][e] * (float)xv[i][e];
@@ -96,9 +101,13 @@ __device__ __forceinline__ void rms_norm_rows(bf16x8 xv[16], const float* gamma,
     }
 }
 
-template <bool NORM>
-__global__ __launch_bounds__(128) void pool_pyramid_kernel(PoolParams p) {
-    __shared__ __align__(16) bf16 stage[16 * 128 * 8];
+// STREAM (a launch that writes both tiles of a tensor, i.e. the backward's too): the rows are read past the caches.  In a
+// training step nothing reads them again, and the tiles, which the attention kernels gather from the caches right
+// afterwards, have the more room (24 x 4096 and 15 x 7168 tokens: 2 % of the step, 6 x 65536: 1 %).  Writing the tiles
+// that way makes this pass faster still (49 -> 43 us) and every reader slower by more.
+template <bool NORM, bool STREAM>
+__global__ __launch_bounds__(128, 4) void pool_pyramid_kernel(PoolParams p) {
+    __shared__ __align__(16) bf16 stage[2][8 * 64 * 8];
     // (items interleaved along x: q and k with their rotation are arithmetic-heavy, v with its two tiles is store-heavy,
     // and workgroups start in x order -- a launch that runs one item after the other works in phases)
     const int item = (int)blockIdx.x % p.n_items, bx = (int)blockIdx.x / p.n_items;
@@ -107,69 +116,80 @@ __global__ __launch_bounds__(128) void pool_pyramid_kernel(PoolParams p) {
     if (bx * 16 >= n1) return;                    // uniform over the workgroup
     const int bh = blockIdx.y, b = bh / p.H, h = bh % p.H;
     const int t = threadIdx.x, c = t & 7, r = t >> 3;
+    const int wave = t >> 6, lane = t & 63;
     const int blk = bx * 16 + r;
     const bool valid = blk < n1;
     const int n_valid = min(16, n1 - bx * 16);
+    bf16* const st = &stage[wave][0];
+    const int rw = r & 7;                         // block of the wave
 
     bf16x8 xv[16];
-    bf16x8 y = zero8();
-    if (valid) {
-        const bf16* x = (const bf16*)it.x + b * it.sxb + h * it.sxh + (int64_t)blk * kBlk * it.sxn + c * 8;
+    const bf16* x = (const bf16*)it.x + b * it.sxb + h * it.sxh + (int64_t)min(blk, n1 - 1) * kBlk * it.sxn + c * 8;
 #pragma unroll
-        for (int i = 0; i < 16; i++) xv[i] = ld16(x + i * it.sxn);
-        if (NORM && it.gamma != nullptr) rms_norm_rows(xv, it.gamma, it.eps, c);
+    for (int i = 0; i < 16; i++) xv[i] = STREAM ? ld16_stream(x + i * it.sxn) : ld16(x + i * it.sxn);
+    float g[8];
+    const bool norm = NORM && it.gamma != nullptr;
+    if (norm) {
+#pragma unroll
+        for (int e = 0; e < 8; e++) g[e] = it.gamma[c * 8 + e];
+    }
+    const bool pooled = it.y1 != nullptr || it.y2 != nullptr || it.y1r != nullptr || it.y1t != nullptr;
+    float acc[8];
+#pragma unroll
+    for (int e = 0; e < 8; e++) acc[e] = 0.f;
+#pragma unroll
+    for (int hf = 0; hf < 2; hf++) {              // rows 0..7, then 8..15 of the thread's block
+        bf16x8* xh = xv + 8 * hf;
+        if (norm) rms_norm_rows(xh, g, it.eps);
         if (it.rope) {
-            const bf16* f = p.freq + ((int64_t)blk * kBlk) * kD + c * 8;
+            const bf16* f = p.freq + ((int64_t)min(blk, n1 - 1) * kBlk + 8 * hf) * kD + c * 8;
 #pragma unroll
-            for (int i = 0; i < 16; i++) xv[i] = rope_chunk_fwd(xv[i], ld16(f + i * kD));
+            for (int i = 0; i < 8; i++) xh[i] = rope_chunk_fwd(xh[i], ld16(f + i * kD));
         }
-        if (it.xrot != nullptr) {        // the rows as the attention sees them (normalised, rotated), row-major
-            bf16* xo = (bf16*)it.xrot + ((int64_t)bh * it.n + (int64_t)blk * kBlk) * kD + c * 8;
+        if (it.xrot != nullptr && valid) {        // the rows as the attention sees them (normalised, rotated), row-major
+            bf16* xo = (bf16*)it.xrot + ((int64_t)bh * it.n + (int64_t)blk * kBlk + 8 * hf) * kD + c * 8;
 #pragma unroll
-            for (int i = 0; i < 16; i++) st16(xo + i * kD, xv[i]);
+            for (int i = 0; i < 8; i++) st16(xo + i * kD, xh[i]);
         }
-        if (it.y1 != nullptr || it.y2 != nullptr || it.y1r != nullptr || it.y1t != nullptr) {
-            float acc[8];
+        if (it.xr != nullptr) {                   // R tile: chunk c of row i is 16-byte unit c * 16 + i of the block
 #pragma unroll
-            for (int e = 0; e < 8; e++) acc[e] = 0.f;
-#pragma unroll
-            for (int i = 0; i < 16; i++)
-#pragma unroll
-                for (int e = 0; e < 8; e++) acc[e] = rn_bf16(acc[e] + (float)xv[i][e]);
-#pragma unroll
-            for (int e = 0; e < 8; e++) y[e] = (bf16)(acc[e] * 0.0625f);
-            if (it.y1 != nullptr) st16((bf16*)it.y1 + ((int64_t)bh * n1 + blk) * kD + c * 8, y);
+            for (int i = 0; i < 8; i++) st16(st + (rw * 64 + swz_r(c * 8 + i, rw)) * 8, xh[i]);
+            stage_out<true>(st, (bf16*)it.xr + ((int64_t)bh * n1 + bx * 16) * kTile, lane, wave * 8, n_valid, hf);
         }
-    }
-    if (it.xr != nullptr) {              // R tile: chunk c of row i is 16-byte unit c * 16 + i of the block
-        if (valid) {
+        if (it.xt != nullptr) {                   // T tile: channels 8c+e, 8c+e+1 of tokens 4q..4q+3 are one 16-byte unit
 #pragma unroll
-            for (int i = 0; i < 16; i++) st16(stage + (r * 128 + swz_r(c * 16 + i, r)) * 8, xv[i]);
-        }
-        stage_out(stage, (bf16*)it.xr + ((int64_t)bh * n1 + bx * 16) * kTile, t, n_valid, true);
-    }
-    if (it.xt != nullptr) {              // T tile: channels 8c+e, 8c+e+1 of tokens 4q..4q+3 are one 16-byte unit
-        if (valid) {
-#pragma unroll
-            for (int q = 0; q < 4; q++)
+            for (int q = 0; q < 2; q++)
 #pragma unroll
                 for (int ep = 0; ep < 4; ep++) {
                     bf16x8 v;
 #pragma unroll
                     for (int j = 0; j < 4; j++) {
-                        v[j] = xv[4 * q + j][2 * ep];
-                        v[4 + j] = xv[4 * q + j][2 * ep + 1];
+                        v[j] = xh[4 * q + j][2 * ep];
+                        v[4 + j] = xh[4 * q + j][2 * ep + 1];
                     }
-                    const int u = t_tile_off(4 * q, 8 * c + 2 * ep) / 8;      // 16-byte unit inside the tile
-                    st16(stage + (r * 128 + swz_t(u)) * 8, v);
+                    const int u = (c >> 1) * 16 + q * 8 + (c & 1) * 4 + ep;
+                    st16(st + (rw * 64 + swz_t(u, rw)) * 8, v);
                 }
+            stage_out<false>(st, (bf16*)it.xt + ((int64_t)bh * n1 + bx * 16) * kTile, lane, wave * 8, n_valid, hf);
         }
-        stage_out(stage, (bf16*)it.xt + ((int64_t)bh * n1 + bx * 16) * kTile, t, n_valid, false);
+        if (pooled) {
+#pragma unroll
+            for (int i = 0; i < 8; i++)
+#pragma unroll
+                for (int e = 0; e < 8; e++) acc[e] = rn_bf16(acc[e] + (float)xh[i][e]);
+        }
+    }
+    bf16x8 y = zero8();
+    if (pooled && valid) {
+#pragma unroll
+        for (int e = 0; e < 8; e++) y[e] = (bf16)(acc[e] * 0.0625f);
+        if (it.y1 != nullptr) st16((bf16*)it.y1 + ((int64_t)bh * n1 + blk) * kD + c * 8, y);
     }
     if (it.y2 == nullptr && it.y1r == nullptr && it.y1t == nullptr && it.y2r == nullptr && it.y2t == nullptr) return;   // uniform over the workgroup
 
     // the 16 pooled rows of this workgroup are one block of the next level
-    bf16 (*sm)[kD] = reinterpret_cast<bf16 (*)[kD]>(stage);
+    __syncthreads();                              // (both waves are done with their staging buffers)
+    bf16 (*sm)[kD] = reinterpret_cast<bf16 (*)[kD]>(&stage[0][0]);
     st16(&sm[r][c * 8], y);
     __syncthreads();
     const int n2 = it.n / (kBlk * kBlk);
@@ -392,10 +412,13 @@ extern "C" int llsa_pool_pyramid_fwd(const llsa_pool_item* items, int n_items, c
     for (int i = 0; i < n_items; i++) norm = norm || items[i].gamma != nullptr;
     p.n_items = n_items;
     dim3 grid((max_n + 255) / 256 * n_items, B * H);
-    if (norm)
-        hipLaunchKernelGGL(HIP_KERNEL_NAME(pool_pyramid_kernel<true>), grid, dim3(128), 0, (hipStream_t)stream, p);
-    else
-        hipLaunchKernelGGL(HIP_KERNEL_NAME(pool_pyramid_kernel<false>), grid, dim3(128), 0, (hipStream_t)stream, p);
+    bool both = false;
+    for (int i = 0; i < n_items; i++) both = both || (items[i].xr != nullptr && items[i].xt != nullptr);
+    const hipStream_t st = (hipStream_t)stream;
+    if (norm && both) hipLaunchKernelGGL(HIP_KERNEL_NAME(pool_pyramid_kernel<true, true>), grid, dim3(128), 0, st, p);
+    else if (norm) hipLaunchKernelGGL(HIP_KERNEL_NAME(pool_pyramid_kernel<true, false>), grid, dim3(128), 0, st, p);
+    else if (both) hipLaunchKernelGGL(HIP_KERNEL_NAME(pool_pyramid_kernel<false, true>), grid, dim3(128), 0, st, p);
+    else hipLaunchKernelGGL(HIP_KERNEL_NAME(pool_pyramid_kernel<false, false>), grid, dim3(128), 0, st, p);
     return launch_status("pool_pyramid");
 }
 
