@@ -44,7 +44,7 @@ extern "C" {
 #define LLSA_DTYPE_BF16 0
 #define LLSA_DTYPE_F32 1
 
-#define LLSA_ABI_VERSION 204     /* changes with every change of a signature or argument structure below */
+#define LLSA_ABI_VERSION 205     /* changes with every change of a signature or argument structure below */
 int llsa_version(void);          /* LLSA_ABI_VERSION of the built library                                    */
 const char* llsa_last_error_string(void);
 
@@ -75,7 +75,7 @@ typedef struct llsa_pool_item {
     void* xrot;             /* (B,H,n,64) contiguous copy of the normalised / rotated x, or NULL */
     const float* gamma;     /* (64) fp32 or NULL: RMS-normalise every row first (see below)     */
     float eps;
-    int32_t reserved;       /* 0                                                                */
+    int32_t stream;         /* 1: nothing reads x again soon, read it past the caches            */
     void* y2r;              /* (B,H,n/4096,1024) R tiles of y2, or NULL (n % 4096 == 0)         */
     void* y2t;              /* (B,H,n/4096,1024) T tiles of y2, or NULL (n % 4096 == 0)         */
 } llsa_pool_item;
@@ -196,7 +196,8 @@ typedef struct llsa_fwd_level {
 typedef struct llsa_attn_fwd_args {
     const void* qr;                            /* (B,H,N/16,1024)   R tiles of q                  */
     const void* kr;                            /* (B,H,N/16,1024)   R tiles of k                  */
-    const void* vt;                            /* (B,H,N/16,1024)   T tiles of v                  */
+    const void* vt;                            /* (B,H,N/16,1024)   R tiles of v: the fine blocks' T
+                                                  operands are made from them on chip           */
     const int32_t* idx;                        /* (B,H,N/16,T)   selected fine blocks             */
     void* o;        int64_t sob, soh, son;     /* (B,H,N,64) out                                  */
     float* lse;                                /* (B,H,N) out, m + log(l)                          */

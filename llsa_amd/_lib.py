@@ -26,7 +26,7 @@ class PoolItem(C.Structure):
                 ("n", c_int32), ("rope", c_int32),
                 ("y1", c_void_p), ("y2", c_void_p), ("xr", c_void_p), ("xt", c_void_p), ("y1r", c_void_p),
                 ("y1t", c_void_p), ("xrot", c_void_p),
-                ("gamma", c_void_p), ("eps", c_float), ("reserved", c_int32), ("y2r", c_void_p), ("y2t", c_void_p)]
+                ("gamma", c_void_p), ("eps", c_float), ("stream", c_int32), ("y2r", c_void_p), ("y2t", c_void_p)]
 
 
 MAX_LEVELS = 4                                              # LLSA_MAX_LEVELS
@@ -107,7 +107,7 @@ _SIGNATURES = {
 
 EXPORTS = tuple(_SIGNATURES)
 CHUNK_FINE_MAX = 256                                        # LLSA_CHUNK_FINE_MAX of include/llsa_hip.h
-ABI_VERSION = 204                                           # LLSA_ABI_VERSION
+ABI_VERSION = 205                                           # LLSA_ABI_VERSION
 STATIC_PARTIALS_MAX = 262144                                # LLSA_STATIC_PARTIALS_MAX
 
 

@@ -19,14 +19,14 @@
 namespace llsa {
 
 // ---------------------------------------------------------------------------------------
-// dQ: one wave per query block, four consecutive query blocks per workgroup, key blocks taken
+// dQ: Q query blocks per wave, 4 Q consecutive query blocks per workgroup, key blocks taken
 // two at a time (32 keys = one MFMA K step).
 //
 // K and V always reach the MFMA from R tiles.  K is needed twice: as the A operand of S^T (a plain
 // 16-byte read per lane) and, read back with the transposing LDS load, as the A operand of
 // dQ^T += K^T.dS^T -- so K goes through LDS in any case, copied there straight from global memory.
 //  * pooled blocks (level-1 pooled tokens of the parent's coarse blocks, the coarsest level) are
-//    the same for the four query blocks of the workgroup: one copy per workgroup, kGroup blocks
+//    the same for all query blocks of the workgroup: one copy per workgroup, kGroup blocks
 //    of K and V at a time, two buffers;
 //  * fine blocks are private: afterwards each wave re-uses a quarter of the same LDS as two slots
 //    for the K tiles of a pair (the copy of pair t+1 in flight during pair t), V stays in registers.
@@ -129,23 +129,35 @@ __device__ __forceinline__ void dq_end(const DqSide& sd, const llsa_attn_bwd_arg
         st8(op + dt * 16, o);
     }
 }
-__device__ __forceinline__ void dq_pair_of_blocks(DqSide& sd, const PairR& r, const PairT& t, float log2w) {
-    dq_accum(sd.dq, t, dq_scores(r, sd.bq, sd.bdo, sd.lse2 - log2w, sd.dl));
+// in0, in1 (wave-uniform): whether the query block reads the pair's first / second block
+__device__ __forceinline__ void dq_pair_of_blocks(DqSide& sd, const PairR& r, const PairT& t, float log2w, bool in0 = true, bool in1 = true) {
+    bf16x8 bds = dq_scores(r, sd.bq, sd.bdo, sd.lse2 - log2w, sd.dl);
+#pragma unroll
+    for (int e = 0; e < 4; e++) {
+        if (!in0) bds[e] = (bf16)0.f;
+        if (!in1) bds[4 + e] = (bf16)0.f;
+    }
+    dq_accum(sd.dq, t, bds);
 }
 
-__global__ __launch_bounds__(256) void attn_dq_kernel(llsa_attn_bwd_args a, float* __restrict__ delta,
-                                                      bf16* __restrict__ dor) {
+// Q sibling query blocks per wave (see attn_fwd_kernel): the pooled blocks and the fine blocks both rows selected are read once
+// -- from memory and, what weighs more here, from LDS, where every key block is read three times (K rows, V rows, K
+// transposed) -- and multiplied twice.
+template <int Q, int R>
+__global__ __launch_bounds__(256, Q == 1 ? 4 : 3) void attn_dq_kernel(llsa_attn_bwd_args a, float* __restrict__ delta,
+                                                                      bf16* __restrict__ dor) {
     __shared__ __align__(16) bf16 sh[2][kGroup][2 * kTile];   // per block: R tile of K, R tile of V
+    __shared__ int order[4][R * kWave];
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int N1 = a.N / kBlk;
+    const int N1 = a.N / kBlk, T = a.T;
     const int lid = xcd_logical_id();
-    const int g = (lid % (int)gridDim.x) * 4 + wave;          // < N1: the host checks N1 % 4 == 0
+    const int g = (lid % (int)gridDim.x) * (4 * Q) + Q * wave;        // query blocks g .. g + Q - 1 (the host checks N1 % 4 Q == 0)
     const int bh = lid / (int)gridDim.x, b = bh / a.H, h = bh % a.H;
 
     const bf16* kr = (const bf16*)a.kr + (int64_t)bh * N1 * kTile;
     const bf16* vr = (const bf16*)a.vr + (int64_t)bh * N1 * kTile;
-    const int* ip = a.idx + ((int64_t)bh * N1 + g) * a.T;
+    const int* ip = a.idx + ((int64_t)bh * N1 + g) * T;
 
     // shared list: the selected blocks of every pooled level below the coarsest, then every block of the coarsest
     SharedList sl = shared_list(a.lvl, a.levels, a.N, bh, g, lane);
@@ -162,114 +174,16 @@ __global__ __launch_bounds__(256) void attn_dq_kernel(llsa_attn_bwd_args a, floa
         copy16_global_to_lds(vb + 512 + lane * 8, dst + kTile + 512);
     };
     issue_group(0);
-    int mine = (lane < min(kWave, a.T)) ? ip[lane] : 0;       // first 64 fine indices, entry i in lane i
+    MergedLists<Q, R> ml = merge_lists<Q, R>(ip, min(T, kWave * R / Q), N1, lane, order[wave]);
 
-    DqSide sd;
-    dq_begin(sd, a, delta, dor, bh, b, h, g, lane);
+    DqSide sd[Q];
+#pragma unroll
+    for (int u = 0; u < Q; u++) dq_begin(sd[u], a, delta, dor, bh, b, h, g + u, lane);
 
     // ---- pooled blocks out of the shared copy.  The barrier at the top of round grp says: every
     // wave's part of group grp has landed, and every wave is done reading the other buffer.  All
     // LDS reads of a round come before the next fetch is issued (the compiler makes an LDS read
     // wait for every copy into LDS issued before it).
-    for (int grp = 0; grp < n_groups; grp++) {
-        wait_vm0();
-        __syncthreads();
-        const float w = __builtin_amdgcn_logf(a.lvl[shared_level(a.lvl, a.levels, kGroup * grp)].w);   // log2
-        const bf16* blk = sh0 + (grp & 1) * kGroup * (2 * kTile);
-        PairR r0;
-        PairT t0;
-        read_k_r(r0, blk, blk + 2 * kTile, lane);
-        read_v_r(r0, blk + kTile, blk + 3 * kTile, lane);
-        read_k_t(t0, blk, blk + 2 * kTile, lane);
-        dq_pair_of_blocks(sd, r0, t0, w);
-        read_k_r(r0, blk + 4 * kTile, blk + 6 * kTile, lane);
-        read_v_r(r0, blk + 5 * kTile, blk + 7 * kTile, lane);
-        read_k_t(t0, blk + 4 * kTile, blk + 6 * kTile, lane);
-        if (grp + 1 < n_groups) issue_group(grp + 1);
-        dq_pair_of_blocks(sd, r0, t0, w);
-    }
-    __syncthreads();                                          // the shared copy is dead: its LDS becomes private slots
-
-    // ---- fine blocks: K of pair t+1 is copied into the wave's other slot and V of pair t+1 loaded
-    // into registers while pair t is worked on.  Nothing may be in flight when the wave ends (a copy
-    // landing in LDS that already belongs to another workgroup), so the last pair fetches nothing.
-    bf16* const priv = sh0 + wave * (4 * kTile);              // two slots of two K tiles
-    for (int c0 = 0; c0 < a.T; c0 += kWave) {
-        const int cn = min(kWave, a.T - c0);
-        if (c0 > 0) mine = (lane < cn) ? ip[c0 + lane] : 0;
-        const int n_pairs = cn / 2;
-        PairR ra, rb;
-        auto fetch = [=](int t, PairR& dst) __attribute__((always_inline)) {
-            bf16* slot = priv + (t & 1) * (2 * kTile);
-#pragma unroll
-            for (int j = 0; j < 2; j++) {
-                const int blk = clampi(__builtin_amdgcn_readlane(mine, 2 * t + j), 0, N1 - 1);
-                const bf16* kb = kr + (int64_t)blk * kTile;
-                const bf16* vb = vr + (int64_t)blk * kTile;
-                copy16_global_to_lds(kb + lane * 8, slot + j * kTile);
-                copy16_global_to_lds(kb + 512 + lane * 8, slot + j * kTile + 512);
-                dst.v[j][0] = ld16(vb + lane * 8);
-                dst.v[j][1] = ld16(vb + 512 + lane * 8);
-            }
-        };
-        auto work = [&](int t, PairR& cur, PairR& nxt) __attribute__((always_inline)) {
-            wait_vm0();
-            const bf16* slot = priv + (t & 1) * (2 * kTile);
-            PairT tt;
-            read_k_r(cur, slot, slot + kTile, lane);
-            read_k_t(tt, slot, slot + kTile, lane);
-            if (t + 1 < n_pairs) fetch(t + 1, nxt);
-            dq_pair_of_blocks(sd, cur, tt, 0.f);
-        };
-        fetch(0, ra);
-        for (int t = 0; t < n_pairs; t += 2) {                // n_pairs is even (T % 4 == 0)
-            work(t, ra, rb);
-            work(t + 1, rb, ra);
-        }
-    }
-    dq_end(sd, a, b, h, g, lane);
-}
-
-// Two sibling query blocks per wave (topk <= 32 R <= kPairMaxTopk): the pooled blocks and the fine blocks both rows
-// selected are read once -- from memory and, what weighs more here, from LDS, where every key block is read
-// three times (K rows, V rows, K transposed) -- and multiplied twice.  See pair_order for the walk.
-template <int R>
-__global__ __launch_bounds__(256, 3) void attn_dq_pair_kernel(llsa_attn_bwd_args a, float* __restrict__ delta,
-                                                              bf16* __restrict__ dor) {
-    __shared__ __align__(16) bf16 sh[2][kGroup][2 * kTile];
-    __shared__ int order[4][R * kWave];
-    const int lane = threadIdx.x & 63;
-    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int N1 = a.N / kBlk, T = a.T;
-    const int lid = xcd_logical_id();
-    const int g = (lid % (int)gridDim.x) * 8 + 2 * wave;      // query blocks g and g + 1 (the host checks N1 % 8 == 0)
-    const int bh = lid / (int)gridDim.x, b = bh / a.H, h = bh % a.H;
-
-    const bf16* kr = (const bf16*)a.kr + (int64_t)bh * N1 * kTile;
-    const bf16* vr = (const bf16*)a.vr + (int64_t)bh * N1 * kTile;
-    const int* ip = a.idx + ((int64_t)bh * N1 + g) * T;
-
-    SharedList sl = shared_list(a.lvl, a.levels, a.N, bh, g, lane);
-    const int n_groups = sl.n_blocks / kGroup;
-    bf16* const sh0 = &sh[0][0][0];
-    auto issue_group = [&](int grp) __attribute__((always_inline)) {
-        const SharedBlock sb = shared_block(sl, a.lvl, a.levels, a.N, bh, kGroup * grp + wave);
-        const bf16* kb = (const bf16*)a.lvl[sb.level].kr + sb.tile;
-        const bf16* vb = (const bf16*)a.lvl[sb.level].vr + sb.tile;
-        bf16* dst = sh0 + ((grp & 1) * kGroup + wave) * (2 * kTile);
-        copy16_global_to_lds(kb + lane * 8, dst);
-        copy16_global_to_lds(kb + 512 + lane * 8, dst + 512);
-        copy16_global_to_lds(vb + lane * 8, dst + kTile);
-        copy16_global_to_lds(vb + 512 + lane * 8, dst + kTile + 512);
-    };
-    issue_group(0);
-    const PairOrder<R> po = pair_order<R>(ip, T, N1, lane, order[wave]);
-    const int steps_both = po.n_both / 2, steps_only = (T - po.n_both) / 2, n_steps = steps_both + 2 * steps_only;
-
-    DqSide sd[2];
-    dq_begin(sd[0], a, delta, dor, bh, b, h, g, lane);
-    dq_begin(sd[1], a, delta, dor, bh, b, h, g + 1, lane);
-
     // (two groups per trip: the buffer a group sits in is then a constant and every LDS address a lane-invariant
     // base plus an immediate)
     auto shared_group = [&](int grp, const bf16* blk) __attribute__((always_inline)) {
@@ -281,53 +195,68 @@ __global__ __launch_bounds__(256, 3) void attn_dq_pair_kernel(llsa_attn_bwd_args
         read_k_r(r0, blk, blk + 2 * kTile, lane);
         read_v_r(r0, blk + kTile, blk + 3 * kTile, lane);
         read_k_t(t0, blk, blk + 2 * kTile, lane);
-        dq_pair_of_blocks(sd[0], r0, t0, w);
-        dq_pair_of_blocks(sd[1], r0, t0, w);
+#pragma unroll
+        for (int u = 0; u < Q; u++) dq_pair_of_blocks(sd[u], r0, t0, w);
         read_k_r(r0, blk + 4 * kTile, blk + 6 * kTile, lane);
         read_v_r(r0, blk + 5 * kTile, blk + 7 * kTile, lane);
         read_k_t(t0, blk + 4 * kTile, blk + 6 * kTile, lane);
         if (grp + 1 < n_groups) issue_group(grp + 1);
-        dq_pair_of_blocks(sd[0], r0, t0, w);
-        dq_pair_of_blocks(sd[1], r0, t0, w);
+#pragma unroll
+        for (int u = 0; u < Q; u++) dq_pair_of_blocks(sd[u], r0, t0, w);
     };
     for (int grp = 0; grp < n_groups; grp += 2) {
         shared_group(grp, sh0);
         if (grp + 1 < n_groups) shared_group(grp + 1, sh0 + kGroup * (2 * kTile));
     }
-    __syncthreads();
+    __syncthreads();                                          // the shared copy is dead: its LDS becomes private slots
 
-    bf16* const priv = sh0 + wave * (4 * kTile);
-    PairR ra, rb;
-    auto fetch = [=](int t, PairR& dst) __attribute__((always_inline)) {
-        bf16* slot = priv + (t & 1) * (2 * kTile);
+    // ---- fine blocks: K of step t+1 is copied into the wave's other slot and V of step t+1 loaded
+    // into registers while step t is worked on.  Nothing may be in flight when the wave ends (a copy
+    // landing in LDS that already belongs to another workgroup), so the last step fetches nothing.
+    bf16* const priv = sh0 + wave * (4 * kTile);              // two slots of two K tiles
+    auto fine = [&]() __attribute__((always_inline)) {
+        const int n_steps = (ml.n + 1) / 2;
+        PairR ra, rb;
+        auto fetch = [&](int t, PairR& dst) __attribute__((always_inline)) {
+            bf16* slot = priv + (t & 1) * (2 * kTile);
 #pragma unroll
-        for (int j = 0; j < 2; j++) {
-            const int blk = po.entry(2 * t + j);
-            const bf16* kb = kr + (int64_t)blk * kTile;
-            const bf16* vb = vr + (int64_t)blk * kTile;
-            copy16_global_to_lds(kb + lane * 8, slot + j * kTile);
-            copy16_global_to_lds(kb + 512 + lane * 8, slot + j * kTile + 512);
-            dst.v[j][0] = ld16(vb + lane * 8);
-            dst.v[j][1] = ld16(vb + 512 + lane * 8);
+            for (int j = 0; j < 2; j++) {
+                const int64_t at = (int64_t)ml.block(min(2 * t + j, ml.n - 1)) * kTile + lane * 8;
+                copy16_global_to_lds(kr + at, slot + j * kTile);
+                copy16_global_to_lds(kr + at + 512, slot + j * kTile + 512);
+                dst.v[j][0] = ld16(vr + at);
+                dst.v[j][1] = ld16(vr + at + 512);
+            }
+        };
+        auto work = [&](int t, PairR& cur, PairR& nxt) __attribute__((always_inline)) {
+            const unsigned m0 = ml.rows(2 * t), m1 = 2 * t + 1 < ml.n ? ml.rows(2 * t + 1) : 0u;
+            wait_vm0();
+            const bf16* slot = priv + (t & 1) * (2 * kTile);
+            PairT tt;
+            read_k_r(cur, slot, slot + kTile, lane);
+            read_k_t(tt, slot, slot + kTile, lane);
+            if (t + 1 < n_steps) fetch(t + 1, nxt);
+#pragma unroll
+            for (int u = 0; u < Q; u++) {
+                const bool in0 = (m0 >> u) & 1u, in1 = (m1 >> u) & 1u;
+                if (in0 || in1) dq_pair_of_blocks(sd[u], cur, tt, 0.f, in0, in1);
+            }
+        };
+        fetch(0, ra);
+        for (int t = 0; t < n_steps; t += 2) {
+            work(t, ra, rb);
+            if (t + 1 < n_steps) work(t + 1, rb, ra);
         }
     };
-    auto work = [&](int t, PairR& cur, PairR& nxt) __attribute__((always_inline)) {
-        wait_vm0();
-        const bf16* slot = priv + (t & 1) * (2 * kTile);
-        PairT tt;
-        read_k_r(cur, slot, slot + kTile, lane);
-        read_k_t(tt, slot, slot + kTile, lane);
-        if (t + 1 < n_steps) fetch(t + 1, nxt);
-        if (t < steps_both + steps_only) dq_pair_of_blocks(sd[0], cur, tt, 0.f);
-        if (t < steps_both || t >= steps_both + steps_only) dq_pair_of_blocks(sd[1], cur, tt, 0.f);
-    };
-    fetch(0, ra);
-    for (int t = 0; t < n_steps; t += 2) {
-        work(t, ra, rb);
-        if (t + 1 < n_steps) work(t + 1, rb, ra);
+    fine();
+    if constexpr (Q == 1) {                                   // longer lists: 64 entries at a time
+        for (int c0 = kWave * R; c0 < T; c0 += kWave * R) {
+            ml = merge_lists<Q, R>(ip + c0, min(T - c0, kWave * R), N1, lane, order[wave]);
+            fine();
+        }
     }
-    dq_end(sd[0], a, b, h, g, lane);
-    dq_end(sd[1], a, b, h, g + 1, lane);
+#pragma unroll
+    for (int u = 0; u < Q; u++) dq_end(sd[u], a, b, h, g + u, lane);
 }
 
 // ---------------------------------------------------------------------------------------
@@ -1262,11 +1191,14 @@ extern "C" int llsa_attn_bwd(const llsa_attn_bwd_args* a, void* stream) {
 
     const int stages = a->stages ? a->stages : (0x7fffffff & ~LLSA_BWD_NO_REDUCE);
     if (stages & LLSA_BWD_DQ) {
-        if (a->T <= kPairMaxTopk && N1 % 8 == 0 && (int64_t)N1 / 8 * BH >= kPairMinGroups)
-            if (a->T <= 32) hipLaunchKernelGGL(HIP_KERNEL_NAME(attn_dq_pair_kernel<1>), dim3(N1 / 8, BH), dim3(256), 0, s, *a, delta, dor);
-            else hipLaunchKernelGGL(HIP_KERNEL_NAME(attn_dq_pair_kernel<2>), dim3(N1 / 8, BH), dim3(256), 0, s, *a, delta, dor);
+        // (two query blocks per wave win from 512 groups of eight on, see kPairMinGroups: 12 x 16384 tokens 79 against 82.6 us,
+        // 6 x 262144 1022 against 1113)
+        if (a->T > kPairMaxTopk || N1 % 8 != 0 || (int64_t)N1 / 8 * BH < kPairMinGroups)
+            hipLaunchKernelGGL(HIP_KERNEL_NAME(attn_dq_kernel<1, 1>), dim3(N1 / 4, BH), dim3(256), 0, s, *a, delta, dor);
+        else if (a->T <= 32)
+            hipLaunchKernelGGL(HIP_KERNEL_NAME(attn_dq_kernel<2, 1>), dim3(N1 / 8, BH), dim3(256), 0, s, *a, delta, dor);
         else
-            hipLaunchKernelGGL(attn_dq_kernel, dim3((N1 + 3) / 4, BH), dim3(256), 0, s, *a, delta, dor);
+            hipLaunchKernelGGL(HIP_KERNEL_NAME(attn_dq_kernel<2, 2>), dim3(N1 / 8, BH), dim3(256), 0, s, *a, delta, dor);
     }
 
     ReduceParams rp;

@@ -1,6 +1,6 @@
 // Block-sparse flash-attention forward for llsa_l1 / llsa_l2.
 //
-// One wave owns one query block (16 queries).  All products run on the bf16 16x16x32 MFMA
+// One wave owns one or two query blocks (16 queries each).  All products run on the bf16 16x16x32 MFMA
 // in the "transposed" orientation, keys on the M axis and queries on the N axis:
 //     S^T (16 keys x 16 queries) = K_blk (16x64) . Q^T            A = R tile of K, B = R tile of Q
 //     O^T (64 ch  x 16 queries) += V_blk^T (64x32 keys) . P^T     A = T tiles of V, B = P^T
@@ -35,26 +35,6 @@ struct KvRegs {
     bf16x8 k[NB][2];     // K rows (R tile): block j, channel half
     bf16x8 v[NB / 2][4]; // V (T tiles of a pair of blocks): channel tile dt, keys 4*(l/16)..+3 of the first block, then of the second
 };
-
-// Where one step's blocks live: kb[j] is the R tile of key block j, vtb[j] the T tile of its values.
-struct StepDesc {
-    const bf16* kb[NB];
-    const bf16* vtb[NB];
-};
-
-__device__ __forceinline__ void load_step(KvRegs& t, const StepDesc& d, int lane) {
-#pragma unroll
-    for (int j = 0; j < NB; j++) {
-        t.k[j][0] = ld16(d.kb[j] + lane * 8);
-        t.k[j][1] = ld16(d.kb[j] + 512 + lane * 8);
-    }
-    // (the two halves of an operand are loaded one after the other so that they land in adjacent registers)
-#pragma unroll
-    for (int c = 0; c < NB / 2; c++)
-#pragma unroll
-        for (int dt = 0; dt < 4; dt++)
-            t.v[c][dt] = cat(ld8(d.vtb[2 * c] + dt * 256 + lane * 4), ld8(d.vtb[2 * c + 1] + dt * 256 + lane * 4));
-}
 
 __device__ __forceinline__ void init_state(SoftmaxState& st) {
     st.m2 = 0.f;
@@ -131,9 +111,12 @@ __device__ __forceinline__ void accumulate(SoftmaxState& st, const float x[NB][4
             st.acc[dt] = mfma_bf16(t.v[c][dt], bp[c], st.acc[dt]);
 }
 
-__device__ __forceinline__ void compute_step(SoftmaxState& st, const bf16x8 bq[2], const KvRegs& t) {
+// in0, in1 (wave-uniform): whether the query block reads the step's first / second block
+__device__ __forceinline__ void compute_step(SoftmaxState& st, const bf16x8 bq[2], const KvRegs& t, bool in0 = true, bool in1 = true) {
     float x[NB][4];
     exponents(x, st, bq, t);
+    if (!in0) x[0][0] = x[0][1] = x[0][2] = x[0][3] = -INFINITY;
+    if (!in1) x[1][0] = x[1][1] = x[1][2] = x[1][3] = -INFINITY;
     const float top = largest(x);
     if (__ballot(top > kMaxSlack) != 0) move_reference(st, x, top);
     accumulate(st, x, t);
@@ -156,7 +139,7 @@ __device__ __forceinline__ void compute_step2(SoftmaxState& sa, SoftmaxState& sb
 
 // Operands of one step out of the workgroup's LDS copy of shared blocks (4 KB per block: R tile
 // of the keys, then T tile of the values).
-__device__ __forceinline__ void load_step_lds(KvRegs& t, const bf16* blocks, int lane) {
+__device__ __forceinline__ void load_step_shared(KvRegs& t, const bf16* blocks, int lane) {
 #pragma unroll
     for (int j = 0; j < NB; j++) {
         t.k[j][0] = lds_ld16(blocks + j * 2 * kTile + lane * 8);
@@ -171,6 +154,15 @@ __device__ __forceinline__ void load_step_lds(KvRegs& t, const bf16* blocks, int
             __builtin_amdgcn_sched_barrier(0);    // (keeps the two reads one paired LDS read: paired with any other read they need moves)
         }
 }
+// The values of a pair of fine blocks out of the wave's own copy of their R tiles: the transposing read makes the T operands.
+// (So the tokens' values need no T tile in memory, which would be a tenth of all that the pooling pass moves.)
+__device__ __forceinline__ void load_v_fine(KvRegs& t, const bf16* tiles, int lane) {
+#pragma unroll
+    for (int c = 0; c < NB / 2; c++)
+#pragma unroll
+        for (int dt = 0; dt < 4; dt++)
+            t.v[c][dt] = cat(lds_t_operand(tiles + (2 * c) * kTile, dt, lane), lds_t_operand(tiles + (2 * c + 1) * kTile, dt, lane));
+}
 
 __device__ __forceinline__ void finish_query_block(const llsa_attn_fwd_args& a, const SoftmaxState& st, int bh, int b, int h, int g, int lane) {
     const int r = lane & 15, quad = lane >> 4;
@@ -182,35 +174,30 @@ __device__ __forceinline__ void finish_query_block(const llsa_attn_fwd_args& a, 
     if (quad == 0) a.lse[(int64_t)bh * a.N + g * kBlk + r] = (st.m2 + __builtin_amdgcn_logf(L)) * kLn2;
 }
 
-// One wave per query block, four consecutive query blocks per workgroup.
+// Q sibling query blocks per wave, 4 Q consecutive query blocks per workgroup.
 //
-// The pooled blocks -- the level-1 pooled tokens of the parent's coarse blocks and the coarsest
-// level -- are the same for all query blocks of a 256-token parent, hence for the four waves of
-// the workgroup: they are fetched once per workgroup, kGroup at a time, straight into LDS (two
-// buffers, the next fetch in flight during the arithmetic), and every wave reads its operands
-// from there.  The T fine blocks differ from query block to query block: every wave then walks
-// its own in steps of NB blocks, the loads of step t+1 issued before the arithmetic of step t
-// (two register buffers, ping-pong).  The shared phase comes first because the compiler drains
-// the whole vector-memory queue at every wait while a copy into LDS is outstanding, which would
-// undo the register ping-pong.  This is what bounds the kernel: without the sharing every wave
-// pulls all of its 4 KB per block through the L2, and the L2's bandwidth, not the MFMA, sets the time.
-__global__ __launch_bounds__(256, 4) void attn_fwd_kernel(llsa_attn_fwd_args a) {
+// The pooled blocks -- the selected blocks of every pooled level below the coarsest and the coarsest level itself -- are
+// the same for all query blocks of a 256-token group, hence for the four waves of the workgroup: they are fetched once
+// per workgroup, kGroup at a time, straight into LDS (two buffers, the next fetch in flight during the arithmetic).
+// The T fine blocks differ from query block to query block, but siblings have many in common (of 2 x 16 entries 24 are
+// different on image-like inputs; four siblings per wave would fetch 34 of 64, but leave two long waves per SIMD: 83 against
+// 62 us for 12 x 16384 tokens): the wave merges its lists (merge_lists) and walks the union, two blocks per step, every
+// block fetched once and multiplied with the query blocks that selected it.  What bounds the fine part is the rate at which
+// tiles arrive from the L2, and waves enough to keep the fetches in flight.
+template <int Q, int R>
+__global__ __launch_bounds__(256, Q == 1 ? 4 : 3) void attn_fwd_kernel(llsa_attn_fwd_args a) {
     static_assert(NB == 2 && kGroup == 4, "the shared phase reads an LDS buffer of four blocks as two steps of two");
     __shared__ __align__(16) bf16 sh[2][kGroup][2 * kTile];
+    __shared__ int order[4][R * kWave];
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int N1 = a.N / kBlk;
+    const int N1 = a.N / kBlk, T = a.T;
     const int lid = xcd_logical_id();
-    const int g = (lid % (int)gridDim.x) * 4 + wave;          // < N1: the host checks N1 % 4 == 0
+    const int g = (lid % (int)gridDim.x) * (4 * Q) + Q * wave;        // query blocks g .. g + Q - 1 (the host checks N1 % 4 Q == 0)
     const int bh = lid / (int)gridDim.x, b = bh / a.H, h = bh % a.H;
 
     const bf16* kr = (const bf16*)a.kr + (int64_t)bh * N1 * kTile;
-    const bf16* vt = (const bf16*)a.vt + (int64_t)bh * N1 * kTile;
-    const int* ip = a.idx + ((int64_t)bh * N1 + g) * a.T;
-
-    // Shared list: for every pooled level below the coarsest the blocks its ancestor group selected (level 1 first),
-    // then every block of the coarsest level.  The selected entries of all levels together (at most 64: the host
-    // checks) live one per lane, entry i in lane i.
+    const bf16* vr = (const bf16*)a.vt + (int64_t)bh * N1 * kTile;
     SharedList sl = shared_list(a.lvl, a.levels, a.N, bh, g, lane);
     bf16* const sh0 = &sh[0][0][0];
     auto issue_group = [&](int grp) __attribute__((always_inline)) {   // this wave brings in block kGroup*grp + wave
@@ -225,185 +212,105 @@ __global__ __launch_bounds__(256, 4) void attn_fwd_kernel(llsa_attn_fwd_args a) 
     };
     const int n_groups = sl.n_blocks / kGroup;                // every level's count is a multiple of kGroup (host checks)
     issue_group(0);
-    int mine = (lane < min(kWave, a.T)) ? ip[lane] : 0;       // first 64 fine indices, entry i in lane i
+    const int* ip = a.idx + ((int64_t)bh * N1 + g) * T;
+    MergedLists<Q, R> ml = merge_lists<Q, R>(ip, min(T, kWave * R / Q), N1, lane, order[wave]);
 
-    bf16x8 bq[2];
-    {
-        const bf16* qp = (const bf16*)a.qr + ((int64_t)bh * N1 + g) * kTile + lane * 8;
-        bq[0] = ld16(qp);       // 1/sqrt(64) is a power of two: scaling q before the product (as the
-        bq[1] = ld16(qp + 512); // reference does) equals scaling the fp32 scores, done in the exponent
+    bf16x8 bq[Q][2];
+    SoftmaxState st[Q];
+#pragma unroll
+    for (int u = 0; u < Q; u++) {
+        const bf16* qp = (const bf16*)a.qr + ((int64_t)bh * N1 + g + u) * kTile + lane * 8;
+        bq[u][0] = ld16(qp);       // 1/sqrt(64) is a power of two: scaling q before the product (as the
+        bq[u][1] = ld16(qp + 512); // reference does) equals scaling the fp32 scores, done in the exponent
+        init_state(st[u]);
     }
-    SoftmaxState st;
-    init_state(st);
-
-    KvRegs ra, rb;
+    auto step_all = [&](const KvRegs& t) __attribute__((always_inline)) {    // the operands in t against every query block of the wave
+        if constexpr (Q == 1) compute_step(st[0], bq[0], t);
+        else
+#pragma unroll
+            for (int u = 0; u < Q; u += 2) compute_step2(st[u], st[u + 1], bq[u], bq[u + 1], t);
+    };
 
     // ---- shared blocks, out of LDS.  The barrier at the top of round grp says two things: every
     // wave's part of group grp has landed, and every wave is done reading the other buffer
-    // (group grp - 1), which the next fetch overwrites.
+    // (group grp - 1), which the next fetch overwrites.  (LDS reads of a group come before the next fetch: the compiler
+    // makes every LDS read wait for all copies into LDS that were issued before it.)
     float w_prev = 1.f;
     for (int grp = 0; grp < n_groups; grp++) {
         wait_vm0();
         __syncthreads();
         // weight(previous segment) / weight(this one); nothing is accumulated before group 0
         const float w_here = a.lvl[shared_level(a.lvl, a.levels, kGroup * grp)].w;
-        if (grp > 0 && w_here != w_prev) rescale(st, w_prev / w_here);
-        w_prev = w_here;
-        // (LDS reads first: the compiler makes every LDS read wait for all copies into LDS that
-        // were issued before it, which would serialise the next fetch with the arithmetic of this group)
-        load_step_lds(ra, &sh[grp & 1][0][0], lane);
-        load_step_lds(rb, &sh[grp & 1][NB][0], lane);
-        if (grp + 1 < n_groups) issue_group(grp + 1);
-        if (grp == 0) start_reference(st, bq, ra);
-        compute_step(st, bq, ra);
-        compute_step(st, bq, rb);
-    }
-    rescale(st, w_prev);                                      // fine tokens weigh 1
-
-    wait_all_mem();     // nothing is in flight here: said for the compiler (see wait_all_mem)
-    // ---- fine blocks, private to the wave.  Their indices are fetched 64 at a time, entry i into
-    // lane i, and handed out with readlane (a copy into LDS counts as a store for the compiler,
-    // after which it no longer turns uniform loads into scalar loads; a vector load inside the
-    // pipelined loop would wait for every tile load issued before it).
-    for (int c0 = 0; c0 < a.T; c0 += kWave) {
-        const int cn = min(kWave, a.T - c0);                  // a multiple of 4: an even number of steps
-        if (c0 > 0) mine = (lane < cn) ? ip[c0 + lane] : 0;
-        const int n_fine = cn / NB;
-        auto describe = [=](int t, StepDesc& d) __attribute__((always_inline)) {
-#pragma unroll
-            for (int j = 0; j < NB; j++) {
-                const int blk = clampi(__builtin_amdgcn_readlane(mine, NB * t + j), 0, N1 - 1);
-                d.kb[j] = kr + (int64_t)blk * kTile;
-                d.vtb[j] = vt + (int64_t)blk * kTile;
-            }
-        };
-        // The prefetch is unconditional (past the end it re-reads the last step) so that the loop
-        // body is straight-line code: with the loads inside a branch the compiler has to drain the
-        // memory queue (s_waitcnt vmcnt(0)) before every step and the overlap is lost.
-        StepDesc d;
-        describe(0, d);
-        load_step(ra, d, lane);
-        for (int t = 0; t < n_fine; t += 2) {
-            describe(min(t + 1, n_fine - 1), d);
-            load_step(rb, d, lane);
-            compute_step(st, bq, ra);
-            if (t + 1 >= n_fine) break;
-            describe(min(t + 2, n_fine - 1), d);
-            load_step(ra, d, lane);
-            compute_step(st, bq, rb);
-        }
-    }
-
-    finish_query_block(a, st, bh, b, h, g, lane);
-}
-
-// ---------------------------------------------------------------------------------------
-// Two sibling query blocks per wave (topk <= 32 R, R = 1 or 2).  Both walk the same pooled blocks, and on coherent inputs most
-// of their fine blocks coincide, so every operand tile that both need is fetched once and multiplied twice: the
-// wave first sorts the two fine lists into [blocks both selected | only the first | only the second] and walks
-// that list in steps of NB blocks, a step of the first part feeding both soft-max states.  What bounds these
-// kernels is the rate at which tiles arrive from the L2, and this removes a quarter to a half of them.
-// A row that names a block twice keeps the plain walk (nothing is shared).
-// ---------------------------------------------------------------------------------------
-
-template <int R>
-__global__ __launch_bounds__(256, 3) void attn_fwd_pair_kernel(llsa_attn_fwd_args a) {
-    static_assert(NB == 2 && kGroup == 4, "the shared phase reads an LDS buffer of four blocks as two steps of two");
-    __shared__ __align__(16) bf16 sh[2][kGroup][2 * kTile];
-    __shared__ int order[4][R * kWave];
-    const int lane = threadIdx.x & 63;
-    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int N1 = a.N / kBlk, T = a.T;
-    const int lid = xcd_logical_id();
-    const int g = (lid % (int)gridDim.x) * 8 + 2 * wave;      // query blocks g and g + 1 (the host checks N1 % 8 == 0)
-    const int bh = lid / (int)gridDim.x, b = bh / a.H, h = bh % a.H;
-
-    const bf16* kr = (const bf16*)a.kr + (int64_t)bh * N1 * kTile;
-    const bf16* vt = (const bf16*)a.vt + (int64_t)bh * N1 * kTile;
-    const int* ip = a.idx + ((int64_t)bh * N1 + g) * T;
-
-    SharedList sl = shared_list(a.lvl, a.levels, a.N, bh, g, lane);
-    bf16* const sh0 = &sh[0][0][0];
-    auto issue_group = [&](int grp) __attribute__((always_inline)) {
-        const SharedBlock sb = shared_block(sl, a.lvl, a.levels, a.N, bh, kGroup * grp + wave);
-        const bf16* kb = (const bf16*)a.lvl[sb.level].kr + sb.tile;
-        const bf16* vb = (const bf16*)a.lvl[sb.level].vt + sb.tile;
-        bf16* dst = sh0 + ((grp & 1) * kGroup + wave) * (2 * kTile);
-        copy16_global_to_lds(kb + lane * 8, dst);
-        copy16_global_to_lds(kb + 512 + lane * 8, dst + 512);
-        copy16_global_to_lds(vb + lane * 8, dst + kTile);
-        copy16_global_to_lds(vb + 512 + lane * 8, dst + kTile + 512);
-    };
-    const int n_groups = sl.n_blocks / kGroup;
-    issue_group(0);
-
-    // ---- the two fine lists, sorted into [both | only the first | only the second]; entry i ends in lane i
-    const PairOrder<R> po = pair_order<R>(ip, T, N1, lane, order[wave]);
-    const int steps_both = po.n_both / NB, steps_only = (T - po.n_both) / NB, n_steps = steps_both + 2 * steps_only;
-
-    bf16x8 bq[2][2];
-#pragma unroll
-    for (int u = 0; u < 2; u++) {
-        const bf16* qp = (const bf16*)a.qr + ((int64_t)bh * N1 + g + u) * kTile + lane * 8;
-        bq[u][0] = ld16(qp);
-        bq[u][1] = ld16(qp + 512);
-    }
-    SoftmaxState st[2];
-    init_state(st[0]);
-    init_state(st[1]);
-    KvRegs ra, rb;
-
-    float w_prev = 1.f;
-    for (int grp = 0; grp < n_groups; grp++) {
-        wait_vm0();
-        __syncthreads();
-        const float w_here = a.lvl[shared_level(a.lvl, a.levels, kGroup * grp)].w;
         if (grp > 0 && w_here != w_prev) {
-            rescale(st[0], w_prev / w_here);
-            rescale(st[1], w_prev / w_here);
+#pragma unroll
+            for (int u = 0; u < Q; u++) rescale(st[u], w_prev / w_here);
         }
         w_prev = w_here;
-        load_step_lds(ra, &sh[grp & 1][0][0], lane);
-        load_step_lds(rb, &sh[grp & 1][NB][0], lane);
+        const bf16* blk = &sh[grp & 1][0][0];
+        KvRegs t, t2;
+        load_step_shared(t, blk, lane);
+        load_step_shared(t2, blk + NB * 2 * kTile, lane);
         if (grp + 1 < n_groups) issue_group(grp + 1);
         if (grp == 0) {
-            start_reference(st[0], bq[0], ra);
-            start_reference(st[1], bq[1], ra);
-        }
-        compute_step2(st[0], st[1], bq[0], bq[1], ra);
-        compute_step2(st[0], st[1], bq[0], bq[1], rb);
-    }
-    rescale(st[0], w_prev);                                   // fine tokens weigh 1
-    rescale(st[1], w_prev);
-    wait_all_mem();
-
-    auto describe = [=](int t, StepDesc& d) __attribute__((always_inline)) {
 #pragma unroll
-        for (int j = 0; j < NB; j++) {
-            const int blk = po.entry(NB * t + j);
-            d.kb[j] = kr + (int64_t)blk * kTile;
-            d.vtb[j] = vt + (int64_t)blk * kTile;
+            for (int u = 0; u < Q; u++) start_reference(st[u], bq[u], t);
+        }
+        step_all(t);
+        step_all(t2);
+    }
+#pragma unroll
+    for (int u = 0; u < Q; u++) rescale(st[u], w_prev);       // fine tokens weigh 1
+    __syncthreads();                                          // the shared copy is dead: its LDS becomes private slots
+
+    // ---- fine blocks, two per step: the keys of step s + 1 are loaded into registers and its values copied into the wave's other
+    // LDS slot while step s is worked on.  (The LDS reads of a step come before the next fetch, see above; the products with
+    // the keys do not wait for them.)  Nothing may be in flight when the wave ends (a copy landing in LDS that already
+    // belongs to another workgroup), so the last step fetches nothing.
+    bf16* const slots = sh0 + wave * (4 * kTile);             // two slots of the V tiles of two blocks
+    auto fine = [&]() __attribute__((always_inline)) {
+        const int n_steps = (ml.n + 1) / 2;
+        auto fetch = [&](int s, KvRegs& dst) __attribute__((always_inline)) {
+            bf16* slot = slots + (s & 1) * (2 * kTile);
+#pragma unroll
+            for (int j = 0; j < 2; j++) {
+                const int64_t at = (int64_t)ml.block(min(2 * s + j, ml.n - 1)) * kTile + lane * 8;
+                dst.k[j][0] = ld16(kr + at);
+                dst.k[j][1] = ld16(kr + at + 512);
+                copy16_global_to_lds(vr + at, slot + j * kTile);
+                copy16_global_to_lds(vr + at + 512, slot + j * kTile + 512);
+            }
+        };
+        auto work = [&](int s, KvRegs& cur, KvRegs& nxt) __attribute__((always_inline)) {
+            const unsigned m0 = ml.rows(2 * s), m1 = 2 * s + 1 < ml.n ? ml.rows(2 * s + 1) : 0u;
+            wait_vm0();
+            load_v_fine(cur, slots + (s & 1) * (2 * kTile), lane);
+            if (s + 1 < n_steps) fetch(s + 1, nxt);
+            if ((m0 & m1) == (1u << Q) - 1u) {
+                step_all(cur);
+            } else {
+#pragma unroll
+                for (int u = 0; u < Q; u++) {
+                    const bool in0 = (m0 >> u) & 1u, in1 = (m1 >> u) & 1u;
+                    if (in0 || in1) compute_step(st[u], bq[u], cur, in0, in1);
+                }
+            }
+        };
+        KvRegs ra, rb;
+        fetch(0, ra);
+        for (int s = 0; s < n_steps; s += 2) {
+            work(s, ra, rb);
+            if (s + 1 < n_steps) work(s + 1, rb, ra);
         }
     };
-    auto work = [&](int t, const KvRegs& regs) __attribute__((always_inline)) {
-        if (t < steps_both) compute_step2(st[0], st[1], bq[0], bq[1], regs);
-        else if (t < steps_both + steps_only) compute_step(st[0], bq[0], regs);
-        else compute_step(st[1], bq[1], regs);
-    };
-    StepDesc d;
-    describe(0, d);
-    load_step(ra, d, lane);
-    for (int t = 0; t < n_steps; t += 2) {
-        describe(min(t + 1, n_steps - 1), d);
-        load_step(rb, d, lane);
-        work(t, ra);
-        if (t + 1 >= n_steps) break;
-        describe(min(t + 2, n_steps - 1), d);
-        load_step(ra, d, lane);
-        work(t + 1, rb);
+    fine();
+    if constexpr (Q == 1) {                                   // longer lists: 64 entries at a time
+        for (int c0 = kWave * R; c0 < T; c0 += kWave * R) {
+            ml = merge_lists<Q, R>(ip + c0, min(T - c0, kWave * R), N1, lane, order[wave]);
+            fine();
+        }
     }
-    finish_query_block(a, st[0], bh, b, h, g, lane);
-    finish_query_block(a, st[1], bh, b, h, g + 1, lane);
+#pragma unroll
+    for (int u = 0; u < Q; u++) finish_query_block(a, st[u], bh, b, h, g + u, lane);
 }
 
 }  // namespace llsa
@@ -437,13 +344,20 @@ extern "C" int llsa_attn_fwd(const llsa_attn_fwd_args* a, void* stream) {
                  LLSA_POOLED_TOPK_MAX);
     LLSA_REQUIRE(aligned16(a->qr) && aligned16(a->kr) && aligned16(a->vt) && aligned16(a->o), "attn_fwd: tensors must be 16-byte aligned");
     LLSA_REQUIRE((a->sob % 4 == 0) && (a->soh % 4 == 0) && (a->son % 4 == 0), "attn_fwd: rows of o must be 8-byte aligned");
-    const int N1 = a->N / 16;
-    if (a->T <= kPairMaxTopk && N1 % 8 == 0 && (int64_t)N1 / 8 * a->B * a->H >= kPairMinGroups)
-        if (a->T <= 32)
-            hipLaunchKernelGGL(HIP_KERNEL_NAME(attn_fwd_pair_kernel<1>), dim3(N1 / 8, a->B * a->H), dim3(256), 0, (hipStream_t)stream, *a);
-        else
-            hipLaunchKernelGGL(HIP_KERNEL_NAME(attn_fwd_pair_kernel<2>), dim3(N1 / 8, a->B * a->H), dim3(256), 0, (hipStream_t)stream, *a);
-    else
-        hipLaunchKernelGGL(attn_fwd_kernel, dim3((N1 + 3) / 4, a->B * a->H), dim3(256), 0, (hipStream_t)stream, *a);
+    const int N1 = a->N / 16, BH = a->B * a->H;
+    // Two query blocks per wave halve the LDS reads of the pooled blocks and save a quarter of the fine fetches; one per wave
+    // leaves more and shorter waves.  Two win where the pooled blocks are most of the walk (11 x 32768 tokens, topk 8,
+    // 128 pooled blocks: 273 against 295 us) and on large grids (48 x 16384: 263 against 280), one elsewhere (12 x 16384: 62
+    // against 68, 3 x 49152 at topk 64 144 against 155).
+    int64_t shared = listed, coarsest = a->N / 256;
+    for (int l = 1; l < a->levels; l++) coarsest /= 16;
+    shared += coarsest;
+    const int64_t groups = (int64_t)N1 / 8 * BH;
+    const bool pairs = a->T <= kPairMaxTopk && N1 % 8 == 0 && groups >= kPairMinGroups && (shared >= 4 * a->T || groups >= 2048);
+    const dim3 grid(N1 / (pairs ? 8 : 4), BH);
+    const hipStream_t st = (hipStream_t)stream;
+    if (!pairs) hipLaunchKernelGGL(HIP_KERNEL_NAME(attn_fwd_kernel<1, 1>), grid, dim3(256), 0, st, *a);
+    else if (a->T <= 32) hipLaunchKernelGGL(HIP_KERNEL_NAME(attn_fwd_kernel<2, 1>), grid, dim3(256), 0, st, *a);
+    else hipLaunchKernelGGL(HIP_KERNEL_NAME(attn_fwd_kernel<2, 2>), grid, dim3(256), 0, st, *a);
     return launch_status("attn_fwd");
 }

@@ -196,7 +196,7 @@ struct Layout {
     int L, chunk;
     int32_t topk[kL];
     int64_t pq[kL + 1], pk[kL + 1], pv[kL + 1];             // pooled rows, index = level
-    int64_t qr, kr, vr = -1, vt;                            // operand tiles of the tokens
+    int64_t qr, kr, vr;                                     // operand tiles of the tokens
     int64_t pkr[kL + 1], pvr[kL + 1], pvt[kL + 1];          // and of the pooled levels
     int64_t sel[kL], off[kL], flat[kL], inv[kL], work = -1; // sel[0]: fine blocks per query block, sel[l]: blocks of level l per group of 16^(l+1) queries
     int64_t lse, bytes;
@@ -220,8 +220,7 @@ struct Layout {
         for (int l = 1; l <= L; l++) pv[l] = take(n[l] * 128);
         qr = take(n[1] * 2048);
         kr = take(n[1] * 2048);
-        vr = take(n[1] * 2048, grad);
-        vt = take(n[1] * 2048);
+        vr = take(n[1] * 2048);
         for (int l = 1; l <= L; l++) {
             pkr[l] = take(n[l + 1] * 2048);
             pvr[l] = take(n[l + 1] * 2048, grad);
@@ -419,7 +418,7 @@ Tensor attend(const std::shared_ptr<Library>& lib, const Tensor& q_in, const Ten
                     p.x = x.data_ptr(); p.sxb = x.stride(0); p.sxh = x.stride(1); p.sxn = x.stride(2);
                     p.rope = i < 2 && freq.defined();
                     p.xr = pa(i == 0 ? y.qr : i == 1 ? y.kr : y.vr);
-                    if (i == 2) p.xt = pa(y.vt);
+                    p.stream = grad;
                     const Tensor& g = i == 0 ? gq : gk;
                     if (i < 2 && g.defined()) {
                         p.gamma = g.data_ptr<float>();
@@ -470,7 +469,7 @@ Tensor attend(const std::shared_ptr<Library>& lib, const Tensor& q_in, const Ten
         if (beside) hip_check(hipEventRecord(side_events(dev).ready, static_cast<hipStream_t>(stream)));
 
         llsa_attn_fwd_args f{};
-        f.qr = pa(y.qr); f.kr = pa(y.kr); f.vt = pa(y.vt); f.idx = ints(y.sel[0]);
+        f.qr = pa(y.qr); f.kr = pa(y.kr); f.vt = pa(y.vr); f.idx = ints(y.sel[0]);
         f.o = o.data_ptr(); f.sob = o.stride(0); f.soh = o.stride(1); f.son = o.stride(2);
         f.lse = static_cast<float*>(pa(y.lse));
         f.B = b; f.H = h; f.N = static_cast<int32_t>(N); f.T = y.topk[0]; f.levels = L;

@@ -213,60 +213,99 @@ __device__ __forceinline__ SharedBlock shared_block(const SharedList& sl, const 
     return sb;
 }
 
-// The fine lists of two sibling query blocks (rows ip[0..T) and ip[T..2T), T <= 32 R), sorted into
-// [blocks both rows name | only the first | only the second]: entry i of that order ends in lane i % 64 of register i / 64
-// (2T - n_both entries), indices clamped to [0, N1).  n_both is even (an odd common block out is listed once for each row).
-// A row that names a block twice shares nothing (n_both = 0).  `scratch`: R * kWave ints of LDS private to the wave.
-constexpr int kPairMaxTopk = 64;
-// Fewer groups of eight query blocks than this: one query block per wave.  The chip then has room for all of the waves either way
-// (four workgroups of four single blocks or three of four pairs per CU), and a wave of one block has half the serial chain:
-// 6 x 1024 tokens, topk 8: forward 8.7 -> 5.9 us, dQ 14.0 -> 8.5; 6 x 8192, topk 16: step 147 -> 138 us; even at 8 x 8192.
-constexpr int kPairMinGroups = 512;
-template <int R>
-struct PairOrder {
-    int mine[R];
-    int n_both;
-    __device__ __forceinline__ int entry(int i) const {       // i is wave-uniform
-        const int v = __builtin_amdgcn_readlane(mine[0], i & (kWave - 1));
+// The fine lists of Q sibling query blocks (ip: Q rows of T entries one after the other, Q * T <= 64 R), merged: the
+// distinct blocks, each with the set of rows that name it (bit u: row u), ordered by that set.  A row that names a block twice
+// keeps all lists as they are (every entry on its own).  Entry i of the result sits in lane i % 64 of register i / 64.
+// `scratch`: 64 R ints of LDS private to the wave.
+template <int Q, int R>
+struct MergedLists {
+    int packed[R];                                            // block | set << 24 (there are fewer than 2^21 blocks)
+    int n;
+    __device__ __forceinline__ int at(int i) const {          // i is wave-uniform
+        const int v = __builtin_amdgcn_readlane(packed[0], i & (kWave - 1));
         if (R == 1) return v;
-        const int o = __builtin_amdgcn_readlane(mine[R - 1], i & (kWave - 1));
+        const int o = __builtin_amdgcn_readlane(packed[R - 1], i & (kWave - 1));
         return i < kWave ? v : o;
     }
+    __device__ __forceinline__ int block(int i) const { return at(i) & 0xffffff; }
+    __device__ __forceinline__ unsigned rows(int i) const { return (unsigned)at(i) >> 24; }
 };
-template <int R>
-__device__ __forceinline__ PairOrder<R> pair_order(const int* ip, int T, int N1, int lane, int* scratch) {
-    const int first = (lane < T) ? clampi(ip[lane], 0, N1 - 1) : -1 - lane;       // (distinct negative fillers)
-    const int second = (lane < T) ? clampi(ip[T + lane], 0, N1 - 1) : -65 - lane;
-    bool in_second = false, in_first = false, twice = false;
-    for (int j = 0; j < T; j++) {
-        const int fj = __builtin_amdgcn_readlane(first, j), sj = __builtin_amdgcn_readlane(second, j);
-        in_second |= first == sj;
-        in_first |= second == fj;
-        twice |= (first == fj && lane != j) || (second == sj && lane != j);
+template <int Q, int R>
+__device__ __forceinline__ MergedLists<Q, R> merge_lists(const int* ip, int T, int N1, int lane, int* scratch) {
+    static_assert(R <= 2, "entries sit in one or two registers");
+    MergedLists<Q, R> ml;
+    int v[R], row[R];
+#pragma unroll
+    for (int k = 0; k < R; k++) {
+        const int i = k * kWave + lane;
+        v[k] = i < Q * T ? clampi(ip[i], 0, N1 - 1) : -1 - i;         // (distinct negative fillers)
+        row[k] = 0;
+#pragma unroll
+        for (int u = 1; u < Q; u++) row[k] += i >= u * T ? 1 : 0;
     }
-    if (__ballot(twice) != 0) in_second = in_first = false;
-    unsigned long long both = __ballot(in_second);
-    if (__popcll(both) & 1) {
-        const int last = 63 - __builtin_clzll(both);
-        const int dropped = __builtin_amdgcn_readlane(first, last);
-        in_second = in_second && lane != last;
-        in_first = in_first && second != dropped;
-        both &= ~(1ull << last);
+    if constexpr (Q == 1) {
+#pragma unroll
+        for (int k = 0; k < R; k++) ml.packed[k] = v[k] | (1 << 24);
+        ml.n = T;
+        return ml;
     }
-    const int n_both = __popcll(both), n_only = T - n_both;
+    unsigned long long in[Q][R], twice = 0;                   // which lanes' blocks row u names
+#pragma unroll
+    for (int u = 0; u < Q; u++)
+#pragma unroll
+        for (int k = 0; k < R; k++) in[u][k] = 0;
+#pragma unroll
+    for (int u = 0; u < Q; u++)
+#pragma unroll 1
+        for (int s = 0; s < T; s++) {
+            const int j = u * T + s;
+            int o = __builtin_amdgcn_readlane(v[0], j & (kWave - 1));
+            if (R > 1) {
+                const int o1 = __builtin_amdgcn_readlane(v[R - 1], j & (kWave - 1));
+                o = j < kWave ? o : o1;
+            }
+#pragma unroll
+            for (int k = 0; k < R; k++) {
+                const unsigned long long eq = __ballot(v[k] == o);
+                twice |= in[u][k] & eq & __ballot(row[k] == u);       // named by this row before
+                in[u][k] |= eq;
+            }
+        }
+    int set[R];
+    bool lead[R];
+#pragma unroll
+    for (int k = 0; k < R; k++) {
+        set[k] = 0;
+#pragma unroll
+        for (int u = 0; u < Q; u++) set[k] |= ((in[u][k] >> lane) & 1ull) ? 1 << u : 0;
+        if (twice != 0) set[k] = 1 << row[k];
+        lead[k] = k * kWave + lane < Q * T && (set[k] & ((1 << row[k]) - 1)) == 0;
+    }
     const unsigned long long below = (1ull << lane) - 1ull;
-    const unsigned long long only1 = __ballot(lane < T && !in_second), only2 = __ballot(lane < T && !in_first);
-    if (lane < T) scratch[in_second ? __popcll(both & below) : n_both + __popcll(only1 & below)] = first;
-    if (lane < T && !in_first) scratch[n_both + n_only + __popcll(only2 & below)] = second;
+    int n = 0;
+#pragma unroll 1
+    for (int c = (1 << Q) - 1; c > 0; c--) {
+#pragma unroll
+        for (int k = 0; k < R; k++) {
+            const unsigned long long m = __ballot(lead[k] && set[k] == c);
+            if (lead[k] && set[k] == c) scratch[n + __popcll(m & below)] = v[k] | (c << 24);
+            n += __popcll(m);
+        }
+    }
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
     __builtin_amdgcn_wave_barrier();
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-    PairOrder<R> po;
 #pragma unroll
-    for (int k = 0; k < R; k++) po.mine[k] = scratch[k * kWave + lane];
-    po.n_both = n_both;
-    return po;
+    for (int k = 0; k < R; k++) ml.packed[k] = scratch[k * kWave + lane];
+    ml.n = n;
+    return ml;
 }
+// Two query blocks per wave are possible up to this topk (their lists then fit two registers) ...
+constexpr int kPairMaxTopk = 64;
+// ... and considered from this many groups of eight query blocks on.  Below, the chip has room for all of the waves either way
+// (four workgroups of four single blocks or three of four pairs per CU), and a wave of one block has half the serial chain:
+// 6 x 1024 tokens, topk 8: forward 8.7 -> 5.9 us, dQ 14.0 -> 8.5; 6 x 8192, topk 16: step 147 -> 138 us; even at 8 x 8192.
+constexpr int kPairMinGroups = 512;
 
 // 16- and 8-byte reads that are LDS reads by construction (ds_read_b128 / ds_read_b64)
 __device__ __forceinline__ bf16x8 lds_ld16(const bf16* p) {

@@ -101,8 +101,7 @@ __device__ __forceinline__ void rms_norm_rows(bf16x8* xv, const float (&g)[8], f
     }
 }
 
-// STREAM (a launch that writes both tiles of a tensor, i.e. the backward's too): the rows are read past the caches.  In a
-// training step nothing reads them again, and the tiles, which the attention kernels gather from the caches right
+// STREAM (llsa_pool_item.stream): the rows are read past the caches.  In a training step nothing reads them again, and the tiles, which the attention kernels gather from the caches right
 // afterwards, have the more room (24 x 4096 and 15 x 7168 tokens: 2 % of the step, 6 x 65536: 1 %).  Writing the tiles
 // that way makes this pass faster still (49 -> 43 us) and every reader slower by more.
 template <bool NORM, bool STREAM>
@@ -412,12 +411,12 @@ extern "C" int llsa_pool_pyramid_fwd(const llsa_pool_item* items, int n_items, c
     for (int i = 0; i < n_items; i++) norm = norm || items[i].gamma != nullptr;
     p.n_items = n_items;
     dim3 grid((max_n + 255) / 256 * n_items, B * H);
-    bool both = false;
-    for (int i = 0; i < n_items; i++) both = both || (items[i].xr != nullptr && items[i].xt != nullptr);
+    bool past = false;
+    for (int i = 0; i < n_items; i++) past = past || items[i].stream != 0;
     const hipStream_t st = (hipStream_t)stream;
-    if (norm && both) hipLaunchKernelGGL(HIP_KERNEL_NAME(pool_pyramid_kernel<true, true>), grid, dim3(128), 0, st, p);
+    if (norm && past) hipLaunchKernelGGL(HIP_KERNEL_NAME(pool_pyramid_kernel<true, true>), grid, dim3(128), 0, st, p);
     else if (norm) hipLaunchKernelGGL(HIP_KERNEL_NAME(pool_pyramid_kernel<true, false>), grid, dim3(128), 0, st, p);
-    else if (both) hipLaunchKernelGGL(HIP_KERNEL_NAME(pool_pyramid_kernel<false, true>), grid, dim3(128), 0, st, p);
+    else if (past) hipLaunchKernelGGL(HIP_KERNEL_NAME(pool_pyramid_kernel<false, true>), grid, dim3(128), 0, st, p);
     else hipLaunchKernelGGL(HIP_KERNEL_NAME(pool_pyramid_kernel<false, false>), grid, dim3(128), 0, st, p);
     return launch_status("pool_pyramid");
 }

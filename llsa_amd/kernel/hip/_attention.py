@@ -50,7 +50,7 @@ def _tiles(tiles, need):
 
 def attn_fwd(q, k, v, pk, pv, indices, token_weight, pk2=None, pv2=None, p_indices=None, token_weight_2=1.0,
              tiles=None):
-    """Forward.  `tiles` may carry operand tiles the caller already has (keys qr, kr, vt, pkr, pvt,
+    """Forward.  `tiles` may carry operand tiles the caller already has (keys qr, kr, vr, pkr, pvt,
     pk2r, pv2t); the rest are computed here.  Returns (o, lse)."""
     levels = 1 if pk2 is None else 2
     lib = lib_for(q, k, v, pk, pv, pk2, pv2)
@@ -60,7 +60,7 @@ def attn_fwd(q, k, v, pk, pv, indices, token_weight, pk2=None, pv2=None, p_indic
     B, H, N, D = q.shape
     T = indices.shape[-1]
     T2 = p_indices.shape[-1] if levels == 2 else 0
-    need = dict(qr=(q, "r"), kr=(k, "r"), vt=(v, "t"), pkr=(pk, "r"), pvt=(pv, "t"))
+    need = dict(qr=(q, "r"), kr=(k, "r"), vr=(v, "r"), pkr=(pk, "r"), pvt=(pv, "t"))
     if levels == 2:
         need.update(pk2r=(pk2, "r"), pv2t=(pv2, "t"))
     tl = _tiles(tiles, need)
@@ -69,7 +69,7 @@ def attn_fwd(q, k, v, pk, pv, indices, token_weight, pk2=None, pv2=None, p_indic
     o = torch.empty_like(q) if rows_ok8(q) else torch.empty(q.shape, device=q.device, dtype=q.dtype)
     lse = torch.empty(B, H, N, device=q.device, dtype=torch.float32)
     a = AttnFwdArgs()
-    a.qr, a.kr, a.vt = (tl[n].data_ptr() for n in ("qr", "kr", "vt"))
+    a.qr, a.kr, a.vt = (tl[n].data_ptr() for n in ("qr", "kr", "vr"))
     a.idx = idx.data_ptr()
     a.o, (a.sob, a.soh, a.son) = o.data_ptr(), s3(o)
     a.lse = lse.data_ptr()
