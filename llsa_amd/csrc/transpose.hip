@@ -11,8 +11,10 @@
 
 namespace llsa {
 
-constexpr int kTrThreads = 1024;
-constexpr int kTrWaves = kTrThreads / kWave;
+// Threads per workgroup: 1024 where the kernel has the chip to itself.  Beside the forward attention kernel on another stream
+// 256: a CU that kernel fills leaves room for one more wave of few registers per SIMD, and a workgroup of sixteen waves
+// waits until the CU has drained.
+constexpr int kTrThreads = 1024, kTrThreadsBeside = 256;
 
 __device__ __forceinline__ int wave_incl_scan(int v, int lane) {
 #pragma unroll
@@ -23,20 +25,22 @@ __device__ __forceinline__ int wave_incl_scan(int v, int lane) {
     return v;
 }
 
-constexpr int kTrPart = 16 * kTrThreads;       // entries per workgroup of the split path
+constexpr int kTrPart = 16 * kTrThreadsBeside; // entries per workgroup of the split path
+constexpr int kTrSplitMin = 65536;             // entries from which the split path is taken
 
 // The middle step of every form of the transpose: counts per key block -> offsets, segment starts and the work list.
 // count_of(i): entries of key block i; set_start(i, start): where the caller wants the start of segment i (its cursor);
-// wave_tot: 5 * kTrWaves ints of LDS.  Called by all kTrThreads threads of the workgroup; `work` already points at the
+// wave_tot: 5 * NT / 64 ints of LDS.  Called by all NT threads of the workgroup; `work` already points at the
 // (b,h)'s list (or is nullptr).  E: the sum of all counts.  write_out = false: only set_start is called, offsets and work list
 // stay untouched (a workgroup that shares the (b,h) with others and leaves these writes to one of them).
-template <typename CountFn, typename StartFn>
+template <int NT, typename CountFn, typename StartFn>
 __device__ __forceinline__ int offsets_and_work_list(CountFn count_of, StartFn set_start, int* wave_tot, int* __restrict__ offsets,
                                                       int* __restrict__ work, int Kb, int E_items, int E_total, int chunk,
                                                       bool write_out = true) {
+    constexpr int NW = NT / kWave;
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     // exclusive scan over the counts: each thread owns `per` consecutive counters
-    const int per = (Kb + kTrThreads - 1) / kTrThreads;
+    const int per = (Kb + NT - 1) / NT;
     const int c0 = min(tid * per, Kb), c1 = min(c0 + per, Kb);
     // l_items: short items, l_long: long items (more than chunk/2 entries)
     const int long_min = chunk / 2 + 1;
@@ -58,19 +62,19 @@ __device__ __forceinline__ int offsets_and_work_list(CountFn count_of, StartFn s
     const int incl_l = wave_incl_scan(l_long, lane);
     if (lane == kWave - 1) {
         wave_tot[wave] = incl;
-        wave_tot[kTrWaves + wave] = incl_i;
-        wave_tot[2 * kTrWaves + wave] = incl_s;
-        wave_tot[3 * kTrWaves + wave] = incl_m;
-        wave_tot[4 * kTrWaves + wave] = incl_l;
+        wave_tot[NW + wave] = incl_i;
+        wave_tot[2 * NW + wave] = incl_s;
+        wave_tot[3 * NW + wave] = incl_m;
+        wave_tot[4 * NW + wave] = incl_l;
     }
     __syncthreads();
     int run = incl - local, run_i = incl_i - l_items, run_s = incl_s - l_slots, run_m = incl_m - l_multi, run_l = incl_l - l_long;
     // (five LDS reads in flight together; the sums over the waves go by readlane)
     int total_long = 0, tot[5];
 #pragma unroll
-    for (int k = 0; k < 5; k++) tot[k] = wave_tot[k * kTrWaves + (lane & (kTrWaves - 1))];
+    for (int k = 0; k < 5; k++) tot[k] = wave_tot[k * NW + (lane & (NW - 1))];
 #pragma unroll
-    for (int w = 0; w < kTrWaves; w++) {
+    for (int w = 0; w < NW; w++) {
         int o[5];
 #pragma unroll
         for (int k = 0; k < 5; k++) o[k] = __builtin_amdgcn_readlane(tot[k], w);
@@ -110,8 +114,8 @@ __device__ __forceinline__ int offsets_and_work_list(CountFn count_of, StartFn s
             run_s += (nch > 1) ? nch : 0;
         }
     }
-    if (write_out && tid == kTrThreads - 1) offsets[Kb] = run;        // (the last thread's running sum is the total)
-    if (write_out && work != nullptr && tid == kTrThreads - 1) {
+    if (write_out && tid == NT - 1) offsets[Kb] = run;        // (the last thread's running sum is the total)
+    if (write_out && work != nullptr && tid == NT - 1) {
         work[0] = run_i;                                      // (the last thread's short items end the list)
         work[1] = run_s;
         work[2] = run_m;
@@ -138,16 +142,17 @@ __device__ __forceinline__ int offsets_and_work_list(CountFn count_of, StartFn s
 // offsets and work list and leaves every segment's start in the same place as the cursor that
 // tr_scatter_kernel advances.
 template <bool SPLIT>
-__global__ __launch_bounds__(kTrThreads) void transpose_indices_kernel(const int* __restrict__ idx, int* __restrict__ offsets,
+__global__ __launch_bounds__(SPLIT ? kTrThreadsBeside : kTrThreads) void transpose_indices_kernel(const int* __restrict__ idx, int* __restrict__ offsets,
                                                                       int* __restrict__ flat, int* __restrict__ work,
                                                                       int Mb, int Kb, int T, int chunk, int work_stride) {
     // These kernels run beside the forward attention kernel on a second stream and are on the
     // critical path of nothing until the backward starts, but one slow workgroup per (b,h) is all
     // there is of them: let their waves go first when they share a CU.
     __builtin_amdgcn_s_setprio(3);
+    constexpr int NT = SPLIT ? kTrThreadsBeside : kTrThreads;
     HIP_DYNAMIC_SHARED(int, smem)
     int* pos = smem;                               // Kb
-    int* wave_tot = smem + (SPLIT ? 0 : Kb);       // 5 * kTrWaves (the split form keeps no counters in LDS)
+    int* wave_tot = smem + (SPLIT ? 0 : Kb);       // 5 ints per wave (the split form keeps no counters in LDS)
 
     const int tid = threadIdx.x;
     const int bh = blockIdx.x;
@@ -159,25 +164,25 @@ __global__ __launch_bounds__(kTrThreads) void transpose_indices_kernel(const int
     constexpr int kBatch = 16;
     int* tail = SPLIT ? work + (int64_t)bh * work_stride + (work_stride - work_tail_len(Kb)) : nullptr;
     if (!SPLIT) {
-        for (int i = tid; i < Kb; i += kTrThreads) pos[i] = 0;
+        for (int i = tid; i < Kb; i += NT) pos[i] = 0;
     }
     __syncthreads();
     // entries are taken 16 per thread at a time, all 16 loads issued before the first is used
-    for (int e0 = 0; e0 < (SPLIT ? 0 : E); e0 += kBatch * kTrThreads) {
+    for (int e0 = 0; e0 < (SPLIT ? 0 : E); e0 += kBatch * NT) {
         int v[kBatch];
 #pragma unroll
         for (int k = 0; k < kBatch; k++) {
-            const int e = e0 + k * kTrThreads + tid;
+            const int e = e0 + k * NT + tid;
             v[k] = (e < E) ? idx[e] : -1;
         }
 #pragma unroll
         for (int k = 0; k < kBatch; k++)
-            if (e0 + k * kTrThreads + tid < E) atomicAdd(&pos[clampi(v[k], 0, Kb - 1)], 1);
+            if (e0 + k * NT + tid < E) atomicAdd(&pos[clampi(v[k], 0, Kb - 1)], 1);
     }
     __syncthreads();
 
     if (work != nullptr) work += (int64_t)bh * work_stride;
-    offsets_and_work_list([&](int i) { return SPLIT ? tail[i] : pos[i]; },
+    offsets_and_work_list<NT>([&](int i) { return SPLIT ? tail[i] : pos[i]; },
                           [&](int i, int start) {
                               if (SPLIT) tail[i] = start;
                               else pos[i] = start;
@@ -185,16 +190,16 @@ __global__ __launch_bounds__(kTrThreads) void transpose_indices_kernel(const int
                           wave_tot, offsets, work, Kb, E, E, chunk);
     __syncthreads();
 
-    for (int e0 = 0; e0 < (SPLIT ? 0 : E); e0 += kBatch * kTrThreads) {
+    for (int e0 = 0; e0 < (SPLIT ? 0 : E); e0 += kBatch * NT) {
         int v[kBatch];
 #pragma unroll
         for (int k = 0; k < kBatch; k++) {
-            const int e = e0 + k * kTrThreads + tid;
+            const int e = e0 + k * NT + tid;
             v[k] = (e < E) ? idx[e] : -1;
         }
 #pragma unroll
         for (int k = 0; k < kBatch; k++) {
-            const int e = e0 + k * kTrThreads + tid;
+            const int e = e0 + k * NT + tid;
             if (e < E) flat[atomicAdd(&pos[clampi(v[k], 0, Kb - 1)], 1)] = e / T;
         }
     }
@@ -225,19 +230,19 @@ struct TrJobs {
 __host__ __device__ inline int tr_stride(int Mb) { return (Mb + 31) / 32 + 1; }
 
 // calls fn(key block, query block) for every entry of the (b,h), each in one thread
-template <typename Fn>
+template <int NT, typename Fn>
 __device__ __forceinline__ void tr_entries(const TrJob& jb, const int* __restrict__ idx, Fn fn) {
     const int tid = threadIdx.x, n = jb.quads ? jb.Mb * jb.T / 4 : jb.Mb * jb.T;
     constexpr int kBatch = 8;
     auto query = [&](int i) { return jb.row_magic == 0 ? i : (int)(((unsigned long long)(unsigned)i * jb.row_magic) >> 32); };
     if (jb.quads) {
-        for (int i0 = 0; i0 < n; i0 += kBatch * kTrThreads) {     // eight loads in flight per thread
+        for (int i0 = 0; i0 < n; i0 += kBatch * NT) {     // eight loads in flight per thread
             i32x4 v[kBatch];
 #pragma unroll
-            for (int k = 0; k < kBatch; k++) v[k] = reinterpret_cast<const i32x4*>(idx)[min(i0 + k * kTrThreads + tid, n - 1)];
+            for (int k = 0; k < kBatch; k++) v[k] = reinterpret_cast<const i32x4*>(idx)[min(i0 + k * NT + tid, n - 1)];
 #pragma unroll
             for (int k = 0; k < kBatch; k++) {
-                const int i = i0 + k * kTrThreads + tid;
+                const int i = i0 + k * NT + tid;
                 if (i < n) {
                     const int q = query(i);
 #pragma unroll
@@ -246,13 +251,15 @@ __device__ __forceinline__ void tr_entries(const TrJob& jb, const int* __restric
             }
         }
     } else {
-        for (int i = tid; i < n; i += kTrThreads) fn(clampi(idx[i], 0, jb.Kb - 1), query(i), i);
+        for (int i = tid; i < n; i += NT) fn(clampi(idx[i], 0, jb.Kb - 1), query(i), i);
     }
 }
 
-__global__ __launch_bounds__(kTrThreads) void transpose_bitmap_kernel(TrJobs jobs) {
+template <int NT>
+__global__ __launch_bounds__(NT) void transpose_bitmap_kernel(TrJobs jobs) {
+    constexpr int NW = NT / kWave;
     HIP_DYNAMIC_SHARED(int, smem)
-    __shared__ int wave_tot[5 * kTrWaves];
+    __shared__ int wave_tot[5 * NW];
     const int bh = blockIdx.x / jobs.wgs;
     int part = blockIdx.x % jobs.wgs, ji = 0;
     while (ji < jobs.n_jobs - 1 && part > jobs.job[ji].parts) part -= jobs.job[ji++].parts + 1;
@@ -262,11 +269,11 @@ __global__ __launch_bounds__(kTrThreads) void transpose_bitmap_kernel(TrJobs job
     const int* idx = jb.idx + (int64_t)bh * E;
 
     if (part == jb.parts) {                                   // offsets and work list
-        for (int i = tid; i < Kb; i += kTrThreads) smem[i] = 0;
+        for (int i = tid; i < Kb; i += NT) smem[i] = 0;
         __syncthreads();
-        tr_entries(jb, idx, [&](int n, int, int) { atomicAdd(&smem[n], 1); });
+        tr_entries<NT>(jb, idx, [&](int n, int, int) { atomicAdd(&smem[n], 1); });
         __syncthreads();
-        offsets_and_work_list([&](int i) { return smem[i]; }, [](int, int) {}, wave_tot, jb.offsets + (int64_t)bh * (Kb + 1),
+        offsets_and_work_list<NT>([&](int i) { return smem[i]; }, [](int, int) {}, wave_tot, jb.offsets + (int64_t)bh * (Kb + 1),
                               jb.work ? jb.work + (int64_t)bh * jb.work_stride : nullptr, Kb, E, E, jb.chunk);
         return;
     }
@@ -274,10 +281,10 @@ __global__ __launch_bounds__(kTrThreads) void transpose_bitmap_kernel(TrJobs job
     const int words = (Mb + 31) / 32, stride = words + 1;
     const int lo = part * jb.rows, nr = min(jb.rows, Kb - lo);       // > 0: the host leaves no range empty
     unsigned* bm = reinterpret_cast<unsigned*>(smem);         // [nr][stride]
-    for (int i = tid; i < nr * stride; i += kTrThreads) bm[i] = 0u;
+    for (int i = tid; i < nr * stride; i += NT) bm[i] = 0u;
     __syncthreads();
     int below = 0;
-    tr_entries(jb, idx, [&](int n, int q, int) {
+    tr_entries<NT>(jb, idx, [&](int n, int q, int) {
         const int r = n - lo;
         below += r < 0 ? 1 : 0;
         if ((unsigned)r < (unsigned)nr) {
@@ -288,17 +295,17 @@ __global__ __launch_bounds__(kTrThreads) void transpose_bitmap_kernel(TrJobs job
     below = wave_incl_scan(below, lane);
     if (lane == kWave - 1) wave_tot[wave] = below;
     __syncthreads();
-    int start = 0, tot = wave_tot[lane & (kTrWaves - 1)];     // (one LDS read; the sums over the waves go by readlane)
+    int start = 0, tot = wave_tot[lane & (NW - 1)];     // (one LDS read; the sums over the waves go by readlane)
 #pragma unroll
-    for (int w = 0; w < kTrWaves; w++) start += __builtin_amdgcn_readlane(tot, w);
-    {   // the rows' starts take the place of the counts (a range has at most kTrThreads rows)
+    for (int w = 0; w < NW; w++) start += __builtin_amdgcn_readlane(tot, w);
+    {   // the rows' starts take the place of the counts (a range has at most 256 rows)
         const int c = tid < nr ? (int)bm[tid * stride + words] : 0;
         const int incl = wave_incl_scan(c, lane);
-        if (lane == kWave - 1) wave_tot[kTrWaves + wave] = incl;
+        if (lane == kWave - 1) wave_tot[NW + wave] = incl;
         __syncthreads();
-        tot = wave_tot[kTrWaves + (lane & (kTrWaves - 1))];
+        tot = wave_tot[NW + (lane & (NW - 1))];
 #pragma unroll
-        for (int w = 0; w < kTrWaves; w++) {
+        for (int w = 0; w < NW; w++) {
             const int o = __builtin_amdgcn_readlane(tot, w);
             start += w < wave ? o : 0;
         }
@@ -307,7 +314,7 @@ __global__ __launch_bounds__(kTrThreads) void transpose_bitmap_kernel(TrJobs job
     __syncthreads();
     if (jb.inv != nullptr) {
         int* inv = jb.inv + (int64_t)bh * E;
-        tr_entries(jb, idx, [&](int n, int q, int e) {
+        tr_entries<NT>(jb, idx, [&](int n, int q, int e) {
             const int r = n - lo;
             if ((unsigned)r >= (unsigned)nr) return;
             const unsigned* row = bm + r * stride;
@@ -322,7 +329,7 @@ __global__ __launch_bounds__(kTrThreads) void transpose_bitmap_kernel(TrJobs job
     // segment has entries.)
     const int sub = tid & 7, wps = (words + 7) / 8, w_lo = min(words, sub * wps), w_hi = min(words, w_lo + wps);
     int* flat = jb.flat + (int64_t)bh * E;
-    for (int r0 = 0; r0 < nr; r0 += kTrThreads / 8) {
+    for (int r0 = 0; r0 < nr; r0 += NT / 8) {
         const int r = r0 + (tid >> 3);
         const unsigned* row = bm + min(r, nr - 1) * stride;
         int mine = 0;
@@ -347,11 +354,11 @@ __global__ __launch_bounds__(kTrThreads) void transpose_bitmap_kernel(TrJobs job
 }
 
 // Split path, first and last step: one workgroup per kTrPart entries.
-__global__ __launch_bounds__(kTrThreads) void tr_zero_kernel(int* __restrict__ work, int Kb, int work_stride) {
+__global__ __launch_bounds__(kTrThreadsBeside) void tr_zero_kernel(int* __restrict__ work, int Kb, int work_stride) {
     int* tail = work + (int64_t)blockIdx.x * work_stride + (work_stride - work_tail_len(Kb));
-    for (int i = threadIdx.x; i < Kb; i += kTrThreads) tail[i] = 0;
+    for (int i = threadIdx.x; i < Kb; i += kTrThreadsBeside) tail[i] = 0;
 }
-__global__ __launch_bounds__(kTrThreads) void tr_count_kernel(const int* __restrict__ idx, int* __restrict__ work, int E, int Kb,
+__global__ __launch_bounds__(kTrThreadsBeside) void tr_count_kernel(const int* __restrict__ idx, int* __restrict__ work, int E, int Kb,
                                                              int work_stride) {
     // (global atomics, no LDS histogram: this kernel runs beside the forward attention kernel, whose
     // workgroups leave no room for 64 KB of LDS, and its workgroups would wait for that kernel to end)
@@ -362,14 +369,14 @@ __global__ __launch_bounds__(kTrThreads) void tr_count_kernel(const int* __restr
     int v[16];
 #pragma unroll
     for (int k = 0; k < 16; k++) {
-        const int e = blockIdx.x * kTrPart + k * kTrThreads + tid;
+        const int e = blockIdx.x * kTrPart + k * kTrThreadsBeside + tid;
         v[k] = (e < E) ? idx[e] : -1;
     }
 #pragma unroll
     for (int k = 0; k < 16; k++)
-        if (blockIdx.x * kTrPart + k * kTrThreads + tid < E) atomicAdd(&tail[clampi(v[k], 0, Kb - 1)], 1);
+        if (blockIdx.x * kTrPart + k * kTrThreadsBeside + tid < E) atomicAdd(&tail[clampi(v[k], 0, Kb - 1)], 1);
 }
-__global__ __launch_bounds__(kTrThreads) void tr_scatter_kernel(const int* __restrict__ idx, int* __restrict__ flat,
+__global__ __launch_bounds__(kTrThreadsBeside) void tr_scatter_kernel(const int* __restrict__ idx, int* __restrict__ flat,
                                                                int* __restrict__ work, int E, int Kb, int T, int work_stride) {
     __builtin_amdgcn_s_setprio(3);
     const int tid = threadIdx.x, bh = blockIdx.y;
@@ -379,12 +386,12 @@ __global__ __launch_bounds__(kTrThreads) void tr_scatter_kernel(const int* __res
     int v[16];
 #pragma unroll
     for (int k = 0; k < 16; k++) {
-        const int e = blockIdx.x * kTrPart + k * kTrThreads + tid;
+        const int e = blockIdx.x * kTrPart + k * kTrThreadsBeside + tid;
         v[k] = (e < E) ? idx[e] : -1;
     }
 #pragma unroll
     for (int k = 0; k < 16; k++) {
-        const int e = blockIdx.x * kTrPart + k * kTrThreads + tid;
+        const int e = blockIdx.x * kTrPart + k * kTrThreadsBeside + tid;
         if (e < E) flat[atomicAdd(&cursor[clampi(v[k], 0, Kb - 1)], 1)] = e / T;      // order inside a segment: sorted afterwards
     }
 }
@@ -492,7 +499,7 @@ constexpr int kTrLdsInts = 16 * 1024;
 static int tr_parts(int Mb, int Kb, int T, int BH) {
     const int64_t stride = tr_stride(Mb), E = (int64_t)Mb * T;
     if (stride > kTrLdsInts || Kb > 2 * kTrLdsInts) return 0;
-    const int most_rows = (int)std::min<int64_t>(kTrLdsInts / stride, kTrThreads);
+    const int most_rows = (int)std::min<int64_t>(kTrLdsInts / stride, kTrThreadsBeside);
     const int least = (Kb + most_rows - 1) / most_rows;
     if (E > 1 << 16) return 0;
     const int parts = std::max({least, std::min(std::max(128 / BH - 1, 4), Kb / 32), 1});
@@ -501,7 +508,7 @@ static int tr_parts(int Mb, int Kb, int T, int BH) {
 }
 
 // the jobs that are small enough, all in one launch
-static int launch_bitmap_jobs(TrJobs& jobs, int n_jobs, int B, int H, hipStream_t st) {
+static int launch_bitmap_jobs(TrJobs& jobs, int n_jobs, int B, int H, bool beside, hipStream_t st) {
     int64_t ints = 0;
     jobs.wgs = 0;
     jobs.n_jobs = n_jobs;
@@ -511,19 +518,23 @@ static int launch_bitmap_jobs(TrJobs& jobs, int n_jobs, int B, int H, hipStream_
         jobs.wgs += j.parts + 1;
     }
     const size_t lds = sizeof(int) * (size_t)ints;
+    const void* kernel = beside ? (const void*)transpose_bitmap_kernel<kTrThreadsBeside> : (const void*)transpose_bitmap_kernel<kTrThreads>;
     if (lds > 60 * 1024) {
-        hipError_t e = hipFuncSetAttribute((const void*)transpose_bitmap_kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+        hipError_t e = hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
         if (e != hipSuccess) return fail(-101, "transpose_indices: cannot raise dynamic LDS to %zu bytes: %s", lds, hipGetErrorString(e));
     }
-    hipLaunchKernelGGL(transpose_bitmap_kernel, dim3(B * H * jobs.wgs), dim3(kTrThreads), lds, st, jobs);
+    if (beside)
+        hipLaunchKernelGGL(HIP_KERNEL_NAME(transpose_bitmap_kernel<kTrThreadsBeside>), dim3(B * H * jobs.wgs), dim3(kTrThreadsBeside), lds, st, jobs);
+    else
+        hipLaunchKernelGGL(HIP_KERNEL_NAME(transpose_bitmap_kernel<kTrThreads>), dim3(B * H * jobs.wgs), dim3(kTrThreads), lds, st, jobs);
     return launch_status("transpose_indices");
 }
 
 static int transpose_general(const int32_t* idx, int32_t* offsets, int32_t* flat, int32_t* work, int32_t* inv, int B, int H, int Mb, int Kb,
                              int T, int chunk, void* stream) {
     const size_t lds = sizeof(int) * ((size_t)Kb + 128);
-    static_assert(5 * kTrWaves <= 128, "wave totals must fit their LDS slot");
-    LLSA_REQUIRE(lds <= 160 * 1024 || (work != nullptr && (int64_t)Mb * T >= 4 * kTrPart),
+    static_assert(5 * kTrThreads / kWave <= 128, "wave totals must fit their LDS slot");
+    LLSA_REQUIRE(lds <= 160 * 1024 || (work != nullptr && (int64_t)Mb * T >= kTrSplitMin),
                  "transpose_indices: Kb=%d needs %zu bytes of LDS (limit 163840)", Kb, lds);
     // the segment sort keeps one bitmap over the query blocks per wave: four waves a workgroup while they fit, then two, then one
     const size_t bitmap = sizeof(unsigned) * ((size_t)(Mb + 31) / 32);
@@ -531,7 +542,7 @@ static int transpose_general(const int32_t* idx, int32_t* offsets, int32_t* flat
     const size_t lds_sort = bitmap * sort_waves;
     LLSA_REQUIRE(lds_sort <= 160 * 1024, "transpose_indices: Mb=%d needs %zu bytes of LDS for the segment sort (limit 163840)", Mb, lds_sort);
     const int64_t E = (int64_t)Mb * T;
-    const bool split = work != nullptr && E >= 4 * kTrPart;
+    const bool split = work != nullptr && E >= kTrSplitMin;
     if (!split && lds > 64 * 1024) {
         hipError_t e = hipFuncSetAttribute((const void*)transpose_indices_kernel<false>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
         if (e != hipSuccess) return fail(-101, "transpose_indices: cannot raise dynamic LDS to %zu bytes: %s", lds, hipGetErrorString(e));
@@ -541,11 +552,11 @@ static int transpose_general(const int32_t* idx, int32_t* offsets, int32_t* flat
     if (split) {
         // many entries: histogram and scatter spread over E / kTrPart workgroups per (b,h)
         const int parts = (int)((E + kTrPart - 1) / kTrPart);
-        hipLaunchKernelGGL(tr_zero_kernel, dim3(B * H), dim3(kTrThreads), 0, st, work, Kb, wl);
-        hipLaunchKernelGGL(tr_count_kernel, dim3(parts, B * H), dim3(kTrThreads), 0, st, idx, work, (int)E, Kb, wl);
-        hipLaunchKernelGGL(HIP_KERNEL_NAME(transpose_indices_kernel<true>), dim3(B * H), dim3(kTrThreads), sizeof(int) * 128, st, idx,
+        hipLaunchKernelGGL(tr_zero_kernel, dim3(B * H), dim3(kTrThreadsBeside), 0, st, work, Kb, wl);
+        hipLaunchKernelGGL(tr_count_kernel, dim3(parts, B * H), dim3(kTrThreadsBeside), 0, st, idx, work, (int)E, Kb, wl);
+        hipLaunchKernelGGL(HIP_KERNEL_NAME(transpose_indices_kernel<true>), dim3(B * H), dim3(kTrThreadsBeside), sizeof(int) * 128, st, idx,
                            offsets, flat, work, Mb, Kb, T, chunk, wl);
-        hipLaunchKernelGGL(tr_scatter_kernel, dim3(parts, B * H), dim3(kTrThreads), 0, st, idx, flat, work, (int)E, Kb, T, wl);
+        hipLaunchKernelGGL(tr_scatter_kernel, dim3(parts, B * H), dim3(kTrThreadsBeside), 0, st, idx, flat, work, (int)E, Kb, T, wl);
     } else {
         hipLaunchKernelGGL(HIP_KERNEL_NAME(transpose_indices_kernel<false>), dim3(B * H), dim3(kTrThreads), lds, st, idx, offsets, flat,
                            work, Mb, Kb, T, chunk, wl);
@@ -593,7 +604,7 @@ extern "C" int llsa_transpose_indices_multi(const llsa_transpose_job* jobs, int 
             if (rc != 0) return rc;
         }
     }
-    if (n_small > 0) return launch_bitmap_jobs(small, n_small, B, H, (hipStream_t)stream);
+    if (n_small > 0) return launch_bitmap_jobs(small, n_small, B, H, n_small < n_jobs, (hipStream_t)stream);
     return 0;
 }
 
