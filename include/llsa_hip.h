@@ -44,7 +44,7 @@ extern "C" {
 #define LLSA_DTYPE_BF16 0
 #define LLSA_DTYPE_F32 1
 
-#define LLSA_ABI_VERSION 205     /* changes with every change of a signature or argument structure below */
+#define LLSA_ABI_VERSION 206     /* changes with every change of a signature or argument structure below */
 int llsa_version(void);          /* LLSA_ABI_VERSION of the built library                                    */
 const char* llsa_last_error_string(void);
 
@@ -275,6 +275,18 @@ typedef struct llsa_bwd_level {
     int32_t reserved;
 } llsa_bwd_level;
 
+/* The qk RMS norm that stood between x and what the operator attended with (llsa_pool_item.gamma): given here, dq (dk) leaves as
+ * the gradient of x and dgamma (64) receives the weights' gradient.  What llsa_rmsnorm_bwd does to the finished dq (dk),
+ * inside the kernels that write it. */
+typedef struct llsa_norm_back {
+    const void* x; int64_t sxb, sxh, sxn;        /* (B,H,N,64) bf16, rows 16-byte aligned; NULL: no norm          */
+    const float* gamma;                          /* (64)                                                          */
+    float* dgamma;                               /* (64) out                                                      */
+    float* partials;                             /* B*H*N/16*64 floats of scratch                                 */
+    float eps;
+    int32_t reserved;
+} llsa_norm_back;
+
 typedef struct llsa_attn_bwd_args {
     const void* dout; int64_t sdob, sdoh, sdon;  /* (B,H,N,64) upstream gradient                 */
     const void* o;    int64_t sob, soh, son;     /* (B,H,N,64) forward output                     */
@@ -298,6 +310,7 @@ typedef struct llsa_attn_bwd_args {
                                                     and dk is rotated back with freq_dk                */
     int32_t reserved;
     llsa_bwd_level lvl[LLSA_MAX_LEVELS];         /* lvl[l - 1] = pooled level l                     */
+    llsa_norm_back norm_q, norm_k;               /* norm_k needs fold_pooled                        */
 } llsa_attn_bwd_args;
 
 /* `stages` is a diagnostic for timing kernels one at a time: a mask other than 0 launches only the named kernels.

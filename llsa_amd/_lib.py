@@ -53,6 +53,11 @@ class BwdLevel(C.Structure):
                 ("dk", c_void_p), ("dv", c_void_p), ("T", c_int32), ("w", c_float), ("gw", c_float), ("reserved", c_int32)]
 
 
+class NormBack(C.Structure):
+    _fields_ = [("x", c_void_p), ("sxb", c_int64), ("sxh", c_int64), ("sxn", c_int64), ("gamma", c_void_p), ("dgamma", c_void_p),
+                ("partials", c_void_p), ("eps", c_float), ("reserved", c_int32)]
+
+
 class AttnBwdArgs(C.Structure):
     _fields_ = (
         [("dout", c_void_p), ("sdob", c_int64), ("sdoh", c_int64), ("sdon", c_int64)]
@@ -65,7 +70,7 @@ class AttnBwdArgs(C.Structure):
         + [("workspace", c_void_p), ("workspace_bytes", c_int64), ("freq_dq", c_void_p), ("freq_dk", c_void_p),
            ("B", c_int32), ("H", c_int32), ("N", c_int32), ("T", c_int32), ("levels", c_int32),
            ("stages", c_int32), ("fold_pooled", c_int32), ("reserved", c_int32),
-           ("lvl", BwdLevel * MAX_LEVELS)])
+           ("lvl", BwdLevel * MAX_LEVELS), ("norm_q", NormBack), ("norm_k", NormBack)])
 
 
 P64 = C.POINTER(c_int64)
@@ -107,7 +112,7 @@ _SIGNATURES = {
 
 EXPORTS = tuple(_SIGNATURES)
 CHUNK_FINE_MAX = 256                                        # LLSA_CHUNK_FINE_MAX of include/llsa_hip.h
-ABI_VERSION = 205                                           # LLSA_ABI_VERSION
+ABI_VERSION = 206                                           # LLSA_ABI_VERSION
 STATIC_PARTIALS_MAX = 262144                                # LLSA_STATIC_PARTIALS_MAX
 
 

@@ -15,6 +15,7 @@
 #include "llsa_device.h"
 #include "llsa_host.h"
 #include "../../include/llsa_hip.h"
+#include <algorithm>
 
 namespace llsa {
 
@@ -82,6 +83,61 @@ __device__ __forceinline__ void dq_accum(f32x4 dq[4], const PairT& p, bf16x8 bds
     for (int dt = 0; dt < 4; dt++) dq[dt] = mfma_bf16(cat(p.t[0][dt], p.t[1][dt]), bds, dq[dt]);
 }
 
+// A gradient block (16 tokens x 64 channels, one lane: channels 16 dt + 4 (l/16) ..+3 of token l%16) back through the RMS norm of
+// its rows x, as rmsnorm_bwd_kernel does it: with xn = x rstd and g = dy gamma, dx = rstd (g - xn mean(g xn)).  contrib: dy xn,
+// added up for the weights' gradient.  x: the lane's channels of its token; gamma: its channels' weights.
+// Inside the kernels that write dq and dk because a pass of its own is bound by memory: it reads the finished gradient and x and
+// writes the gradient again (300 MB for q and k of 8 x 6 x 16384 tokens, plus four launches).  Here x is all that is read, by
+// waves that have their arithmetic still to do: 1368 -> 1298 us for that step, 215 -> 200 us at 4 x 6 x 4096.
+__device__ __forceinline__ void norm_back(bf16x4 (&dy)[4], const bf16x4 (&x)[4], const f32x4 (&gamma)[4], float eps, float (&contrib)[16]) {
+    float ss = 0.f;
+#pragma unroll
+    for (int dt = 0; dt < 4; dt++)
+#pragma unroll
+        for (int e = 0; e < 4; e++) ss += (float)x[dt][e] * (float)x[dt][e];
+    const float rstd = rsqrtf(quad_sum(ss) * (1.f / kD) + eps);
+    float dot = 0.f;
+#pragma unroll
+    for (int dt = 0; dt < 4; dt++)
+#pragma unroll
+        for (int e = 0; e < 4; e++) {
+            const float xn = (float)x[dt][e] * rstd, g = (float)dy[dt][e];
+            dot += g * gamma[dt][e] * xn;
+            contrib[dt * 4 + e] += g * xn;
+        }
+    dot = quad_sum(dot) * (1.f / kD);
+#pragma unroll
+    for (int dt = 0; dt < 4; dt++)
+#pragma unroll
+        for (int e = 0; e < 4; e++)
+            dy[dt][e] = (bf16)(rstd * ((float)dy[dt][e] * gamma[dt][e] - (float)x[dt][e] * rstd * dot));
+}
+__device__ __forceinline__ void norm_load(bf16x4 (&x)[4], f32x4 (&gamma)[4], const llsa_norm_back& nb, int b, int h, int tok, int quad) {
+    const bf16* p = (const bf16*)nb.x + b * nb.sxb + h * nb.sxh + (int64_t)tok * nb.sxn + quad * 4;
+#pragma unroll
+    for (int dt = 0; dt < 4; dt++) {
+        x[dt] = ld8(p + dt * 16);
+#pragma unroll
+        for (int e = 0; e < 4; e++) gamma[dt][e] = nb.gamma[dt * 16 + quad * 4 + e];
+    }
+}
+// Sum of the sixteen contrib[] over the sixteen tokens of a quad, by exchanging halves: lane l ends with the sum for
+// channel 16 (i/4) + 4 (l/16) + i%4, i = the lane's low four bits.
+__device__ __forceinline__ float norm_contrib_sum(const float (&contrib)[16], int lane, int& channel) {
+    float a8[8], a4[4], a2[2];
+    const bool b3 = lane & 8, b2 = lane & 4, b1 = lane & 2, b0 = lane & 1;
+#pragma unroll
+    for (int i = 0; i < 8; i++) a8[i] = (b3 ? contrib[8 + i] : contrib[i]) + __shfl_xor(b3 ? contrib[i] : contrib[8 + i], 8);
+#pragma unroll
+    for (int i = 0; i < 4; i++) a4[i] = (b2 ? a8[4 + i] : a8[i]) + __shfl_xor(b2 ? a8[i] : a8[4 + i], 4);
+#pragma unroll
+    for (int i = 0; i < 2; i++) a2[i] = (b1 ? a4[2 + i] : a4[i]) + __shfl_xor(b1 ? a4[i] : a4[2 + i], 2);
+    const float s = (b0 ? a2[1] : a2[0]) + __shfl_xor(b0 ? a2[0] : a2[1], 1);
+    const int i = lane & 15;
+    channel = 16 * (i >> 2) + 4 * (lane >> 4) + (i & 3);
+    return s;
+}
+
 // What a wave keeps per query block
 struct DqSide {
     bf16x8 bq[2], bdo[2];          // R operands of q and dO
@@ -118,16 +174,22 @@ __device__ __forceinline__ void dq_begin(DqSide& sd, const llsa_attn_bwd_args& a
 #pragma unroll
     for (int dt = 0; dt < 4; dt++) sd.dq[dt] = f32x4{0.f, 0.f, 0.f, 0.f};
 }
-__device__ __forceinline__ void dq_end(const DqSide& sd, const llsa_attn_bwd_args& a, int b, int h, int g, int lane) {
+template <bool NORM>
+__device__ __forceinline__ void dq_end(const DqSide& sd, const llsa_attn_bwd_args& a, int b, int h, int g, int lane, float (&contrib)[16]) {
     const int r = lane & 15, quad = lane >> 4, tok = g * kBlk + r;
     bf16* op = (bf16*)a.dq + b * a.sdqb + h * a.sdqh + (int64_t)tok * a.sdqn + quad * 4;
     const bf16* fq = a.freq_dq ? (const bf16*)a.freq_dq + (int64_t)tok * kD + quad * 4 : nullptr;
+    bf16x4 x[4], o[4];
+    f32x4 gamma[4];
+    if (NORM) norm_load(x, gamma, a.norm_q, b, h, tok, quad);
 #pragma unroll
     for (int dt = 0; dt < 4; dt++) {
-        bf16x4 o = cvt4(sd.dq[dt] * kScale);
-        if (fq != nullptr) o = rope_bwd4(o, ld8(fq + dt * 16));   // rotate the gradient back
-        st8(op + dt * 16, o);
+        o[dt] = cvt4(sd.dq[dt] * kScale);
+        if (fq != nullptr) o[dt] = rope_bwd4(o[dt], ld8(fq + dt * 16));   // rotate the gradient back
     }
+    if (NORM) norm_back(o, x, gamma, a.norm_q.eps, contrib);
+#pragma unroll
+    for (int dt = 0; dt < 4; dt++) st8(op + dt * 16, o[dt]);
 }
 // in0, in1 (wave-uniform): whether the query block reads the pair's first / second block
 __device__ __forceinline__ void dq_pair_of_blocks(DqSide& sd, const PairR& r, const PairT& t, float log2w, bool in0 = true, bool in1 = true) {
@@ -143,7 +205,7 @@ __device__ __forceinline__ void dq_pair_of_blocks(DqSide& sd, const PairR& r, co
 // Q sibling query blocks per wave (see attn_fwd_kernel): the pooled blocks and the fine blocks both rows selected are read once
 // -- from memory and, what weighs more here, from LDS, where every key block is read three times (K rows, V rows, K
 // transposed) -- and multiplied twice.
-template <int Q, int R>
+template <int Q, int R, bool NORM>
 __global__ __launch_bounds__(256, Q == 1 ? 4 : 3) void attn_dq_kernel(llsa_attn_bwd_args a, float* __restrict__ delta,
                                                                       bf16* __restrict__ dor) {
     __shared__ __align__(16) bf16 sh[2][kGroup][2 * kTile];   // per block: R tile of K, R tile of V
@@ -255,8 +317,23 @@ __global__ __launch_bounds__(256, Q == 1 ? 4 : 3) void attn_dq_kernel(llsa_attn_
             fine();
         }
     }
+    float contrib[16];
 #pragma unroll
-    for (int u = 0; u < Q; u++) dq_end(sd[u], a, b, h, g + u, lane);
+    for (int i = 0; i < 16; i++) contrib[i] = 0.f;
+#pragma unroll
+    for (int u = 0; u < Q; u++) dq_end<NORM>(sd[u], a, b, h, g + u, lane, contrib);
+    if (NORM) {                                               // one row of partial sums per workgroup
+        float* const red = reinterpret_cast<float*>(sh0);     // (the private slots: every wave is done with its own only after the barrier)
+        __syncthreads();
+        int ch;
+        const float s = norm_contrib_sum(contrib, lane, ch);
+        red[wave * kD + ch] = s;
+        __syncthreads();
+        if (threadIdx.x < kD) {
+            const int t = threadIdx.x;
+            a.norm_q.partials[((int64_t)bh * gridDim.x + lid % (int)gridDim.x) * kD + t] = (red[t] + red[kD + t]) + (red[2 * kD + t] + red[3 * kD + t]);
+        }
+    }
 }
 
 // ---------------------------------------------------------------------------------------
@@ -321,6 +398,7 @@ struct KSideParams {
     int64_t slot_stride;                          // partial slots per (b,h)
     float w;
     PoolFold fold;                                // fine pass only
+    llsa_norm_back norm;                          // fine pass: the norm of k (x: nullptr without)
     int stripes, stripe_len;                      // fine pass: how the items are dealt to the XCDs (see kside_item)
 };
 
@@ -404,6 +482,7 @@ __device__ __forceinline__ bool kside_item(const KSideParams& p, int& bh, int& i
 // One work item of the fine pass: a key block and a piece (at most fine_chunk(N) <= LLSA_CHUNK_FINE_MAX entries) of its list.
 // One wave = one workgroup per item (items differ a lot in length; a wave that shared its workgroup
 // with a longer one would keep its registers and LDS allocated while idle).
+template <bool NORM>
 __global__ __launch_bounds__(64) void attn_kside_kernel(KSideParams p) {
     __shared__ __align__(16) bf16 stage[4 * kTile];           // 2 query blocks x {Q, dO} R tiles
     __shared__ __align__(16) float stats[64];                 // their lse and delta rows
@@ -529,6 +608,9 @@ __global__ __launch_bounds__(64) void attn_kside_kernel(KSideParams p) {
     }
     bf16* kp = p.dk + b * p.sdkb + h * p.sdkh + (int64_t)(unit * kBlk + r) * p.sdkn + quad * 4;
     bf16* vp = p.dv + b * p.sdvb + h * p.sdvh + (int64_t)(unit * kBlk + r) * p.sdvn + quad * 4;
+    bf16x4 nx[4];
+    f32x4 ngamma[4];
+    if (NORM) norm_load(nx, ngamma, p.norm, b, h, unit * kBlk + r, quad);
     if (folding) {
         wait_vm0();                                           // the copies into fold_buf (long since done)
         // the chain of pooled levels collapses into one row for dk and one for dv, left where level 1's rows were:
@@ -544,17 +626,29 @@ __global__ __launch_bounds__(64) void attn_kside_kernel(KSideParams p) {
         __builtin_amdgcn_wave_barrier();
         __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
     }
+    bf16x4 ok[4];
 #pragma unroll
     for (int dt = 0; dt < 4; dt++) {
-        bf16x4 ok = cvt4(dk[dt] * kScale), ov = cvt4(dv[dt]);
+        ok[dt] = cvt4(dk[dt] * kScale);
+        bf16x4 ov = cvt4(dv[dt]);
         if (folding) {
             const int c0 = dt * 16 + quad * 4;
-            ok = fold_math(ok, lds_ld8(fold_buf + c0), p.fold.freq != nullptr, lds_ld8(fold_buf + kFoldRows + r * kD + c0));
+            ok[dt] = fold_math(ok[dt], lds_ld8(fold_buf + c0), p.fold.freq != nullptr, lds_ld8(fold_buf + kFoldRows + r * kD + c0));
             ov = fold_math(ov, lds_ld8(fold_buf + kD + c0), false, ov);
         }
-        st8(kp + dt * 16, ok);
         st8(vp + dt * 16, ov);
     }
+    if (NORM) {
+        float contrib[16];
+#pragma unroll
+        for (int i = 0; i < 16; i++) contrib[i] = 0.f;
+        norm_back(ok, nx, ngamma, p.norm.eps, contrib);
+        int ch;
+        const float s = norm_contrib_sum(contrib, lane, ch);
+        p.norm.partials[((int64_t)bh * p.n_units + unit) * kD + ch] = s;       // (a unit cut into pieces: kside_reduce_kernel's row)
+    }
+#pragma unroll
+    for (int dt = 0; dt < 4; dt++) st8(kp + dt * 16, ok[dt]);
 }
 
 // ---------------------------------------------------------------------------------------
@@ -944,6 +1038,7 @@ struct ReduceJob {
     int64_t work_stride, slot_stride;
     int n_chunks;            // dense job: partials per unit, at stride BH * n_units slots
     PoolFold fold;           // fine job only
+    llsa_norm_back norm;     // fine job only: the norm of k (x: nullptr without)
 };
 struct ReduceParams {
     ReduceJob job[LLSA_MAX_LEVELS + 1];
@@ -968,6 +1063,7 @@ __global__ __launch_bounds__(256) void kside_reduce_kernel(ReduceParams rp) {
     // (reduce_slots of them), which walk the job's units with that stride: the number of units with several pieces is
     // known only on the device and usually small, and a grid sized for the worst case would be mostly workgroups that
     // start, look and leave.
+    __shared__ float row_ss[4][kBlk], row_dot[4][kBlk];
     const int bh = blockIdx.y, b = bh / rp.H, h = bh % rp.H;
     int u0 = blockIdx.x >> 1, j = 0;
     while (j < rp.n_jobs && u0 >= reduce_slots(rp.job[j].max_units)) {
@@ -1052,8 +1148,65 @@ __global__ __launch_bounds__(256) void kside_reduce_kernel(ReduceParams rp) {
         bf16x4 out = cvt4(which ? acc : acc * kScale);
         if (jb.fold.depth > 0)
             out = fold_pooled(out, jb.fold, which, bh, rp.N, unit * kBlk + r, dt * 16 + quad * 4);
+        if (jb.norm.x != nullptr && which == 0) {             // (uniform over the workgroup: fp32 partial sums, dK in one workgroup)
+            // wave dt holds channels 16 dt .. of the unit's rows: norm_back with the sums over a row's channels through LDS
+            const llsa_norm_back& nb = jb.norm;
+            const int c0 = dt * 16 + quad * 4;
+            const bf16x4 x = ld8((const bf16*)nb.x + b * nb.sxb + h * nb.sxh + (int64_t)(unit * kBlk + r) * nb.sxn + c0);
+            const f32x4 gamma = {nb.gamma[c0], nb.gamma[c0 + 1], nb.gamma[c0 + 2], nb.gamma[c0 + 3]};
+            float ss = 0.f, dot = 0.f;
+#pragma unroll
+            for (int e = 0; e < 4; e++) {
+                ss += (float)x[e] * (float)x[e];
+                dot += (float)out[e] * gamma[e] * (float)x[e];
+            }
+            ss = quad_sum(ss);
+            dot = quad_sum(dot);
+            __syncthreads();                                  // (the previous unit's sums have been read)
+            if (quad == 0) {
+                row_ss[dt][r] = ss;
+                row_dot[dt][r] = dot;
+            }
+            __syncthreads();
+            const float rstd = rsqrtf(((row_ss[0][r] + row_ss[1][r]) + (row_ss[2][r] + row_ss[3][r])) * (1.f / kD) + nb.eps);
+            dot = ((row_dot[0][r] + row_dot[1][r]) + (row_dot[2][r] + row_dot[3][r])) * rstd * (1.f / kD);
+            f32x4 contrib;
+#pragma unroll
+            for (int e = 0; e < 4; e++) {
+                contrib[e] = (float)out[e] * (float)x[e] * rstd;
+                out[e] = (bf16)(rstd * ((float)out[e] * gamma[e] - (float)x[e] * rstd * dot));
+            }
+#pragma unroll
+            for (int d = 1; d < 16; d <<= 1)
+#pragma unroll
+                for (int e = 0; e < 4; e++) contrib[e] += __shfl_xor(contrib[e], d);
+            if (r == 0) *reinterpret_cast<f32x4*>(nb.partials + ((int64_t)bh * jb.n_units + unit) * kD + c0) = contrib;
+        }
         st8(dst + quad * 4 + dt * 16, out);
         if (half) st8(dst + quad * 4 + (dt + 1) * 16, cvt4(which ? acc2 : acc2 * kScale));      // (no fold on these jobs)
+    }
+}
+
+// The weights' gradients of the norms: dgamma = column sums of the rows of partial sums.  Two launches for both norms (blockIdx.y):
+// workgroup x of X adds rows x, x + X, ... of `in` into row x of `out`, then one workgroup adds those.  With out == in a
+// workgroup overwrites a row that only it has read.
+struct NormSums {
+    const float* in[2]; float* out[2];
+    int64_t rows[2];
+};
+__global__ __launch_bounds__(1024) void norm_sums_kernel(NormSums p) {
+    __shared__ float red[16][kD];
+    const int ch = threadIdx.x & 63, j = threadIdx.x >> 6;
+    const float* in = p.in[blockIdx.y];
+    float s = 0.f;
+#pragma unroll 4
+    for (int64_t r = blockIdx.x + (int64_t)j * gridDim.x; r < p.rows[blockIdx.y]; r += 16 * (int64_t)gridDim.x) s += in[r * kD + ch];
+    red[j][ch] = s;
+    __syncthreads();
+    if (j == 0) {
+#pragma unroll
+        for (int k = 1; k < 16; k++) s += red[k][ch];
+        p.out[blockIdx.y][(int64_t)blockIdx.x * kD + ch] = s;
     }
 }
 
@@ -1188,17 +1341,36 @@ extern "C" int llsa_attn_bwd(const llsa_attn_bwd_args* a, void* stream) {
     bf16* dor = (bf16*)(ws + wsp.dor);
     const bool fold = a->fold_pooled != 0;
     LLSA_REQUIRE(fold || a->freq_dk == nullptr, "attn_bwd: freq_dk needs fold_pooled");
+    LLSA_REQUIRE(fold || a->norm_k.x == nullptr, "attn_bwd: norm_k needs fold_pooled");
+    for (const llsa_norm_back* nb : {&a->norm_q, &a->norm_k}) {
+        if (nb->x == nullptr) continue;
+        LLSA_REQUIRE(nb->gamma && nb->dgamma && nb->partials && nb->eps >= 0.f, "attn_bwd: norm without gamma, dgamma or partials");
+        LLSA_REQUIRE(aligned16(nb->x) && stride_ok(nb->sxb) && stride_ok(nb->sxh) && stride_ok(nb->sxn) && aligned16(nb->partials),
+                     "attn_bwd: rows of the norm's input must be 16-byte aligned");
+    }
+    NormSums sums;
+    int n_sums = 0;
 
     const int stages = a->stages ? a->stages : (0x7fffffff & ~LLSA_BWD_NO_REDUCE);
     if (stages & LLSA_BWD_DQ) {
         // (two query blocks per wave win from 512 groups of eight on, see kPairMinGroups: 12 x 16384 tokens 79 against 82.6 us,
         // 6 x 262144 1022 against 1113)
-        if (a->T > kPairMaxTopk || N1 % 8 != 0 || (int64_t)N1 / 8 * BH < kPairMinGroups)
-            hipLaunchKernelGGL(HIP_KERNEL_NAME(attn_dq_kernel<1, 1>), dim3(N1 / 4, BH), dim3(256), 0, s, *a, delta, dor);
-        else if (a->T <= 32)
-            hipLaunchKernelGGL(HIP_KERNEL_NAME(attn_dq_kernel<2, 1>), dim3(N1 / 8, BH), dim3(256), 0, s, *a, delta, dor);
-        else
-            hipLaunchKernelGGL(HIP_KERNEL_NAME(attn_dq_kernel<2, 2>), dim3(N1 / 8, BH), dim3(256), 0, s, *a, delta, dor);
+        const bool pairs = a->T <= kPairMaxTopk && N1 % 8 == 0 && (int64_t)N1 / 8 * BH >= kPairMinGroups;
+        const dim3 grid(N1 / (pairs ? 8 : 4), BH);
+#define LLSA_DQ(Q, R)                                                                                                                  \
+    do {                                                                                                                               \
+        if (a->norm_q.x) hipLaunchKernelGGL(HIP_KERNEL_NAME(attn_dq_kernel<Q, R, true>), grid, dim3(256), 0, s, *a, delta, dor);       \
+        else hipLaunchKernelGGL(HIP_KERNEL_NAME(attn_dq_kernel<Q, R, false>), grid, dim3(256), 0, s, *a, delta, dor);                  \
+    } while (0)
+        if (!pairs) LLSA_DQ(1, 1);
+        else if (a->T <= 32) LLSA_DQ(2, 1);
+        else LLSA_DQ(2, 2);
+#undef LLSA_DQ
+        if (a->norm_q.x) {
+            sums.in[n_sums] = a->norm_q.partials;
+            sums.out[n_sums] = a->norm_q.dgamma;
+            sums.rows[n_sums++] = (int64_t)grid.x * BH;
+        }
     }
 
     ReduceParams rp;
@@ -1217,6 +1389,7 @@ extern "C" int llsa_attn_bwd(const llsa_attn_bwd_args* a, void* stream) {
         j.n_units = p.n_units; j.chunk = chunk; j.max_units = max_units;
         j.work_stride = p.work_stride; j.slot_stride = p.slot_stride; j.n_chunks = n_chunks;
         j.fold = p.fold;
+        j.norm = p.norm;
     };
     auto run_reduce = [&]() {
         if (stages & LLSA_BWD_NO_REDUCE) rp.n_jobs = 0;       // (profiling: time the K-side kernels alone)
@@ -1231,6 +1404,7 @@ extern "C" int llsa_attn_bwd(const llsa_attn_bwd_args* a, void* stream) {
     base.lse = a->lse; base.delta = delta;
     base.H = H; base.N = N; base.chunk_len = 0;
     base.fold = no_fold;
+    base.norm = llsa_norm_back{};
     // pooled level l: N / 16^l tokens per (b,h), contiguous (B,H,n,64) gradients
     auto level_tokens = [&](int l) {
         int n = N;
@@ -1262,7 +1436,16 @@ extern "C" int llsa_attn_bwd(const llsa_attn_bwd_args* a, void* stream) {
         while (BH % g != 0) g /= 2;
         p.stripes = kXcds / g;
         p.stripe_len = max_items / p.stripes + 2;             // ceil(long / stripes) + ceil(short / stripes) at most
-        hipLaunchKernelGGL(attn_kside_kernel, dim3((unsigned)(p.stripe_len * p.stripes * BH)), dim3(64), 0, s, p);
+        p.norm = a->norm_k;
+        const dim3 grid((unsigned)(p.stripe_len * p.stripes * BH));
+        if (p.norm.x) {
+            hipLaunchKernelGGL(HIP_KERNEL_NAME(attn_kside_kernel<true>), grid, dim3(64), 0, s, p);
+            sums.in[n_sums] = p.norm.partials;
+            sums.out[n_sums] = p.norm.dgamma;
+            sums.rows[n_sums++] = (int64_t)N1 * BH;
+        } else {
+            hipLaunchKernelGGL(HIP_KERNEL_NAME(attn_kside_kernel<false>), grid, dim3(64), 0, s, p);
+        }
         add_job(p, chunk, N1 * a->T / chunk + 1, 0);
     };
     // pooled levels under an ancestor's selection, group-major (one launch for all of them, plus the dense level when it is small)
@@ -1295,6 +1478,7 @@ extern "C" int llsa_attn_bwd(const llsa_attn_bwd_args* a, void* stream) {
             j.n_units = sgm.n_units; j.chunk = 1; j.max_units = sgm.n_units;
             j.work_stride = 0; j.slot_stride = sgm.slots; j.n_chunks = 0;
             j.fold = no_fold;
+            j.norm = llsa_norm_back{};
         }
     };
     // dense coarsest level: every unit (16 pooled tokens) meets every query block; the query
@@ -1334,6 +1518,19 @@ extern "C" int llsa_attn_bwd(const llsa_attn_bwd_args* a, void* stream) {
         run_groups();
         run_dense();
         run_reduce();
+    }
+    if (n_sums > 0) {
+        // (rows of the first stage's results: at most as many as there are rows)
+        constexpr int kSumGroups = 128;
+        NormSums first = sums;
+        int groups = kSumGroups;
+        for (int i = 0; i < n_sums; i++) {
+            first.out[i] = const_cast<float*>(sums.in[i]);
+            groups = (int)std::min<int64_t>(groups, sums.rows[i]);
+        }
+        hipLaunchKernelGGL(norm_sums_kernel, dim3(groups, n_sums), dim3(1024), 0, s, first);
+        for (int i = 0; i < n_sums; i++) sums.rows[i] = groups;
+        hipLaunchKernelGGL(norm_sums_kernel, dim3(1, n_sums), dim3(1024), 0, s, sums);
     }
     return launch_status("attn_bwd");
 }

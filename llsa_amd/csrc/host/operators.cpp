@@ -5,7 +5,7 @@
 //               topk_dense / topk_cascade [+ topk_sparse ...]
 //               attn_fwd
 //               transpose_indices_multi  (second stream beside the attention kernel at the long sequences)
-//     backward  attn_bwd with fold_pooled = 1  (dq, dk, dv complete, rotated back) [+ rmsnorm_bwd]
+//     backward  attn_bwd with fold_pooled = 1  (dq, dk, dv complete, rotated back and back through the qk-norm)
 //
 // Native because at the short sequences a step is bound by its host side: at B=1, H=6, N=1024 the kernels of a forward
 // take about 20 us and those of a forward + backward 70, while the same sequence issued from Python took 33 and 100 to
@@ -103,8 +103,6 @@ struct Library {
     decltype(&llsa_fine_chunk) fine_chunk;
     decltype(&llsa_attn_bwd_workspace_bytes) attn_bwd_workspace_bytes;
     decltype(&llsa_attn_bwd) attn_bwd;
-    decltype(&llsa_rmsnorm_bwd_partials) rmsnorm_bwd_partials;
-    decltype(&llsa_rmsnorm_bwd) rmsnorm_bwd;
     decltype(&llsa_gather_rows) gather_rows;
     bool device;                          // false: the CPU emulation build the tests install
 
@@ -123,8 +121,6 @@ struct Library {
         get("llsa_fine_chunk", fine_chunk);
         get("llsa_attn_bwd_workspace_bytes", attn_bwd_workspace_bytes);
         get("llsa_attn_bwd", attn_bwd);
-        get("llsa_rmsnorm_bwd_partials", rmsnorm_bwd_partials);
-        get("llsa_rmsnorm_bwd", rmsnorm_bwd);
         get("llsa_gather_rows", gather_rows);
     }
     void check(int rc, const char* what) const {
@@ -321,23 +317,26 @@ struct LlsaBackward : public Node {
         if (fr.defined()) a.freq_dq = a.freq_dk = fr.data_ptr();
         a.B = static_cast<int32_t>(B); a.H = static_cast<int32_t>(H); a.N = static_cast<int32_t>(N); a.T = y.topk[0]; a.levels = y.L;
         a.fold_pooled = 1;
-        void* const stream = lib->stream(out);
-        lib->check(lib->attn_bwd(&a, stream), "attn_bwd");
-        Tensor dgq, dgk;
-        if (wq.defined() || wk.defined()) {                  // back through the qk-norm, in place on dq / dk
+        Tensor dgq, dgk, P;
+        if (wq.defined() || wk.defined()) {                  // back through the qk-norm, inside the kernels that write dq and dk
             const auto f32 = opts.dtype(at::kFloat);
-            const Tensor P = at::empty({lib->rmsnorm_bwd_partials(a.B, a.H, a.N)}, f32);
-            auto norm = [&](const Tensor& gamma, const Tensor& x, Tensor& dx, at::ScalarType type) {
-                Tensor dg = at::empty({64}, f32);
-                lib->check(lib->rmsnorm_bwd(dx.data_ptr(), dx.strides().data(), x.data_ptr(), x.strides().data(), gamma.data_ptr<float>(),
-                                            static_cast<float>(eps), dx.data_ptr(), dx.strides().data(), dg.data_ptr<float>(), P.data_ptr<float>(),
-                                            a.B, a.H, a.N, stream),
-                           "rmsnorm_bwd");
-                return dg.to(type);
+            const int64_t rows = B * H * (N / 16);
+            P = at::empty({2 * rows * 64}, f32);
+            auto norm = [&](llsa_norm_back& nb, const Tensor& gamma, const Tensor& x, int64_t at) {
+                const Tensor dg = at::empty({64}, f32);
+                nb.x = x.data_ptr(); nb.sxb = x.stride(0); nb.sxh = x.stride(1); nb.sxn = x.stride(2);
+                nb.gamma = gamma.data_ptr<float>();
+                nb.dgamma = dg.data_ptr<float>();
+                nb.partials = P.data_ptr<float>() + at;
+                nb.eps = static_cast<float>(eps);
+                return dg;
             };
-            if (wq.defined()) dgq = norm(wq, q.unpack(), dq, type_gq);
-            if (wk.defined()) dgk = norm(wk, k.unpack(), dk, type_gk);
+            if (wq.defined()) dgq = norm(a.norm_q, wq, q.unpack(), 0);
+            if (wk.defined()) dgk = norm(a.norm_k, wk, k.unpack(), rows * 64);
         }
+        lib->check(lib->attn_bwd(&a, lib->stream(out)), "attn_bwd");
+        if (dgq.defined()) dgq = dgq.to(type_gq);
+        if (dgk.defined()) dgk = dgk.to(type_gk);
         variable_list r{dq, dk, dv};
         if (has_gq) r.push_back(dgq);
         if (has_gk) r.push_back(dgk);
