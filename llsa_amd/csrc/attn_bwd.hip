@@ -59,21 +59,22 @@ __device__ __forceinline__ void read_k_t(PairT& o, const bf16* k0, const bf16* k
     }
 }
 // dS^T of a pair of key blocks, as the B operand of the dQ product
-// (lse2w: the query's log-sum-exp minus log2 of the segment's weight, log2 units: the weight rides in the exponent)
-__device__ __forceinline__ bf16x8 dq_scores(const PairR& p, const bf16x8 bq[2], const bf16x8 bdo[2], float lse2w,
-                                            float delta) {
+// (nlse2w: log2 of the segment's weight minus the query's log-sum-exp, log2 units: the weight rides in the exponent; ndl:
+// -delta in all four places, what the product dP starts from, which saves a subtraction per score)
+__device__ __forceinline__ bf16x8 dq_scores(const PairR& p, const bf16x8 bq[2], const bf16x8 bdo[2], float nlse2w,
+                                            const f32x4& ndl) {
     bf16x8 bds;
 #pragma unroll
     for (int j = 0; j < 2; j++) {
-        f32x4 s = {0.f, 0.f, 0.f, 0.f}, dp = {0.f, 0.f, 0.f, 0.f};
+        f32x4 s = {0.f, 0.f, 0.f, 0.f}, dp = ndl;
         s = mfma_bf16(p.k[j][0], bq[0], s);
         s = mfma_bf16(p.k[j][1], bq[1], s);
         dp = mfma_bf16(p.v[j][0], bdo[0], dp);
         dp = mfma_bf16(p.v[j][1], bdo[1], dp);
 #pragma unroll
         for (int e = 0; e < 4; e++) {
-            const float pe = exp2_fast(fmaf(s[e], kScaleLog2e, -lse2w));
-            bds[j * 4 + e] = (bf16)(pe * (dp[e] - delta));
+            const float pe = exp2_fast(fmaf(s[e], kScaleLog2e, nlse2w));
+            bds[j * 4 + e] = (bf16)(pe * dp[e]);
         }
     }
     return bds;
@@ -138,10 +139,18 @@ __device__ __forceinline__ float norm_contrib_sum(const float (&contrib)[16], in
     return s;
 }
 
+// What the K-side kernels need of a query block besides its tiles, as their products take it: minus the log-sum-exp (log2
+// units) of its 16 queries, then minus their deltas, one 128-byte line per block.
+// (The products dP start from minus delta, and the exponent is one multiply-add: 16 + 8 of 136 vector-ALU slots a score pair in the
+// dense K side, 16 of 120 in the dQ kernel, which are half and two thirds busy with them: step of 6 x 262144 tokens with the
+// forward's share 4404 -> 4263 us, of 12 x 16384 337 -> 330.)
+constexpr int kStats = 2 * kBlk;
+
 // What a wave keeps per query block
 struct DqSide {
     bf16x8 bq[2], bdo[2];          // R operands of q and dO
-    float lse2, dl;                // log-sum-exp (log2 units) and delta of query l%16
+    float nlse2;                   // -log-sum-exp (log2 units) of query l%16
+    f32x4 ndl;                     // -delta of query l%16, four times
     f32x4 dq[4];                   // dQ^T: channel 16*dt + 4*(l/16) + e of query l%16
 };
 
@@ -149,7 +158,7 @@ struct DqSide {
 // (lane l: row l%16, channels 8*(l/16)..+7 and 32 + 8*(l/16)..+7).  The wave also does the
 // pre-pass the K-side kernels need: delta = rowsum(O * dO) in fp32 (the reference sums in the
 // tensor dtype, sparse_attention_res_1.py:153-177) and dO as an R tile.
-__device__ __forceinline__ void dq_begin(DqSide& sd, const llsa_attn_bwd_args& a, float* __restrict__ delta, bf16* __restrict__ dor,
+__device__ __forceinline__ void dq_begin(DqSide& sd, const llsa_attn_bwd_args& a, float* __restrict__ stats, bf16* __restrict__ dor,
                                          int bh, int b, int h, int g, int lane) {
     const int N1 = a.N / kBlk, r = lane & 15, quad = lane >> 4, tok = g * kBlk + r;
     const bf16* qp = (const bf16*)a.qr + ((int64_t)bh * N1 + g) * kTile + lane * 8;
@@ -165,12 +174,13 @@ __device__ __forceinline__ void dq_begin(DqSide& sd, const llsa_attn_bwd_args& a
     for (int e = 0; e < 8; e++) acc += (float)o0[e] * (float)sd.bdo[0][e];
 #pragma unroll
     for (int e = 0; e < 8; e++) acc += (float)o1[e] * (float)sd.bdo[1][e];
-    sd.dl = quad_sum(acc);
+    const float ndl = -quad_sum(acc);
+    sd.ndl = f32x4{ndl, ndl, ndl, ndl};
     bf16* tile = dor + ((int64_t)bh * N1 + g) * kTile + lane * 8;
     st16(tile, sd.bdo[0]);
     st16(tile + 512, sd.bdo[1]);
-    if (quad == 0) delta[(int64_t)bh * a.N + tok] = sd.dl;
-    sd.lse2 = a.lse[(int64_t)bh * a.N + tok] * kLog2e;
+    sd.nlse2 = -a.lse[(int64_t)bh * a.N + tok] * kLog2e;
+    if (quad < 2) stats[((int64_t)bh * N1 + g) * kStats + lane] = quad == 0 ? sd.nlse2 : ndl;
 #pragma unroll
     for (int dt = 0; dt < 4; dt++) sd.dq[dt] = f32x4{0.f, 0.f, 0.f, 0.f};
 }
@@ -193,7 +203,7 @@ __device__ __forceinline__ void dq_end(const DqSide& sd, const llsa_attn_bwd_arg
 }
 // in0, in1 (wave-uniform): whether the query block reads the pair's first / second block
 __device__ __forceinline__ void dq_pair_of_blocks(DqSide& sd, const PairR& r, const PairT& t, float log2w, bool in0 = true, bool in1 = true) {
-    bf16x8 bds = dq_scores(r, sd.bq, sd.bdo, sd.lse2 - log2w, sd.dl);
+    bf16x8 bds = dq_scores(r, sd.bq, sd.bdo, sd.nlse2 + log2w, sd.ndl);
 #pragma unroll
     for (int e = 0; e < 4; e++) {
         if (!in0) bds[e] = (bf16)0.f;
@@ -206,7 +216,7 @@ __device__ __forceinline__ void dq_pair_of_blocks(DqSide& sd, const PairR& r, co
 // -- from memory and, what weighs more here, from LDS, where every key block is read three times (K rows, V rows, K
 // transposed) -- and multiplied twice.
 template <int Q, int R, bool NORM>
-__global__ __launch_bounds__(256, Q == 1 ? 4 : 3) void attn_dq_kernel(llsa_attn_bwd_args a, float* __restrict__ delta,
+__global__ __launch_bounds__(256, Q == 1 ? 4 : 3) void attn_dq_kernel(llsa_attn_bwd_args a, float* __restrict__ stats,
                                                                       bf16* __restrict__ dor) {
     __shared__ __align__(16) bf16 sh[2][kGroup][2 * kTile];   // per block: R tile of K, R tile of V
     __shared__ int order[4][R * kWave];
@@ -240,7 +250,7 @@ __global__ __launch_bounds__(256, Q == 1 ? 4 : 3) void attn_dq_kernel(llsa_attn_
 
     DqSide sd[Q];
 #pragma unroll
-    for (int u = 0; u < Q; u++) dq_begin(sd[u], a, delta, dor, bh, b, h, g + u, lane);
+    for (int u = 0; u < Q; u++) dq_begin(sd[u], a, stats, dor, bh, b, h, g + u, lane);
 
     // ---- pooled blocks out of the shared copy.  The barrier at the top of round grp says: every
     // wave's part of group grp has landed, and every wave is done reading the other buffer.  All
@@ -385,7 +395,7 @@ constexpr int kFoldElems = kFoldRows + kBlk * kD;
 
 struct KSideParams {
     const bf16* qr;  const bf16* dor;             // R tiles of q and dO, (BH, N1, 1024)
-    const float* lse; const float* delta;         // (BH, N)
+    const float* stats;                           // (BH, N1, kStats)
     const bf16* kk;  const bf16* vv;              // R tiles the unit's 16 key rows come from, (BH, n_units, 1024)
     const int* off;  const int* flat;             // CSR of the transposed selection (per K block)
     const int* work;                              // work list over that CSR (see transpose.hip)
@@ -403,7 +413,7 @@ struct KSideParams {
 };
 
 // Two query blocks against the unit's 16 key rows, operands out of a wave-private piece of LDS: `stage` holds the
-// R tiles of Q and dO of the two blocks (block u: Q at 2u, dO at 2u + 1), `stats` their lse and delta rows.  The tiles
+// R tiles of Q and dO of the two blocks (block u: Q at 2u, dO at 2u + 1), `stats` their statistics (kStats each).  The tiles
 // are read twice, plainly as the A operands of S = Q.K^T and dP = dO.V^T and with the transposing read as the T
 // operands of dV^T += dO^T.P and dK^T += Q^T.dS.
 struct KsideOperands {
@@ -426,8 +436,8 @@ __device__ __forceinline__ void kside_read(KsideOperands& o, const bf16* stage, 
             o.tq[u][dt] = lds_t_operand(q, dt, lane);
             o.tg[u][dt] = lds_t_operand(g, dt, lane);
         }
-        o.l4[u] = *reinterpret_cast<const f32x4*>(stats + u * 32 + quad * 4);
-        o.d4[u] = *reinterpret_cast<const f32x4*>(stats + u * 32 + 16 + quad * 4);
+        o.l4[u] = *reinterpret_cast<const f32x4*>(stats + u * kStats + quad * 4);
+        o.d4[u] = *reinterpret_cast<const f32x4*>(stats + u * kStats + kBlk + quad * 4);
     }
 }
 __device__ __forceinline__ void kside_pair(f32x4 dk[4], f32x4 dv[4], const bf16x8 bk[2], const bf16x8 bv[2], const KsideOperands& o,
@@ -435,17 +445,17 @@ __device__ __forceinline__ void kside_pair(f32x4 dk[4], f32x4 dv[4], const bf16x
     bf16x8 bp, bds;
 #pragma unroll
     for (int u = 0; u < 2; u++) {
-        f32x4 s = {0.f, 0.f, 0.f, 0.f}, dp = {0.f, 0.f, 0.f, 0.f};
+        f32x4 s = {0.f, 0.f, 0.f, 0.f}, dp = o.d4[u];
         s = mfma_bf16(o.aq[u][0], bk[0], s);
         s = mfma_bf16(o.aq[u][1], bk[1], s);
         dp = mfma_bf16(o.ag[u][0], bv[0], dp);
         dp = mfma_bf16(o.ag[u][1], bv[1], dp);
 #pragma unroll
         for (int e = 0; e < 4; e++) {
-            float pe = exp2_fast(fmaf(s[e], kScaleLog2e, -o.l4[u][e] * kLog2e));
+            float pe = exp2_fast(fmaf(s[e], kScaleLog2e, o.l4[u][e]));
             if (u == 1 && !second_valid) pe = 0.f;
             bp[u * 4 + e] = (bf16)pe;
-            bds[u * 4 + e] = (bf16)(pe * (dp[e] - o.d4[u][e]));
+            bds[u * 4 + e] = (bf16)(pe * dp[e]);
         }
     }
 #pragma unroll
@@ -485,7 +495,7 @@ __device__ __forceinline__ bool kside_item(const KSideParams& p, int& bh, int& i
 template <bool NORM>
 __global__ __launch_bounds__(64) void attn_kside_kernel(KSideParams p) {
     __shared__ __align__(16) bf16 stage[4 * kTile];           // 2 query blocks x {Q, dO} R tiles
-    __shared__ __align__(16) float stats[64];                 // their lse and delta rows
+    __shared__ __align__(16) float stats[64];                 // their statistics
     __shared__ __align__(16) bf16 fold_buf[kFoldElems];
     int bh, item;
     if (!kside_item(p, bh, item)) return;
@@ -560,8 +570,7 @@ __global__ __launch_bounds__(64) void attn_kside_kernel(KSideParams p) {
         bv[1] = ld16(vp + 512);
         const bf16* qrb = p.qr + (int64_t)bh * N1 * kTile;
         const bf16* dorb = p.dor + (int64_t)bh * N1 * kTile;
-        const float* lseb = p.lse + (int64_t)bh * p.N;
-        const float* dlb = p.delta + (int64_t)bh * p.N;
+        const float* stb = p.stats + (int64_t)bh * N1 * kStats;
         // The operands of entries i, i + 1 are copied straight into LDS (no registers) while entries i - 2, i - 1 are
         // worked on: a round reads everything it needs out of LDS first, then starts the next copy into the same
         // place, then does its arithmetic.
@@ -580,8 +589,8 @@ __global__ __launch_bounds__(64) void attn_kside_kernel(KSideParams p) {
             copy16_global_to_lds(q1 + 512, stage + 2 * kTile + 512);
             copy16_global_to_lds(d1, stage + 3 * kTile);
             copy16_global_to_lds(d1 + 512, stage + 3 * kTile + 512);
-            if (lane < 16) {                                  // four floats a lane: lse g0, delta g0, lse g1, delta g1
-                const float* src = ((lane & 4) ? dlb : lseb) + ((lane & 8) ? g1 : g0) * kBlk + (lane & 3) * 4;
+            if (lane < 16) {                                  // four floats a lane: the statistics of g0, of g1
+                const float* src = stb + (int64_t)((lane & 8) ? g1 : g0) * kStats + (lane & 7) * 4;
                 copy16_global_to_lds(reinterpret_cast<const bf16*>(src), reinterpret_cast<bf16*>(stats));
             }
         };
@@ -669,7 +678,7 @@ constexpr int kDenseWaves = 4;                    // waves per workgroup
 template <int UPW>
 __global__ __launch_bounds__(64 * kDenseWaves) void attn_kside_dense_kernel(KSideParams p) {
     __shared__ __align__(16) bf16 sh[2][4 * kTile];           // per pair: Q0, dO0, Q1, dO1 as R tiles
-    __shared__ __align__(16) float sh_stats[2][64];           // per pair: lse of its 32 queries, then delta
+    __shared__ __align__(16) float sh_stats[2][64];           // per pair: the statistics of its two query blocks
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int quad = lane >> 4;
@@ -687,8 +696,7 @@ __global__ __launch_bounds__(64 * kDenseWaves) void attn_kside_dense_kernel(KSid
     if (n_pairs <= 0) return;                                 // uniform over the workgroup
     const bf16* qrb = p.qr + ((int64_t)bh * N1 + start) * kTile;
     const bf16* dorb = p.dor + ((int64_t)bh * N1 + start) * kTile;
-    const float* lseb = p.lse + (int64_t)bh * p.N + start * kBlk;
-    const float* dlb = p.delta + (int64_t)bh * p.N + start * kBlk;
+    const float* stb = p.stats + ((int64_t)bh * N1 + start) * kStats;
 
     // wave w moves tile w of a pair's four (query block w/2; Q for even w, dO for odd w); the first 16 lanes of wave 0
     // also its 64 statistics.  Rounds past the end re-read the last pair (no branch around loads).
@@ -702,7 +710,7 @@ __global__ __launch_bounds__(64 * kDenseWaves) void attn_kside_dense_kernel(KSid
         // (every lane of every wave loads, lanes 16.. the same as lane % 16: a load inside a branch makes the compiler lose
         // count of the loads in flight, after which it waits for all of them in every round)
         const int sl = lane & 15;
-        st.s = *reinterpret_cast<const f32x4*>((sl < 8 ? lseb : dlb) + 2 * t * kBlk + (sl & 7) * 4);
+        st.s = *reinterpret_cast<const f32x4*>(stb + (int64_t)(2 * t) * kStats + sl * 4);
     };
     auto deposit = [&](int t, const Stage& st) __attribute__((always_inline)) {
         bf16* dst = &sh[t & 1][wave * kTile];
@@ -755,32 +763,27 @@ __global__ __launch_bounds__(64 * kDenseWaves) void attn_kside_dense_kernel(KSid
                 tq[u][dt] = lds_t_operand(b + (2 * u) * kTile, dt, lane);
                 tg[u][dt] = lds_t_operand(b + (2 * u + 1) * kTile, dt, lane);
             }
-            l4[u] = *reinterpret_cast<const f32x4*>(&sh_stats[t & 1][u * kBlk + quad * 4]);
-            d4[u] = *reinterpret_cast<const f32x4*>(&sh_stats[t & 1][32 + u * kBlk + quad * 4]);
+            l4[u] = *reinterpret_cast<const f32x4*>(&sh_stats[t & 1][u * kStats + quad * 4]);
+            d4[u] = *reinterpret_cast<const f32x4*>(&sh_stats[t & 1][u * kStats + kBlk + quad * 4]);
         }
         deposit(t + 1, nxt);
         request(t + 3, nxt);
         if (!active) return;
-        float nl[2][4];
-#pragma unroll
-        for (int u = 0; u < 2; u++)
-#pragma unroll
-            for (int e = 0; e < 4; e++) nl[u][e] = -l4[u][e] * kLog2e;
 #pragma unroll
         for (int j = 0; j < UPW; j++) {
             bf16x8 bp, bds;
 #pragma unroll
             for (int u = 0; u < 2; u++) {
-                f32x4 s = {0.f, 0.f, 0.f, 0.f}, dp = {0.f, 0.f, 0.f, 0.f};
+                f32x4 s = {0.f, 0.f, 0.f, 0.f}, dp = d4[u];
                 s = mfma_bf16(aq[u][0], bk[j][0], s);
                 s = mfma_bf16(aq[u][1], bk[j][1], s);
                 dp = mfma_bf16(ag[u][0], bv[j][0], dp);
                 dp = mfma_bf16(ag[u][1], bv[j][1], dp);
 #pragma unroll
                 for (int e = 0; e < 4; e++) {
-                    const float pe = exp2_fast(fmaf(s[e], kScaleLog2e, nl[u][e]));
+                    const float pe = exp2_fast(fmaf(s[e], kScaleLog2e, l4[u][e]));
                     bp[u * 4 + e] = (bf16)pe;
-                    bds[u * 4 + e] = (bf16)(pe * (dp[e] - d4[u][e]));
+                    bds[u * 4 + e] = (bf16)(pe * dp[e]);
                 }
             }
 #pragma unroll
@@ -847,7 +850,7 @@ struct GroupSeg {
 };
 struct GroupParams {
     const bf16* qr; const bf16* dor;              // R tiles of q and dO, (BH, N1, 1024)
-    const float* lse; const float* delta;         // (BH, N)
+    const float* stats;                           // (BH, N1, kStats)
     int H, N, n_segs, n_blocks;
     GroupSeg seg[kGroupSegs];
 };
@@ -857,7 +860,7 @@ struct GroupStats { f32x4 l[2], d[2]; };
 // UPW key blocks against the group's 16 query blocks, two query blocks per step, operands out of LDS.
 template <int UPW>
 __device__ __forceinline__ void group_pass(const bf16x8 (&bk)[2][2], const bf16x8 (&bv)[2][2], const float (&w)[2], bf16x8* const (&dst)[2],
-                                           const bf16* shq, const bf16* shg, const float* lseb, const float* dlb, int lane) {
+                                           const bf16* shq, const bf16* shg, const float* stb, int lane) {
     const int quad = lane >> 4;
     f32x4 dk[UPW][4], dv[UPW][4];
 #pragma unroll
@@ -870,8 +873,8 @@ __device__ __forceinline__ void group_pass(const bf16x8 (&bk)[2][2], const bf16x
     auto load_stats = [=](int t, GroupStats& st) __attribute__((always_inline)) {
 #pragma unroll
         for (int u = 0; u < 2; u++) {
-            st.l[u] = *reinterpret_cast<const f32x4*>(lseb + (2 * t + u) * kBlk + quad * 4);
-            st.d[u] = *reinterpret_cast<const f32x4*>(dlb + (2 * t + u) * kBlk + quad * 4);
+            st.l[u] = *reinterpret_cast<const f32x4*>(stb + (2 * t + u) * kStats + quad * 4);
+            st.d[u] = *reinterpret_cast<const f32x4*>(stb + (2 * t + u) * kStats + kBlk + quad * 4);
         }
     };
     auto step = [&](int t, const GroupStats& cur) __attribute__((always_inline)) {
@@ -891,26 +894,21 @@ __device__ __forceinline__ void group_pass(const bf16x8 (&bk)[2][2], const bf16x
                 tg[u][dt] = lds_t_operand(g, dt, lane);
             }
         }
-        float nl[2][4];
-#pragma unroll
-        for (int u = 0; u < 2; u++)
-#pragma unroll
-            for (int e = 0; e < 4; e++) nl[u][e] = -cur.l[u][e] * kLog2e;
 #pragma unroll
         for (int j = 0; j < UPW; j++) {
             bf16x8 bp, bds;
 #pragma unroll
             for (int u = 0; u < 2; u++) {
-                f32x4 sc = {0.f, 0.f, 0.f, 0.f}, dp = {0.f, 0.f, 0.f, 0.f};
+                f32x4 sc = {0.f, 0.f, 0.f, 0.f}, dp = cur.d[u];
                 sc = mfma_bf16(aq[u][0], bk[j][0], sc);
                 sc = mfma_bf16(aq[u][1], bk[j][1], sc);
                 dp = mfma_bf16(ag[u][0], bv[j][0], dp);
                 dp = mfma_bf16(ag[u][1], bv[j][1], dp);
 #pragma unroll
                 for (int e = 0; e < 4; e++) {
-                    const float pe = exp2_fast(fmaf(sc[e], kScaleLog2e, nl[u][e]));   // (the weight multiplies the sums below)
+                    const float pe = exp2_fast(fmaf(sc[e], kScaleLog2e, cur.l[u][e]));   // (the weight multiplies the sums below)
                     bp[u * 4 + e] = (bf16)pe;
-                    bds[u * 4 + e] = (bf16)(pe * (dp[e] - cur.d[u][e]));
+                    bds[u * 4 + e] = (bf16)(pe * dp[e]);
                 }
             }
 #pragma unroll
@@ -984,8 +982,7 @@ __global__ __launch_bounds__(64 * kGroupWaves, 2) void attn_kside_group_kernel(G
             }
         }
     }
-    const float* lseb = p.lse + (int64_t)bh * p.N + (int64_t)G * kBlk * kBlk;
-    const float* dlb = p.delta + (int64_t)bh * p.N + (int64_t)G * kBlk * kBlk;
+    const float* stb = p.stats + ((int64_t)bh * N1 + (int64_t)G * kBlk) * kStats;
     // this wave's key blocks: a contiguous share, taken two at a time (the last alone if the share is odd)
     const int per = (p.n_blocks + kGroupWaves - 1) / kGroupWaves;
     const int lo = min(wave * per, p.n_blocks), hi = min(lo + per, p.n_blocks);
@@ -1017,8 +1014,8 @@ __global__ __launch_bounds__(64 * kGroupWaves, 2) void attn_kside_group_kernel(G
             fetch(j, 0);
             if (two) fetch(j + 1, 1);
         }
-        if (two) group_pass<2>(bk, bv, w, dst, &sh[0][0], &sh[1][0], lseb, dlb, lane);
-        else group_pass<1>(bk, bv, w, dst, &sh[0][0], &sh[1][0], lseb, dlb, lane);
+        if (two) group_pass<2>(bk, bv, w, dst, &sh[0][0], &sh[1][0], stb, lane);
+        else group_pass<1>(bk, bv, w, dst, &sh[0][0], &sh[1][0], stb, lane);
     }
 }
 
@@ -1254,7 +1251,7 @@ static int64_t align256(int64_t x) { return (x + 255) & ~(int64_t)255; }
 constexpr int64_t kSlotBytes = 8 * kWave * sizeof(f32x4);     // one partial: 16 rows x 64 ch x (dK, dV) fp32
 
 struct BwdWorkspace {
-    int64_t delta, dor, part_fine, part_dense, total;
+    int64_t stats, dor, part_fine, part_dense, total;
     int64_t part_level[LLSA_MAX_LEVELS];                        // partial sums of pooled level l (below the coarsest) at [l - 1]
     int64_t slots_fine, slots_level[LLSA_MAX_LEVELS];           // per (b,h)
 };
@@ -1268,7 +1265,7 @@ static BwdWorkspace bwd_workspace(int B, int H, int N, const int32_t* topk, int 
     // E/chunk such blocks with at most E/chunk + E/chunk chunks in total
     w.slots_fine = 2 * (N1 * topk[0] / fine_chunk(N)) + 2;
     int64_t o = 0;
-    w.delta = o;        o += align256(BH * N * 4);
+    w.stats = o;        o += align256(BH * N / kBlk * kStats * 4);
     w.dor = o;          o += align256(BH * N * 64 * 2);
     w.part_fine = o;    o += align256(BH * w.slots_fine * kSlotBytes);
     // group-major pooled passes: one partial sum per (group of 16 query blocks, entry of its ancestor's list)
@@ -1337,7 +1334,7 @@ extern "C" int llsa_attn_bwd(const llsa_attn_bwd_args* a, void* stream) {
     const int B = a->B, H = a->H, N = a->N, N1 = N / 16, N2 = N1 / 16, BH = B * H, L = a->levels;
     const DensePlan d = dense_plan(B, H, N, L);
     char* ws = (char*)a->workspace;
-    float* delta = (float*)(ws + wsp.delta);
+    float* stats = (float*)(ws + wsp.stats);
     bf16* dor = (bf16*)(ws + wsp.dor);
     const bool fold = a->fold_pooled != 0;
     LLSA_REQUIRE(fold || a->freq_dk == nullptr, "attn_bwd: freq_dk needs fold_pooled");
@@ -1359,8 +1356,8 @@ extern "C" int llsa_attn_bwd(const llsa_attn_bwd_args* a, void* stream) {
         const dim3 grid(N1 / (pairs ? 8 : 4), BH);
 #define LLSA_DQ(Q, R)                                                                                                                  \
     do {                                                                                                                               \
-        if (a->norm_q.x) hipLaunchKernelGGL(HIP_KERNEL_NAME(attn_dq_kernel<Q, R, true>), grid, dim3(256), 0, s, *a, delta, dor);       \
-        else hipLaunchKernelGGL(HIP_KERNEL_NAME(attn_dq_kernel<Q, R, false>), grid, dim3(256), 0, s, *a, delta, dor);                  \
+        if (a->norm_q.x) hipLaunchKernelGGL(HIP_KERNEL_NAME(attn_dq_kernel<Q, R, true>), grid, dim3(256), 0, s, *a, stats, dor);       \
+        else hipLaunchKernelGGL(HIP_KERNEL_NAME(attn_dq_kernel<Q, R, false>), grid, dim3(256), 0, s, *a, stats, dor);                  \
     } while (0)
         if (!pairs) LLSA_DQ(1, 1);
         else if (a->T <= 32) LLSA_DQ(2, 1);
@@ -1401,7 +1398,7 @@ extern "C" int llsa_attn_bwd(const llsa_attn_bwd_args* a, void* stream) {
     };
     KSideParams base;
     base.qr = (const bf16*)a->qr; base.dor = dor;
-    base.lse = a->lse; base.delta = delta;
+    base.stats = stats;
     base.H = H; base.N = N; base.chunk_len = 0;
     base.fold = no_fold;
     base.norm = llsa_norm_back{};
@@ -1452,7 +1449,7 @@ extern "C" int llsa_attn_bwd(const llsa_attn_bwd_args* a, void* stream) {
     auto run_groups = [&]() {
         if (L < 2 || !(stages & LLSA_BWD_DPKV1)) return;
         GroupParams g;
-        g.qr = (const bf16*)a->qr; g.dor = dor; g.lse = a->lse; g.delta = delta;
+        g.qr = (const bf16*)a->qr; g.dor = dor; g.stats = stats;
         g.H = H; g.N = N; g.n_segs = 0; g.n_blocks = 0;
         auto add_seg = [&](const void* kk, const void* vv, const int* sel, const int* inv, int64_t part_off, int n_units, int shift,
                            int cnt, int64_t slots, float w) {

@@ -21,20 +21,18 @@
 
 namespace llsa {
 
-constexpr float kMaxSlack = 8.f;     // log2 units
-constexpr int NB = 2;                // 16-key blocks per pipeline step: 32 keys, one K step of the second product
+constexpr float kMaxSum = 256.f;
 
 struct SoftmaxState {
-    float m2;        // reference point of the exponentials (at most kMaxSlack below the running max), log2 units
+    float m2;        // reference point of the exponentials (at most log2(kMaxSum) below the running max), log2 units
     f32x4 acc[4];    // O^T: channel 16*dt + 4*(l/16) + e of query l%16, in units of the current weight
     float lsum;      // this lane's share of the running sum of the query's p
 };
 
-// Operands of one step = NB 16-key blocks, as they sit in registers between load and use.
-struct KvRegs {
-    bf16x8 k[NB][2];     // K rows (R tile): block j, channel half
-    bf16x8 v[NB / 2][4]; // V (T tiles of a pair of blocks): channel tile dt, keys 4*(l/16)..+3 of the first block, then of the second
-};
+// Operands of one step = NB 16-key blocks (NB even: a pair of blocks is one K step of the second product), as they sit in
+// registers between load and use.
+template <int NB> struct KeyRegs { bf16x8 k[NB][2]; };       // K rows (R tile): block j, channel half
+template <int NB> struct ValueRegs { bf16x8 v[NB / 2][4]; }; // V (T tiles of a pair of blocks): channel tile dt, keys 4*(l/16)..+3 of the first block, then of the second
 
 __device__ __forceinline__ void init_state(SoftmaxState& st) {
     st.m2 = 0.f;
@@ -50,21 +48,23 @@ __device__ __forceinline__ void rescale(SoftmaxState& st, float f) {
     for (int dt = 0; dt < 4; dt++) st.acc[dt] *= f;
 }
 
-// The exponentials refer to st.m2, which follows the running maximum lazily: it moves only when the maximum
-// has grown by more than kMaxSlack (then p <= 2^kMaxSlack, harmless in bf16 and in the fp32 sums), so that the
-// accumulator is rescaled a few times per query block instead of at most steps; O = acc / sum and
-// lse = m2 + log2(sum) hold for any reference point.  The common path therefore needs no maximum over the quad
-// of lanes that share a query: every lane checks its own exponents against the slack, and only when one in the
-// wave exceeds it is the reference point moved (for all four lanes of a query alike, by the quad's largest
-// exponent).  st.m2 starts at the largest score of the first block (start_reference), so it is always finite.
-__device__ __forceinline__ void start_reference(SoftmaxState& st, const bf16x8 bq[2], const KvRegs& t) {
+// The exponentials refer to st.m2, which follows the running maximum lazily: it moves only when p has become large
+// (some lane's eight p of a step add up to more than kMaxSum; smaller ones are harmless in bf16 and in the fp32 sums), so
+// that the accumulator is rescaled a few times per query block instead of at most steps; O = acc / sum and
+// lse = m2 + log2(sum) hold for any reference point.  The common path therefore needs no maximum, neither over the quad of
+// lanes that share a query nor over a lane's own exponents: the sum that is taken anyway tells (overflow included), and only
+// when one in the wave is too large is the reference point moved (for all four lanes of a query alike, by the quad's largest
+// exponent) and the step's p taken again.  st.m2 starts at the largest score of the first block (start_reference), so it is
+// always finite.
+__device__ __forceinline__ void start_reference(SoftmaxState& st, const bf16x8 bq[2], bf16x8 k0, bf16x8 k1) {
     f32x4 z = {0.f, 0.f, 0.f, 0.f};
-    const f32x4 s = mfma_bf16(t.k[0][1], bq[1], mfma_bf16(t.k[0][0], bq[0], z));
+    const f32x4 s = mfma_bf16(k1, bq[1], mfma_bf16(k0, bq[0], z));
     st.m2 = quad_max(fmaxf(fmaxf(s[0], s[1]), fmaxf(s[2], s[3]))) * kScaleLog2e;
 }
 
-// x: the exponents of one step (NB blocks) relative to st.m2
-__device__ __forceinline__ void exponents(float x[NB][4], const SoftmaxState& st, const bf16x8 bq[2], const KvRegs& t) {
+// x: the exponents of one step relative to st.m2
+template <int NB>
+__device__ __forceinline__ void exponents(float x[NB][4], const SoftmaxState& st, const bf16x8 bq[2], const KeyRegs<NB>& t) {
 #pragma unroll
     for (int j = 0; j < NB; j++) {
         f32x4 z = {0.f, 0.f, 0.f, 0.f};
@@ -73,36 +73,48 @@ __device__ __forceinline__ void exponents(float x[NB][4], const SoftmaxState& st
         for (int e = 0; e < 4; e++) x[j][e] = fmaf(s[e], kScaleLog2e, -st.m2);
     }
 }
-__device__ __forceinline__ float largest(const float x[NB][4]) {
+// p of one step as the B operands of the second product; returns the lane's sum of them.  (The empty asm keeps the compiler from
+// moving the conversion behind the branch that follows, where the fp32 values would occupy twice the registers.)
+template <int NB>
+__device__ __forceinline__ float probabilities(bf16x8 bp[NB / 2], const float x[NB][4]) {
+    float rs[2];
+#pragma unroll
+    for (int j = 0; j < NB; j++)
+#pragma unroll
+        for (int e = 0; e < 4; e++) {
+            const float p = exp2_fast(x[j][e]);
+            if (j < 2 && e == 0) rs[j] = p;
+            else rs[j & 1] += p;
+            bp[j >> 1][(j & 1) * 4 + e] = (bf16)p;
+        }
+#pragma unroll
+    for (int c = 0; c < NB / 2; c++) asm volatile("" : "+v"(bp[c]));
+    return rs[0] + rs[1];
+}
+// in0, in1 (wave-uniform): whether the query block reads the step's first / second block
+__device__ __forceinline__ void leave_out(float x[2][4], bool in0, bool in1) {
+    if (!in0) x[0][0] = x[0][1] = x[0][2] = x[0][3] = -INFINITY;
+    if (!in1) x[1][0] = x[1][1] = x[1][2] = x[1][3] = -INFINITY;
+}
+// the rare path, from the step's exponents taken once more: moves the reference point of every query whose largest one is above it
+template <int NB>
+__device__ __forceinline__ float move_reference(SoftmaxState& st, bf16x8 bp[NB / 2], float x[NB][4]) {
     float top = x[0][0];
 #pragma unroll
     for (int j = 0; j < NB; j++)
 #pragma unroll
         for (int e = 0; e < 4; e++) top = fmaxf(top, x[j][e]);
-    return top;
-}
-// the rare path: moves the reference point of every query whose largest exponent exceeds the slack
-__device__ __forceinline__ void move_reference(SoftmaxState& st, float x[NB][4], float top) {
-    top = quad_max(top);
-    const float shift = (top > kMaxSlack) ? top : 0.f;
+    const float shift = fmaxf(quad_max(top), 0.f);
     st.m2 += shift;
     rescale(st, exp2_fast(-shift));
 #pragma unroll
     for (int j = 0; j < NB; j++)
 #pragma unroll
         for (int e = 0; e < 4; e++) x[j][e] -= shift;
+    return probabilities<NB>(bp, x);
 }
-__device__ __forceinline__ void accumulate(SoftmaxState& st, const float x[NB][4], const KvRegs& t) {
-    bf16x8 bp[NB / 2];
-    float rs = 0.f;
-#pragma unroll
-    for (int j = 0; j < NB; j++)
-#pragma unroll
-        for (int e = 0; e < 4; e++) {
-            const float p = exp2_fast(x[j][e]);
-            rs += p;
-            bp[j >> 1][(j & 1) * 4 + e] = (bf16)p;
-        }
+template <int NB>
+__device__ __forceinline__ void accumulate(SoftmaxState& st, float rs, const bf16x8 bp[NB / 2], const ValueRegs<NB>& t) {
     st.lsum += rs;
 #pragma unroll
     for (int c = 0; c < NB / 2; c++)
@@ -111,42 +123,54 @@ __device__ __forceinline__ void accumulate(SoftmaxState& st, const float x[NB][4
             st.acc[dt] = mfma_bf16(t.v[c][dt], bp[c], st.acc[dt]);
 }
 
-// in0, in1 (wave-uniform): whether the query block reads the step's first / second block
-__device__ __forceinline__ void compute_step(SoftmaxState& st, const bf16x8 bq[2], const KvRegs& t, bool in0 = true, bool in1 = true) {
-    float x[NB][4];
-    exponents(x, st, bq, t);
-    if (!in0) x[0][0] = x[0][1] = x[0][2] = x[0][3] = -INFINITY;
-    if (!in1) x[1][0] = x[1][1] = x[1][2] = x[1][3] = -INFINITY;
-    const float top = largest(x);
-    if (__ballot(top > kMaxSlack) != 0) move_reference(st, x, top);
-    accumulate(st, x, t);
-}
-
-// The same step for two query blocks that read the same operands, written as one straight-line piece so that the
-// products of one block overlap with the exponentials of the other (one test for the rare path covers both).
-__device__ __forceinline__ void compute_step2(SoftmaxState& sa, SoftmaxState& sb, const bf16x8 qa[2], const bf16x8 qb[2], const KvRegs& t) {
-    float xa[NB][4], xb[NB][4];
-    exponents(xa, sa, qa, t);
-    exponents(xb, sb, qb, t);
-    const float ta = largest(xa), tb = largest(xb);
-    if (__ballot(fmaxf(ta, tb) > kMaxSlack) != 0) {
-        move_reference(sa, xa, ta);
-        move_reference(sb, xb, tb);
-    }
-    accumulate(sa, xa, t);
-    accumulate(sb, xb, t);
-}
-
-// Operands of one step out of the workgroup's LDS copy of shared blocks (4 KB per block: R tile
-// of the keys, then T tile of the values).
-__device__ __forceinline__ void load_step_shared(KvRegs& t, const bf16* blocks, int lane) {
+// One step of two blocks for Q query blocks that read the same operands, written as one straight-line piece so that the products of one query block overlap with the
+// exponentials of the other (one test for the rare path covers all).
+template <int Q>
+__device__ __forceinline__ void compute_step(SoftmaxState (&st)[Q], const bf16x8 (&bq)[Q][2], const KeyRegs<2>& k, const ValueRegs<2>& v) {
+    bf16x8 bp[Q][1];
+    float rs[Q], most = 0.f;
 #pragma unroll
-    for (int j = 0; j < NB; j++) {
+    for (int u = 0; u < Q; u++) {
+        float x[2][4];
+        exponents<2>(x, st[u], bq[u], k);
+        rs[u] = probabilities<2>(bp[u], x);
+        most = fmaxf(most, rs[u]);
+    }
+    if (__ballot(most > kMaxSum) != 0)
+#pragma unroll
+        for (int u = 0; u < Q; u++) {
+            float x[2][4];
+            exponents<2>(x, st[u], bq[u], k);
+            rs[u] = move_reference<2>(st[u], bp[u], x);
+        }
+#pragma unroll
+    for (int u = 0; u < Q; u++) accumulate<2>(st[u], rs[u], bp[u], v);
+}
+__device__ __forceinline__ void compute_step(SoftmaxState& st, const bf16x8 (&bq)[2], const KeyRegs<2>& k, const ValueRegs<2>& v, bool in0, bool in1) {
+    bf16x8 bp[1];
+    float x[2][4];
+    exponents<2>(x, st, bq, k);
+    leave_out(x, in0, in1);
+    float rs = probabilities<2>(bp, x);
+    if (__ballot(rs > kMaxSum) != 0) {
+        exponents<2>(x, st, bq, k);
+        leave_out(x, in0, in1);
+        rs = move_reference<2>(st, bp, x);
+    }
+    accumulate<2>(st, rs, bp, v);
+}
+
+// Operands out of the workgroup's LDS copy of shared blocks (4 KB per block: R tile of the keys, then T tile of the values).
+__device__ __forceinline__ void load_keys_shared(KeyRegs<kGroup>& t, const bf16* blocks, int lane) {
+#pragma unroll
+    for (int j = 0; j < kGroup; j++) {
         t.k[j][0] = lds_ld16(blocks + j * 2 * kTile + lane * 8);
         t.k[j][1] = lds_ld16(blocks + j * 2 * kTile + 512 + lane * 8);
     }
+}
+__device__ __forceinline__ void load_values_shared(ValueRegs<kGroup>& t, const bf16* blocks, int lane) {
 #pragma unroll
-    for (int c = 0; c < NB / 2; c++)
+    for (int c = 0; c < kGroup / 2; c++)
 #pragma unroll
         for (int dt = 0; dt < 4; dt++) {
             t.v[c][dt] = cat(lds_ld8(blocks + (2 * c) * 2 * kTile + kTile + dt * 256 + lane * 4),
@@ -156,12 +180,9 @@ __device__ __forceinline__ void load_step_shared(KvRegs& t, const bf16* blocks, 
 }
 // The values of a pair of fine blocks out of the wave's own copy of their R tiles: the transposing read makes the T operands.
 // (So the tokens' values need no T tile in memory, which would be a tenth of all that the pooling pass moves.)
-__device__ __forceinline__ void load_v_fine(KvRegs& t, const bf16* tiles, int lane) {
+__device__ __forceinline__ void load_values_fine(ValueRegs<2>& t, const bf16* tiles, int lane) {
 #pragma unroll
-    for (int c = 0; c < NB / 2; c++)
-#pragma unroll
-        for (int dt = 0; dt < 4; dt++)
-            t.v[c][dt] = cat(lds_t_operand(tiles + (2 * c) * kTile, dt, lane), lds_t_operand(tiles + (2 * c + 1) * kTile, dt, lane));
+    for (int dt = 0; dt < 4; dt++) t.v[0][dt] = cat(lds_t_operand(tiles, dt, lane), lds_t_operand(tiles + kTile, dt, lane));
 }
 
 __device__ __forceinline__ void finish_query_block(const llsa_attn_fwd_args& a, const SoftmaxState& st, int bh, int b, int h, int g, int lane) {
@@ -186,7 +207,6 @@ __device__ __forceinline__ void finish_query_block(const llsa_attn_fwd_args& a, 
 // tiles arrive from the L2, and waves enough to keep the fetches in flight.
 template <int Q, int R>
 __global__ __launch_bounds__(256, Q == 1 ? 4 : 3) void attn_fwd_kernel(llsa_attn_fwd_args a) {
-    static_assert(NB == 2 && kGroup == 4, "the shared phase reads an LDS buffer of four blocks as two steps of two");
     __shared__ __align__(16) bf16 sh[2][kGroup][2 * kTile];
     __shared__ int order[4][R * kWave];
     const int lane = threadIdx.x & 63;
@@ -224,13 +244,6 @@ __global__ __launch_bounds__(256, Q == 1 ? 4 : 3) void attn_fwd_kernel(llsa_attn
         bq[u][1] = ld16(qp + 512); // reference does) equals scaling the fp32 scores, done in the exponent
         init_state(st[u]);
     }
-    auto step_all = [&](const KvRegs& t) __attribute__((always_inline)) {    // the operands in t against every query block of the wave
-        if constexpr (Q == 1) compute_step(st[0], bq[0], t);
-        else
-#pragma unroll
-            for (int u = 0; u < Q; u += 2) compute_step2(st[u], st[u + 1], bq[u], bq[u + 1], t);
-    };
-
     // ---- shared blocks, out of LDS.  The barrier at the top of round grp says two things: every
     // wave's part of group grp has landed, and every wave is done reading the other buffer
     // (group grp - 1), which the next fetch overwrites.  (LDS reads of a group come before the next fetch: the compiler
@@ -247,16 +260,43 @@ __global__ __launch_bounds__(256, Q == 1 ? 4 : 3) void attn_fwd_kernel(llsa_attn
         }
         w_prev = w_here;
         const bf16* blk = &sh[grp & 1][0][0];
-        KvRegs t, t2;
-        load_step_shared(t, blk, lane);
-        load_step_shared(t2, blk + NB * 2 * kTile, lane);
-        if (grp + 1 < n_groups) issue_group(grp + 1);
         if (grp == 0) {
+            const bf16x8 k0 = lds_ld16(blk + lane * 8), k1 = lds_ld16(blk + 512 + lane * 8);
 #pragma unroll
-            for (int u = 0; u < Q; u++) start_reference(st[u], bq[u], t);
+            for (int u = 0; u < Q; u++) start_reference(st[u], bq[u], k0, k1);
         }
-        step_all(t);
-        step_all(t2);
+        // All four blocks are one step: one test for the rare path, and the keys' registers are free before the values are used.
+        // Three quarters of the vector-ALU slots are taken on long walks (8 x 65536 tokens, topk 8, 256 pooled blocks), so what
+        // counts is the instructions per score: without the maximum, and with one test per four blocks, 850 -> 805 us.
+        bf16x8 bp[Q][kGroup / 2];
+        float rs[Q], most = 0.f;
+        ValueRegs<kGroup> v;
+        {
+            KeyRegs<kGroup> k;
+            load_keys_shared(k, blk, lane);
+            load_values_shared(v, blk, lane);
+            if (grp + 1 < n_groups) issue_group(grp + 1);
+#pragma unroll
+            for (int u = 0; u < Q; u++) {
+                float x[kGroup][4];
+                exponents<kGroup>(x, st[u], bq[u], k);
+                rs[u] = probabilities<kGroup>(bp[u], x);
+                most = fmaxf(most, rs[u]);
+            }
+        }
+        if (__ballot(most > kMaxSum) != 0) {                  // (reads the keys once more rather than keep them for this)
+            asm volatile("" ::: "memory");
+            KeyRegs<kGroup> k;
+            load_keys_shared(k, blk, lane);
+#pragma unroll
+            for (int u = 0; u < Q; u++) {
+                float x[kGroup][4];
+                exponents<kGroup>(x, st[u], bq[u], k);
+                rs[u] = move_reference<kGroup>(st[u], bp[u], x);
+            }
+        }
+#pragma unroll
+        for (int u = 0; u < Q; u++) accumulate<kGroup>(st[u], rs[u], bp[u], v);
     }
 #pragma unroll
     for (int u = 0; u < Q; u++) rescale(st[u], w_prev);       // fine tokens weigh 1
@@ -269,7 +309,7 @@ __global__ __launch_bounds__(256, Q == 1 ? 4 : 3) void attn_fwd_kernel(llsa_attn
     bf16* const slots = sh0 + wave * (4 * kTile);             // two slots of the V tiles of two blocks
     auto fine = [&]() __attribute__((always_inline)) {
         const int n_steps = (ml.n + 1) / 2;
-        auto fetch = [&](int s, KvRegs& dst) __attribute__((always_inline)) {
+        auto fetch = [&](int s, KeyRegs<2>& dst) __attribute__((always_inline)) {
             bf16* slot = slots + (s & 1) * (2 * kTile);
 #pragma unroll
             for (int j = 0; j < 2; j++) {
@@ -280,22 +320,23 @@ __global__ __launch_bounds__(256, Q == 1 ? 4 : 3) void attn_fwd_kernel(llsa_attn
                 copy16_global_to_lds(vr + at + 512, slot + j * kTile + 512);
             }
         };
-        auto work = [&](int s, KvRegs& cur, KvRegs& nxt) __attribute__((always_inline)) {
+        auto work = [&](int s, KeyRegs<2>& cur, KeyRegs<2>& nxt) __attribute__((always_inline)) {
             const unsigned m0 = ml.rows(2 * s), m1 = 2 * s + 1 < ml.n ? ml.rows(2 * s + 1) : 0u;
             wait_vm0();
-            load_v_fine(cur, slots + (s & 1) * (2 * kTile), lane);
+            ValueRegs<2> v;
+            load_values_fine(v, slots + (s & 1) * (2 * kTile), lane);
             if (s + 1 < n_steps) fetch(s + 1, nxt);
             if ((m0 & m1) == (1u << Q) - 1u) {
-                step_all(cur);
+                compute_step<Q>(st, bq, cur, v);
             } else {
 #pragma unroll
                 for (int u = 0; u < Q; u++) {
                     const bool in0 = (m0 >> u) & 1u, in1 = (m1 >> u) & 1u;
-                    if (in0 || in1) compute_step(st[u], bq[u], cur, in0, in1);
+                    if (in0 || in1) compute_step(st[u], bq[u], cur, v, in0, in1);
                 }
             }
         };
-        KvRegs ra, rb;
+        KeyRegs<2> ra, rb;
         fetch(0, ra);
         for (int s = 0; s < n_steps; s += 2) {
             work(s, ra, rb);
