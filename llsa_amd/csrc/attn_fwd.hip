@@ -73,8 +73,8 @@ __device__ __forceinline__ void exponents(float x[NB][4], const SoftmaxState& st
         for (int e = 0; e < 4; e++) x[j][e] = fmaf(s[e], kScaleLog2e, -st.m2);
     }
 }
-// p of one step as the B operands of the second product; returns the lane's sum of them.  (The empty asm keeps the compiler from
-// moving the conversion behind the branch that follows, where the fp32 values would occupy twice the registers.)
+// p of one step as the B operands of the second product; returns the lane's sum of them.  (pin_in_registers keeps the compiler
+// from moving the conversion behind the branch that follows, where the fp32 values would occupy twice the registers.)
 template <int NB>
 __device__ __forceinline__ float probabilities(bf16x8 bp[NB / 2], const float x[NB][4]) {
     float rs[2];
@@ -88,7 +88,7 @@ __device__ __forceinline__ float probabilities(bf16x8 bp[NB / 2], const float x[
             bp[j >> 1][(j & 1) * 4 + e] = (bf16)p;
         }
 #pragma unroll
-    for (int c = 0; c < NB / 2; c++) asm volatile("" : "+v"(bp[c]));
+    for (int c = 0; c < NB / 2; c++) pin_in_registers(bp[c]);
     return rs[0] + rs[1];
 }
 // in0, in1 (wave-uniform): whether the query block reads the step's first / second block

@@ -61,6 +61,14 @@ __device__ __forceinline__ bf16x4 cvt4(f32x4 v) {
     return r;
 }
 
+// The value has to exist in vector registers here: what computes it cannot be moved to its use.  (The register class is the
+// GPU's; the CPU build of these sources has no such constraint and nothing to hold back.)
+__device__ __forceinline__ void pin_in_registers(bf16x8& v) {
+#ifndef LLSA_CPU_EMU_BUILD
+    asm volatile("" : "+v"(v));
+#endif
+}
+
 // round-to-nearest-even through bf16, value kept in fp32
 __device__ __forceinline__ float rn_bf16(float x) { return (float)(bf16)x; }
 
