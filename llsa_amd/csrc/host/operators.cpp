@@ -154,6 +154,19 @@ Tensor as_rows(const Tensor& t) { return rows_ok(t) ? t : t.contiguous(); }
 
 int64_t align_up(int64_t n, int64_t a) { return (n + a - 1) / a * a; }
 
+// What torch.autograd.Function refuses for the operators written in Python, an operator whose node is native has to refuse itself:
+// inputs that carry a tangent (the kernels have no forward-mode rule; without this the result would carry none, which reads
+// as a derivative of zero) and torch.func's transforms, whose tensors have no data.
+void refuse_transforms(std::initializer_list<const Tensor*> inputs) {
+    const c10::DispatchKeySet active = c10::impl::tls_local_dispatch_key_set().included_;
+    if (active.has(c10::DispatchKey::FuncTorchDynamicLayerFrontMode) || active.has(c10::DispatchKey::FuncTorchDynamicLayerBackMode))
+        fail(Failure::kRuntime, "llsa_amd operators do not work under functorch transforms (vmap, grad, jvp, jacrev, ...)");
+    for (const Tensor* t : inputs)
+        if (t != nullptr && t->_fw_grad(/*level=*/0).defined())
+            fail(Failure::kNotImplemented, "llsa_amd operators have no jvp function: forward mode AD is not supported");
+}
+const Tensor* address(const std::optional<Tensor>& t) { return t.has_value() ? &*t : nullptr; }
+
 // ---------------------------------------------------------------------------------------
 // The second stream of a device, and the two events that tie it to the caller's.  The events are a thread's own: a wait
 // refers to the last record before it in issue order, so a thread may record them again in its next call.
@@ -355,6 +368,7 @@ bool wants_grad(const std::optional<Tensor>& t) { return t.has_value() && t->req
 Tensor attend(const std::shared_ptr<Library>& lib, const Tensor& q_in, const Tensor& k_in, const Tensor& v_in, std::vector<int64_t> topks,
               int64_t block_size, const std::optional<Tensor>& freq_in, const std::optional<Tensor>& gq_in, const std::optional<Tensor>& gk_in,
               double eps) {
+    refuse_transforms({&q_in, &k_in, &v_in, address(freq_in), address(gq_in), address(gk_in)});
     if (block_size != 16) fail(Failure::kNotImplemented, "block_size must be 16");
     for (const Tensor* t : {&q_in, &k_in, &v_in}) {
         lib->on_device(*t);
@@ -596,6 +610,7 @@ struct PermuteBackward : public Node {
 };
 
 Tensor permute(const std::shared_ptr<Library>& lib, const Tensor& x, const Tensor& perm, const Tensor& inv) {
+    refuse_transforms({&x});
     Tensor y = gather(*lib, x, perm);
     if (at::GradMode::is_enabled() && x.requires_grad()) {
         auto node = std::shared_ptr<PermuteBackward>(new PermuteBackward, torch::autograd::deleteNode);
