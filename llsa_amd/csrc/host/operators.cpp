@@ -151,6 +151,11 @@ bool rows_ok(const Tensor& t) {
     return t.stride(-1) == 1 && reinterpret_cast<uintptr_t>(t.data_ptr()) % 16 == 0 && strides_multiple(t.strides(), 8);
 }
 Tensor as_rows(const Tensor& t) { return rows_ok(t) ? t : t.contiguous(); }
+// a saved tensor as the kernels need it, wherever and with whatever strides a saved-tensor hook has put it
+Tensor restored(const Tensor& t, bool contiguous = false) {
+    const bool usable = !t.defined() || (rows_ok(t) && (!contiguous || t.is_contiguous()));
+    return usable ? t : t.clone(at::MemoryFormat::Contiguous);
+}
 
 int64_t align_up(int64_t n, int64_t a) { return (n + a - 1) / a * a; }
 
@@ -271,28 +276,35 @@ struct LlsaBackward : public Node {
     double eps;
     bool has_gq = false, has_gk = false;
     at::ScalarType type_gq = at::kFloat, type_gk = at::kFloat;
-    Tensor arena;                                            // nobody else sees it
-    SavedVariable o, freq, gq, gk, q, k;
+    // (everything kept is a SavedVariable: saved-tensor hooks -- offloading, the non-reentrant checkpoint -- see all of it)
+    SavedVariable arena, o, freq, gq, gk, q, k;
     bool released = false;
 
     std::string name() const override { return "LlsaBackward"; }
     void release_variables() override {
         std::lock_guard<std::mutex> lock(mutex_);
         released = true;
-        arena.reset();
-        for (SavedVariable* s : {&o, &freq, &gq, &gk, &q, &k}) s->reset_data();
+        for (SavedVariable* s : {&arena, &o, &freq, &gq, &gk, &q, &k}) s->reset_data();
     }
     variable_list apply(variable_list&& grads) override {
         std::lock_guard<std::mutex> lock(mutex_);
         return in_engine([&] { return run(grads[0]); });
     }
+    Tensor unpack_arena() const {
+        const Tensor t = restored(arena.unpack(), true);
+        if (t.scalar_type() != at::kByte || t.numel() != lay->bytes)
+            fail(Failure::kRuntime, "llsa_amd: a saved-tensor hook returned another tensor than it was given");
+        return t;
+    }
     variable_list run(const Tensor& grad_out) {
         if (released) fail(Failure::kRuntime, torch::autograd::ERR_BACKWARD_TWICE);
+        // (before the autograd keys are left out: a hook may run the forward again)
+        const Tensor saved = unpack_arena(), out = restored(o.unpack(shared_from_this()));
+        const Tensor fr = restored(freq.unpack(), true), wq = gq.unpack(), wk = gk.unpack();
+        const Tensor qs = restored(q.unpack()), ks = restored(k.unpack());
         at::AutoDispatchBelowADInplaceOrView below;
-        const Tensor out = o.unpack(shared_from_this());
         c10::OptionalDeviceGuard guard(lib->device ? std::optional<at::Device>(out.device()) : std::nullopt);
         const Tensor d = as_rows(grad_out.defined() ? grad_out : at::zeros_like(out));
-        const Tensor fr = freq.unpack(), wq = gq.unpack(), wk = gk.unpack();
         const auto opts = out.options();
         const std::array<int64_t, 4> shape{B, H, N, 64};
         auto like = [&](const std::array<int64_t, 4>& st) {  // gradients have the layout of their primals when the 8-byte stores allow it
@@ -300,7 +312,7 @@ struct LlsaBackward : public Node {
         };
         Tensor dq = like(sq), dk = like(sk), dv = like(sv);
         const Tensor W = at::empty({lay->bwd_bytes}, opts.dtype(at::kByte));
-        char* const a0 = static_cast<char*>(arena.data_ptr());
+        char* const a0 = static_cast<char*>(saved.data_ptr());
         char* const w0 = static_cast<char*>(W.data_ptr());
         const Layout& y = *lay;
         llsa_attn_bwd_args a{};
@@ -344,8 +356,8 @@ struct LlsaBackward : public Node {
                 nb.eps = static_cast<float>(eps);
                 return dg;
             };
-            if (wq.defined()) dgq = norm(a.norm_q, wq, q.unpack(), 0);
-            if (wk.defined()) dgk = norm(a.norm_k, wk, k.unpack(), rows * 64);
+            if (wq.defined()) dgq = norm(a.norm_q, wq, qs, 0);
+            if (wk.defined()) dgk = norm(a.norm_k, wk, ks, rows * 64);
         }
         lib->check(lib->attn_bwd(&a, lib->stream(out)), "attn_bwd");
         if (dgq.defined()) dgq = dgq.to(type_gq);
@@ -388,25 +400,26 @@ Tensor attend(const std::shared_ptr<Library>& lib, const Tensor& q_in, const Ten
     for (int l = 0; l < L; l++, per *= 16) topks[l] = std::min(topks[l], N / per);
 
     const bool grad = at::GradMode::is_enabled() && (q_in.requires_grad() || k_in.requires_grad() || v_in.requires_grad() || wants_grad(gq_in) || wants_grad(gk_in));
-    Tensor o;
+    Tensor o, arena, freq, q, k, gq, gk;
     std::shared_ptr<LlsaBackward> node;
     {
         at::AutoDispatchBelowADInplaceOrView below;
         c10::OptionalDeviceGuard guard(lib->device ? std::optional<at::Device>(q_in.device()) : std::nullopt);
-        Tensor freq, gq, gk;
         if (freq_in.has_value()) {
             if (freq_in->scalar_type() != at::kBFloat16 || freq_in->dim() != 2 || freq_in->size(0) != N || freq_in->size(1) != 64)
                 fail(Failure::kValue, "rope table must be bf16 (N, 64)");
             freq = freq_in->contiguous();
         }
-        const Tensor q = as_rows(q_in), k = as_rows(k_in), v = as_rows(v_in);
+        const Tensor v = as_rows(v_in);
+        q = as_rows(q_in);
+        k = as_rows(k_in);
         if (gq_in.has_value()) gq = gq_in->to(q.device(), at::kFloat).contiguous();
         if (gk_in.has_value()) gk = gk_in->to(q.device(), at::kFloat).contiguous();
         for (const Tensor* g : {&gq, &gk})
             if (g->defined() && g->numel() != 64) fail(Failure::kValue, "qk-norm weights must have 64 entries");
         const Layout y(*lib, B, H, N, topks, grad);
         const int64_t* n = y.n;
-        const Tensor arena = at::empty({y.bytes}, q.options().dtype(at::kByte));
+        arena = at::empty({y.bytes}, q.options().dtype(at::kByte));
         o = strides_multiple(q.strides(), 4) ? at::empty_like(q) : at::empty(q.sizes(), q.options());
         char* const a0 = static_cast<char*>(arena.data_ptr());
         auto pa = [&](int64_t at) -> void* { return at < 0 ? nullptr : a0 + at; };
@@ -525,19 +538,13 @@ Tensor attend(const std::shared_ptr<Library>& lib, const Tensor& q_in, const Ten
                 node->sv[i] = v.stride(i);
             }
             node->eps = eps;
-            node->arena = arena;
-            node->freq = SavedVariable(freq, false);
-            if (gq.defined()) {                              // (q and k themselves are needed again only by the backward of the qk-norm)
+            if (gq.defined()) {
                 node->has_gq = true;
                 node->type_gq = gq_in->scalar_type();
-                node->gq = SavedVariable(gq.is_same(*gq_in) ? *gq_in : gq, false);
-                node->q = SavedVariable(q.is_same(q_in) ? q_in : q, false);
             }
             if (gk.defined()) {
                 node->has_gk = true;
                 node->type_gk = gk_in->scalar_type();
-                node->gk = SavedVariable(gk.is_same(*gk_in) ? *gk_in : gk, false);
-                node->k = SavedVariable(k.is_same(k_in) ? k_in : k, false);
             }
         }
     }
@@ -547,7 +554,18 @@ Tensor attend(const std::shared_ptr<Library>& lib, const Tensor& q_in, const Ten
         if (node->has_gk) inputs.push_back(*gk_in);
         node->set_next_edges(torch::autograd::collect_next_edges(inputs));
         torch::autograd::set_history(o, node);
+        // (in the state the caller is in: a hook that packs a tensor may compute with it)
+        node->arena = SavedVariable(arena, false);
         node->o = SavedVariable(o, true);
+        if (freq.defined()) node->freq = SavedVariable(freq, false);
+        if (gq.defined()) {                                  // (q and k themselves are needed again only by the backward of the qk-norm)
+            node->gq = SavedVariable(gq.is_same(*gq_in) ? *gq_in : gq, false);
+            node->q = SavedVariable(q.is_same(q_in) ? q_in : q, false);
+        }
+        if (gk.defined()) {
+            node->gk = SavedVariable(gk.is_same(*gk_in) ? *gk_in : gk, false);
+            node->k = SavedVariable(k.is_same(k_in) ? k_in : k, false);
+        }
     }
     return o;
 }
@@ -558,10 +576,11 @@ std::vector<Tensor> selection(const Tensor& out) {
     if (node == nullptr) fail(Failure::kValue, "not an output of a fused operator that records its backward");
     if (node->released) fail(Failure::kRuntime, torch::autograd::ERR_BACKWARD_TWICE);
     const Layout& y = *node->lay;
+    const Tensor arena = node->unpack_arena();
     std::vector<Tensor> r;
     for (int l = 0; l < y.L; l++) {
         const int64_t count = node->B * node->H * y.n[l + 1] * y.topk[l];
-        r.push_back(node->arena.narrow(0, y.sel[l], 4 * count).view(at::kInt).view({node->B, node->H, y.n[l + 1], y.topk[l]}));
+        r.push_back(arena.narrow(0, y.sel[l], 4 * count).view(at::kInt).view({node->B, node->H, y.n[l + 1], y.topk[l]}));
     }
     return r;
 }
