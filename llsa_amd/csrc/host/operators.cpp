@@ -18,6 +18,7 @@
 #include <torch/csrc/autograd/functions/utils.h>
 #include <torch/csrc/autograd/saved_variable.h>
 #include <torch/csrc/autograd/variable.h>
+#include <torch/csrc/jit/frontend/tracer.h>
 #include <torch/csrc/utils/pybind.h>
 #include <torch/extension.h>
 #include <c10/hip/HIPStream.h>
@@ -380,6 +381,8 @@ bool wants_grad(const std::optional<Tensor>& t) { return t.has_value() && t->req
 Tensor attend(const std::shared_ptr<Library>& lib, const Tensor& q_in, const Tensor& k_in, const Tensor& v_in, std::vector<int64_t> topks,
               int64_t block_size, const std::optional<Tensor>& freq_in, const std::optional<Tensor>& gq_in, const std::optional<Tensor>& gk_in,
               double eps) {
+    // (a recorded graph would hold the allocations and none of the launches)
+    if (torch::jit::tracer::isTracing()) fail(Failure::kRuntime, "llsa_amd attention operators cannot be recorded by torch.jit.trace");
     refuse_transforms({&q_in, &k_in, &v_in, address(freq_in), address(gq_in), address(gk_in)});
     if (block_size != 16) fail(Failure::kNotImplemented, "block_size must be 16");
     for (const Tensor* t : {&q_in, &k_in, &v_in}) {

@@ -15,7 +15,24 @@ def gather_tokens(x: torch.Tensor, index: torch.Tensor) -> torch.Tensor:
     return lib.host.gather(lib.host_library, x, index)
 
 
+class _TracedPermutation(torch.autograd.Function):
+    """permute_tokens while torch.jit.trace records: it keeps a Python function's call as one node of the graph, of a native
+    call nothing but the output's allocation."""
+
+    @staticmethod
+    def forward(ctx, x, perm, inv):
+        ctx.save_for_backward(inv)
+        return gather_tokens(x, perm)
+
+    @staticmethod
+    def backward(ctx, dy):
+        inv, = ctx.saved_tensors
+        return gather_tokens(dy, inv), None, None
+
+
 def permute_tokens(x: torch.Tensor, perm: torch.Tensor, inv: torch.Tensor) -> torch.Tensor:
     """x[:, perm, :] for a permutation `perm` whose inverse is `inv`: the gradient is dy[:, inv, :]."""
+    if torch._C._get_tracing_state() is not None:
+        return _TracedPermutation.apply(x, perm, inv)
     lib = current_lib()
     return lib.host.permute(lib.host_library, x, perm, inv)

@@ -164,3 +164,19 @@ def test_a_hook_that_returns_another_tensor_is_an_error(dev):
         o = llsa_amd.llsa_l1(*leaves[:3], 8, 16)
     with pytest.raises(RuntimeError, match="another tensor"):
         o.backward(torch.ones_like(o))
+
+
+@pytest.mark.parametrize("grad", [False, True])
+def test_trace(dev, grad):
+    """A traced permutation computes, on other inputs too; the attention operators refuse to be traced."""
+    x, y = (torch.randn(2, 64, 8, generator=torch.Generator().manual_seed(s)).to(dev).requires_grad_(grad) for s in (1, 2))
+    perm, inv = _permutation(dev)
+    traced = torch.jit.trace(lambda a: llsa_amd.permute_tokens(a * 2, perm, inv), (x,), check_trace=False)
+    got, ref = traced(y), 2 * y.detach()[:, perm.long(), :]
+    assert torch.equal(got, ref)
+    if grad:
+        got.backward(ref)
+        assert torch.equal(y.grad, 4 * y.detach())
+    q, k, v = _inputs(dev)
+    with pytest.raises(RuntimeError, match="torch.jit.trace"):
+        torch.jit.trace(lambda a: llsa_amd.llsa_l1(a, k, v, 8, 16), (q,), check_trace=False)
