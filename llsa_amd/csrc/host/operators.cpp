@@ -13,6 +13,8 @@
 //
 // The library's entry points are called through the table of addresses its ctypes binding (llsa_amd/_lib.py) passes in, so
 // that this file works on whatever build of the library the binding has loaded.
+#include <torch/csrc/Dtype.h>
+#include <torch/csrc/DynamicTypes.h>
 #include <torch/csrc/Exceptions.h>
 #include <torch/csrc/autograd/function.h>
 #include <torch/csrc/autograd/functions/utils.h>
@@ -372,24 +374,21 @@ struct LlsaBackward : public Node {
 
 bool wants_grad(const std::optional<Tensor>& t) { return t.has_value() && t->requires_grad(); }
 
-// forward(q, k, v, topks, block_size, freq, gamma_q, gamma_k, eps) -> o
+// forward(q, k, v, topks, freq, gamma_q, gamma_k, eps) -> o
 //
 // topks: one entry per pooled level, (topk1, topk2, ...): the fine blocks a query block keeps, then the blocks of
 // pooled level 1, 2, ... its ancestor groups keep; one entry is llsa_l1, two are llsa_l2.
 // gamma_q / gamma_k ((64,) or none): RMS-normalise q / k over the head dimension first (the qk-norm of the reference's
 // attention processor), inside the pooling pass; they receive gradients.
 Tensor attend(const std::shared_ptr<Library>& lib, const Tensor& q_in, const Tensor& k_in, const Tensor& v_in, std::vector<int64_t> topks,
-              int64_t block_size, const std::optional<Tensor>& freq_in, const std::optional<Tensor>& gq_in, const std::optional<Tensor>& gk_in,
-              double eps) {
+              const std::optional<Tensor>& freq_in, const std::optional<Tensor>& gq_in, const std::optional<Tensor>& gk_in, double eps) {
     // (a recorded graph would hold the allocations and none of the launches)
     if (torch::jit::tracer::isTracing()) fail(Failure::kRuntime, "llsa_amd attention operators cannot be recorded by torch.jit.trace");
     refuse_transforms({&q_in, &k_in, &v_in, address(freq_in), address(gq_in), address(gk_in)});
-    if (block_size != 16) fail(Failure::kNotImplemented, "block_size must be 16");
     for (const Tensor* t : {&q_in, &k_in, &v_in}) {
         lib->on_device(*t);
         if (t->scalar_type() != at::kBFloat16)
-            fail(Failure::kNotImplemented, "llsa_amd attention kernels are bf16 only (got torch." + std::string(
-                     t->scalar_type() == at::kFloat ? "float32" : t->scalar_type() == at::kHalf ? "float16" : c10::toString(t->scalar_type())) + ")");
+            fail(Failure::kNotImplemented, "llsa_amd attention kernels are bf16 only (got torch." + std::string(torch::getTHPDtype(t->scalar_type())->name) + ")");
     }
     if (q_in.dim() != 4 || q_in.size(3) != 64) fail(Failure::kNotImplemented, "llsa_amd attention kernels need (B,H,N,64) tensors (got " + text_of(q_in.sizes()) + ")");
     if (k_in.sizes() != q_in.sizes() || v_in.sizes() != q_in.sizes()) fail(Failure::kValue, "self-attention only: q, k, v must have the same shape");
@@ -626,18 +625,20 @@ struct PermuteBackward : public Node {
         return in_engine([&]() -> variable_list {
             if (released) fail(Failure::kRuntime, torch::autograd::ERR_BACKWARD_TWICE);
             if (!grads[0].defined()) return {Tensor()};
-            return {gather(*lib, grads[0], inv.unpack())};
+            const Tensor index = inv.unpack();
+            if (!index.defined()) fail(Failure::kValue, "permute_tokens: the gradient needs the inverse permutation");
+            return {gather(*lib, grads[0], index)};
         });
     }
 };
 
-Tensor permute(const std::shared_ptr<Library>& lib, const Tensor& x, const Tensor& perm, const Tensor& inv) {
+Tensor permute(const std::shared_ptr<Library>& lib, const Tensor& x, const Tensor& perm, const std::optional<Tensor>& inv) {
     refuse_transforms({&x});
     Tensor y = gather(*lib, x, perm);
     if (at::GradMode::is_enabled() && x.requires_grad()) {
         auto node = std::shared_ptr<PermuteBackward>(new PermuteBackward, torch::autograd::deleteNode);
         node->lib = lib;
-        node->inv = SavedVariable(inv, false);
+        if (inv.has_value()) node->inv = SavedVariable(*inv, false);
         node->set_next_edges(torch::autograd::collect_next_edges(x));
         torch::autograd::set_history(y, node);
     }
@@ -652,15 +653,15 @@ PYBIND11_MODULE(_llsa_host, m) {
     m.def("set_library_error", [](py::object type) { g_library_error = type.release().ptr(); });
     m.attr("abi_version") = LLSA_ABI_VERSION;
     m.def("attend", torch::wrap_pybind_function([](const std::shared_ptr<Library>& lib, const Tensor& q, const Tensor& k, const Tensor& v,
-                                                   const std::vector<int64_t>& topks, int64_t block_size, const std::optional<Tensor>& freq,
+                                                   const std::vector<int64_t>& topks, const std::optional<Tensor>& freq,
                                                    const std::optional<Tensor>& gq, const std::optional<Tensor>& gk, double eps) {
-        return without_interpreter([&] { return attend(lib, q, k, v, topks, block_size, freq, gq, gk, eps); });
+        return without_interpreter([&] { return attend(lib, q, k, v, topks, freq, gq, gk, eps); });
     }));
     m.def("selection", torch::wrap_pybind_function([](const Tensor& out) { return without_interpreter([&] { return selection(out); }); }));
     m.def("gather", torch::wrap_pybind_function([](const std::shared_ptr<Library>& lib, const Tensor& x, const Tensor& index) {
         return without_interpreter([&] { return gather(*lib, x, index); });
     }));
-    m.def("permute", torch::wrap_pybind_function([](const std::shared_ptr<Library>& lib, const Tensor& x, const Tensor& perm, const Tensor& inv) {
+    m.def("permute", torch::wrap_pybind_function([](const std::shared_ptr<Library>& lib, const Tensor& x, const Tensor& perm, const std::optional<Tensor>& inv) {
         return without_interpreter([&] { return permute(lib, x, perm, inv); });
     }));
 }

@@ -14,9 +14,11 @@ def attend(q, k, v, topks, block_size, freq, qk_norm):
     """topks: one entry per pooled level, (topk1, topk2, ...): the fine blocks a query block keeps, then the blocks of
     pooled level 1, 2, ... its ancestor groups keep; len(topks) = 1 is llsa_l1, 2 is llsa_l2.
     freq: RoPE table or None; qk_norm: (gamma_q, gamma_k, eps) or None."""
+    if block_size != 16:
+        raise NotImplementedError("block_size must be 16")
     lib = current_lib()
     gq, gk, eps = qk_norm if qk_norm is not None else (None, None, 0.0)
-    return lib.host.attend(lib.host_library, q, k, v, topks, block_size, freq, gq, gk, eps)
+    return lib.host.attend(lib.host_library, q, k, v, topks, freq, gq, gk, eps)
 
 
 def selection(out):

@@ -180,3 +180,23 @@ def test_trace(dev, grad):
     q, k, v = _inputs(dev)
     with pytest.raises(RuntimeError, match="torch.jit.trace"):
         torch.jit.trace(lambda a: llsa_amd.llsa_l1(a, k, v, 8, 16), (q,), check_trace=False)
+
+
+def test_arguments(dev):
+    """Any block_size that equals 16 is one; errors name dtypes as torch does; a permutation that is never differentiated needs
+    no inverse."""
+    import numpy as np
+    q, k, v = _inputs(dev)
+    for size in (16.0, np.int64(16), torch.tensor(16)):
+        assert llsa_amd.llsa_l1(q, k, v, 8, size).shape == q.shape
+    for size in (8, None):
+        with pytest.raises(NotImplementedError, match="block_size must be 16"):
+            llsa_amd.llsa_l1(q, k, v, 8, size)
+    for dtype in (torch.float64, torch.float32, torch.float16, torch.int64, torch.bool, torch.float8_e4m3fn):
+        with pytest.raises(NotImplementedError, match=f"got {dtype}"):
+            llsa_amd.llsa_l1(q.to(dtype), k, v, 8, 16)
+    x, (perm, inv) = torch.randn(1, 64, 8, device=dev).requires_grad_(), _permutation(dev)
+    y = llsa_amd.permute_tokens(x, perm, None)
+    assert torch.equal(y, x[:, perm.long(), :])
+    with pytest.raises(ValueError, match="inverse"):
+        y.sum().backward()
