@@ -172,9 +172,8 @@ int llsa_topk_cascade_max_parents(void);
  * (sparse_attention_res_2.py); deeper hierarchies have no counterpart in the reference and continue
  * the scheme by induction on sparse_attention_res_2.py:94-149.  The coarsest level is walked in
  * groups of four blocks: N must be a multiple of 64 * 16^levels.  Indices outside their range are
- * clamped into it; a row of idx that names a block twice counts it twice in the forward and in dq
- * (as the reference's gather does) -- the K-side gradients need distinct entries, see
- * llsa_transpose_indices.
+ * clamped into it; a row that names a block twice counts it twice, in the forward and in all
+ * gradients (as the reference's gather does).
  * ---------------------------------------------------------------------------------------- */
 #define LLSA_MAX_LEVELS 4
 #define LLSA_POOLED_TOPK_MAX 56     /* the T of the pooled levels below the coarsest may add up to this much (forward and backward) */
@@ -211,11 +210,10 @@ int llsa_attn_fwd(const llsa_attn_fwd_args* a, void* stream);
  * Index transpose.  Replaces transpose_indices (kernel/triton/indices_transpose.py:104-109):
  * idx (B,H,Mb,T) -> offsets (B,H,Kb+1) with offsets[0] = 0 and flat (B,H,Mb*T); segment n of
  * flat lists the query blocks that selected key block n in ASCENDING order (the reference's
- * order is whatever its atomics produce).  Rows of idx must hold distinct values in [0, Kb): a
- * value named twice in a row collapses to one list entry and leaves the tail of the segment
- * undefined (nothing is read or written out of bounds).
+ * order is whatever its atomics produce).  A value outside [0, Kb) is clamped into it; a value
+ * that a row names several times is that many entries of its segment, side by side, as in the reference.
  * With `inv` (B,H,Mb,T) the inverse is written too: inv[q][t] = position in flat of the entry
- * that (query block q, slot t) became.  llsa_attn_bwd needs it for the selections of the pooled
+ * that (query block q, slot t) became (a permutation of 0 .. Mb*T - 1).  llsa_attn_bwd needs it for the selections of the pooled
  * levels (lvl[].sel): the partial sums of a key block are stored at the positions of its list.
  * ---------------------------------------------------------------------------------------- */
 int llsa_transpose_indices(const int32_t* idx, int32_t* offsets, int32_t* flat, int32_t* work /* or NULL */,

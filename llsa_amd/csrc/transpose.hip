@@ -3,7 +3,7 @@
 // histogram (LDS atomics), exclusive scan, scatter with an LDS cursor, and finally every
 // segment is put in ascending query-block order with a per-wave bitmap (set one bit per
 // entry, then read the bits back in order), which makes the result -- and therefore the
-// accumulation order of dK/dV -- independent of atomic timing.
+// accumulation order of dK/dV -- independent of atomic timing.  An entry that its row repeats counts as often as it is there.
 #include "llsa_device.h"
 #include "llsa_host.h"
 #include "../../include/llsa_hip.h"
@@ -209,10 +209,13 @@ __global__ __launch_bounds__(SPLIT ? kTrThreadsBeside : kTrThreads) void transpo
 // The transpose of all levels of one operator call in one launch, sorted as it is built.  A workgroup owns a range of key
 // blocks of one (b,h): it reads all entries, keeps one bitmap over the query blocks per key block of its range in LDS (one
 // word of padding per row keeps the rows off each other's banks), and counts the entries below its range -- which is
-// where its first segment starts, so that no word passes between workgroups.  A key block's count is the population of
-// its row, its segment is written by reading the row's bits back in order -- ascending query blocks with no scatter through
-// atomic cursors and no sorting pass afterwards; the inverse position of an entry is its segment's start plus the bits below
-// its own.  One more workgroup per (b,h) makes a histogram over all key blocks and from it offsets and work list.
+// where its first segment starts, so that no word passes between workgroups.  A key block's segment is written by reading its
+// row's bits back in order -- ascending query blocks with no scatter through atomic cursors and no sorting pass
+// afterwards; the inverse position of an entry is its segment's start plus the bits below its own.  One more workgroup per (b,h)
+// makes a histogram over all key blocks and from it offsets and work list.
+// All counts are of entries.  A query block that names a key block twice (a top-k does not, a caller's own indices may) is one
+// bit but two entries, and its segment is longer than its row has bits: such a segment is written again with as many copies of
+// every query block as it has entries (write_repeats), and so is the range's part of the inverse.
 // Reading every entry once per range is cheap (4 a lane and load, from the L2), clearing and filling the bitmaps of
 // the whole matrix in every workgroup was not (two levels of 12 x 16384 tokens 15.9 us), and a range fits LDS where the
 // matrix does not.
@@ -255,11 +258,34 @@ __device__ __forceinline__ void tr_entries(const TrJob& jb, const int* __restric
     }
 }
 
+// how often the first `slots` entries of query block q name key block n
+__device__ __forceinline__ int entries_naming(const int* __restrict__ idx, int q, int n, int T, int slots, int Kb) {
+    int c = 0;
+    for (int t = 0; t < slots; t++) c += clampi(idx[(int64_t)q * T + t], 0, Kb - 1) == n ? 1 : 0;
+    return c;
+}
+// The segment of key block n from its row of bits and idx, one wave, every query block as often as it names n.  Rare: only for a
+// segment that is longer than its row has bits, after the bits alone have been written to it.
+__device__ __forceinline__ void write_repeats(const int* __restrict__ idx, const unsigned* row, int w_hi, int n, int T, int Kb, int* segment, int lane, int w_lo = 0) {
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    for (int w = w_lo; w < w_hi; w++)
+        for (unsigned wd = (unsigned)__builtin_amdgcn_readfirstlane((int)row[w]); wd != 0u; wd &= wd - 1u) {
+            const int q = w * 32 + __ffs((int)wd) - 1;
+            for (int t0 = 0; t0 < T; t0 += kWave) {
+                const int c = __popcll(__ballot(t0 + lane < T && clampi(idx[(int64_t)q * T + min(t0 + lane, T - 1)], 0, Kb - 1) == n));
+                if (lane < c) segment[lane] = q;
+                segment += c;
+            }
+        }
+}
+
 template <int NT>
 __global__ __launch_bounds__(NT) void transpose_bitmap_kernel(TrJobs jobs) {
     constexpr int NW = NT / kWave;
     HIP_DYNAMIC_SHARED(int, smem)
     __shared__ int wave_tot[5 * NW];
+    __shared__ int range_end, repeats;                        // where the range's last segment ends; whether a row has fewer bits than entries
     const int bh = blockIdx.x / jobs.wgs;
     int part = blockIdx.x % jobs.wgs, ji = 0;
     while (ji < jobs.n_jobs - 1 && part > jobs.job[ji].parts) part -= jobs.job[ji++].parts + 1;
@@ -282,6 +308,7 @@ __global__ __launch_bounds__(NT) void transpose_bitmap_kernel(TrJobs jobs) {
     const int lo = part * jb.rows, nr = min(jb.rows, Kb - lo);       // > 0: the host leaves no range empty
     unsigned* bm = reinterpret_cast<unsigned*>(smem);         // [nr][stride]
     for (int i = tid; i < nr * stride; i += NT) bm[i] = 0u;
+    if (tid == 0) repeats = 0;
     __syncthreads();
     int below = 0;
     tr_entries<NT>(jb, idx, [&](int n, int q, int) {
@@ -310,6 +337,7 @@ __global__ __launch_bounds__(NT) void transpose_bitmap_kernel(TrJobs jobs) {
             start += w < wave ? o : 0;
         }
         if (tid < nr) bm[tid * stride + words] = (unsigned)(start + incl - c);
+        if (tid == nr - 1) range_end = start + incl;
     }
     __syncthreads();
     if (jb.inv != nullptr) {
@@ -341,15 +369,41 @@ __global__ __launch_bounds__(NT) void transpose_bitmap_kernel(TrJobs jobs) {
             const int o = __shfl_up(incl, d, 8);
             if (sub >= d) incl += o;
         }
-        if (r >= nr) continue;
-        int out = (int)row[words] + incl - mine;
-        for (int w = w_lo; w < w_hi; w++) {
-            unsigned wd = row[w];
-            while (wd) {
-                flat[out++] = w * 32 + __ffs((int)wd) - 1;
-                wd &= wd - 1u;
+        if (r < nr) {
+            int out = (int)row[words] + incl - mine;
+            for (int w = w_lo; w < w_hi; w++) {
+                unsigned wd = row[w];
+                while (wd) {
+                    flat[out++] = w * 32 + __ffs((int)wd) - 1;
+                    wd &= wd - 1u;
+                }
             }
         }
+        // the rows with fewer bits than entries: bit 8 i + 7 is the wave's i-th row
+        const int end = r + 1 < nr ? (int)row[stride + words] : range_end;
+        unsigned long long longer = __ballot(r < nr && sub == 7 && (int)row[words] + incl != end);
+        if (longer == 0) continue;                            // (uniform over the wave)
+        repeats = 1;
+        for (; longer != 0; longer &= longer - 1) {
+            const int rr = r0 + wave * 8 + (__ffsll(longer) >> 3) - 1;
+            const unsigned* rrow = bm + rr * stride;
+            write_repeats(idx, rrow, words, lo + rr, T, Kb, flat + rrow[words], lane);
+        }
+    }
+    if (jb.inv == nullptr) return;
+    __syncthreads();
+    if (repeats != 0) {                                       // (uniform) the inverse once more, by counting entries
+        int* inv = jb.inv + (int64_t)bh * E;
+        tr_entries<NT>(jb, idx, [&](int n, int q, int e) {
+            const int r = n - lo;
+            if ((unsigned)r >= (unsigned)nr) return;
+            const unsigned* row = bm + r * stride;
+            int pos = (int)row[words];
+            for (int w = 0; w <= (q >> 5); w++)
+                for (unsigned wd = w < (q >> 5) ? row[w] : row[w] & ((1u << (q & 31)) - 1u); wd != 0u; wd &= wd - 1u)
+                    pos += entries_naming(idx, w * 32 + __ffs((int)wd) - 1, n, T, T, Kb);
+            inv[e] = pos + entries_naming(idx, q, n, T, e - q * T, Kb);
+        });
     }
 }
 
@@ -398,15 +452,17 @@ __global__ __launch_bounds__(kTrThreadsBeside) void tr_scatter_kernel(const int*
 
 // Puts every segment of `flat` in ascending order: one wave per key block sets one bit per
 // entry in a private LDS bitmap over the query blocks and reads the bits back in order.  Only the
-// words between the smallest and the largest query block of the segment are cleared and read.
-__global__ __launch_bounds__(256) void sort_segments_kernel(const int* __restrict__ offsets, int* __restrict__ flat, int Mb,
-                                                            int Kb, int T) {
+// words between the smallest and the largest query block of the segment are cleared and read.  A segment with more entries than
+// bits (a query block that names the key block twice) is written again (write_repeats).
+__global__ __launch_bounds__(256) void sort_segments_kernel(const int* __restrict__ idx, const int* __restrict__ offsets,
+                                                            int* __restrict__ flat, int Mb, int Kb, int T) {
     __builtin_amdgcn_s_setprio(3);
     HIP_DYNAMIC_SHARED(unsigned, bitmaps)                     // waves x words
     const int words = (Mb + 31) / 32;
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int bh = blockIdx.y, n = blockIdx.x * (int)(blockDim.x >> 6) + wave;
     if (n >= Kb) return;                                      // no workgroup barrier below
+    idx += (int64_t)bh * Mb * T;
     flat += (int64_t)bh * Mb * T;
     const int* o = offsets + (int64_t)bh * (Kb + 1) + n;
     const int s = o[0], e = o[1];
@@ -446,11 +502,12 @@ __global__ __launch_bounds__(256) void sort_segments_kernel(const int* __restric
         }
         out += __shfl(incl2, kWave - 1);
     }
+    if (out != e) write_repeats(idx, bm, w_hi, n, T, Kb, flat + s, lane, w_lo);        // (the same in every lane)
 }
 
 // The inverse of the sorted lists: entry (query block q, slot t) of idx names key block n, and q sits somewhere in
-// n's ascending segment of flat -- one thread per entry finds where by bisection.  (A row that names a key block
-// twice owns one position only; both slots receive it.)
+// n's ascending segment of flat -- one thread per entry finds where by bisection.  (The copies of a query block that names the key
+// block several times are neighbours there and belong to its slots in order.)
 __global__ __launch_bounds__(256) void inverse_positions_kernel(const int* __restrict__ idx, const int* __restrict__ offsets,
                                                                 const int* __restrict__ flat, int* __restrict__ inv, int Mb, int Kb,
                                                                 int T) {
@@ -467,6 +524,7 @@ __global__ __launch_bounds__(256) void inverse_positions_kernel(const int* __res
         if (f[mid] < q) lo = mid + 1;
         else hi = mid;
     }
+    if (lo + 1 < o[1] && f[lo + 1] == q) lo += entries_naming(idx + (int64_t)bh * E, q, n, T, e - q * T, Kb);
     inv[(int64_t)bh * E + e] = clampi(lo, 0, E - 1);
 }
 
@@ -566,7 +624,7 @@ static int transpose_general(const int32_t* idx, int32_t* offsets, int32_t* flat
         if (e != hipSuccess) return fail(-101, "transpose_indices: cannot raise dynamic LDS to %zu bytes: %s", lds_sort, hipGetErrorString(e));
     }
     hipLaunchKernelGGL(sort_segments_kernel, dim3((Kb + sort_waves - 1) / sort_waves, B * H), dim3(64 * sort_waves), lds_sort,
-                       (hipStream_t)stream, (const int*)offsets, flat, Mb, Kb, T);
+                       (hipStream_t)stream, idx, (const int*)offsets, flat, Mb, Kb, T);
     if (inv != nullptr)
         hipLaunchKernelGGL(inverse_positions_kernel, dim3((unsigned)((E + 255) / 256), B * H), dim3(256), 0, (hipStream_t)stream, idx,
                            (const int*)offsets, (const int*)flat, inv, Mb, Kb, T);

@@ -119,8 +119,7 @@ def attn_bwd(do, q, k, v, pk, pv, o, lse, indices, token_weight, coarse_grad_wei
     else:
         off, flat, work = transpose_indices(idx, N // BLOCK, lib.fine_chunk(N))
         if levels == 2:
-            # A row that names a block twice would give both entries one inverse position and leave another slot of the
-            # segment unwritten (the kernels assume what a top-k guarantees): a caller's own p_indices are checked.
+            # (the kernels would count a block that a row names twice, but for a caller's own p_indices that is taken for a mistake)
             if T2 > 1 and bool((pidx.sort(-1).values.diff(dim=-1) == 0).any()):
                 raise ValueError("p_indices: a row names a block twice")
             poff, _, pinv = transpose_indices(pidx, N // (BLOCK * BLOCK), inverse=True)
