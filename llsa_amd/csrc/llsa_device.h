@@ -225,9 +225,11 @@ __device__ __forceinline__ SharedBlock shared_block(const SharedList& sl, const 
 // distinct blocks, each with the set of rows that name it (bit u: row u), ordered by that set.  A row that names a block twice
 // keeps all lists as they are (every entry on its own).  Entry i of the result sits in lane i % 64 of register i / 64.
 // `scratch`: 64 R ints of LDS private to the wave.
+constexpr int kSetShift = 28;     // an entry is block | set << 28: a sequence of fewer than 2^31 tokens has fewer than 2^27 blocks
 template <int Q, int R>
 struct MergedLists {
-    int packed[R];                                            // block | set << 24 (there are fewer than 2^21 blocks)
+    static_assert(Q <= 32 - kSetShift, "a set has one bit per row");
+    int packed[R];
     int n;
     __device__ __forceinline__ int at(int i) const {          // i is wave-uniform
         const int v = __builtin_amdgcn_readlane(packed[0], i & (kWave - 1));
@@ -235,8 +237,8 @@ struct MergedLists {
         const int o = __builtin_amdgcn_readlane(packed[R - 1], i & (kWave - 1));
         return i < kWave ? v : o;
     }
-    __device__ __forceinline__ int block(int i) const { return at(i) & 0xffffff; }
-    __device__ __forceinline__ unsigned rows(int i) const { return (unsigned)at(i) >> 24; }
+    __device__ __forceinline__ int block(int i) const { return at(i) & ((1 << kSetShift) - 1); }
+    __device__ __forceinline__ unsigned rows(int i) const { return (unsigned)at(i) >> kSetShift; }
 };
 template <int Q, int R>
 __device__ __forceinline__ MergedLists<Q, R> merge_lists(const int* ip, int T, int N1, int lane, int* scratch) {
@@ -253,7 +255,7 @@ __device__ __forceinline__ MergedLists<Q, R> merge_lists(const int* ip, int T, i
     }
     if constexpr (Q == 1) {
 #pragma unroll
-        for (int k = 0; k < R; k++) ml.packed[k] = v[k] | (1 << 24);
+        for (int k = 0; k < R; k++) ml.packed[k] = v[k] | (1 << kSetShift);
         ml.n = T;
         return ml;
     }
@@ -296,7 +298,7 @@ __device__ __forceinline__ MergedLists<Q, R> merge_lists(const int* ip, int T, i
 #pragma unroll
         for (int k = 0; k < R; k++) {
             const unsigned long long m = __ballot(lead[k] && set[k] == c);
-            if (lead[k] && set[k] == c) scratch[n + __popcll(m & below)] = v[k] | (c << 24);
+            if (lead[k] && set[k] == c) scratch[n + __popcll(m & below)] = v[k] | (int)((unsigned)c << kSetShift);
             n += __popcll(m);
         }
     }
