@@ -44,7 +44,7 @@ extern "C" {
 #define LLSA_DTYPE_BF16 0
 #define LLSA_DTYPE_F32 1
 
-#define LLSA_ABI_VERSION 206     /* changes with every change of a signature or argument structure below */
+#define LLSA_ABI_VERSION 207     /* changes with every change of a signature or argument structure below */
 int llsa_version(void);          /* LLSA_ABI_VERSION of the built library                                    */
 const char* llsa_last_error_string(void);
 
@@ -236,7 +236,8 @@ int llsa_transpose_one_launch(int Mb, int Kb, int T, int B, int H);
  * per chunk, so that a key block selected by very many query blocks is spread over many waves
  * (the reference walks each segment serially, sparse_attention_res_1.py:300-322).  `work` is
  * (B,H,llsa_work_list_len(Mb,Kb,T,chunk)) int32, 16-byte aligned; llsa_attn_bwd needs the
- * work list of idx with chunk = llsa_fine_chunk(N) (the pooled levels need none).  Per (b,h), in int32:
+ * work list of idx, with the chunk it was built with in llsa_attn_bwd_args.chunk (the pooled levels need none).  Per (b,h),
+ * in int32:
  *   [0] items, [1] partial-sum slots, [2] key blocks with more than one chunk,
  *   [3] items with more than chunk/2 entries
  *   [4 + 4i ..]              item i = {key block, first entry in flat, entries, partial-sum slot or -1};
@@ -245,12 +246,14 @@ int llsa_transpose_one_launch(int Mb, int Kb, int T, int B, int H);
  *   then Kb ints (rounded up to a multiple of 4) that the transpose itself uses as scratch
  * with max_items = Mb*T/chunk + Kb; every key block has at least one item. */
 int64_t llsa_work_list_len(int Mb, int Kb, int T, int chunk);
-/* Entries per work item of the fine level for a sequence of N tokens: 64 up to N = 16384, where a step is short and a long
- * item would end it alone, 256 beyond, where fewer items and fewer partial sums count for more (N = 65536: -2 %,
- * N = 262144: -3 % of the step); 16 up to N = 1024 and 32 up to 2048, where the whole pass is a few hundred waves and lasts
- * as long as its longest item (6 x 1024 tokens, topk 8: 18 -> 10 us).  Never more than LLSA_CHUNK_FINE_MAX.  No
- * counterpart in the reference, which walks a key block's whole list in one program (sparse_attention_res_1.py:300-322). */
+/* Entries per work item of the fine level.  llsa_fine_chunk: by the token count alone, 64 up to N = 16384, where a step is
+ * short and a long item would end it alone, 256 beyond, where fewer items and fewer partial sums count for more (N = 65536:
+ * -2 %, N = 262144: -3 % of the step).  llsa_fine_chunk_for: the same, but 16 or 32 for the few entries of short sequences
+ * (N <= 2048 and up to 2^14 / 2^16 entries B*H*N/16*T in all), where the pass lasts as long as its longest item (6 heads of
+ * 1024 tokens, topk 8: 25 -> 15 us with the reduction).  Both never more than LLSA_CHUNK_FINE_MAX.  No counterpart in the
+ * reference, which walks a key block's whole list in one program (sparse_attention_res_1.py:300-322). */
 int llsa_fine_chunk(int N);
+int llsa_fine_chunk_for(int B, int H, int N, int T);
 #define LLSA_CHUNK_FINE_MAX 256
 
 /* ------------------------------------------------------------------------------------------
@@ -306,7 +309,9 @@ typedef struct llsa_attn_bwd_args {
                                                     also receive the pooled gradients of their blocks, with the
                                                     same bf16 roundings (= llsa_pool_bwd_accum, level by level),
                                                     and dk is rotated back with freq_dk                */
-    int32_t reserved;
+    int32_t chunk;                               /* entries per item `work` was built with, from llsa_fine_chunk_for(B,H,N,T)
+                                                    (the least the workspace has room for) to LLSA_CHUNK_FINE_MAX;
+                                                    0: llsa_fine_chunk(N)                               */
     llsa_bwd_level lvl[LLSA_MAX_LEVELS];         /* lvl[l - 1] = pooled level l                     */
     llsa_norm_back norm_q, norm_k;               /* norm_k needs fold_pooled                        */
 } llsa_attn_bwd_args;

@@ -69,7 +69,7 @@ class AttnBwdArgs(C.Structure):
            ("dv", c_void_p), ("sdvb", c_int64), ("sdvh", c_int64), ("sdvn", c_int64)]
         + [("workspace", c_void_p), ("workspace_bytes", c_int64), ("freq_dq", c_void_p), ("freq_dk", c_void_p),
            ("B", c_int32), ("H", c_int32), ("N", c_int32), ("T", c_int32), ("levels", c_int32),
-           ("stages", c_int32), ("fold_pooled", c_int32), ("reserved", c_int32),
+           ("stages", c_int32), ("fold_pooled", c_int32), ("chunk", c_int32),
            ("lvl", BwdLevel * MAX_LEVELS), ("norm_q", NormBack), ("norm_k", NormBack)])
 
 
@@ -106,13 +106,14 @@ _SIGNATURES = {
     "llsa_transpose_one_launch": (c_int, [c_int, c_int, c_int, c_int, c_int]),
     "llsa_work_list_len": (c_int64, [c_int, c_int, c_int, c_int]),
     "llsa_fine_chunk": (c_int, [c_int]),
+    "llsa_fine_chunk_for": (c_int, [c_int, c_int, c_int, c_int]),
     "llsa_attn_bwd_workspace_bytes": (c_int64, [c_int, c_int, c_int, C.POINTER(c_int32), c_int]),
     "llsa_attn_bwd": (c_int, [C.POINTER(AttnBwdArgs), c_void_p]),
 }
 
 EXPORTS = tuple(_SIGNATURES)
 CHUNK_FINE_MAX = 256                                        # LLSA_CHUNK_FINE_MAX of include/llsa_hip.h
-ABI_VERSION = 206                                           # LLSA_ABI_VERSION
+ABI_VERSION = 207                                           # LLSA_ABI_VERSION
 STATIC_PARTIALS_MAX = 262144                                # LLSA_STATIC_PARTIALS_MAX
 
 

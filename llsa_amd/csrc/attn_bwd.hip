@@ -489,7 +489,7 @@ __device__ __forceinline__ bool kside_item(const KSideParams& p, int& bh, int& i
     return at < nl + ns;
 }
 
-// One work item of the fine pass: a key block and a piece (at most fine_chunk(N) <= LLSA_CHUNK_FINE_MAX entries) of its list.
+// One work item of the fine pass: a key block and a piece (at most LLSA_CHUNK_FINE_MAX entries) of its list.
 // One wave = one workgroup per item (items differ a lot in length; a wave that shared its workgroup
 // with a longer one would keep its registers and LDS allocated while idle).
 template <bool NORM>
@@ -1262,8 +1262,8 @@ static BwdWorkspace bwd_workspace(int B, int H, int N, const int32_t* topk, int 
     const DensePlan d = dense_plan(B, H, N, levels);
     BwdWorkspace w;
     // a key block has several chunks only if it has more than `chunk` entries, so at most
-    // E/chunk such blocks with at most E/chunk + E/chunk chunks in total
-    w.slots_fine = 2 * (N1 * topk[0] / fine_chunk(N)) + 2;
+    // E/chunk such blocks with at most E/chunk + E/chunk chunks in total (fine_chunk_for: the shortest chunk a call may use)
+    w.slots_fine = 2 * (N1 * topk[0] / fine_chunk_for(BH, N, topk[0])) + 2;
     int64_t o = 0;
     w.stats = o;        o += align256(BH * N / kBlk * kStats * 4);
     w.dor = o;          o += align256(BH * N * 64 * 2);
@@ -1329,6 +1329,9 @@ extern "C" int llsa_attn_bwd(const llsa_attn_bwd_args* a, void* stream) {
     LLSA_REQUIRE(a->workspace_bytes >= wsp.total, "attn_bwd: workspace too small (%lld < %lld)", (long long)a->workspace_bytes,
                  (long long)wsp.total);
     LLSA_REQUIRE(a->work != nullptr, "attn_bwd: work list missing");
+    const int chunk_fine = a->chunk != 0 ? a->chunk : fine_chunk(a->N), least_chunk = fine_chunk_for((int64_t)a->B * a->H, a->N, a->T);
+    LLSA_REQUIRE(chunk_fine >= least_chunk && chunk_fine <= LLSA_CHUNK_FINE_MAX, "attn_bwd: chunk=%d must be in %d..%d", chunk_fine, least_chunk,
+                 LLSA_CHUNK_FINE_MAX);
 
     hipStream_t s = (hipStream_t)stream;
     const int B = a->B, H = a->H, N = a->N, N1 = N / 16, N2 = N1 / 16, BH = B * H, L = a->levels;
@@ -1414,7 +1417,7 @@ extern "C" int llsa_attn_bwd(const llsa_attn_bwd_args* a, void* stream) {
         KSideParams p = base;
         p.kk = (const bf16*)a->kr; p.vv = (const bf16*)a->vr;
         p.off = a->off; p.flat = a->flat; p.flat_stride = (int64_t)N1 * a->T;
-        const int chunk = fine_chunk(N);
+        const int chunk = chunk_fine;
         p.work = a->work; p.work_stride = llsa_work_list_len(N1, N1, a->T, chunk);
         p.part = (f32x4*)(ws + wsp.part_fine); p.slot_stride = wsp.slots_fine;
         p.dk = (bf16*)a->dk; p.sdkb = a->sdkb; p.sdkh = a->sdkh; p.sdkn = a->sdkn;

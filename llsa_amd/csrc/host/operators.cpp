@@ -103,7 +103,7 @@ struct Library {
     decltype(&llsa_transpose_indices_multi) transpose_indices_multi;
     decltype(&llsa_transpose_one_launch) transpose_one_launch;
     decltype(&llsa_work_list_len) work_list_len;
-    decltype(&llsa_fine_chunk) fine_chunk;
+    decltype(&llsa_fine_chunk_for) fine_chunk_for;
     decltype(&llsa_attn_bwd_workspace_bytes) attn_bwd_workspace_bytes;
     decltype(&llsa_attn_bwd) attn_bwd;
     decltype(&llsa_gather_rows) gather_rows;
@@ -121,7 +121,7 @@ struct Library {
         get("llsa_transpose_indices_multi", transpose_indices_multi);
         get("llsa_transpose_one_launch", transpose_one_launch);
         get("llsa_work_list_len", work_list_len);
-        get("llsa_fine_chunk", fine_chunk);
+        get("llsa_fine_chunk_for", fine_chunk_for);
         get("llsa_attn_bwd_workspace_bytes", attn_bwd_workspace_bytes);
         get("llsa_attn_bwd", attn_bwd);
         get("llsa_gather_rows", gather_rows);
@@ -245,7 +245,7 @@ struct Layout {
         }
         for (int l = 0; l < L; l++) sel[l] = take(4 * n[l + 1] * topk[l]);
         lse = take(4 * N);
-        chunk = lib.fine_chunk(static_cast<int>(N));
+        chunk = lib.fine_chunk_for(static_cast<int>(B), static_cast<int>(H), static_cast<int>(N), topk[0]);
         if (grad) {
             for (int l = 0; l < L; l++) {
                 off[l] = take(4 * (n[l + 1] + 1));
@@ -344,7 +344,7 @@ struct LlsaBackward : public Node {
         a.workspace = w0 + y.ws; a.workspace_bytes = y.ws_bytes;
         if (fr.defined()) a.freq_dq = a.freq_dk = fr.data_ptr();
         a.B = static_cast<int32_t>(B); a.H = static_cast<int32_t>(H); a.N = static_cast<int32_t>(N); a.T = y.topk[0]; a.levels = y.L;
-        a.fold_pooled = 1;
+        a.fold_pooled = 1; a.chunk = y.chunk;
         Tensor dgq, dgk, P;
         if (wq.defined() || wk.defined()) {                  // back through the qk-norm, inside the kernels that write dq and dk
             const auto f32 = opts.dtype(at::kFloat);

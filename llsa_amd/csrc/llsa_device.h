@@ -154,7 +154,21 @@ __device__ __forceinline__ bf16x4 rope_bwd4(bf16x4 o, bf16x4 f) {
 // ints at the end of a (b,h)'s work list (see transpose.hip) that the transpose of many entries uses as
 // histogram, then as cursors
 __host__ __device__ inline int work_tail_len(int Kb) { return (Kb + 3) & ~3; }
-__host__ __device__ inline int fine_chunk(int N) { return N > 16384 ? 256 : N > 2048 ? 64 : N > 1024 ? 32 : 16; }      // llsa_fine_chunk
+__host__ __device__ inline int fine_chunk(int N) { return N > 16384 ? 256 : 64; }      // llsa_fine_chunk
+// llsa_fine_chunk_for.  Short pieces trade the length of the longest item, which is what a pass over few entries takes, for fp32
+// partial sums (8 KB a piece) and their reduction, which is what it takes over many.  So the lines are drawn on the entries of
+// all heads, up to 2048 tokens, where they were measured: K-side pass + reduction in us with pieces of 16 / 32 / 64, smooth
+// inputs, N = 1024 unless given --
+//     6 heads, topk 8    (3 Ki entries)    15 / 18 / 25          96 heads, topk 8  (48 Ki)     44 / 37 / 38
+//     24 heads, topk 8   (12 Ki)           20 / 21 / 26          24 heads, topk 32 (48 Ki)     34 / 34 / 36
+//     24 heads, topk 16  (24 Ki)           25 / 24 / 27          24 x 2048, topk 16 (48 Ki)    37 / 31 / 35
+//     6 x 2048, topk 32  (24 Ki)           25 / 25 / 31          24 heads, topk 64 (96 Ki)     43 / 42 / 39
+//     96 heads, topk 64  (384 Ki)         163 / 138 / 97         384 heads, topk 64           748 / 599 / 367
+inline int fine_chunk_for(int64_t BH, int N, int T) {
+    const int64_t entries = BH * (N / kBlk) * T;
+    if (N > 2048 || entries > (1 << 16)) return fine_chunk(N);
+    return entries > (1 << 14) ? 32 : 16;
+}
 
 constexpr int kGroup = 4;      // pooled blocks per LDS buffer in the query-side attention kernels (one per wave)
 

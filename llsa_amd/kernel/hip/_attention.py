@@ -89,13 +89,14 @@ def rows_ok8(t):
 
 def attn_bwd(do, q, k, v, pk, pv, o, lse, indices, token_weight, coarse_grad_weight, pk2=None, pv2=None,
              p_indices=None, token_weight_2=1.0, tiles=None, freq_dq: Optional[torch.Tensor] = None, stages: int = 0,
-             csr=None, fold_pooled: bool = False, freq_dk: Optional[torch.Tensor] = None):
+             csr=None, fold_pooled: bool = False, freq_dk: Optional[torch.Tensor] = None, chunk: int = 0):
     """Backward.  Returns (dq, dk, dv, dpk, dpv[, dpk2, dpv2]) with the reference's conventions:
     every gradient is `empty_like` of its primal; the pooled gradients are NOT yet folded
     into dk / dv (autograd, or pool_bwd_accum, does that) unless `fold_pooled` is set, in which case
     the fine pass adds them on its way out (same roundings) and rotates dk back with `freq_dk`.  `tiles` may carry operand tiles the
     caller already has (qr, kr, vr, pkr, pvr, pk2r, pv2r).  `stages` (a mask of
-    the LLSA_BWD_* bits of include/llsa_hip.h) launches only some of the kernels, for profiling."""
+    the LLSA_BWD_* bits of include/llsa_hip.h) launches only some of the kernels, for profiling.  `chunk`: the one the
+    work list in `csr` was built with (0: llsa_fine_chunk)."""
     levels = 1 if pk2 is None else 2
     lib = lib_for(do, q, k, v, pk, pv, pk2, pv2, o, lse)
     require_bf16(do, q, k, v, pk, pv, pk2, pv2, o)
@@ -117,7 +118,8 @@ def attn_bwd(do, q, k, v, pk, pv, o, lse, indices, token_weight, coarse_grad_wei
         if levels == 2:
             poff, _, pinv = csr[3:6]
     else:
-        off, flat, work = transpose_indices(idx, N // BLOCK, lib.fine_chunk(N))
+        chunk = lib.fine_chunk_for(B, H, N, T)
+        off, flat, work = transpose_indices(idx, N // BLOCK, chunk)
         if levels == 2:
             # (the kernels would count a block that a row names twice, but for a caller's own p_indices that is taken for a mistake)
             if T2 > 1 and bool((pidx.sort(-1).values.diff(dim=-1) == 0).any()):
@@ -163,5 +165,6 @@ def attn_bwd(do, q, k, v, pk, pv, o, lse, indices, token_weight, coarse_grad_wei
         a.freq_dk = freq_dk.data_ptr()
     a.stages = stages
     a.fold_pooled = int(bool(fold_pooled))
+    a.chunk = chunk
     lib.check(lib.attn_bwd(C.byref(a), stream_of(lib, q)), "attn_bwd")
     return tuple(outs)
