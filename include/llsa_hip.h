@@ -28,9 +28,8 @@
  *   T tile (products that contract over the block's 16 tokens: P.V, dS.K, P^T.dO, dS^T.Q)
  *        offset = (((c >> 4) * 4 + (t >> 2)) * 16 + (c & 15)) * 4 + (t & 3)
  * Tiled tensors are (B,H,n/16,1024) contiguous.  llsa_pool_pyramid_fwd writes them.  Only the
- * forward's P.V product reads T tiles from memory (of v and the pooled v); the backward
- * kernels fetch R tiles only and produce the token-major orientation on chip with the
- * transposing LDS read of gfx950.
+ * forward's product with the pooled v reads T tiles from memory; everything else fetches R
+ * tiles and makes the token-major orientation on chip with the transposing LDS read of gfx950.
  */
 #ifndef LLSA_HIP_H
 #define LLSA_HIP_H
@@ -195,7 +194,7 @@ typedef struct llsa_fwd_level {
 typedef struct llsa_attn_fwd_args {
     const void* qr;                            /* (B,H,N/16,1024)   R tiles of q                  */
     const void* kr;                            /* (B,H,N/16,1024)   R tiles of k                  */
-    const void* vt;                            /* (B,H,N/16,1024)   R tiles of v: the fine blocks' T
+    const void* vt;                            /* (B,H,N/16,1024)   R (not T) tiles of v: the T
                                                   operands are made from them on chip           */
     const int32_t* idx;                        /* (B,H,N/16,T)   selected fine blocks             */
     void* o;        int64_t sob, soh, son;     /* (B,H,N,64) out                                  */

@@ -141,9 +141,9 @@ __device__ __forceinline__ float norm_contrib_sum(const float (&contrib)[16], in
 
 // What the K-side kernels need of a query block besides its tiles, as their products take it: minus the log-sum-exp (log2
 // units) of its 16 queries, then minus their deltas, one 128-byte line per block.
-// (The products dP start from minus delta, and the exponent is one multiply-add: 16 + 8 of 136 vector-ALU slots a score pair in the
-// dense K side, 16 of 120 in the dQ kernel, which are half and two thirds busy with them: step of 6 x 262144 tokens with the
-// forward's share 4404 -> 4263 us, of 12 x 16384 337 -> 330.)
+// (The products dP start from minus delta and the exponent is one multiply-add: no subtraction per score, no product per query
+// and pass.  The vector ALU is busy 37 % of the time in the dense K side and 50 % in the dQ kernel at 6 x 262144 tokens; with
+// the forward's soft-max without a maximum that step went from 4404 to 4263 us, of 12 x 16384 337 -> 330.)
 constexpr int kStats = 2 * kBlk;
 
 // What a wave keeps per query block
@@ -1353,8 +1353,8 @@ extern "C" int llsa_attn_bwd(const llsa_attn_bwd_args* a, void* stream) {
 
     const int stages = a->stages ? a->stages : (0x7fffffff & ~LLSA_BWD_NO_REDUCE);
     if (stages & LLSA_BWD_DQ) {
-        // (two query blocks per wave win from 512 groups of eight on, see kPairMinGroups: 12 x 16384 tokens 79 against 82.6 us,
-        // 6 x 262144 1022 against 1113)
+        // (two query blocks per wave from 512 groups of eight on, see kPairMinGroups: 12 x 16384 tokens 69.4 against 72.4 us,
+        // 48 x 16384 268 against 310, 6 x 262144 963 against 1109; 24 x 4096 even, 15 x 7168 at topk 12 46.6 against 42.1)
         const bool pairs = a->T <= kPairMaxTopk && N1 % 8 == 0 && (int64_t)N1 / 8 * BH >= kPairMinGroups;
         const dim3 grid(N1 / (pairs ? 8 : 4), BH);
 #define LLSA_DQ(Q, R)                                                                                                                  \

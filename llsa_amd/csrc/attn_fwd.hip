@@ -49,8 +49,8 @@ __device__ __forceinline__ void rescale(SoftmaxState& st, float f) {
 }
 
 // The exponentials refer to st.m2, which follows the running maximum lazily: it moves only when p has become large
-// (some lane's eight p of a step add up to more than kMaxSum; smaller ones are harmless in bf16 and in the fp32 sums), so
-// that the accumulator is rescaled a few times per query block instead of at most steps; O = acc / sum and
+// (some lane's p of a step -- eight of two fine blocks, sixteen of four pooled ones -- add up to more than kMaxSum; smaller
+// ones are harmless in bf16 and in the fp32 sums), so that the accumulator is rescaled a few times per query block instead of at most steps; O = acc / sum and
 // lse = m2 + log2(sum) hold for any reference point.  The common path therefore needs no maximum, neither over the quad of
 // lanes that share a query nor over a lane's own exponents: the sum that is taken anyway tells (overflow included), and only
 // when one in the wave is too large is the reference point moved (for all four lanes of a query alike, by the quad's largest
@@ -266,8 +266,9 @@ __global__ __launch_bounds__(256, Q == 1 ? 4 : 3) void attn_fwd_kernel(llsa_attn
             for (int u = 0; u < Q; u++) start_reference(st[u], bq[u], k0, k1);
         }
         // All four blocks are one step: one test for the rare path, and the keys' registers are free before the values are used.
-        // Three quarters of the vector-ALU slots are taken on long walks (8 x 65536 tokens, topk 8, 256 pooled blocks), so what
-        // counts is the instructions per score: without the maximum, and with one test per four blocks, 850 -> 805 us.
+        // On long walks (8 x 65536 tokens, topk 8, 256 pooled blocks) the vector ALU is busy 57 % of the time and the matrix
+        // cores 37 %, and the instructions per score count: without the maximum, and with one test per four blocks, that forward
+        // call went from 850 to 805 us.
         bf16x8 bp[Q][kGroup / 2];
         float rs[Q], most = 0.f;
         ValueRegs<kGroup> v;
@@ -388,8 +389,9 @@ extern "C" int llsa_attn_fwd(const llsa_attn_fwd_args* a, void* stream) {
     const int N1 = a->N / 16, BH = a->B * a->H;
     // Two query blocks per wave halve the LDS reads of the pooled blocks and save a quarter of the fine fetches; one per wave
     // leaves more and shorter waves.  Two win where the pooled blocks are most of the walk (11 x 32768 tokens, topk 8,
-    // 128 pooled blocks: 273 against 295 us) and on large grids (48 x 16384: 263 against 280), one elsewhere (12 x 16384: 62
-    // against 68, 3 x 49152 at topk 64 144 against 155).
+    // 128 pooled blocks: 227 against 267 us) and on large grids (48 x 16384: 228 against 271, 6 x 262144: 929 against 1057), one
+    // on smaller ones (15 x 7168, topk 12: 33.5 against 37.6; 8 x 16384, topk 8: 26.6 against 28.6; 24 x 4096 and 12 x 16384 at
+    // topk 16 are even, 3 x 49152 at topk 64 161 against 156).
     int64_t shared = listed, coarsest = a->N / 256;
     for (int l = 1; l < a->levels; l++) coarsest /= 16;
     shared += coarsest;

@@ -328,7 +328,7 @@ __device__ __forceinline__ MergedLists<Q, R> merge_lists(const int* ip, int T, i
 constexpr int kPairMaxTopk = 64;
 // ... and considered from this many groups of eight query blocks on.  Below, the chip has room for all of the waves either way
 // (four workgroups of four single blocks or three of four pairs per CU), and a wave of one block has half the serial chain:
-// 6 x 1024 tokens, topk 8: forward 8.7 -> 5.9 us, dQ 14.0 -> 8.5; 6 x 8192, topk 16: step 147 -> 138 us; even at 8 x 8192.
+// 6 x 1024 tokens, topk 8: forward 10.3 -> 6.2 us, dQ 11.0 -> 7.9; 6 x 8192, topk 16: 26.2 -> 20.9 and 31.3 -> 26.8.
 constexpr int kPairMinGroups = 512;
 
 // 16- and 8-byte reads that are LDS reads by construction (ds_read_b128 / ds_read_b64)

@@ -1,9 +1,9 @@
-// Index transpose: query-major top-k lists -> key-major CSR (offsets + flat list), used by
-// the dK/dV passes.  One workgroup per (b,h) does the whole counting sort in LDS:
-// histogram (LDS atomics), exclusive scan, scatter with an LDS cursor, and finally every
-// segment is put in ascending query-block order with a per-wave bitmap (set one bit per
-// entry, then read the bits back in order), which makes the result -- and therefore the
-// accumulation order of dK/dV -- independent of atomic timing.  An entry that its row repeats counts as often as it is there.
+// Index transpose: query-major top-k lists -> key-major CSR (offsets + flat list), used by the dK/dV passes.  Up to 65536
+// entries per (b,h) one launch makes the lists of all levels from bitmaps in LDS (transpose_bitmap_kernel).  Larger lists are
+// a counting sort -- histogram, exclusive scan, scatter with a cursor -- after which every segment is put in ascending
+// query-block order with a per-wave bitmap (set one bit per entry, then read the bits back in order).  Either way the result,
+// and therefore the accumulation order of dK/dV, does not depend on the timing of atomics.  An entry that its row repeats
+// counts as often as it is there.
 #include "llsa_device.h"
 #include "llsa_host.h"
 #include "../../include/llsa_hip.h"
@@ -31,12 +31,10 @@ constexpr int kTrSplitMin = 65536;             // entries from which the split p
 // The middle step of every form of the transpose: counts per key block -> offsets, segment starts and the work list.
 // count_of(i): entries of key block i; set_start(i, start): where the caller wants the start of segment i (its cursor);
 // wave_tot: 5 * NT / 64 ints of LDS.  Called by all NT threads of the workgroup; `work` already points at the
-// (b,h)'s list (or is nullptr).  E: the sum of all counts.  write_out = false: only set_start is called, offsets and work list
-// stay untouched (a workgroup that shares the (b,h) with others and leaves these writes to one of them).
+// (b,h)'s list (or is nullptr).  E: the sum of all counts.
 template <int NT, typename CountFn, typename StartFn>
-__device__ __forceinline__ int offsets_and_work_list(CountFn count_of, StartFn set_start, int* wave_tot, int* __restrict__ offsets,
-                                                      int* __restrict__ work, int Kb, int E_items, int E_total, int chunk,
-                                                      bool write_out = true) {
+__device__ __forceinline__ void offsets_and_work_list(CountFn count_of, StartFn set_start, int* wave_tot, int* __restrict__ offsets,
+                                                       int* __restrict__ work, int Kb, int E, int chunk) {
     constexpr int NW = NT / kWave;
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     // exclusive scan over the counts: each thread owns `per` consecutive counters
@@ -88,13 +86,13 @@ __device__ __forceinline__ int offsets_and_work_list(CountFn count_of, StartFn s
         }
     }
     run_i += total_long;                                      // short items follow the long ones
-    const int max_items = E_items / chunk + Kb;
+    const int max_items = E / chunk + Kb;
     for (int i = c0; i < c1; i++) {
         const int c = count_of(i);
-        if (write_out) offsets[i] = run;
+        offsets[i] = run;
         set_start(i, run);
         run += c;
-        if (work != nullptr && write_out) {
+        if (work != nullptr) {
             const int nch = max(1, (c + chunk - 1) / chunk);
             for (int ci = 0; ci < nch; ci++) {
                 const int n_ent = min(chunk, c - ci * chunk);
@@ -114,15 +112,13 @@ __device__ __forceinline__ int offsets_and_work_list(CountFn count_of, StartFn s
             run_s += (nch > 1) ? nch : 0;
         }
     }
-    if (write_out && tid == NT - 1) offsets[Kb] = run;        // (the last thread's running sum is the total)
-    if (write_out && work != nullptr && tid == NT - 1) {
+    if (tid == NT - 1) offsets[Kb] = run;        // (the last thread's running sum is the total)
+    if (work != nullptr && tid == NT - 1) {
         work[0] = run_i;                                      // (the last thread's short items end the list)
         work[1] = run_s;
         work[2] = run_m;
         work[3] = total_long;
     }
-    (void)E_total;
-    return run;                                               // the end of this thread's key blocks: the total for the last thread
 }
 
 // Work list (optional): the K-side kernels walk each key block's segment in chunks of at most
@@ -187,7 +183,7 @@ __global__ __launch_bounds__(SPLIT ? kTrThreadsBeside : kTrThreads) void transpo
                               if (SPLIT) tail[i] = start;
                               else pos[i] = start;
                           },
-                          wave_tot, offsets, work, Kb, E, E, chunk);
+                          wave_tot, offsets, work, Kb, E, chunk);
     __syncthreads();
 
     for (int e0 = 0; e0 < (SPLIT ? 0 : E); e0 += kBatch * NT) {
@@ -300,7 +296,7 @@ __global__ __launch_bounds__(NT) void transpose_bitmap_kernel(TrJobs jobs) {
         tr_entries<NT>(jb, idx, [&](int n, int, int) { atomicAdd(&smem[n], 1); });
         __syncthreads();
         offsets_and_work_list<NT>([&](int i) { return smem[i]; }, [](int, int) {}, wave_tot, jb.offsets + (int64_t)bh * (Kb + 1),
-                              jb.work ? jb.work + (int64_t)bh * jb.work_stride : nullptr, Kb, E, E, jb.chunk);
+                              jb.work ? jb.work + (int64_t)bh * jb.work_stride : nullptr, Kb, E, jb.chunk);
         return;
     }
 

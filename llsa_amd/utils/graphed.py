@@ -1,8 +1,7 @@
 """A forward + backward step captured in one HIP graph.
 
-The operators launch ~25 small kernels per step through Python; at the sizes where those
-kernels take a few hundred microseconds in total, issuing them costs about as much host
-time as they take to run.  Replaying a captured graph issues the whole step with one call.
+A step of an operator is about ten launches; at the shortest sequences issuing them takes longer
+than they run.  Replaying a captured graph issues the whole step with one call.
 Everything the kernels of this package do is capturable: no allocation inside the library,
 no host synchronisation, no memset nodes, all work on the stream it is given (the lists for
 the backward are built on a second stream that forks from and joins the capturing one).

@@ -250,8 +250,8 @@ def check_topk_cascade(dev, B=1, H=2, N1=1024, T=8, T2=4):
 
 
 def check_transpose(dev, B=2, H=2, Mb=64, T=8, Kb=None, chunk=0):
-    """chunk > 0 also asks for the work list, which with Mb*T >= 65536 entries switches the kernel to
-    its split form (histogram and scatter over many workgroups)."""
+    """chunk > 0 also asks for the work list, with which more than 65536 entries take the split form (histogram and
+    scatter over many workgroups)."""
     from llsa_amd.kernel.hip.indices_transpose import transpose_indices
     g = torch.Generator().manual_seed(12)
     kb = Kb or Mb

@@ -66,7 +66,8 @@ def test_op_l1_qk_norm():
 def test_transpose():
     P.check_transpose(DEV, Mb=64, T=8)
     P.check_transpose(DEV, B=1, H=1, Mb=64, T=4, Kb=16)
-    P.check_transpose(DEV, B=1, H=2, Mb=4096, T=16, chunk=64)        # 65536 entries: the split form
+    P.check_transpose(DEV, B=1, H=2, Mb=4096, T=16, chunk=64)        # 65536 entries: the most the one launch takes
+    P.check_transpose(DEV, B=1, H=1, Mb=4112, T=16, chunk=64)        # more: the split form
     P.check_transpose_hot_block(DEV)
     P.check_transpose_levels(DEV, B=1, H=2, sizes=((256, 8), (16, 4)))
     P.check_transpose(DEV, B=1, H=1, Mb=40, T=4, Kb=2048, chunk=2)   # more key blocks than threads

@@ -67,7 +67,7 @@ def test_topk_dense(dev):
     P.check_topk_dense(dev, B=2, H=3, n=256, T=16, round_scores=True)
     P.check_topk_dense(dev, B=1, H=2, n=64, T=16, round_scores=False, min_safe=0.9)
     P.check_topk_dense(dev, B=1, H=2, n=1024, T=16, round_scores=False, min_safe=0.9)
-    P.check_topk_dense(dev, B=1, H=2, n=2048, T=16, round_scores=False, min_safe=0.9)     # rows longer than the radix kernel keeps: chunked arg-max
+    P.check_topk_dense(dev, B=1, H=2, n=2048, T=16, round_scores=False, min_safe=0.9)     # rows longer than the registers hold: streamed
     P.check_topk_dense(dev, B=1, H=1, n=4096, T=8, round_scores=True)
     P.check_topk_dense_ties(dev)
 
