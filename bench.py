@@ -16,7 +16,8 @@ One JSON line is printed:
                the reference's harness reports
   roofline     the slowest MFMA kernel of the step, timed with HIP events on the launch stream in a
                second pass that runs the same kernels stage by stage; `traffic` = its HBM-side bytes per
-               launch as the committed rocprofv3 summary named in `traffic_source` holds them
+               launch as the committed rocprofv3 summary named in `traffic_source` holds them, null
+               where that summary was taken with other kernels
   roofline_hbm the pooling pyramid (the q, k, v launch) against the HBM peak, on its algorithmic bytes
   cpu_baseline the CPU oracle (plain PyTorch restatement) on the host cores, same workload in fp32, and
                under `c1` benchmark configuration 1 (llsa_l1 forward, fp32, N = 1024), median of 10
@@ -48,17 +49,22 @@ PEAK_HBM_GBS = 8000.0          # MI355X HBM3E
 # HBM-side bytes per launch (L2 <-> fabric, reads + writes) come from the rocprofv3 --pmc FETCH_SIZE / WRITE_SIZE
 # summaries under profiles/ (each counter scaled by what it reads for a 256 MiB elementwise copy; the files say how):
 # the table of the workload is parsed at run time, so the figure printed is the one the committed profile holds.
-TRAFFIC_KERNELS = {"attn_fwd": "attn_fwd_pair_kernel", "bwd_dq": "attn_dq_pair_kernel", "bwd_dkv": "attn_kside_kernel",
+# A profile counts only while the kernels it was taken with are the tree's: its "kernel sources" line is compared with theirs.
+TRAFFIC_KERNELS = {"attn_fwd": "attn_fwd_kernel", "bwd_dq": "attn_dq_kernel", "bwd_dkv": "attn_kside_kernel",
                    "bwd_pooled_groups": "attn_kside_group_kernel", "bwd_dpkv_dense": "attn_kside_dense_kernel",
                    "pool_pyramid": "pool_pyramid_kernel", "topk_sparse": "topk_sparse_kernel", "topk_cascade": "topk_sparse_kernel",
-                   "topk_dense": "topk_dense_radix_kernel"}
+                   "topk_dense": "topk_dense_kernel"}
 
 
 def measured_traffic(workload):
-    """{stage: bytes per launch} and the file they were read from (None, None if the profile is missing)."""
+    """{stage: bytes per launch} and the file they were read from ({} and the reason where there is no such measurement)."""
+    from llsa_amd.build import kernel_sources_digest
     path = os.path.join(ROOT, "profiles", f"step_kernels_{workload}_hbm_traffic.txt")
     if not os.path.exists(path):
         return {}, None
+    rel = os.path.relpath(path, ROOT)
+    if f"kernel sources: {kernel_sources_digest()}\n" not in open(path).read():
+        return {}, f"none: {rel} was taken with other kernels"
     rows = {}
     for line in open(path):
         parts = line.split()
@@ -72,7 +78,7 @@ def measured_traffic(workload):
         for name, val in rows.items():
             if name.split("<")[0] == "llsa::" + kern or name.startswith("llsa::" + kern + "<"):
                 out.setdefault(stage, val)
-    return out, os.path.relpath(path, ROOT)
+    return out, rel
 
 
 WORKLOADS = {
@@ -120,6 +126,15 @@ def stage_profile(op, q, k, v, do, t1, t2, freq, iters, torch):
     from llsa_amd.kernel.hip.indices_transpose import transpose_indices_levels
     from llsa_amd.kernel.hip.mean_pool import PoolSpec, pool_pyramid
     from llsa_amd.kernel.hip.topk import compute_topk_indices_sparse, gen_sparse_indices
+    # (queued behind ten passes over half a gigabyte, so that stages of a few microseconds are timed back to back on the GPU
+    # and not at the rate Python issues them)
+    filler = torch.empty(1 << 27, device=q.device, dtype=torch.float32)
+
+    def stage_time(fn, iters, torch):
+        for _ in range(10):
+            filler.mul_(1.0)
+        return timed(fn, iters, torch)
+
     B, H, N, D = q.shape
     l2 = op == "l2"
     rope = freq is not None
@@ -128,43 +143,46 @@ def stage_profile(op, q, k, v, do, t1, t2, freq, iters, torch):
     def pyramid():
         return pool_pyramid([PoolSpec(q, y1=True, y2=l2, xr=True, rope=rope),
                              PoolSpec(k, y1=True, y2=l2, xr=True, y1r=True, rope=rope, y2r=l2),
-                             PoolSpec(v, y1=True, y2=l2, xr=True, xt=True, y1r=True, y1t=True, y2r=l2, y2t=l2)], freq)
+                             PoolSpec(v, y1=True, y2=l2, xr=True, y1r=True, y1t=True, y2r=l2, y2t=l2)], freq)
 
     oq, ok, ov = pyramid()
-    res["pool_pyramid"] = timed(pyramid, iters, torch)
+    res["pool_pyramid"] = stage_time(pyramid, iters, torch)
     pq, pk, pv = oq["y1"], ok["y1"], ov["y1"]
-    tiles = dict(qr=oq["xr"], kr=ok["xr"], vr=ov["xr"], vt=ov["xt"], pkr=ok["y1r"], pvr=ov["y1r"], pvt=ov["y1t"])
+    tiles = dict(qr=oq["xr"], kr=ok["xr"], vr=ov["xr"], pkr=ok["y1r"], pvr=ov["y1r"], pvt=ov["y1t"])
     if l2:
         pq2, pk2, pv2 = oq["y2"], ok["y2"], ov["y2"]
         tiles.update(pk2r=ok["y2r"], pv2r=ov["y2r"], pv2t=ov["y2t"])
         from llsa_amd._lib import current_lib
-        if N // 256 <= current_lib().topk_cascade_max_parents():      # what the operator launches at this size: both in one
+        n2 = N // 256
+        if n2 <= current_lib().topk_cascade_max_parents() and (n2 <= 64 or B * H * n2 < 2048):      # the operator's rule: both in one launch
             from llsa_amd.kernel.hip.topk import topk_cascade
             pidx, idx = topk_cascade(pq2, pk2, pq, pk, t1, t2)
-            res["topk_cascade"] = timed(lambda: topk_cascade(pq2, pk2, pq, pk, t1, t2), iters, torch)
+            res["topk_cascade"] = stage_time(lambda: topk_cascade(pq2, pk2, pq, pk, t1, t2), iters, torch)
         else:
             pidx = gen_sparse_indices(pq2, pk2, t2)
-            res["topk_dense"] = timed(lambda: gen_sparse_indices(pq2, pk2, t2), iters, torch)
+            res["topk_dense"] = stage_time(lambda: gen_sparse_indices(pq2, pk2, t2), iters, torch)
             idx = compute_topk_indices_sparse(pq, pk, pidx, t1, t2)
-            res["topk_sparse"] = timed(lambda: compute_topk_indices_sparse(pq, pk, pidx, t1, t2), iters, torch)
+            res["topk_sparse"] = stage_time(lambda: compute_topk_indices_sparse(pq, pk, pidx, t1, t2), iters, torch)
         kw = dict(pk2=pk2, pv2=pv2, p_indices=pidx, token_weight_2=256.0)
         cgw = 16.0
     else:
         pidx = None
         idx = gen_sparse_indices(pq, pk, t1)
-        res["topk_dense"] = timed(lambda: gen_sparse_indices(pq, pk, t1), iters, torch)
+        res["topk_dense"] = stage_time(lambda: gen_sparse_indices(pq, pk, t1), iters, torch)
         kw = {}
         cgw = 1.0
     o, lse = A.attn_fwd(q, k, v, pk, pv, idx, 16.0, tiles=tiles, **kw)
-    res["attn_fwd"] = timed(lambda: A.attn_fwd(q, k, v, pk, pv, idx, 16.0, tiles=tiles, **kw), iters, torch)
+    res["attn_fwd"] = stage_time(lambda: A.attn_fwd(q, k, v, pk, pv, idx, 16.0, tiles=tiles, **kw), iters, torch)
+
+    chunk = _cur().fine_chunk_for(B, H, N, t1)
 
     def transposes():          # all levels with one call, as the operator does it
-        r = transpose_indices_levels([idx, pidx] if l2 else [idx], _cur().fine_chunk(N))
+        r = transpose_indices_levels([idx, pidx] if l2 else [idx], chunk)
         return r[0] + r[1] if l2 else r[0]
 
     csr = transposes()
-    res["transpose_indices"] = timed(transposes, iters, torch)
-    bkw = dict(kw, tiles=tiles, csr=csr)
+    res["transpose_indices"] = stage_time(transposes, iters, torch)
+    bkw = dict(kw, tiles=tiles, csr=csr, chunk=chunk)
     # as the fused operator calls it: pooled gradients folded into dk / dv by the fine pass
     run = lambda st: A.attn_bwd(do, q, k, v, pk, pv, o, lse, idx, 16.0, cgw, stages=st, freq_dq=freq, fold_pooled=True,
                                 freq_dk=freq, **bkw)
@@ -180,9 +198,9 @@ def stage_profile(op, q, k, v, do, t1, t2, freq, iters, torch):
     for name, st in stages:
         # a stage run alone reads whatever workspace the allocator hands back (the block the complete call
         # above filled with delta and the dO tiles); only its duration is used
-        res[name] = timed(lambda: run(st), iters, torch)
+        res[name] = stage_time(lambda: run(st), iters, torch)
     # the K-side passes with the launches that add up their partial sums, in one piece (no difference of timings)
-    res["bwd_kside_all_with_reductions"] = timed(lambda: run(4 | 8 | 16), iters, torch)
+    res["bwd_kside_all_with_reductions"] = stage_time(lambda: run(4 | 8 | 16), iters, torch)
     return res
 
 
@@ -427,6 +445,7 @@ def main():
     import torch
     import llsa_amd
     from llsa_amd._lib import get_lib
+    from llsa_amd.build import kernel_sources_digest
     from llsa_amd.utils.rope_table import rope_table
     get_lib()
     assert torch.cuda.is_available(), "bench.py needs the GPU"
@@ -467,7 +486,7 @@ def main():
         torch.cuda.synchronize()
         return (time.perf_counter() - t0) * 1e3 / args.steps
 
-    # `value` is the step as a user's training loop issues it: ~25 launches from Python.
+    # `value` is the step as a user's training loop issues it: one operator call and its backward, about ten launches.
     ms = time_steps(eager_step)
 
     def step_quantiles(step, n):
@@ -507,7 +526,7 @@ def main():
                                + (" (unfused composition)" if args.unfused else ""),
                    "n_kv_per_query": nkv, "algorithmic_gflop": flops / 1e9},
         "frac_of_bf16_mfma_peak": flops / (ms * 1e-3) / 1e12 / PEAK_BF16_TFLOPS,
-        "step_event_times": quant,
+        "step_event_times": quant, "kernel_sources": kernel_sources_digest(),
     }
 
     if not args.no_extras and op != "l3":      # (the stage profile and the CPU baseline know one and two levels)

@@ -9,7 +9,9 @@ checkout that was built once can be used on a machine without recompiling.
 from __future__ import annotations
 
 import concurrent.futures as cf
+import hashlib
 import os
+import re
 import shutil
 import subprocess
 import sys
@@ -34,6 +36,16 @@ FLAGS = [
 
 def sources():
     return sorted(f for f in os.listdir(CSRC) if f.endswith(".hip"))
+
+
+def kernel_sources_digest() -> str:
+    """Names the kernels a measurement was made with: a digest of the device sources without their comments and white space."""
+    h = hashlib.sha256()
+    for f in sorted(f for f in os.listdir(CSRC) if f.endswith((".hip", ".h"))):
+        text = open(os.path.join(CSRC, f)).read()
+        text = re.sub(r"/\*.*?\*/", "", re.sub(r"//[^\n]*", "", text), flags=re.S)
+        h.update(f.encode() + b"\0" + re.sub(r"\s+", "", text).encode() + b"\0")
+    return h.hexdigest()[:16]
 
 
 def _compile(src: str) -> str:

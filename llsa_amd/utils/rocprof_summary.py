@@ -51,13 +51,13 @@ with open(f'{out}/step_kernels_{wl}_kernel_trace.txt', 'w') as f:
     for n, cnt, a, mn, mx, s in rows:
         f.write(f"{short(n):62s} {cnt:6d} {a/1e3:9.1f} {mn/1e3:9.1f} {mx/1e3:9.1f} {s/1e3/steps:9.1f} {100*s/tot:6.1f}\n")
     f.write(f"\nsum of kernel time per step: {tot/1e3/steps:.1f} us\n")
-    if wl in ('c2', 'c3'):
-        f.write("(up to N = 16384 every kernel runs on the one stream: the index transposes of all levels are one launch,\n"
-                " transpose_bitmap_kernel, behind the forward attention kernel)\n")
+    if wl in ('c2', 'c3', 'n65536'):
+        f.write("(up to 65536 entries per (b,h) every kernel runs on the one stream: the index transposes of all levels are one\n"
+                " launch, transpose_bitmap_kernel, behind the forward attention kernel)\n")
     else:
-        f.write("(the index transposes -- transpose_indices_kernel, tr_*_kernel, sort_segments_kernel, inverse_positions_kernel, and\n"
-                " transpose_bitmap_kernel for the pooled levels -- run on a second stream beside the forward attention kernel: their\n"
-                " durations overlap with it and are stretched by it, so the sum exceeds the step time)\n")
+        f.write("(the index transposes -- transpose_indices_kernel, tr_*_kernel, sort_segments_kernel, and transpose_bitmap_kernel for\n"
+                " the pooled levels -- run on a second stream beside the forward attention kernel: their durations overlap with it\n"
+                " and are stretched by it, so the sum exceeds the step time)\n")
 
 # ---- HBM traffic
 fd, fdur = counters(f'{raw}/fetch/p_results.db')
@@ -72,7 +72,8 @@ with open(f'{out}/step_kernels_{wl}_hbm_traffic.txt', 'w') as f:
     f.write(f"  rocprofv3 --pmc WRITE_SIZE --kernel-trace -d prof/write -o p -- {bench} --steps 5 --warmup 2 --calibrate\n")
     f.write("--calibrate adds a plain elementwise copy of 256 MiB (torch.mul(src, 1.0, out=dst), fp32: reads 262144 KiB, writes 262144 KiB).\n")
     f.write(f"That copy reads FETCH_SIZE={fd[copyk]['FETCH_SIZE']:.0f} KiB and WRITE_SIZE={wd[copyk]['WRITE_SIZE']:.0f} KiB per dispatch, so\n")
-    f.write(f"scale factors: fetch x{f_fac:.3f}, write x{w_fac:.3f}.  Values below are averages per dispatch over all dispatches of the kernel.\n\n")
+    f.write(f"scale factors: fetch x{f_fac:.3f}, write x{w_fac:.3f}.  Values below are averages per dispatch over all dispatches of the kernel.\n")
+    f.write(f"kernel sources: {j['kernel_sources']}\n\n")
     f.write("A kernel launched with several grids (the pooling pass of three levels, the reductions) has one row per grid (threads).\n\n")
     f.write(f"{'kernel':62s} {'grid':>9s} {'avg_us':>8s} {'FETCH_KiB':>10s} {'WRITE_KiB':>10s} {'read_MB':>9s} {'write_MB':>9s} {'GB/s':>8s}\n")
     traffic = {}
