@@ -392,6 +392,8 @@ Tensor attend(const std::shared_ptr<Library>& lib, const Tensor& q_in, const Ten
     }
     if (q_in.dim() != 4 || q_in.size(3) != 64) fail(Failure::kNotImplemented, "llsa_amd attention kernels need (B,H,N,64) tensors (got " + text_of(q_in.sizes()) + ")");
     if (k_in.sizes() != q_in.sizes() || v_in.sizes() != q_in.sizes()) fail(Failure::kValue, "self-attention only: q, k, v must have the same shape");
+    for (const Tensor* t : {&k_in, &v_in, address(freq_in)})  // (a kernel that follows a pointer into other memory faults the GPU)
+        if (t != nullptr && t->device() != q_in.device()) fail(Failure::kValue, "q, k, v and the rope table must be on one device");
     const int64_t B = q_in.size(0), H = q_in.size(1), N = q_in.size(2);
     const int L = static_cast<int>(topks.size());
     if (L < 1 || L > kL) fail(Failure::kValue, "1 to " + std::to_string(kL) + " pooled levels (got " + std::to_string(L) + ")");

@@ -195,6 +195,12 @@ def test_arguments(dev):
     for dtype in (torch.float64, torch.float32, torch.float16, torch.int64, torch.bool, torch.float8_e4m3fn):
         with pytest.raises(NotImplementedError, match=f"got {dtype}"):
             llsa_amd.llsa_l1(q.to(dtype), k, v, 8, 16)
+    for bad in ({"k": k.to("meta")}, {"v": v.to("meta")}, {"rope": torch.zeros(1024, 64, device="meta").bfloat16()}):
+        args = {"k": k, "v": v, "rope": None, **bad}
+        if dev.type == "cuda" and args["rope"] is None:
+            continue                                          # (a tensor that is on no GPU at all has an error of its own)
+        with pytest.raises(ValueError, match="one device"):
+            llsa_amd.llsa_l1(q, args["k"], args["v"], 8, 16, rope=args["rope"])
     x, (perm, inv) = torch.randn(1, 64, 8, device=dev).requires_grad_(), _permutation(dev)
     y = llsa_amd.permute_tokens(x, perm, None)
     assert torch.equal(y, x[:, perm.long(), :])
