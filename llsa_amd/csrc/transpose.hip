@@ -211,7 +211,7 @@ __global__ __launch_bounds__(SPLIT ? kTrThreadsBeside : kTrThreads) void transpo
 // makes a histogram over all key blocks and from it offsets and work list.
 // All counts are of entries.  A query block that names a key block twice (a top-k does not, a caller's own indices may) is one
 // bit but two entries, and its segment is longer than its row has bits: such a segment is written again with as many copies of
-// every query block as it has entries (write_repeats), and so is the range's part of the inverse.
+// every query block as it has entries (write_repeats), and so are those entries' places in the inverse.
 // Reading every entry once per range is cheap (4 a lane and load, from the L2), clearing and filling the bitmaps of
 // the whole matrix in every workgroup was not (two levels of 12 x 16384 tokens 15.9 us), and a range fits LDS where the
 // matrix does not.
@@ -254,24 +254,24 @@ __device__ __forceinline__ void tr_entries(const TrJob& jb, const int* __restric
     }
 }
 
-// how often the first `slots` entries of query block q name key block n
-__device__ __forceinline__ int entries_naming(const int* __restrict__ idx, int q, int n, int T, int slots, int Kb) {
-    int c = 0;
-    for (int t = 0; t < slots; t++) c += clampi(idx[(int64_t)q * T + t], 0, Kb - 1) == n ? 1 : 0;
-    return c;
-}
-// The segment of key block n from its row of bits and idx, one wave, every query block as often as it names n.  Rare: only for a
-// segment that is longer than its row has bits, after the bits alone have been written to it.
-__device__ __forceinline__ void write_repeats(const int* __restrict__ idx, const unsigned* row, int w_hi, int n, int T, int Kb, int* segment, int lane, int w_lo = 0) {
-    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-    __builtin_amdgcn_wave_barrier();
+// The segment of key block n (places `start` .. of flat) from words w_lo .. w_hi of its row of bits and from idx, one wave: every query
+// block as often as it names n, and with `inv` the places of those entries.  Rare: only for a segment that is longer than its row has
+// bits, after the bits alone have been written to it.
+__device__ __forceinline__ void write_repeats(const int* __restrict__ idx, const unsigned* row, int w_lo, int w_hi, int n, int T, int Kb,
+                                              int* flat, int* inv, int start, int lane) {
     for (int w = w_lo; w < w_hi; w++)
         for (unsigned wd = (unsigned)__builtin_amdgcn_readfirstlane((int)row[w]); wd != 0u; wd &= wd - 1u) {
             const int q = w * 32 + __ffs((int)wd) - 1;
             for (int t0 = 0; t0 < T; t0 += kWave) {
-                const int c = __popcll(__ballot(t0 + lane < T && clampi(idx[(int64_t)q * T + min(t0 + lane, T - 1)], 0, Kb - 1) == n));
-                if (lane < c) segment[lane] = q;
-                segment += c;
+                const int64_t e = (int64_t)q * T + min(t0 + lane, T - 1);
+                const bool names = t0 + lane < T && clampi(idx[e], 0, Kb - 1) == n;
+                const unsigned long long all = __ballot(names);
+                const int at = start + __popcll(all & ((1ull << lane) - 1ull));
+                if (names) {
+                    flat[at] = q;
+                    if (inv != nullptr) inv[e] = at;
+                }
+                start += __popcll(all);
             }
         }
 }
@@ -281,7 +281,7 @@ __global__ __launch_bounds__(NT) void transpose_bitmap_kernel(TrJobs jobs) {
     constexpr int NW = NT / kWave;
     HIP_DYNAMIC_SHARED(int, smem)
     __shared__ int wave_tot[5 * NW];
-    __shared__ int range_end, repeats;                        // where the range's last segment ends; whether a row has fewer bits than entries
+    __shared__ int range_end, repeats;                        // where the range's last segment ends; whether a row of it has fewer bits than entries
     const int bh = blockIdx.x / jobs.wgs;
     int part = blockIdx.x % jobs.wgs, ji = 0;
     while (ji < jobs.n_jobs - 1 && part > jobs.job[ji].parts) part -= jobs.job[ji++].parts + 1;
@@ -375,31 +375,17 @@ __global__ __launch_bounds__(NT) void transpose_bitmap_kernel(TrJobs jobs) {
                 }
             }
         }
-        // the rows with fewer bits than entries: bit 8 i + 7 is the wave's i-th row
-        const int end = r + 1 < nr ? (int)row[stride + words] : range_end;
-        unsigned long long longer = __ballot(r < nr && sub == 7 && (int)row[words] + incl != end);
-        if (longer == 0) continue;                            // (uniform over the wave)
-        repeats = 1;
-        for (; longer != 0; longer &= longer - 1) {
-            const int rr = r0 + wave * 8 + (__ffsll(longer) >> 3) - 1;
-            const unsigned* rrow = bm + rr * stride;
-            write_repeats(idx, rrow, words, lo + rr, T, Kb, flat + rrow[words], lane);
-        }
+        if (r < nr && sub == 7 && (int)row[words] + incl != (r + 1 < nr ? (int)row[stride + words] : range_end)) repeats = 1;
     }
-    if (jb.inv == nullptr) return;
     __syncthreads();
-    if (repeats != 0) {                                       // (uniform) the inverse once more, by counting entries
-        int* inv = jb.inv + (int64_t)bh * E;
-        tr_entries<NT>(jb, idx, [&](int n, int q, int e) {
-            const int r = n - lo;
-            if ((unsigned)r >= (unsigned)nr) return;
-            const unsigned* row = bm + r * stride;
-            int pos = (int)row[words];
-            for (int w = 0; w <= (q >> 5); w++)
-                for (unsigned wd = w < (q >> 5) ? row[w] : row[w] & ((1u << (q & 31)) - 1u); wd != 0u; wd &= wd - 1u)
-                    pos += entries_naming(idx, w * 32 + __ffs((int)wd) - 1, n, T, T, Kb);
-            inv[e] = pos + entries_naming(idx, q, n, T, e - q * T, Kb);
-        });
+    if (repeats == 0) return;                                 // (uniform)
+    for (int r = wave; r < nr; r += NW) {
+        const unsigned* row = bm + r * stride;
+        const int start_r = __builtin_amdgcn_readfirstlane((int)row[words]);
+        const int end = __builtin_amdgcn_readfirstlane(r + 1 < nr ? (int)row[stride + words] : range_end);
+        int bits = 0;
+        for (int w = 0; w < words; w++) bits += __popc((unsigned)__builtin_amdgcn_readfirstlane((int)row[w]));
+        if (bits != end - start_r) write_repeats(idx, row, 0, words, lo + r, T, Kb, flat, jb.inv ? jb.inv + (int64_t)bh * E : nullptr, start_r, lane);
     }
 }
 
@@ -498,7 +484,10 @@ __global__ __launch_bounds__(256) void sort_segments_kernel(const int* __restric
         }
         out += __shfl(incl2, kWave - 1);
     }
-    if (out != e) write_repeats(idx, bm, w_hi, n, T, Kb, flat + s, lane, w_lo);        // (the same in every lane)
+    if (out == e) return;                                     // (the same in every lane)
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    write_repeats(idx, bm, w_lo, w_hi, n, T, Kb, flat, nullptr, s, lane);
 }
 
 // The inverse of the sorted lists: entry (query block q, slot t) of idx names key block n, and q sits somewhere in
@@ -520,7 +509,8 @@ __global__ __launch_bounds__(256) void inverse_positions_kernel(const int* __res
         if (f[mid] < q) lo = mid + 1;
         else hi = mid;
     }
-    if (lo + 1 < o[1] && f[lo + 1] == q) lo += entries_naming(idx + (int64_t)bh * E, q, n, T, e - q * T, Kb);
+    if (lo + 1 < o[1] && f[lo + 1] == q)
+        for (int t = 0; t < e - q * T; t++) lo += clampi(idx[(int64_t)bh * E + q * T + t], 0, Kb - 1) == n ? 1 : 0;
     inv[(int64_t)bh * E + e] = clampi(lo, 0, E - 1);
 }
 

@@ -51,6 +51,15 @@ def test_lists(dev, B, H, Mb, T, Kb, chunk):
     _check(idx, Kb, res[0], res[1], res[-1])
 
 
+@pytest.mark.parametrize("Mb,T,Kb,blocks", [(4096, 16, 4096, 1), (1024, 64, 1024, 3), (4112, 16, 4112, 2)])
+def test_few_blocks_named_by_all(dev, Mb, T, Kb, blocks):
+    """Segments with tens of thousands of entries, nearly all of them repeats."""
+    from llsa_amd.kernel.hip.indices_transpose import transpose_indices
+    idx = torch.randint(7, 7 + blocks, (1, 1, Mb, T), generator=torch.Generator().manual_seed(blocks))
+    res = transpose_indices(idx.int().to(dev), Kb, 64, inverse=True)
+    _check(idx, Kb, res[0], res[1], res[-1])
+
+
 def test_lists_of_several_levels(dev):
     """A small job beside a large one: workgroups of four waves."""
     from llsa_amd.kernel.hip.indices_transpose import transpose_indices_levels
