@@ -40,16 +40,16 @@ struct PairT {
 };
 
 __device__ __forceinline__ void read_k_r(PairR& o, const bf16* k0, const bf16* k1, int lane) {
-    o.k[0][0] = lds_ld16(k0 + lane * 8);
-    o.k[0][1] = lds_ld16(k0 + 512 + lane * 8);
-    o.k[1][0] = lds_ld16(k1 + lane * 8);
-    o.k[1][1] = lds_ld16(k1 + 512 + lane * 8);
+    o.k[0][0] = lds_ld16(k0 + r_unit(lane));
+    o.k[0][1] = lds_ld16(k0 + 512 + r_unit(lane));
+    o.k[1][0] = lds_ld16(k1 + r_unit(lane));
+    o.k[1][1] = lds_ld16(k1 + 512 + r_unit(lane));
 }
 __device__ __forceinline__ void read_v_r(PairR& o, const bf16* v0, const bf16* v1, int lane) {
-    o.v[0][0] = lds_ld16(v0 + lane * 8);
-    o.v[0][1] = lds_ld16(v0 + 512 + lane * 8);
-    o.v[1][0] = lds_ld16(v1 + lane * 8);
-    o.v[1][1] = lds_ld16(v1 + 512 + lane * 8);
+    o.v[0][0] = lds_ld16(v0 + r_unit(lane));
+    o.v[0][1] = lds_ld16(v0 + 512 + r_unit(lane));
+    o.v[1][0] = lds_ld16(v1 + r_unit(lane));
+    o.v[1][1] = lds_ld16(v1 + 512 + r_unit(lane));
 }
 __device__ __forceinline__ void read_k_t(PairT& o, const bf16* k0, const bf16* k1, int lane) {
 #pragma unroll
@@ -220,7 +220,7 @@ __global__ __launch_bounds__(256, Q == 1 ? 4 : 3) void attn_dq_kernel(llsa_attn_
                                                                       bf16* __restrict__ dor) {
     __shared__ __align__(16) bf16 sh[2][kGroup][2 * kTile];   // per block: R tile of K, R tile of V
     __shared__ int order[4][R * kWave];
-    const int lane = threadIdx.x & 63;
+    const int lane = threadIdx.x & 63, unit = r_unit(lane);
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int N1 = a.N / kBlk, T = a.T;
     const int lid = xcd_logical_id();
@@ -240,10 +240,10 @@ __global__ __launch_bounds__(256, Q == 1 ? 4 : 3) void attn_dq_kernel(llsa_attn_
         const bf16* kb = (const bf16*)a.lvl[sb.level].kr + sb.tile;
         const bf16* vb = (const bf16*)a.lvl[sb.level].vr + sb.tile;
         bf16* dst = sh0 + ((grp & 1) * kGroup + wave) * (2 * kTile);
-        copy16_global_to_lds(kb + lane * 8, dst);
-        copy16_global_to_lds(kb + 512 + lane * 8, dst + 512);
-        copy16_global_to_lds(vb + lane * 8, dst + kTile);
-        copy16_global_to_lds(vb + 512 + lane * 8, dst + kTile + 512);
+        copy16_global_to_lds(kb + unit, dst);
+        copy16_global_to_lds(kb + 512 + unit, dst + 512);
+        copy16_global_to_lds(vb + unit, dst + kTile);
+        copy16_global_to_lds(vb + 512 + unit, dst + kTile + 512);
     };
     issue_group(0);
     MergedLists<Q, R> ml = merge_lists<Q, R>(ip, min(T, kWave * R / Q), N1, lane, order[wave]);
@@ -293,11 +293,11 @@ __global__ __launch_bounds__(256, Q == 1 ? 4 : 3) void attn_dq_kernel(llsa_attn_
             bf16* slot = priv + (t & 1) * (2 * kTile);
 #pragma unroll
             for (int j = 0; j < 2; j++) {
-                const int64_t at = (int64_t)ml.block(min(2 * t + j, ml.n - 1)) * kTile + lane * 8;
-                copy16_global_to_lds(kr + at, slot + j * kTile);
-                copy16_global_to_lds(kr + at + 512, slot + j * kTile + 512);
-                dst.v[j][0] = ld16(vr + at);
-                dst.v[j][1] = ld16(vr + at + 512);
+                const int64_t at = (int64_t)ml.block(min(2 * t + j, ml.n - 1)) * kTile;
+                copy16_global_to_lds(kr + at + unit, slot + j * kTile);
+                copy16_global_to_lds(kr + at + unit + 512, slot + j * kTile + 512);
+                dst.v[j][0] = ld16(vr + at + lane * 8);
+                dst.v[j][1] = ld16(vr + at + lane * 8 + 512);
             }
         };
         auto work = [&](int t, PairR& cur, PairR& nxt) __attribute__((always_inline)) {
@@ -427,10 +427,10 @@ __device__ __forceinline__ void kside_read(KsideOperands& o, const bf16* stage, 
     for (int u = 0; u < 2; u++) {
         const bf16* q = stage + (2 * u) * kTile;
         const bf16* g = stage + (2 * u + 1) * kTile;
-        o.aq[u][0] = lds_ld16(q + lane * 8);
-        o.aq[u][1] = lds_ld16(q + 512 + lane * 8);
-        o.ag[u][0] = lds_ld16(g + lane * 8);
-        o.ag[u][1] = lds_ld16(g + 512 + lane * 8);
+        o.aq[u][0] = lds_ld16(q + r_unit(lane));
+        o.aq[u][1] = lds_ld16(q + 512 + r_unit(lane));
+        o.ag[u][0] = lds_ld16(g + r_unit(lane));
+        o.ag[u][1] = lds_ld16(g + 512 + r_unit(lane));
 #pragma unroll
         for (int dt = 0; dt < 4; dt++) {
             o.tq[u][dt] = lds_t_operand(q, dt, lane);
@@ -577,10 +577,10 @@ __global__ __launch_bounds__(64) void attn_kside_kernel(KSideParams p) {
         auto fetch = [&](int i) __attribute__((always_inline)) {
             const int g0 = entry(i);
             const int g1 = (i + 1 < cnt) ? entry(i + 1) : g0;
-            const bf16* q0 = qrb + (int64_t)g0 * kTile + lane * 8;
-            const bf16* d0 = dorb + (int64_t)g0 * kTile + lane * 8;
-            const bf16* q1 = qrb + (int64_t)g1 * kTile + lane * 8;
-            const bf16* d1 = dorb + (int64_t)g1 * kTile + lane * 8;
+            const bf16* q0 = qrb + (int64_t)g0 * kTile + r_unit(lane);
+            const bf16* d0 = dorb + (int64_t)g0 * kTile + r_unit(lane);
+            const bf16* q1 = qrb + (int64_t)g1 * kTile + r_unit(lane);
+            const bf16* d1 = dorb + (int64_t)g1 * kTile + r_unit(lane);
             copy16_global_to_lds(q0, stage);
             copy16_global_to_lds(q0 + 512, stage + 512);
             copy16_global_to_lds(d0, stage + kTile);
@@ -662,21 +662,34 @@ __global__ __launch_bounds__(64) void attn_kside_kernel(KSideParams p) {
 
 // ---------------------------------------------------------------------------------------
 // Dense coarsest level.  Every unit (16 pooled tokens) meets every query block, so the Q / dO
-// tiles are the same for all units: a workgroup takes 4 * UPW units (UPW per wave) and one piece
+// tiles are the same for all units: a workgroup takes WAVES * UPW units (UPW per wave) and one piece
 // of the query range and streams that piece through LDS, a pair of query blocks (8 KB) per
-// round, once for all of its units.  The more units a workgroup holds, the fewer times the whole
-// of Q and dO is streamed through the chip: with many coarsest tokens (long sequences) that
-// stream is what the pass costs.
-// The stream is three rounds deep: the tiles of round t + 3 are requested from memory (every wave a
-// quarter, into registers) while those of round t + 1 move from registers into the other LDS buffer
-// and round t is worked on, so a tile has two rounds of arithmetic to arrive.  (Copies straight
-// into LDS cannot be run ahead like that: the compiler waits for all of them before any LDS read.)
-// Each wave ends with the partial sums of its units over this piece of the range.
+// round, once for all of its units.  The stream is three rounds deep: the tiles of round t + 3 are requested from memory (every
+// wave its share, into registers) while those of round t + 1 move from registers into the other LDS buffer and round t is worked on,
+// so a tile has two rounds of arithmetic to arrive.  (Copies straight into LDS cannot be run ahead like that: the compiler
+// waits for all of them before any LDS read.)  Each wave ends with the partial sums of its units over this piece of the range.
+//
+// What bounds it is the instruction stream of a SIMD.  A round of two units is 32 MFMAs of 16 cycles, which keep vector instructions
+// from being issued for 8 of them, 48 vector instructions of 4 cycles and 16 exponentials of 8: 576 cycles if nothing waits.  Waves
+// that run alike read LDS at the same time and then multiply at the same time: four waves of two units took 1009 cycles a round at 6 x
+// 262144 tokens (51 % of the matrix cores' cycles busy).  So
+//  * the vector instructions of one unit are placed between the products of the other (interleave): 960, and
+//  * eight waves take turns: four of them, one per SIMD, fetch their operands from LDS while the other four multiply (862 cycles, 59 %;
+//    820 -> 715 us).  A barrier ends each half; the second four start half a round late.
+// (Tried: the row operands of the next round fetched under the products, exponentials in the half of the LDS reads: both slower;
+// products of 32 x 32, which block vector instructions half as long, with a ring of eight pairs in LDS: 1058, their operands are
+// all needed before the first exponential.)
 // ---------------------------------------------------------------------------------------
-constexpr int kDenseWaves = 4;                    // waves per workgroup
+// Everything one unit's products of a round (two query blocks) need of the round's tiles and statistics
+struct DenseOps {
+    bf16x8 q[2][2], g[2][2];       // R operands of Q and dO
+    bf16x4 tq[2][4], tg[2][4];     // T operands
+    f32x4 l[2], d[2];              // statistics
+};
 
-template <int UPW>
-__global__ __launch_bounds__(64 * kDenseWaves) void attn_kside_dense_kernel(KSideParams p) {
+template <int WAVES, int UPW>
+__global__ __launch_bounds__(64 * WAVES, UPW == 2 ? 2 : 3) void attn_kside_dense_kernel(KSideParams p) {
+    static_assert(WAVES == 4 || WAVES == 8, "a wave moves one or two of the eight half tiles of a pair");
     __shared__ __align__(16) bf16 sh[2][4 * kTile];           // per pair: Q0, dO0, Q1, dO1 as R tiles
     __shared__ __align__(16) float sh_stats[2][64];           // per pair: the statistics of its two query blocks
     const int lane = threadIdx.x & 63;
@@ -685,11 +698,11 @@ __global__ __launch_bounds__(64 * kDenseWaves) void attn_kside_dense_kernel(KSid
     const int N1 = p.N / kBlk;
     // Workgroups that stream the same piece of the query range (one per group of units) get neighbouring logical ids,
     // which xcd_logical_id keeps on one XCD: the piece then comes out of that XCD's L2 for all but the first of them.
-    const int unit_groups = (p.n_units + kDenseWaves * UPW - 1) / (kDenseWaves * UPW);
+    const int unit_groups = (p.n_units + WAVES * UPW - 1) / (WAVES * UPW);
     const int lid = xcd_logical_id();                          // grid: (unit_groups * chunks, BH)
     const int piece = (lid % (int)gridDim.x) / unit_groups;
     const int bh = lid / (int)gridDim.x;
-    const int unit0 = (((lid % (int)gridDim.x) % unit_groups) * kDenseWaves + wave) * UPW;
+    const int unit0 = (((lid % (int)gridDim.x) % unit_groups) * WAVES + wave) * UPW;
     const bool active = unit0 < p.n_units;                    // (n_units is a multiple of UPW; a wave past the end only moves tiles)
     const int start = piece * p.chunk_len;
     const int n_pairs = min(p.chunk_len, N1 - start) / 2;     // even: chunk_len and N1 are multiples of 4
@@ -698,28 +711,29 @@ __global__ __launch_bounds__(64 * kDenseWaves) void attn_kside_dense_kernel(KSid
     const bf16* dorb = p.dor + ((int64_t)bh * N1 + start) * kTile;
     const float* stb = p.stats + ((int64_t)bh * N1 + start) * kStats;
 
-    // wave w moves tile w of a pair's four (query block w/2; Q for even w, dO for odd w); the first 16 lanes of wave 0
-    // also its 64 statistics.  Rounds past the end re-read the last pair (no branch around loads).
-    struct Stage { bf16x8 a, b; f32x4 s; };
+    // The four tiles of a pair are eight half tiles: tile i/2 (query block i/4; Q for even tiles, dO for odd ones), half i%2.  Wave w
+    // moves half tile w (of eight waves) or 2 w and 2 w + 1 (of four); the first 16 lanes of wave 0 also the pair's 64 statistics.
+    // Rounds past the end re-read the last pair (no branch around loads).
+    constexpr int HALVES = 8 / WAVES;
+    struct Stage { bf16x8 h[HALVES]; f32x4 s; };
     const bool stat_lane = wave == 0 && lane < 16;
+    const int half0 = wave * HALVES;
     auto request = [=](int t, Stage& st) __attribute__((always_inline)) {
         t = min(t, n_pairs - 1);
-        const bf16* src = ((wave & 1) ? dorb : qrb) + (int64_t)(2 * t + (wave >> 1)) * kTile;
-        st.a = ld16(src + lane * 8);
-        st.b = ld16(src + 512 + lane * 8);
+        const bf16* src = (((half0 >> 1) & 1) ? dorb : qrb) + (int64_t)(2 * t + (half0 >> 2)) * kTile + (half0 & 1) * 512;
+#pragma unroll
+        for (int i = 0; i < HALVES; i++) st.h[i] = ld16(src + i * 512 + lane * 8);
         // (every lane of every wave loads, lanes 16.. the same as lane % 16: a load inside a branch makes the compiler lose
         // count of the loads in flight, after which it waits for all of them in every round)
-        const int sl = lane & 15;
-        st.s = *reinterpret_cast<const f32x4*>(stb + (int64_t)(2 * t) * kStats + sl * 4);
+        st.s = *reinterpret_cast<const f32x4*>(stb + (int64_t)(2 * t) * kStats + (lane & 15) * 4);
     };
     auto deposit = [&](int t, const Stage& st) __attribute__((always_inline)) {
-        bf16* dst = &sh[t & 1][wave * kTile];
-        st16(dst + lane * 8, st.a);
-        st16(dst + 512 + lane * 8, st.b);
+        bf16* dst = &sh[t & 1][half0 * 512];
+#pragma unroll
+        for (int i = 0; i < HALVES; i++) st16(dst + i * 512 + r_unit(lane), st.h[i]);
         if (stat_lane) *reinterpret_cast<f32x4*>(&sh_stats[t & 1][lane * 4]) = st.s;
     };
     Stage s0, s1;
-    s0.s = s1.s = f32x4{0.f, 0.f, 0.f, 0.f};
     request(0, s0);
     request(1, s1);
     bf16x8 bk[UPW][2], bv[UPW][2];
@@ -743,61 +757,120 @@ __global__ __launch_bounds__(64 * kDenseWaves) void attn_kside_dense_kernel(KSid
             dk[j][dt] = f32x4{0.f, 0.f, 0.f, 0.f};
             dv[j][dt] = f32x4{0.f, 0.f, 0.f, 0.f};
         }
-    // Round t.  The barrier at its top says: buffer t & 1 is filled (every wave deposited its part during round t - 1)
-    // and everybody is done reading the other buffer, which this round refills for round t + 1 out of the registers
-    // `nxt` -- which then take the request for round t + 3.
-    auto round = [&](int t, Stage& nxt) __attribute__((always_inline)) {
-        __syncthreads();
+
+    DenseOps o;
+    f32x4 sc[UPW][2], dp[UPW][2];
+    bf16x8 bp[UPW], bds[UPW];
+    // First half of a round: this wave's operands out of LDS, its share of the next pair into the other buffer, the request for
+    // the pair after the next but one.
+    auto gather = [&](int t, Stage& nxt) __attribute__((always_inline)) {
         const bf16* b = &sh[t & 1][0];
-        bf16x8 aq[2][2], ag[2][2];
-        bf16x4 tq[2][4], tg[2][4];
-        f32x4 l4[2], d4[2];
 #pragma unroll
         for (int u = 0; u < 2; u++) {
-            aq[u][0] = lds_ld16(b + (2 * u) * kTile + lane * 8);
-            aq[u][1] = lds_ld16(b + (2 * u) * kTile + 512 + lane * 8);
-            ag[u][0] = lds_ld16(b + (2 * u + 1) * kTile + lane * 8);
-            ag[u][1] = lds_ld16(b + (2 * u + 1) * kTile + 512 + lane * 8);
+            const bf16* q = b + (2 * u) * kTile;
+            const bf16* g = b + (2 * u + 1) * kTile;
+            o.q[u][0] = lds_ld16(q + r_unit(lane));
+            o.q[u][1] = lds_ld16(q + 512 + r_unit(lane));
+            o.g[u][0] = lds_ld16(g + r_unit(lane));
+            o.g[u][1] = lds_ld16(g + 512 + r_unit(lane));
+            o.l[u] = *reinterpret_cast<const f32x4*>(&sh_stats[t & 1][u * kStats + quad * 4]);
+            o.d[u] = *reinterpret_cast<const f32x4*>(&sh_stats[t & 1][u * kStats + kBlk + quad * 4]);
+        }
+#pragma unroll
+        for (int u = 0; u < 2; u++)
 #pragma unroll
             for (int dt = 0; dt < 4; dt++) {
-                tq[u][dt] = lds_t_operand(b + (2 * u) * kTile, dt, lane);
-                tg[u][dt] = lds_t_operand(b + (2 * u + 1) * kTile, dt, lane);
+                o.tq[u][dt] = lds_t_operand(b + (2 * u) * kTile, dt, lane);
+                o.tg[u][dt] = lds_t_operand(b + (2 * u + 1) * kTile, dt, lane);
             }
-            l4[u] = *reinterpret_cast<const f32x4*>(&sh_stats[t & 1][u * kStats + quad * 4]);
-            d4[u] = *reinterpret_cast<const f32x4*>(&sh_stats[t & 1][u * kStats + kBlk + quad * 4]);
-        }
         deposit(t + 1, nxt);
         request(t + 3, nxt);
-        if (!active) return;
+    };
+    auto scores = [&](int j) __attribute__((always_inline)) {
 #pragma unroll
-        for (int j = 0; j < UPW; j++) {
-            bf16x8 bp, bds;
+        for (int u = 0; u < 2; u++) {
+            const f32x4 z = {0.f, 0.f, 0.f, 0.f};
+            sc[j][u] = mfma_bf16(o.q[u][0], bk[j][0], z);
+            dp[j][u] = mfma_bf16(o.g[u][0], bv[j][0], o.d[u]);
+        }
 #pragma unroll
-            for (int u = 0; u < 2; u++) {
-                f32x4 s = {0.f, 0.f, 0.f, 0.f}, dp = d4[u];
-                s = mfma_bf16(aq[u][0], bk[j][0], s);
-                s = mfma_bf16(aq[u][1], bk[j][1], s);
-                dp = mfma_bf16(ag[u][0], bv[j][0], dp);
-                dp = mfma_bf16(ag[u][1], bv[j][1], dp);
-#pragma unroll
-                for (int e = 0; e < 4; e++) {
-                    const float pe = exp2_fast(fmaf(s[e], kScaleLog2e, l4[u][e]));
-                    bp[u * 4 + e] = (bf16)pe;
-                    bds[u * 4 + e] = (bf16)(pe * dp[e]);
-                }
-            }
-#pragma unroll
-            for (int dt = 0; dt < 4; dt++) {
-                dv[j][dt] = mfma_bf16(cat(tg[0][dt], tg[1][dt]), bp, dv[j][dt]);
-                dk[j][dt] = mfma_bf16(cat(tq[0][dt], tq[1][dt]), bds, dk[j][dt]);
-            }
+        for (int u = 0; u < 2; u++) {
+            sc[j][u] = mfma_bf16(o.q[u][1], bk[j][1], sc[j][u]);
+            dp[j][u] = mfma_bf16(o.g[u][1], bv[j][1], dp[j][u]);
         }
     };
-    // (two rounds per trip without a branch between them: n_pairs is even, and with a conditional second round the
-    // compiler loses count of the loads in flight where the loop closes and waits for all of them)
-    for (int t = 0; t < n_pairs; t += 2) {
-        round(t, s1);
-        round(t + 1, s0);
+    auto exponentials = [&](int j) __attribute__((always_inline)) {
+#pragma unroll
+        for (int u = 0; u < 2; u++)
+#pragma unroll
+            for (int e = 0; e < 4; e++) {
+                const float pe = exp2_fast(fmaf(sc[j][u][e], kScaleLog2e, o.l[u][e]));
+                bp[j][u * 4 + e] = (bf16)pe;
+                bds[j][u * 4 + e] = (bf16)(pe * dp[j][u][e]);
+            }
+    };
+    auto sums = [&](int j) __attribute__((always_inline)) {
+#pragma unroll
+        for (int dt = 0; dt < 4; dt++) {
+            dv[j][dt] = mfma_bf16(cat(o.tg[0][dt], o.tg[1][dt]), bp[j], dv[j][dt]);
+            dk[j][dt] = mfma_bf16(cat(o.tq[0][dt], o.tq[1][dt]), bds[j], dk[j][dt]);
+        }
+    };
+    // the vector instructions of one unit between the products of the other, in this order
+    auto interleave = [&]() __attribute__((always_inline)) {
+#pragma unroll
+        for (int i = 0; i < 8; i++) {
+            __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);      // one MFMA
+            __builtin_amdgcn_sched_group_barrier(0x002, 4, 0);      // four vector ALU instructions (and the exponentials among them)
+        }
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    auto multiply = [&]() __attribute__((always_inline)) {
+        __builtin_amdgcn_sched_barrier(0);
+        scores(0);
+        __builtin_amdgcn_sched_barrier(0);
+        if constexpr (UPW == 2) {
+            scores(1);
+            exponentials(0);
+            interleave();
+            sums(0);
+            exponentials(1);
+            interleave();
+            sums(1);
+        } else {
+            exponentials(0);
+            sums(0);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    if constexpr (WAVES == 8) {
+        // Buffer (t + 1) & 1 is refilled in the first half of round t, by the first four waves while the others multiply round t - 1
+        // and by those while the first multiply round t: nobody reads it then, and it is whole before anybody reads round t + 1.
+        auto round = [&](int t, Stage& nxt) __attribute__((always_inline)) {
+            gather(t, nxt);
+            __syncthreads();
+            if (active) multiply();
+            __syncthreads();
+        };
+        __syncthreads();
+        if (wave >= 4) __syncthreads();
+        for (int t = 0; t < n_pairs; t += 2) {
+            round(t, s1);
+            round(t + 1, s0);
+        }
+        if (wave < 4) __syncthreads();
+    } else {
+        auto round = [&](int t, Stage& nxt) __attribute__((always_inline)) {
+            __syncthreads();
+            gather(t, nxt);
+            if (active) multiply();
+        };
+        // (two rounds per trip without a branch between them: n_pairs is even, and with a conditional second round the
+        // compiler loses count of the loads in flight where the loop closes and waits for all of them)
+        for (int t = 0; t < n_pairs; t += 2) {
+            round(t, s1);
+            round(t + 1, s0);
+        }
     }
     if (!active) return;
 #pragma unroll
@@ -884,10 +957,10 @@ __device__ __forceinline__ void group_pass(const bf16x8 (&bk)[2][2], const bf16x
         for (int u = 0; u < 2; u++) {
             const bf16* q = shq + (2 * t + u) * kTile;
             const bf16* g = shg + (2 * t + u) * kTile;
-            aq[u][0] = lds_ld16(q + lane * 8);
-            aq[u][1] = lds_ld16(q + 512 + lane * 8);
-            ag[u][0] = lds_ld16(g + lane * 8);
-            ag[u][1] = lds_ld16(g + 512 + lane * 8);
+            aq[u][0] = lds_ld16(q + r_unit(lane));
+            aq[u][1] = lds_ld16(q + 512 + r_unit(lane));
+            ag[u][0] = lds_ld16(g + r_unit(lane));
+            ag[u][1] = lds_ld16(g + 512 + r_unit(lane));
 #pragma unroll
             for (int dt = 0; dt < 4; dt++) {
                 tq[u][dt] = lds_t_operand(q, dt, lane);
@@ -954,8 +1027,8 @@ __global__ __launch_bounds__(64 * kGroupWaves, 2) void attn_kside_group_kernel(G
 #pragma unroll
         for (int i = 0; i < 2 * kBlk / kGroupWaves; i++) {
             const int piece = i * kGroupWaves + wave;
-            copy16_global_to_lds(qsrc + piece * 512 + lane * 8, &sh[0][piece * 512]);
-            copy16_global_to_lds(gsrc + piece * 512 + lane * 8, &sh[1][piece * 512]);
+            copy16_global_to_lds(qsrc + piece * 512 + r_unit(lane), &sh[0][piece * 512]);
+            copy16_global_to_lds(gsrc + piece * 512 + r_unit(lane), &sh[1][piece * 512]);
         }
     }
     // Key block j of the group's lists lives in lane j: which tile, which weight, where its partial sum goes.
@@ -1209,7 +1282,7 @@ __global__ __launch_bounds__(1024) void norm_sums_kernel(NormSums p) {
 
 struct DensePlan {
     int n_tok;       // tokens of the dense coarsest level per (b,h)
-    int upw;         // units per wave (1 or 2): a workgroup holds 4 * upw units
+    int wg_units;    // units per workgroup: 16 (eight waves of two), 8 (four waves of two) or 4 (four waves of one)
     int chunks;      // query range split
     int chunk_len;   // query blocks per chunk (a multiple of 4)
     bool merged;     // the dense blocks ride on the group-major pass (one partial sum per group of 16 query blocks)
@@ -1221,16 +1294,17 @@ static DensePlan dense_plan(int B, int H, int N, int levels) {
     d.n_tok = N1;                                             // tokens of pooled level `levels`
     for (int l = 1; l < levels; l++) d.n_tok /= 16;
     const int n_units = d.n_tok / 16;
-    // Q and dO are streamed n_units / (4 * upw) times (mostly out of an L2: see the kernel); four units per wave would
-    // halve that again but leave one wave per SIMD, which measured slower (1.07 ms against 0.93 ms at N = 262144)
-    d.upw = n_units >= 16 ? 2 : 1;
-    const int groups = (n_units + kDenseWaves * d.upw - 1) / (kDenseWaves * d.upw) * B * H;   // workgroups per piece of the query range
+    // Eight waves of two units, unless their last workgroup would be at most half full and there are few of them (N = 5120, 12
+    // heads: 20 units as two workgroups of sixteen 19.8 us, as three of eight 18.5; 28 units, N = 7168: 32 against 35 us).
+    const int last = n_units % 16;
+    d.wg_units = n_units < 16 ? 4 : (last == 0 || last > 8 || n_units > 64 ? 16 : 8);
+    const int groups = (n_units + d.wg_units - 1) / d.wg_units * B * H;   // workgroups per piece of the query range
     // The query range is cut so that the workgroups fill the chip's resident slots (256 CUs x the workgroups the
     // registers allow per CU) a whole number of times: a count just above a multiple of the slots leaves a last round in
     // which a few workgroups run alone.  Three times where the pieces are long even so, which evens out their progress
     // (N = 262144: 862 us against 920 for once); once where they are short, for a third of the partial sums (N = 7168, 15
-    // heads: the reduction 13.6 -> 7.6 us, the pass itself the same).
-    const int slots = 256 * (d.upw == 2 ? 2 : 3);
+    // heads: the reduction 13.6 -> 7.6 us, the pass itself the same).  (Both measured with four waves of two units.)
+    const int slots = 256 * (d.wg_units == 16 ? 1 : d.wg_units == 8 ? 2 : 3);
     int chunks = slots / groups;
     if (chunks < 1 || N1 / chunks > 256) chunks = 3 * slots / groups;
     if (chunks > N1 / 16) chunks = N1 / 16;
@@ -1500,9 +1574,10 @@ extern "C" int llsa_attn_bwd(const llsa_attn_bwd_args* a, void* stream) {
             rp.job[rp.n_jobs - 1].half_part = 1;
             return;
         }
-        const dim3 grid((p.n_units + kDenseWaves * d.upw - 1) / (kDenseWaves * d.upw) * d.chunks, BH), block(64 * kDenseWaves);
-        if (d.upw == 2) hipLaunchKernelGGL(HIP_KERNEL_NAME(attn_kside_dense_kernel<2>), grid, block, 0, s, p);
-        else hipLaunchKernelGGL(HIP_KERNEL_NAME(attn_kside_dense_kernel<1>), grid, block, 0, s, p);
+        const dim3 grid((p.n_units + d.wg_units - 1) / d.wg_units * d.chunks, BH);
+        if (d.wg_units == 16) hipLaunchKernelGGL(HIP_KERNEL_NAME(attn_kside_dense_kernel<8, 2>), grid, dim3(512), 0, s, p);
+        else if (d.wg_units == 8) hipLaunchKernelGGL(HIP_KERNEL_NAME(attn_kside_dense_kernel<4, 2>), grid, dim3(256), 0, s, p);
+        else hipLaunchKernelGGL(HIP_KERNEL_NAME(attn_kside_dense_kernel<4, 1>), grid, dim3(256), 0, s, p);
         add_job(p, 1, p.n_units, d.chunks);
     };
 

@@ -209,7 +209,7 @@ template <int Q, int R>
 __global__ __launch_bounds__(256, Q == 1 ? 4 : 3) void attn_fwd_kernel(llsa_attn_fwd_args a) {
     __shared__ __align__(16) bf16 sh[2][kGroup][2 * kTile];
     __shared__ int order[4][R * kWave];
-    const int lane = threadIdx.x & 63;
+    const int lane = threadIdx.x & 63, unit = r_unit(lane);
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int N1 = a.N / kBlk, T = a.T;
     const int lid = xcd_logical_id();
@@ -314,11 +314,11 @@ __global__ __launch_bounds__(256, Q == 1 ? 4 : 3) void attn_fwd_kernel(llsa_attn
             bf16* slot = slots + (s & 1) * (2 * kTile);
 #pragma unroll
             for (int j = 0; j < 2; j++) {
-                const int64_t at = (int64_t)ml.block(min(2 * s + j, ml.n - 1)) * kTile + lane * 8;
-                dst.k[j][0] = ld16(kr + at);
-                dst.k[j][1] = ld16(kr + at + 512);
-                copy16_global_to_lds(vr + at, slot + j * kTile);
-                copy16_global_to_lds(vr + at + 512, slot + j * kTile + 512);
+                const int64_t at = (int64_t)ml.block(min(2 * s + j, ml.n - 1)) * kTile;
+                dst.k[j][0] = ld16(kr + at + lane * 8);
+                dst.k[j][1] = ld16(kr + at + lane * 8 + 512);
+                copy16_global_to_lds(vr + at + unit, slot + j * kTile);
+                copy16_global_to_lds(vr + at + unit + 512, slot + j * kTile + 512);
             }
         };
         auto work = [&](int s, KeyRegs<2>& cur, KeyRegs<2>& nxt) __attribute__((always_inline)) {

@@ -115,10 +115,17 @@ __device__ __forceinline__ int t_tile_off(int t, int c) { return (((c >> 4) * 4 
 // 16*dt + 4*(j%4) ..+3) therefore hands lane i tokens 4*(l/16)..+3 of channel 16*dt + i: the T
 // operand.  So K/Q/dO are fetched from HBM once, as R tiles, and the second orientation is
 // made on chip instead of being read from a second copy.
+//
+// In LDS such a tile is kept with the rows of every odd 8-channel chunk permuted (row ^ 12).  In the layout of memory the transposing
+// read's groups of 16 lanes take 64 bytes of chunk 2 dt and 64 bytes of chunk 2 dt + 1, which lie 256 bytes further and so in the
+// same banks, and every one of these reads takes two cycles more: a quarter to a third of all LDS cycles of the backward kernels.
+// The permutation costs nothing: the lane that copies a 16-byte unit into LDS fetches another one of the same kilobyte
+// (r_unit), and plain reads use the same lane-dependent offset.
 typedef __attribute__((ext_vector_type(4))) short s16x4;
+__device__ __forceinline__ int r_unit(int lane) { return (lane ^ ((lane >> 4) & 1) * 12) * 8; }    // element offset of a lane's unit in half a tile
 __device__ __forceinline__ bf16x4 lds_t_operand(const bf16* r_tile_in_lds, int dt, int lane) {
     const int j = lane & 15, q = lane >> 4;
-    const bf16* p = r_tile_in_lds + r_tile_off(4 * q + (j >> 2), 16 * dt + 4 * (j & 3));
+    const bf16* p = r_tile_in_lds + r_tile_off((4 * q + (j >> 2)) ^ ((j >> 1) & 1) * 12, 16 * dt + 4 * (j & 3));
     const s16x4 v = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) s16x4*)p);
     return __builtin_bit_cast(bf16x4, v);
 }
