@@ -43,7 +43,7 @@ extern "C" {
 #define LLSA_DTYPE_BF16 0
 #define LLSA_DTYPE_F32 1
 
-#define LLSA_ABI_VERSION 207     /* changes with every change of a signature or argument structure below */
+#define LLSA_ABI_VERSION 208     /* changes with every change of a signature or argument structure below */
 int llsa_version(void);          /* LLSA_ABI_VERSION of the built library                                    */
 const char* llsa_last_error_string(void);
 
@@ -228,6 +228,9 @@ typedef struct llsa_transpose_job {
     int32_t Mb, Kb, T, chunk;
 } llsa_transpose_job;
 int llsa_transpose_indices_multi(const llsa_transpose_job* jobs, int n_jobs, int B, int H, void* stream);
+/* llsa_attn_fwd and llsa_transpose_indices_multi (of the selections the attention reads, the same B and H) in one call.  Jobs that
+ * are small enough are made by workgroups of the attention launch, beside its own; otherwise they follow it on the stream. */
+int llsa_attn_fwd_lists(const llsa_attn_fwd_args* a, const llsa_transpose_job* jobs, int n_jobs, void* stream);
 int llsa_transpose_one_launch(int Mb, int Kb, int T, int B, int H);
 
 /* Work list for the K-side backward kernels, written by llsa_transpose_indices when `work` is

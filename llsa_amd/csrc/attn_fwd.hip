@@ -17,6 +17,7 @@
 // are kept in units of the current segment's weight, converted once at each segment boundary.
 #include "llsa_device.h"
 #include "llsa_host.h"
+#include "transpose_device.h"
 #include "../../include/llsa_hip.h"
 
 namespace llsa {
@@ -205,14 +206,27 @@ __device__ __forceinline__ void finish_query_block(const llsa_attn_fwd_args& a, 
 // 62 us for 12 x 16384 tokens): the wave merges its lists (merge_lists) and walks the union, two blocks per step, every
 // block fetched once and multiplied with the query blocks that selected it.  What bounds the fine part is the rate at which
 // tiles arrive from the L2, and waves enough to keep the fetches in flight.
+// The first `list_rows` rows of the grid make the index transposes of the backward (transpose_device.h): they need the selection
+// and nothing else, and are latency for the most part, which the attention's workgroups fill.  In a launch of their own behind this
+// one the chip waited for them: step of 12 x 16384 tokens 317 -> 309 us, of 24 x 4096 163 -> 156, of 48 x 16384 1284 -> 1264; both
+// kernels of 6 x 65536 157 -> 154, where 75 workgroups a head read all its 65536 entries each.
+constexpr int kTrLdsFwd = 2 * kGroup * 2 * kTile / 2 - 32;    // ints of the kernel's LDS they work in (32 for their scratch)
+static_assert(tr_scratch_ints(256) <= 32, "the scratch of a transposing workgroup");
+
 template <int Q, int R>
-__global__ __launch_bounds__(256, Q == 1 ? 4 : 3) void attn_fwd_kernel(llsa_attn_fwd_args a) {
+__global__ __launch_bounds__(256, Q == 1 ? 4 : 3) void attn_fwd_kernel(llsa_attn_fwd_args a, TrJobs lists, int list_rows) {
     __shared__ __align__(16) bf16 sh[2][kGroup][2 * kTile];
     __shared__ int order[4][R * kWave];
+    if ((int)blockIdx.y < list_rows) {
+        const int block = (int)(blockIdx.y * gridDim.x + blockIdx.x);
+        int* const lds = reinterpret_cast<int*>(&sh[0][0][0]);
+        if (block < lists.wgs * ((int)gridDim.y - list_rows)) transpose_block<256>(lists, block, lds, lds + kTrLdsFwd);
+        return;
+    }
     const int lane = threadIdx.x & 63, unit = r_unit(lane);
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int N1 = a.N / kBlk, T = a.T;
-    const int lid = xcd_logical_id();
+    const int lid = xcd_logical_id(list_rows);
     const int g = (lid % (int)gridDim.x) * (4 * Q) + Q * wave;        // query blocks g .. g + Q - 1 (the host checks N1 % 4 Q == 0)
     const int bh = lid / (int)gridDim.x, b = bh / a.H, h = bh % a.H;
 
@@ -359,7 +373,8 @@ __global__ __launch_bounds__(256, Q == 1 ? 4 : 3) void attn_fwd_kernel(llsa_attn
 
 using namespace llsa;
 
-extern "C" int llsa_attn_fwd(const llsa_attn_fwd_args* a, void* stream) {
+// jobs: the index transposes that ride along, or nullptr
+static int attn_fwd(const llsa_attn_fwd_args* a, const llsa_transpose_job* jobs, int n_jobs, void* stream) {
     LLSA_REQUIRE(a != nullptr, "attn_fwd: null args");
     LLSA_REQUIRE(a->levels >= 1 && a->levels <= LLSA_MAX_LEVELS, "attn_fwd: levels must be 1..%d", LLSA_MAX_LEVELS);
     LLSA_REQUIRE(a->B > 0 && a->H > 0 && a->N > 0, "attn_fwd: bad B/H/N");
@@ -397,10 +412,23 @@ extern "C" int llsa_attn_fwd(const llsa_attn_fwd_args* a, void* stream) {
     shared += coarsest;
     const int64_t groups = (int64_t)N1 / 8 * BH;
     const bool pairs = a->T <= kPairMaxTopk && N1 % 8 == 0 && groups >= kPairMinGroups && (shared >= 4 * a->T || groups >= 2048);
-    const dim3 grid(N1 / (pairs ? 8 : 4), BH);
+    TrJobs lists{};
+    const int width = N1 / (pairs ? 8 : 4);                   // (a multiple of 8: N is one of 1024)
+    const bool ride = jobs != nullptr && plan_transpose(jobs, n_jobs, a->B, a->H, kTrLdsFwd, lists);
+    const int rows = ride ? (int)(((int64_t)lists.wgs * BH + width - 1) / width) : 0;
+    const dim3 grid(width, BH + rows);
     const hipStream_t st = (hipStream_t)stream;
-    if (!pairs) hipLaunchKernelGGL(HIP_KERNEL_NAME(attn_fwd_kernel<1, 1>), grid, dim3(256), 0, st, *a);
-    else if (a->T <= 32) hipLaunchKernelGGL(HIP_KERNEL_NAME(attn_fwd_kernel<2, 1>), grid, dim3(256), 0, st, *a);
-    else hipLaunchKernelGGL(HIP_KERNEL_NAME(attn_fwd_kernel<2, 2>), grid, dim3(256), 0, st, *a);
-    return launch_status("attn_fwd");
+    if (!pairs) hipLaunchKernelGGL(HIP_KERNEL_NAME(attn_fwd_kernel<1, 1>), grid, dim3(256), 0, st, *a, lists, rows);
+    else if (a->T <= 32) hipLaunchKernelGGL(HIP_KERNEL_NAME(attn_fwd_kernel<2, 1>), grid, dim3(256), 0, st, *a, lists, rows);
+    else hipLaunchKernelGGL(HIP_KERNEL_NAME(attn_fwd_kernel<2, 2>), grid, dim3(256), 0, st, *a, lists, rows);
+    const int rc = launch_status("attn_fwd");
+    if (rc != 0 || jobs == nullptr || ride) return rc;
+    return llsa_transpose_indices_multi(jobs, n_jobs, a->B, a->H, stream);
+}
+
+extern "C" int llsa_attn_fwd(const llsa_attn_fwd_args* a, void* stream) { return attn_fwd(a, nullptr, 0, stream); }
+
+extern "C" int llsa_attn_fwd_lists(const llsa_attn_fwd_args* a, const llsa_transpose_job* jobs, int n_jobs, void* stream) {
+    LLSA_REQUIRE(jobs != nullptr && n_jobs >= 1 && n_jobs <= LLSA_MAX_LEVELS, "attn_fwd_lists: 1..%d jobs, got %d", LLSA_MAX_LEVELS, n_jobs);
+    return attn_fwd(a, jobs, n_jobs, stream);
 }

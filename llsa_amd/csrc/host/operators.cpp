@@ -100,6 +100,7 @@ struct Library {
     decltype(&llsa_topk_cascade) topk_cascade;
     decltype(&llsa_topk_cascade_max_parents) topk_cascade_max_parents;
     decltype(&llsa_attn_fwd) attn_fwd;
+    decltype(&llsa_attn_fwd_lists) attn_fwd_lists;
     decltype(&llsa_transpose_indices_multi) transpose_indices_multi;
     decltype(&llsa_transpose_one_launch) transpose_one_launch;
     decltype(&llsa_work_list_len) work_list_len;
@@ -118,6 +119,7 @@ struct Library {
         get("llsa_topk_cascade", topk_cascade);
         get("llsa_topk_cascade_max_parents", topk_cascade_max_parents);
         get("llsa_attn_fwd", attn_fwd);
+        get("llsa_attn_fwd_lists", attn_fwd_lists);
         get("llsa_transpose_indices_multi", transpose_indices_multi);
         get("llsa_transpose_one_launch", transpose_one_launch);
         get("llsa_work_list_len", work_list_len);
@@ -488,8 +490,8 @@ Tensor attend(const std::shared_ptr<Library>& lib, const Tensor& q_in, const Ten
                                         y.topk[l], stream),
                        "compute_topk_indices_sparse");
 
-        // The lists of the backward (the transposed selections of all levels).  Where one launch makes them all they follow
-        // the attention kernel on the same stream; the several kernels per level of the longest sequences run on a second
+        // The lists of the backward (the transposed selections of all levels).  Where one launch can make them all they ride in
+        // the attention kernel's (or follow it on the same stream); the several kernels per level of the longest sequences run on a second
         // stream beside the attention kernel: the attention kernel is issued first (the GPU is waiting for it), and an
         // event recorded before it lets the second stream start as soon as the selection is done.  With few tokens over all
         // heads the event calls cost more than the overlap saves: everything then goes to the one stream.
@@ -513,22 +515,21 @@ Tensor attend(const std::shared_ptr<Library>& lib, const Tensor& q_in, const Ten
                 lv.T = y.topk[l];
             }
         }
-        lib->check(lib->attn_fwd(&f, stream), "attn_fwd");
+        llsa_transpose_job jobs[kL];
+        for (int l = 0; l < L && grad; l++) {
+            const int32_t m = static_cast<int32_t>(n[l + 1]);
+            jobs[l] = llsa_transpose_job{ints(y.sel[l]), ints(y.off[l]), ints(y.flat[l]), l == 0 ? ints(y.work) : nullptr, l == 0 ? nullptr : ints(y.inv[l]),
+                                         m, m, y.topk[l], l == 0 ? y.chunk : 1};
+        }
+        if (grad && !beside) lib->check(lib->attn_fwd_lists(&f, jobs, L, stream), "attn_fwd");
+        else lib->check(lib->attn_fwd(&f, stream), "attn_fwd");
 
         if (grad) {
-            llsa_transpose_job jobs[kL];
-            for (int l = 0; l < L; l++) {
-                const int32_t m = static_cast<int32_t>(n[l + 1]);
-                jobs[l] = llsa_transpose_job{ints(y.sel[l]), ints(y.off[l]), ints(y.flat[l]), l == 0 ? ints(y.work) : nullptr, l == 0 ? nullptr : ints(y.inv[l]),
-                                             m, m, y.topk[l], l == 0 ? y.chunk : 1};
-            }
-            void* lists = stream;
             if (beside) {
-                lists = side_stream(dev);
+                void* lists = side_stream(dev);
                 hip_check(hipStreamWaitEvent(static_cast<hipStream_t>(lists), side_events(dev).ready, 0));       // (the arena is older than the selection, so this covers it too)
-            }
-            lib->check(lib->transpose_indices_multi(jobs, L, b, h, lists), "transpose_indices");
-            if (beside) {                                    // (and the arena is not handed out again before the second stream is done)
+                lib->check(lib->transpose_indices_multi(jobs, L, b, h, lists), "transpose_indices");
+                // (and the arena is not handed out again before the second stream is done)
                 hip_check(hipEventRecord(side_events(dev).done, static_cast<hipStream_t>(lists)));
                 hip_check(hipStreamWaitEvent(static_cast<hipStream_t>(stream), side_events(dev).done, 0));
             }

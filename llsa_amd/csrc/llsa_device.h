@@ -355,9 +355,10 @@ __device__ __forceinline__ void lds_st8(bf16* p, bf16x4 v) {
 // L2: this maps the hardware id to a logical id such that every XCD walks one contiguous
 // range of the (x, y) grid.  Returns the logical linear id in [0, gridDim.x * gridDim.y).
 constexpr int kXcds = 8;
-__device__ __forceinline__ int xcd_logical_id() {
-    const int total = gridDim.x * gridDim.y;
-    const int lin = blockIdx.y * gridDim.x + blockIdx.x;
+// `rows_before`: rows of the grid in front that do other work (their number times gridDim.x is a multiple of 8).
+__device__ __forceinline__ int xcd_logical_id(int rows_before = 0) {
+    const int total = gridDim.x * (gridDim.y - rows_before);
+    const int lin = (blockIdx.y - rows_before) * gridDim.x + blockIdx.x;
     const int xcd = lin % kXcds, slot = lin / kXcds;
     const int q = total / kXcds, rem = total % kXcds;
     return xcd * q + (xcd < rem ? xcd : rem) + slot;
