@@ -1092,30 +1092,101 @@ __global__ __launch_bounds__(64 * kGroupWaves, 2) void attn_kside_group_kernel(G
     }
 }
 
-// Finishes the units whose list was cut into several pieces: the result is the sum of the
-// unit's partial slots, added in chunk order, so it does not depend on scheduling.  One launch
-// serves the three K-side passes.
-struct ReduceJob {
-    const f32x4* part;       // fp32 partial sums, or, with half_part, the bf16 ones of the group-major pass (as bf16x4)
+// The gradients of the pooled levels out of their partial sums: a workgroup of 1024 threads per unit.  A bf16 partial sum (group-major
+// pass) is 16 bytes a thread of 256, an fp32 one (dense pass) of 512: four or two slices of the workgroup take every fourth or every
+// second one, four loads in flight a thread, and their sums meet in LDS in slice order, so that the result does not depend on
+// scheduling.  The kernel is a few round trips to memory one after the other: with one workgroup of 256 threads a unit and sixteen
+// loads in flight it took 17 us at 12 x 16384 tokens (14 now), 110 at 6 x 262144 (102), 53 at 48 x 16384 (45.5); eight loads in
+// flight, or 512 threads, 2 to 5 % more.
+struct PooledJob {
+    const void* part;        // fp32 (f32x4[8][64] a slot) or, with half_part, bf16 (bf16x8[4][64] a slot) partial sums
     int half_part;
-    const int* off;          // CSR offsets (list-driven jobs) or nullptr (dense job)
-    const int* work;         // work list (fine job); nullptr with `off`: the partial sums of unit u are slots
-                             // [off[u] << csr_shift, off[u + 1] << csr_shift) (group-major pooled jobs)
+    const int* off;          // the partial sums of unit u are slots [off[u] << csr_shift, off[u + 1] << csr_shift) of its (b,h), or ...
     int csr_shift;
+    int64_t slot_stride;     // slots per (b,h)
+    int n_chunks;            // ... (off == nullptr) this many at stride BH * n_units slots
+    int n_units;
+    bf16* dk; bf16* dv;      // (B,H,16 n_units,64), contiguous
+};
+struct PooledJobs {
+    PooledJob job[LLSA_MAX_LEVELS];
+    int n_jobs;
+};
+constexpr int kReduceThreads = 1024;
+__global__ __launch_bounds__(kReduceThreads, 8) void pooled_reduce_kernel(PooledJobs jobs) {
+    __shared__ __align__(16) float sums[3 * 256 * 8];         // of all slices but the first
+    // grid.x: the units of all jobs, the coarsest level's first: they have the most partial sums
+    int u = blockIdx.x, ji = jobs.n_jobs - 1;
+    while (u >= jobs.job[ji].n_units) u -= jobs.job[ji--].n_units;
+    const PooledJob& jb = jobs.job[ji];
+    const int bh = blockIdx.y, width = jb.half_part ? 256 : 512, slices = kReduceThreads / width;
+    const int slice = (int)threadIdx.x / width, pos = (int)threadIdx.x % width;
+    int64_t first, stride;
+    int n;
+    if (jb.off != nullptr) {
+        const int* o = jb.off + (int64_t)bh * (jb.n_units + 1) + u;
+        const int o0 = o[0];
+        n = (o[1] - o0) << jb.csr_shift;
+        first = (int64_t)bh * jb.slot_stride + ((int64_t)o0 << jb.csr_shift);
+        stride = 1;
+    } else {
+        n = jb.n_chunks;
+        first = (int64_t)bh * jb.n_units + u;
+        stride = (int64_t)gridDim.y * jb.n_units;
+    }
+    constexpr int kBatch = 4;
+    f32x4 acc = {0.f, 0.f, 0.f, 0.f}, acc2 = {0.f, 0.f, 0.f, 0.f};
+    const i32x4* ps = reinterpret_cast<const i32x4*>(jb.part) + first * width + pos;
+    for (int c0 = slice; c0 < n; c0 += kBatch * slices) {
+        i32x4 v[kBatch];
+#pragma unroll
+        for (int k = 0; k < kBatch; k++) v[k] = ps[(int64_t)min(c0 + k * slices, n - 1) * stride * width];
+#pragma unroll
+        for (int k = 0; k < kBatch; k++)
+            if (c0 + k * slices < n) {
+                if (jb.half_part) {
+                    const bf16x8 x = __builtin_bit_cast(bf16x8, v[k]);
+                    acc += f32x4{(float)x[0], (float)x[1], (float)x[2], (float)x[3]};
+                    acc2 += f32x4{(float)x[4], (float)x[5], (float)x[6], (float)x[7]};
+                } else {
+                    acc += __builtin_bit_cast(f32x4, v[k]);
+                }
+            }
+    }
+    if (slice > 0) {
+        f32x4* dst = reinterpret_cast<f32x4*>(sums);
+        dst[(slice - 1) * width + pos] = acc;
+        if (jb.half_part) dst[(3 + slice - 1) * width + pos] = acc2;
+    }
+    __syncthreads();
+    if (slice > 0) return;
+    const f32x4* src = reinterpret_cast<const f32x4*>(sums);
+    for (int i = 0; i + 1 < slices; i++) {
+        acc += src[i * width + pos];
+        if (jb.half_part) acc2 += src[(3 + i) * width + pos];
+    }
+    const int lane = pos & 63, r = lane & 15, quad = lane >> 4, reg = jb.half_part ? 2 * (pos >> 6) : pos >> 6;       // (bf16: registers reg, reg + 1)
+    const int dt = reg & 3;
+    const bool is_k = reg < 4;
+    bf16* dst = (is_k ? jb.dk : jb.dv) + (((int64_t)bh * jb.n_units + u) * kBlk + r) * kD + dt * 16 + quad * 4;
+    st8(dst, cvt4(is_k ? acc * kScale : acc));
+    if (jb.half_part) st8(dst + 16, cvt4(is_k ? acc2 * kScale : acc2));
+}
+
+// Finishes the fine units whose list was cut into several pieces: the result is the sum of the
+// unit's fp32 partial slots, added in piece order, so it does not depend on scheduling.
+struct ReduceParams {
+    const f32x4* part;
+    const int* work;         // work list
     bf16* dk; int64_t sdkb, sdkh, sdkn;
     bf16* dv; int64_t sdvb, sdvh, sdvn;
-    int n_units, chunk, max_units;       // max_units: upper bound of units this job can have per (b,h)
+    int n_units, max_units, H, N;        // max_units: upper bound of units that can have several pieces per (b,h)
     int64_t work_stride, slot_stride;
-    int n_chunks;            // dense job: partials per unit, at stride BH * n_units slots
-    PoolFold fold;           // fine job only
-    llsa_norm_back norm;     // fine job only: the norm of k (x: nullptr without)
-};
-struct ReduceParams {
-    ReduceJob job[LLSA_MAX_LEVELS + 1];
-    int n_jobs, H, N;
+    PoolFold fold;
+    llsa_norm_back norm;     // the norm of k (x: nullptr without)
 };
 
-// Unit positions per job and (b,h) that are walked in parallel: a quarter of the most units the job can have,
+// Unit positions per (b,h) that are walked in parallel: a quarter of the most units there can be,
 // between 32 and 256.  Usually a few per cent of the units have several pieces, and every position beyond
 // them is a pair of workgroups that starts, reads one record and leaves (at 256 positions for a job of at
 // most 257 units that cost 4 us per launch).
@@ -1125,102 +1196,51 @@ __host__ __device__ inline int reduce_slots(int max_units) {
     return q < 32 ? 32 : (q > 256 ? 256 : q);
 }
 
-__global__ __launch_bounds__(256) void kside_reduce_kernel(ReduceParams rp) {
-    // fp32 partial sums: two workgroups per unit; every thread owns one f32x4 of the unit's 8 x 64 accumulator
-    // registers and streams that position of all partials, sixteen loads in flight.  bf16 partial sums (the group-major
-    // pass): one workgroup per unit, every thread owns a pair of registers (16 bytes a partial, like the fp32 loads), and
-    // the two workgroups of a position take alternate units.  Every job has its own range of workgroup pairs
-    // (reduce_slots of them), which walk the job's units with that stride: the number of units with several pieces is
-    // known only on the device and usually small, and a grid sized for the worst case would be mostly workgroups that
-    // start, look and leave.
+__global__ __launch_bounds__(256) void kside_reduce_kernel(ReduceParams p) {
+    // Two workgroups per unit (dK, dV); every thread owns one f32x4 of the unit's 8 x 64 accumulator registers and streams that
+    // position of all partials, sixteen loads in flight.  The workgroups (reduce_slots pairs of them) walk the units with that
+    // stride: the number of units with several pieces is known only on the device and usually small, and a grid sized for the worst
+    // case would be mostly workgroups that start, look and leave.
     __shared__ float row_ss[4][kBlk], row_dot[4][kBlk];
-    const int bh = blockIdx.y, b = bh / rp.H, h = bh % rp.H;
-    int u0 = blockIdx.x >> 1, j = 0;
-    while (j < rp.n_jobs && u0 >= reduce_slots(rp.job[j].max_units)) {
-        u0 -= reduce_slots(rp.job[j].max_units);
-        j++;
-    }
-    if (j >= rp.n_jobs) return;
-    const ReduceJob& jb = rp.job[j];
-    const int half = jb.half_part;
-    const int pos = half ? (int)threadIdx.x : (int)((blockIdx.x & 1) * 256 + threadIdx.x);
-    const int reg = half ? 2 * (pos >> 6) : (pos >> 6), lane = pos & 63;     // (half: registers reg, reg + 1)
+    const int bh = blockIdx.y, b = bh / p.H, h = bh % p.H;
+    const int u0 = blockIdx.x >> 1;
+    const int which = blockIdx.x & 1;                         // 0: dK, 1: dV
+    const int dt = (int)(threadIdx.x >> 6), lane = (int)(threadIdx.x & 63);
     const int r = lane & 15, quad = lane >> 4;
-    const int dt = reg & 3;
-    const int which = reg >> 2;                               // 0: dK, 1: dV
-    const int step = reduce_slots(jb.max_units) * (half ? 2 : 1);
-    if (half) u0 = 2 * u0 + (int)(blockIdx.x & 1);
-    const int* work = jb.work ? jb.work + (int64_t)bh * jb.work_stride : nullptr;
-    const int max_items = (int)(jb.work_stride - work_tail_len(jb.n_units) - 4 - 4 * jb.max_units) / 4;
+    const int step = reduce_slots(p.max_units);
+    const int* work = p.work + (int64_t)bh * p.work_stride;
+    const int max_items = (int)(p.work_stride - work_tail_len(p.n_units) - 4 - 4 * p.max_units) / 4;
     // the unit's record is fetched together with the count it is checked against (u0 is always
     // inside the list's storage): one memory round trip instead of two
-    const int* multi = work ? work + 4 + 4 * max_items : nullptr;
-    int rec_unit = 0, rec_first = 0, rec_n = 0;
-    if (work != nullptr) {
-        rec_unit = multi[4 * u0];
-        rec_first = multi[4 * u0 + 1];
-        rec_n = multi[4 * u0 + 2];
-    }
-    const int count = work ? min(work[2], jb.max_units) : jb.n_units;
+    const int* multi = work + 4 + 4 * max_items;
+    int rec_unit = multi[4 * u0], rec_first = multi[4 * u0 + 1], rec_n = multi[4 * u0 + 2];
+    const int count = min(work[2], p.max_units);
     for (int u = u0; u < count; u += step) {
-        int unit, n;
-        int64_t first, stride;
-        if (work != nullptr) {
-            if (u != u0) {
-                rec_unit = multi[4 * u];
-                rec_first = multi[4 * u + 1];
-                rec_n = multi[4 * u + 2];
-            }
-            unit = rec_unit;
-            n = rec_n;
-            first = (int64_t)bh * jb.slot_stride + rec_first;
-            stride = 1;
-        } else if (jb.off != nullptr) {
-            const int* o = jb.off + (int64_t)bh * (jb.n_units + 1) + u;
-            const int o0 = o[0], o1 = o[1];
-            unit = u;
-            n = (o1 - o0) << jb.csr_shift;
-            first = (int64_t)bh * jb.slot_stride + ((int64_t)o0 << jb.csr_shift);
-            stride = 1;
-        } else {
-            unit = u;
-            n = jb.n_chunks;
-            first = (int64_t)bh * jb.n_units + unit;
-            stride = (int64_t)gridDim.y * jb.n_units;
+        if (u != u0) {
+            rec_unit = multi[4 * u];
+            rec_first = multi[4 * u + 1];
+            rec_n = multi[4 * u + 2];
         }
-        f32x4 acc = {0.f, 0.f, 0.f, 0.f}, acc2 = {0.f, 0.f, 0.f, 0.f};
-        if (half) {
-            const bf16x8* ps = reinterpret_cast<const bf16x8*>(jb.part) + first * (4 * kWave) + (reg >> 1) * kWave + lane;
-            for (int c0 = 0; c0 < n; c0 += 16) {
-                bf16x8 v[16];
+        const int unit = rec_unit, n = rec_n;
+        const int64_t first = (int64_t)bh * p.slot_stride + rec_first;
+        f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+        const f32x4* ps = p.part + first * (8 * kWave) + (4 * which + dt) * kWave + lane;
+        for (int c0 = 0; c0 < n; c0 += 16) {
+            f32x4 v[16];
 #pragma unroll
-                for (int k = 0; k < 16; k++) v[k] = ps[(int64_t)min(c0 + k, n - 1) * stride * (4 * kWave)];
+            for (int k = 0; k < 16; k++) v[k] = ps[(int64_t)min(c0 + k, n - 1) * (8 * kWave)];
 #pragma unroll
-                for (int k = 0; k < 16; k++)
-                    if (c0 + k < n) {
-                        acc += f32x4{(float)v[k][0], (float)v[k][1], (float)v[k][2], (float)v[k][3]};
-                        acc2 += f32x4{(float)v[k][4], (float)v[k][5], (float)v[k][6], (float)v[k][7]};
-                    }
-            }
-        } else {
-            const f32x4* ps = jb.part + first * (8 * kWave) + reg * kWave + lane;
-            for (int c0 = 0; c0 < n; c0 += 16) {
-                f32x4 v[16];
-#pragma unroll
-                for (int k = 0; k < 16; k++) v[k] = ps[(int64_t)min(c0 + k, n - 1) * stride * (8 * kWave)];
-#pragma unroll
-                for (int k = 0; k < 16; k++)
-                    if (c0 + k < n) acc += v[k];               // chunk order: the sum does not depend on scheduling
-            }
+            for (int k = 0; k < 16; k++)
+                if (c0 + k < n) acc += v[k];
         }
-        bf16* dst = which ? jb.dv + b * jb.sdvb + h * jb.sdvh + (int64_t)(unit * kBlk + r) * jb.sdvn
-                          : jb.dk + b * jb.sdkb + h * jb.sdkh + (int64_t)(unit * kBlk + r) * jb.sdkn;
+        bf16* dst = which ? p.dv + b * p.sdvb + h * p.sdvh + (int64_t)(unit * kBlk + r) * p.sdvn
+                          : p.dk + b * p.sdkb + h * p.sdkh + (int64_t)(unit * kBlk + r) * p.sdkn;
         bf16x4 out = cvt4(which ? acc : acc * kScale);
-        if (jb.fold.depth > 0)
-            out = fold_pooled(out, jb.fold, which, bh, rp.N, unit * kBlk + r, dt * 16 + quad * 4);
-        if (jb.norm.x != nullptr && which == 0) {             // (uniform over the workgroup: fp32 partial sums, dK in one workgroup)
+        if (p.fold.depth > 0)
+            out = fold_pooled(out, p.fold, which, bh, p.N, unit * kBlk + r, dt * 16 + quad * 4);
+        if (p.norm.x != nullptr && which == 0) {              // (uniform over the workgroup)
             // wave dt holds channels 16 dt .. of the unit's rows: norm_back with the sums over a row's channels through LDS
-            const llsa_norm_back& nb = jb.norm;
+            const llsa_norm_back& nb = p.norm;
             const int c0 = dt * 16 + quad * 4;
             const bf16x4 x = ld8((const bf16*)nb.x + b * nb.sxb + h * nb.sxh + (int64_t)(unit * kBlk + r) * nb.sxn + c0);
             const f32x4 gamma = {nb.gamma[c0], nb.gamma[c0 + 1], nb.gamma[c0 + 2], nb.gamma[c0 + 3]};
@@ -1250,10 +1270,9 @@ __global__ __launch_bounds__(256) void kside_reduce_kernel(ReduceParams rp) {
             for (int d = 1; d < 16; d <<= 1)
 #pragma unroll
                 for (int e = 0; e < 4; e++) contrib[e] += __shfl_xor(contrib[e], d);
-            if (r == 0) *reinterpret_cast<f32x4*>(nb.partials + ((int64_t)bh * jb.n_units + unit) * kD + c0) = contrib;
+            if (r == 0) *reinterpret_cast<f32x4*>(nb.partials + ((int64_t)bh * p.n_units + unit) * kD + c0) = contrib;
         }
         st8(dst + quad * 4 + dt * 16, out);
-        if (half) st8(dst + quad * 4 + (dt + 1) * 16, cvt4(which ? acc2 : acc2 * kScale));      // (no fold on these jobs)
     }
 }
 
@@ -1447,31 +1466,18 @@ extern "C" int llsa_attn_bwd(const llsa_attn_bwd_args* a, void* stream) {
         }
     }
 
-    ReduceParams rp;
-    rp.n_jobs = 0;
-    rp.H = H;
-    rp.N = N;
+    PooledJobs pooled;
+    pooled.n_jobs = 0;
     PoolFold no_fold;
     for (int l = 0; l < LLSA_MAX_LEVELS; l++) no_fold.gk[l] = no_fold.gv[l] = nullptr;
     no_fold.freq = nullptr;
     no_fold.depth = 0;
-    auto add_job = [&](const KSideParams& p, int chunk, int max_units, int n_chunks) {
-        ReduceJob& j = rp.job[rp.n_jobs++];
-        j.part = p.part; j.half_part = 0; j.off = p.off; j.work = p.work; j.csr_shift = 0;
-        j.dk = p.dk; j.sdkb = p.sdkb; j.sdkh = p.sdkh; j.sdkn = p.sdkn;
-        j.dv = p.dv; j.sdvb = p.sdvb; j.sdvh = p.sdvh; j.sdvn = p.sdvn;
-        j.n_units = p.n_units; j.chunk = chunk; j.max_units = max_units;
-        j.work_stride = p.work_stride; j.slot_stride = p.slot_stride; j.n_chunks = n_chunks;
-        j.fold = p.fold;
-        j.norm = p.norm;
-    };
-    auto run_reduce = [&]() {
-        if (stages & LLSA_BWD_NO_REDUCE) rp.n_jobs = 0;       // (profiling: time the K-side kernels alone)
-        if (rp.n_jobs == 0) return;
-        int slots = 0;
-        for (int i = 0; i < rp.n_jobs; i++) slots += reduce_slots(rp.job[i].max_units);
-        hipLaunchKernelGGL(kside_reduce_kernel, dim3(slots * 2, BH), dim3(256), 0, s, rp);
-        rp.n_jobs = 0;
+    // the finished gradients of the pooled levels
+    auto reduce_pooled = [&]() {
+        if (pooled.n_jobs == 0 || (stages & LLSA_BWD_NO_REDUCE)) return;     // (profiling: time the K-side kernels alone)
+        int units = 0;
+        for (int i = 0; i < pooled.n_jobs; i++) units += pooled.job[i].n_units;
+        hipLaunchKernelGGL(pooled_reduce_kernel, dim3(units, BH), dim3(kReduceThreads), 0, s, pooled);
     };
     KSideParams base;
     base.qr = (const bf16*)a->qr; base.dor = dor;
@@ -1520,7 +1526,16 @@ extern "C" int llsa_attn_bwd(const llsa_attn_bwd_args* a, void* stream) {
         } else {
             hipLaunchKernelGGL(HIP_KERNEL_NAME(attn_kside_kernel<false>), grid, dim3(64), 0, s, p);
         }
-        add_job(p, chunk, N1 * a->T / chunk + 1, 0);
+        if (stages & LLSA_BWD_NO_REDUCE) return;
+        ReduceParams r;
+        r.part = p.part; r.work = p.work;
+        r.dk = p.dk; r.sdkb = p.sdkb; r.sdkh = p.sdkh; r.sdkn = p.sdkn;
+        r.dv = p.dv; r.sdvb = p.sdvb; r.sdvh = p.sdvh; r.sdvn = p.sdvn;
+        r.n_units = p.n_units; r.max_units = N1 * a->T / chunk + 1; r.H = H; r.N = N;
+        r.work_stride = p.work_stride; r.slot_stride = p.slot_stride;
+        r.fold = p.fold;
+        r.norm = p.norm;
+        hipLaunchKernelGGL(kside_reduce_kernel, dim3(2 * reduce_slots(r.max_units), BH), dim3(256), 0, s, r);
     };
     // pooled levels under an ancestor's selection, group-major (one launch for all of them, plus the dense level when it is small)
     auto run_groups = [&]() {
@@ -1544,15 +1559,10 @@ extern "C" int llsa_attn_bwd(const llsa_attn_bwd_args* a, void* stream) {
         hipLaunchKernelGGL(attn_kside_group_kernel, dim3(N2, BH), dim3(64 * kGroupWaves), 0, s, g);
         for (int l = 1; l < L; l++) {
             const GroupSeg& sgm = g.seg[l - 1];
-            const int64_t n = level_tokens(l);
-            ReduceJob& j = rp.job[rp.n_jobs++];
-            j.part = (const f32x4*)sgm.part; j.half_part = 1; j.off = a->lvl[l - 1].off; j.work = nullptr; j.csr_shift = sgm.owner_shift;
-            j.dk = (bf16*)a->lvl[l - 1].dk; j.sdkb = (int64_t)H * n * 64; j.sdkh = n * 64; j.sdkn = 64;
-            j.dv = (bf16*)a->lvl[l - 1].dv; j.sdvb = (int64_t)H * n * 64; j.sdvh = n * 64; j.sdvn = 64;
-            j.n_units = sgm.n_units; j.chunk = 1; j.max_units = sgm.n_units;
-            j.work_stride = 0; j.slot_stride = sgm.slots; j.n_chunks = 0;
-            j.fold = no_fold;
-            j.norm = llsa_norm_back{};
+            PooledJob& j = pooled.job[pooled.n_jobs++];
+            j.part = sgm.part; j.half_part = 1; j.off = a->lvl[l - 1].off; j.csr_shift = sgm.owner_shift; j.slot_stride = sgm.slots;
+            j.n_chunks = 0; j.n_units = sgm.n_units;
+            j.dk = (bf16*)a->lvl[l - 1].dk; j.dv = (bf16*)a->lvl[l - 1].dv;
         }
     };
     // dense coarsest level: every unit (16 pooled tokens) meets every query block; the query
@@ -1562,37 +1572,32 @@ extern "C" int llsa_attn_bwd(const llsa_attn_bwd_args* a, void* stream) {
         KSideParams p = base;
         const llsa_bwd_level& lv = a->lvl[L - 1];
         p.kk = (const bf16*)lv.kr; p.vv = (const bf16*)lv.vr;
-        p.dk = (bf16*)lv.dk; p.dv = (bf16*)lv.dv;
-        p.sdkb = p.sdvb = (int64_t)H * d.n_tok * 64; p.sdkh = p.sdvh = (int64_t)d.n_tok * 64;
         p.w = lv.gw;
-        p.sdkn = p.sdvn = 64;
         p.off = nullptr; p.flat = nullptr; p.flat_stride = 0; p.work = nullptr; p.work_stride = 0; p.slot_stride = 0;
         p.part = (f32x4*)(ws + wsp.part_dense);
         p.n_units = d.n_tok / 16; p.chunk_len = d.chunk_len;
-        if (d.merged) {                                       // the group-major pass has written one partial sum per group
-            add_job(p, 1, p.n_units, d.chunks);
-            rp.job[rp.n_jobs - 1].half_part = 1;
-            return;
-        }
+        PooledJob& j = pooled.job[pooled.n_jobs++];           // (merged: the group-major pass has written one bf16 partial sum per group)
+        j.part = p.part; j.half_part = d.merged; j.off = nullptr; j.csr_shift = 0; j.slot_stride = 0;
+        j.n_chunks = d.chunks; j.n_units = p.n_units;
+        j.dk = (bf16*)lv.dk; j.dv = (bf16*)lv.dv;
+        if (d.merged) return;
         const dim3 grid((p.n_units + d.wg_units - 1) / d.wg_units * d.chunks, BH);
         if (d.wg_units == 16) hipLaunchKernelGGL(HIP_KERNEL_NAME(attn_kside_dense_kernel<8, 2>), grid, dim3(512), 0, s, p);
         else if (d.wg_units == 8) hipLaunchKernelGGL(HIP_KERNEL_NAME(attn_kside_dense_kernel<4, 2>), grid, dim3(256), 0, s, p);
         else hipLaunchKernelGGL(HIP_KERNEL_NAME(attn_kside_dense_kernel<4, 1>), grid, dim3(256), 0, s, p);
-        add_job(p, 1, p.n_units, d.chunks);
     };
 
     if (fold) {
         // the fine pass adds the finished pooled gradients on its way out, so they come first
         run_groups();
         run_dense();
-        run_reduce();
+        reduce_pooled();
         run_fine();
-        run_reduce();
     } else {
         run_fine();
         run_groups();
         run_dense();
-        run_reduce();
+        reduce_pooled();
     }
     if (n_sums > 0) {
         // (rows of the first stage's results: at most as many as there are rows)
