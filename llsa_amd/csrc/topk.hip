@@ -11,6 +11,8 @@
 //
 // The order is total -- higher score first, equal scores by smaller key index -- so the result does not depend on how the
 // work is split.
+#include <numeric>
+#include <algorithm>
 #include "llsa_device.h"
 #include "llsa_host.h"
 #include "../../include/llsa_hip.h"
@@ -308,16 +310,21 @@ __global__ __launch_bounds__(64 * W) void topk_dense_kernel(const bf16* __restri
 }
 
 // Dense selection for longer rows: the keys stream by, and only those that can still be among a row's T best are kept.
-// A wave owns sixteen rows (PARTS = 1: four waves of a workgroup = 64 rows, which share the key tiles through LDS) or a
-// quarter of the keys of sixteen rows (PARTS = 4, for grids too small to fill the chip otherwise).  Every row has a buffer
+// A wave owns sixteen rows (PARTS = 1) or a quarter of the keys of sixteen rows (PARTS = 4, for grids too small to fill the chip
+// otherwise).  Every row has a buffer
 // of kBuf keys in LDS and a threshold; a tile whose scores all lie below their rows' thresholds costs a handful of
 // instructions, the others append what passes.  When a buffer is nearly full the wave cuts all sixteen back to little more
-// than their T best, which also raises the thresholds.  In a stream of random order about T ln(n / T) keys of a row pass.
+// than their T best, which also raises the thresholds.  In a stream of random order about T ln(n / T) keys of a row pass, in one
+// whose neighbours are alike more, so the tiles are taken in steps of 0.62 of the row of tiles.  What bounds the kernel is a wave's chain of
+// instructions and LDS round trips for the tiles that pass (a third of them at 4096 keys, T = 8) and three cuts; so the waves do not
+// wait for each other: key tiles shared through LDS cost a barrier per four tiles, at which three waves waited for the one with a
+// cut (37 % of the time).  8 x 4096 rows of 4096 keys 156 -> 137 us, 12 x 4096 290 -> 197, 16 x 2048 of 2048 110 -> 82; a quarter of
+// the keys per wave, 5 x 3072 77 -> 71.  (Four tiles on their way, places in the buffers by lane swaps instead of an LDS counter: the same.)
 // Key: the 32-bit packed key (scores rounded to bf16, n <= kMaxPackedKeys) or the 64-bit wide key.
 // (A T-step arg-max over chunks of 512 keys per row took 1480 us for 8 x 4096 rows of 4096 keys, T = 8.)
 constexpr int kBuf = 128, kBufFull = kBuf - 16;   // a tile adds at most 16 keys to a row
 constexpr int kStreamWaves = 4;
-constexpr int kStageKeys = 64;                    // keys per LDS buffer (one tile per wave)
+constexpr int kAhead = 2;                         // key tiles on their way to a wave while as many are worked on
 
 template <typename Key>
 struct StreamKey;
@@ -347,7 +354,7 @@ __device__ __forceinline__ float score_floor(unsigned k) {
 
 template <typename Key, int PARTS>
 __global__ __launch_bounds__(64 * kStreamWaves) void topk_stream_kernel(const bf16* __restrict__ pq, const bf16* __restrict__ pk,
-                                                                        int* __restrict__ out, int n, int T, int round_scores) {
+                                                                        int* __restrict__ out, int n, int T, int round_scores, int step) {
     constexpr int kE = kBuf / 4;                              // keys of a row's buffer per lane
     // a wave's buffers; at the end a row tile's winners take their place
     constexpr int kKeys = 16 * (kBuf + 1), kWide = 16 * kWinStride, kPer = sizeof(Key) == 8 ? kKeys : (kKeys + 1) / 2 > kWide ? (kKeys + 1) / 2 : kWide;
@@ -355,7 +362,6 @@ __global__ __launch_bounds__(64 * kStreamWaves) void topk_stream_kernel(const bf
     __shared__ int cnt[kStreamWaves][16];
     __shared__ int n_win[kStreamWaves / PARTS][16];
     __shared__ RowShare<PARTS> share;
-    __shared__ __align__(16) bf16 stage[PARTS == 1 ? 2 : 1][PARTS == 1 ? kStageKeys * kD : 8];
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), quad = lane >> 4, r = lane & 15;
     const int part = PARTS == 1 ? 0 : wave, rowt = PARTS == 1 ? wave : 0;
     const int bh = blockIdx.y, q0 = blockIdx.x * (PARTS == 1 ? 64 : 16) + rowt * 16;      // n is a multiple of 64 where PARTS == 1
@@ -431,53 +437,42 @@ __global__ __launch_bounds__(64 * kStreamWaves) void topk_stream_kernel(const bf
         if (__ballot(slot > kBufFull) != 0) cut();
     };
 
-    if (PARTS == 1) {
-        // key tiles through LDS, 64 keys per buffer, in the order the lanes read them (R tile: 16-byte unit
-        // chunk * 16 + row), so each is fetched once per workgroup; the next buffer's copy runs during this one's work
-        auto fetch = [&](int c) __attribute__((always_inline)) {
-            const bf16* src = pkb + ((int64_t)c * kStageKeys + wave * 16 + r) * kD + quad * 8;
-            copy16_global_to_lds(src, &stage[c & 1][wave * kTile]);
-            copy16_global_to_lds(src + 32, &stage[c & 1][wave * kTile + 512]);
-        };
-        const int n_chunks = n / kStageKeys;
-        fetch(0);
-        for (int c = 0; c < n_chunks; c++) {
-            wait_vm0();
-            __syncthreads();                                  // everybody's part has landed, and the other buffer is free
-            bf16x8 ka[4][2];
+    // key tiles straight into registers, kAhead on their way while as many are worked on
+    const int tiles = n / 16;
+    const bf16* p = pkb + r * kD + quad * 8;
+    int t_load = (int)((int64_t)part * step % tiles), t_work = t_load;
+    const int hop = (int)((int64_t)PARTS * step % tiles);
+    auto after = [&](int t) __attribute__((always_inline)) { return t + hop - (t + hop >= tiles ? tiles : 0); };
+    struct Tiles { bf16x8 k[kAhead][2]; } ta, tb;
+    auto load = [&](Tiles& o) __attribute__((always_inline)) {
 #pragma unroll
-            for (int a = 0; a < 4; a++) {
-                ka[a][0] = lds_ld16(&stage[c & 1][a * kTile + lane * 8]);
-                ka[a][1] = lds_ld16(&stage[c & 1][a * kTile + 512 + lane * 8]);
-            }
-            wait_all_mem();
-            if (c + 1 < n_chunks) fetch(c + 1);
-#pragma unroll 1
-            for (int a = 0; a < 4; a += 2) {
-                f32x4 z = {0.f, 0.f, 0.f, 0.f};
-                const bf16x8 k0 = a ? ka[2][0] : ka[0][0], k1 = a ? ka[2][1] : ka[0][1];
-                const bf16x8 k2 = a ? ka[3][0] : ka[1][0], k3 = a ? ka[3][1] : ka[1][1];
-                const f32x4 s0 = mfma_bf16(k1, bq[1], mfma_bf16(k0, bq[0], z)), s1 = mfma_bf16(k3, bq[1], mfma_bf16(k2, bq[0], z));
-                take(s0, c * kStageKeys + a * 16);
-                take(s1, c * kStageKeys + a * 16 + 16);
-            }
+        for (int i = 0; i < kAhead; i++) {
+            o.k[i][0] = ld16(p + (int64_t)t_load * 16 * kD);
+            o.k[i][1] = ld16(p + (int64_t)t_load * 16 * kD + 32);
+            t_load = after(t_load);
         }
-    } else {
-        const int tiles = n / 16, per = (tiles + PARTS - 1) / PARTS, lo = min(part * per, tiles), hi = min(lo + per, tiles);
-        const bf16* p = pkb + r * kD + quad * 8;
-        bf16x8 k0 = zero8(), k1 = zero8();
-        if (lo < hi) {
-            k0 = ld16(p + (int64_t)lo * 16 * kD);
-            k1 = ld16(p + (int64_t)lo * 16 * kD + 32);
-        }
-        for (int t = lo; t < hi; t++) {
-            const bf16* nx = p + (int64_t)min(t + 1, hi - 1) * 16 * kD;
-            const bf16x8 n0 = ld16(nx), n1 = ld16(nx + 32);
+    };
+    int left = (tiles - part + PARTS - 1) / PARTS;            // tiles this wave still has to look at
+    auto work = [&](const Tiles& o) __attribute__((always_inline)) {
+        f32x4 s[kAhead];
+#pragma unroll
+        for (int i = 0; i < kAhead; i++) {
             f32x4 z = {0.f, 0.f, 0.f, 0.f};
-            take(mfma_bf16(k1, bq[1], mfma_bf16(k0, bq[0], z)), t * 16);
-            k0 = n0;
-            k1 = n1;
+            s[i] = mfma_bf16(o.k[i][1], bq[1], mfma_bf16(o.k[i][0], bq[0], z));
         }
+#pragma unroll
+        for (int i = 0; i < kAhead; i++) {
+            if (i < left) take(s[i], t_work * 16);
+            t_work = after(t_work);
+        }
+        left -= kAhead;
+    };
+    load(ta);
+    while (left > 0) {
+        load(tb);
+        work(ta);
+        load(ta);
+        if (left > 0) work(tb);
     }
     cut();
     // at most T + kSpare keys are left in this wave's buffer of every row (all of its keys if it saw fewer)
@@ -695,10 +690,12 @@ extern "C" int llsa_topk_dense(const void* pq, const void* pk, int32_t* out_idx,
         const bool wide = !round_scores || n > kMaxPackedKeys;
         const bool whole = n % 64 == 0 && (int64_t)n / 16 * B * H >= 2048;
         const dim3 grid(whole ? n / 64 : n / 16, B * H), block(64 * kStreamWaves);
-        if (whole && !wide) hipLaunchKernelGGL(HIP_KERNEL_NAME(topk_stream_kernel<unsigned, 1>), grid, block, 0, st, q, k, out_idx, n, T, round_scores);
-        else if (whole) hipLaunchKernelGGL(HIP_KERNEL_NAME(topk_stream_kernel<unsigned long long, 1>), grid, block, 0, st, q, k, out_idx, n, T, round_scores);
-        else if (!wide) hipLaunchKernelGGL(HIP_KERNEL_NAME(topk_stream_kernel<unsigned, 4>), grid, block, 0, st, q, k, out_idx, n, T, round_scores);
-        else hipLaunchKernelGGL(HIP_KERNEL_NAME(topk_stream_kernel<unsigned long long, 4>), grid, block, 0, st, q, k, out_idx, n, T, round_scores);
+        int step = (int)(0.618 * (n / 16));                   // (without a common divisor, so that every tile has its turn)
+        while (std::gcd(step, n / 16) != 1) step++;
+        if (whole && !wide) hipLaunchKernelGGL(HIP_KERNEL_NAME(topk_stream_kernel<unsigned, 1>), grid, block, 0, st, q, k, out_idx, n, T, round_scores, step);
+        else if (whole) hipLaunchKernelGGL(HIP_KERNEL_NAME(topk_stream_kernel<unsigned long long, 1>), grid, block, 0, st, q, k, out_idx, n, T, round_scores, step);
+        else if (!wide) hipLaunchKernelGGL(HIP_KERNEL_NAME(topk_stream_kernel<unsigned, 4>), grid, block, 0, st, q, k, out_idx, n, T, round_scores, step);
+        else hipLaunchKernelGGL(HIP_KERNEL_NAME(topk_stream_kernel<unsigned long long, 4>), grid, block, 0, st, q, k, out_idx, n, T, round_scores, step);
     }
     return launch_status("topk_dense");
 }
