@@ -240,9 +240,9 @@ __global__ __launch_bounds__(256, Q == 1 ? 4 : 3) void attn_fwd_kernel(llsa_attn
         const bf16* vb = (const bf16*)a.lvl[sb.level].vt + sb.tile;
         bf16* dst = sh0 + ((grp & 1) * kGroup + wave) * (2 * kTile);
         copy16_global_to_lds(kb + lane * 8, dst);
-        copy16_global_to_lds(kb + 512 + lane * 8, dst + 512);
+        copy16_global_to_lds<512>(kb + lane * 8, dst);
         copy16_global_to_lds(vb + lane * 8, dst + kTile);
-        copy16_global_to_lds(vb + 512 + lane * 8, dst + kTile + 512);
+        copy16_global_to_lds<512>(vb + lane * 8, dst + kTile);
     };
     const int n_groups = sl.n_blocks / kGroup;                // every level's count is a multiple of kGroup (host checks)
     issue_group(0);
@@ -329,10 +329,11 @@ __global__ __launch_bounds__(256, Q == 1 ? 4 : 3) void attn_fwd_kernel(llsa_attn
 #pragma unroll
             for (int j = 0; j < 2; j++) {
                 const int64_t at = (int64_t)ml.block(min(2 * s + j, ml.n - 1)) * kTile;
-                dst.k[j][0] = ld16(kr + at + lane * 8);
-                dst.k[j][1] = ld16(kr + at + lane * 8 + 512);
-                copy16_global_to_lds(vr + at + unit, slot + j * kTile);
-                copy16_global_to_lds(vr + at + unit + 512, slot + j * kTile + 512);
+                const bf16 *kb = kr + at, *vb = vr + at;
+                dst.k[j][0] = ld16(kb + lane * 8);
+                dst.k[j][1] = ld16(kb + lane * 8 + 512);
+                copy16_global_to_lds(vb + unit, slot + j * kTile);
+                copy16_global_to_lds<512>(vb + unit, slot + j * kTile);
             }
         };
         auto work = [&](int s, KeyRegs<2>& cur, KeyRegs<2>& nxt) __attribute__((always_inline)) {

@@ -12,6 +12,7 @@ typedef __attribute__((ext_vector_type(4))) __bf16 bf16x4;
 typedef __attribute__((ext_vector_type(8))) __bf16 bf16x8;
 typedef __attribute__((ext_vector_type(2))) float f32x2;
 typedef __attribute__((ext_vector_type(4))) float f32x4;
+typedef __attribute__((ext_vector_type(4))) unsigned u32x4;
 typedef __attribute__((ext_vector_type(4))) int i32x4;
 
 constexpr int kWave = 64;        // CDNA wavefront
@@ -134,9 +135,11 @@ __device__ __forceinline__ bf16x4 lds_t_operand(const bf16* r_tile_in_lds, int d
 // lane l's 16 bytes land at lds_wave_base + 16*l, so a wave moves 1 KB that is contiguous in
 // LDS.  lds_wave_base must be the same in every lane.  The copy is tracked by the vector-memory
 // counter: wait_vm0() before the data (or a barrier that publishes it) is relied on.
+// OFF: elements, added on both sides by the instruction itself, where a second pair of addresses costs registers and vector adds.
+template <int OFF = 0>
 __device__ __forceinline__ void copy16_global_to_lds(const bf16* g_lane, bf16* lds_wave_base) {
     __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)g_lane,
-                                     (__attribute__((address_space(3))) void*)lds_wave_base, 16, 0, 0);
+                                     (__attribute__((address_space(3))) void*)lds_wave_base, 16, OFF * (int)sizeof(bf16), 0);
 }
 __device__ __forceinline__ void wait_vm0() { __builtin_amdgcn_s_waitcnt(0x0F70); }   // vmcnt(0), other counters untouched
 // vmcnt(0) and lgkmcnt(0).  The compiler books a copy into LDS against both counters; until it has seen

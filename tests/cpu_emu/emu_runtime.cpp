@@ -131,25 +131,6 @@ f32x4_t mfma_16x16x32_bf16(bf16x8_t a, bf16x8_t b, f32x4_t c) {
     return d;
 }
 
-// D = A(32x16) * B(16x32) + C.  Lane l holds A[row l%32][k = 8*(l/32) + e], B[k = 8*(l/32) + e][col l%32]
-// and D[row 8*(r/4) + 4*(l/32) + r%4][col l%32], r = 0..15.
-f32x16_t mfma_32x32x16_bf16(bf16x8_t a, bf16x8_t b, f32x16_t c) {
-    WaveSync& ws = waves[cur / kWave];
-    const int l = cur % kWave, col = l % 32;
-    ws.a[l] = a;
-    ws.b[l] = b;
-    wave_barrier();
-    f32x16_t d = c;
-    for (int r = 0; r < 16; r++) {
-        const int row = 8 * (r / 4) + 4 * (l / 32) + r % 4;
-        float s = 0.f;
-        for (int k = 0; k < 16; k++) s += (float)ws.a[row + 32 * (k / 8)][k % 8] * (float)ws.b[col + 32 * (k / 8)][k % 8];
-        d[r] += s;
-    }
-    wave_barrier();
-    return d;
-}
-
 // ds_read_b64_tr_b16: in each group of 16 lanes, lane i gets element i%4 of the 8-byte chunks
 // addressed by lanes i/4, 4 + i/4, 8 + i/4, 12 + i/4 (behaviour observed on gfx950 hardware).
 s16x4_t ds_read_tr16_b64(const void* p) {

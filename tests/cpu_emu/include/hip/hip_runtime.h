@@ -56,8 +56,6 @@ int lane_id();
 typedef __attribute__((ext_vector_type(8))) __bf16 bf16x8_t;
 typedef __attribute__((ext_vector_type(4))) float f32x4_t;
 f32x4_t mfma_16x16x32_bf16(bf16x8_t a, bf16x8_t b, f32x4_t c);
-typedef __attribute__((ext_vector_type(16))) float f32x16_t;
-f32x16_t mfma_32x32x16_bf16(bf16x8_t a, bf16x8_t b, f32x16_t c);
 typedef __attribute__((ext_vector_type(4))) short s16x4_t;
 s16x4_t ds_read_tr16_b64(const void* p);
 }  // namespace emu
@@ -120,7 +118,6 @@ inline int __ffs(int x) { return __builtin_ffs(x); }
 inline int __clz(int x) { return x ? __builtin_clz((unsigned)x) : 32; }
 
 #define __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, x, y, z) emu::mfma_16x16x32_bf16((a), (b), (c))
-#define __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, c, x, y, z) emu::mfma_32x32x16_bf16((a), (b), (c))
 #define __builtin_amdgcn_ds_read_tr16_b64_v4i16(p) emu::ds_read_tr16_b64((const void*)(p))
 #define __builtin_amdgcn_exp2f(x) exp2f(x)
 #define __builtin_amdgcn_logf(x) log2f(x)
@@ -130,7 +127,7 @@ inline int __clz(int x) { return x ? __builtin_clz((unsigned)x) : 32; }
 #define __builtin_amdgcn_sched_group_barrier(mask, n, id) ((void)0)
 #define __builtin_amdgcn_wave_barrier() emu::wave_sync()
 #define __builtin_amdgcn_global_load_lds(g, l, size, off, aux) \
-    __builtin_memcpy((char*)(l) + (size) * emu::lane_id(), (const char*)(g), (size))
+    __builtin_memcpy((char*)(l) + (off) + (size) * emu::lane_id(), (const char*)(g) + (off), (size))
 // the wave-wide effect of a wait (all lanes' copies into LDS have landed) needs a rendezvous of the lanes here
 #define __builtin_amdgcn_s_waitcnt(x) emu::wave_sync()
 #define __builtin_amdgcn_s_setprio(x) ((void)0)
