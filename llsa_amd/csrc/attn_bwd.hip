@@ -1448,9 +1448,7 @@ extern "C" int llsa_attn_bwd(const llsa_attn_bwd_args* a, void* stream) {
 
     const int stages = a->stages ? a->stages : (0x7fffffff & ~LLSA_BWD_NO_REDUCE);
     if (stages & LLSA_BWD_DQ) {
-        // (two query blocks per wave from 512 groups of eight on, see kPairMinGroups: 12 x 16384 tokens 69.4 against 72.4 us,
-        // 48 x 16384 268 against 310, 6 x 262144 963 against 1109; 24 x 4096 even, 15 x 7168 at topk 12 46.6 against 42.1)
-        const bool pairs = a->T <= kPairMaxTopk && N1 % 8 == 0 && (int64_t)N1 / 8 * BH >= kPairMinGroups;
+        const bool pairs = a->T <= kPairMaxTopk && N1 % 8 == 0 && pairs_fill((int64_t)N1 / 8 * BH);
         const dim3 grid(N1 / (pairs ? 8 : 4), BH);
 #define LLSA_DQ(Q, R)                                                                                                                  \
     do {                                                                                                                               \

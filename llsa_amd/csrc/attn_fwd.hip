@@ -405,14 +405,15 @@ static int attn_fwd(const llsa_attn_fwd_args* a, const llsa_transpose_job* jobs,
     const int N1 = a->N / 16, BH = a->B * a->H;
     // Two query blocks per wave halve the LDS reads of the pooled blocks and save a quarter of the fine fetches; one per wave
     // leaves more and shorter waves.  Two win where the pooled blocks are most of the walk (11 x 32768 tokens, topk 8,
-    // 128 pooled blocks: 227 against 267 us) and on large grids (48 x 16384: 228 against 271, 6 x 262144: 929 against 1057), one
-    // on smaller ones (15 x 7168, topk 12: 33.5 against 37.6; 8 x 16384, topk 8: 26.6 against 28.6; 24 x 4096 and 12 x 16384 at
-    // topk 16 are even, 3 x 49152 at topk 64 161 against 156).
+    // 128 pooled blocks: 227 against 267 us) and on large grids (16 x 16384, topk 16: 78.2 against 83.7; 48 x 16384: 228 against 271; 6 x
+    // 262144: 929 against 1057), one on smaller ones (12 x 16384: 58.5 against 64.6; 24 x 4096: 30.1 against 31.2; 3 x 49152 at topk 64
+    // even) and, as in the backward pass, where the last round would be mostly empty (see pairs_fill; 2 x 65536, topk 8:
+    // 45.0 against 48.0; 7 x 16384, topk 8, 64 pooled blocks: 50.6 against 54.3).
     int64_t shared = listed, coarsest = a->N / 256;
     for (int l = 1; l < a->levels; l++) coarsest /= 16;
     shared += coarsest;
     const int64_t groups = (int64_t)N1 / 8 * BH;
-    const bool pairs = a->T <= kPairMaxTopk && N1 % 8 == 0 && groups >= kPairMinGroups && (shared >= 4 * a->T || groups >= 2048);
+    const bool pairs = a->T <= kPairMaxTopk && N1 % 8 == 0 && pairs_fill(groups) && (shared >= 4 * a->T || groups >= 2048);
     TrJobs lists{};
     const int width = N1 / (pairs ? 8 : 4);                   // (a multiple of 8: N is one of 1024)
     const bool ride = jobs != nullptr && plan_transpose(jobs, n_jobs, a->B, a->H, kTrLdsFwd, lists);

@@ -336,10 +336,19 @@ __device__ __forceinline__ MergedLists<Q, R> merge_lists(const int* ip, int T, i
 }
 // Two query blocks per wave are possible up to this topk (their lists then fit two registers) ...
 constexpr int kPairMaxTopk = 64;
-// ... and considered from this many groups of eight query blocks on.  Below, the chip has room for all of the waves either way
-// (four workgroups of four single blocks or three of four pairs per CU), and a wave of one block has half the serial chain:
-// 6 x 1024 tokens, topk 8: forward 10.3 -> 6.2 us, dQ 11.0 -> 7.9; 6 x 8192, topk 16: 26.2 -> 20.9 and 31.3 -> 26.8.
-constexpr int kPairMinGroups = 512;
+// ... and considered where their workgroups (four waves, a group of eight query blocks) fill the chip.  It holds three of them per CU
+// (single query blocks: four of half the work), so a last round that is mostly empty costs a whole one: at most 30 % more places than
+// groups.  And below 5/6 of a round the chip has room for all of the waves either way, and a wave of one block has half the
+// serial chain.  dQ, one / two, us (topk 16 but for 7168 and 1024 tokens):
+//   groups 384 (6 x 8192) 26.8 / 31.3;  512 (16 x 4096) 24.4 / 26.5;  640 (20 x 4096) 30.6 / 32.2
+//   728 (13 x 7168, topk 12) 37.0 / 34.8;  768 (24 x 4096) 34.7 / 34.1;  784 (14 x 7168) 39.6 / 43.6;  840 (15 x 7168) 40.8 / 45.0
+//   1024 (8 x 8192) 51.1 / 51.8;  1152 (16 x 9216) 60.8 / 63.7;  1280 (20 x 8192) 64.2 / 60.7;  1536 (24 x 8192) 78.6 / 73.2
+//   1568 (28 x 7168) 69.6 / 72.8;  2048 (16 x 16384) 101.6 / 90.8;  3072 (24 x 16384) 144.4 / 134.4
+constexpr int kPairPlaces = 256 * 3;
+inline bool pairs_fill(int64_t groups) {
+    const int64_t places = (groups + kPairPlaces - 1) / kPairPlaces * kPairPlaces;
+    return groups > 640 && (places - groups) * 10 <= groups * 3;
+}
 
 // 16- and 8-byte reads that are LDS reads by construction (ds_read_b128 / ds_read_b64)
 __device__ __forceinline__ bf16x8 lds_ld16(const bf16* p) {

@@ -1,6 +1,5 @@
-"""The query-side kernels that give a wave two sibling query blocks (from 512 groups of eight query blocks on) at the edges of
-their topk ranges: one register of list entries per lane up to 32 entries a row, two up to 64; and the smallest grid that
-takes them against the largest that does not."""
+"""The query-side kernels around 512 groups of eight query blocks, the size of half a round of the chip, at the edges of the topk
+ranges that the list registers have: one register of entries per lane up to 32 entries a row, two up to 64."""
 import pytest
 import torch
 
