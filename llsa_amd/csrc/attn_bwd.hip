@@ -689,6 +689,88 @@ struct DenseOps {
     f32x4 l[2], d[2];              // statistics
 };
 
+// ... read out of LDS (tiles of the two query blocks, `stats` of the first, the second's behind them)
+__device__ __forceinline__ void dense_operands(DenseOps& o, const bf16* q0, const bf16* g0, const bf16* q1, const bf16* g1, const float* stats,
+                                               int lane) {
+    const int quad = lane >> 4;
+#pragma unroll
+    for (int u = 0; u < 2; u++) {
+        const bf16 *q = u ? q1 : q0, *g = u ? g1 : g0;
+        o.q[u][0] = lds_ld16(q + r_unit(lane));
+        o.q[u][1] = lds_ld16(q + 512 + r_unit(lane));
+        o.g[u][0] = lds_ld16(g + r_unit(lane));
+        o.g[u][1] = lds_ld16(g + 512 + r_unit(lane));
+        o.l[u] = *reinterpret_cast<const f32x4*>(stats + u * kStats + quad * 4);
+        o.d[u] = *reinterpret_cast<const f32x4*>(stats + u * kStats + kBlk + quad * 4);
+    }
+#pragma unroll
+    for (int u = 0; u < 2; u++)
+#pragma unroll
+        for (int dt = 0; dt < 4; dt++) {
+            o.tq[u][dt] = lds_t_operand(u ? q1 : q0, dt, lane);
+            o.tg[u][dt] = lds_t_operand(u ? g1 : g0, dt, lane);
+        }
+}
+// A round's products of UPW units (a weight is left out of the exponentials: it multiplies the sums at the end)
+template <int UPW>
+__device__ __forceinline__ void dense_products(f32x4 (*dk)[4], f32x4 (*dv)[4], const bf16x8 (*bk)[2], const bf16x8 (*bv)[2], const DenseOps& o) {
+    f32x4 sc[UPW][2], dp[UPW][2];
+    bf16x8 bp[UPW], bds[UPW];
+    auto scores = [&](int j) __attribute__((always_inline)) {
+#pragma unroll
+        for (int u = 0; u < 2; u++) {
+            const f32x4 z = {0.f, 0.f, 0.f, 0.f};
+            sc[j][u] = mfma_bf16(o.q[u][0], bk[j][0], z);
+            dp[j][u] = mfma_bf16(o.g[u][0], bv[j][0], o.d[u]);
+        }
+#pragma unroll
+        for (int u = 0; u < 2; u++) {
+            sc[j][u] = mfma_bf16(o.q[u][1], bk[j][1], sc[j][u]);
+            dp[j][u] = mfma_bf16(o.g[u][1], bv[j][1], dp[j][u]);
+        }
+    };
+    auto exponentials = [&](int j) __attribute__((always_inline)) {
+#pragma unroll
+        for (int u = 0; u < 2; u++)
+#pragma unroll
+            for (int e = 0; e < 4; e++) {
+                const float pe = exp2_fast(fmaf(sc[j][u][e], kScaleLog2e, o.l[u][e]));
+                bp[j][u * 4 + e] = (bf16)pe;
+                bds[j][u * 4 + e] = (bf16)(pe * dp[j][u][e]);
+            }
+    };
+    auto sums = [&](int j) __attribute__((always_inline)) {
+#pragma unroll
+        for (int dt = 0; dt < 4; dt++) {
+            dv[j][dt] = mfma_bf16(cat(o.tg[0][dt], o.tg[1][dt]), bp[j], dv[j][dt]);
+            dk[j][dt] = mfma_bf16(cat(o.tq[0][dt], o.tq[1][dt]), bds[j], dk[j][dt]);
+        }
+    };
+    // the vector instructions of one unit between the products of the other, in this order
+    auto interleave = [&]() __attribute__((always_inline)) {
+#pragma unroll
+        for (int i = 0; i < 8; i++) {
+            __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);      // one MFMA
+            __builtin_amdgcn_sched_group_barrier(0x002, 4, 0);      // four vector ALU instructions (and the exponentials among them)
+        }
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    scores(0);
+    if constexpr (UPW == 2) {
+        __builtin_amdgcn_sched_barrier(0);
+        scores(1);
+        exponentials(0);
+        interleave();
+        sums(0);
+        exponentials(1);
+        interleave();
+        sums(1);
+    } else {
+        exponentials(0);
+        sums(0);
+    }
+}
+
 template <int WAVES, int UPW>
 __global__ __launch_bounds__(64 * WAVES, UPW == 2 ? 2 : 3) void attn_kside_dense_kernel(KSideParams p) {
     static_assert(WAVES == 4 || WAVES == 8, "a wave moves one or two of the eight half tiles of a pair");
@@ -696,7 +778,6 @@ __global__ __launch_bounds__(64 * WAVES, UPW == 2 ? 2 : 3) void attn_kside_dense
     __shared__ __align__(16) float sh_stats[2][64];           // per pair: the statistics of its two query blocks
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int quad = lane >> 4;
     const int N1 = p.N / kBlk;
     // Workgroups that stream the same piece of the query range (one per group of units) get neighbouring logical ids,
     // which xcd_logical_id keeps on one XCD: the piece then comes out of that XCD's L2 for all but the first of them.
@@ -761,88 +842,17 @@ __global__ __launch_bounds__(64 * WAVES, UPW == 2 ? 2 : 3) void attn_kside_dense
         }
 
     DenseOps o;
-    f32x4 sc[UPW][2], dp[UPW][2];
-    bf16x8 bp[UPW], bds[UPW];
     // First half of a round: this wave's operands out of LDS, its share of the next pair into the other buffer, the request for
     // the pair after the next but one.
     auto gather = [&](int t, Stage& nxt) __attribute__((always_inline)) {
         const bf16* b = &sh[t & 1][0];
-#pragma unroll
-        for (int u = 0; u < 2; u++) {
-            const bf16* q = b + (2 * u) * kTile;
-            const bf16* g = b + (2 * u + 1) * kTile;
-            o.q[u][0] = lds_ld16(q + r_unit(lane));
-            o.q[u][1] = lds_ld16(q + 512 + r_unit(lane));
-            o.g[u][0] = lds_ld16(g + r_unit(lane));
-            o.g[u][1] = lds_ld16(g + 512 + r_unit(lane));
-            o.l[u] = *reinterpret_cast<const f32x4*>(&sh_stats[t & 1][u * kStats + quad * 4]);
-            o.d[u] = *reinterpret_cast<const f32x4*>(&sh_stats[t & 1][u * kStats + kBlk + quad * 4]);
-        }
-#pragma unroll
-        for (int u = 0; u < 2; u++)
-#pragma unroll
-            for (int dt = 0; dt < 4; dt++) {
-                o.tq[u][dt] = lds_t_operand(b + (2 * u) * kTile, dt, lane);
-                o.tg[u][dt] = lds_t_operand(b + (2 * u + 1) * kTile, dt, lane);
-            }
+        dense_operands(o, b, b + kTile, b + 2 * kTile, b + 3 * kTile, sh_stats[t & 1], lane);
         deposit(t + 1, nxt);
         request(t + 3, nxt);
     };
-    auto scores = [&](int j) __attribute__((always_inline)) {
-#pragma unroll
-        for (int u = 0; u < 2; u++) {
-            const f32x4 z = {0.f, 0.f, 0.f, 0.f};
-            sc[j][u] = mfma_bf16(o.q[u][0], bk[j][0], z);
-            dp[j][u] = mfma_bf16(o.g[u][0], bv[j][0], o.d[u]);
-        }
-#pragma unroll
-        for (int u = 0; u < 2; u++) {
-            sc[j][u] = mfma_bf16(o.q[u][1], bk[j][1], sc[j][u]);
-            dp[j][u] = mfma_bf16(o.g[u][1], bv[j][1], dp[j][u]);
-        }
-    };
-    auto exponentials = [&](int j) __attribute__((always_inline)) {
-#pragma unroll
-        for (int u = 0; u < 2; u++)
-#pragma unroll
-            for (int e = 0; e < 4; e++) {
-                const float pe = exp2_fast(fmaf(sc[j][u][e], kScaleLog2e, o.l[u][e]));
-                bp[j][u * 4 + e] = (bf16)pe;
-                bds[j][u * 4 + e] = (bf16)(pe * dp[j][u][e]);
-            }
-    };
-    auto sums = [&](int j) __attribute__((always_inline)) {
-#pragma unroll
-        for (int dt = 0; dt < 4; dt++) {
-            dv[j][dt] = mfma_bf16(cat(o.tg[0][dt], o.tg[1][dt]), bp[j], dv[j][dt]);
-            dk[j][dt] = mfma_bf16(cat(o.tq[0][dt], o.tq[1][dt]), bds[j], dk[j][dt]);
-        }
-    };
-    // the vector instructions of one unit between the products of the other, in this order
-    auto interleave = [&]() __attribute__((always_inline)) {
-#pragma unroll
-        for (int i = 0; i < 8; i++) {
-            __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);      // one MFMA
-            __builtin_amdgcn_sched_group_barrier(0x002, 4, 0);      // four vector ALU instructions (and the exponentials among them)
-        }
-        __builtin_amdgcn_sched_barrier(0);
-    };
     auto multiply = [&]() __attribute__((always_inline)) {
         __builtin_amdgcn_sched_barrier(0);
-        scores(0);
-        __builtin_amdgcn_sched_barrier(0);
-        if constexpr (UPW == 2) {
-            scores(1);
-            exponentials(0);
-            interleave();
-            sums(0);
-            exponentials(1);
-            interleave();
-            sums(1);
-        } else {
-            exponentials(0);
-            sums(0);
-        }
+        dense_products<UPW>(dk, dv, bk, bv, o);
         __builtin_amdgcn_sched_barrier(0);
     };
     if constexpr (WAVES == 8) {
@@ -901,6 +911,12 @@ __global__ __launch_bounds__(64 * WAVES, UPW == 2 ? 2 : 3) void attn_kside_dense
 // selected it, T2 times in all.
 // With few tokens on the dense coarsest level its blocks are appended to the lists (every group
 // meets all of them), which saves that level a pass of its own over Q and dO.
+// What bounds it is the instruction stream, as in the dense pass, and the waits at both ends of a wave's pass over the queries: two
+// workgroups a CU (64 KB of tiles each) fill them for one another.  The vector instructions of one key block stand between the
+// products of the other, the statistics lie in LDS beside the tiles, and a pass's key blocks are requested before the sums of the pass before
+// it are rounded and stored: 163 -> 148 us at 48 x 16384 tokens (20 blocks a group), 255 -> 225 at 6 x 262144 (16), 490 -> 441 with 36 blocks;
+// 45 at 12 x 16384 either way (768 workgroups, 512 places).  (Tried: one workgroup of eight waves per CU that stays, the next
+// group's tiles copied into a second buffer meanwhile and the halves taking turns as in the dense pass: 186, 254, 588.)
 // ---------------------------------------------------------------------------------------
 constexpr int kGroupWaves = 4;
 constexpr int kGroupSegs = LLSA_MAX_LEVELS;
@@ -930,13 +946,11 @@ struct GroupParams {
     GroupSeg seg[kGroupSegs];
 };
 
-struct GroupStats { f32x4 l[2], d[2]; };
-
-// UPW key blocks against the group's 16 query blocks, two query blocks per step, operands out of LDS.
-template <int UPW>
-__device__ __forceinline__ void group_pass(const bf16x8 (&bk)[2][2], const bf16x8 (&bv)[2][2], const float (&w)[2], bf16x8* const (&dst)[2],
-                                           const bf16* shq, const bf16* shg, const float* stb, int lane) {
-    const int quad = lane >> 4;
+// UPW key blocks against the group's 16 query blocks, two query blocks per step, operands out of LDS.  `next` starts the loads of the
+// wave's next key blocks, into bk and bv, where these are no longer needed: they arrive while the sums are rounded and stored.
+template <int UPW, typename NEXT>
+__device__ __forceinline__ void group_pass(const bf16x8 (&bk)[2][2], const bf16x8 (&bv)[2][2], const float (&weights)[2], bf16x8* const (&slots)[2],
+                                           const bf16* shq, const bf16* shg, const float* sh_stats, int lane, NEXT&& next) {
     f32x4 dk[UPW][4], dv[UPW][4];
 #pragma unroll
     for (int j = 0; j < UPW; j++)
@@ -945,63 +959,21 @@ __device__ __forceinline__ void group_pass(const bf16x8 (&bk)[2][2], const bf16x
             dk[j][dt] = f32x4{0.f, 0.f, 0.f, 0.f};
             dv[j][dt] = f32x4{0.f, 0.f, 0.f, 0.f};
         }
-    auto load_stats = [=](int t, GroupStats& st) __attribute__((always_inline)) {
-#pragma unroll
-        for (int u = 0; u < 2; u++) {
-            st.l[u] = *reinterpret_cast<const f32x4*>(stb + (2 * t + u) * kStats + quad * 4);
-            st.d[u] = *reinterpret_cast<const f32x4*>(stb + (2 * t + u) * kStats + kBlk + quad * 4);
-        }
-    };
-    auto step = [&](int t, const GroupStats& cur) __attribute__((always_inline)) {
-        bf16x8 aq[2][2], ag[2][2];
-        bf16x4 tq[2][4], tg[2][4];
-#pragma unroll
-        for (int u = 0; u < 2; u++) {
-            const bf16* q = shq + (2 * t + u) * kTile;
-            const bf16* g = shg + (2 * t + u) * kTile;
-            aq[u][0] = lds_ld16(q + r_unit(lane));
-            aq[u][1] = lds_ld16(q + 512 + r_unit(lane));
-            ag[u][0] = lds_ld16(g + r_unit(lane));
-            ag[u][1] = lds_ld16(g + 512 + r_unit(lane));
-#pragma unroll
-            for (int dt = 0; dt < 4; dt++) {
-                tq[u][dt] = lds_t_operand(q, dt, lane);
-                tg[u][dt] = lds_t_operand(g, dt, lane);
-            }
-        }
-#pragma unroll
-        for (int j = 0; j < UPW; j++) {
-            bf16x8 bp, bds;
-#pragma unroll
-            for (int u = 0; u < 2; u++) {
-                f32x4 sc = {0.f, 0.f, 0.f, 0.f}, dp = cur.d[u];
-                sc = mfma_bf16(aq[u][0], bk[j][0], sc);
-                sc = mfma_bf16(aq[u][1], bk[j][1], sc);
-                dp = mfma_bf16(ag[u][0], bv[j][0], dp);
-                dp = mfma_bf16(ag[u][1], bv[j][1], dp);
-#pragma unroll
-                for (int e = 0; e < 4; e++) {
-                    const float pe = exp2_fast(fmaf(sc[e], kScaleLog2e, cur.l[u][e]));   // (the weight multiplies the sums below)
-                    bp[u * 4 + e] = (bf16)pe;
-                    bds[u * 4 + e] = (bf16)(pe * dp[e]);
-                }
-            }
-#pragma unroll
-            for (int dt = 0; dt < 4; dt++) {
-                dv[j][dt] = mfma_bf16(cat(tg[0][dt], tg[1][dt]), bp, dv[j][dt]);
-                dk[j][dt] = mfma_bf16(cat(tq[0][dt], tq[1][dt]), bds, dk[j][dt]);
-            }
-        }
-    };
-    GroupStats sa, sb;
-    load_stats(0, sa);
 #pragma unroll 1
-    for (int t = 0; t < kBlk / 2; t += 2) {
-        load_stats(t + 1, sb);
-        step(t, sa);
-        load_stats((t + 2) & (kBlk / 2 - 1), sa);             // (the last one re-reads step 0: no branch around loads)
-        step(t + 1, sb);
+    for (int t = 0; t < kBlk / 2; t++) {
+        DenseOps o;
+        dense_operands(o, shq + 2 * t * kTile, shg + 2 * t * kTile, shq + (2 * t + 1) * kTile, shg + (2 * t + 1) * kTile,
+                       sh_stats + 2 * t * kStats, lane);
+        dense_products<UPW>(dk, dv, bk, bv, o);
     }
+    float w[UPW];
+    bf16x8* dst[UPW];
+#pragma unroll
+    for (int j = 0; j < UPW; j++) {
+        w[j] = weights[j];
+        dst[j] = slots[j];
+    }
+    next();
     // The partial sums of this pass leave as bf16 (see GroupSeg::part): the sum over the group's 256 queries was
     // taken in fp32, and the result the reduction makes of them is a bf16 tensor.
 #pragma unroll
@@ -1015,6 +987,7 @@ __device__ __forceinline__ void group_pass(const bf16x8 (&bk)[2][2], const bf16x
 
 __global__ __launch_bounds__(64 * kGroupWaves, 2) void attn_kside_group_kernel(GroupParams p) {
     __shared__ __align__(16) bf16 sh[2][kBlk * kTile];        // R tiles of the group's 16 query blocks: Q, then dO
+    __shared__ __align__(16) float sh_stats[kBlk * kStats];   // their statistics
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int N1 = p.N / kBlk;
@@ -1032,6 +1005,8 @@ __global__ __launch_bounds__(64 * kGroupWaves, 2) void attn_kside_group_kernel(G
             copy16_global_to_lds(qsrc + piece * 512 + r_unit(lane), &sh[0][piece * 512]);
             copy16_global_to_lds(gsrc + piece * 512 + r_unit(lane), &sh[1][piece * 512]);
         }
+        const float* ssrc = p.stats + ((int64_t)bh * N1 + (int64_t)G * kBlk) * kStats;
+        if (wave < 2) copy16_global_to_lds(reinterpret_cast<const bf16*>(ssrc + wave * 256 + lane * 4), reinterpret_cast<bf16*>(sh_stats + wave * 256));
     }
     // Key block j of the group's lists lives in lane j: which tile, which weight, where its partial sum goes.
     int my_unit = 0, my_seg = 0;
@@ -1057,7 +1032,6 @@ __global__ __launch_bounds__(64 * kGroupWaves, 2) void attn_kside_group_kernel(G
             }
         }
     }
-    const float* stb = p.stats + ((int64_t)bh * N1 + (int64_t)G * kBlk) * kStats;
     // this wave's key blocks: a contiguous share, taken two at a time (the last alone if the share is odd)
     const int per = (p.n_blocks + kGroupWaves - 1) / kGroupWaves;
     const int lo = min(wave * per, p.n_blocks), hi = min(lo + per, p.n_blocks);
@@ -1084,13 +1058,12 @@ __global__ __launch_bounds__(64 * kGroupWaves, 2) void attn_kside_group_kernel(G
     wait_vm0();
     __syncthreads();                                          // the copies into LDS are everybody's
     for (int j = lo; j < hi; j += 2) {
-        const bool two = j + 1 < hi;
-        if (j != lo) {
-            fetch(j, 0);
-            if (two) fetch(j + 1, 1);
-        }
-        if (two) group_pass<2>(bk, bv, w, dst, &sh[0][0], &sh[1][0], stb, lane);
-        else group_pass<1>(bk, bv, w, dst, &sh[0][0], &sh[1][0], stb, lane);
+        auto next = [&]() __attribute__((always_inline)) {
+            if (j + 2 < hi) fetch(j + 2, 0);
+            if (j + 3 < hi) fetch(j + 3, 1);
+        };
+        if (j + 1 < hi) group_pass<2>(bk, bv, w, dst, &sh[0][0], &sh[1][0], sh_stats, lane, next);
+        else group_pass<1>(bk, bv, w, dst, &sh[0][0], &sh[1][0], sh_stats, lane, next);
     }
 }
 
