@@ -771,8 +771,15 @@ __device__ __forceinline__ void dense_products(f32x4 (*dk)[4], f32x4 (*dv)[4], c
     }
 }
 
-template <int WAVES, int UPW>
-__global__ __launch_bounds__(64 * WAVES, UPW == 2 ? 2 : 3) void attn_kside_dense_kernel(KSideParams p) {
+// With LISTS the units are those of a selection (level 2 of llsa_l3 and above): piece i of the query range belongs to owner i >> chunk_shift,
+// the common ancestor of its query blocks, whose list names the units; the partial sum of an entry and a piece is left where the
+// transposed selection puts the entry, 1 << chunk_shift of them side by side.
+struct KSideLists {
+    const int* sel; const int* inv;               // (BH, owners, cnt)
+    int cnt, chunk_shift;
+};
+template <int WAVES, int UPW, bool LISTS>
+__global__ __launch_bounds__(64 * WAVES, UPW == 2 ? 2 : 3) void attn_kside_dense_kernel(KSideParams p, KSideLists ls) {
     static_assert(WAVES == 4 || WAVES == 8, "a wave moves one or two of the eight half tiles of a pair");
     __shared__ __align__(16) bf16 sh[2][4 * kTile];           // per pair: Q0, dO0, Q1, dO1 as R tiles
     __shared__ __align__(16) float sh_stats[2][64];           // per pair: the statistics of its two query blocks
@@ -781,12 +788,14 @@ __global__ __launch_bounds__(64 * WAVES, UPW == 2 ? 2 : 3) void attn_kside_dense
     const int N1 = p.N / kBlk;
     // Workgroups that stream the same piece of the query range (one per group of units) get neighbouring logical ids,
     // which xcd_logical_id keeps on one XCD: the piece then comes out of that XCD's L2 for all but the first of them.
-    const int unit_groups = (p.n_units + WAVES * UPW - 1) / (WAVES * UPW);
-    const int lid = xcd_logical_id();                          // grid: (unit_groups * chunks, BH)
+    const int n_met = LISTS ? ls.cnt : p.n_units;              // units that meet a piece
+    const int unit_groups = (n_met + WAVES * UPW - 1) / (WAVES * UPW);
+    const int lid = xcd_logical_id();                          // grid: (unit_groups * pieces, BH)
     const int piece = (lid % (int)gridDim.x) / unit_groups;
     const int bh = lid / (int)gridDim.x;
     const int unit0 = (((lid % (int)gridDim.x) % unit_groups) * WAVES + wave) * UPW;
-    const bool active = unit0 < p.n_units;                    // (n_units is a multiple of UPW; a wave past the end only moves tiles)
+    const bool active = unit0 < n_met;                        // (n_met is a multiple of UPW; a wave past the end only moves tiles)
+    const int64_t entry0 = LISTS ? ((int64_t)bh * (((int)gridDim.x / unit_groups) >> ls.chunk_shift) + (piece >> ls.chunk_shift)) * ls.cnt : 0;
     const int start = piece * p.chunk_len;
     const int n_pairs = min(p.chunk_len, N1 - start) / 2;     // even: chunk_len and N1 are multiples of 4
     if (n_pairs <= 0) return;                                 // uniform over the workgroup
@@ -822,7 +831,8 @@ __global__ __launch_bounds__(64 * WAVES, UPW == 2 ? 2 : 3) void attn_kside_dense
     bf16x8 bk[UPW][2], bv[UPW][2];
 #pragma unroll
     for (int j = 0; j < UPW; j++) {
-        const int unit = min(unit0 + j, p.n_units - 1);
+        int unit = min(unit0 + j, n_met - 1);
+        if (LISTS) unit = clampi(ls.sel[entry0 + unit], 0, p.n_units - 1);
         const bf16* kp = p.kk + ((int64_t)bh * p.n_units + unit) * kTile + lane * 8;
         const bf16* vp = p.vv + ((int64_t)bh * p.n_units + unit) * kTile + lane * 8;
         bk[j][0] = ld16(kp);
@@ -887,7 +897,12 @@ __global__ __launch_bounds__(64 * WAVES, UPW == 2 ? 2 : 3) void attn_kside_dense
     if (!active) return;
 #pragma unroll
     for (int j = 0; j < UPW; j++) {
-        f32x4* ps = part_slot(p.part, ((int64_t)piece * gridDim.y + bh) * p.n_units + unit0 + j);
+        int64_t slot = ((int64_t)piece * gridDim.y + bh) * p.n_units + unit0 + j;
+        if (LISTS) {
+            const int pos = clampi(ls.inv[entry0 + unit0 + j], 0, (int)(p.slot_stride >> ls.chunk_shift) - 1);
+            slot = (int64_t)bh * p.slot_stride + ((int64_t)pos << ls.chunk_shift) + (piece & ((1 << ls.chunk_shift) - 1));
+        }
+        f32x4* ps = part_slot(p.part, slot);
 #pragma unroll
         for (int dt = 0; dt < 4; dt++) {
             ps[dt * kWave + lane] = dk[j][dt] * p.w;         // (the weight, left out of the exponentials)
@@ -1315,6 +1330,21 @@ static DensePlan dense_plan(int B, int H, int N, int levels) {
     return d;
 }
 
+// A pooled level whose lists belong to `owners` ancestors of `range` query blocks each (a power of 16): into how many pieces, as a power of
+// two, the list form of the dense kernel cuts every owner's range, or -1 for the group-major pass.  The list form leaves one partial
+// sum per piece, in fp32, where the other leaves one per 16 query blocks, in bf16; but its workgroup is sixteen entries and a whole CU: it is taken
+// for full workgroups, three rounds of the chip and pieces of 128 query blocks or more.  Both passes and the reduction, us, group-major / list
+// (llsa_l3 at 262144 tokens): 6 heads, T3 = 16: 724 / 682; 12 heads: 1374 / 1273; but 2 heads (512 workgroups) 284 / 291, 3 heads with T3 = 12
+// 294 / 318, one head with T3 = 20 170 / 186.
+static int list_chunk_shift(int BH, int owners, int range, int T) {
+    constexpr int kMinWorkgroups = 3 * 256, kMinPiece = 128;
+    if (range < kMinPiece || T % 16 != 0) return -1;
+    const int64_t lists = (int64_t)BH * owners * (T / 16);
+    int shift = 0;
+    while ((lists << shift) < kMinWorkgroups && (range >> shift) > kMinPiece) shift++;
+    return (lists << shift) >= kMinWorkgroups ? shift : -1;
+}
+
 static int64_t align256(int64_t x) { return (x + 255) & ~(int64_t)255; }
 constexpr int64_t kSlotBytes = 8 * kWave * sizeof(f32x4);     // one partial: 16 rows x 64 ch x (dK, dV) fp32
 
@@ -1525,18 +1555,28 @@ extern "C" int llsa_attn_bwd(const llsa_attn_bwd_args* a, void* stream) {
         };
         for (int l = 1; l < L; l++) {                         // level l: blocks N / 16^(l+1), one list per 16^(l-1) groups
             const llsa_bwd_level& lv = a->lvl[l - 1];
-            add_seg(lv.kr, lv.vr, lv.sel, lv.inv, wsp.part_level[l - 1], level_tokens(l + 1), 4 * (l - 1), lv.T, wsp.slots_level[l - 1], lv.gw);
+            PooledJob& j = pooled.job[pooled.n_jobs++];
+            j.part = ws + wsp.part_level[l - 1]; j.off = lv.off; j.n_chunks = 0; j.n_units = level_tokens(l + 1);
+            j.dk = (bf16*)lv.dk; j.dv = (bf16*)lv.dv;
+            const int owners = N2 >> (4 * (l - 1)), shift = list_chunk_shift(BH, owners, N1 / owners, lv.T);
+            j.half_part = shift < 0;
+            j.csr_shift = shift < 0 ? 4 * (l - 1) : shift;
+            j.slot_stride = shift < 0 ? wsp.slots_level[l - 1] : (int64_t)owners * lv.T << shift;
+            if (shift < 0) {
+                add_seg(lv.kr, lv.vr, lv.sel, lv.inv, wsp.part_level[l - 1], j.n_units, j.csr_shift, lv.T, j.slot_stride, lv.gw);
+                continue;
+            }
+            KSideParams p = base;
+            p.kk = (const bf16*)lv.kr; p.vv = (const bf16*)lv.vr; p.w = lv.gw;
+            p.off = nullptr; p.flat = nullptr; p.flat_stride = 0; p.work = nullptr; p.work_stride = 0; p.slot_stride = j.slot_stride;
+            p.part = (f32x4*)(ws + wsp.part_level[l - 1]); p.n_units = j.n_units; p.chunk_len = (N1 / owners) >> shift;
+            const dim3 grid(lv.T / 16 * (owners << shift), BH);
+            hipLaunchKernelGGL(HIP_KERNEL_NAME(attn_kside_dense_kernel<8, 2, true>), grid, dim3(512), 0, s, p,
+                               KSideLists{lv.sel, lv.inv, lv.T, shift});
         }
         if (d.merged && (stages & LLSA_BWD_DENSE))
             add_seg(a->lvl[L - 1].kr, a->lvl[L - 1].vr, nullptr, nullptr, wsp.part_dense, d.n_tok / 16, 0, d.n_tok / 16, 0, a->lvl[L - 1].gw);
         hipLaunchKernelGGL(attn_kside_group_kernel, dim3(N2, BH), dim3(64 * kGroupWaves), 0, s, g);
-        for (int l = 1; l < L; l++) {
-            const GroupSeg& sgm = g.seg[l - 1];
-            PooledJob& j = pooled.job[pooled.n_jobs++];
-            j.part = sgm.part; j.half_part = 1; j.off = a->lvl[l - 1].off; j.csr_shift = sgm.owner_shift; j.slot_stride = sgm.slots;
-            j.n_chunks = 0; j.n_units = sgm.n_units;
-            j.dk = (bf16*)a->lvl[l - 1].dk; j.dv = (bf16*)a->lvl[l - 1].dv;
-        }
     };
     // dense coarsest level: every unit (16 pooled tokens) meets every query block; the query
     // range is cut into d.chunks pieces whose partial sums are added afterwards
@@ -1555,9 +1595,10 @@ extern "C" int llsa_attn_bwd(const llsa_attn_bwd_args* a, void* stream) {
         j.dk = (bf16*)lv.dk; j.dv = (bf16*)lv.dv;
         if (d.merged) return;
         const dim3 grid((p.n_units + d.wg_units - 1) / d.wg_units * d.chunks, BH);
-        if (d.wg_units == 16) hipLaunchKernelGGL(HIP_KERNEL_NAME(attn_kside_dense_kernel<8, 2>), grid, dim3(512), 0, s, p);
-        else if (d.wg_units == 8) hipLaunchKernelGGL(HIP_KERNEL_NAME(attn_kside_dense_kernel<4, 2>), grid, dim3(256), 0, s, p);
-        else hipLaunchKernelGGL(HIP_KERNEL_NAME(attn_kside_dense_kernel<4, 1>), grid, dim3(256), 0, s, p);
+        const KSideLists none{nullptr, nullptr, 0, 0};
+        if (d.wg_units == 16) hipLaunchKernelGGL(HIP_KERNEL_NAME(attn_kside_dense_kernel<8, 2, false>), grid, dim3(512), 0, s, p, none);
+        else if (d.wg_units == 8) hipLaunchKernelGGL(HIP_KERNEL_NAME(attn_kside_dense_kernel<4, 2, false>), grid, dim3(256), 0, s, p, none);
+        else hipLaunchKernelGGL(HIP_KERNEL_NAME(attn_kside_dense_kernel<4, 1, false>), grid, dim3(256), 0, s, p, none);
     };
 
     if (fold) {
