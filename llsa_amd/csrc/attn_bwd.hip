@@ -354,7 +354,8 @@ __global__ __launch_bounds__(256, Q == 1 ? 4 : 3) void attn_dq_kernel(llsa_attn_
 // block, or 16 tokens of the dense coarsest level).  Three kernels: attn_kside_kernel walks the
 // transposed selection of the fine blocks (unit-major: a unit and the list of query blocks that
 // selected it), attn_kside_group_kernel the pooled levels under an ancestor's selection
-// (query-group-major), attn_kside_dense_kernel the dense coarsest level.
+// (query-group-major), attn_kside_dense_kernel the dense coarsest level and, on large grids, the lists that
+// sixteen groups or more share (llsa_l3 and above).
 // ---------------------------------------------------------------------------------------
 
 // Optional last step of the fine dK / dV: add the pooled gradients the token's block received
@@ -919,7 +920,7 @@ __global__ __launch_bounds__(64 * WAVES, UPW == 2 ? 2 : 3) void attn_kside_dense
 // dO tiles into LDS once (64 KB) and meets every key block of the group's lists there; a wave
 // takes its share of the key blocks, two at a time, and ends each with that block's dK / dV summed
 // over the group's 256 queries.  A key block selected by several ancestors receives one such
-// partial sum per selecting group, written where kside_reduce_kernel finds the partial sums of a
+// partial sum per selecting group, written where pooled_reduce_kernel finds the partial sums of a
 // key block side by side: at the position the transposed selection gives the (ancestor, entry)
 // pair.  Walking the transposed lists instead (key block major, the reference's order,
 // sparse_attention_res_2.py:492-575) fetches the 64 KB of a group once per key block that

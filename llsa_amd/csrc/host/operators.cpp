@@ -3,8 +3,8 @@
 //
 //     forward   pool_pyramid_fwd (q, k, v: pooled rows, RoPE, operand tiles) [+ deeper levels]
 //               topk_dense / topk_cascade [+ topk_sparse ...]
-//               attn_fwd
-//               transpose_indices_multi  (second stream beside the attention kernel at the long sequences)
+//               attn_fwd_lists  (the attention kernel, the transposed selections in the same launch), or at the long sequences
+//               attn_fwd and, on a second stream beside it, transpose_indices_multi
 //     backward  attn_bwd with fold_pooled = 1  (dq, dk, dv complete, rotated back and back through the qk-norm)
 //
 // Native because at the short sequences a step is bound by its host side: at B=1, H=6, N=1024 the kernels of a forward

@@ -52,8 +52,8 @@ with open(f'{out}/step_kernels_{wl}_kernel_trace.txt', 'w') as f:
         f.write(f"{short(n):62s} {cnt:6d} {a/1e3:9.1f} {mn/1e3:9.1f} {mx/1e3:9.1f} {s/1e3/steps:9.1f} {100*s/tot:6.1f}\n")
     f.write(f"\nsum of kernel time per step: {tot/1e3/steps:.1f} us\n")
     if wl in ('c2', 'c3', 'n65536'):
-        f.write("(up to 65536 entries per (b,h) every kernel runs on the one stream: the index transposes of all levels are one\n"
-                " launch, transpose_bitmap_kernel, behind the forward attention kernel)\n")
+        f.write("(up to 65536 entries per (b,h) every kernel runs on the one stream: the index transposes of all levels are\n"
+                " workgroups of the forward attention kernel's launch)\n")
     else:
         f.write("(the index transposes -- transpose_indices_kernel, tr_*_kernel, sort_segments_kernel, and transpose_bitmap_kernel for\n"
                 " the pooled levels -- run on a second stream beside the forward attention kernel: their durations overlap with it\n"
