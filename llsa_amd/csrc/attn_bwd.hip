@@ -1087,7 +1087,7 @@ __global__ __launch_bounds__(64 * kGroupWaves, 2) void attn_kside_group_kernel(G
 // pass) is 16 bytes a thread of 256, an fp32 one (dense pass) of 512: four or two slices of the workgroup take every fourth or every
 // second one, four loads in flight a thread, and their sums meet in LDS in slice order, so that the result does not depend on
 // scheduling.  The kernel is a few round trips to memory one after the other: with one workgroup of 256 threads a unit and sixteen
-// loads in flight it took 17 us at 12 x 16384 tokens (14 now), 110 at 6 x 262144 (102), 53 at 48 x 16384 (45.5); eight loads in
+// loads in flight it took 17 us at 12 x 16384 tokens (14 now), 110 at 6 x 262144 (102, and 98 past the caches), 53 at 48 x 16384 (45.5); eight loads in
 // flight, or 512 threads, 2 to 5 % more.
 struct PooledJob {
     const void* part;        // fp32 (f32x4[8][64] a slot) or, with half_part, bf16 (bf16x8[4][64] a slot) partial sums
@@ -1104,6 +1104,11 @@ struct PooledJobs {
     int n_jobs;
 };
 constexpr int kReduceThreads = 1024;
+// With STREAM the partial sums are read past the caches: more of them than the 256 MB of the memory-side cache would only push one another
+// out of it.  6 x 262144 tokens, three levels (0.6 GB): 192 -> 160 us, two levels (0.5 GB) 102.6 -> 98; below that line loads through the
+// caches win (3 x 49152, 78 MB: 20 against 22; 12 x 16384, 63 MB: 14.9 against 15.7; 48 x 16384, 252 MB: even).
+constexpr int64_t kReduceStreamBytes = (int64_t)256 << 20;
+template <bool STREAM>
 __global__ __launch_bounds__(kReduceThreads, 8) void pooled_reduce_kernel(PooledJobs jobs) {
     __shared__ __align__(16) float sums[3 * 256 * 8];         // of all slices but the first
     // grid.x: the units of all jobs, the coarsest level's first: they have the most partial sums
@@ -1131,7 +1136,10 @@ __global__ __launch_bounds__(kReduceThreads, 8) void pooled_reduce_kernel(Pooled
     for (int c0 = slice; c0 < n; c0 += kBatch * slices) {
         i32x4 v[kBatch];
 #pragma unroll
-        for (int k = 0; k < kBatch; k++) v[k] = ps[(int64_t)min(c0 + k * slices, n - 1) * stride * width];
+        for (int k = 0; k < kBatch; k++) {
+            const i32x4* at = ps + (int64_t)min(c0 + k * slices, n - 1) * stride * width;
+            v[k] = STREAM ? __builtin_nontemporal_load(at) : *at;
+        }
 #pragma unroll
         for (int k = 0; k < kBatch; k++)
             if (c0 + k * slices < n) {
@@ -1480,8 +1488,14 @@ extern "C" int llsa_attn_bwd(const llsa_attn_bwd_args* a, void* stream) {
     auto reduce_pooled = [&]() {
         if (pooled.n_jobs == 0 || (stages & LLSA_BWD_NO_REDUCE)) return;     // (profiling: time the K-side kernels alone)
         int units = 0;
-        for (int i = 0; i < pooled.n_jobs; i++) units += pooled.job[i].n_units;
-        hipLaunchKernelGGL(pooled_reduce_kernel, dim3(units, BH), dim3(kReduceThreads), 0, s, pooled);
+        int64_t bytes = 0;
+        for (int i = 0; i < pooled.n_jobs; i++) {
+            const PooledJob& j = pooled.job[i];
+            units += j.n_units;
+            bytes += BH * (j.off != nullptr ? j.slot_stride : (int64_t)j.n_chunks * j.n_units) * (j.half_part ? kSlotBytes / 2 : kSlotBytes);
+        }
+        if (bytes > kReduceStreamBytes) hipLaunchKernelGGL(pooled_reduce_kernel<true>, dim3(units, BH), dim3(kReduceThreads), 0, s, pooled);
+        else hipLaunchKernelGGL(pooled_reduce_kernel<false>, dim3(units, BH), dim3(kReduceThreads), 0, s, pooled);
     };
     KSideParams base;
     base.qr = (const bf16*)a->qr; base.dor = dor;
