@@ -212,6 +212,7 @@ __device__ __forceinline__ void finish_query_block(const llsa_attn_fwd_args& a, 
 // kernels of 6 x 65536 157 -> 154, where 75 workgroups a head read all its 65536 entries each.
 constexpr int kTrLdsFwd = 2 * kGroup * 2 * kTile / 2 - 32;    // ints of the kernel's LDS they work in (32 for their scratch)
 static_assert(tr_scratch_ints(256) <= 32, "the scratch of a transposing workgroup");
+constexpr int kGridRows = 65535;                              // rows a grid can have
 
 template <int Q, int R>
 __global__ __launch_bounds__(256, Q == 1 ? 4 : 3) void attn_fwd_kernel(llsa_attn_fwd_args a, TrJobs lists, int list_rows) {
@@ -416,8 +417,10 @@ static int attn_fwd(const llsa_attn_fwd_args* a, const llsa_transpose_job* jobs,
     const bool pairs = a->T <= kPairMaxTopk && N1 % 8 == 0 && pairs_fill(groups) && (shared >= 4 * a->T || groups >= 2048);
     TrJobs lists{};
     const int width = N1 / (pairs ? 8 : 4);                   // (a multiple of 8: N is one of 1024)
-    const bool ride = jobs != nullptr && plan_transpose(jobs, n_jobs, a->B, a->H, kTrLdsFwd, lists);
-    const int rows = ride ? (int)(((int64_t)lists.wgs * BH + width - 1) / width) : 0;
+    bool ride = jobs != nullptr && plan_transpose(jobs, n_jobs, a->B, a->H, kTrLdsFwd, lists);
+    const int64_t list_rows = ride ? ((int64_t)lists.wgs * BH + width - 1) / width : 0;
+    ride = ride && BH + list_rows <= kGridRows;               // else in launches of their own
+    const int rows = ride ? (int)list_rows : 0;
     const dim3 grid(width, BH + rows);
     const hipStream_t st = (hipStream_t)stream;
     if (!pairs) hipLaunchKernelGGL(HIP_KERNEL_NAME(attn_fwd_kernel<1, 1>), grid, dim3(256), 0, st, *a, lists, rows);
