@@ -906,8 +906,14 @@ __global__ __launch_bounds__(64 * WAVES, UPW == 2 ? 2 : 3) void attn_kside_dense
         f32x4* ps = part_slot(p.part, slot);
 #pragma unroll
         for (int dt = 0; dt < 4; dt++) {
-            ps[dt * kWave + lane] = dk[j][dt] * p.w;         // (the weight, left out of the exponentials)
-            ps[(4 + dt) * kWave + lane] = dv[j][dt] * p.w;
+            const f32x4 k = dk[j][dt] * p.w, v = dv[j][dt] * p.w;      // (the weight, left out of the exponentials)
+            if constexpr (LISTS) {                           // (large grids only: past the caches, see kGroupStreamBytes)
+                __builtin_nontemporal_store(k, &ps[dt * kWave + lane]);
+                __builtin_nontemporal_store(v, &ps[(4 + dt) * kWave + lane]);
+            } else {
+                ps[dt * kWave + lane] = k;
+                ps[(4 + dt) * kWave + lane] = v;
+            }
         }
     }
 }
@@ -938,6 +944,12 @@ constexpr int kGroupWaves = 4;
 constexpr int kGroupSegs = LLSA_MAX_LEVELS;
 constexpr int kGroupMaxBlocks = 64;               // key blocks per group over all its lists (their ids live in one lane each)
 constexpr int kGroupDenseMax = 8;                 // dense blocks are appended up to this many
+// From this many bytes of partial sums on, and with this many key blocks a group, they are stored past the caches (STREAM): they are read once, by a
+// later kernel, and push the tiles of q and dO that the fine pass gathers out of the caches meanwhile.  Forward and backward, us, through the
+// caches / past them: 18 x 16384 tokens, 94 MB: 460 / 451; 24 x 16384 606 / 588; 48 x 16384 1193 / 1176; 6 x 65536, 101 MB: 701 / 694; 16 x 65536
+// 1800 / 1785; but 12 x 16384, 63 MB: 310 / 311, and 48 x 16384 with 12 key blocks, 151 MB: 1049 / 1052.
+constexpr int64_t kGroupStreamBytes = (int64_t)80 << 20;
+constexpr int kGroupStreamBlocks = 16;
 static_assert(LLSA_POOLED_TOPK_MAX + kGroupDenseMax <= kGroupMaxBlocks, "a group's lists must fit one lane per key block");
 
 struct GroupSeg {
@@ -964,7 +976,7 @@ struct GroupParams {
 
 // UPW key blocks against the group's 16 query blocks, two query blocks per step, operands out of LDS.  `next` starts the loads of the
 // wave's next key blocks, into bk and bv, where these are no longer needed: they arrive while the sums are rounded and stored.
-template <int UPW, typename NEXT>
+template <int UPW, bool STREAM, typename NEXT>
 __device__ __forceinline__ void group_pass(const bf16x8 (&bk)[2][2], const bf16x8 (&bv)[2][2], const float (&weights)[2], bf16x8* const (&slots)[2],
                                            const bf16* shq, const bf16* shg, const float* sh_stats, int lane, NEXT&& next) {
     f32x4 dk[UPW][4], dv[UPW][4];
@@ -996,11 +1008,19 @@ __device__ __forceinline__ void group_pass(const bf16x8 (&bk)[2][2], const bf16x
     for (int j = 0; j < UPW; j++)
 #pragma unroll
         for (int pr = 0; pr < 2; pr++) {                      // registers 2 pr, 2 pr + 1 of dK, then of dV: 16 bytes a lane and store
-            dst[j][pr * kWave + lane] = cat(cvt4(dk[j][2 * pr] * w[j]), cvt4(dk[j][2 * pr + 1] * w[j]));
-            dst[j][(2 + pr) * kWave + lane] = cat(cvt4(dv[j][2 * pr] * w[j]), cvt4(dv[j][2 * pr + 1] * w[j]));
+            const bf16x8 k = cat(cvt4(dk[j][2 * pr] * w[j]), cvt4(dk[j][2 * pr + 1] * w[j]));
+            const bf16x8 v = cat(cvt4(dv[j][2 * pr] * w[j]), cvt4(dv[j][2 * pr + 1] * w[j]));
+            if constexpr (STREAM) {
+                __builtin_nontemporal_store(k, &dst[j][pr * kWave + lane]);
+                __builtin_nontemporal_store(v, &dst[j][(2 + pr) * kWave + lane]);
+            } else {
+                dst[j][pr * kWave + lane] = k;
+                dst[j][(2 + pr) * kWave + lane] = v;
+            }
         }
 }
 
+template <bool STREAM>
 __global__ __launch_bounds__(64 * kGroupWaves, 2) void attn_kside_group_kernel(GroupParams p) {
     __shared__ __align__(16) bf16 sh[2][kBlk * kTile];        // R tiles of the group's 16 query blocks: Q, then dO
     __shared__ __align__(16) float sh_stats[kBlk * kStats];   // their statistics
@@ -1078,8 +1098,8 @@ __global__ __launch_bounds__(64 * kGroupWaves, 2) void attn_kside_group_kernel(G
             if (j + 2 < hi) fetch(j + 2, 0);
             if (j + 3 < hi) fetch(j + 3, 1);
         };
-        if (j + 1 < hi) group_pass<2>(bk, bv, w, dst, &sh[0][0], &sh[1][0], sh_stats, lane, next);
-        else group_pass<1>(bk, bv, w, dst, &sh[0][0], &sh[1][0], sh_stats, lane, next);
+        if (j + 1 < hi) group_pass<2, STREAM>(bk, bv, w, dst, &sh[0][0], &sh[1][0], sh_stats, lane, next);
+        else group_pass<1, STREAM>(bk, bv, w, dst, &sh[0][0], &sh[1][0], sh_stats, lane, next);
     }
 }
 
@@ -1591,7 +1611,9 @@ extern "C" int llsa_attn_bwd(const llsa_attn_bwd_args* a, void* stream) {
         }
         if (d.merged && (stages & LLSA_BWD_DENSE))
             add_seg(a->lvl[L - 1].kr, a->lvl[L - 1].vr, nullptr, nullptr, wsp.part_dense, d.n_tok / 16, 0, d.n_tok / 16, 0, a->lvl[L - 1].gw);
-        hipLaunchKernelGGL(attn_kside_group_kernel, dim3(N2, BH), dim3(64 * kGroupWaves), 0, s, g);
+        const int64_t bytes = (int64_t)BH * N2 * g.n_blocks * (kSlotBytes / 2);
+        if (bytes > kGroupStreamBytes && g.n_blocks >= kGroupStreamBlocks) hipLaunchKernelGGL(attn_kside_group_kernel<true>, dim3(N2, BH), dim3(64 * kGroupWaves), 0, s, g);
+        else hipLaunchKernelGGL(attn_kside_group_kernel<false>, dim3(N2, BH), dim3(64 * kGroupWaves), 0, s, g);
     };
     // dense coarsest level: every unit (16 pooled tokens) meets every query block; the query
     // range is cut into d.chunks pieces whose partial sums are added afterwards
