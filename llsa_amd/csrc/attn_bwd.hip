@@ -1127,6 +1127,8 @@ constexpr int kReduceThreads = 1024;
 // With STREAM the partial sums are read past the caches: more of them than the 256 MB of the memory-side cache would only push one another
 // out of it.  6 x 262144 tokens, three levels (0.6 GB): 192 -> 160 us, two levels (0.5 GB) 102.6 -> 98; below that line loads through the
 // caches win (3 x 49152, 78 MB: 20 against 22; 12 x 16384, 63 MB: 14.9 against 15.7; 48 x 16384, 252 MB: even).
+// (Measured with sums that had been stored through the caches; since kGroupStreamBytes those of the large grids are not, and this
+// kernel takes 176 us for three levels and 98 for two: what it loses at three is less than the other passes gain.)
 constexpr int64_t kReduceStreamBytes = (int64_t)256 << 20;
 template <bool STREAM>
 __global__ __launch_bounds__(kReduceThreads, 8) void pooled_reduce_kernel(PooledJobs jobs) {
