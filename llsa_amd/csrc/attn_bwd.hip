@@ -869,19 +869,21 @@ __global__ __launch_bounds__(64 * WAVES, UPW == 2 ? 2 : 3) void attn_kside_dense
     if constexpr (WAVES == 8) {
         // Buffer (t + 1) & 1 is refilled in the first half of round t, by the first four waves while the others multiply round t - 1
         // and by those while the first multiply round t: nobody reads it then, and it is whole before anybody reads round t + 1.
+        // The halves are half a round apart, so the barrier that ends one half's products ends the other's fetches: they stand at
+        // different places.  Both arrive 2 n_pairs + 2 times, the second four waves one time more in front and one time less behind.
         auto round = [&](int t, Stage& nxt) __attribute__((always_inline)) {
             gather(t, nxt);
-            __syncthreads();
+            counted_barrier();
             if (active) multiply();
-            __syncthreads();
+            counted_barrier();
         };
-        __syncthreads();
-        if (wave >= 4) __syncthreads();
+        counted_barrier();
+        if (wave >= 4) counted_barrier();
         for (int t = 0; t < n_pairs; t += 2) {
             round(t, s1);
             round(t + 1, s0);
         }
-        if (wave < 4) __syncthreads();
+        if (wave < 4) counted_barrier();
     } else {
         auto round = [&](int t, Stage& nxt) __attribute__((always_inline)) {
             __syncthreads();

@@ -142,6 +142,14 @@ __device__ __forceinline__ void copy16_global_to_lds(const bf16* g_lane, bf16* l
                                      (__attribute__((address_space(3))) void*)lds_wave_base, 16, OFF * (int)sizeof(bf16), 0);
 }
 __device__ __forceinline__ void wait_vm0() { __builtin_amdgcn_s_waitcnt(0x0F70); }   // vmcnt(0), other counters untouched
+// A workgroup barrier of which waves may stand at different places in the code: the hardware's barrier counts arrivals, one per wave,
+// whatever instruction they come from.  __syncthreads() is the same instructions, but promises this only where all waves meet at
+// the same one.  Every wave must arrive equally often, and the branch between the places must be wave-uniform.
+__device__ __forceinline__ void counted_barrier() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
+    __builtin_amdgcn_s_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
+}
 // vmcnt(0) and lgkmcnt(0).  The compiler books a copy into LDS against both counters; until it has seen
 // both drained it takes the vector-memory queue for out of order and turns every later wait into vmcnt(0).
 __device__ __forceinline__ void wait_all_mem() { __builtin_amdgcn_s_waitcnt(0x0070); }

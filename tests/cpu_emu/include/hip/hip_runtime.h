@@ -132,6 +132,7 @@ inline int __clz(int x) { return x ? __builtin_clz((unsigned)x) : 32; }
 #define __builtin_amdgcn_s_waitcnt(x) emu::wave_sync()
 #define __builtin_amdgcn_s_setprio(x) ((void)0)
 #define __builtin_amdgcn_fence(order, scope) ((void)0)
+#define __builtin_amdgcn_s_barrier() emu::block_barrier()
 #define hipFuncAttributeMaxDynamicSharedMemorySize 0
 template <typename F>
 inline hipError_t hipFuncSetAttribute(F, int, int) { return hipSuccess; }
