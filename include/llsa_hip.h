@@ -43,7 +43,7 @@ extern "C" {
 #define LLSA_DTYPE_BF16 0
 #define LLSA_DTYPE_F32 1
 
-#define LLSA_ABI_VERSION 208     /* changes with every change of a signature or argument structure below */
+#define LLSA_ABI_VERSION 209     /* changes with every change of a signature or argument structure below */
 int llsa_version(void);          /* LLSA_ABI_VERSION of the built library                                    */
 const char* llsa_last_error_string(void);
 
@@ -204,6 +204,9 @@ typedef struct llsa_attn_fwd_args {
 } llsa_attn_fwd_args;
 
 int llsa_attn_fwd(const llsa_attn_fwd_args* a, void* stream);
+/* How many query blocks (1 or 2) a wave of llsa_attn_fwd (backward = 0) or of llsa_attn_bwd's dQ kernel (backward = 1) takes at
+ * these sizes; topk: of every level, finest first. */
+int llsa_query_blocks_per_wave(int B, int H, int N, const int32_t* topk, int levels, int backward);
 
 /* ------------------------------------------------------------------------------------------
  * Index transpose.  Replaces transpose_indices (kernel/triton/indices_transpose.py:104-109):

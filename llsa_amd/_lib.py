@@ -101,6 +101,7 @@ _SIGNATURES = {
     "llsa_topk_cascade": (c_int, [c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_int, c_void_p]),
     "llsa_topk_cascade_max_parents": (c_int, []),
     "llsa_attn_fwd": (c_int, [C.POINTER(AttnFwdArgs), c_void_p]),
+    "llsa_query_blocks_per_wave": (c_int, [c_int, c_int, c_int, C.POINTER(c_int32), c_int, c_int]),
     "llsa_transpose_indices": (c_int, [c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_int, c_int, c_void_p]),
     "llsa_transpose_indices_multi": (c_int, [C.POINTER(TransposeJob), c_int, c_int, c_int, c_void_p]),
     "llsa_attn_fwd_lists": (c_int, [C.POINTER(AttnFwdArgs), C.POINTER(TransposeJob), c_int, c_void_p]),
@@ -114,7 +115,7 @@ _SIGNATURES = {
 
 EXPORTS = tuple(_SIGNATURES)
 CHUNK_FINE_MAX = 256                                        # LLSA_CHUNK_FINE_MAX of include/llsa_hip.h
-ABI_VERSION = 208                                           # LLSA_ABI_VERSION
+ABI_VERSION = 209                                           # LLSA_ABI_VERSION
 STATIC_PARTIALS_MAX = 262144                                # LLSA_STATIC_PARTIALS_MAX
 
 

@@ -1484,7 +1484,7 @@ extern "C" int llsa_attn_bwd(const llsa_attn_bwd_args* a, void* stream) {
 
     const int stages = a->stages ? a->stages : (0x7fffffff & ~LLSA_BWD_NO_REDUCE);
     if (stages & LLSA_BWD_DQ) {
-        const bool pairs = a->T <= kPairMaxTopk && N1 % 8 == 0 && pairs_fill((int64_t)N1 / 8 * BH);
+        const bool pairs = two_blocks_per_wave(BH, N, topk, L, false);
         const dim3 grid(N1 / (pairs ? 8 : 4), BH);
 #define LLSA_DQ(Q, R)                                                                                                                  \
     do {                                                                                                                               \

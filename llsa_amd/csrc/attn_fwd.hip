@@ -387,6 +387,7 @@ static int attn_fwd(const llsa_attn_fwd_args* a, const llsa_transpose_job* jobs,
                  "attn_fwd: %d level(s) need N %% %lld == 0 (N=%d): the coarsest level is walked in 64-token tiles of its N/16^levels pooled tokens",
                  a->levels, (long long)mult, a->N);
     int listed = 0;
+    int32_t topk[LLSA_MAX_LEVELS] = {a->T};
     int64_t span = 256;                                       // tokens under one block of level l
     for (int l = 1; l <= a->levels; l++, span *= 16) {
         const llsa_fwd_level& lv = a->lvl[l - 1];
@@ -397,6 +398,7 @@ static int attn_fwd(const llsa_attn_fwd_args* a, const llsa_transpose_job* jobs,
             LLSA_REQUIRE(lv.T >= 4 && lv.T % 4 == 0 && lv.T <= a->N / span, "attn_fwd: topk of level %d (%d) must be a multiple of 4 and <= N/%lld",
                          l, lv.T, (long long)span);
             listed += lv.T;
+            topk[l] = lv.T;
         }
     }
     LLSA_REQUIRE(listed <= LLSA_POOLED_TOPK_MAX, "attn_fwd: the topk of the pooled levels together (%d) must not exceed %d", listed,
@@ -408,13 +410,8 @@ static int attn_fwd(const llsa_attn_fwd_args* a, const llsa_transpose_job* jobs,
     // leaves more and shorter waves.  Two win where the pooled blocks are most of the walk (11 x 32768 tokens, topk 8,
     // 128 pooled blocks: 227 against 267 us) and on large grids (16 x 16384, topk 16: 78.2 against 83.7; 48 x 16384: 228 against 271; 6 x
     // 262144: 929 against 1057), one on smaller ones (12 x 16384: 58.5 against 64.6; 24 x 4096: 30.1 against 31.2; 3 x 49152 at topk 64
-    // even) and, as in the backward pass, where the last round would be mostly empty (see pairs_fill; 2 x 65536, topk 8:
-    // 45.0 against 48.0; 7 x 16384, topk 8, 64 pooled blocks: 50.6 against 54.3).
-    int64_t shared = listed, coarsest = a->N / 256;
-    for (int l = 1; l < a->levels; l++) coarsest /= 16;
-    shared += coarsest;
-    const int64_t groups = (int64_t)N1 / 8 * BH;
-    const bool pairs = a->T <= kPairMaxTopk && N1 % 8 == 0 && pairs_fill(groups) && (shared >= 4 * a->T || groups >= 2048);
+    // even) and where the last round would be mostly empty (see pairs_pay).
+    const bool pairs = two_blocks_per_wave(BH, a->N, topk, a->levels, true);
     TrJobs lists{};
     const int width = N1 / (pairs ? 8 : 4);                   // (a multiple of 8: N is one of 1024)
     bool ride = jobs != nullptr && plan_transpose(jobs, n_jobs, a->B, a->H, kTrLdsFwd, lists);
@@ -429,6 +426,11 @@ static int attn_fwd(const llsa_attn_fwd_args* a, const llsa_transpose_job* jobs,
     const int rc = launch_status("attn_fwd");
     if (rc != 0 || jobs == nullptr || ride) return rc;
     return llsa_transpose_indices_multi(jobs, n_jobs, a->B, a->H, stream);
+}
+
+extern "C" int llsa_query_blocks_per_wave(int B, int H, int N, const int32_t* topk, int levels, int backward) {
+    LLSA_REQUIRE(B > 0 && H > 0 && N > 0 && topk != nullptr && levels >= 1 && levels <= LLSA_MAX_LEVELS, "query_blocks_per_wave: bad shape");
+    return two_blocks_per_wave((int64_t)B * H, N, topk, levels, backward == 0) ? 2 : 1;
 }
 
 extern "C" int llsa_attn_fwd(const llsa_attn_fwd_args* a, void* stream) { return attn_fwd(a, nullptr, 0, stream); }

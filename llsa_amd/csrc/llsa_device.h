@@ -352,10 +352,38 @@ constexpr int kPairMaxTopk = 64;
 //   728 (13 x 7168, topk 12) 37.0 / 34.8;  768 (24 x 4096) 34.7 / 34.1;  784 (14 x 7168) 39.6 / 43.6;  840 (15 x 7168) 40.8 / 45.0
 //   1024 (8 x 8192) 51.1 / 51.8;  1152 (16 x 9216) 60.8 / 63.7;  1280 (20 x 8192) 64.2 / 60.7;  1536 (24 x 8192) 78.6 / 73.2
 //   1568 (28 x 7168) 69.6 / 72.8;  2048 (16 x 16384) 101.6 / 90.8;  3072 (24 x 16384) 144.4 / 134.4
+// The forward's waves are shorter.  It gains from two as soon as the single blocks no longer fit the chip at once (512 groups), and up to a round of pairs
+// its rounds may be emptier.  Sampling, topk 8, the whole pass: 512 (8 x 8192) 43.9 / 45.2;  576 (9 x 8192) 53.9 / 52.3;  640 (10 x 8192) 53.5 / 53.0
+//   832 (13 x 8192) 62.1 / 65.9;  960 (15 x 8192) 66.7 / 68.0;  1152 (18 x 8192) 76.9 / 78.9;  1280 (20 x 8192) 81.3 / 80.8
+// Where most of the walk is pooled blocks, which a wave of two reads once for both, two win from 512 groups on and with as much as 60 % more
+// places than groups.  Sampling, and in brackets the training step with one / two in dQ, topk 8 unless given:
+//   512 (2 x 32768, 128 pooled blocks) 97.4 / 94.7 (263.5 / 260.7);  512 (65536, 256) 147.3 / 139.5 (423.4 / 415.4), at topk 16 156.7 / 149.8 (455.9 / 448.4)
+//   512 (4 x 16384, 64) 61.1 / 60.4 (182.3 / 181.7);  640 (2 x 40960, 160) 128.6 / 125.7 (366.7 / 364.1);  960 (5 x 24576, 96) 121.7 / 118.5 (350.8 / 345.3)
+//   1024 (8 x 16384) 100.8 / 97.8 (300.2 / 295.6);  1024 (2 x 65536) 239.7 / 224.5 (749.9 / 729.6);  1664 (13 x 16384) 155.1 / 151.2 (467.0 / 461.8)
+//   but 800 (5 x 20480, 80) 102.3 / 106.7 (276.8 / 282.2);  896 (4 x 28672, 112) 125.3 / 127.7 (359.3 / 361.6)
+// With a larger topk from a full round on: 1024 (8 x 16384, topk 16) 109.1 / 107.2 (332.8 / 328.8);  960 (5 x 24576, topk 24) 154.5 / 151.7 (457.7 / 450.9)
+//   1024 (2 x 65536, topk 64) 368.7 / 358.3 (1166.0 / 1147.2);  but 512 (4 x 16384, topk 16) 65.3 / 65.8 (196.7 / 196.9);  512 (65536, topk 64) 217.3 / 221.2
 constexpr int kPairPlaces = 256 * 3;
-inline bool pairs_fill(int64_t groups) {
-    const int64_t places = (groups + kPairPlaces - 1) / kPairPlaces * kPairPlaces;
-    return groups > 640 && (places - groups) * 10 <= groups * 3;
+inline bool pairs_pay(int64_t groups, int64_t pooled_blocks, int T, bool forward) {
+    const int64_t places = (groups + kPairPlaces - 1) / kPairPlaces * kPairPlaces, idle = (places - groups) * 10;
+    if (pooled_blocks >= 64 && pooled_blocks >= 4 * T && groups >= (pooled_blocks >= 8 * T ? 512 : kPairPlaces) && idle <= groups * 6) return true;
+    if (forward && groups <= kPairPlaces) return groups > 512;
+    return groups > 640 && idle <= groups * 3;
+}
+// Blocks of the pooled levels every query block reads, all levels (topk: of every level, finest first)
+inline int64_t pooled_blocks_read(int N, const int32_t* topk, int levels) {
+    int64_t blocks = N / 256;
+    for (int l = 1; l < levels; l++) blocks /= 16;
+    for (int l = 1; l < levels; l++) blocks += topk[l];
+    return blocks;
+}
+// Whether a wave of the forward / dQ kernel takes two query blocks
+inline bool two_blocks_per_wave(int64_t BH, int N, const int32_t* topk, int levels, bool forward) {
+    const int64_t groups = (int64_t)N / 128 * BH, pooled = pooled_blocks_read(N, topk, levels);
+    if (topk[0] > kPairMaxTopk || N % 128 != 0 || !pairs_pay(groups, pooled, topk[0], forward)) return false;
+    // Where the fine blocks are most of the walk the forward gains little from two on grids of a few rounds (topk 8, 16 pooled blocks: 17 x
+    // 4096 tokens 44.3 / 42.8, 20 x 4096 45.1 / 43.9, but 28 x 4096 52.9 / 55.8, 32 x 4096 55.8 / 57.7, 36 x 4096 62.7 / 64.9, 40 x 4096 66.2 / 66.7)
+    return !forward || pooled >= 4 * topk[0] || groups >= 2048;
 }
 
 // 16- and 8-byte reads that are LDS reads by construction (ds_read_b128 / ds_read_b64)
