@@ -105,6 +105,7 @@ _SIGNATURES = {
     "llsa_transpose_indices": (c_int, [c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_int, c_int, c_void_p]),
     "llsa_transpose_indices_multi": (c_int, [C.POINTER(TransposeJob), c_int, c_int, c_int, c_void_p]),
     "llsa_attn_fwd_lists": (c_int, [C.POINTER(AttnFwdArgs), C.POINTER(TransposeJob), c_int, c_void_p]),
+    "llsa_lists_ride": (c_int, [c_int, c_int, c_int, C.POINTER(c_int32), c_int]),
     "llsa_transpose_one_launch": (c_int, [c_int, c_int, c_int, c_int, c_int]),
     "llsa_work_list_len": (c_int64, [c_int, c_int, c_int, c_int]),
     "llsa_fine_chunk": (c_int, [c_int]),

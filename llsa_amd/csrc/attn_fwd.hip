@@ -209,9 +209,14 @@ __device__ __forceinline__ void finish_query_block(const llsa_attn_fwd_args& a, 
 // The first `list_rows` rows of the grid make the index transposes of the backward (transpose_device.h): they need the selection
 // and nothing else, and are latency for the most part, which the attention's workgroups fill.  In a launch of their own behind this
 // one the chip waited for them: step of 12 x 16384 tokens 317 -> 309 us, of 24 x 4096 163 -> 156, of 48 x 16384 1284 -> 1264; both
-// kernels of 6 x 65536 157 -> 154, where 75 workgroups a head read all its 65536 entries each.
+// kernels of 6 x 65536 157 -> 154, where 67 workgroups a head (66 ranges and the histogram) read all its 65536 entries each.
+// That reading is what bounds them on the largest grids: their workgroups then fill the chip by themselves for rounds, and a launch of their own, with
+// twice the LDS and so half the ranges, reads less.  Steps behind the forward / riding, us, by entries read over all workgroups (topk 16, 65536
+// tokens): 8 heads (35 M) 932 / 914;  16 (70 M) 1768 / 1759;  20 (88 M) 2257 / 2251;  24 (105 M) 2651 / 2665;  28 (123 M) 3128 / 3140;  32 (141 M)
+// 3474 / 3493, on another card 3503 / 3543.  42 x 49152, topk 20 (98 M) 3233 / 3251;  64 x 32768, topk 32 (76 M) even.
 constexpr int kTrLdsFwd = 2 * kGroup * 2 * kTile / 2 - 32;    // ints of the kernel's LDS they work in (32 for their scratch)
 static_assert(tr_scratch_ints(256) <= 32, "the scratch of a transposing workgroup");
+constexpr int64_t kRideMaxReads = (int64_t)88 << 20;          // entries the riding workgroups may read in all
 constexpr int kGridRows = 65535;                              // rows a grid can have
 
 template <int Q, int R>
@@ -375,6 +380,16 @@ __global__ __launch_bounds__(256, Q == 1 ? 4 : 3) void attn_fwd_kernel(llsa_attn
 
 using namespace llsa;
 
+// Rows of a grid of `width` workgroups that the index transposes take in front of the attention's, or -1: launches of their own
+static int64_t plan_list_rows(const llsa_transpose_job* jobs, int n_jobs, int B, int H, int width, TrJobs& lists) {
+    if (!plan_transpose(jobs, n_jobs, B, H, kTrLdsFwd, lists)) return -1;
+    const int64_t BH = (int64_t)B * H, rows = (lists.wgs * BH + width - 1) / width;
+    int64_t reads = 0;
+    for (int i = 0; i < lists.n_jobs; i++) reads += (lists.job[i].parts + 1) * BH * lists.job[i].Mb * lists.job[i].T;
+    return reads > kRideMaxReads || BH + rows > kGridRows ? -1 : rows;
+}
+static int forward_width(int N, bool pairs) { return N / (pairs ? 128 : 64); }   // workgroups of a (b,h); a multiple of 8: N is one of 1024
+
 // jobs: the index transposes that ride along, or nullptr
 static int attn_fwd(const llsa_attn_fwd_args* a, const llsa_transpose_job* jobs, int n_jobs, void* stream) {
     LLSA_REQUIRE(a != nullptr, "attn_fwd: null args");
@@ -405,7 +420,7 @@ static int attn_fwd(const llsa_attn_fwd_args* a, const llsa_transpose_job* jobs,
                  LLSA_POOLED_TOPK_MAX);
     LLSA_REQUIRE(aligned16(a->qr) && aligned16(a->kr) && aligned16(a->vt) && aligned16(a->o), "attn_fwd: tensors must be 16-byte aligned");
     LLSA_REQUIRE((a->sob % 4 == 0) && (a->soh % 4 == 0) && (a->son % 4 == 0), "attn_fwd: rows of o must be 8-byte aligned");
-    const int N1 = a->N / 16, BH = a->B * a->H;
+    const int BH = a->B * a->H;
     // Two query blocks per wave halve the LDS reads of the pooled blocks and save a quarter of the fine fetches; one per wave
     // leaves more and shorter waves.  Two win where the pooled blocks are most of the walk (11 x 32768 tokens, topk 8,
     // 128 pooled blocks: 227 against 267 us) and on large grids (16 x 16384, topk 16: 78.2 against 83.7; 48 x 16384: 228 against 271; 6 x
@@ -413,10 +428,9 @@ static int attn_fwd(const llsa_attn_fwd_args* a, const llsa_transpose_job* jobs,
     // even) and where the last round would be mostly empty (see pairs_pay).
     const bool pairs = two_blocks_per_wave(BH, a->N, topk, a->levels, true);
     TrJobs lists{};
-    const int width = N1 / (pairs ? 8 : 4);                   // (a multiple of 8: N is one of 1024)
-    bool ride = jobs != nullptr && plan_transpose(jobs, n_jobs, a->B, a->H, kTrLdsFwd, lists);
-    const int64_t list_rows = ride ? ((int64_t)lists.wgs * BH + width - 1) / width : 0;
-    ride = ride && BH + list_rows <= kGridRows;               // else in launches of their own
+    const int width = forward_width(a->N, pairs);
+    const int64_t list_rows = jobs != nullptr ? plan_list_rows(jobs, n_jobs, a->B, a->H, width, lists) : -1;
+    const bool ride = list_rows >= 0;
     const int rows = ride ? (int)list_rows : 0;
     const dim3 grid(width, BH + rows);
     const hipStream_t st = (hipStream_t)stream;
@@ -431,6 +445,15 @@ static int attn_fwd(const llsa_attn_fwd_args* a, const llsa_transpose_job* jobs,
 extern "C" int llsa_query_blocks_per_wave(int B, int H, int N, const int32_t* topk, int levels, int backward) {
     LLSA_REQUIRE(B > 0 && H > 0 && N > 0 && topk != nullptr && levels >= 1 && levels <= LLSA_MAX_LEVELS, "query_blocks_per_wave: bad shape");
     return two_blocks_per_wave((int64_t)B * H, N, topk, levels, backward == 0) ? 2 : 1;
+}
+
+extern "C" int llsa_lists_ride(int B, int H, int N, const int32_t* topk, int levels) {
+    LLSA_REQUIRE(B > 0 && H > 0 && N > 0 && topk != nullptr && levels >= 1 && levels <= LLSA_MAX_LEVELS, "lists_ride: bad shape");
+    llsa_transpose_job jobs[LLSA_MAX_LEVELS];
+    int32_t* const some = reinterpret_cast<int32_t*>(16);     // (the plan only looks whether there is a list)
+    for (int l = 0, m = N / 16; l < levels; l++, m /= 16) jobs[l] = llsa_transpose_job{some, some, some, nullptr, nullptr, m, m, topk[l], 1};
+    TrJobs lists{};
+    return plan_list_rows(jobs, levels, B, H, forward_width(N, two_blocks_per_wave((int64_t)B * H, N, topk, levels, true)), lists) >= 0;
 }
 
 extern "C" int llsa_attn_fwd(const llsa_attn_fwd_args* a, void* stream) { return attn_fwd(a, nullptr, 0, stream); }

@@ -1,5 +1,8 @@
 """The index transposes made by workgroups of the forward attention launch: the same lists, and the same output, as in launches of
-their own -- one range and many, rows that do not divide, repeated entries, and lists too long to ride along."""
+their own -- one range and many, rows that do not divide, repeated entries, grids of one and of two query blocks a wave, and lists too long or
+too many to ride along."""
+import ctypes as C
+
 import pytest
 import torch
 
@@ -48,6 +51,36 @@ def _check(dev, monkeypatch, B, H, N, T, T2, chunk):
 def test_cpu(monkeypatch, B, H, N, T, T2, chunk):
     with override_library_for_tests(emu_lib()):
         _check(torch.device("cpu"), monkeypatch, B, H, N, T, T2, chunk)
+
+
+def _ride(B, H, N, *topk):
+    return current_lib().lists_ride(B, H, N, (C.c_int32 * len(topk))(*topk), len(topk))
+
+
+def test_lines_of_the_rule():
+    assert _ride(1, 6, 1024, 8) and _ride(2, 6, 16384, 16, 16) and _ride(1, 6, 65536, 16, 16) and _ride(3, 5, 7168, 12)
+    assert _ride(1, 20, 65536, 16, 16) and not _ride(1, 24, 65536, 16, 16) and not _ride(1, 32, 65536, 16, 16)    # entries read: 88, 105 and 141 million
+    assert _ride(16, 8, 16384, 64, 16) and _ride(128, 16, 1024, 8)
+    assert not _ride(1, 1, 65536, 20, 8)                      # more than 65536 entries
+    assert _ride(1, 1, 130048, 8) and not _ride(1, 1, 131072, 8, 4)      # 8128 and 8192 key blocks: their histogram takes 8160 ints of LDS at most
+    assert not _ride(1, 65535, 1024, 4)                       # more rows than a grid has
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("B,H,N,T,T2,chunk", [(1, 24, 4096, 4, 0, 64), (1, 16, 16384, 48, 4, 64)])
+def test_two_query_blocks_a_wave(monkeypatch, B, H, N, T, T2, chunk):
+    topk = (T, T2) if T2 else (T,)
+    assert current_lib().query_blocks_per_wave(B, H, N, (C.c_int32 * len(topk))(*topk), len(topk), 0) == 2 and _ride(B, H, N, *topk)
+    _check(torch.device("cuda"), monkeypatch, B, H, N, T, T2, chunk)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("B,H,N,T,T2,chunk", [(1, 1, 131072, 8, 4, 256), (1, 24, 65536, 16, 4, 256)])
+def test_behind_the_forward(monkeypatch, B, H, N, T, T2, chunk):
+    """Lists that one launch could make, but not beside the attention: too many key blocks, too many entries over all heads."""
+    topk = (C.c_int32 * 2)(T, T2)
+    assert current_lib().transpose_one_launch(N // 16, N // 16, T, B, H) and not current_lib().lists_ride(B, H, N, topk, 2)
+    _check(torch.device("cuda"), monkeypatch, B, H, N, T, T2, chunk)
 
 
 @pytest.mark.gpu
