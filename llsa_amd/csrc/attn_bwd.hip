@@ -1343,12 +1343,17 @@ static DensePlan dense_plan(int B, int H, int N, int levels) {
     const int groups = (n_units + d.wg_units - 1) / d.wg_units * B * H;   // workgroups per piece of the query range
     // The query range is cut so that the workgroups fill the chip's resident slots (256 CUs x the workgroups the
     // registers allow per CU) a whole number of times: a count just above a multiple of the slots leaves a last round in
-    // which a few workgroups run alone.  Three times where the pieces are long even so, which evens out their progress
-    // (N = 262144: 862 us against 920 for once); once where they are short, for a third of the partial sums (N = 7168, 15
-    // heads: the reduction 13.6 -> 7.6 us, the pass itself the same).  (Both measured with four waves of two units.)
+    // which a few workgroups run alone.  Once, for the fewest partial sums; where the pieces are long and once leaves more than a
+    // fifth of the slots empty, twice or three times.  Training steps cut for one / two / three rounds, us, in brackets how full:
+    //   4 x 8 x 16384 1078 (1.00) / 1090 / 1104;  8 x 32768 788 (1.00) / 796 / 807;  3 x 49152 693 (.98) / 701 / 711;  2 x 65536 769 (1.00) / 777 / 788
+    //   3 x 6 x 16384 630 (.84) / 637 (.98) / 651 (.94);  7 x 65536 2350 (.88) / 2364 / 2384;  two levels: 8 x 131072 1666 (1.00) / 1675 / 1691
+    //   3 x 262144 2031 (.98) / 2046 / 2043;  6 x 262144 even;  but 4 x 6 x 16384 743 (.75) / 738 (.94) / 745 (1.00);  6 x 65536 2129 (.75) / 2037 (.94) /
+    //   2041 (1.00);  5 x 8 x 16384 1256 (.62) / 1200 (.94) / 1228 (.83);  8 x 6 x 16384 1460 (.75) / 1476 (.75) / 1441 (1.00)
+    //   short pieces: 3 x 5 x 7168 191 (.94) / 197 / 205;  4 x 6 x 4096 162.5 (.94) / 169 / 169
     const int slots = 256 * (d.wg_units == 16 ? 1 : d.wg_units == 8 ? 2 : 3);
     int chunks = slots / groups;
-    if (chunks < 1 || N1 / chunks > 256) chunks = 3 * slots / groups;
+    for (int rounds = 2; rounds <= 3 && (chunks < 1 || (N1 / chunks > 256 && (int64_t)chunks * groups * 5 < (int64_t)(rounds - 1) * slots * 4)); rounds++)
+        chunks = rounds * slots / groups;
     if (chunks > N1 / 16) chunks = N1 / 16;
     if (chunks < 1) chunks = 1;
     int len = (N1 + chunks - 1) / chunks;

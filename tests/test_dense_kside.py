@@ -1,5 +1,5 @@
 """The K side of the dense coarsest level against the oracle where its forms begin and end: groups of 4, 8 and 16 units (a unit is 16
-coarsest tokens), the last group full, with idle waves, and almost empty."""
+coarsest tokens), the last group full, with idle waves, and almost empty; and the query range cut for one, two and three rounds of the chip."""
 import pytest
 import torch
 
@@ -30,6 +30,7 @@ def test_dense_cpu(N):
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("B,H,N", [(1, 1, 1024), (1, 2, 3072), (1, 1, 4096), (2, 3, 4096), (1, 2, 5120), (1, 3, 6144), (2, 2, 7168), (1, 2, 9216), (1, 1, 17408)])
+@pytest.mark.parametrize("B,H,N", [(1, 1, 1024), (1, 2, 3072), (1, 1, 4096), (2, 3, 4096), (1, 2, 5120), (1, 3, 6144), (2, 2, 7168), (1, 2, 9216), (1, 1, 17408),
+                                   (1, 8, 32768), (4, 6, 16384), (2, 24, 16384)])          # 4, 5 and 4 long pieces
 def test_dense_gpu(B, H, N):
     _run(torch.device("cuda"), B, H, N)
