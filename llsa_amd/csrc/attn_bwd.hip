@@ -1126,12 +1126,13 @@ struct PooledJobs {
     int n_jobs;
 };
 constexpr int kReduceThreads = 1024;
-// With STREAM the partial sums are read past the caches: more of them than the 256 MB of the memory-side cache would only push one another
-// out of it.  6 x 262144 tokens, three levels (0.6 GB): 192 -> 160 us, two levels (0.5 GB) 102.6 -> 98; below that line loads through the
-// caches win (3 x 49152, 78 MB: 20 against 22; 12 x 16384, 63 MB: 14.9 against 15.7; 48 x 16384, 252 MB: even).
-// (Measured with sums that had been stored through the caches; since kGroupStreamBytes those of the large grids are not, and this
-// kernel takes 176 us for three levels and 98 for two: what it loses at three is less than the other passes gain.)
-constexpr int64_t kReduceStreamBytes = (int64_t)256 << 20;
+// With STREAM the partial sums are read past the caches: they are read once, and what they push out of the caches the fine pass behind this
+// kernel needs.  Few of them push out little.  Training steps, through the caches / past them, us: two levels, 14 x 16384 tokens, 73 MB, 356 / 352;
+// 18 x 16384, 94 MB, 442.5 / 432; 24 x 16384 575 / 561; 48 x 16384, 252 MB, 1146 / 1143; 6 x 65536, 133 MB, 686 / 672; 4 x 49152, topk 32, 126 MB,
+// 429 / 423; three levels of 262144 704 / 694; 3 x 49152, topk 32, 98 MB, and 6 x 262144 with two (0.5 GB) and three levels (0.6) even.  Below the
+// line either may win by a little: 2 x 131072, 67 MB, 457 / 458.5, 12 x 16384, 63 MB, 306 / 304.5, one level of 6 x 16384, 31 MB, 246.5 / 247.4, of
+// 4 x 6 x 4096, 31 MB, 163.0 / 163.4, of 8 x 6 x 4096, 31 MB, 266.3 / 265.0, of 64 x 6 x 1024, 25 MB, 439 / 434.
+constexpr int64_t kReduceStreamBytes = (int64_t)64 << 20;
 template <bool STREAM>
 __global__ __launch_bounds__(kReduceThreads, 8) void pooled_reduce_kernel(PooledJobs jobs) {
     __shared__ __align__(16) float sums[3 * 256 * 8];         // of all slices but the first
