@@ -947,9 +947,15 @@ constexpr int kGroupSegs = LLSA_MAX_LEVELS;
 constexpr int kGroupMaxBlocks = 64;               // key blocks per group over all its lists (their ids live in one lane each)
 constexpr int kGroupDenseMax = 8;                 // dense blocks are appended up to this many
 // From this many bytes of partial sums on, and with this many key blocks a group, they are stored past the caches (STREAM): they are read once, by a
-// later kernel, and push the tiles of q and dO that the fine pass gathers out of the caches meanwhile.  Forward and backward, us, through the
-// caches / past them: 18 x 16384 tokens, 94 MB: 460 / 451; 24 x 16384 606 / 588; 48 x 16384 1193 / 1176; 6 x 65536, 101 MB: 701 / 694; 16 x 65536
-// 1800 / 1785; but 12 x 16384, 63 MB: 310 / 311, and 48 x 16384 with 12 key blocks, 151 MB: 1049 / 1052.
+// later kernel, and push the tiles of q and dO that the fine pass gathers out of the caches meanwhile.  Training steps, us, through the
+// caches / past them, read past them either way (kReduceStreamBytes):
+//   20 key blocks: 16 x 16384 tokens, 80 MiB, 392 / 385;  18 x 16384 443 / 436;  24 x 16384 581 / 568.5;  48 x 16384 1159 / 1147
+//   24: 8 x 32768, 96 MiB, 424 / 421;  12 x 32768 620 / 612.5     36: 12 x 16384, 108 MiB, 372 / 366     16: 6 x 65536, 96 MiB, 682 / 677;  8 x 65536 909 /
+//   906;  36 x 16384, 144 MiB, 838 / 830.5;  24 x 16384, 96 MiB, 535 / 538;  48 x 16384, 16 x 65536 and 3 x 262144 even;  24 x 32768 1092 / 1096
+//   12: 30 x 16384, 90 MiB, 644.5 / 647;  48 x 16384 1019 / 1024;  72 x 16384 1494 / 1505;  24 x 32768 1014 / 1022
+//   three levels: 3 x 262144 even, but 1 x 262144, 36 key blocks, 144 MiB, 691 / 699
+// The number of key blocks is a multiple of 4 (topk and coarsest blocks are), so 12 and 16 are neighbours.  Below the byte line, 64 to 80 MiB: 13 x
+// 16384 338 / 336, 6 x 32768 335 / 330.5, but 6 x 49152 510 / 512, 3 x 49152 with 32 key blocks 678 / 679; 10 x 16384, 50 MiB, 267.9 / 268.2.
 constexpr int64_t kGroupStreamBytes = (int64_t)80 << 20;
 constexpr int kGroupStreamBlocks = 16;
 static_assert(LLSA_POOLED_TOPK_MAX + kGroupDenseMax <= kGroupMaxBlocks, "a group's lists must fit one lane per key block");

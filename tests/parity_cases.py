@@ -649,10 +649,11 @@ def _compare_op_l2(tag, q, k, v, do, o, dq, dk, dv, dev_idx, dev_pidx, T, T2, fr
     MEASURED[tag]["indices (same, tie-free)"] = selection_sparse_vs_oracle("indices", ctx["pq"], ctx["pk"], pidx, idx, T, strict=not qk_norm)
 
 
-def check_op_l3(dev, B=1, H=1, N=262144, T=16, T2=16, T3=16, rope=True, qk_norm=False):
+def check_op_l3(dev, B=1, H=1, N=262144, T=16, T2=16, T3=16, rope=True, qk_norm=False, heads=None):
     """llsa_l3 through autograd against the oracle's three-level composition fed with the device's own
     selection; the selection itself must be a legal cascade (every block under a block its parent chose) and,
-    on these smooth inputs, equal to the oracle's at the two coarse levels wherever the bf16 scores do not tie."""
+    on these smooth inputs, equal to the oracle's at the two coarse levels wherever the bf16 scores do not tie.
+    heads: those the oracle is run on (no head sees another); None = all."""
     import llsa_amd
     from llsa_amd.kernel.torch_op._fused import selection
     from llsa_amd.utils.rope_table import rope_table
@@ -669,6 +670,8 @@ def check_op_l3(dev, B=1, H=1, N=262144, T=16, T2=16, T3=16, rope=True, qk_norm=
     o, dq, dk, dv = _grads(run, q, k, v, do)
     idx, pidx, ppidx = captured["sel"]
     assert idx.shape == (B, H, N // 16, T) and pidx.shape == (B, H, N // 256, T2) and ppidx.shape == (B, H, N // 4096, T3)
+    if heads is not None:
+        q, k, v, do, o, dq, dk, dv, idx, pidx, ppidx = (t[:, heads] for t in (q, k, v, do, o, dq, dk, dv, idx, pidx, ppidx))
     par = pidx.repeat_interleave(16, dim=2)
     assert ((idx[..., :, None] // 16) == par[..., None, :]).any(-1).all(), "a fine block outside its parent's selection"
     gpar = ppidx.repeat_interleave(16, dim=2)
@@ -698,8 +701,9 @@ def check_op_lk_sparse_dout(dev, N=4194304, topks=(16, 16, 16, 16), H=1, query_b
     dK / dV follows from those few queries -- enumerated here in fp64 (torch.autograd over each query's key set, taken
     from the device's own selection: its fine blocks, the pooled blocks of every level, the dense coarsest level) and
     pushed down the chain of mean pools (a pooled token's gradient goes to its 16 children, divided by 16) and back
-    through the rotation.  This pins what the single-query checks of o and dq cannot: the group-major pass of every
-    level (its list owners 16, 256, ... groups wide), the partial sums placed by inverse positions, their reduction,
+    through the rotation.  This pins what the single-query checks of o and dq cannot: the pooled passes of every
+    level (list owners 1, 16, 256, ... groups wide: the group-major pass, and at four levels of 4194304 tokens the list form
+    of the dense kernel for levels 2 and 3), the partial sums placed by inverse positions, their reduction,
     the dense coarsest level, and the fold of the whole chain into the fine dK / dV."""
     import llsa_amd
     from llsa_amd.kernel.torch_op._fused import selection

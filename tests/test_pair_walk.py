@@ -1,5 +1,5 @@
-"""The query-side kernels around 512 groups of eight query blocks, the size of half a round of the chip, at the edges of the topk
-ranges that the list registers have: one register of entries per lane up to 32 entries a row, two up to 64."""
+"""The query-side kernels with one query block a wave, at and just below 512 groups of eight query blocks, where their workgroups fill
+the chip once: topk up to the 64 entries that a wave's list register holds."""
 import pytest
 import torch
 
