@@ -234,7 +234,7 @@ int llsa_transpose_indices_multi(const llsa_transpose_job* jobs, int n_jobs, int
 /* llsa_attn_fwd and llsa_transpose_indices_multi (of the selections the attention reads, the same B and H) in one call.  Jobs that
  * are small enough, and few enough, are made by workgroups of the attention launch, beside its own; otherwise they follow it on the stream. */
 int llsa_attn_fwd_lists(const llsa_attn_fwd_args* a, const llsa_transpose_job* jobs, int n_jobs, void* stream);
-/* Whether they ride in that launch: 1, or 0 if they follow it (topk: of every level, finest first; a job for each). */
+/* Whether they ride in that launch: 1, or 0 if they follow it (topk: of every level, finest first; a job for each); negative: no such shape. */
 int llsa_lists_ride(int B, int H, int N, const int32_t* topk, int levels);
 int llsa_transpose_one_launch(int Mb, int Kb, int T, int B, int H);
 

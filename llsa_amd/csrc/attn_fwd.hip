@@ -442,13 +442,20 @@ static int attn_fwd(const llsa_attn_fwd_args* a, const llsa_transpose_job* jobs,
     return llsa_transpose_indices_multi(jobs, n_jobs, a->B, a->H, stream);
 }
 
+static int check_plan_query(const char* what, int B, int H, int N, const int32_t* topk, int levels) {
+    LLSA_REQUIRE(topk != nullptr && levels >= 1 && levels <= LLSA_MAX_LEVELS, "%s: levels must be 1..%d", what, LLSA_MAX_LEVELS);
+    LLSA_REQUIRE(B > 0 && H > 0 && N > 0 && N % coarsest_multiple(levels) == 0, "%s: bad B/H/N", what);
+    for (int l = 0; l < levels; l++) LLSA_REQUIRE(topk[l] > 0, "%s: topk must be > 0", what);
+    return 0;
+}
+
 extern "C" int llsa_query_blocks_per_wave(int B, int H, int N, const int32_t* topk, int levels, int backward) {
-    LLSA_REQUIRE(B > 0 && H > 0 && N > 0 && topk != nullptr && levels >= 1 && levels <= LLSA_MAX_LEVELS, "query_blocks_per_wave: bad shape");
+    if (const int rc = check_plan_query("query_blocks_per_wave", B, H, N, topk, levels)) return rc;
     return two_blocks_per_wave((int64_t)B * H, N, topk, levels, backward == 0) ? 2 : 1;
 }
 
 extern "C" int llsa_lists_ride(int B, int H, int N, const int32_t* topk, int levels) {
-    LLSA_REQUIRE(B > 0 && H > 0 && N > 0 && topk != nullptr && levels >= 1 && levels <= LLSA_MAX_LEVELS, "lists_ride: bad shape");
+    if (const int rc = check_plan_query("lists_ride", B, H, N, topk, levels)) return rc;
     llsa_transpose_job jobs[LLSA_MAX_LEVELS];
     int32_t* const some = reinterpret_cast<int32_t*>(16);     // (the plan only looks whether there is a list)
     for (int l = 0, m = N / 16; l < levels; l++, m /= 16) jobs[l] = llsa_transpose_job{some, some, some, nullptr, nullptr, m, m, topk[l], 1};

@@ -75,6 +75,11 @@ def test_entry_points_reject_bad_arguments(lib):
     assert lib.attn_bwd_workspace_bytes(2, 6, 16384, topk(16, 16), 2) > 0
     assert lib.attn_bwd_workspace_bytes(1, 1, 262144, topk(16, 16, 16), 3) > lib.attn_bwd_workspace_bytes(1, 1, 262144, topk(16, 16), 2) > 0
     assert lib.attn_bwd_workspace_bytes(2, 6, 16384, topk(16, 16, 16, 16, 16), 5) < 0
+    for ask in (lambda *a: lib.lists_ride(*a), lambda *a: lib.query_blocks_per_wave(*a, 0)):
+        assert ask(2, 6, 16384, topk(16, 16), 2) in (0, 1, 2)
+        for B, H, N, t, levels in ((0, 1, 1024, topk(8), 1), (1, 1, 32, topk(8), 1), (1, 1, 1000, topk(8), 1), (1, 1, 1024, None, 1), (1, 1, 1024, topk(0), 1),
+                                   (1, 1, 4096, topk(8, 8), 2), (1, 1, 1024, topk(8), 0), (1, 1, 16384, topk(8, 8, 8, 8, 8), 5)):
+            assert ask(B, H, N, t, levels) < 0
     # a token count the coarsest level cannot tile is an error, not a division by zero in the work split
     assert lib.attn_bwd_workspace_bytes(1, 1, 512, topk(8), 1) < 0
     assert lib.attn_bwd_workspace_bytes(1, 1, 4096, topk(8, 8), 2) < 0
