@@ -11,8 +11,6 @@
 //
 // The order is total -- higher score first, equal scores by smaller key index -- so the result does not depend on how the
 // work is split.
-#include <numeric>
-#include <algorithm>
 #include "llsa_device.h"
 #include "llsa_host.h"
 #include "../../include/llsa_hip.h"
@@ -309,22 +307,23 @@ __global__ __launch_bounds__(64 * W) void topk_dense_kernel(const bf16* __restri
     write_winners<W>(win, n_win, T, out + ((int64_t)bh * n + q0) * T, T, tid, wide_index);
 }
 
-// Dense selection for longer rows: the keys stream by, and only those that can still be among a row's T best are kept.
-// A wave owns sixteen rows (PARTS = 1) or a quarter of the keys of sixteen rows (PARTS = 4, for grids too small to fill the chip
-// otherwise).  Every row has a buffer
-// of kBuf keys in LDS and a threshold; a tile whose scores all lie below their rows' thresholds costs a handful of
-// instructions, the others append what passes.  When a buffer is nearly full the wave cuts all sixteen back to little more
-// than their T best, which also raises the thresholds.  In a stream of random order about T ln(n / T) keys of a row pass, in one
-// whose neighbours are alike more, so the tiles are taken in steps of 0.62 of the row of tiles.  What bounds the kernel is a wave's chain of
-// instructions and LDS round trips for the tiles that pass (a third of them at 4096 keys, T = 8) and three cuts; so the waves do not
-// wait for each other: key tiles shared through LDS cost a barrier per four tiles, at which three waves waited for the one with a
-// cut (37 % of the time).  8 x 4096 rows of 4096 keys 156 -> 137 us, 12 x 4096 290 -> 197, 16 x 2048 of 2048 110 -> 82; a quarter of
-// the keys per wave, 5 x 3072 77 -> 71.  (Four tiles on their way, places in the buffers by lane swaps instead of an LDS counter: the same.)
+// Dense selection for longer rows: two looks at all scores, and between them a bound of every row's T-th best.
+//  * First look: the largest score of each of G groups of a row's keys.  The T-th largest of those is a bound: at least T keys reach
+//    it, and few more do if the groups are many and neighbours, which score alike, fall into different ones.  So a group is a
+//    position among the sixteen keys of a tile, by wave (a tile in four) and, for T > 16, by a further one or two bits of the tile: 64
+//    consecutive keys, which are a patch of 8 x 8 on image-like data, are in 64 groups.
+//  * Second look: the keys that reach the bound go to their row's buffer in LDS, and the T best of those are ranked.
+// A workgroup is 16 RT rows, and its four waves take every fourth key tile of the row each, four tiles on their way to registers while four are worked
+// on.  What bounds it is the rate at which key tiles come out of the L2 -- each is read once per workgroup and look, hence many
+// rows a workgroup where the grid is large -- and the chain through LDS for the tiles that hold a key that passes.
+// A row whose bound lets more than kBuf keys through (ties; a period of the image that puts the best keys into few groups) has its bound
+// moved up by bisection, a look at all scores per step, at most one step per bit of a key, for no two keys of a row are equal.
 // Key: the 32-bit packed key (scores rounded to bf16, n <= kMaxPackedKeys) or the 64-bit wide key.
-// (A T-step arg-max over chunks of 512 keys per row took 1480 us for 8 x 4096 rows of 4096 keys, T = 8.)
-constexpr int kBuf = 128, kBufFull = kBuf - 16;   // a tile adds at most 16 keys to a row
+// (8 x 4096 rows of 4096 keys, T = 8: 72 us, T = 64 151.  A T-step arg-max over chunks of 512
+// keys per row 1480; a running threshold per row, raised whenever a buffer was full, by a wave for itself 128 and 183, with key tiles
+// shared through LDS behind barriers 157.  5 x 3072, T = 16: 69 -> 38;  1 x 4096, T = 32: 57 -> 43;  1 x 1088, T = 8: 21 -> 17.)
 constexpr int kStreamWaves = 4;
-constexpr int kAhead = 2;                         // key tiles on their way to a wave while as many are worked on
+constexpr int kAhead = 4;                         // key tiles on their way to a wave while as many are worked on
 
 template <typename Key>
 struct StreamKey;
@@ -332,6 +331,9 @@ template <>
 struct StreamKey<unsigned> {
     static __device__ __forceinline__ unsigned make(float s, int idx, bool) { return packed_key(s, idx); }
     static __device__ __forceinline__ unsigned long long wide(unsigned k) { return wide_key(k & 0xFFFF0000u, 0xFFFF - (int)(k & 0xFFFFu)); }
+    // the smallest and the largest key a score (given as ordered key of the score before rounding) can make
+    static __device__ __forceinline__ unsigned least(unsigned score, bool) { return ordered_key(rn_bf16(key_score(score))) & 0xFFFF0000u; }
+    static __device__ __forceinline__ unsigned most(unsigned score, bool r) { return least(score, r) | 0xFFFFu; }
     // a score below this cannot make a key of at least t: one bf16 step below t's score
     static __device__ __forceinline__ unsigned score_bits(unsigned t) { return t & 0xFFFF0000u; }
 };
@@ -341,6 +343,10 @@ struct StreamKey<unsigned long long> {
         return wide_key(ordered_key(round ? rn_bf16(s) : s), idx);
     }
     static __device__ __forceinline__ unsigned long long wide(unsigned long long k) { return k; }
+    static __device__ __forceinline__ unsigned long long least(unsigned score, bool round) {
+        return (unsigned long long)(round ? ordered_key(rn_bf16(key_score(score))) : score) << 32;
+    }
+    static __device__ __forceinline__ unsigned long long most(unsigned score, bool round) { return least(score, round) | 0xFFFFFFFFull; }
     static __device__ __forceinline__ unsigned score_bits(unsigned long long t) { return (unsigned)(t >> 32) & 0xFFFF0000u; }
 };
 // The largest float that is certainly below (or rounds below) the score of key bits `k` (its low 16 bits are zero).
@@ -351,162 +357,254 @@ __device__ __forceinline__ float score_floor(unsigned k) {
     const float f = __uint_as_float(b);
     return (f != f) ? -INFINITY : f;
 }
+__device__ __forceinline__ float largest(const f32x4& s) { return fmaxf(fmaxf(s[0], s[1]), fmaxf(s[2], s[3])); }
 
-template <typename Key, int PARTS>
+// RT: sixteens of rows per workgroup (n is a multiple of 16 RT); SETS: groups per row / 64
+template <typename Key, int RT, int SETS>
 __global__ __launch_bounds__(64 * kStreamWaves) void topk_stream_kernel(const bf16* __restrict__ pq, const bf16* __restrict__ pk,
-                                                                        int* __restrict__ out, int n, int T, int round_scores, int step) {
-    constexpr int kE = kBuf / 4;                              // keys of a row's buffer per lane
-    // a wave's buffers; at the end a row tile's winners take their place
-    constexpr int kKeys = 16 * (kBuf + 1), kWide = 16 * kWinStride, kPer = sizeof(Key) == 8 ? kKeys : (kKeys + 1) / 2 > kWide ? (kKeys + 1) / 2 : kWide;
-    __shared__ unsigned long long space[kStreamWaves][kPer];
-    __shared__ int cnt[kStreamWaves][16];
-    __shared__ int n_win[kStreamWaves / PARTS][16];
-    __shared__ RowShare<PARTS> share;
+                                                                        int* __restrict__ out, int n, int T, int round_scores) {
+    static_assert(RT == 1 || RT == 2 || RT == 4, "the waves are dealt to the row tiles");
+    static_assert(kAhead % SETS == 0, "a tile's set of groups is known at compile time");
+    constexpr int W = kStreamWaves, kPer = W / RT;            // waves per row tile where the rows are finished
+    constexpr int kRows = 16 * RT, kGroups = 64 * SETS;
+    constexpr bool kWide = sizeof(Key) == 8;                  // (the buffers in 64 KB of LDS)
+    constexpr int kBuf = RT == 4 ? (kWide ? 96 : 128) : SETS < 4 ? 128 : (kWide && RT == 2) ? 224 : 256;
+    // one piece of LDS, for the groups' largest scores, then the rows' buffers, then what is ranked
+    constexpr int kBytesGroups = kRows * (kGroups + 1) * 4, kBytesBuf = kRows * (kBuf + 1) * (int)sizeof(Key), kBytesWin = kRows * kWinStride * 8;
+    constexpr int kBytes = kBytesGroups > kBytesBuf ? (kBytesGroups > kBytesWin ? kBytesGroups : kBytesWin)
+                                                    : (kBytesBuf > kBytesWin ? kBytesBuf : kBytesWin);
+    __shared__ unsigned long long space[(kBytes + 7) / 8];
+    __shared__ Key bound[kRows], ceiling[kRows];
+    __shared__ int cnt[kRows], n_win[RT][16], part[W][kRows];
+    unsigned (*const groups)[kGroups + 1] = reinterpret_cast<unsigned (*)[kGroups + 1]>(space);
+    Key (*const buf)[kBuf + 1] = reinterpret_cast<Key (*)[kBuf + 1]>(space);
+    unsigned long long (*const win)[16][kWinStride] = reinterpret_cast<unsigned long long (*)[16][kWinStride]>(space);
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), quad = lane >> 4, r = lane & 15;
-    const int part = PARTS == 1 ? 0 : wave, rowt = PARTS == 1 ? wave : 0;
-    const int bh = blockIdx.y, q0 = blockIdx.x * (PARTS == 1 ? 64 : 16) + rowt * 16;      // n is a multiple of 64 where PARTS == 1
+    const int lid = xcd_logical_id();                         // (a (b,h)'s keys on one XCD)
+    const int bh = lid / (int)gridDim.x, q0 = lid % (int)gridDim.x * kRows;
     const bf16* pqb = pq + ((int64_t)bh * n + q0) * kD;
-    const bf16* pkb = pk + (int64_t)bh * n * kD;
-    if (lane < 16) cnt[wave][lane] = 0;
-    if (lane < 16 && part == 0) n_win[rowt][lane] = 0;
-    bf16x8 bq[2];
-    bq[0] = ld16(pqb + r * kD + quad * 8);
-    bq[1] = ld16(pqb + r * kD + quad * 8 + 32);
-    Key tau = 1;                                              // keys below it are not among the row's T best
-    float low = -INFINITY;                                    // scores below it do not make such a key
-    Key (*const my)[kBuf + 1] = reinterpret_cast<Key (*)[kBuf + 1]>(space[wave]);
-    unsigned long long (*const win)[kWinStride] = reinterpret_cast<unsigned long long (*)[kWinStride]>(space[rowt]);
-    auto settle = [&]() __attribute__((always_inline)) {      // LDS of this wave: all writes land before what follows reads
-        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-        __builtin_amdgcn_wave_barrier();
-    };
-    settle();
-
-    // cuts every row's buffer back to its T best keys
-    auto cut = [&]() __attribute__((always_inline)) {
-        settle();
-        const int have = cnt[wave][r];
-        Key key[kE], top = 0;
+    const bf16* pkb = pk + (int64_t)bh * n * kD + r * kD + quad * 8;
+    const int tiles = n / 16;
+    const bool round = round_scores != 0;
+    bf16x8 bq[RT][2];
 #pragma unroll
-        for (int i = 0; i < kE; i++) {
+    for (int rt = 0; rt < RT; rt++) {
+        bq[rt][0] = ld16(pqb + (rt * 16 + r) * kD + quad * 8);
+        bq[rt][1] = ld16(pqb + (rt * 16 + r) * kD + quad * 8 + 32);
+    }
+    // A look at all scores: see(s, i, tile) gets the scores of all row tiles against a key tile of this wave's, i (known at compile
+    // time) = its place among the wave's tiles modulo kAhead
+    auto look = [&](auto&& see) __attribute__((always_inline)) {
+        struct Tiles { bf16x8 k[kAhead][2]; } ta, tb;
+        auto load = [&](Tiles& o, int t) __attribute__((always_inline)) {
+#pragma unroll
+            for (int i = 0; i < kAhead; i++) {
+                const bf16* p = pkb + (int64_t)min(t + i * W, tiles - 1) * 16 * kD;
+                o.k[i][0] = ld16(p);
+                o.k[i][1] = ld16(p + 32);
+            }
+        };
+        auto work = [&](const Tiles& o, int t) __attribute__((always_inline)) {
+#pragma unroll
+            for (int i = 0; i < kAhead; i++) {
+                if (t + i * W < tiles) {
+                    f32x4 s[RT];
+#pragma unroll
+                    for (int rt = 0; rt < RT; rt++) {
+                        f32x4 z = {0.f, 0.f, 0.f, 0.f};
+                        s[rt] = mfma_bf16(o.k[i][1], bq[rt][1], mfma_bf16(o.k[i][0], bq[rt][0], z));
+                    }
+                    see(s, i, t + i * W);
+                }
+            }
+        };
+        constexpr int kStep = kAhead * W;
+        load(ta, wave);
+        for (int t = wave; t < tiles; t += 2 * kStep) {
+            load(tb, t + kStep);
+            work(ta, t);
+            load(ta, t + 2 * kStep);
+            work(tb, t + kStep);
+        }
+    };
+
+    // ---- the groups' largest scores
+    f32x4 most[RT][SETS];
+#pragma unroll
+    for (int rt = 0; rt < RT; rt++)
+#pragma unroll
+        for (int g = 0; g < SETS; g++) most[rt][g] = f32x4{-INFINITY, -INFINITY, -INFINITY, -INFINITY};
+    look([&](const f32x4 (&s)[RT], int i, int) __attribute__((always_inline)) {
+#pragma unroll
+        for (int rt = 0; rt < RT; rt++)
+#pragma unroll
+            for (int e = 0; e < 4; e++) most[rt][i % SETS][e] = fmaxf(most[rt][i % SETS][e], s[rt][e]);
+    });
+    if (tid < kRows) cnt[tid] = 0;
+    if (tid < 16 * RT) n_win[tid / 16][tid % 16] = 0;
+#pragma unroll
+    for (int rt = 0; rt < RT; rt++)
+#pragma unroll
+        for (int g = 0; g < SETS; g++)
+#pragma unroll
+            for (int e = 0; e < 4; e++) groups[rt * 16 + r][((wave * SETS + g) * 4 + e) * 4 + quad] = ordered_key(most[rt][g][e]);
+    __syncthreads();
+    const int own_rt = wave / kPer;                           // the row tile this wave finishes, if it is the first of that tile's waves
+    const bool finishes = wave % kPer == 0;
+    if (finishes) {
+        unsigned key[kGroups / 4], top;
+#pragma unroll
+        for (int i = 0; i < kGroups / 4; i++) key[i] = groups[own_rt * 16 + r][i * 4 + quad];
+        int turn = 0, n_ge;
+        const unsigned lo = row_bound<kGroups / 16, 1>(key, kGroups / 16, T, top, (RowShare<1>*)nullptr, turn, 0, lane);
+        const unsigned t = row_threshold<kGroups / 4, 1>(key, T, lo, top, (RowShare<1>*)nullptr, turn, 0, lane, n_ge);
+        // (a group without a number has the score -infinity, and below that there are keys yet: those of NaNs)
+        if (quad == 0) {
+            bound[own_rt * 16 + r] = t <= ordered_key(-INFINITY) ? (Key)1 : StreamKey<Key>::least(t, round);
+            ceiling[own_rt * 16 + r] = StreamKey<Key>::most(top, round);
+        }
+    }
+    __syncthreads();
+
+    // ---- the keys that reach the bound
+    Key tau[RT];                                              // keys below it are not among the row's T best
+    float low[RT];                                            // scores below it do not make such a key
+    auto set_bounds = [&](int rt, Key t) __attribute__((always_inline)) {
+        tau[rt] = t;
+        low[rt] = score_floor(StreamKey<Key>::score_bits(t));
+    };
+    auto collect = [&]() __attribute__((always_inline)) {
+        look([&](const f32x4 (&s)[RT], int, int tile) __attribute__((always_inline)) {
+            bool pass[RT], any = false;
+#pragma unroll
+            for (int rt = 0; rt < RT; rt++) {
+                pass[rt] = !(largest(s[rt]) < low[rt]);       // (a NaN passes: it has to be able to fill a row that has nothing better)
+                any |= pass[rt];
+            }
+            if (__ballot(any) == 0) return;
+#pragma unroll
+            for (int rt = 0; rt < RT; rt++) {
+                if (!pass[rt]) continue;
+                Key k[4];
+                int mine = 0;
+#pragma unroll
+                for (int e = 0; e < 4; e++) {
+                    k[e] = StreamKey<Key>::make(s[rt][e], tile * 16 + 4 * quad + e, round);
+                    mine += k[e] >= tau[rt] ? 1 : 0;
+                }
+                if (mine > 0) {
+                    int slot = atomicAdd(&cnt[rt * 16 + r], mine);
+#pragma unroll
+                    for (int e = 0; e < 4; e++)
+                        if (k[e] >= tau[rt]) buf[rt * 16 + r][min(slot++, kBuf)] = k[e];
+                }
+            }
+        });
+    };
+#pragma unroll
+    for (int rt = 0; rt < RT; rt++) set_bounds(rt, bound[rt * 16 + r]);
+    collect();
+    __syncthreads();
+    bool over = false;
+#pragma unroll
+    for (int rt = 0; rt < RT; rt++) over |= cnt[rt * 16 + r] > kBuf;
+    if (__ballot(over) != 0) {                                // (the same in all waves)
+        Key lo[RT], hi[RT], mid[RT];
+        int c_lo[RT];
+#pragma unroll
+        for (int rt = 0; rt < RT; rt++) {
+            lo[rt] = tau[rt];
+            hi[rt] = ceiling[rt * 16 + r] + 1;                // (below the largest integer)
+            c_lo[rt] = cnt[rt * 16 + r];
+        }
+        for (int step = 0;; step++) {
+            bool open = false;
+#pragma unroll
+            for (int rt = 0; rt < RT; rt++) {
+                const Key half = lo[rt] + ((hi[rt] - lo[rt]) >> 1), of_score = middle_key(lo[rt], hi[rt]);
+                const bool on = c_lo[rt] > kBuf && hi[rt] - lo[rt] > 1;
+                mid[rt] = !on ? lo[rt] : (step < kScoreSteps && of_score > lo[rt] && of_score < hi[rt]) ? of_score : half;
+                open |= on;
+            }
+            if (__ballot(open) == 0) break;                   // (the same in all waves: so are the counts)
+            int c[RT];
+            float floor[RT];
+#pragma unroll
+            for (int rt = 0; rt < RT; rt++) {
+                c[rt] = 0;
+                floor[rt] = score_floor(StreamKey<Key>::score_bits(mid[rt]));
+            }
+            look([&](const f32x4 (&s)[RT], int, int tile) __attribute__((always_inline)) {
+#pragma unroll
+                for (int rt = 0; rt < RT; rt++) {
+                    if (largest(s[rt]) < floor[rt]) continue;
+#pragma unroll
+                    for (int e = 0; e < 4; e++) c[rt] += StreamKey<Key>::make(s[rt][e], tile * 16 + 4 * quad + e, round) >= mid[rt] ? 1 : 0;
+                }
+            });
+            __syncthreads();                                  // (the counts of the step before have been read)
+#pragma unroll
+            for (int rt = 0; rt < RT; rt++) {
+                c[rt] = quad_sum_i(c[rt]);
+                if (quad == 0) part[wave][rt * 16 + r] = c[rt];
+            }
+            __syncthreads();
+#pragma unroll
+            for (int rt = 0; rt < RT; rt++) {
+                int sum = 0;
+#pragma unroll
+                for (int w = 0; w < W; w++) sum += part[w][rt * 16 + r];
+                if (mid[rt] == lo[rt]) continue;              // (decided)
+                if (sum >= T) {
+                    lo[rt] = mid[rt];
+                    c_lo[rt] = sum;
+                } else {
+                    hi[rt] = mid[rt];
+                }
+            }
+        }
+        __syncthreads();
+        if (tid < kRows) cnt[tid] = 0;
+        __syncthreads();
+#pragma unroll
+        for (int rt = 0; rt < RT; rt++) set_bounds(rt, lo[rt]);
+        collect();
+        __syncthreads();
+    }
+
+    // ---- little more than the T best of a row's buffer, and those ranked
+    Key key[kBuf / 4], t = 1;
+    if (finishes) {
+        const int have = min(cnt[own_rt * 16 + r], kBuf);
+        Key top = 0, least = 0;
+#pragma unroll
+        for (int i = 0; i < kBuf / 4; i++) {
             const int at = i * 4 + quad;
-            key[i] = at < have ? my[r][at] : (Key)0;
+            key[i] = at < have ? buf[own_rt * 16 + r][at] : (Key)0;
             top = key[i] > top ? key[i] : top;
         }
-        top = quad_max_u(top);
-        int turn = 0, n_ge;
-        // (a row that has fewer than T keys keeps them all)
-        const Key t = row_threshold<kE, 1, Key>(key, min(T, have), tau, top > tau ? top : tau, (RowShare<1>*)nullptr, turn, 0, lane, n_ge);
+#pragma unroll
+        for (int rt = 0; rt < RT; rt++) least = rt == own_rt ? tau[rt] : least;
+        t = least;                                            // (all of them, where they are few enough to be ranked)
+        if (__ballot(have > kWin) != 0) {
+            top = quad_max_u(top);
+            int turn = 0, n_ge;
+            t = row_threshold<kBuf / 4, 1, Key>(key, T, least, top, (RowShare<1>*)nullptr, turn, 0, lane, n_ge);
+        }
+    }
+    __syncthreads();                                          // (the buffers have been read: what is ranked takes their place)
+    if (finishes) {
         int mine = 0;
 #pragma unroll
-        for (int i = 0; i < kE; i++) mine += key[i] >= t ? 1 : 0;
-        settle();
-        if (lane < 16) cnt[wave][lane] = 0;
-        settle();
-        int slot = mine > 0 ? atomicAdd(&cnt[wave][r], mine) : 0;
+        for (int i = 0; i < kBuf / 4; i++) mine += key[i] >= t ? 1 : 0;
+        int slot = mine > 0 ? atomicAdd(&n_win[own_rt][r], mine) : 0;
         const Key t2 = compare_again(t, slot);
 #pragma unroll
-        for (int i = 0; i < kE; i++)
-            if (key[i] >= t2) my[r][min(slot++, kBuf)] = key[i];
-        if (have >= T) {
-            tau = t;
-            low = score_floor(StreamKey<Key>::score_bits(t));
-        }
-        settle();
-    };
-    auto take = [&](const f32x4 s, int key0) __attribute__((always_inline)) {      // the scores of one key tile
-        // (a NaN passes the test -- it has to be able to fill a row that has nothing better)
-        const bool any = !(fmaxf(fmaxf(s[0], s[1]), fmaxf(s[2], s[3])) < low);
-        if (__ballot(any) == 0) return;
-        Key k[4];
-        int mine = 0;
-#pragma unroll
-        for (int e = 0; e < 4; e++) {
-            k[e] = StreamKey<Key>::make(s[e], key0 + 4 * quad + e, round_scores != 0);
-            mine += k[e] >= tau ? 1 : 0;
-        }
-        int slot = 0;
-        if (mine > 0) {
-            slot = atomicAdd(&cnt[wave][r], mine);
-            const int full = slot + mine;
-#pragma unroll
-            for (int e = 0; e < 4; e++)
-                if (k[e] >= tau) my[r][min(slot++, kBuf)] = k[e];
-            slot = full;
-        }
-        if (__ballot(slot > kBufFull) != 0) cut();
-    };
-
-    // key tiles straight into registers, kAhead on their way while as many are worked on
-    const int tiles = n / 16;
-    const bf16* p = pkb + r * kD + quad * 8;
-    int t_load = (int)((int64_t)part * step % tiles), t_work = t_load;
-    const int hop = (int)((int64_t)PARTS * step % tiles);
-    auto after = [&](int t) __attribute__((always_inline)) { return t + hop - (t + hop >= tiles ? tiles : 0); };
-    struct Tiles { bf16x8 k[kAhead][2]; } ta, tb;
-    auto load = [&](Tiles& o) __attribute__((always_inline)) {
-#pragma unroll
-        for (int i = 0; i < kAhead; i++) {
-            o.k[i][0] = ld16(p + (int64_t)t_load * 16 * kD);
-            o.k[i][1] = ld16(p + (int64_t)t_load * 16 * kD + 32);
-            t_load = after(t_load);
-        }
-    };
-    int left = (tiles - part + PARTS - 1) / PARTS;            // tiles this wave still has to look at
-    auto work = [&](const Tiles& o) __attribute__((always_inline)) {
-        f32x4 s[kAhead];
-#pragma unroll
-        for (int i = 0; i < kAhead; i++) {
-            f32x4 z = {0.f, 0.f, 0.f, 0.f};
-            s[i] = mfma_bf16(o.k[i][1], bq[1], mfma_bf16(o.k[i][0], bq[0], z));
-        }
-#pragma unroll
-        for (int i = 0; i < kAhead; i++) {
-            if (i < left) take(s[i], t_work * 16);
-            t_work = after(t_work);
-        }
-        left -= kAhead;
-    };
-    load(ta);
-    while (left > 0) {
-        load(tb);
-        work(ta);
-        load(ta);
-        if (left > 0) work(tb);
+        for (int i = 0; i < kBuf / 4; i++)
+            if (key[i] >= t2) win[own_rt][r][min(slot++, kWin)] = StreamKey<Key>::wide(key[i]);
     }
-    cut();
-    // at most T + kSpare keys are left in this wave's buffer of every row (all of its keys if it saw fewer)
-    const int have = cnt[wave][r];
-    Key key[kWin / 4], top = 0;
-#pragma unroll
-    for (int i = 0; i < kWin / 4; i++) {
-        const int at = i * 4 + quad;
-        key[i] = at < have ? my[r][at] : (Key)0;
-        top = key[i] > top ? key[i] : top;
-    }
-    Key t = 1;
-    if (PARTS > 1) {                                          // little more than the T best of the parts' keys
-        __shared__ Key tops[PARTS][16];
-        top = quad_max_u(top);
-        if (lane < 16) tops[wave][lane] = top;
-        __syncthreads();
-        for (int w = 0; w < PARTS; w++) top = tops[w][r] > top ? tops[w][r] : top;
-        int turn = 0, n_ge;
-        t = row_threshold<kWin / 4, PARTS, Key>(key, T, (Key)1, top, &share, turn, wave, lane, n_ge);
-    }
-    int mine = 0;
-#pragma unroll
-    for (int i = 0; i < kWin / 4; i++) mine += key[i] >= t ? 1 : 0;
     __syncthreads();
-    int slot = mine > 0 ? atomicAdd(&n_win[rowt][r], mine) : 0;
-    const Key t2 = compare_again(t, slot);
-#pragma unroll
-    for (int i = 0; i < kWin / 4; i++)
-        if (key[i] >= t2) win[r][min(slot++, kWin)] = StreamKey<Key>::wide(key[i]);
-    __syncthreads();
-    int* o = out + ((int64_t)bh * n + q0) * T;
-    if (PARTS == 1) write_winners<1>(win, n_win[rowt], T, o, T, lane, wide_index);
-    else write_winners<kStreamWaves>(win, n_win[0], T, o, T, tid, wide_index);
+    write_winners<kPer>(win[own_rt], n_win[own_rt], T, out + ((int64_t)bh * n + q0 + own_rt * 16) * T, T, tid % (64 * kPer), wide_index);
 }
 
 // Parent-guided selection: 16 sibling rows per workgroup against the 16 * T2 tokens under their parent's T2 blocks, W waves
@@ -686,16 +784,27 @@ extern "C" int llsa_topk_dense(const void* pq, const void* pk, int32_t* out_idx,
         else LLSA_DENSE(16, 4);
 #undef LLSA_DENSE
     } else {
-        // one wave per sixteen rows while that fills the chip twice over (1024 SIMDs), four waves with a quarter of the keys each below
+        // Rows per workgroup: sixteen while every workgroup has a CU of its own, 32 while half of them do, else 64 (32 beyond T = 32, whose
+        // groups and buffers are larger): a workgroup reads the row of keys twice, whatever it has rows.  us with 16 / 32 / 64 rows, T = 8:
+        //   128 row tiles (2048 keys) 21 / 23 / 26;  256 (4096) 36 / 37 / 40;  400 (1280) 30 / 19 / 23;  512 (4096) 66 / 38 / 41;  512 (2048) 38 / 23 / 28
+        //   544 (1088) 43 / 30 / 23;  576 (3072) 74 / 52 / 34;  1024 (2048) 71 / 39 / 28;  2048 (4096) 243 / 130 / 72
+        // T = 32: 256 (4096) 43 / 46 / 58;  512 (4096) 74 / 49 / 58;  544 (1088) 50 / 37 / 41;  576 (3072) 81 / 58 / 50;  2048 (4096) 251 / 139 / 90
+        const int64_t tiles = (int64_t)n / 16 * B * H;        // sixteens of rows
+        const int rt = tiles <= 256 || n % 32 != 0 ? 1 : tiles <= 512 || n % 64 != 0 || T > 32 ? 2 : 4;
+#define LLSA_STREAM(KEY, RT, SETS)                                                                                                              \
+    hipLaunchKernelGGL(HIP_KERNEL_NAME(topk_stream_kernel<KEY, RT, SETS>), dim3(n / (16 * RT), B * H), dim3(64 * kStreamWaves), 0, st, q, k, out_idx, n, T, \
+                       round_scores)
         const bool wide = !round_scores || n > kMaxPackedKeys;
-        const bool whole = n % 64 == 0 && (int64_t)n / 16 * B * H >= 2048;
-        const dim3 grid(whole ? n / 64 : n / 16, B * H), block(64 * kStreamWaves);
-        int step = (int)(0.618 * (n / 16));                   // (without a common divisor, so that every tile has its turn)
-        while (std::gcd(step, n / 16) != 1) step++;
-        if (whole && !wide) hipLaunchKernelGGL(HIP_KERNEL_NAME(topk_stream_kernel<unsigned, 1>), grid, block, 0, st, q, k, out_idx, n, T, round_scores, step);
-        else if (whole) hipLaunchKernelGGL(HIP_KERNEL_NAME(topk_stream_kernel<unsigned long long, 1>), grid, block, 0, st, q, k, out_idx, n, T, round_scores, step);
-        else if (!wide) hipLaunchKernelGGL(HIP_KERNEL_NAME(topk_stream_kernel<unsigned, 4>), grid, block, 0, st, q, k, out_idx, n, T, round_scores, step);
-        else hipLaunchKernelGGL(HIP_KERNEL_NAME(topk_stream_kernel<unsigned long long, 4>), grid, block, 0, st, q, k, out_idx, n, T, round_scores, step);
+        if (wide && rt == 1) LLSA_STREAM(unsigned long long, 1, 4);
+        else if (wide && rt == 2) LLSA_STREAM(unsigned long long, 2, 4);
+        else if (wide) LLSA_STREAM(unsigned long long, 4, 2);
+        else if (rt == 1 && T <= 16) LLSA_STREAM(unsigned, 1, 1);
+        else if (rt == 1) LLSA_STREAM(unsigned, 1, 4);
+        else if (rt == 2 && T <= 16) LLSA_STREAM(unsigned, 2, 1);
+        else if (rt == 2) LLSA_STREAM(unsigned, 2, 4);
+        else if (T <= 16) LLSA_STREAM(unsigned, 4, 1);
+        else LLSA_STREAM(unsigned, 4, 2);
+#undef LLSA_STREAM
     }
     return launch_status("topk_dense");
 }
