@@ -43,7 +43,7 @@ extern "C" {
 #define LLSA_DTYPE_BF16 0
 #define LLSA_DTYPE_F32 1
 
-#define LLSA_ABI_VERSION 209     /* changes with every change of a signature or argument structure below */
+#define LLSA_ABI_VERSION 210     /* changes with every change of a signature or argument structure below */
 int llsa_version(void);          /* LLSA_ABI_VERSION of the built library                                    */
 const char* llsa_last_error_string(void);
 
@@ -160,6 +160,14 @@ int llsa_topk_sparse(const void* pq, const void* pk, const int32_t* parent_idx, 
 int llsa_topk_cascade(const void* pq_parent, const void* pk_parent, int32_t* parent_out, const void* pq, const void* pk,
                       int32_t* out_idx, int B, int H, int N1, int T, int T2, void* stream);
 int llsa_topk_cascade_max_parents(void);
+/* The same selections with the keys as R tiles of sixteen rows (llsa_pool_item: y1r, y2r; 1024 elements a tile, the sixteen rows'
+ * own place) instead of rows: the same results, and loads of whole kilobytes. */
+int llsa_topk_dense_tiles(const void* pq, const void* pk_tiles, int32_t* out_idx, int B, int H, int n, int T,
+                          int round_scores, void* stream);
+int llsa_topk_sparse_tiles(const void* pq, const void* pk_tiles, const int32_t* parent_idx, int32_t* out_idx,
+                           int B, int H, int N1, int T, int T2, void* stream);
+int llsa_topk_cascade_tiles(const void* pq_parent, const void* pk_parent_tiles, int32_t* parent_out, const void* pq, const void* pk_tiles,
+                            int32_t* out_idx, int B, int H, int N1, int T, int T2, void* stream);
 
 /* ------------------------------------------------------------------------------------------
  * The hierarchy.  Pooled level l = 1 .. levels: its tokens are means of 16^l input tokens and weigh

@@ -95,9 +95,9 @@ auto in_engine(Fn fn) {
 struct Library {
     decltype(&llsa_last_error_string) last_error_string;
     decltype(&llsa_pool_pyramid_fwd) pool_pyramid_fwd;
-    decltype(&llsa_topk_dense) topk_dense;
-    decltype(&llsa_topk_sparse) topk_sparse;
-    decltype(&llsa_topk_cascade) topk_cascade;
+    decltype(&llsa_topk_dense_tiles) topk_dense_tiles;
+    decltype(&llsa_topk_sparse_tiles) topk_sparse_tiles;
+    decltype(&llsa_topk_cascade_tiles) topk_cascade_tiles;
     decltype(&llsa_topk_cascade_max_parents) topk_cascade_max_parents;
     decltype(&llsa_attn_fwd) attn_fwd;
     decltype(&llsa_attn_fwd_lists) attn_fwd_lists;
@@ -114,9 +114,9 @@ struct Library {
         auto get = [&](const char* name, auto& fn) { fn = reinterpret_cast<std::decay_t<decltype(fn)>>(at_.at(name)); };
         get("llsa_last_error_string", last_error_string);
         get("llsa_pool_pyramid_fwd", pool_pyramid_fwd);
-        get("llsa_topk_dense", topk_dense);
-        get("llsa_topk_sparse", topk_sparse);
-        get("llsa_topk_cascade", topk_cascade);
+        get("llsa_topk_dense_tiles", topk_dense_tiles);
+        get("llsa_topk_sparse_tiles", topk_sparse_tiles);
+        get("llsa_topk_cascade_tiles", topk_cascade_tiles);
         get("llsa_topk_cascade_max_parents", topk_cascade_max_parents);
         get("llsa_attn_fwd", attn_fwd);
         get("llsa_attn_fwd_lists", attn_fwd_lists);
@@ -235,8 +235,9 @@ struct Layout {
             return at;
         };
         for (int l = 1; l <= L; l++) pq[l] = take(n[l] * 128);
-        for (int l = 1; l <= L; l++) pk[l] = take(n[l] * 128);
-        for (int l = 1; l <= L; l++) pv[l] = take(n[l] * 128);
+        // (the selection reads the keys as tiles: rows of k and v are wanted only where the next pooling pass starts from them)
+        for (int l = 1; l <= L; l++) pk[l] = take(n[l] * 128, l % 2 == 0 && l < L);
+        for (int l = 1; l <= L; l++) pv[l] = take(n[l] * 128, l % 2 == 0 && l < L);
         qr = take(n[1] * 2048);
         kr = take(n[1] * 2048);
         vr = take(n[1] * 2048);
@@ -477,17 +478,17 @@ Tensor attend(const std::shared_ptr<Library>& lib, const Tensor& q_in, const Ten
         if (L >= 2 && n[L] <= lib->topk_cascade_max_parents() && (n[L] <= 64 || B * H * n[L] < 2048)) {
             // the dense selection rides in the workgroups of the first parent-guided one: one launch less (more than 64
             // parent tokens in a large grid: sixteen rows a wave side by side in a launch of their own are cheaper)
-            lib->check(lib->topk_cascade(pa(y.pq[L]), pa(y.pk[L]), ints(y.sel[L - 1]), pa(y.pq[L - 1]), pa(y.pk[L - 1]), ints(y.sel[L - 2]), b, h,
-                                         static_cast<int>(n[L - 1]), y.topk[L - 2], y.topk[L - 1], stream),
+            lib->check(lib->topk_cascade_tiles(pa(y.pq[L]), pa(y.pkr[L]), ints(y.sel[L - 1]), pa(y.pq[L - 1]), pa(y.pkr[L - 1]), ints(y.sel[L - 2]), b, h,
+                                               static_cast<int>(n[L - 1]), y.topk[L - 2], y.topk[L - 1], stream),
                        "topk_cascade");
             first = L - 2;
         } else {
-            lib->check(lib->topk_dense(pa(y.pq[L]), pa(y.pk[L]), ints(y.sel[L - 1]), b, h, static_cast<int>(n[L]), y.topk[L - 1], 1, stream),
+            lib->check(lib->topk_dense_tiles(pa(y.pq[L]), pa(y.pkr[L]), ints(y.sel[L - 1]), b, h, static_cast<int>(n[L]), y.topk[L - 1], 1, stream),
                        "gen_sparse_indices");
         }
         for (int l = first; l > 0; l--)
-            lib->check(lib->topk_sparse(pa(y.pq[l]), pa(y.pk[l]), ints(y.sel[l]), ints(y.sel[l - 1]), b, h, static_cast<int>(n[l]), y.topk[l - 1],
-                                        y.topk[l], stream),
+            lib->check(lib->topk_sparse_tiles(pa(y.pq[l]), pa(y.pkr[l]), ints(y.sel[l]), ints(y.sel[l - 1]), b, h, static_cast<int>(n[l]), y.topk[l - 1],
+                                              y.topk[l], stream),
                        "compute_topk_indices_sparse");
 
         // The lists of the backward (the transposed selections of all levels).  Where one launch can make them all they ride in

@@ -57,21 +57,30 @@ __device__ __forceinline__ unsigned long long quad_max_u(unsigned long long v) {
     return ((unsigned long long)hi << 32) | lo;
 }
 
+// Where a lane's two pieces of sixteen keys are: in rows of 64 channels, or in an R tile, which is the same sixteen keys in the same place in
+// the order the lanes read them.  Out of rows each of the 64 pieces of a load is an access of its own in the L1, whose rate the selection of
+// long rows then runs at; out of tiles a load is one contiguous kilobyte: 8 x 4096 rows
+// of 4096 keys, T = 8, 71.5 -> 48.9 us; 6 x 1024 of 1024, in registers, 19.3 -> 14.6; 24 x 256 8.2 -> 7.0; parent-guided, 6 x 16384 rows, 54.4 -> 49.3.
+struct KeyPieces {
+    int first, second;                                        // elements from the sixteen keys' start
+    __device__ __forceinline__ KeyPieces(int tiled, int lane)
+        : first(tiled ? lane * 8 : (lane & 15) * kD + (lane >> 4) * 8), second(first + (tiled ? kTile / 2 : kD / 2)) {}
+};
+
 // S^T tiles: rows = 16 keys starting at row_of(a) * kD elements into `keys`, columns = the wave's 16 queries (bq).  Lane l
 // gets the scores of query l%16 against keys 4*(l/16) .. +3 of tile a.  No branch around the loads, so that they are all in
 // flight together: the caller clamps the rows of tiles that do not exist and drops their scores.
 template <int TILES, typename RowOf>
-__device__ __forceinline__ void score_tiles(f32x4 (&s)[TILES], const bf16* keys, RowOf row_of, const bf16x8 bq[2], int lane) {
+__device__ __forceinline__ void score_tiles(f32x4 (&s)[TILES], const bf16* keys, RowOf row_of, const bf16x8 bq[2], const KeyPieces& pieces) {
     constexpr int kBatch = TILES < 8 ? TILES : 8;
-    const int at = (lane & 15) * kD + (lane >> 4) * 8;
 #pragma unroll
     for (int a0 = 0; a0 < TILES; a0 += kBatch) {
         bf16x8 k[kBatch][2];
 #pragma unroll
         for (int a = 0; a < kBatch; a++) {
-            const bf16* p = keys + (int64_t)row_of(a0 + a) * kD + at;
-            k[a][0] = ld16(p);
-            k[a][1] = ld16(p + 32);
+            const bf16* p = keys + (int64_t)row_of(a0 + a) * kD;
+            k[a][0] = ld16(p + pieces.first);
+            k[a][1] = ld16(p + pieces.second);
         }
 #pragma unroll
         for (int a = 0; a < kBatch; a++) {
@@ -234,7 +243,7 @@ constexpr int kRegMaxN = 1024;        // keys per row the register kernel takes:
 // one row per wave and a ballot per score it took 17 us at n = 256, 24 rows of heads, and 44 us at n = 1024, 6.
 template <int TPW, int W, bool PACK>
 __global__ __launch_bounds__(64 * W) void topk_dense_kernel(const bf16* __restrict__ pq, const bf16* __restrict__ pk, int* __restrict__ out,
-                                                         int n, int T) {
+                                                         int n, int T, int tiled) {
     constexpr int E = 4 * TPW;
     __shared__ RowShare<W> share;
     __shared__ unsigned long long win[16][kWinStride];
@@ -249,7 +258,7 @@ __global__ __launch_bounds__(64 * W) void topk_dense_kernel(const bf16* __restri
     bq[1] = ld16(pqb + r * kD + quad * 8 + 32);
     unsigned key[E];
     f32x4 s[TPW];
-    score_tiles<TPW>(s, pkb, [=](int a) { return min(a * W + wave, n / 16 - 1) * 16; }, bq, lane);
+    score_tiles<TPW>(s, pkb, [=](int a) { return min(a * W + wave, n / 16 - 1) * 16; }, bq, KeyPieces(tiled, lane));
 #pragma unroll
     for (int a = 0; a < TPW; a++) {
         const int tile = a * W + wave;
@@ -314,14 +323,14 @@ __global__ __launch_bounds__(64 * W) void topk_dense_kernel(const bf16* __restri
 //    consecutive keys, which are a patch of 8 x 8 on image-like data, are in 64 groups.
 //  * Second look: the keys that reach the bound go to their row's buffer in LDS, and the T best of those are ranked.
 // A workgroup is 16 RT rows, and its four waves take every fourth key tile of the row each, four tiles on their way to registers while four are worked
-// on.  What bounds it is the rate at which key tiles come out of the L2 -- each is read once per workgroup and look, hence many
+// on.  What bounds it is the rate at which key tiles arrive -- each is read once per workgroup and look, hence many
 // rows a workgroup where the grid is large -- and the chain through LDS for the tiles that hold a key that passes.
 // A row whose bound lets more than kBuf keys through (ties; a period of the image that puts the best keys into few groups) has its bound
 // moved up by bisection, a look at all scores per step, at most one step per bit of a key, for no two keys of a row are equal.
 // Key: the 32-bit packed key (scores rounded to bf16, n <= kMaxPackedKeys) or the 64-bit wide key.
-// (8 x 4096 rows of 4096 keys, T = 8: 72 us, T = 64 151.  A T-step arg-max over chunks of 512
-// keys per row 1480; a running threshold per row, raised whenever a buffer was full, by a wave for itself 128 and 183, with key tiles
-// shared through LDS behind barriers 157.  5 x 3072, T = 16: 69 -> 38;  1 x 4096, T = 32: 57 -> 43;  1 x 1088, T = 8: 21 -> 17.)
+// (8 x 4096 rows of 4096 keys out of tiles: 49 us, T = 32 68; out of rows 72 and 84.  Out of rows, a T-step arg-max over chunks of 512 keys per row took
+// 1480; a running threshold per row, raised whenever a buffer was full, by a wave for itself 128 and 142, with key tiles shared through LDS
+// behind barriers 157.  5 x 3072, T = 16: 69 / 38, tiles 30;  1 x 4096, T = 32: 57 / 43, tiles 28;  1 x 1088, T = 8: 21 / 17, tiles 11.)
 constexpr int kStreamWaves = 4;
 constexpr int kAhead = 4;                         // key tiles on their way to a wave while as many are worked on
 
@@ -362,7 +371,7 @@ __device__ __forceinline__ float largest(const f32x4& s) { return fmaxf(fmaxf(s[
 // RT: sixteens of rows per workgroup (n is a multiple of 16 RT); SETS: groups per row / 64
 template <typename Key, int RT, int SETS>
 __global__ __launch_bounds__(64 * kStreamWaves) void topk_stream_kernel(const bf16* __restrict__ pq, const bf16* __restrict__ pk,
-                                                                        int* __restrict__ out, int n, int T, int round_scores) {
+                                                                        int* __restrict__ out, int n, int T, int round_scores, int tiled) {
     static_assert(RT == 1 || RT == 2 || RT == 4, "the waves are dealt to the row tiles");
     static_assert(kAhead % SETS == 0, "a tile's set of groups is known at compile time");
     constexpr int W = kStreamWaves, kPer = W / RT;            // waves per row tile where the rows are finished
@@ -383,7 +392,8 @@ __global__ __launch_bounds__(64 * kStreamWaves) void topk_stream_kernel(const bf
     const int lid = xcd_logical_id();                         // (a (b,h)'s keys on one XCD)
     const int bh = lid / (int)gridDim.x, q0 = lid % (int)gridDim.x * kRows;
     const bf16* pqb = pq + ((int64_t)bh * n + q0) * kD;
-    const bf16* pkb = pk + (int64_t)bh * n * kD + r * kD + quad * 8;
+    const bf16* pkb = pk + (int64_t)bh * n * kD;
+    const KeyPieces pieces(tiled, lane);
     const int tiles = n / 16;
     const bool round = round_scores != 0;
     bf16x8 bq[RT][2];
@@ -400,8 +410,8 @@ __global__ __launch_bounds__(64 * kStreamWaves) void topk_stream_kernel(const bf
 #pragma unroll
             for (int i = 0; i < kAhead; i++) {
                 const bf16* p = pkb + (int64_t)min(t + i * W, tiles - 1) * 16 * kD;
-                o.k[i][0] = ld16(p);
-                o.k[i][1] = ld16(p + 32);
+                o.k[i][0] = ld16(p + pieces.first);
+                o.k[i][1] = ld16(p + pieces.second);
             }
         };
         auto work = [&](const Tiles& o, int t) __attribute__((always_inline)) {
@@ -618,7 +628,7 @@ template <int TPW, int W, int P>
 __global__ __launch_bounds__(64 * W) void topk_sparse_kernel(const bf16* __restrict__ pq, const bf16* __restrict__ pk,
                                                              const int* __restrict__ pidx, int* __restrict__ out, int N1, int T, int T2,
                                                              const bf16* __restrict__ pq_par, const bf16* __restrict__ pk_par,
-                                                             int* __restrict__ par_out) {
+                                                             int* __restrict__ par_out, int tiled) {
     constexpr int E = 4 * TPW;
     __shared__ RowShare<W> share;
     __shared__ unsigned long long win[16][kWinStride];
@@ -630,6 +640,7 @@ __global__ __launch_bounds__(64 * W) void topk_sparse_kernel(const bf16* __restr
     const int N2 = N1 / kBlk;
     const bf16* pqb = pq + ((int64_t)bh * N1 + G * kBlk) * kD;
     const bf16* pkb = pk + (int64_t)bh * N1 * kD;
+    const KeyPieces pieces(tiled, lane);
     bf16x8 bq[2];
     bq[0] = ld16(pqb + r * kD + quad * 8);
     bq[1] = ld16(pqb + r * kD + quad * 8 + 32);
@@ -645,7 +656,7 @@ __global__ __launch_bounds__(64 * W) void topk_sparse_kernel(const bf16* __restr
         unsigned key[4 * P], top;
         f32x4 sp[P];
         int turn = 0, n_ge;
-        score_tiles<P>(sp, pk_par + (int64_t)bh * N2 * kD, [=](int a) { return min(a * W + wave, N2 / 16 - 1) * 16; }, bp, lane);
+        score_tiles<P>(sp, pk_par + (int64_t)bh * N2 * kD, [=](int a) { return min(a * W + wave, N2 / 16 - 1) * 16; }, bp, pieces);
 #pragma unroll
         for (int a = 0; a < P; a++)
 #pragma unroll
@@ -702,7 +713,7 @@ __global__ __launch_bounds__(64 * W) void topk_sparse_kernel(const bf16* __restr
 #pragma unroll
     for (int a = 0; a < TPW; a++) blk[a] = __builtin_amdgcn_readlane(mine_par, min(a * W + wave, T2 - 1)) * kBlk;
     f32x4 s[TPW];
-    score_tiles<TPW>(s, pkb, [&](int a) { return blk[a]; }, bq, lane);
+    score_tiles<TPW>(s, pkb, [&](int a) { return blk[a]; }, bq, pieces);
 #pragma unroll
     for (int a = 0; a < TPW; a++)
 #pragma unroll
@@ -761,8 +772,7 @@ __global__ __launch_bounds__(64 * W) void topk_sparse_kernel(const bf16* __restr
 
 using namespace llsa;
 
-extern "C" int llsa_topk_dense(const void* pq, const void* pk, int32_t* out_idx, int B, int H, int n, int T,
-                               int round_scores, void* stream) {
+static int topk_dense(const void* pq, const void* pk, int32_t* out_idx, int B, int H, int n, int T, int round_scores, int tiled, void* stream) {
     LLSA_REQUIRE(pq && pk && out_idx, "topk_dense: null argument");
     LLSA_REQUIRE(B > 0 && H > 0 && n > 0 && n % 16 == 0, "topk_dense: n=%d must be a positive multiple of 16", n);
     LLSA_REQUIRE(T >= 1 && T <= kMaxT && T <= n, "topk_dense: need 1 <= T <= min(%d, n=%d), got %d", kMaxT, n, T);
@@ -774,8 +784,8 @@ extern "C" int llsa_topk_dense(const void* pq, const void* pk, int32_t* out_idx,
 #define LLSA_DENSE(TPW, W)                                                                                                               \
     do {                                                                                                                                 \
         if (round_scores)                                                                                                                \
-            hipLaunchKernelGGL(HIP_KERNEL_NAME(topk_dense_kernel<TPW, W, true>), grid, dim3(64 * W), 0, st, q, k, out_idx, n, T);        \
-        else hipLaunchKernelGGL(HIP_KERNEL_NAME(topk_dense_kernel<TPW, W, false>), grid, dim3(64 * W), 0, st, q, k, out_idx, n, T);      \
+            hipLaunchKernelGGL(HIP_KERNEL_NAME(topk_dense_kernel<TPW, W, true>), grid, dim3(64 * W), 0, st, q, k, out_idx, n, T, tiled); \
+        else hipLaunchKernelGGL(HIP_KERNEL_NAME(topk_dense_kernel<TPW, W, false>), grid, dim3(64 * W), 0, st, q, k, out_idx, n, T, tiled); \
     } while (0)
         if (n <= 64) LLSA_DENSE(4, 1);
         else if (n <= 128) LLSA_DENSE(2, 4);
@@ -784,16 +794,24 @@ extern "C" int llsa_topk_dense(const void* pq, const void* pk, int32_t* out_idx,
         else LLSA_DENSE(16, 4);
 #undef LLSA_DENSE
     } else {
-        // Rows per workgroup: sixteen while every workgroup has a CU of its own, 32 while half of them do, else 64 (32 beyond T = 32, whose
-        // groups and buffers are larger): a workgroup reads the row of keys twice, whatever it has rows.  us with 16 / 32 / 64 rows, T = 8:
-        //   128 row tiles (2048 keys) 21 / 23 / 26;  256 (4096) 36 / 37 / 40;  400 (1280) 30 / 19 / 23;  512 (4096) 66 / 38 / 41;  512 (2048) 38 / 23 / 28
-        //   544 (1088) 43 / 30 / 23;  576 (3072) 74 / 52 / 34;  1024 (2048) 71 / 39 / 28;  2048 (4096) 243 / 130 / 72
-        // T = 32: 256 (4096) 43 / 46 / 58;  512 (4096) 74 / 49 / 58;  544 (1088) 50 / 37 / 41;  576 (3072) 81 / 58 / 50;  2048 (4096) 251 / 139 / 90
+        // Rows per workgroup.  A workgroup reads the row of keys twice however many rows it has, so 64 on large grids (32 beyond T = 32,
+        // whose groups and buffers are larger), and 16 while those workgroups find room beside one another.  Tiles, us with 16 / 32 / 64, by sixteens of rows
+        // (keys per row):
+        //   T = 8: 256 (4096) 20.1 / 22.9 / 33.9;  400 (1280) 14.3 / 14.0 / 19.7;  448 (3584) 24.2 / 22.0 / 32.1;  512 (2048) 18.1 / 16.6 / 23.6
+        //     544 (1088) 17.2 / 15.8 / 18.6;  1024 (2048) 27.9 / 21.7 / 24.8;  1536 (4096) 63.9 / 42.5 / 47.9;  1792 (2048) 42.5 / 35.9 / 31.1
+        //     1920 (1536) 39.2 / 30.8 / 26.9;  2048 (4096) 82.3 / 56.3 / 48.8
+        //   T = 16: 448 (3584) 25.0 / 24.1 / 35.0;  480 (1536) 16.4 / 17.1 / 23.6;  512 (2048) 18.7 / 19.4 / 26.7;  576 (3072) 29.3 / 28.1 / 35.1
+        //     1536 (4096) 64.5 / 45.6 / 52.6;  1792 (2048) 44.7 / 38.5 / 35.2
+        //   T = 32: 512 (2048) 27.8 / 29.3 / 42.5;  544 (1088) 24.6 / 27.2 / 34.8;  576 (3072) 35.4 / 36.3 / 46.0;  1024 (2048) 34.6 / 33.7 / 41.5
+        //     1536 (4096) 74.0 / 55.5 / 66.8;  2048 (4096) 92.4 / 77.3 / 67.7
+        // Rows, whose loads are what takes the time, T = 8: 128 (2048) 21 / 23 / 26;  256 (4096) 36 / 37 / 40;  400 (1280) 30 / 20 / 23;  512 (4096) 66 /
+        //   38 / 40;  544 (1088) 43 / 30 / 22;  576 (3072) 73 / 52 / 33;  2048 (4096) 243 / 127 / 71
         const int64_t tiles = (int64_t)n / 16 * B * H;        // sixteens of rows
-        const int rt = tiles <= 256 || n % 32 != 0 ? 1 : tiles <= 512 || n % 64 != 0 || T > 32 ? 2 : 4;
+        const int64_t line1 = !tiled ? 256 : T <= 8 ? 400 : 560, line2 = !tiled ? 512 : 1536;
+        const int rt = tiles <= line1 || n % 32 != 0 ? 1 : tiles <= line2 || n % 64 != 0 || T > 32 ? 2 : 4;
 #define LLSA_STREAM(KEY, RT, SETS)                                                                                                              \
     hipLaunchKernelGGL(HIP_KERNEL_NAME(topk_stream_kernel<KEY, RT, SETS>), dim3(n / (16 * RT), B * H), dim3(64 * kStreamWaves), 0, st, q, k, out_idx, n, T, \
-                       round_scores)
+                       round_scores, tiled)
         const bool wide = !round_scores || n > kMaxPackedKeys;
         if (wide && rt == 1) LLSA_STREAM(unsigned long long, 1, 4);
         else if (wide && rt == 2) LLSA_STREAM(unsigned long long, 2, 4);
@@ -808,12 +826,18 @@ extern "C" int llsa_topk_dense(const void* pq, const void* pk, int32_t* out_idx,
     }
     return launch_status("topk_dense");
 }
+extern "C" int llsa_topk_dense(const void* pq, const void* pk, int32_t* out_idx, int B, int H, int n, int T, int round_scores, void* stream) {
+    return topk_dense(pq, pk, out_idx, B, H, n, T, round_scores, 0, stream);
+}
+extern "C" int llsa_topk_dense_tiles(const void* pq, const void* pk_tiles, int32_t* out_idx, int B, int H, int n, int T, int round_scores, void* stream) {
+    return topk_dense(pq, pk_tiles, out_idx, B, H, n, T, round_scores, 1, stream);
+}
 
 static void launch_sparse(const bf16* pq, const bf16* pk, const int* pidx, int* out, int B, int H, int N1, int T, int T2, const bf16* pq_par,
-                          const bf16* pk_par, int* par_out, hipStream_t st) {
+                          const bf16* pk_par, int* par_out, int tiled, hipStream_t st) {
     const dim3 grid(N1 / 16, B * H);
 #define LLSA_SPARSE_P(TPW, W, P) \
-    hipLaunchKernelGGL(HIP_KERNEL_NAME(topk_sparse_kernel<TPW, W, P>), grid, dim3(64 * W), 0, st, pq, pk, pidx, out, N1, T, T2, pq_par, pk_par, par_out)
+    hipLaunchKernelGGL(HIP_KERNEL_NAME(topk_sparse_kernel<TPW, W, P>), grid, dim3(64 * W), 0, st, pq, pk, pidx, out, N1, T, T2, pq_par, pk_par, par_out, tiled)
 #define LLSA_SPARSE(TPW, W)                                    \
     do {                                                       \
         if (pq_par == nullptr) LLSA_SPARSE_P(TPW, W, 0);       \
@@ -833,22 +857,30 @@ static void launch_sparse(const bf16* pq, const bf16* pk, const int* pidx, int* 
 #undef LLSA_SPARSE_P
 }
 
-extern "C" int llsa_topk_sparse(const void* pq, const void* pk, const int32_t* parent_idx, int32_t* out_idx, int B, int H,
-                                int N1, int T, int T2, void* stream) {
+static int topk_sparse(const void* pq, const void* pk, const int32_t* parent_idx, int32_t* out_idx, int B, int H, int N1, int T, int T2, int tiled,
+                       void* stream) {
     LLSA_REQUIRE(pq && pk && parent_idx && out_idx, "topk_sparse: null argument");
     LLSA_REQUIRE(B > 0 && H > 0 && N1 > 0 && N1 % 16 == 0, "topk_sparse: N1=%d must be a positive multiple of 16", N1);
     LLSA_REQUIRE(T2 >= 1 && T2 * 16 <= kMaxCand && T2 <= N1 / 16, "topk_sparse: need 1 <= T2 <= min(%d, N1/16), got %d", kMaxCand / 16, T2);
     LLSA_REQUIRE(T >= 1 && T <= kMaxT && T <= T2 * 16, "topk_sparse: need 1 <= T <= min(%d, 16*T2), got %d", kMaxT, T);
     LLSA_REQUIRE(aligned16(pq) && aligned16(pk), "topk_sparse: inputs must be 16-byte aligned");
-    launch_sparse((const bf16*)pq, (const bf16*)pk, parent_idx, out_idx, B, H, N1, T, T2, nullptr, nullptr, nullptr, (hipStream_t)stream);
+    launch_sparse((const bf16*)pq, (const bf16*)pk, parent_idx, out_idx, B, H, N1, T, T2, nullptr, nullptr, nullptr, tiled, (hipStream_t)stream);
     return launch_status("topk_sparse");
+}
+extern "C" int llsa_topk_sparse(const void* pq, const void* pk, const int32_t* parent_idx, int32_t* out_idx, int B, int H, int N1, int T, int T2,
+                                void* stream) {
+    return topk_sparse(pq, pk, parent_idx, out_idx, B, H, N1, T, T2, 0, stream);
+}
+extern "C" int llsa_topk_sparse_tiles(const void* pq, const void* pk_tiles, const int32_t* parent_idx, int32_t* out_idx, int B, int H, int N1, int T,
+                                      int T2, void* stream) {
+    return topk_sparse(pq, pk_tiles, parent_idx, out_idx, B, H, N1, T, T2, 1, stream);
 }
 
 // (a wave selects its parent row sixteen times over: beyond a few hundred parent tokens the separate dense kernel is faster)
 extern "C" int llsa_topk_cascade_max_parents(void) { return kCascadeMaxParents; }
 
-extern "C" int llsa_topk_cascade(const void* pq_parent, const void* pk_parent, int32_t* parent_out, const void* pq, const void* pk,
-                                 int32_t* out_idx, int B, int H, int N1, int T, int T2, void* stream) {
+static int topk_cascade(const void* pq_parent, const void* pk_parent, int32_t* parent_out, const void* pq, const void* pk, int32_t* out_idx, int B, int H,
+                        int N1, int T, int T2, int tiled, void* stream) {
     LLSA_REQUIRE(pq_parent && pk_parent && parent_out && pq && pk && out_idx, "topk_cascade: null argument");
     LLSA_REQUIRE(B > 0 && H > 0 && N1 > 0 && N1 % 256 == 0, "topk_cascade: N1=%d must be a positive multiple of 256", N1);
     LLSA_REQUIRE(N1 / 16 <= kCascadeMaxParents, "topk_cascade: at most %d parent tokens (got %d): use llsa_topk_dense and llsa_topk_sparse",
@@ -857,6 +889,14 @@ extern "C" int llsa_topk_cascade(const void* pq_parent, const void* pk_parent, i
     LLSA_REQUIRE(T >= 1 && T <= kMaxT && T <= T2 * 16, "topk_cascade: need 1 <= T <= min(%d, 16*T2), got %d", kMaxT, T);
     LLSA_REQUIRE(aligned16(pq) && aligned16(pk) && aligned16(pq_parent) && aligned16(pk_parent), "topk_cascade: inputs must be 16-byte aligned");
     launch_sparse((const bf16*)pq, (const bf16*)pk, nullptr, out_idx, B, H, N1, T, T2, (const bf16*)pq_parent, (const bf16*)pk_parent, parent_out,
-                  (hipStream_t)stream);
+                  tiled, (hipStream_t)stream);
     return launch_status("topk_cascade");
+}
+extern "C" int llsa_topk_cascade(const void* pq_parent, const void* pk_parent, int32_t* parent_out, const void* pq, const void* pk, int32_t* out_idx,
+                                 int B, int H, int N1, int T, int T2, void* stream) {
+    return topk_cascade(pq_parent, pk_parent, parent_out, pq, pk, out_idx, B, H, N1, T, T2, 0, stream);
+}
+extern "C" int llsa_topk_cascade_tiles(const void* pq_parent, const void* pk_parent_tiles, int32_t* parent_out, const void* pq, const void* pk_tiles,
+                                       int32_t* out_idx, int B, int H, int N1, int T, int T2, void* stream) {
+    return topk_cascade(pq_parent, pk_parent_tiles, parent_out, pq, pk_tiles, out_idx, B, H, N1, T, T2, 1, stream);
 }

@@ -5,7 +5,8 @@ import pytest
 import torch
 
 from emu_util import emu_lib
-from llsa_amd._lib import override_library_for_tests
+from llsa_amd._lib import current_lib, override_library_for_tests
+from llsa_amd.kernel.hip._common import stream_of
 
 
 def expected(pq, pk, T):
@@ -17,6 +18,11 @@ def expected(pq, pk, T):
 def ints(seed, *shape, hi=2):
     g = torch.Generator().manual_seed(seed)
     return torch.randint(-(hi - 1), hi, shape, generator=g).bfloat16()
+
+
+def tiles(x):
+    """(1, BH, n, 64) rows as R tiles: of sixteen rows, 8-channel chunk by chunk."""
+    return x.reshape(-1, x.shape[2] // 16, 16, 8, 8).transpose(2, 3).contiguous()
 
 
 def check(dev, n, T, BH, kind, round_scores=True):
@@ -33,8 +39,12 @@ def check(dev, n, T, BH, kind, round_scores=True):
         pk[:, :, 40, :] = 0
         pk[:, :, 40, 0] = float("inf")
         pq[:, :, :, 0] = 1
-    got = gen_sparse_indices(pq.to(dev), pk.to(dev), T, round_scores=round_scores).cpu().long()
-    assert torch.equal(got, expected(pq, pk, T))
+    got = gen_sparse_indices(pq.to(dev), pk.to(dev), T, round_scores=round_scores)
+    assert torch.equal(got.cpu().long(), expected(pq, pk, T))
+    q, k, out = pq.to(dev), tiles(pk).to(dev), torch.empty_like(got)
+    lib = current_lib()
+    lib.check(lib.topk_dense_tiles(q.data_ptr(), k.data_ptr(), out.data_ptr(), 1, BH, n, T, int(round_scores), stream_of(lib, q)), "topk_dense_tiles")
+    assert torch.equal(out, got)
 
 
 @pytest.mark.parametrize("n,T,kind", [(1040, 1, "plain"), (1088, 16, "few groups"), (1040, 17, "nan"), (1056, 64, "equal")])
@@ -43,11 +53,41 @@ def test_cpu(n, T, kind):
         check(torch.device("cpu"), n, T, 1, kind)
 
 
-# 16 rows a workgroup: at most 256 sixteens of rows, or an odd number of them; 32: at most 512, n no multiple of 64, or T > 32; 64 beyond
+def check_guided(dev, N1, T, T2, BH):
+    """The parent-guided selection and the cascade: out of tiles what they give out of rows."""
+    from llsa_amd.kernel.hip.topk import topk_cascade
+    pq, pk, pq2, pk2 = (torch.randn(1, BH, n, 64, generator=torch.Generator().manual_seed(n + i)).bfloat16() for i, n in
+                        enumerate((N1, N1, N1 // 16, N1 // 16)))
+    par, sel = topk_cascade(pq2.to(dev), pk2.to(dev), pq.to(dev), pk.to(dev), T, T2)
+    q, k, q2, k2 = pq.to(dev), tiles(pk).to(dev), pq2.to(dev), tiles(pk2).to(dev)
+    lib, p1, s1, s2 = current_lib(), torch.empty_like(par), torch.empty_like(sel), torch.empty_like(sel)
+    st = stream_of(lib, q)
+    lib.check(lib.topk_cascade_tiles(q2.data_ptr(), k2.data_ptr(), p1.data_ptr(), q.data_ptr(), k.data_ptr(), s1.data_ptr(), 1, BH, N1, T, T2, st), "cascade")
+    lib.check(lib.topk_sparse_tiles(q.data_ptr(), k.data_ptr(), p1.data_ptr(), s2.data_ptr(), 1, BH, N1, T, T2, st), "sparse")
+    assert torch.equal(p1, par) and torch.equal(s1, sel) and torch.equal(s2, sel)
+
+
+GUIDED = [(256, 4, 1, 1), (512, 16, 5, 1), (768, 8, 17, 2), (1024, 64, 32, 1)]
+
+
+@pytest.mark.parametrize("N1,T,T2,BH", GUIDED[:3])
+def test_guided_tiles_cpu(N1, T, T2, BH):
+    with override_library_for_tests(emu_lib()):
+        check_guided(torch.device("cpu"), N1, T, T2, BH)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("N1,T,T2,BH", GUIDED + [(4096, 16, 16, 12)])
+def test_guided_tiles_gpu(N1, T, T2, BH):
+    check_guided(torch.device("cuda"), N1, T, T2, BH)
+
+
+# Rows / tiles: 16 rows a workgroup up to 256 / 400 or 560 sixteens of rows, or where they are odd; 32 up to 512 / 1536, where n is no multiple of
+# 64, or T > 32; 64 beyond
 @pytest.mark.gpu
 @pytest.mark.parametrize("kind", ["plain", "few groups", "equal", "nan"])
 @pytest.mark.parametrize("n,T,BH", [(1040, 16, 8), (2048, 32, 2), (4096, 16, 1), (1056, 16, 8), (1056, 33, 9), (2064, 8, 1), (1088, 17, 4), (1088, 16, 8),
-                                    (1088, 17, 8), (3072, 32, 3), (1088, 64, 8), (4096, 64, 2)])
+                                    (1088, 17, 8), (3072, 32, 3), (1088, 64, 8), (4096, 64, 2), (1088, 8, 6), (1088, 32, 23), (1088, 8, 23)])
 def test_gpu(n, T, BH, kind):
     check(torch.device("cuda"), n, T, BH, kind)
 
