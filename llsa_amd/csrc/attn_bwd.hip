@@ -187,7 +187,6 @@ __device__ __forceinline__ void dq_begin(DqSide& sd, const llsa_attn_bwd_args& a
 template <bool NORM>
 __device__ __forceinline__ void dq_end(const DqSide& sd, const llsa_attn_bwd_args& a, int b, int h, int g, int lane, float (&contrib)[16]) {
     const int r = lane & 15, quad = lane >> 4, tok = g * kBlk + r;
-    bf16* op = (bf16*)a.dq + b * a.sdqb + h * a.sdqh + (int64_t)tok * a.sdqn + quad * 4;
     const bf16* fq = a.freq_dq ? (const bf16*)a.freq_dq + (int64_t)tok * kD + quad * 4 : nullptr;
     bf16x4 x[4], o[4];
     f32x4 gamma[4];
@@ -198,8 +197,7 @@ __device__ __forceinline__ void dq_end(const DqSide& sd, const llsa_attn_bwd_arg
         if (fq != nullptr) o[dt] = rope_bwd4(o[dt], ld8(fq + dt * 16));   // rotate the gradient back
     }
     if (NORM) norm_back(o, x, gamma, a.norm_q.eps, contrib);
-#pragma unroll
-    for (int dt = 0; dt < 4; dt++) st8(op + dt * 16, o[dt]);
+    store_rows((bf16*)a.dq + b * a.sdqb + h * a.sdqh + (int64_t)tok * a.sdqn, o, quad, rows_wide(a.dq, a.sdqb, a.sdqh, a.sdqn));
 }
 __device__ __forceinline__ void dq_pair_of_blocks(DqSide& sd, const PairR& r, const PairT& t, float log2w) {
     dq_accum(sd.dq, t, dq_scores(r, sd.bq, sd.bdo, sd.nlse2 + log2w, sd.ndl));
@@ -618,8 +616,8 @@ __global__ __launch_bounds__(64) void attn_kside_kernel(KSideParams p) {
         }
         return;
     }
-    bf16* kp = p.dk + b * p.sdkb + h * p.sdkh + (int64_t)(unit * kBlk + r) * p.sdkn + quad * 4;
-    bf16* vp = p.dv + b * p.sdvb + h * p.sdvh + (int64_t)(unit * kBlk + r) * p.sdvn + quad * 4;
+    bf16* kp = p.dk + b * p.sdkb + h * p.sdkh + (int64_t)(unit * kBlk + r) * p.sdkn;
+    bf16* vp = p.dv + b * p.sdvb + h * p.sdvh + (int64_t)(unit * kBlk + r) * p.sdvn;
     bf16x4 nx[4];
     f32x4 ngamma[4];
     if (NORM) norm_load(nx, ngamma, p.norm, b, h, unit * kBlk + r, quad);
@@ -638,18 +636,18 @@ __global__ __launch_bounds__(64) void attn_kside_kernel(KSideParams p) {
         __builtin_amdgcn_wave_barrier();
         __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
     }
-    bf16x4 ok[4];
+    bf16x4 ok[4], ov[4];
 #pragma unroll
     for (int dt = 0; dt < 4; dt++) {
         ok[dt] = cvt4(dk[dt] * kScale);
-        bf16x4 ov = cvt4(dv[dt]);
+        ov[dt] = cvt4(dv[dt]);
         if (folding) {
             const int c0 = dt * 16 + quad * 4;
             ok[dt] = fold_math(ok[dt], lds_ld8(fold_buf + c0), p.fold.freq != nullptr, lds_ld8(fold_buf + kFoldRows + r * kD + c0));
-            ov = fold_math(ov, lds_ld8(fold_buf + kD + c0), false, ov);
+            ov[dt] = fold_math(ov[dt], lds_ld8(fold_buf + kD + c0), false, ov[dt]);
         }
-        st8(vp + dt * 16, ov);
     }
+    store_rows(vp, ov, quad, rows_wide(p.dv, p.sdvb, p.sdvh, p.sdvn));
     if (NORM) {
         float contrib[16];
 #pragma unroll
@@ -659,8 +657,7 @@ __global__ __launch_bounds__(64) void attn_kside_kernel(KSideParams p) {
         const float s = norm_contrib_sum(contrib, lane, ch);
         p.norm.partials[((int64_t)bh * p.n_units + unit) * kD + ch] = s;       // (a unit cut into pieces: kside_reduce_kernel's row)
     }
-#pragma unroll
-    for (int dt = 0; dt < 4; dt++) st8(kp + dt * 16, ok[dt]);
+    store_rows(kp, ok, quad, rows_wide(p.dk, p.sdkb, p.sdkh, p.sdkn));
 }
 
 // ---------------------------------------------------------------------------------------

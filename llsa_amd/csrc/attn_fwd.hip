@@ -190,9 +190,10 @@ __device__ __forceinline__ void finish_query_block(const llsa_attn_fwd_args& a, 
     const int r = lane & 15, quad = lane >> 4;
     const float L = quad_sum(st.lsum);
     const float inv = 1.f / L;
-    bf16* op = (bf16*)a.o + b * a.sob + h * a.soh + (int64_t)(g * kBlk + r) * a.son + quad * 4;
+    bf16x4 o[4];
 #pragma unroll
-    for (int dt = 0; dt < 4; dt++) st8(op + dt * 16, cvt4(st.acc[dt] * inv));
+    for (int dt = 0; dt < 4; dt++) o[dt] = cvt4(st.acc[dt] * inv);
+    store_rows((bf16*)a.o + b * a.sob + h * a.soh + (int64_t)(g * kBlk + r) * a.son, o, quad, rows_wide(a.o, a.sob, a.soh, a.son));
     if (quad == 0) a.lse[(int64_t)bh * a.N + g * kBlk + r] = (st.m2 + __builtin_amdgcn_logf(L)) * kLn2;
 }
 

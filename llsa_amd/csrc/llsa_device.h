@@ -94,6 +94,29 @@ __device__ __forceinline__ float quad_sum(float v) {
     return __uint_as_float(b[0]) + __uint_as_float(b[1]);
 }
 
+// Sixteen token rows out of the accumulator layout: this lane's o[dt] are channels 16 dt + 4 (l/16) .. +3 of token l%16, whose row starts at `row`.
+// In pieces of 8 bytes of sixteen rows at a time every piece is an access of its own in the L1, and a work item of the K side had as many of
+// those in its stores as in the tiles of eight list entries.  Swapped between neighbouring sixteens of lanes the pieces are 16 bytes and the half
+// rows of a store 64.  48 x 16384 tokens, forward 237 -> 230 us, K side 319 -> 306.5; 24 x 4096, topk 16, 29.9 -> 28.6 and 39.8 -> 38.3; 6 x 262144, K
+// side 702 -> 665.  (Through 2 KB of LDS, whole rows a store: 654 there, but 311 and 67.3 against 66.0 at 12 x 16384, and the step the same.)
+// wide: rows 16-byte aligned (uniform); stored as they are otherwise.
+__device__ __forceinline__ void store_rows(bf16* row, const bf16x4 (&o)[4], int quad, bool wide) {
+    if (wide) {
+#pragma unroll
+        for (int p = 0; p < 2; p++) {
+            const u32x2 a = __builtin_bit_cast(u32x2, o[2 * p]), b = __builtin_bit_cast(u32x2, o[2 * p + 1]);
+            const u32x2 lo = __builtin_amdgcn_permlane16_swap(a[0], b[0], false, false), hi = __builtin_amdgcn_permlane16_swap(a[1], b[1], false, false);
+            st16(row + 32 * p + 16 * (quad & 1) + 8 * (quad >> 1), __builtin_bit_cast(bf16x8, u32x4{lo[0], hi[0], lo[1], hi[1]}));
+        }
+    } else {
+#pragma unroll
+        for (int dt = 0; dt < 4; dt++) st8(row + 16 * dt + 4 * quad, o[dt]);
+    }
+}
+__device__ __forceinline__ bool rows_wide(const void* p, int64_t sb, int64_t sh, int64_t sn) {
+    return ((reinterpret_cast<uintptr_t>(p) & 15u) | ((sb | sh | sn) & 7)) == 0;
+}
+
 // Operand tiles.  The attention kernels never read K/V/Q/dO row-major: a 16-row x 64-channel
 // block (1024 bf16 = 2 KB) is stored twice, each time in exactly the order the 64 lanes of a
 // wave consume it as an MFMA operand, so that every operand load is one fully coalesced
