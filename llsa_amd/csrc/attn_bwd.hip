@@ -114,13 +114,11 @@ __device__ __forceinline__ void norm_back(bf16x4 (&dy)[4], const bf16x4 (&x)[4],
             dy[dt][e] = (bf16)(rstd * ((float)dy[dt][e] * gamma[dt][e] - (float)x[dt][e] * rstd * dot));
 }
 __device__ __forceinline__ void norm_load(bf16x4 (&x)[4], f32x4 (&gamma)[4], const llsa_norm_back& nb, int b, int h, int tok, int quad) {
-    const bf16* p = (const bf16*)nb.x + b * nb.sxb + h * nb.sxh + (int64_t)tok * nb.sxn + quad * 4;
+    load_rows(x, (const bf16*)nb.x + b * nb.sxb + h * nb.sxh + (int64_t)tok * nb.sxn, quad);
 #pragma unroll
-    for (int dt = 0; dt < 4; dt++) {
-        x[dt] = ld8(p + dt * 16);
+    for (int dt = 0; dt < 4; dt++)
 #pragma unroll
         for (int e = 0; e < 4; e++) gamma[dt][e] = nb.gamma[dt * 16 + quad * 4 + e];
-    }
 }
 // Sum of the sixteen contrib[] over the sixteen tokens of a quad, by exchanging halves: lane l ends with the sum for
 // channel 16 (i/4) + 4 (l/16) + i%4, i = the lane's low four bits.
@@ -154,26 +152,48 @@ struct DqSide {
     f32x4 dq[4];                   // dQ^T: channel 16*dt + 4*(l/16) + e of query l%16
 };
 
-// dO comes straight from the caller's tensor, already in the register layout of an R operand
-// (lane l: row l%16, channels 8*(l/16)..+7 and 32 + 8*(l/16)..+7).  The wave also does the
-// pre-pass the K-side kernels need: delta = rowsum(O * dO) in fp32 (the reference sums in the
+// dO comes straight from the caller's tensor, as R operand (lane l: row l%16, channels 8*(l/16)..+7 and
+// 32 + 8*(l/16)..+7).  The wave also does the pre-pass the K-side kernels need: delta = rowsum(O * dO) in fp32 (the reference sums in the
 // tensor dtype, sparse_attention_res_1.py:153-177) and dO as an R tile.
-__device__ __forceinline__ void dq_begin(DqSide& sd, const llsa_attn_bwd_args& a, float* __restrict__ stats, bf16* __restrict__ dor,
-                                         int bh, int b, int h, int g, int lane) {
+// The rows of dO and O arrive eight whole rows a load and change into the operand layout through LDS (`place`: 2 KB of the wave's own for each): in the
+// operand layout straight from memory each of a load's 64 pieces is an access of its own in the L1.  With the
+// normalised rows and rotations of the epilogues in 16-byte pieces (load_rows) 12 x 16384 tokens 74.4 -> 70.0 us, 48 x 16384 with the qk norm 335.6 ->
+// 310.4 and its K side 306.5 -> 301.5, 24 x 4096 33.5 -> 31.2, 15 x 7168 44.3 -> 42.3, 6 x 1024 8.2 -> 7.3; 3 x 49152 at topk 64 even.
+struct DqRows { bf16x8 g[2], o[2]; };
+__device__ __forceinline__ void dq_request(DqRows& rows, const llsa_attn_bwd_args& a, int b, int h, int g, int lane) {
+#pragma unroll
+    for (int i = 0; i < 2; i++) {
+        const int64_t tok = g * kBlk + 8 * i + (lane >> 3);
+        rows.g[i] = ld16((const bf16*)a.dout + b * a.sdob + h * a.sdoh + tok * a.sdon + (lane & 7) * 8);
+        rows.o[i] = ld16((const bf16*)a.o + b * a.sob + h * a.soh + tok * a.son + (lane & 7) * 8);
+    }
+}
+__device__ __forceinline__ void dq_operands(bf16x8 (&x)[2], const bf16x8 (&rows)[2], bf16* place, int lane) {
+    const int r = lane & 15, quad = lane >> 4;
+#pragma unroll
+    for (int i = 0; i < 2; i++) {                             // (a row's eight pieces in an order of its own: rows start in the same banks)
+        const int row = 8 * i + (lane >> 3);
+        lds_st16(place + row * kD + ((lane & 7) ^ (row & 7)) * 8, rows[i]);
+    }
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+#pragma unroll
+    for (int i = 0; i < 2; i++) x[i] = lds_ld16(place + r * kD + ((quad + 4 * i) ^ (r & 7)) * 8);
+}
+__device__ __forceinline__ void dq_begin(DqSide& sd, const DqRows& rows, const llsa_attn_bwd_args& a, float* __restrict__ stats, bf16* __restrict__ dor,
+                                         int bh, int g, int lane, bf16* place) {
     const int N1 = a.N / kBlk, r = lane & 15, quad = lane >> 4, tok = g * kBlk + r;
     const bf16* qp = (const bf16*)a.qr + ((int64_t)bh * N1 + g) * kTile + lane * 8;
     sd.bq[0] = ld16(qp);
     sd.bq[1] = ld16(qp + 512);
-    const bf16* gp = (const bf16*)a.dout + b * a.sdob + h * a.sdoh + (int64_t)tok * a.sdon + quad * 8;
-    const bf16* op = (const bf16*)a.o + b * a.sob + h * a.soh + (int64_t)tok * a.son + quad * 8;
-    sd.bdo[0] = ld16(gp);
-    sd.bdo[1] = ld16(gp + 32);
-    const bf16x8 o0 = ld16(op), o1 = ld16(op + 32);
+    bf16x8 o[2];
+    dq_operands(sd.bdo, rows.g, place, lane);
+    dq_operands(o, rows.o, place + kTile, lane);
     float acc = 0.f;
 #pragma unroll
-    for (int e = 0; e < 8; e++) acc += (float)o0[e] * (float)sd.bdo[0][e];
+    for (int e = 0; e < 8; e++) acc += (float)o[0][e] * (float)sd.bdo[0][e];
 #pragma unroll
-    for (int e = 0; e < 8; e++) acc += (float)o1[e] * (float)sd.bdo[1][e];
+    for (int e = 0; e < 8; e++) acc += (float)o[1][e] * (float)sd.bdo[1][e];
     const float ndl = -quad_sum(acc);
     sd.ndl = f32x4{ndl, ndl, ndl, ndl};
     bf16* tile = dor + ((int64_t)bh * N1 + g) * kTile + lane * 8;
@@ -183,18 +203,22 @@ __device__ __forceinline__ void dq_begin(DqSide& sd, const llsa_attn_bwd_args& a
     if (quad < 2) stats[((int64_t)bh * N1 + g) * kStats + lane] = quad == 0 ? sd.nlse2 : ndl;
 #pragma unroll
     for (int dt = 0; dt < 4; dt++) sd.dq[dt] = f32x4{0.f, 0.f, 0.f, 0.f};
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
 }
 template <bool NORM>
 __device__ __forceinline__ void dq_end(const DqSide& sd, const llsa_attn_bwd_args& a, int b, int h, int g, int lane, float (&contrib)[16]) {
     const int r = lane & 15, quad = lane >> 4, tok = g * kBlk + r;
-    const bf16* fq = a.freq_dq ? (const bf16*)a.freq_dq + (int64_t)tok * kD + quad * 4 : nullptr;
     bf16x4 x[4], o[4];
     f32x4 gamma[4];
     if (NORM) norm_load(x, gamma, a.norm_q, b, h, tok, quad);
 #pragma unroll
-    for (int dt = 0; dt < 4; dt++) {
-        o[dt] = cvt4(sd.dq[dt] * kScale);
-        if (fq != nullptr) o[dt] = rope_bwd4(o[dt], ld8(fq + dt * 16));   // rotate the gradient back
+    for (int dt = 0; dt < 4; dt++) o[dt] = cvt4(sd.dq[dt] * kScale);
+    if (a.freq_dq != nullptr) {                               // rotate the gradient back
+        bf16x4 f[4];
+        load_rows(f, (const bf16*)a.freq_dq + (int64_t)tok * kD, quad);
+#pragma unroll
+        for (int dt = 0; dt < 4; dt++) o[dt] = rope_bwd4(o[dt], f[dt]);
     }
     if (NORM) norm_back(o, x, gamma, a.norm_q.eps, contrib);
     store_rows((bf16*)a.dq + b * a.sdqb + h * a.sdqh + (int64_t)tok * a.sdqn, o, quad, rows_wide(a.dq, a.sdqb, a.sdqh, a.sdqn));
@@ -245,12 +269,15 @@ __global__ __launch_bounds__(256, Q == 1 ? 4 : 3) void attn_dq_kernel(llsa_attn_
         copy16_global_to_lds(vb + unit, dst + kTile);
         copy16_global_to_lds<512>(vb + unit, dst + kTile);
     };
+    DqRows rows[Q];
+#pragma unroll
+    for (int u = 0; u < Q; u++) dq_request(rows[u], a, b, h, g + u, lane);
     issue_group(0);
     MergedLists<Q, R> ml = merge_lists<Q, R>(ip, min(T, kWave * R / Q), N1, lane, order[wave]);
 
-    DqSide sd[Q];
+    DqSide sd[Q];                                             // (the second buffer is not filled before the barrier of group 0)
 #pragma unroll
-    for (int u = 0; u < Q; u++) dq_begin(sd[u], a, stats, dor, bh, b, h, g + u, lane);
+    for (int u = 0; u < Q; u++) dq_begin(sd[u], rows[u], a, stats, dor, bh, g + u, lane, &sh[1][wave][0]);
 
     // ---- pooled blocks out of the shared copy.  The barrier at the top of round grp says: every
     // wave's part of group grp has landed, and every wave is done reading the other buffer.  All

@@ -113,6 +113,16 @@ __device__ __forceinline__ void store_rows(bf16* row, const bf16x4 (&o)[4], int 
         for (int dt = 0; dt < 4; dt++) st8(row + 16 * dt + 4 * quad, o[dt]);
     }
 }
+// The other way round: x[dt] = channels 16 dt + 4 (l/16) .. +3 of the row at `row` (16-byte aligned)
+__device__ __forceinline__ void load_rows(bf16x4 (&x)[4], const bf16* row, int quad) {
+#pragma unroll
+    for (int p = 0; p < 2; p++) {
+        const u32x4 v = __builtin_bit_cast(u32x4, ld16(row + 32 * p + 16 * (quad & 1) + 8 * (quad >> 1)));
+        const u32x2 lo = __builtin_amdgcn_permlane16_swap(v[0], v[2], false, false), hi = __builtin_amdgcn_permlane16_swap(v[1], v[3], false, false);
+        x[2 * p] = __builtin_bit_cast(bf16x4, u32x2{lo[0], hi[0]});
+        x[2 * p + 1] = __builtin_bit_cast(bf16x4, u32x2{lo[1], hi[1]});
+    }
+}
 __device__ __forceinline__ bool rows_wide(const void* p, int64_t sb, int64_t sh, int64_t sn) {
     return ((reinterpret_cast<uintptr_t>(p) & 15u) | ((sb | sh | sn) & 7)) == 0;
 }
@@ -415,6 +425,9 @@ __device__ __forceinline__ bf16x8 lds_ld16(const bf16* p) {
 }
 __device__ __forceinline__ bf16x4 lds_ld8(const bf16* p) {
     return *reinterpret_cast<const __attribute__((address_space(3))) bf16x4*>((const __attribute__((address_space(3))) bf16*)p);
+}
+__device__ __forceinline__ void lds_st16(bf16* p, bf16x8 v) {
+    *reinterpret_cast<__attribute__((address_space(3))) bf16x8*>((__attribute__((address_space(3))) bf16*)p) = v;
 }
 __device__ __forceinline__ void lds_st8(bf16* p, bf16x4 v) {
     *reinterpret_cast<__attribute__((address_space(3))) bf16x4*>((__attribute__((address_space(3))) bf16*)p) = v;
