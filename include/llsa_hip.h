@@ -43,7 +43,7 @@ extern "C" {
 #define LLSA_DTYPE_BF16 0
 #define LLSA_DTYPE_F32 1
 
-#define LLSA_ABI_VERSION 210     /* changes with every change of a signature or argument structure below */
+#define LLSA_ABI_VERSION 211     /* changes with every change of a signature or argument structure below */
 int llsa_version(void);          /* LLSA_ABI_VERSION of the built library                                    */
 const char* llsa_last_error_string(void);
 
@@ -237,6 +237,7 @@ int llsa_transpose_indices(const int32_t* idx, int32_t* offsets, int32_t* flat, 
 typedef struct llsa_transpose_job {
     const int32_t* idx; int32_t* offsets; int32_t* flat; int32_t* work /* or NULL */; int32_t* inv /* or NULL */;
     int32_t Mb, Kb, T, chunk;
+    void* nested /* or NULL */;
 } llsa_transpose_job;
 int llsa_transpose_indices_multi(const llsa_transpose_job* jobs, int n_jobs, int B, int H, void* stream);
 /* llsa_attn_fwd and llsa_transpose_indices_multi (of the selections the attention reads, the same B and H) in one call.  Jobs that
@@ -245,6 +246,11 @@ int llsa_attn_fwd_lists(const llsa_attn_fwd_args* a, const llsa_transpose_job* j
 /* Whether they ride in that launch: 1, or 0 if they follow it (topk: of every level, finest first; a job for each); negative: no such shape. */
 int llsa_lists_ride(int B, int H, int N, const int32_t* topk, int levels);
 int llsa_transpose_one_launch(int Mb, int Kb, int T, int B, int H);
+/* llsa_transpose_indices_multi's job i with `nested` (llsa_transpose_nested_bytes of 16-byte aligned scratch memory, T_parent = the T of job i + 1):
+ * its entries are children of job i + 1's -- query block q names key blocks 16 n + 0 .. 15 of key blocks n that query block q / 16 of job
+ * i + 1 names, each at most once -- as the selections of one operator call are.  Its lists, the same ones, are then made from those of
+ * job i + 1, which must ask for its inverse; an entry that is no such child is left out.  Pays for the lists that do not fit one launch. */
+int64_t llsa_transpose_nested_bytes(int Mb, int Kb, int T_parent, int B, int H);
 
 /* Work list for the K-side backward kernels, written by llsa_transpose_indices when `work` is
  * given: every key block's segment is cut into chunks of at most `chunk` entries, one work item

@@ -78,7 +78,7 @@ P64 = C.POINTER(c_int64)
 
 class TransposeJob(C.Structure):
     _fields_ = [("idx", c_void_p), ("offsets", c_void_p), ("flat", c_void_p), ("work", c_void_p), ("inv", c_void_p),
-                ("Mb", c_int32), ("Kb", c_int32), ("T", c_int32), ("chunk", c_int32)]
+                ("Mb", c_int32), ("Kb", c_int32), ("T", c_int32), ("chunk", c_int32), ("nested", c_void_p)]
 
 
 _SIGNATURES = {
@@ -110,6 +110,7 @@ _SIGNATURES = {
     "llsa_attn_fwd_lists": (c_int, [C.POINTER(AttnFwdArgs), C.POINTER(TransposeJob), c_int, c_void_p]),
     "llsa_lists_ride": (c_int, [c_int, c_int, c_int, C.POINTER(c_int32), c_int]),
     "llsa_transpose_one_launch": (c_int, [c_int, c_int, c_int, c_int, c_int]),
+    "llsa_transpose_nested_bytes": (c_int64, [c_int, c_int, c_int, c_int, c_int]),
     "llsa_work_list_len": (c_int64, [c_int, c_int, c_int, c_int]),
     "llsa_fine_chunk": (c_int, [c_int]),
     "llsa_fine_chunk_for": (c_int, [c_int, c_int, c_int, c_int]),
@@ -119,7 +120,7 @@ _SIGNATURES = {
 
 EXPORTS = tuple(_SIGNATURES)
 CHUNK_FINE_MAX = 256                                        # LLSA_CHUNK_FINE_MAX of include/llsa_hip.h
-ABI_VERSION = 210                                           # LLSA_ABI_VERSION
+ABI_VERSION = 211                                           # LLSA_ABI_VERSION
 STATIC_PARTIALS_MAX = 262144                                # LLSA_STATIC_PARTIALS_MAX
 
 

@@ -103,6 +103,7 @@ struct Library {
     decltype(&llsa_attn_fwd_lists) attn_fwd_lists;
     decltype(&llsa_transpose_indices_multi) transpose_indices_multi;
     decltype(&llsa_transpose_one_launch) transpose_one_launch;
+    decltype(&llsa_transpose_nested_bytes) transpose_nested_bytes;
     decltype(&llsa_work_list_len) work_list_len;
     decltype(&llsa_fine_chunk_for) fine_chunk_for;
     decltype(&llsa_attn_bwd_workspace_bytes) attn_bwd_workspace_bytes;
@@ -122,6 +123,7 @@ struct Library {
         get("llsa_attn_fwd_lists", attn_fwd_lists);
         get("llsa_transpose_indices_multi", transpose_indices_multi);
         get("llsa_transpose_one_launch", transpose_one_launch);
+        get("llsa_transpose_nested_bytes", transpose_nested_bytes);
         get("llsa_work_list_len", work_list_len);
         get("llsa_fine_chunk_for", fine_chunk_for);
         get("llsa_attn_bwd_workspace_bytes", attn_bwd_workspace_bytes);
@@ -217,7 +219,7 @@ struct Layout {
     int64_t pq[kL + 1], pk[kL + 1], pv[kL + 1];             // pooled rows, index = level
     int64_t qr, kr, vr;                                     // operand tiles of the tokens
     int64_t pkr[kL + 1], pvr[kL + 1], pvt[kL + 1];          // and of the pooled levels
-    int64_t sel[kL], off[kL], flat[kL], inv[kL], work = -1; // sel[0]: fine blocks per query block, sel[l]: blocks of level l per group of 16^(l+1) queries
+    int64_t sel[kL], off[kL], flat[kL], inv[kL], work = -1, nested = -1; // sel[0]: fine blocks per query block, sel[l]: blocks of level l per group of 16^(l+1) queries
     int64_t lse, bytes;
     int64_t dpk[kL + 1], dpv[kL + 1], ws, ws_bytes = 0, bwd_bytes;       // the backward's arena
 
@@ -256,6 +258,12 @@ struct Layout {
                 inv[l] = take(4 * n[l + 1] * topk[l], l > 0);
             }
             work = take(4 * lib.work_list_len(static_cast<int>(n[1]), static_cast<int>(n[1]), topk[0], chunk));
+            // (lists too long for one launch are made from those of the level above, which the selection is nested in)
+            const int m = static_cast<int>(n[1]), b = static_cast<int>(B), h = static_cast<int>(H);
+            const int64_t scratch = L > 1 && !lib.transpose_one_launch(m, m, topk[0], b, h) ? lib.transpose_nested_bytes(m, m, topk[1], b, h) : -1;
+            nested = o;
+            o = align_up(o + std::max<int64_t>(scratch, 0), 256);
+            if (scratch < 0) nested = -1;
         }
         bytes = o;
         o = 0;
@@ -523,7 +531,7 @@ Tensor attend(const std::shared_ptr<Library>& lib, const Tensor& q_in, const Ten
         for (int l = 0; l < L && grad; l++) {
             const int32_t m = static_cast<int32_t>(n[l + 1]);
             jobs[l] = llsa_transpose_job{ints(y.sel[l]), ints(y.off[l]), ints(y.flat[l]), l == 0 ? ints(y.work) : nullptr, l == 0 ? nullptr : ints(y.inv[l]),
-                                         m, m, y.topk[l], l == 0 ? y.chunk : 1};
+                                         m, m, y.topk[l], l == 0 ? y.chunk : 1, l == 0 ? pa(y.nested) : nullptr};
         }
         if (grad && !beside) lib->check(lib->attn_fwd_lists(&f, jobs, L, stream), "attn_fwd");
         else lib->check(lib->attn_fwd(&f, stream), "attn_fwd");

@@ -1,9 +1,10 @@
 // Index transpose: query-major top-k lists -> key-major CSR (offsets + flat list), used by the dK/dV passes.  Up to 65536
-// entries per (b,h) one launch makes the lists of all levels from bitmaps in LDS (transpose_bitmap_kernel).  Larger lists are
-// a counting sort -- histogram, exclusive scan, scatter with a cursor -- after which every segment is put in ascending
-// query-block order with a per-wave bitmap (set one bit per entry, then read the bits back in order).  Either way the result,
-// and therefore the accumulation order of dK/dV, does not depend on the timing of atomics.  An entry that its row repeats
-// counts as often as it is there.
+// entries per (b,h) one launch makes the lists of all levels from bitmaps in LDS (transpose_bitmap_kernel).  Larger lists of a
+// selection that is nested in the level above's are made from that one's (nested_*_kernel).  Any other larger list is a counting
+// sort -- histogram, exclusive scan, scatter with a cursor -- after which every segment is put in ascending query-block order with
+// a per-wave bitmap (set one bit per entry, then read the bits back in order).  Every way the result, and therefore the
+// accumulation order of dK/dV, does not depend on the timing of atomics.  An entry that its row repeats counts as often as it is
+// there (a nested selection has none).
 #include "llsa_device.h"
 #include "llsa_host.h"
 #include "transpose_device.h"
@@ -233,6 +234,220 @@ __global__ __launch_bounds__(256) void inverse_positions_kernel(const int* __res
     inv[(int64_t)bh * E + e] = clampi(lo, 0, E - 1);
 }
 
+// The lists of a level whose selection is nested (llsa_transpose_job.nested): the key blocks a query block names are children of those
+// its parent, one of the next job's query blocks, names, each once.  So the sixteen segments under a parent key block are made of
+// the query blocks under that parent's own segment, in its order, and no entry has to be looked for or sorted: a cell of sixteen by sixteen
+// bits per entry of the parents' lists says which of the sixteen query blocks names which of the sixteen key blocks, and the cells of
+// a parent key block lie side by side in its segment's order (the parents' inverse positions).  Four kernels: the cells, out of every
+// entry once; the counts under every parent key block; their sums in front of each; the segments, offsets and work list.  They run beside the forward attention
+// kernel, in waves of at most 32 registers, which fit beside that kernel's; so do the kernels for any list, whose atomics and sorting pass they replace.  The
+// four alone / those kernels beside the forward, us: 6 x 16384 lists of 16 37 / 417, the forward with them 920 -> 850 (790 alone), 676 -> 600 with three
+// levels (546 alone); 3 x 3072 lists of 64 35 / 153, 168 -> 148 (144 alone).  Training steps 4055 -> 3890, 3070 -> 2925, 676 -> 645.  (On the
+// forward's own stream 3884, 2929 and 672.)
+struct NestedJob {
+    const int* idx; int* offsets; int* flat; int* work;       // the level itself
+    const int* p_sel; const int* p_inv; const int* p_off; const int* p_flat;      // the parents' selection and its transpose
+    unsigned* cells;                                          // (BH, owners * p_T, 8): bit 16 (j % 2) + i of word j / 2: query block i names key block j
+    int* sums;                                                // (BH, parents, kNestedSums): see there
+    int Mb, Kb, T, chunk, work_stride;
+    int owners, parents, p_T;                                 // Mb / 16, Kb / 16
+};
+constexpr int kNestedMaxParents = kWave;                      // a parent's list lives in one lane per entry
+// What is known of the sixteen key blocks under a parent key block: 0..4 their entries, items, slots, cut blocks and long items, then (after
+// nested_scan_kernel) those of everything in front, 8..23 the entries of each.
+constexpr int kNestedSums = 8 + kBlk;
+
+__global__ __launch_bounds__(256) void nested_cells_kernel(NestedJob p) {
+    __builtin_amdgcn_s_setprio(3);
+    __shared__ unsigned rows[4][kNestedMaxParents * kBlk];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int G = blockIdx.x * 4 + wave, bh = blockIdx.y;
+    if (G >= p.owners) return;                                // no workgroup barrier below
+    unsigned* const mine = rows[wave];
+    const int64_t list = ((int64_t)bh * p.owners + G) * p.p_T;
+    const int parent = lane < p.p_T ? clampi(p.p_sel[list + lane], 0, p.parents - 1) : -1;
+    const int pos = lane < p.p_T ? clampi(p.p_inv[list + lane], 0, p.owners * p.p_T - 1) : 0;
+    for (int i = lane; i < p.p_T * kBlk; i += kWave) mine[i] = 0u;
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    const int per = p.T / 4, n = kBlk * per;                  // (T is a multiple of 4, rows are 16-byte aligned)
+    const i32x4* e = reinterpret_cast<const i32x4*>(p.idx + ((int64_t)bh * p.Mb + (int64_t)G * kBlk) * p.T);
+    for (int i0 = 0; i0 < n; i0 += kWave) {
+        const int i = min(i0 + lane, n - 1), row = i / per;
+        const i32x4 v = e[i];
+        int at[4] = {-1, -1, -1, -1};
+        for (int s = 0; s < p.p_T; s++) {
+            const int o = __builtin_amdgcn_readlane(parent, s);
+#pragma unroll
+            for (int k = 0; k < 4; k++) at[k] = (clampi(v[k], 0, p.Kb - 1) >> 4) == o ? s : at[k];
+        }
+        if (i0 + lane < n)
+#pragma unroll
+            for (int k = 0; k < 4; k++)
+                if (at[k] >= 0) atomicOr(&mine[at[k] * kBlk + (clampi(v[k], 0, p.Kb - 1) & (kBlk - 1))], 1u << row);
+    }
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    unsigned* const out = p.cells + (int64_t)bh * p.owners * p.p_T * 8;
+    for (int i0 = 0; i0 < p.p_T * 8; i0 += kWave) {           // (every lane takes part in the shuffle)
+        const int i = min(i0 + lane, p.p_T * 8 - 1);
+        const int at = __shfl(pos, i >> 3);
+        if (i0 + lane < p.p_T * 8) out[(int64_t)at * 8 + (i & 7)] = mine[2 * i] | mine[2 * i + 1] << 16;
+    }
+}
+
+struct NestedItems { int entries, items, slots, multi, longs; };     // of a key block (offsets_and_work_list's counts), or sums of those
+__device__ __forceinline__ NestedItems nested_items(int c, int chunk) {
+    const int nch = max(1, (c + chunk - 1) / chunk);
+    NestedItems t;
+    t.entries = c;
+    t.longs = (nch - 1) + ((c - (nch - 1) * chunk >= chunk / 2 + 1) ? 1 : 0);
+    t.items = nch - t.longs;
+    t.slots = nch > 1 ? nch : 0;
+    t.multi = nch > 1 ? 1 : 0;
+    return t;
+}
+template <typename Fn>
+__device__ __forceinline__ NestedItems nested_each(const NestedItems& a, Fn fn) {
+    return NestedItems{fn(a.entries), fn(a.items), fn(a.slots), fn(a.multi), fn(a.longs)};
+}
+__device__ __forceinline__ NestedItems operator+(const NestedItems& a, const NestedItems& b) {
+    return NestedItems{a.entries + b.entries, a.items + b.items, a.slots + b.slots, a.multi + b.multi, a.longs + b.longs};
+}
+__device__ __forceinline__ NestedItems nested_load(const int* t) {
+    const i32x4 v = *reinterpret_cast<const i32x4*>(t);
+    return NestedItems{v[0], v[1], v[2], v[3], t[4]};
+}
+__device__ __forceinline__ void nested_store(int* t, const NestedItems& v) {
+    *reinterpret_cast<i32x4*>(t) = i32x4{v.entries, v.items, v.slots, v.multi};
+    t[4] = v.longs;
+}
+__device__ __forceinline__ void nested_range(const NestedJob& p, int bh, int c, int& p0, int& p1) {
+    const int* o = p.p_off + (int64_t)bh * (p.parents + 1) + c;
+    p0 = clampi(o[0], 0, p.owners * p.p_T);
+    p1 = clampi(o[1], p0, p.owners * p.p_T);
+}
+
+__global__ __launch_bounds__(256) void nested_totals_kernel(NestedJob p) {
+    __builtin_amdgcn_s_setprio(3);
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int c = blockIdx.x * 4 + wave, bh = blockIdx.y;
+    if (c >= p.parents) return;
+    int p0, p1;
+    nested_range(p, bh, c, p0, p1);
+    const unsigned short* cells = reinterpret_cast<const unsigned short*>(p.cells + (int64_t)bh * p.owners * p.p_T * 8);
+    int n = 0;                                                // entries of key block 16 c + j: a quarter of the cells a lane
+#pragma unroll 4
+    for (int q = p0 + (lane >> 4); q < p1; q += 4) n += __popc(cells[(int64_t)q * kBlk + (lane & 15)]);
+    n += __shfl_xor(n, 16);
+    n += __shfl_xor(n, 32);
+    int* o = p.sums + ((int64_t)bh * p.parents + c) * kNestedSums;
+    if (lane < kBlk) o[8 + lane] = n;
+    NestedItems t = nested_items(n, p.chunk);
+#pragma unroll
+    for (int d = 1; d < kBlk; d <<= 1) t = t + nested_each(t, [&](int v) { return __shfl_xor(v, d); });
+    if (lane == 0) nested_store(o, t);
+}
+
+// One workgroup per (b,h): the sums become those of everything in front of a parent key block, short items counted from the last long one on.
+__global__ __launch_bounds__(256) void nested_scan_kernel(NestedJob p) {
+    __builtin_amdgcn_s_setprio(3);
+    __shared__ NestedItems wave_sum[4];
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, bh = blockIdx.x;
+    int* const sums = p.sums + (int64_t)bh * p.parents * kNestedSums;
+    const int per = (p.parents + 255) / 256, c0 = min(tid * per, p.parents), c1 = min(c0 + per, p.parents);
+    NestedItems own{0, 0, 0, 0, 0};
+    for (int c = c0; c < c1; c++) own = own + nested_load(sums + (int64_t)c * kNestedSums);
+    NestedItems incl = own;
+#pragma unroll
+    for (int d = 1; d < kWave; d <<= 1) {
+        const NestedItems o = nested_each(incl, [&](int v) { return __shfl_up(v, d); });
+        if (lane >= d) incl = incl + o;
+    }
+    if (lane == kWave - 1) wave_sum[wave] = incl;
+    __syncthreads();
+    NestedItems run = incl + nested_each(own, [](int v) { return -v; }), all{0, 0, 0, 0, 0};
+#pragma unroll
+    for (int w = 0; w < 4; w++) {
+        const NestedItems o = wave_sum[w];
+        all = all + o;
+        if (w < wave) run = run + o;
+    }
+    run.items += all.longs;
+    for (int c = c0; c < c1; c++) {
+        const NestedItems t = nested_load(sums + (int64_t)c * kNestedSums);
+        nested_store(sums + (int64_t)c * kNestedSums, run);
+        run = run + t;
+    }
+    if (tid == 0) {
+        p.offsets[(int64_t)bh * (p.Kb + 1) + p.Kb] = all.entries;
+        if (p.work != nullptr)
+            *reinterpret_cast<i32x4*>(p.work + (int64_t)bh * p.work_stride) = i32x4{all.longs + all.items, all.slots, all.multi, all.longs};
+    }
+}
+
+// A wave per parent key block: offsets, work list and segments of its sixteen key blocks.
+__global__ __launch_bounds__(256) void nested_lists_kernel(NestedJob p) {
+    __builtin_amdgcn_s_setprio(3);
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, j = lane & 15, part = lane >> 4;
+    const int c = blockIdx.x * 4 + wave, bh = blockIdx.y;
+    if (c >= p.parents) return;                               // no workgroup barrier below
+    int p0, p1;
+    nested_range(p, bh, c, p0, p1);
+    const int* sums = p.sums + ((int64_t)bh * p.parents + c) * kNestedSums;
+    const int count = sums[8 + j], E = p.Mb * p.T;
+    const NestedItems own = nested_items(count, p.chunk);
+    NestedItems incl = own;                                   // over the sixteen key blocks
+#pragma unroll
+    for (int d = 1; d < kBlk; d <<= 1) {
+        const NestedItems o = nested_each(incl, [&](int v) { return __shfl_up(v, d, kBlk); });
+        if (j >= d) incl = incl + o;
+    }
+    const NestedItems at = nested_load(sums) + nested_each(own, [](int v) { return -v; }) + incl;
+    if (part == 0) {
+        const int n = c * kBlk + j;
+        p.offsets[(int64_t)bh * (p.Kb + 1) + n] = at.entries;
+        if (p.work != nullptr) {
+            int* const work = p.work + (int64_t)bh * p.work_stride;
+            const int nch = max(1, (count + p.chunk - 1) / p.chunk), max_items = E / p.chunk + p.Kb;
+            int i_long = at.longs, i_short = at.items;
+            for (int ci = 0; ci < nch; ci++) {
+                const int n_ent = min(p.chunk, count - ci * p.chunk);
+                int* it = work + 4 + 4 * ((n_ent >= p.chunk / 2 + 1) ? i_long++ : i_short++);
+                *reinterpret_cast<i32x4*>(it) = i32x4{n, at.entries + ci * p.chunk, n_ent, nch > 1 ? at.slots + ci : -1};
+            }
+            if (nch > 1) *reinterpret_cast<i32x4*>(work + 4 + 4 * max_items + 4 * at.multi) = i32x4{n, at.slots, nch, 0};
+        }
+    }
+    // the segments: four cells of the parent's segment at a time, in order; the loads of two such steps go out together (of more: more registers than the forward's waves leave)
+    const unsigned short* cells = reinterpret_cast<const unsigned short*>(p.cells + (int64_t)bh * p.owners * p.p_T * 8);
+    const int* owner = p.p_flat + (int64_t)bh * p.owners * p.p_T;
+    int* const flat = p.flat + (int64_t)bh * E;
+    int base = at.entries;
+    constexpr int kBatch = 2;
+    for (int q0 = p0; q0 < p1; q0 += 4 * kBatch) {
+        unsigned bits[kBatch];
+        int first[kBatch];
+#pragma unroll
+        for (int k = 0; k < kBatch; k++) {
+            const int q = q0 + 4 * k + part, in = min(q, p1 - 1);
+            bits[k] = cells[(int64_t)in * kBlk + j];
+            first[k] = owner[in] * kBlk;
+            if (q >= p1) bits[k] = 0u;
+        }
+#pragma unroll
+        for (int k = 0; k < kBatch; k++) {
+            const int n = __popc(bits[k]), n0 = __shfl(n, j), n1 = __shfl(n, 16 + j), n2 = __shfl(n, 32 + j), n3 = __shfl(n, 48 + j);
+            int out = base + (part > 0 ? n0 : 0) + (part > 1 ? n1 : 0) + (part > 2 ? n2 : 0);
+            while (bits[k]) {
+                flat[out++] = first[k] + __ffs((int)bits[k]) - 1;
+                bits[k] &= bits[k] - 1u;
+            }
+            base += (n0 + n1) + (n2 + n3);
+        }
+    }
+}
+
 }  // namespace llsa
 
 using namespace llsa;
@@ -260,8 +475,8 @@ static int check_transpose_job(const int32_t* idx, const int32_t* offsets, const
 // More than 65536 entries (65536 tokens at topk 16) take as long here as the several kernels for large jobs take
 // beside the attention kernel on another stream (131072 entries: step 928 against 923 us, 196608: 672 against 664).
 constexpr int kTrLdsInts = 16 * 1024;
-static int tr_parts(int Mb, int Kb, int T, int BH, int lds_ints = kTrLdsInts, int histogram_ints = 2 * kTrLdsInts) {
-    const int64_t stride = tr_stride(Mb), E = (int64_t)Mb * T;
+static int tr_parts(int Mb, int Kb, int T, int BH, bool inverse, int lds_ints = kTrLdsInts, int histogram_ints = 2 * kTrLdsInts) {
+    const int64_t stride = tr_stride(Mb, inverse), E = (int64_t)Mb * T;
     if (stride > lds_ints || Kb > histogram_ints) return 0;
     const int most_rows = (int)std::min<int64_t>(lds_ints / stride, kTrThreadsBeside);
     const int least = (Kb + most_rows - 1) / most_rows;
@@ -289,7 +504,7 @@ bool llsa::plan_transpose(const llsa_transpose_job* jobs, int n_jobs, int B, int
     for (int i = 0; i < n_jobs; i++) {
         const llsa_transpose_job& j = jobs[i];
         if (check_transpose_job(j.idx, j.offsets, j.flat, j.work, B, H, j.Mb, j.Kb, j.T, j.chunk) != 0) return false;
-        const int parts = tr_parts(j.Mb, j.Kb, j.T, B * H, lds_ints, lds_ints);
+        const int parts = tr_parts(j.Mb, j.Kb, j.T, B * H, j.inv != nullptr, lds_ints, lds_ints);
         if (parts == 0) return false;
         add_to_plan(plan, j, parts);
     }
@@ -301,7 +516,7 @@ static int launch_bitmap_jobs(const TrJobs& jobs, int B, int H, bool beside, hip
     int64_t ints = 0;
     for (int i = 0; i < jobs.n_jobs; i++) {
         const TrJob& j = jobs.job[i];
-        ints = std::max<int64_t>(ints, std::max<int64_t>((int64_t)j.rows * tr_stride(j.Mb), j.Kb));
+        ints = std::max<int64_t>(ints, std::max<int64_t>((int64_t)j.rows * tr_stride(j.Mb, j.inv != nullptr), j.Kb));
     }
     const size_t lds = sizeof(int) * (size_t)ints;
     const void* kernel = beside ? (const void*)transpose_bitmap_kernel<kTrThreadsBeside> : (const void*)transpose_bitmap_kernel<kTrThreads>;
@@ -360,7 +575,37 @@ static int transpose_general(const int32_t* idx, int32_t* offsets, int32_t* flat
 }
 
 extern "C" int llsa_transpose_one_launch(int Mb, int Kb, int T, int B, int H) {
-    return Mb > 0 && Kb > 0 && T > 0 && B > 0 && H > 0 && tr_parts(Mb, Kb, T, B * H) > 0;
+    return Mb > 0 && Kb > 0 && T > 0 && B > 0 && H > 0 && tr_parts(Mb, Kb, T, B * H, false) > 0;
+}
+
+extern "C" int64_t llsa_transpose_nested_bytes(int Mb, int Kb, int T_parent, int B, int H) {
+    if (Mb <= 0 || Kb <= 0 || Mb % kBlk != 0 || Kb % kBlk != 0 || T_parent <= 0 || T_parent > kNestedMaxParents || B <= 0 || H <= 0) return -1;
+    return (int64_t)B * H * ((int64_t)(Mb / kBlk) * T_parent * 32 + (int64_t)(Kb / kBlk) * kNestedSums * (int64_t)sizeof(int));
+}
+
+static int check_nested_job(const llsa_transpose_job& j, const llsa_transpose_job& above, int B, int H) {
+    LLSA_REQUIRE(j.inv == nullptr && above.inv != nullptr && above.Mb * kBlk == j.Mb && above.Kb * kBlk == j.Kb && above.T <= kNestedMaxParents,
+                 "transpose_indices: a nested job needs no inverse, and the job above its parents' lists with theirs");
+    LLSA_REQUIRE(j.T % 4 == 0 && aligned16(j.idx) && aligned16(j.work) && aligned16(j.nested) && (int64_t)j.Mb * j.T < (int64_t)1 << 31 && B * H <= 65535,
+                 "transpose_indices: a nested job's entries are read four at a time");
+    return 0;
+}
+// job: its lists are made from those of `above`, which are there
+static int transpose_nested(const llsa_transpose_job& j, const llsa_transpose_job& above, int B, int H, hipStream_t st) {
+    NestedJob p;
+    p.idx = j.idx; p.offsets = j.offsets; p.flat = j.flat; p.work = j.work;
+    p.p_sel = above.idx; p.p_inv = above.inv; p.p_off = above.offsets; p.p_flat = above.flat;
+    p.Mb = j.Mb; p.Kb = j.Kb; p.T = j.T; p.chunk = j.chunk < 1 ? 1 : j.chunk;
+    p.work_stride = j.work ? (int)llsa_work_list_len(j.Mb, j.Kb, j.T, p.chunk) : 0;
+    p.owners = above.Mb; p.parents = above.Kb; p.p_T = above.T;
+    p.cells = (unsigned*)j.nested;
+    p.sums = (int*)j.nested + (int64_t)B * H * p.owners * p.p_T * 8;
+    const int BH = B * H;
+    hipLaunchKernelGGL(nested_cells_kernel, dim3((p.owners + 3) / 4, BH), dim3(256), 0, st, p);
+    hipLaunchKernelGGL(nested_totals_kernel, dim3((p.parents + 3) / 4, BH), dim3(256), 0, st, p);
+    hipLaunchKernelGGL(nested_scan_kernel, dim3(BH), dim3(256), 0, st, p);
+    hipLaunchKernelGGL(nested_lists_kernel, dim3((p.parents + 3) / 4, BH), dim3(256), 0, st, p);
+    return launch_status("transpose_indices");
 }
 
 extern "C" int llsa_transpose_indices_multi(const llsa_transpose_job* jobs, int n_jobs, int B, int H, void* stream) {
@@ -370,24 +615,42 @@ extern "C" int llsa_transpose_indices_multi(const llsa_transpose_job* jobs, int 
         const llsa_transpose_job& j = jobs[i];
         const int rc = check_transpose_job(j.idx, j.offsets, j.flat, j.work, B, H, j.Mb, j.Kb, j.T, j.chunk);
         if (rc != 0) return rc;
+        if (j.nested == nullptr) continue;
+        LLSA_REQUIRE(i + 1 < n_jobs, "transpose_indices: no job above a nested one");
+        const int rc2 = check_nested_job(j, jobs[i + 1], B, H);
+        if (rc2 != 0) return rc2;
     }
+    bool several = false;                                     // kernels of small workgroups beside the forward
     for (int i = 0; i < n_jobs; i++) {
         const llsa_transpose_job& j = jobs[i];
-        const int chunk = j.chunk < 1 ? 1 : j.chunk, parts = tr_parts(j.Mb, j.Kb, j.T, B * H);
+        if (j.nested != nullptr) {
+            several = true;
+            continue;
+        }
+        const int chunk = j.chunk < 1 ? 1 : j.chunk, parts = tr_parts(j.Mb, j.Kb, j.T, B * H, j.inv != nullptr);
         if (parts > 0) {
             add_to_plan(small, j, parts);
         } else {
             const int rc = transpose_general(j.idx, j.offsets, j.flat, j.work, j.inv, B, H, j.Mb, j.Kb, j.T, chunk, stream);
             if (rc != 0) return rc;
+            several = true;
         }
     }
-    if (small.n_jobs > 0) return launch_bitmap_jobs(small, B, H, small.n_jobs < n_jobs, (hipStream_t)stream);
+    if (small.n_jobs > 0) {
+        const int rc = launch_bitmap_jobs(small, B, H, several, (hipStream_t)stream);
+        if (rc != 0) return rc;
+    }
+    for (int i = n_jobs - 2; i >= 0; i--) {                   // from the coarsest down: every one's parents are done
+        if (jobs[i].nested == nullptr) continue;
+        const int rc = transpose_nested(jobs[i], jobs[i + 1], B, H, (hipStream_t)stream);
+        if (rc != 0) return rc;
+    }
     return 0;
 }
 
 extern "C" int llsa_transpose_indices(const int32_t* idx, int32_t* offsets, int32_t* flat, int32_t* work, int32_t* inv, int B, int H,
                                       int Mb, int Kb, int T, int chunk, void* stream) {
-    llsa_transpose_job j;
+    llsa_transpose_job j{};
     j.idx = idx; j.offsets = offsets; j.flat = flat; j.work = work; j.inv = inv;
     j.Mb = Mb; j.Kb = Kb; j.T = T; j.chunk = chunk;
     return llsa_transpose_indices_multi(&j, 1, B, H, stream);
