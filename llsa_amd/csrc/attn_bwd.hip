@@ -155,10 +155,9 @@ struct DqSide {
 // dO comes straight from the caller's tensor, as R operand (lane l: row l%16, channels 8*(l/16)..+7 and
 // 32 + 8*(l/16)..+7).  The wave also does the pre-pass the K-side kernels need: delta = rowsum(O * dO) in fp32 (the reference sums in the
 // tensor dtype, sparse_attention_res_1.py:153-177) and dO as an R tile.
-// The rows of dO and O arrive eight whole rows a load and change into the operand layout through LDS (`place`: 2 KB of the wave's own for each): in the
-// operand layout straight from memory each of a load's 64 pieces is an access of its own in the L1.  With the
-// normalised rows and rotations of the epilogues in 16-byte pieces (load_rows) 12 x 16384 tokens 74.4 -> 70.0 us, 48 x 16384 with the qk norm 335.6 ->
-// 310.4 and its K side 306.5 -> 301.5, 24 x 4096 33.5 -> 31.2, 15 x 7168 44.3 -> 42.3, 6 x 1024 8.2 -> 7.3; 3 x 49152 at topk 64 even.
+// The rows of dO and O arrive whole and change into the operand layout through LDS (rows_to_operand; `place`: 2 KB of the wave's own for each).
+// With the normalised rows and rotations of the epilogues in 16-byte pieces (load_rows) 12 x 16384 tokens 74.4 -> 70.0 us, 48 x 16384 with the
+// qk norm 335.6 -> 310.4 and its K side 306.5 -> 301.5, 24 x 4096 33.5 -> 31.2, 15 x 7168 44.3 -> 42.3, 6 x 1024 8.2 -> 7.3; 3 x 49152 at topk 64 even.
 struct DqRows { bf16x8 g[2], o[2]; };
 __device__ __forceinline__ void dq_request(DqRows& rows, const llsa_attn_bwd_args& a, int b, int h, int g, int lane) {
 #pragma unroll
@@ -168,18 +167,6 @@ __device__ __forceinline__ void dq_request(DqRows& rows, const llsa_attn_bwd_arg
         rows.o[i] = ld16((const bf16*)a.o + b * a.sob + h * a.soh + tok * a.son + (lane & 7) * 8);
     }
 }
-__device__ __forceinline__ void dq_operands(bf16x8 (&x)[2], const bf16x8 (&rows)[2], bf16* place, int lane) {
-    const int r = lane & 15, quad = lane >> 4;
-#pragma unroll
-    for (int i = 0; i < 2; i++) {                             // (a row's eight pieces in an order of its own: rows start in the same banks)
-        const int row = 8 * i + (lane >> 3);
-        lds_st16(place + row * kD + ((lane & 7) ^ (row & 7)) * 8, rows[i]);
-    }
-    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-#pragma unroll
-    for (int i = 0; i < 2; i++) x[i] = lds_ld16(place + r * kD + ((quad + 4 * i) ^ (r & 7)) * 8);
-}
 __device__ __forceinline__ void dq_begin(DqSide& sd, const DqRows& rows, const llsa_attn_bwd_args& a, float* __restrict__ stats, bf16* __restrict__ dor,
                                          int bh, int g, int lane, bf16* place) {
     const int N1 = a.N / kBlk, r = lane & 15, quad = lane >> 4, tok = g * kBlk + r;
@@ -187,8 +174,8 @@ __device__ __forceinline__ void dq_begin(DqSide& sd, const DqRows& rows, const l
     sd.bq[0] = ld16(qp);
     sd.bq[1] = ld16(qp + 512);
     bf16x8 o[2];
-    dq_operands(sd.bdo, rows.g, place, lane);
-    dq_operands(o, rows.o, place + kTile, lane);
+    rows_to_operand(sd.bdo, rows.g, place, lane);
+    rows_to_operand(o, rows.o, place + kTile, lane);
     float acc = 0.f;
 #pragma unroll
     for (int e = 0; e < 8; e++) acc += (float)o[0][e] * (float)sd.bdo[0][e];

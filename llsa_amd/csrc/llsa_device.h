@@ -187,6 +187,26 @@ __device__ __forceinline__ void counted_barrier() {
 // both drained it takes the vector-memory queue for out of order and turns every later wait into vmcnt(0).
 __device__ __forceinline__ void wait_all_mem() { __builtin_amdgcn_s_waitcnt(0x0070); }
 
+// ---------------------------------------------------------------------------------------
+// rotation of one 8-channel chunk (4 interleaved pairs) with bf16 rounding after every
+// multiply and add, the arithmetic the reference performs in the tensor dtype
+// ---------------------------------------------------------------------------------------
+//
+// Contraction must stay off here: with it the compiler narrows the fp32 expression to bf16
+// arithmetic and then fuses multiply and add into one bf16 FMA, i.e. one rounding fewer.
+__device__ __forceinline__ bf16x8 rope_chunk_fwd(bf16x8 x, bf16x8 f) {
+#pragma clang fp contract(off)
+    bf16x8 y;
+#pragma unroll
+    for (int j = 0; j < 4; j++) {
+        float s = (float)f[2 * j], c = (float)f[2 * j + 1];
+        float xe = (float)x[2 * j], xo = (float)x[2 * j + 1];
+        y[2 * j] = (bf16)(rn_bf16(c * xe) - rn_bf16(s * xo));
+        y[2 * j + 1] = (bf16)(rn_bf16(s * xe) + rn_bf16(c * xo));
+    }
+    return y;
+}
+
 // Rotates a gradient back through the 2-D RoPE: 4 consecutive channels = two (even, odd) pairs, f
 // holds their [sin, cos] entries.  Every product and sum is rounded to bf16 like the forward rotation.
 __device__ __forceinline__ bf16x4 rope_bwd4(bf16x4 o, bf16x4 f) {
@@ -431,6 +451,33 @@ __device__ __forceinline__ void lds_st16(bf16* p, bf16x8 v) {
 }
 __device__ __forceinline__ void lds_st8(bf16* p, bf16x4 v) {
     *reinterpret_cast<__attribute__((address_space(3))) bf16x4*>((__attribute__((address_space(3))) bf16*)p) = v;
+}
+
+// Sixteen rows that arrived eight whole rows a load (rows[i]: row 8 i + l/8, channels 8 (l%8) ..+7) as R operand: lane l gets channels
+// 8 (l/16) ..+7 of row l%16 and those 32 further on.  place: 2 KB of LDS of the wave.  (In the operand layout straight from memory each of
+// a load's 64 pieces is an access of its own in the L1.  A row's eight pieces are in an order of its own: rows start in the same banks.)
+__device__ __forceinline__ void rows_to_operand(bf16x8 (&x)[2], const bf16x8 (&rows)[2], bf16* place, int lane) {
+    const int r = lane & 15, quad = lane >> 4;
+#pragma unroll
+    for (int i = 0; i < 2; i++) {
+        const int row = 8 * i + (lane >> 3);
+        lds_st16(place + row * kD + ((lane & 7) ^ (row & 7)) * 8, rows[i]);
+    }
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+#pragma unroll
+    for (int i = 0; i < 2; i++) x[i] = lds_ld16(place + r * kD + ((quad + 4 * i) ^ (r & 7)) * 8);
+}
+
+// A block's sixteen token rows in LDS as they are in memory, copied eight whole rows at a time, and T operands out of them.  A row's pieces
+// change places in pairs (piece ^ (row & 6)): the transposing read's lanes 0..31 and 32..63 take 32 bytes of each of eight rows of 128, whose
+// banks are those of every second row.
+__device__ __forceinline__ int row_piece(int lane) { return ((lane & 7) ^ ((lane >> 3) & 6)) * 8; }     // the piece of row l/8 (or 8 + l/8) that lane l copies
+__device__ __forceinline__ bf16x4 lds_t_operand_rows(const bf16* rows_in_lds, int dt, int lane) {
+    const int j = lane & 15, row = 4 * (lane >> 4) + (j >> 2);
+    const bf16* p = rows_in_lds + row * kD + ((2 * dt + ((j >> 1) & 1)) ^ (row & 6)) * 8 + 4 * (j & 1);
+    const s16x4 v = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) s16x4*)p);
+    return __builtin_bit_cast(bf16x4, v);
 }
 
 // XCD-aware workgroup order.  The 8 XCDs of the chip each have a private L2 and receive
