@@ -43,7 +43,7 @@ extern "C" {
 #define LLSA_DTYPE_BF16 0
 #define LLSA_DTYPE_F32 1
 
-#define LLSA_ABI_VERSION 211     /* changes with every change of a signature or argument structure below */
+#define LLSA_ABI_VERSION 212     /* changes with every change of a signature or argument structure below */
 int llsa_version(void);          /* LLSA_ABI_VERSION of the built library                                    */
 const char* llsa_last_error_string(void);
 
@@ -209,6 +209,12 @@ typedef struct llsa_attn_fwd_args {
     float* lse;                                /* (B,H,N) out, m + log(l)                          */
     int32_t B, H, N, T, levels, reserved;
     llsa_fwd_level lvl[LLSA_MAX_LEVELS];       /* lvl[l - 1] = pooled level l                     */
+    /* q not NULL (no backward will follow): q and v are read as rows, (B,H,N,64) with 16-byte aligned rows, in place of qr and
+     * vt, and q is normalised (gamma_q (64,) fp32, or NULL) and rotated (freq_q (N,64), or NULL) here, as
+     * llsa_pool_pyramid_fwd does it.  lse may then be NULL. */
+    const void* q;  int64_t sqb, sqh, sqn;
+    const void* v;  int64_t svb, svh, svn;
+    const void* freq_q; const float* gamma_q; float eps_q; int32_t reserved2;
 } llsa_attn_fwd_args;
 
 int llsa_attn_fwd(const llsa_attn_fwd_args* a, void* stream);

@@ -41,7 +41,10 @@ class AttnFwdArgs(C.Structure):
                 ("o", c_void_p), ("sob", c_int64), ("soh", c_int64), ("son", c_int64),
                 ("lse", c_void_p),
                 ("B", c_int32), ("H", c_int32), ("N", c_int32), ("T", c_int32), ("levels", c_int32), ("reserved", c_int32),
-                ("lvl", FwdLevel * MAX_LEVELS)]
+                ("lvl", FwdLevel * MAX_LEVELS),
+                ("q", c_void_p), ("sqb", c_int64), ("sqh", c_int64), ("sqn", c_int64),
+                ("v", c_void_p), ("svb", c_int64), ("svh", c_int64), ("svn", c_int64),
+                ("freq_q", c_void_p), ("gamma_q", c_void_p), ("eps_q", c_float), ("reserved2", c_int32)]
 
 
 def _t3(name):
@@ -120,7 +123,7 @@ _SIGNATURES = {
 
 EXPORTS = tuple(_SIGNATURES)
 CHUNK_FINE_MAX = 256                                        # LLSA_CHUNK_FINE_MAX of include/llsa_hip.h
-ABI_VERSION = 211                                           # LLSA_ABI_VERSION
+ABI_VERSION = 212                                           # LLSA_ABI_VERSION
 STATIC_PARTIALS_MAX = 262144                                # LLSA_STATIC_PARTIALS_MAX
 
 

@@ -186,6 +186,57 @@ __device__ __forceinline__ void load_values_fine(ValueRegs<2>& t, const bf16* ti
     for (int dt = 0; dt < 4; dt++) t.v[0][dt] = cat(lds_t_operand(tiles, dt, lane), lds_t_operand(tiles + kTile, dt, lane));
 }
 
+__device__ __forceinline__ void load_values_fine_rows(ValueRegs<2>& t, const bf16* rows, int lane) {
+#pragma unroll
+    for (int dt = 0; dt < 4; dt++) t.v[0][dt] = cat(lds_t_operand_rows(rows, dt, lane), lds_t_operand_rows(rows + kTile, dt, lane));
+}
+
+// The query blocks' operands out of the rows of q, normalised and rotated here as the pooling pass does it (the sums over a row's chunks
+// in its order): the same bits.
+template <int Q>
+struct QueryRows { bf16x8 x[Q][2], f[Q][2]; };
+template <int Q>
+__device__ __forceinline__ void request_queries(QueryRows<Q>& qr, const llsa_attn_fwd_args& a, int b, int h, int g, int lane) {
+#pragma unroll
+    for (int u = 0; u < Q; u++)
+#pragma unroll
+        for (int i = 0; i < 2; i++) {
+            const int64_t tok = (g + u) * kBlk + 8 * i + (lane >> 3);
+            qr.x[u][i] = ld16((const bf16*)a.q + b * a.sqb + h * a.sqh + tok * a.sqn + (lane & 7) * 8);
+            if (a.freq_q != nullptr) qr.f[u][i] = ld16((const bf16*)a.freq_q + tok * kD + (lane & 7) * 8);
+        }
+}
+template <int Q>
+__device__ __forceinline__ void finish_queries(bf16x8 (&bq)[Q][2], const QueryRows<Q>& qr, const llsa_attn_fwd_args& a, int lane, bf16* place) {
+#pragma unroll
+    for (int u = 0; u < Q; u++) {
+        rows_to_operand(bq[u], qr.x[u], place, lane);
+        if (a.gamma_q != nullptr) {
+            float ss[2];
+#pragma unroll
+            for (int i = 0; i < 2; i++) {
+                ss[i] = 0.f;
+#pragma unroll
+                for (int e = 0; e < 8; e++) ss[i] += (float)bq[u][i][e] * (float)bq[u][i][e];
+                ss[i] = quad_sum(ss[i]);
+            }
+            const float rstd = rsqrtf((ss[0] + ss[1]) * (1.f / kD) + a.eps_q);
+#pragma unroll
+            for (int i = 0; i < 2; i++)
+#pragma unroll
+                for (int e = 0; e < 8; e++) bq[u][i][e] = (bf16)((float)bq[u][i][e] * rstd * a.gamma_q[((lane >> 4) + 4 * i) * 8 + e]);
+        }
+        if (a.freq_q != nullptr) {
+            bf16x8 f[2];
+            rows_to_operand(f, qr.f[u], place + kTile, lane);
+#pragma unroll
+            for (int i = 0; i < 2; i++) bq[u][i] = rope_chunk_fwd(bq[u][i], f[i]);
+        }
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+    }
+}
+
 __device__ __forceinline__ void finish_query_block(const llsa_attn_fwd_args& a, const SoftmaxState& st, int bh, int b, int h, int g, int lane) {
     const int r = lane & 15, quad = lane >> 4;
     const float L = quad_sum(st.lsum);
@@ -194,7 +245,7 @@ __device__ __forceinline__ void finish_query_block(const llsa_attn_fwd_args& a, 
 #pragma unroll
     for (int dt = 0; dt < 4; dt++) o[dt] = cvt4(st.acc[dt] * inv);
     store_rows((bf16*)a.o + b * a.sob + h * a.soh + (int64_t)(g * kBlk + r) * a.son, o, quad, rows_wide(a.o, a.sob, a.soh, a.son));
-    if (quad == 0) a.lse[(int64_t)bh * a.N + g * kBlk + r] = (st.m2 + __builtin_amdgcn_logf(L)) * kLn2;
+    if (quad == 0 && a.lse != nullptr) a.lse[(int64_t)bh * a.N + g * kBlk + r] = (st.m2 + __builtin_amdgcn_logf(L)) * kLn2;
 }
 
 // Q sibling query blocks per wave, 4 Q consecutive query blocks per workgroup.
@@ -220,11 +271,14 @@ static_assert(tr_scratch_ints(256) <= 32, "the scratch of a transposing workgrou
 constexpr int64_t kRideMaxReads = (int64_t)88 << 20;          // entries the riding workgroups may read in all
 constexpr int kGridRows = 65535;                              // rows a grid can have
 
-template <int Q, int R>
+// ROWS (no backward will follow): q and v are read as the caller's rows.  Their tiles are then not written, which is a third of all that the pooling pass
+// moves; every block of v is still copied into LDS in two loads of whole lines.  8 x 65536 tokens, topk 8:
+// pooling 68.7 -> 45.2 us, forward 559 -> 570.
+template <int Q, int R, bool ROWS>
 __global__ __launch_bounds__(256, Q == 1 ? 4 : 3) void attn_fwd_kernel(llsa_attn_fwd_args a, TrJobs lists, int list_rows) {
     __shared__ __align__(16) bf16 sh[2][kGroup][2 * kTile];
     __shared__ int order[4][R * kWave];
-    if ((int)blockIdx.y < list_rows) {
+    if (!ROWS && (int)blockIdx.y < list_rows) {
         const int block = (int)(blockIdx.y * gridDim.x + blockIdx.x);
         int* const lds = reinterpret_cast<int*>(&sh[0][0][0]);
         if (block < lists.wgs * ((int)gridDim.y - list_rows)) transpose_block<256>(lists, block, lds, lds + kTrLdsFwd);
@@ -238,7 +292,8 @@ __global__ __launch_bounds__(256, Q == 1 ? 4 : 3) void attn_fwd_kernel(llsa_attn
     const int bh = lid / (int)gridDim.x, b = bh / a.H, h = bh % a.H;
 
     const bf16* kr = (const bf16*)a.kr + (int64_t)bh * N1 * kTile;
-    const bf16* vr = (const bf16*)a.vt + (int64_t)bh * N1 * kTile;
+    const bf16* vr = ROWS ? (const bf16*)a.v + b * a.svb + h * a.svh + (lane >> 3) * a.svn + row_piece(lane) : (const bf16*)a.vt + (int64_t)bh * N1 * kTile + unit;
+    const int64_t v_block = ROWS ? kBlk * a.svn : kTile;
     SharedList sl = shared_list(a.lvl, a.levels, a.N, bh, g, lane);
     bf16* const sh0 = &sh[0][0][0];
     auto issue_group = [&](int grp) __attribute__((always_inline)) {   // this wave brings in block kGroup*grp + wave
@@ -252,19 +307,26 @@ __global__ __launch_bounds__(256, Q == 1 ? 4 : 3) void attn_fwd_kernel(llsa_attn
         copy16_global_to_lds<512>(vb + lane * 8, dst + kTile);
     };
     const int n_groups = sl.n_blocks / kGroup;                // every level's count is a multiple of kGroup (host checks)
+    QueryRows<Q> rows;
+    if constexpr (ROWS) request_queries<Q>(rows, a, b, h, g, lane);
     issue_group(0);
     const int* ip = a.idx + ((int64_t)bh * N1 + g) * T;
     MergedLists<Q, R> ml = merge_lists<Q, R>(ip, min(T, kWave * R / Q), N1, lane, order[wave]);
 
-    bf16x8 bq[Q][2];
-    SoftmaxState st[Q];
+    bf16x8 bq[Q][2];               // 1/sqrt(64) is a power of two: scaling q before the product (as the
+    SoftmaxState st[Q];            // reference does) equals scaling the fp32 scores, done in the exponent
+    if constexpr (ROWS) {
+        finish_queries<Q>(bq, rows, a, lane, &sh[1][wave][0]);          // (the second buffer is not filled before the barrier of group 0)
+    } else {
 #pragma unroll
-    for (int u = 0; u < Q; u++) {
-        const bf16* qp = (const bf16*)a.qr + ((int64_t)bh * N1 + g + u) * kTile + lane * 8;
-        bq[u][0] = ld16(qp);       // 1/sqrt(64) is a power of two: scaling q before the product (as the
-        bq[u][1] = ld16(qp + 512); // reference does) equals scaling the fp32 scores, done in the exponent
-        init_state(st[u]);
+        for (int u = 0; u < Q; u++) {
+            const bf16* qp = (const bf16*)a.qr + ((int64_t)bh * N1 + g + u) * kTile + lane * 8;
+            bq[u][0] = ld16(qp);
+            bq[u][1] = ld16(qp + 512);
+        }
     }
+#pragma unroll
+    for (int u = 0; u < Q; u++) init_state(st[u]);
     // ---- shared blocks, out of LDS.  The barrier at the top of round grp says two things: every
     // wave's part of group grp has landed, and every wave is done reading the other buffer
     // (group grp - 1), which the next fetch overwrites.  (LDS reads of a group come before the next fetch: the compiler
@@ -335,19 +397,21 @@ __global__ __launch_bounds__(256, Q == 1 ? 4 : 3) void attn_fwd_kernel(llsa_attn
             bf16* slot = slots + (s & 1) * (2 * kTile);
 #pragma unroll
             for (int j = 0; j < 2; j++) {
-                const int64_t at = (int64_t)ml.block(min(2 * s + j, ml.n - 1)) * kTile;
-                const bf16 *kb = kr + at, *vb = vr + at;
+                const int64_t blk = ml.block(min(2 * s + j, ml.n - 1));
+                const bf16 *kb = kr + blk * kTile, *vb = vr + blk * v_block;
                 dst.k[j][0] = ld16(kb + lane * 8);
                 dst.k[j][1] = ld16(kb + lane * 8 + 512);
-                copy16_global_to_lds(vb + unit, slot + j * kTile);
-                copy16_global_to_lds<512>(vb + unit, slot + j * kTile);
+                copy16_global_to_lds(vb, slot + j * kTile);
+                if constexpr (ROWS) copy16_global_to_lds(vb + 8 * a.svn, slot + j * kTile + 512);
+                else copy16_global_to_lds<512>(vb, slot + j * kTile);
             }
         };
         auto work = [&](int s, KeyRegs<2>& cur, KeyRegs<2>& nxt) __attribute__((always_inline)) {
             const unsigned m0 = ml.rows(2 * s), m1 = 2 * s + 1 < ml.n ? ml.rows(2 * s + 1) : 0u;
             wait_vm0();
             ValueRegs<2> v;
-            load_values_fine(v, slots + (s & 1) * (2 * kTile), lane);
+            if constexpr (ROWS) load_values_fine_rows(v, slots + (s & 1) * (2 * kTile), lane);
+            else load_values_fine(v, slots + (s & 1) * (2 * kTile), lane);
             if (s + 1 < n_steps) fetch(s + 1, nxt);
             if ((m0 & m1) == (1u << Q) - 1u) {
                 compute_step<Q>(st, bq, cur, v);
@@ -396,7 +460,14 @@ static int attn_fwd(const llsa_attn_fwd_args* a, const llsa_transpose_job* jobs,
     LLSA_REQUIRE(a != nullptr, "attn_fwd: null args");
     LLSA_REQUIRE(a->levels >= 1 && a->levels <= LLSA_MAX_LEVELS, "attn_fwd: levels must be 1..%d", LLSA_MAX_LEVELS);
     LLSA_REQUIRE(a->B > 0 && a->H > 0 && a->N > 0, "attn_fwd: bad B/H/N");
-    LLSA_REQUIRE(a->qr && a->kr && a->vt && a->idx && a->o && a->lse, "attn_fwd: null tensor");
+    const bool rows_form = a->q != nullptr;
+    LLSA_REQUIRE(a->kr && a->idx && a->o && (rows_form ? a->v != nullptr : a->qr && a->vt && a->lse), "attn_fwd: null tensor");
+    LLSA_REQUIRE(!rows_form || jobs == nullptr, "attn_fwd: no index transposes beside a forward on rows");
+    if (rows_form) {
+        LLSA_REQUIRE(aligned16(a->q) && aligned16(a->v) && aligned16(a->freq_q), "attn_fwd: tensors must be 16-byte aligned");
+        for (const int64_t st : {a->sqb, a->sqh, a->sqn, a->svb, a->svh, a->svn}) LLSA_REQUIRE(stride_ok(st), "attn_fwd: rows must be 16-byte aligned");
+        LLSA_REQUIRE(a->gamma_q == nullptr || a->eps_q >= 0.f, "attn_fwd: eps must be >= 0");
+    }
     LLSA_REQUIRE(a->T >= 4 && a->T % 4 == 0 && a->T <= a->N / 16, "attn_fwd: topk=%d must be a multiple of 4 and <= N/16", a->T);
     const int64_t mult = coarsest_multiple(a->levels);
     LLSA_REQUIRE(a->N % mult == 0,
@@ -435,9 +506,15 @@ static int attn_fwd(const llsa_attn_fwd_args* a, const llsa_transpose_job* jobs,
     const int rows = ride ? (int)list_rows : 0;
     const dim3 grid(width, BH + rows);
     const hipStream_t st = (hipStream_t)stream;
-    if (!pairs) hipLaunchKernelGGL(HIP_KERNEL_NAME(attn_fwd_kernel<1, 1>), grid, dim3(256), 0, st, *a, lists, rows);
-    else if (a->T <= 32) hipLaunchKernelGGL(HIP_KERNEL_NAME(attn_fwd_kernel<2, 1>), grid, dim3(256), 0, st, *a, lists, rows);
-    else hipLaunchKernelGGL(HIP_KERNEL_NAME(attn_fwd_kernel<2, 2>), grid, dim3(256), 0, st, *a, lists, rows);
+#define LLSA_FWD(Q, R)                                                                                                                    \
+    do {                                                                                                                                  \
+        if (rows_form) hipLaunchKernelGGL(HIP_KERNEL_NAME(attn_fwd_kernel<Q, R, true>), grid, dim3(256), 0, st, *a, lists, rows);         \
+        else hipLaunchKernelGGL(HIP_KERNEL_NAME(attn_fwd_kernel<Q, R, false>), grid, dim3(256), 0, st, *a, lists, rows);                  \
+    } while (0)
+    if (!pairs) LLSA_FWD(1, 1);
+    else if (a->T <= 32) LLSA_FWD(2, 1);
+    else LLSA_FWD(2, 2);
+#undef LLSA_FWD
     const int rc = launch_status("attn_fwd");
     if (rc != 0 || jobs == nullptr || ride) return rc;
     return llsa_transpose_indices_multi(jobs, n_jobs, a->B, a->H, stream);

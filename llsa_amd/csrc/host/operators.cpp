@@ -215,6 +215,7 @@ constexpr int kL = LLSA_MAX_LEVELS;
 struct Layout {
     int64_t n[kL + 2];
     int L, chunk;
+    bool rows;                                              // the forward reads q and v as rows (no gradients wanted)
     int32_t topk[kL];
     int64_t pq[kL + 1], pk[kL + 1], pv[kL + 1];             // pooled rows, index = level
     int64_t qr, kr, vr;                                     // operand tiles of the tokens
@@ -240,16 +241,20 @@ struct Layout {
         // (the selection reads the keys as tiles: rows of k and v are wanted only where the next pooling pass starts from them)
         for (int l = 1; l <= L; l++) pk[l] = take(n[l] * 128, l % 2 == 0 && l < L);
         for (int l = 1; l <= L; l++) pv[l] = take(n[l] * 128, l % 2 == 0 && l < L);
-        qr = take(n[1] * 2048);
+        // Without gradients the forward reads q and v as rows, and the pooling pass writes no tiles of them: 8 x 65536 tokens of one level 683 -> 660 us, 96 x
+        // 4096 143 -> 132, 6 x 65536 of two levels 214 -> 199, 3 x 49152 193.0 -> 191.2.  But a wave then starts with rows that are further away and have to be
+        // rotated, which a short pass waits for: 8 x 16384 53.4 / 54.9, 15 x 7168 57.4 / 58.9, 24 x 4096 50.8 / 51.0, 6 x 1024 16.6 / 16.8; 2 x 65536 196.2 / 193.3.
+        rows = !grad && BH * N > (int64_t(1) << 17);
+        qr = take(n[1] * 2048, !rows);
         kr = take(n[1] * 2048);
-        vr = take(n[1] * 2048);
+        vr = take(n[1] * 2048, !rows);
         for (int l = 1; l <= L; l++) {
             pkr[l] = take(n[l + 1] * 2048);
             pvr[l] = take(n[l + 1] * 2048, grad);
             pvt[l] = take(n[l + 1] * 2048);
         }
         for (int l = 0; l < L; l++) sel[l] = take(4 * n[l + 1] * topk[l]);
-        lse = take(4 * N);
+        lse = take(4 * N, !rows);
         chunk = lib.fine_chunk_for(static_cast<int>(B), static_cast<int>(H), static_cast<int>(N), topk[0]);
         if (grad) {
             for (int l = 0; l < L; l++) {
@@ -514,6 +519,15 @@ Tensor attend(const std::shared_ptr<Library>& lib, const Tensor& q_in, const Ten
 
         llsa_attn_fwd_args f{};
         f.qr = pa(y.qr); f.kr = pa(y.kr); f.vt = pa(y.vr); f.idx = ints(y.sel[0]);
+        if (y.rows) {
+            f.q = q.data_ptr(); f.sqb = q.stride(0); f.sqh = q.stride(1); f.sqn = q.stride(2);
+            f.v = v.data_ptr(); f.svb = v.stride(0); f.svh = v.stride(1); f.svn = v.stride(2);
+            if (freq.defined()) f.freq_q = freq.data_ptr();
+            if (gq.defined()) {
+                f.gamma_q = gq.data_ptr<float>();
+                f.eps_q = static_cast<float>(eps);
+            }
+        }
         f.o = o.data_ptr(); f.sob = o.stride(0); f.soh = o.stride(1); f.son = o.stride(2);
         f.lse = static_cast<float*>(pa(y.lse));
         f.B = b; f.H = h; f.N = static_cast<int32_t>(N); f.T = y.topk[0]; f.levels = L;
