@@ -43,7 +43,7 @@ extern "C" {
 #define LLSA_DTYPE_BF16 0
 #define LLSA_DTYPE_F32 1
 
-#define LLSA_ABI_VERSION 212     /* changes with every change of a signature or argument structure below */
+#define LLSA_ABI_VERSION 213     /* changes with every change of a signature or argument structure below */
 int llsa_version(void);          /* LLSA_ABI_VERSION of the built library                                    */
 const char* llsa_last_error_string(void);
 
@@ -215,9 +215,13 @@ typedef struct llsa_attn_fwd_args {
     const void* q;  int64_t sqb, sqh, sqn;
     const void* v;  int64_t svb, svh, svn;
     const void* freq_q; const float* gamma_q; float eps_q; int32_t reserved2;
+    /* pq not NULL (no backward will follow; sizes that llsa_attn_fwd_selects answers 1 for): the pooled queries (B,H,N/16,64); every
+     * query block selects its T blocks itself, as llsa_topk_dense with rounded scores on pq and level 1's keys does, and idx is not read. */
+    const void* pq;
 } llsa_attn_fwd_args;
 
 int llsa_attn_fwd(const llsa_attn_fwd_args* a, void* stream);
+int llsa_attn_fwd_selects(int B, int H, int N, int T, int levels);
 /* How many query blocks (1 or 2) a wave of llsa_attn_fwd (backward = 0) or of llsa_attn_bwd's dQ kernel (backward = 1) takes at
  * these sizes; topk: of every level, finest first. */
 int llsa_query_blocks_per_wave(int B, int H, int N, const int32_t* topk, int levels, int backward);

@@ -44,7 +44,7 @@ class AttnFwdArgs(C.Structure):
                 ("lvl", FwdLevel * MAX_LEVELS),
                 ("q", c_void_p), ("sqb", c_int64), ("sqh", c_int64), ("sqn", c_int64),
                 ("v", c_void_p), ("svb", c_int64), ("svh", c_int64), ("svn", c_int64),
-                ("freq_q", c_void_p), ("gamma_q", c_void_p), ("eps_q", c_float), ("reserved2", c_int32)]
+                ("freq_q", c_void_p), ("gamma_q", c_void_p), ("eps_q", c_float), ("reserved2", c_int32), ("pq", c_void_p)]
 
 
 def _t3(name):
@@ -107,6 +107,7 @@ _SIGNATURES = {
     "llsa_topk_cascade_tiles": (c_int, [c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_int, c_void_p]),
     "llsa_topk_cascade_max_parents": (c_int, []),
     "llsa_attn_fwd": (c_int, [C.POINTER(AttnFwdArgs), c_void_p]),
+    "llsa_attn_fwd_selects": (c_int, [c_int, c_int, c_int, c_int, c_int]),
     "llsa_query_blocks_per_wave": (c_int, [c_int, c_int, c_int, C.POINTER(c_int32), c_int, c_int]),
     "llsa_transpose_indices": (c_int, [c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_int, c_int, c_void_p]),
     "llsa_transpose_indices_multi": (c_int, [C.POINTER(TransposeJob), c_int, c_int, c_int, c_void_p]),
@@ -123,7 +124,7 @@ _SIGNATURES = {
 
 EXPORTS = tuple(_SIGNATURES)
 CHUNK_FINE_MAX = 256                                        # LLSA_CHUNK_FINE_MAX of include/llsa_hip.h
-ABI_VERSION = 212                                           # LLSA_ABI_VERSION
+ABI_VERSION = 213                                           # LLSA_ABI_VERSION
 STATIC_PARTIALS_MAX = 262144                                # LLSA_STATIC_PARTIALS_MAX
 
 

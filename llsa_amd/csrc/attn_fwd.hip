@@ -248,6 +248,54 @@ __device__ __forceinline__ void finish_query_block(const llsa_attn_fwd_args& a, 
     if (quad == 0 && a.lse != nullptr) a.lse[(int64_t)bh * a.N + g * kBlk + r] = (st.m2 + __builtin_amdgcn_logf(L)) * kLn2;
 }
 
+// One query block's selection among the 64 KEYS blocks of a one-level call, by its wave: the T best pooled keys, best
+// first, as topk_dense_kernel finds them -- the same products, scores rounded to bf16, equal ones by index.  Every column of the score tiles is the
+// block's pooled query, so that lane l holds key 16 (l%16 / 4) + 4 (l/16) + l%4 of every 64 and ranks them against all others, handed round with
+// readlane.  Result: entry i in lane i, through `scratch` (64 ints of LDS of the wave).
+template <int KEYS>
+__device__ __forceinline__ int select_blocks(const bf16* pq_row, const bf16* key_tiles, int T, int lane, int* scratch) {
+    const int quad = lane >> 4, r = lane & 15;
+    const bf16x8 q0 = ld16(pq_row + quad * 8), q1 = ld16(pq_row + quad * 8 + 32);
+    bf16x8 k[KEYS][4][2];                                     // (all loads in flight together)
+#pragma unroll
+    for (int m = 0; m < KEYS; m++)
+#pragma unroll
+        for (int a = 0; a < 4; a++) {
+            k[m][a][0] = ld16(key_tiles + (m * 4 + a) * kTile + lane * 8);
+            k[m][a][1] = ld16(key_tiles + (m * 4 + a) * kTile + 512 + lane * 8);
+        }
+    unsigned key[KEYS];
+    int rank[KEYS];
+#pragma unroll
+    for (int m = 0; m < KEYS; m++) {
+        float own = 0.f;
+#pragma unroll
+        for (int a = 0; a < 4; a++) {
+            f32x4 z = {0.f, 0.f, 0.f, 0.f};
+            const f32x4 s = mfma_bf16(k[m][a][1], q1, mfma_bf16(k[m][a][0], q0, z));
+#pragma unroll
+            for (int e = 0; e < 4; e++) own = r == 4 * a + e ? s[e] : own;
+        }
+        key[m] = packed_key(own, m * 64 + 16 * (r >> 2) + 4 * quad + (r & 3));
+        rank[m] = 0;
+    }
+#pragma unroll
+    for (int m = 0; m < KEYS; m++) {
+#pragma unroll 8
+        for (int j = 0; j < kWave; j++) {
+            const unsigned o = (unsigned)__builtin_amdgcn_readlane((int)key[m], j);
+#pragma unroll
+            for (int i = 0; i < KEYS; i++) rank[i] += o > key[i] ? 1 : 0;
+        }
+    }
+#pragma unroll
+    for (int m = 0; m < KEYS; m++)
+        if (rank[m] < T) scratch[rank[m]] = m * 64 + 16 * (r >> 2) + 4 * quad + (r & 3);
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    return scratch[min(lane, T - 1)];
+}
+
 // Q sibling query blocks per wave, 4 Q consecutive query blocks per workgroup.
 //
 // The pooled blocks -- the selected blocks of every pooled level below the coarsest and the coarsest level itself -- are
@@ -274,11 +322,12 @@ constexpr int kGridRows = 65535;                              // rows a grid can
 // ROWS (no backward will follow): q and v are read as the caller's rows.  Their tiles are then not written, which is a third of all that the pooling pass
 // moves; every block of v is still copied into LDS in two loads of whole lines.  8 x 65536 tokens, topk 8:
 // pooling 68.7 -> 45.2 us, forward 559 -> 570.
-template <int Q, int R, bool ROWS>
+// SELECT (no backward either; 64 SELECT blocks of one level, attn_fwd_selects): a wave selects its own blocks, and the selection's launch goes.
+template <int Q, int R, bool ROWS, int SELECT = 0>
 __global__ __launch_bounds__(256, Q == 1 ? 4 : 3) void attn_fwd_kernel(llsa_attn_fwd_args a, TrJobs lists, int list_rows) {
     __shared__ __align__(16) bf16 sh[2][kGroup][2 * kTile];
     __shared__ int order[4][R * kWave];
-    if (!ROWS && (int)blockIdx.y < list_rows) {
+    if (!ROWS && SELECT == 0 && (int)blockIdx.y < list_rows) {
         const int block = (int)(blockIdx.y * gridDim.x + blockIdx.x);
         int* const lds = reinterpret_cast<int*>(&sh[0][0][0]);
         if (block < lists.wgs * ((int)gridDim.y - list_rows)) transpose_block<256>(lists, block, lds, lds + kTrLdsFwd);
@@ -310,8 +359,16 @@ __global__ __launch_bounds__(256, Q == 1 ? 4 : 3) void attn_fwd_kernel(llsa_attn
     QueryRows<Q> rows;
     if constexpr (ROWS) request_queries<Q>(rows, a, b, h, g, lane);
     issue_group(0);
-    const int* ip = a.idx + ((int64_t)bh * N1 + g) * T;
-    MergedLists<Q, R> ml = merge_lists<Q, R>(ip, min(T, kWave * R / Q), N1, lane, order[wave]);
+    const int* ip = SELECT > 0 ? nullptr : a.idx + ((int64_t)bh * N1 + g) * T;
+    MergedLists<Q, R> ml;
+    if constexpr (SELECT > 0) {
+        static_assert(Q == 1 && R == 1, "a row of its own per wave");
+        ml.packed[0] = select_blocks<SELECT>((const bf16*)a.pq + ((int64_t)bh * N1 + g) * kD, (const bf16*)a.lvl[0].kr + (int64_t)bh * N1 * kD, T, lane, order[wave]) |
+                       (1 << kSetShift);
+        ml.n = T;
+    } else {
+        ml = merge_lists<Q, R>(ip, min(T, kWave * R / Q), N1, lane, order[wave]);
+    }
 
     bf16x8 bq[Q][2];               // 1/sqrt(64) is a power of two: scaling q before the product (as the
     SoftmaxState st[Q];            // reference does) equals scaling the fp32 scores, done in the exponent
@@ -431,7 +488,7 @@ __global__ __launch_bounds__(256, Q == 1 ? 4 : 3) void attn_fwd_kernel(llsa_attn
         }
     };
     fine();
-    if constexpr (Q == 1) {                                   // longer lists: 64 entries at a time
+    if constexpr (Q == 1 && SELECT == 0) {                        // longer lists: 64 entries at a time
         for (int c0 = kWave * R; c0 < T; c0 += kWave * R) {
             ml = merge_lists<Q, R>(ip + c0, min(T - c0, kWave * R), N1, lane, order[wave]);
             fine();
@@ -455,19 +512,32 @@ static int64_t plan_list_rows(const llsa_transpose_job* jobs, int n_jobs, int B,
 }
 static int forward_width(int N, bool pairs) { return N / (pairs ? 128 : 64); }   // workgroups of a (b,h); a multiple of 8: N is one of 1024
 
+// Whether the forward selects by itself where no backward follows.  A wave ranks 64 keys in 0.4 us and 128 in 1.2, which waves in the same SIMD add up
+// to, where the launch it saves takes 6 to 10 and its gap.  A pass, us, launch of its own / in the forward:
+//   1024 tokens, topk 8: 6 heads 18.7 / 14.9;  24 25.6 / 22.3;  96 38.8 / 35.3;  128 44.4 / 41.4;  topk 64: 6 34.6 / 24.9;  128 107 / 95
+//   2048 tokens, topk 8: 1 head 18.6 / 16.8;  6 20.9 / 18.5;  24 30.6 / 29.7;  48 40.2 / 40.8;  64 45.8 / 48.5;  topk 32: 6 26.6 / 23.0;  64 70.9 / 69.2
+//   3072 and 4096 tokens, 192 and 256 keys, topk 8: 1 head 20.4 / 21.8 and 21.3 / 25.7
+static bool attn_fwd_selects(int64_t BH, int N, int T, int levels) {
+    const int32_t topk[1] = {T};
+    if (levels != 1 || (N != 1024 && N != 2048) || T < 4 || T > 64 || T % 4 != 0 || two_blocks_per_wave(BH, N, topk, 1, true)) return false;
+    return BH * (N / kBlk) <= (N == 1024 || T >= 32 ? 8192 : 3072);
+}
+
 // jobs: the index transposes that ride along, or nullptr
 static int attn_fwd(const llsa_attn_fwd_args* a, const llsa_transpose_job* jobs, int n_jobs, void* stream) {
     LLSA_REQUIRE(a != nullptr, "attn_fwd: null args");
     LLSA_REQUIRE(a->levels >= 1 && a->levels <= LLSA_MAX_LEVELS, "attn_fwd: levels must be 1..%d", LLSA_MAX_LEVELS);
     LLSA_REQUIRE(a->B > 0 && a->H > 0 && a->N > 0, "attn_fwd: bad B/H/N");
-    const bool rows_form = a->q != nullptr;
-    LLSA_REQUIRE(a->kr && a->idx && a->o && (rows_form ? a->v != nullptr : a->qr && a->vt && a->lse), "attn_fwd: null tensor");
+    const bool rows_form = a->q != nullptr, selects = a->pq != nullptr;
+    LLSA_REQUIRE(a->kr && (a->idx || selects) && a->o && (rows_form ? a->v != nullptr : a->qr && a->vt && a->lse), "attn_fwd: null tensor");
     LLSA_REQUIRE(!rows_form || jobs == nullptr, "attn_fwd: no index transposes beside a forward on rows");
     if (rows_form) {
         LLSA_REQUIRE(aligned16(a->q) && aligned16(a->v) && aligned16(a->freq_q), "attn_fwd: tensors must be 16-byte aligned");
         for (const int64_t st : {a->sqb, a->sqh, a->sqn, a->svb, a->svh, a->svn}) LLSA_REQUIRE(stride_ok(st), "attn_fwd: rows must be 16-byte aligned");
         LLSA_REQUIRE(a->gamma_q == nullptr || a->eps_q >= 0.f, "attn_fwd: eps must be >= 0");
     }
+    LLSA_REQUIRE(!selects || (aligned16(a->pq) && !rows_form && jobs == nullptr && attn_fwd_selects((int64_t)a->B * a->H, a->N, a->T, a->levels)),
+                 "attn_fwd: these sizes are not selected in the forward");
     LLSA_REQUIRE(a->T >= 4 && a->T % 4 == 0 && a->T <= a->N / 16, "attn_fwd: topk=%d must be a multiple of 4 and <= N/16", a->T);
     const int64_t mult = coarsest_multiple(a->levels);
     LLSA_REQUIRE(a->N % mult == 0,
@@ -511,7 +581,9 @@ static int attn_fwd(const llsa_attn_fwd_args* a, const llsa_transpose_job* jobs,
         if (rows_form) hipLaunchKernelGGL(HIP_KERNEL_NAME(attn_fwd_kernel<Q, R, true>), grid, dim3(256), 0, st, *a, lists, rows);         \
         else hipLaunchKernelGGL(HIP_KERNEL_NAME(attn_fwd_kernel<Q, R, false>), grid, dim3(256), 0, st, *a, lists, rows);                  \
     } while (0)
-    if (!pairs) LLSA_FWD(1, 1);
+    if (selects && a->N == 1024) hipLaunchKernelGGL(HIP_KERNEL_NAME(attn_fwd_kernel<1, 1, false, 1>), grid, dim3(256), 0, st, *a, lists, rows);
+    else if (selects) hipLaunchKernelGGL(HIP_KERNEL_NAME(attn_fwd_kernel<1, 1, false, 2>), grid, dim3(256), 0, st, *a, lists, rows);
+    else if (!pairs) LLSA_FWD(1, 1);
     else if (a->T <= 32) LLSA_FWD(2, 1);
     else LLSA_FWD(2, 2);
 #undef LLSA_FWD
@@ -530,6 +602,10 @@ static int check_plan_query(const char* what, int B, int H, int N, const int32_t
 extern "C" int llsa_query_blocks_per_wave(int B, int H, int N, const int32_t* topk, int levels, int backward) {
     if (const int rc = check_plan_query("query_blocks_per_wave", B, H, N, topk, levels)) return rc;
     return two_blocks_per_wave((int64_t)B * H, N, topk, levels, backward == 0) ? 2 : 1;
+}
+
+extern "C" int llsa_attn_fwd_selects(int B, int H, int N, int T, int levels) {
+    return B > 0 && H > 0 && N > 0 && attn_fwd_selects((int64_t)B * H, N, T, levels);
 }
 
 extern "C" int llsa_lists_ride(int B, int H, int N, const int32_t* topk, int levels) {

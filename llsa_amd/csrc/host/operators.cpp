@@ -101,6 +101,7 @@ struct Library {
     decltype(&llsa_topk_cascade_max_parents) topk_cascade_max_parents;
     decltype(&llsa_attn_fwd) attn_fwd;
     decltype(&llsa_attn_fwd_lists) attn_fwd_lists;
+    decltype(&llsa_attn_fwd_selects) attn_fwd_selects;
     decltype(&llsa_transpose_indices_multi) transpose_indices_multi;
     decltype(&llsa_transpose_one_launch) transpose_one_launch;
     decltype(&llsa_transpose_nested_bytes) transpose_nested_bytes;
@@ -121,6 +122,7 @@ struct Library {
         get("llsa_topk_cascade_max_parents", topk_cascade_max_parents);
         get("llsa_attn_fwd", attn_fwd);
         get("llsa_attn_fwd_lists", attn_fwd_lists);
+        get("llsa_attn_fwd_selects", attn_fwd_selects);
         get("llsa_transpose_indices_multi", transpose_indices_multi);
         get("llsa_transpose_one_launch", transpose_one_launch);
         get("llsa_transpose_nested_bytes", transpose_nested_bytes);
@@ -488,7 +490,11 @@ Tensor attend(const std::shared_ptr<Library>& lib, const Tensor& q_in, const Ten
         // Selection, coarse to fine: a dense top-k over the coarsest level's tokens (each of them is a block of the level
         // below), then level by level among the blocks under the parent's selection.
         int first = L - 1;               // the first parent-guided selection still to do
-        if (L >= 2 && n[L] <= lib->topk_cascade_max_parents() && (n[L] <= 64 || B * H * n[L] < 2048)) {
+        // (without gradients nobody else reads the selection of a short sequence: every wave of the forward makes its own)
+        const bool selects = !grad && !y.rows && lib->attn_fwd_selects(b, h, static_cast<int>(N), y.topk[0], L) != 0;
+        if (selects) {
+            first = 0;
+        } else if (L >= 2 && n[L] <= lib->topk_cascade_max_parents() && (n[L] <= 64 || B * H * n[L] < 2048)) {
             // the dense selection rides in the workgroups of the first parent-guided one: one launch less (more than 64
             // parent tokens in a large grid: sixteen rows a wave side by side in a launch of their own are cheaper)
             lib->check(lib->topk_cascade_tiles(pa(y.pq[L]), pa(y.pkr[L]), ints(y.sel[L - 1]), pa(y.pq[L - 1]), pa(y.pkr[L - 1]), ints(y.sel[L - 2]), b, h,
@@ -519,6 +525,7 @@ Tensor attend(const std::shared_ptr<Library>& lib, const Tensor& q_in, const Ten
 
         llsa_attn_fwd_args f{};
         f.qr = pa(y.qr); f.kr = pa(y.kr); f.vt = pa(y.vr); f.idx = ints(y.sel[0]);
+        if (selects) f.pq = pa(y.pq[1]);
         if (y.rows) {
             f.q = q.data_ptr(); f.sqb = q.stride(0); f.sqh = q.stride(1); f.sqn = q.stride(2);
             f.v = v.data_ptr(); f.svb = v.stride(0); f.svh = v.stride(1); f.svn = v.stride(2);

@@ -127,6 +127,19 @@ __device__ __forceinline__ bool rows_wide(const void* p, int64_t sb, int64_t sh,
     return ((reinterpret_cast<uintptr_t>(p) & 15u) | ((sb | sh | sn) & 7)) == 0;
 }
 
+// Unsigned integers that sort like the floats; 0 is kept for empty slots (a NaN becomes 1, below every number).
+__device__ __forceinline__ unsigned ordered_key(float f) {
+    const unsigned b = __float_as_uint(f);
+    const unsigned k = (b & 0x80000000u) ? ~b : (b | 0x80000000u);
+    return (f != f || k == 0u) ? 1u : k;
+}
+// Score rounded to bf16 and key index in one integer: the larger is the better key, equal scores by smaller index, and no
+// two keys of a row are equal.  For indices below 2^16 - 1 (a NaN sorts below every number, by index as well).
+constexpr int kMaxPackedKeys = 65535;
+__device__ __forceinline__ unsigned packed_key(float f, int idx) {
+    return (ordered_key(rn_bf16(f)) & 0xFFFF0000u) | (unsigned)(0xFFFF - idx);
+}
+
 // Operand tiles.  The attention kernels never read K/V/Q/dO row-major: a 16-row x 64-channel
 // block (1024 bf16 = 2 KB) is stored twice, each time in exactly the order the 64 lanes of a
 // wave consume it as an MFMA operand, so that every operand load is one fully coalesced

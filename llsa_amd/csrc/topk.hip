@@ -20,18 +20,6 @@ namespace llsa {
 constexpr int kMaxT = 64;        // largest supported top-k
 constexpr int kMaxCand = 512;    // candidates per parent in the sparse kernel (T2 * 16)
 
-// Unsigned integers that sort like the floats; 0 is kept for empty slots (a NaN becomes 1, below every number).
-__device__ __forceinline__ unsigned ordered_key(float f) {
-    const unsigned b = __float_as_uint(f);
-    const unsigned k = (b & 0x80000000u) ? ~b : (b | 0x80000000u);
-    return (f != f || k == 0u) ? 1u : k;
-}
-// Score rounded to bf16 and key index in one integer: the larger is the better key, equal scores by smaller index, and no
-// two keys of a row are equal.  For indices below 2^16 - 1 (a NaN sorts below every number, by index as well).
-constexpr int kMaxPackedKeys = 65535;
-__device__ __forceinline__ unsigned packed_key(float f, int idx) {
-    return (ordered_key(rn_bf16(f)) & 0xFFFF0000u) | (unsigned)(0xFFFF - idx);
-}
 // Any score, any index: the same order in 64 bits.
 __device__ __forceinline__ unsigned long long wide_key(unsigned score_key, int idx) {
     return ((unsigned long long)score_key << 32) | (unsigned)(0x7FFFFFFF - idx);

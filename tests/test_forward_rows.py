@@ -1,5 +1,5 @@
-"""The forward without gradients, which reads q and v as rows and normalises and rotates q itself, gives bit for bit what the forward on the
-operand tiles gives: one and two query blocks a wave, lists of more than one and two registers, RoPE and qk norm, rows of a packed
+"""The forward without gradients, which selects by itself at 1024 and 2048 tokens and, at the larger sizes, reads q and v as rows and
+normalises and rotates q itself, gives bit for bit what the forward with gradients gives: one and two query blocks a wave, lists of more than one and two registers, RoPE and qk norm, rows of a packed
 projection."""
 import pytest
 import torch
@@ -84,6 +84,31 @@ def test_launch_cpu(monkeypatch, rope, norm):
 @pytest.mark.parametrize("N,T,T2", [(1024, 4, 0), (2048, 128, 0), (7168, 12, 0), (16384, 8, 4)])
 def test_launch_gpu(monkeypatch, N, T, T2, rope, norm):
     _check_launch(torch.device("cuda"), monkeypatch, N, T, T2, rope, norm)
+
+
+@pytest.mark.parametrize("N,T", [(1024, 4), (2048, 64)])
+def test_selecting_cpu(N, T):
+    with override_library_for_tests(emu_lib()):
+        assert current_lib().attn_fwd_selects(1, 1, N, T, 1)
+        _check(torch.device("cpu"), 1, 1, N, (T,), False, False, False)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("B,H,N,T", [(1, 6, 1024, 8), (1, 1, 1024, 64), (3, 5, 1024, 12), (8, 16, 1024, 20), (1, 1, 2048, 4), (2, 3, 2048, 64), (4, 6, 2048, 16)])
+def test_selecting_gpu(B, H, N, T):
+    assert current_lib().attn_fwd_selects(B, H, N, T, 1)
+    _check(torch.device("cuda"), B, H, N, (T,), True, False, True)
+    with pytest.MonkeyPatch.context() as m:                   # equal scores everywhere: by index
+        m.setattr(torch, "randn", lambda *s, generator=None: torch.ones(*s))
+        _check(torch.device("cuda"), B, H, N, (T,), False, False, False)
+
+
+def test_which_sizes_select():
+    with override_library_for_tests(emu_lib()):
+        ask = current_lib().attn_fwd_selects
+        assert ask(8, 16, 1024, 8, 1) and not ask(3, 43, 1024, 8, 1)
+        assert ask(4, 6, 2048, 8, 1) and not ask(5, 5, 2048, 8, 1) and ask(8, 8, 2048, 32, 1) and not ask(5, 13, 2048, 32, 1)
+        assert not ask(1, 1, 3072, 8, 1) and not ask(1, 1, 4096, 8, 1) and not ask(1, 1, 16384, 8, 2) and not ask(1, 1, 1024, 6, 1)
 
 
 # more than 131072 tokens over all heads; one and two query blocks a wave, lists in one and two registers
