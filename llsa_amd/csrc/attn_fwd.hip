@@ -248,49 +248,14 @@ __device__ __forceinline__ void finish_query_block(const llsa_attn_fwd_args& a, 
     if (quad == 0 && a.lse != nullptr) a.lse[(int64_t)bh * a.N + g * kBlk + r] = (st.m2 + __builtin_amdgcn_logf(L)) * kLn2;
 }
 
-// One query block's selection among the 64 KEYS blocks of a one-level call, by its wave: the T best pooled keys, best
-// first, as topk_dense_kernel finds them -- the same products, scores rounded to bf16, equal ones by index.  Every column of the score tiles is the
-// block's pooled query, so that lane l holds key 16 (l%16 / 4) + 4 (l/16) + l%4 of every 64 and ranks them against all others, handed round with
-// readlane.  Result: entry i in lane i, through `scratch` (64 ints of LDS of the wave).
+// One query block's selection among the 64 KEYS blocks of a one-level call, by its wave: the T best pooled keys, best first, as
+// topk_dense_kernel finds them.  Result: entry i in lane i, through `scratch` (64 ints of LDS of the wave).
 template <int KEYS>
 __device__ __forceinline__ int select_blocks(const bf16* pq_row, const bf16* key_tiles, int T, int lane, int* scratch) {
-    const int quad = lane >> 4, r = lane & 15;
-    const bf16x8 q0 = ld16(pq_row + quad * 8), q1 = ld16(pq_row + quad * 8 + 32);
-    bf16x8 k[KEYS][4][2];                                     // (all loads in flight together)
+    RankedKeys<KEYS> ranked = rank_keys<KEYS>(pq_row, key_tiles, lane * 8, 512 + lane * 8, 64 * KEYS, lane);
 #pragma unroll
     for (int m = 0; m < KEYS; m++)
-#pragma unroll
-        for (int a = 0; a < 4; a++) {
-            k[m][a][0] = ld16(key_tiles + (m * 4 + a) * kTile + lane * 8);
-            k[m][a][1] = ld16(key_tiles + (m * 4 + a) * kTile + 512 + lane * 8);
-        }
-    unsigned key[KEYS];
-    int rank[KEYS];
-#pragma unroll
-    for (int m = 0; m < KEYS; m++) {
-        float own = 0.f;
-#pragma unroll
-        for (int a = 0; a < 4; a++) {
-            f32x4 z = {0.f, 0.f, 0.f, 0.f};
-            const f32x4 s = mfma_bf16(k[m][a][1], q1, mfma_bf16(k[m][a][0], q0, z));
-#pragma unroll
-            for (int e = 0; e < 4; e++) own = r == 4 * a + e ? s[e] : own;
-        }
-        key[m] = packed_key(own, m * 64 + 16 * (r >> 2) + 4 * quad + (r & 3));
-        rank[m] = 0;
-    }
-#pragma unroll
-    for (int m = 0; m < KEYS; m++) {
-#pragma unroll 8
-        for (int j = 0; j < kWave; j++) {
-            const unsigned o = (unsigned)__builtin_amdgcn_readlane((int)key[m], j);
-#pragma unroll
-            for (int i = 0; i < KEYS; i++) rank[i] += o > key[i] ? 1 : 0;
-        }
-    }
-#pragma unroll
-    for (int m = 0; m < KEYS; m++)
-        if (rank[m] < T) scratch[rank[m]] = m * 64 + 16 * (r >> 2) + 4 * quad + (r & 3);
+        if (ranked.rank[m] < T) scratch[ranked.rank[m]] = ranked.index(m, lane);
     __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
     __builtin_amdgcn_wave_barrier();
     return scratch[min(lane, T - 1)];

@@ -140,6 +140,56 @@ __device__ __forceinline__ unsigned packed_key(float f, int idx) {
     return (ordered_key(rn_bf16(f)) & 0xFFFF0000u) | (unsigned)(0xFFFF - idx);
 }
 
+// Up to 64 KEYS keys ranked against one query by one wave: the products topk_dense_kernel makes, scores rounded to bf16, equal ones by index.  Every
+// column of the score tiles is the query, so that lane l holds key 16 (l%16 / 4) + 4 (l/16) + l%4 of every 64 and counts the larger ones, handed
+// round with readlane: 0.4 us for 64 keys, where bisection and the exchange of its counts take several.  keys: sixteen at a time in kTile elements, a lane's pieces
+// at `first` and `second`; n (a multiple of 16) of them there are, the others rank last.
+template <int KEYS>
+struct RankedKeys {
+    int rank[KEYS];
+    __device__ __forceinline__ int index(int m, int lane) const { return m * 64 + 16 * ((lane & 15) >> 2) + 4 * (lane >> 4) + (lane & 3); }
+};
+template <int KEYS>
+__device__ __forceinline__ RankedKeys<KEYS> rank_keys(const bf16* q_row, const bf16* keys, int first, int second, int n, int lane) {
+    const int quad = lane >> 4, r = lane & 15;
+    const bf16x8 q0 = ld16(q_row + quad * 8), q1 = ld16(q_row + quad * 8 + 32);
+    bf16x8 k[KEYS][4][2];                                     // (all loads in flight together)
+#pragma unroll
+    for (int m = 0; m < KEYS; m++)
+#pragma unroll
+        for (int a = 0; a < 4; a++) {
+            const bf16* p = keys + min(m * 4 + a, n / 16 - 1) * (16 * kD);
+            k[m][a][0] = ld16(p + first);
+            k[m][a][1] = ld16(p + second);
+        }
+    RankedKeys<KEYS> ranked;
+    unsigned key[KEYS];
+#pragma unroll
+    for (int m = 0; m < KEYS; m++) {
+        float own = 0.f;
+#pragma unroll
+        for (int a = 0; a < 4; a++) {
+            f32x4 z = {0.f, 0.f, 0.f, 0.f};
+            const f32x4 s = mfma_bf16(k[m][a][1], q1, mfma_bf16(k[m][a][0], q0, z));
+#pragma unroll
+            for (int e = 0; e < 4; e++) own = r == 4 * a + e ? s[e] : own;
+        }
+        const int idx = ranked.index(m, lane);
+        key[m] = idx < n ? packed_key(own, idx) : 0u;
+        ranked.rank[m] = 0;
+    }
+#pragma unroll
+    for (int m = 0; m < KEYS; m++) {
+#pragma unroll 8
+        for (int j = 0; j < kWave; j++) {
+            const unsigned o = (unsigned)__builtin_amdgcn_readlane((int)key[m], j);
+#pragma unroll
+            for (int i = 0; i < KEYS; i++) ranked.rank[i] += o > key[i] ? 1 : 0;
+        }
+    }
+    return ranked;
+}
+
 // Operand tiles.  The attention kernels never read K/V/Q/dO row-major: a 16-row x 64-channel
 // block (1024 bf16 = 2 KB) is stored twice, each time in exactly the order the 64 lanes of a
 // wave consume it as an MFMA operand, so that every operand load is one fully coalesced
