@@ -494,9 +494,12 @@ Tensor attend(const std::shared_ptr<Library>& lib, const Tensor& q_in, const Ten
         const bool selects = !grad && !y.rows && lib->attn_fwd_selects(b, h, static_cast<int>(N), y.topk[0], L) != 0;
         if (selects) {
             first = 0;
-        } else if (L >= 2 && n[L] <= lib->topk_cascade_max_parents() && (n[L] <= 64 || B * H * n[L] < 2048)) {
-            // the dense selection rides in the workgroups of the first parent-guided one: one launch less (more than 64
-            // parent tokens in a large grid: sixteen rows a wave side by side in a launch of their own are cheaper)
+        } else if (L >= 2 && n[L] <= lib->topk_cascade_max_parents() && (n[L] <= 64 || (B * H * n[L] < 800 && y.topk[L - 1] > 4))) {
+            // The dense selection rides in the workgroups of the first parent-guided one: one launch less.  More than 64 parent tokens cost every
+            // workgroup more than sixteen rows of them cost a wave of their own launch: two launches / one, us, by groups over all heads
+            //   (topk 8/8) 256 (65536 tokens) 13.1 / 10.8;  384 (32768) 12.3 / 11.2;  576 (49152) 14.0 / 13.2;  1024 (65536) 15.5 / 16.2;  1536 17.6 / 20.4;
+            //   1920 (49152) 19.8 / 23.9;  (16/16) 576 17.5 / 16.6;  1024 19.4 / 20.1;  1536 22.8 / 25.6;  (64/32) 576 32.8 / 31.3;  1152 41.4 / 43.6
+            //   (8/4), one wave a group: 128 (32768) 11.1 / 13.4;  576 12.9 / 14.6;  1536 13.2 / 16.9
             lib->check(lib->topk_cascade_tiles(pa(y.pq[L]), pa(y.pkr[L]), ints(y.sel[L - 1]), pa(y.pq[L - 1]), pa(y.pkr[L - 1]), ints(y.sel[L - 2]), b, h,
                                                static_cast<int>(n[L - 1]), y.topk[L - 2], y.topk[L - 1], stream),
                        "topk_cascade");
