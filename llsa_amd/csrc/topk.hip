@@ -11,6 +11,7 @@
 //
 // The order is total -- higher score first, equal scores by smaller key index -- so the result does not depend on how the
 // work is split.
+#include <algorithm>
 #include "llsa_device.h"
 #include "llsa_host.h"
 #include "../../include/llsa_hip.h"
@@ -302,6 +303,18 @@ __global__ __launch_bounds__(64 * W) void topk_dense_kernel(const bf16* __restri
     }
     __syncthreads();
     write_winners<W>(win, n_win, T, out + ((int64_t)bh * n + q0) * T, T, tid, wide_index);
+}
+
+// Dense selection for n <= 64, scores rounded to bf16, in small grids: a wave per row ranks all its keys.  Sixteen rows a wave (topk_dense_kernel<4, 1>) take
+// fewer instructions over all rows, but a longer chain, which grows with T where the winners are ranked.
+__global__ __launch_bounds__(256) void topk_rank_kernel(const bf16* __restrict__ pq, const bf16* __restrict__ pk, int* __restrict__ out, int n, int T,
+                                                        int tiled) {
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int64_t row = (int64_t)blockIdx.y * n + blockIdx.x * 4 + wave;      // (n is a multiple of 16)
+    const KeyPieces pieces(tiled, lane);
+    const RankedKeys<1> ranked = rank_keys<1>(pq + row * kD, pk + (int64_t)blockIdx.y * n * kD, pieces.first, pieces.second, n, lane);
+    const int idx = ranked.index(0, lane);
+    if (ranked.rank[0] < T && idx < n) out[row * T + ranked.rank[0]] = idx;
 }
 
 // Dense selection for longer rows: two looks at all scores, and between them a bound of every row's T-th best.
@@ -774,7 +787,12 @@ static int topk_dense(const void* pq, const void* pk, int32_t* out_idx, int B, i
     LLSA_REQUIRE(aligned16(pq) && aligned16(pk), "topk_dense: inputs must be 16-byte aligned");
     const hipStream_t st = (hipStream_t)stream;
     const bf16 *q = (const bf16*)pq, *k = (const bf16*)pk;
-    if (n <= kRegMaxN) {
+    // By rows over all heads, us, sixteen a wave / one a wave, 64 keys out of tiles:  T = 4: 384 4.2 / 3.3, 1536 4.2 / 3.9, 6144 4.5 / 6.5;  T = 8: 384 5.1 / 3.3, 1536
+    // 5.2 / 3.9, 6144 5.4 / 6.4;  T = 16: 6144 7.1 / 6.5, 24576 8.5 / 17.2;  T = 32: 384 9.4 / 3.3, 6144 10.1 / 6.5, 24576 12.2 / 17.6;  T = 64: 384 11.6 / 3.4,
+    // 6144 12.7 / 6.6, 24576 16.8 / 17.9.  Out of rows:  T = 8: 1536 5.4 / 5.1, 3072 5.6 / 6.3;  T = 16: 6144 7.4 / 9.3;  T = 32: 6144 10.3 / 9.3
+    if (round_scores && n <= 64 && (int64_t)B * H * n <= std::min((tiled ? 384 : 192) * T, 16384)) {
+        hipLaunchKernelGGL(topk_rank_kernel, dim3(n / 4, B * H), dim3(256), 0, st, q, k, out_idx, n, T, tiled);
+    } else if (n <= kRegMaxN) {
         const dim3 grid(n / 16, B * H);
 #define LLSA_DENSE(TPW, W)                                                                                                               \
     do {                                                                                                                                 \

@@ -1,4 +1,4 @@
-"""Dense selection over rows longer than 1024 keys: the forms of the kernel (rows per workgroup, groups per row, key width) at the
+"""Dense selection over rows of at most 64 keys, one or sixteen rows a wave, and over rows longer than 1024 keys: the forms of the kernel (rows per workgroup, groups per row, key width) at the
 edges of their ranges, and rows whose bound lets more keys through than their buffer holds.  Scores are small integers, exact in
 bf16, so the result is known exactly: score descending, index ascending, NaN below every number."""
 import pytest
@@ -28,6 +28,8 @@ def tiles(x):
 def check(dev, n, T, BH, kind, round_scores=True):
     from llsa_amd.kernel.hip.topk import gen_sparse_indices
     pq, pk = ints(n + T, 1, BH, n, 64), ints(n + T + 1, 1, BH, n, 64)
+    if n <= 64 and kind == "few groups":
+        return
     if kind == "few groups":            # the best keys at T - 1 of the positions modulo 64
         at = torch.arange(n) % 64 < T - 1
         pk[:, :, at] = ints(n, 1, BH, int(at.sum()), 64, hi=4)
@@ -36,8 +38,8 @@ def check(dev, n, T, BH, kind, round_scores=True):
     elif kind == "nan":                 # rows without a number, keys without a number, a row of infinities
         pq[:, :, 5, 3] = float("nan")
         pk[:, :, 1::3, 7] = float("nan")
-        pk[:, :, 40, :] = 0
-        pk[:, :, 40, 0] = float("inf")
+        pk[:, :, min(40, n - 1), :] = 0
+        pk[:, :, min(40, n - 1), 0] = float("inf")
         pq[:, :, :, 0] = 1
     got = gen_sparse_indices(pq.to(dev), pk.to(dev), T, round_scores=round_scores)
     assert torch.equal(got.cpu().long(), expected(pq, pk, T))
@@ -47,7 +49,7 @@ def check(dev, n, T, BH, kind, round_scores=True):
     assert torch.equal(out, got)
 
 
-@pytest.mark.parametrize("n,T,kind", [(1040, 1, "plain"), (1088, 16, "few groups"), (1040, 17, "nan"), (1056, 64, "equal")])
+@pytest.mark.parametrize("n,T,kind", [(16, 16, "nan"), (48, 5, "plain"), (64, 64, "equal"), (1040, 1, "plain"), (1088, 16, "few groups"), (1040, 17, "nan"), (1056, 64, "equal")])
 def test_cpu(n, T, kind):
     with override_library_for_tests(emu_lib()):
         check(torch.device("cpu"), n, T, 1, kind)
@@ -86,7 +88,7 @@ def test_guided_tiles_gpu(N1, T, T2, BH):
 # 64, or T > 32; 64 beyond
 @pytest.mark.gpu
 @pytest.mark.parametrize("kind", ["plain", "few groups", "equal", "nan"])
-@pytest.mark.parametrize("n,T,BH", [(1040, 16, 8), (2048, 32, 2), (4096, 16, 1), (1056, 16, 8), (1056, 33, 9), (2064, 8, 1), (1088, 17, 4), (1088, 16, 8),
+@pytest.mark.parametrize("n,T,BH", [(16, 4, 1), (48, 48, 2), (64, 1, 6), (64, 1, 7), (64, 8, 48), (64, 8, 49), (64, 64, 256), (64, 64, 257), (1040, 16, 8), (2048, 32, 2), (4096, 16, 1), (1056, 16, 8), (1056, 33, 9), (2064, 8, 1), (1088, 17, 4), (1088, 16, 8),
                                     (1088, 17, 8), (3072, 32, 3), (1088, 64, 8), (4096, 64, 2), (1088, 8, 6), (1088, 32, 23), (1088, 8, 23)])
 def test_gpu(n, T, BH, kind):
     check(torch.device("cuda"), n, T, BH, kind)
