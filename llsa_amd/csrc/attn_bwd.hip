@@ -247,14 +247,12 @@ __global__ __launch_bounds__(256, Q == 1 ? 4 : 3) void attn_dq_kernel(llsa_attn_
     const int n_groups = sl.n_blocks / kGroup;
     bf16* const sh0 = &sh[0][0][0];
     auto issue_group = [&](int grp) __attribute__((always_inline)) {   // this wave brings in block kGroup*grp + wave
-        const SharedBlock sb = shared_block(sl, a.lvl, a.levels, a.N, bh, kGroup * grp + wave);
-        const bf16* kb = (const bf16*)a.lvl[sb.level].kr + sb.tile;
-        const bf16* vb = (const bf16*)a.lvl[sb.level].vr + sb.tile;
+        const SharedTiles sb = shared_tiles(sl, a.lvl, bh, kGroup * grp + wave);
         bf16* dst = sh0 + ((grp & 1) * kGroup + wave) * (2 * kTile);
-        copy16_global_to_lds(kb + unit, dst);
-        copy16_global_to_lds<512>(kb + unit, dst);
-        copy16_global_to_lds(vb + unit, dst + kTile);
-        copy16_global_to_lds<512>(vb + unit, dst + kTile);
+        copy16_global_to_lds(sb.k + unit, dst);
+        copy16_global_to_lds<512>(sb.k + unit, dst);
+        copy16_global_to_lds(sb.v + unit, dst + kTile);
+        copy16_global_to_lds<512>(sb.v + unit, dst + kTile);
     };
     DqRows rows[Q];
 #pragma unroll
@@ -272,10 +270,12 @@ __global__ __launch_bounds__(256, Q == 1 ? 4 : 3) void attn_dq_kernel(llsa_attn_
     // wait for every copy into LDS issued before it).
     // (two groups per trip: the buffer a group sits in is then a constant and every LDS address a lane-invariant
     // base plus an immediate)
+    SharedWeight sw = first_weight(a.lvl, a.levels);
     auto shared_group = [&](int grp, const bf16* blk) __attribute__((always_inline)) {
         wait_vm0();
         __syncthreads();
-        const float w = __builtin_amdgcn_logf(a.lvl[shared_level(a.lvl, a.levels, kGroup * grp)].w);   // log2
+        if (grp == sw.next) next_weight(sw, a.lvl, a.levels);
+        const float w = __builtin_amdgcn_logf(sw.w);          // log2
         PairR r0;
         PairT t0;
         read_k_r(r0, blk, blk + 2 * kTile, lane);

@@ -311,14 +311,12 @@ __global__ __launch_bounds__(256, Q == 1 ? 4 : 3) void attn_fwd_kernel(llsa_attn
     SharedList sl = shared_list(a.lvl, a.levels, a.N, bh, g, lane);
     bf16* const sh0 = &sh[0][0][0];
     auto issue_group = [&](int grp) __attribute__((always_inline)) {   // this wave brings in block kGroup*grp + wave
-        const SharedBlock sb = shared_block(sl, a.lvl, a.levels, a.N, bh, kGroup * grp + wave);
-        const bf16* kb = (const bf16*)a.lvl[sb.level].kr + sb.tile;
-        const bf16* vb = (const bf16*)a.lvl[sb.level].vt + sb.tile;
+        const SharedTiles sb = shared_tiles(sl, a.lvl, bh, kGroup * grp + wave);
         bf16* dst = sh0 + ((grp & 1) * kGroup + wave) * (2 * kTile);
-        copy16_global_to_lds(kb + lane * 8, dst);
-        copy16_global_to_lds<512>(kb + lane * 8, dst);
-        copy16_global_to_lds(vb + lane * 8, dst + kTile);
-        copy16_global_to_lds<512>(vb + lane * 8, dst + kTile);
+        copy16_global_to_lds(sb.k + lane * 8, dst);
+        copy16_global_to_lds<512>(sb.k + lane * 8, dst);
+        copy16_global_to_lds(sb.v + lane * 8, dst + kTile);
+        copy16_global_to_lds<512>(sb.v + lane * 8, dst + kTile);
     };
     const int n_groups = sl.n_blocks / kGroup;                // every level's count is a multiple of kGroup (host checks)
     QueryRows<Q> rows;
@@ -353,17 +351,16 @@ __global__ __launch_bounds__(256, Q == 1 ? 4 : 3) void attn_fwd_kernel(llsa_attn
     // wave's part of group grp has landed, and every wave is done reading the other buffer
     // (group grp - 1), which the next fetch overwrites.  (LDS reads of a group come before the next fetch: the compiler
     // makes every LDS read wait for all copies into LDS that were issued before it.)
-    float w_prev = 1.f;
+    SharedWeight sw = first_weight(a.lvl, a.levels);
     for (int grp = 0; grp < n_groups; grp++) {
         wait_vm0();
         __syncthreads();
-        // weight(previous segment) / weight(this one); nothing is accumulated before group 0
-        const float w_here = a.lvl[shared_level(a.lvl, a.levels, kGroup * grp)].w;
-        if (grp > 0 && w_here != w_prev) {
+        if (grp == sw.next) {
+            const float w = sw.w;
+            next_weight(sw, a.lvl, a.levels);
 #pragma unroll
-            for (int u = 0; u < Q; u++) rescale(st[u], w_prev / w_here);
+            for (int u = 0; u < Q; u++) rescale(st[u], w / sw.w);
         }
-        w_prev = w_here;
         const bf16* blk = &sh[grp & 1][0][0];
         if (grp == 0) {
             const bf16x8 k0 = lds_ld16(blk + lane * 8), k1 = lds_ld16(blk + 512 + lane * 8);
@@ -405,7 +402,7 @@ __global__ __launch_bounds__(256, Q == 1 ? 4 : 3) void attn_fwd_kernel(llsa_attn
         for (int u = 0; u < Q; u++) accumulate<kGroup>(st[u], rs[u], bp[u], v);
     }
 #pragma unroll
-    for (int u = 0; u < Q; u++) rescale(st[u], w_prev);       // fine tokens weigh 1
+    for (int u = 0; u < Q; u++) rescale(st[u], sw.w);         // fine tokens weigh 1
     __syncthreads();                                          // the shared copy is dead: its LDS becomes private slots
 
     // ---- fine blocks, two per step: the keys of step s + 1 are loaded into registers and its values copied into the wave's other

@@ -3,6 +3,7 @@
 #pragma once
 #include <hip/hip_runtime.h>
 #include <stdint.h>
+#include "../../include/llsa_hip.h"
 
 namespace llsa {
 
@@ -311,19 +312,27 @@ __device__ __forceinline__ int clampi(int v, int lo, int hi) { return v < lo ? l
 // The blocks of the pooled levels a group of query blocks reads, as the forward and the dQ kernel walk them:
 // level 1's selected blocks, level 2's, ..., then every block of the coarsest level.  `Level` is llsa_fwd_level
 // or llsa_bwd_level (fields sel, T).  Blocks of level l per (b,h): N / 16^(l+1).
+// What a wave looks up per block stays in registers.  With a loop over the levels in the kernel's arguments every block waited for a chain of scalar loads,
+// and with them for its LDS reads (they share a counter): 6 x 262144 tokens of two levels, forward 853 -> 811 us, dQ 996 -> 961; forward of 8 x 65536 of one
+// level 651 -> 627, which is less than its cycles say (these kernels run at the clock the card's power allows, 1.9 GHz and below).
+struct SharedTiles { const bf16 *k, *v; };                    // tiles of a block
 struct SharedList {
-    int mine;          // lane i: the i-th selected entry over all levels below the coarsest
-    int n_listed;      // how many of those there are
-    int n_blocks;      // n_listed + blocks of the coarsest level
-};
-struct SharedBlock {
-    int level;         // index into lvl[] (pooled level - 1)
-    int64_t tile;      // element offset of the block's tile inside the level's tile array
+    int mine;                  // lane i: the i-th selected entry over all levels below the coarsest
+    int n_first, n_listed;     // how many of those there are in level 1, in all
+    int n_blocks;              // n_listed + blocks of the coarsest level
+    int n0;                    // blocks of level 1 per (b,h)
+    SharedTiles first, coarse; // tiles of block 0 of level 1 and of the coarsest
 };
 __host__ __device__ inline int64_t coarsest_multiple(int levels) {       // N must be a multiple of 64 * 16^levels
     int64_t m = 64;
     for (int l = 0; l < levels; l++) m *= 16;
     return m;
+}
+__device__ __forceinline__ const void* value_tiles(const llsa_fwd_level& l) { return l.vt; }
+__device__ __forceinline__ const void* value_tiles(const llsa_bwd_level& l) { return l.vr; }
+template <typename Level>
+__device__ __forceinline__ SharedTiles level_tiles(const Level& l, int64_t block) {
+    return {(const bf16*)l.kr + block * kTile, (const bf16*)value_tiles(l) + block * kTile};
 }
 template <typename Level>
 __device__ __forceinline__ SharedList shared_list(const Level* lvl, int levels, int N, int bh, int g, int lane) {
@@ -331,6 +340,9 @@ __device__ __forceinline__ SharedList shared_list(const Level* lvl, int levels, 
     sl.mine = 0;
     int base = 0, nb = N / (kBlk * kBlk);                     // blocks of level 1 per (b,h) = owners of its selection
     int owner = g / kBlk;
+    sl.n0 = nb;
+    sl.n_first = levels > 1 ? lvl[0].T : 0;
+    sl.first = level_tiles(lvl[0], (int64_t)bh * nb);
     for (int l = 1; l < levels; l++) {
         const int T = lvl[l - 1].T;
         if (lane >= base && lane < base + T) sl.mine = lvl[l - 1].sel[((int64_t)bh * nb + owner) * T + (lane - base)];
@@ -340,33 +352,44 @@ __device__ __forceinline__ SharedList shared_list(const Level* lvl, int levels, 
     }
     sl.n_listed = base;
     sl.n_blocks = base + nb;                                  // nb is now the block count of the coarsest level
+    sl.coarse = level_tiles(lvl[levels - 1], (int64_t)bh * nb);
     return sl;
 }
-// which entry of lvl[] the i-th block of the walk belongs to (i is wave-uniform)
+// the i-th block of the walk (i is wave-uniform)
 template <typename Level>
-__device__ __forceinline__ int shared_level(const Level* lvl, int levels, int i) {
-    int base = 0, l = 1;
-    while (l < levels && i >= base + lvl[l - 1].T) {
-        base += lvl[l - 1].T;
-        l++;
+__device__ __forceinline__ SharedTiles shared_tiles(const SharedList& sl, const Level* lvl, int bh, int i) {
+    if (i >= sl.n_listed) {
+        const int64_t at = (int64_t)(i - sl.n_listed) * kTile;
+        return {sl.coarse.k + at, sl.coarse.v + at};
     }
-    return l - 1;
+    const int entry = __builtin_amdgcn_readlane(sl.mine, i);  // (i < 64 here)
+    if (i < sl.n_first) {
+        const int64_t at = (int64_t)clampi(entry, 0, sl.n0 - 1) * kTile;
+        return {sl.first.k + at, sl.first.v + at};
+    }
+    int base = sl.n_first, nb = sl.n0 / kBlk, l = 1;
+    while (i >= base + lvl[l].T) {
+        base += lvl[l++].T;
+        nb /= kBlk;
+    }
+    return level_tiles(lvl[l], (int64_t)bh * nb + clampi(entry, 0, nb - 1));
+}
+// The weight of the walk's groups of kGroup blocks, which changes from level to level (every level's count is a multiple of kGroup)
+struct SharedWeight {
+    float w;
+    int level, next;           // index into lvl[]; the group it ends in front of
+};
+template <typename Level>
+__device__ __forceinline__ void next_weight(SharedWeight& sw, const Level* lvl, int levels) {
+    sw.level++;
+    sw.w = lvl[sw.level].w;
+    sw.next = sw.level + 1 < levels ? sw.next + lvl[sw.level].T / kGroup : 0x7fffffff;
 }
 template <typename Level>
-__device__ __forceinline__ SharedBlock shared_block(const SharedList& sl, const Level* lvl, int levels, int N, int bh, int i) {
-    SharedBlock sb;
-    int base = 0, nb = N / (kBlk * kBlk), l = 1;
-    while (l < levels && i >= base + lvl[l - 1].T) {
-        base += lvl[l - 1].T;
-        nb /= kBlk;
-        l++;
-    }
-    int blk;
-    if (l < levels) blk = clampi(__builtin_amdgcn_readlane(sl.mine, i), 0, nb - 1);      // (i < 64 there)
-    else blk = i - sl.n_listed;
-    sb.level = l - 1;
-    sb.tile = ((int64_t)bh * nb + blk) * kTile;
-    return sb;
+__device__ __forceinline__ SharedWeight first_weight(const Level* lvl, int levels) {
+    SharedWeight sw{0.f, -1, 0};
+    next_weight(sw, lvl, levels);
+    return sw;
 }
 
 // The fine lists of Q sibling query blocks (ip: Q rows of T entries one after the other, Q * T <= 64 R), merged: the
