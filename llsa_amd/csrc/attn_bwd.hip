@@ -555,20 +555,11 @@ __global__ __launch_bounds__(64) void attn_kside_kernel(KSideParams p) {
         }
     }
     // The item's list entries (at most LLSA_CHUNK_FINE_MAX query blocks) are fetched once, entry i into lane i % 64 of
-    // register i / 64, and handed out with readlane: the walk below then has no load that depends on a load.
+    // register i / 64, and handed out with readlane: the walk below then has no load that depends on a load.  (Lanes behind the last entry have the last.)
     constexpr int kEntryRegs = LLSA_CHUNK_FINE_MAX / kWave;
     int mine[kEntryRegs];
 #pragma unroll
-    for (int k = 0; k < kEntryRegs; k++) mine[k] = (k * kWave + lane < cnt) ? fl[start + k * kWave + lane] : 0;
-    auto entry = [&](int i) -> int {                          // i is wave-uniform
-        int v = __builtin_amdgcn_readlane(mine[0], i & (kWave - 1));
-#pragma unroll
-        for (int k = 1; k < kEntryRegs; k++) {
-            const int o = __builtin_amdgcn_readlane(mine[k], i & (kWave - 1));
-            v = ((i >> 6) == k) ? o : v;
-        }
-        return clampi(v, 0, N1 - 1);
-    };
+    for (int k = 0; k < kEntryRegs; k++) mine[k] = k * kWave < cnt ? clampi(fl[start + min(k * kWave + lane, cnt - 1)], 0, N1 - 1) : 0;
 
     f32x4 dk[4], dv[4];
 #pragma unroll
@@ -590,9 +581,15 @@ __global__ __launch_bounds__(64) void attn_kside_kernel(KSideParams p) {
         // The operands of entries i, i + 1 are copied straight into LDS (no registers) while entries i - 2, i - 1 are
         // worked on: a round reads everything it needs out of LDS first, then starts the next copy into the same
         // place, then does its arithmetic.
-        auto fetch = [&](int i) __attribute__((always_inline)) {
-            const int g0 = entry(i);
-            const int g1 = (i + 1 < cnt) ? entry(i + 1) : g0;
+        int g0 = 0, g1 = 0;                                   // the next two
+        auto next_entries = [&](int i) __attribute__((always_inline)) {       // i: even, from 0 on in steps of two
+            if (i > 0 && i % kWave == 0)                      // the next register moves up to the front
+#pragma unroll
+                for (int k = 1; k < kEntryRegs; k++) mine[k - 1] = mine[k];
+            g0 = __builtin_amdgcn_readlane(mine[0], i % kWave);
+            g1 = __builtin_amdgcn_readlane(mine[0], i % kWave + 1);
+        };
+        auto fetch = [&]() __attribute__((always_inline)) {
             const int at = r_unit(lane);
             const bf16 *q0 = qrb + (int64_t)g0 * kTile, *d0 = dorb + (int64_t)g0 * kTile;
             const bf16 *q1 = qrb + (int64_t)g1 * kTile, *d1 = dorb + (int64_t)g1 * kTile;
@@ -609,14 +606,16 @@ __global__ __launch_bounds__(64) void attn_kside_kernel(KSideParams p) {
                 copy16_global_to_lds(reinterpret_cast<const bf16*>(src), reinterpret_cast<bf16*>(stats));
             }
         };
-        if (cnt > 0) fetch(0);
+        next_entries(0);
+        if (cnt > 0) fetch();
         for (int i = 0; i < cnt; i += 2) {
             wait_vm0();
             KsideOperands o;
             kside_read(o, stage, stats, lane);
+            next_entries(i + 2);                              // (while the reads arrive)
             wait_all_mem();                                   // every lane has its operands: the next copy may land
             __builtin_amdgcn_wave_barrier();
-            if (i + 2 < cnt) fetch(i + 2);
+            if (i + 2 < cnt) fetch();
             kside_pair(dk, dv, bk, bv, o, i + 1 < cnt);
         }
     }
