@@ -95,6 +95,25 @@ __device__ __forceinline__ float quad_sum(float v) {
     return __uint_as_float(b[0]) + __uint_as_float(b[1]);
 }
 
+// The value of lane l ^ XOR, for what a move inside a vector instruction can reach (rows of 16 lanes turned by 8, halves of 8 mirrored, quads permuted): a
+// shuffle goes through the LDS unit.
+template <int XOR>
+__device__ __forceinline__ float across(float v) {
+    static_assert(XOR == 8 || XOR == 7 || XOR == 2 || XOR == 1, "no such move");
+#ifndef LLSA_CPU_EMU_BUILD
+    constexpr int kMove = XOR == 8 ? 0x128 : XOR == 7 ? 0x141 : XOR == 2 ? 0x4E : 0xB1;       // row_ror:8, row_half_mirror, quad_perm
+    return __uint_as_float((unsigned)__builtin_amdgcn_update_dpp(0, (int)__float_as_uint(v), kMove, 0xf, 0xf, true));
+#else
+    return __shfl_xor(v, XOR);
+#endif
+}
+// Sum over lanes l ^ 0 .. 7, the same bits in all eight
+__device__ __forceinline__ float octet_sum(float v) {
+    v += across<1>(v);
+    v += across<2>(v);
+    return v + across<7>(v);                                  // (all lanes of a quad have the same sum)
+}
+
 // Sixteen token rows out of the accumulator layout: this lane's o[dt] are channels 16 dt + 4 (l/16) .. +3 of token l%16, whose row starts at `row`.
 // In pieces of 8 bytes of sixteen rows at a time every piece is an access of its own in the L1, and a work item of the K side had as many of
 // those in its stores as in the tiles of eight list entries.  Swapped between neighbouring sixteens of lanes the pieces are 16 bytes and the half
@@ -114,15 +133,24 @@ __device__ __forceinline__ void store_rows(bf16* row, const bf16x4 (&o)[4], int 
         for (int dt = 0; dt < 4; dt++) st8(row + 16 * dt + 4 * quad, o[dt]);
     }
 }
-// The other way round: x[dt] = channels 16 dt + 4 (l/16) .. +3 of the row at `row` (16-byte aligned)
-__device__ __forceinline__ void load_rows(bf16x4 (&x)[4], const bf16* row, int quad) {
+// The other way round: x[dt] = channels 16 dt + 4 (l/16) .. +3 of the row at `row` (16-byte aligned), requested and, once it is there, put in order
+__device__ __forceinline__ void request_rows(bf16x8 (&raw)[2], const bf16* row, int quad) {
+#pragma unroll
+    for (int p = 0; p < 2; p++) raw[p] = ld16(row + 32 * p + 16 * (quad & 1) + 8 * (quad >> 1));
+}
+__device__ __forceinline__ void arrange_rows(bf16x4 (&x)[4], const bf16x8 (&raw)[2]) {
 #pragma unroll
     for (int p = 0; p < 2; p++) {
-        const u32x4 v = __builtin_bit_cast(u32x4, ld16(row + 32 * p + 16 * (quad & 1) + 8 * (quad >> 1)));
+        const u32x4 v = __builtin_bit_cast(u32x4, raw[p]);
         const u32x2 lo = __builtin_amdgcn_permlane16_swap(v[0], v[2], false, false), hi = __builtin_amdgcn_permlane16_swap(v[1], v[3], false, false);
         x[2 * p] = __builtin_bit_cast(bf16x4, u32x2{lo[0], hi[0]});
         x[2 * p + 1] = __builtin_bit_cast(bf16x4, u32x2{lo[1], hi[1]});
     }
+}
+__device__ __forceinline__ void load_rows(bf16x4 (&x)[4], const bf16* row, int quad) {
+    bf16x8 raw[2];
+    request_rows(raw, row, quad);
+    arrange_rows(x, raw);
 }
 __device__ __forceinline__ bool rows_wide(const void* p, int64_t sb, int64_t sh, int64_t sn) {
     return ((reinterpret_cast<uintptr_t>(p) & 15u) | ((sb | sh | sn) & 7)) == 0;

@@ -73,9 +73,7 @@ __device__ __forceinline__ void rms_norm_rows(bf16x8* xv, const float (&g)[8], f
         float ss = 0.f;
 #pragma unroll
         for (int e = 0; e < 8; e++) ss += (float)xv[i][e] * (float)xv[i][e];
-        ss += __shfl_xor(ss, 1);
-        ss += __shfl_xor(ss, 2);
-        ss += __shfl_xor(ss, 4);
+        ss = octet_sum(ss);
         const float rstd = rsqrtf(ss * (1.f / kD) + eps);
 #pragma unroll
         for (int e = 0; e < 8; e++) xv[i][e] = (bf16)((float)xv[i][e] * rstd * g[e]);
@@ -323,9 +321,7 @@ __global__ __launch_bounds__(256) void rmsnorm_bwd_kernel(const bf16* dy, Stride
         float ss = 0.f;
 #pragma unroll
         for (int e = 0; e < 8; e++) ss += (float)xv[e] * (float)xv[e];
-        ss += __shfl_xor(ss, 1);
-        ss += __shfl_xor(ss, 2);
-        ss += __shfl_xor(ss, 4);
+        ss = octet_sum(ss);
         const float rstd = rsqrtf(ss * (1.f / kD) + eps);
         float xn[8], g[8], dot = 0.f;
 #pragma unroll
@@ -335,9 +331,7 @@ __global__ __launch_bounds__(256) void rmsnorm_bwd_kernel(const bf16* dy, Stride
             dot += g[e] * xn[e];
             contrib[e] += (float)gv[e] * xn[e];
         }
-        dot += __shfl_xor(dot, 1);
-        dot += __shfl_xor(dot, 2);
-        dot += __shfl_xor(dot, 4);
+        dot = octet_sum(dot);
         dot *= 1.f / kD;
         bf16x8 o;
 #pragma unroll
