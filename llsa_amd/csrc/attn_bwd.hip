@@ -1006,9 +1006,24 @@ struct GroupSeg {
 struct GroupParams {
     const bf16* qr; const bf16* dor;              // R tiles of q and dO, (BH, N1, 1024)
     const float* stats;                           // (BH, N1, kStats)
-    int H, N, n_segs, n_blocks;
+    int BH, N, n_segs, n_blocks;
+    int whole, parts;                             // see GroupSplit
     GroupSeg seg[kGroupSegs];
 };
+
+// Workgroups of the group-major pass over an XCD's `groups` groups.  32 CUs take two each; where that leaves a last round at most half full, the key blocks
+// of its groups are dealt out to `parts` workgroups, each with the group's tiles in LDS, and the first `whole` groups are as before.  Every key block is
+// still met by one wave, so the results are the same.  Training steps of two levels, topk 16/16, us, whole / dealt out: 1 x 16384 tokens (8 groups an XCD) 92.4 /
+// 87.5;  10 x 16384 (80) 254.6 / 250.8;  17 x 16384 at 16/12 (136) 381 / 374;  9 x 16384 at 16/32 (72) 296 / 288;  3 x 49152 at 64/32 (72) 639 / 629;  just
+// half full 4 x 16384 (32) 140 / 138.8, 12 x 16384 (96) 293.8 / 293.3, 3 x 32768 even.
+struct GroupSplit { int whole, parts; };
+constexpr int kGroupSlots = 2 * 256 / kXcds;
+constexpr int kGroupPartBlocks = 6;               // key blocks a part has at least
+static GroupSplit group_split(int groups, int n_blocks) {
+    const int rest = groups % kGroupSlots;
+    const int parts = rest == 0 ? 1 : std::min(kGroupSlots / rest, n_blocks / kGroupPartBlocks);
+    return parts < 2 ? GroupSplit{groups, 1} : GroupSplit{groups - rest, parts};
+}
 
 // UPW key blocks against the group's 16 query blocks, two query blocks per step, operands out of LDS.  `next` starts the loads of the
 // wave's next key blocks, into bk and bv, where these are no longer needed: they arrive while the sums are rounded and stored.
@@ -1062,11 +1077,12 @@ __global__ __launch_bounds__(64 * kGroupWaves, 2) void attn_kside_group_kernel(G
     __shared__ __align__(16) float sh_stats[kBlk * kStats];   // their statistics
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int N1 = p.N / kBlk;
-    const int lid = xcd_logical_id();
-    const int G = lid % (int)gridDim.x;                        // group of query blocks 16 G .. 16 G + 15
-    const int bh = lid / (int)gridDim.x;
-    const int n_groups = (int)gridDim.x;
+    const int N1 = p.N / kBlk, n_groups = N1 / kBlk;
+    const int slot = (int)blockIdx.x / kXcds, behind = slot - p.whole;        // (an XCD's workgroups are every eighth)
+    const int part = behind < 0 ? 0 : behind % p.parts, parts = behind < 0 ? 1 : p.parts;
+    const int lid = (int)blockIdx.x % kXcds * (n_groups * p.BH / kXcds) + (behind < 0 ? slot : p.whole + behind / p.parts);
+    const int G = lid % n_groups;                              // group of query blocks 16 G .. 16 G + 15
+    const int bh = lid / n_groups;
 
     {   // 32 KB of Q tiles and 32 KB of dO tiles, contiguous in memory, 1 KB per wave and copy
         const bf16* qsrc = p.qr + ((int64_t)bh * N1 + (int64_t)G * kBlk) * kTile;
@@ -1100,13 +1116,13 @@ __global__ __launch_bounds__(64 * kGroupWaves, 2) void attn_kside_group_kernel(G
                 my_slot = (int64_t)bh * sg.slots + pos;
             } else {
                 my_unit = j;
-                my_slot = ((int64_t)G * gridDim.y + bh) * sg.n_units + j;      // [group][bh][unit]: what the dense reduction walks
+                my_slot = ((int64_t)G * p.BH + bh) * sg.n_units + j;      // [group][bh][unit]: what the dense reduction walks
             }
         }
     }
     // this wave's key blocks: a contiguous share, taken two at a time (the last alone if the share is odd)
-    const int per = (p.n_blocks + kGroupWaves - 1) / kGroupWaves;
-    const int lo = min(wave * per, p.n_blocks), hi = min(lo + per, p.n_blocks);
+    const int per = (p.n_blocks + kGroupWaves * parts - 1) / (kGroupWaves * parts);
+    const int lo = min((part * kGroupWaves + wave) * per, p.n_blocks), hi = min(lo + per, p.n_blocks);
 
     bf16x8 bk[2][2], bv[2][2];
     float w[2];
@@ -1624,7 +1640,7 @@ extern "C" int llsa_attn_bwd(const llsa_attn_bwd_args* a, void* stream) {
         if (L < 2 || !(stages & LLSA_BWD_DPKV1)) return;
         GroupParams g;
         g.qr = (const bf16*)a->qr; g.dor = dor; g.stats = stats;
-        g.H = H; g.N = N; g.n_segs = 0; g.n_blocks = 0;
+        g.BH = BH; g.N = N; g.n_segs = 0; g.n_blocks = 0;
         auto add_seg = [&](const void* kk, const void* vv, const int* sel, const int* inv, int64_t part_off, int n_units, int shift,
                            int cnt, int64_t slots, float w) {
             GroupSeg& sgm = g.seg[g.n_segs++];
@@ -1656,8 +1672,13 @@ extern "C" int llsa_attn_bwd(const llsa_attn_bwd_args* a, void* stream) {
         if (d.merged && (stages & LLSA_BWD_DENSE))
             add_seg(a->lvl[L - 1].kr, a->lvl[L - 1].vr, nullptr, nullptr, wsp.part_dense, d.n_tok / 16, 0, d.n_tok / 16, 0, a->lvl[L - 1].gw);
         const int64_t bytes = (int64_t)BH * N2 * g.n_blocks * (kSlotBytes / 2);
-        if (bytes > kGroupStreamBytes && g.n_blocks >= kGroupStreamBlocks) hipLaunchKernelGGL(attn_kside_group_kernel<true>, dim3(N2, BH), dim3(64 * kGroupWaves), 0, s, g);
-        else hipLaunchKernelGGL(attn_kside_group_kernel<false>, dim3(N2, BH), dim3(64 * kGroupWaves), 0, s, g);
+        const int per_xcd = N2 * BH / kXcds;                  // (two levels need N2 to be a multiple of 64)
+        const GroupSplit split = group_split(per_xcd, g.n_blocks);
+        g.whole = split.whole;
+        g.parts = split.parts;
+        const dim3 grid((unsigned)(kXcds * (split.whole + (per_xcd - split.whole) * split.parts)));
+        if (bytes > kGroupStreamBytes && g.n_blocks >= kGroupStreamBlocks) hipLaunchKernelGGL(attn_kside_group_kernel<true>, grid, dim3(64 * kGroupWaves), 0, s, g);
+        else hipLaunchKernelGGL(attn_kside_group_kernel<false>, grid, dim3(64 * kGroupWaves), 0, s, g);
     };
     // dense coarsest level: every unit (16 pooled tokens) meets every query block; the query
     // range is cut into d.chunks pieces whose partial sums are added afterwards
