@@ -266,11 +266,11 @@ __global__ __launch_bounds__(256, Q == 1 ? 4 : 3) void attn_dq_kernel(llsa_attn_
 #pragma unroll
     for (int u = 0; u < Q; u++) dq_request(rows[u], a, b, h, g + u, lane);
     issue_group(0);
-    MergedLists<Q, R> ml = merge_lists<Q, R>(ip, min(T, kWave * R / Q), N1, lane, order[wave]);
 
     DqSide sd[Q];                                             // (the second buffer is not filled before the barrier of group 0)
 #pragma unroll
     for (int u = 0; u < Q; u++) dq_begin(sd[u], rows[u], a, stats, dor, bh, g + u, lane, &sh[1][wave][0]);
+    MergedLists<Q, R> ml = merge_lists<Q, R>(ip, min(T, kWave * R / Q), N1, lane, order[wave]);
 
     // ---- pooled blocks out of the shared copy.  The barrier at the top of round grp says: every
     // wave's part of group grp has landed, and every wave is done reading the other buffer.  All
