@@ -67,3 +67,26 @@ def test_against_sets(merge, Q, R, T, N1):
             ref[b] = ref.get(b, 0) | 1 << u
     got = merge(rows, N1, R)
     assert len(got) == len(ref) and {b: s for b, s in got} == ref
+
+
+@pytest.mark.parametrize("T", [4, 12, 16, 20, 28, 32])        # two lists in either half of a wave: up to sixteen entries, and beyond
+@pytest.mark.parametrize("shared", ["none", "all turned", "last with first", "one row repeats its last"])
+def test_two_short_lists(merge, T, shared):
+    N1 = 4096
+    rows = torch.randperm(N1, generator=torch.Generator().manual_seed(T))[: 2 * T].reshape(2, T)
+    if shared == "all turned":
+        rows[1] = rows[0].roll(T // 2 + 1)
+    elif shared == "last with first":
+        rows[1, 0] = rows[0, T - 1]
+    elif shared == "one row repeats its last":
+        rows[1, T - 1] = rows[1, 0]
+    got = merge(rows, N1, 1)
+    if shared == "one row repeats its last":                  # every entry on its own
+        assert sorted(map(tuple, got)) == sorted((int(b), 1 << u) for u in range(2) for b in rows[u])
+        return
+    ref = {}
+    for u in range(2):
+        for b in rows[u].tolist():
+            ref[b] = ref.get(b, 0) | 1 << u
+    assert len(got) == len(ref) and {b: s for b, s in got} == ref
+    assert [s for _, s in got] == sorted((s for _, s in got), reverse=True)
