@@ -160,7 +160,7 @@ bool rows_ok(const Tensor& t) {
     return t.stride(-1) == 1 && reinterpret_cast<uintptr_t>(t.data_ptr()) % 16 == 0 && strides_multiple(t.strides(), 8);
 }
 Tensor as_rows(const Tensor& t) { return rows_ok(t) ? t : t.contiguous(); }
-// a saved tensor as the kernels need it, wherever and with whatever strides a saved-tensor hook has put it
+// a tensor as the kernels need it, wherever and with whatever strides a caller or a saved-tensor hook has put it
 Tensor restored(const Tensor& t, bool contiguous = false) {
     const bool usable = !t.defined() || (rows_ok(t) && (!contiguous || t.is_contiguous()));
     return usable ? t : t.clone(at::MemoryFormat::Contiguous);
@@ -430,7 +430,7 @@ Tensor attend(const std::shared_ptr<Library>& lib, const Tensor& q_in, const Ten
         if (freq_in.has_value()) {
             if (freq_in->scalar_type() != at::kBFloat16 || freq_in->dim() != 2 || freq_in->size(0) != N || freq_in->size(1) != 64)
                 fail(Failure::kValue, "rope table must be bf16 (N, 64)");
-            freq = freq_in->contiguous();
+            freq = restored(*freq_in, true);                 // (read in 16-byte pieces; a table may start anywhere in its storage)
         }
         const Tensor v = as_rows(v_in);
         q = as_rows(q_in);
