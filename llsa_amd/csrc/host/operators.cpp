@@ -222,8 +222,9 @@ struct Layout {
     int64_t pq[kL + 1], pk[kL + 1], pv[kL + 1];             // pooled rows, index = level
     int64_t qr, kr, vr;                                     // operand tiles of the tokens
     int64_t pkr[kL + 1], pvr[kL + 1], pvt[kL + 1];          // and of the pooled levels
-    int64_t sel[kL], off[kL], flat[kL], inv[kL], work = -1, nested = -1; // sel[0]: fine blocks per query block, sel[l]: blocks of level l per group of 16^(l+1) queries
+    int64_t sel[kL], off[kL], flat[kL], inv[kL], work = -1; // sel[0]: fine blocks per query block, sel[l]: blocks of level l per group of 16^(l+1) queries
     int64_t lse, bytes;
+    int64_t nested_bytes = 0;                               // scratch of the lists made from those of the level above: of the forward only, not in the arena
     int64_t dpk[kL + 1], dpv[kL + 1], ws, ws_bytes = 0, bwd_bytes;       // the backward's arena
 
     Layout(const Library& lib, int64_t B, int64_t H, int64_t N, const std::vector<int64_t>& topks, bool grad) {
@@ -267,10 +268,7 @@ struct Layout {
             work = take(4 * lib.work_list_len(static_cast<int>(n[1]), static_cast<int>(n[1]), topk[0], chunk));
             // (lists too long for one launch are made from those of the level above, which the selection is nested in)
             const int m = static_cast<int>(n[1]), b = static_cast<int>(B), h = static_cast<int>(H);
-            const int64_t scratch = L > 1 && !lib.transpose_one_launch(m, m, topk[0], b, h) ? lib.transpose_nested_bytes(m, m, topk[1], b, h) : -1;
-            nested = o;
-            o = align_up(o + std::max<int64_t>(scratch, 0), 256);
-            if (scratch < 0) nested = -1;
+            if (L > 1 && !lib.transpose_one_launch(m, m, topk[0], b, h)) nested_bytes = std::max<int64_t>(lib.transpose_nested_bytes(m, m, topk[1], b, h), 0);
         }
         bytes = o;
         o = 0;
@@ -442,6 +440,8 @@ Tensor attend(const std::shared_ptr<Library>& lib, const Tensor& q_in, const Ten
         const Layout y(*lib, B, H, N, topks, grad);
         const int64_t* n = y.n;
         arena = at::empty({y.bytes}, q.options().dtype(at::kByte));
+        Tensor scratch;                                      // (goes at the end of this block, when the caller's stream waits for all that uses it)
+        if (y.nested_bytes > 0) scratch = at::empty({y.nested_bytes}, arena.options());
         o = strides_multiple(q.strides(), 4) ? at::empty_like(q) : at::empty(q.sizes(), q.options());
         char* const a0 = static_cast<char*>(arena.data_ptr());
         auto pa = [&](int64_t at) -> void* { return at < 0 ? nullptr : a0 + at; };
@@ -555,7 +555,7 @@ Tensor attend(const std::shared_ptr<Library>& lib, const Tensor& q_in, const Ten
         for (int l = 0; l < L && grad; l++) {
             const int32_t m = static_cast<int32_t>(n[l + 1]);
             jobs[l] = llsa_transpose_job{ints(y.sel[l]), ints(y.off[l]), ints(y.flat[l]), l == 0 ? ints(y.work) : nullptr, l == 0 ? nullptr : ints(y.inv[l]),
-                                         m, m, y.topk[l], l == 0 ? y.chunk : 1, l == 0 ? pa(y.nested) : nullptr};
+                                         m, m, y.topk[l], l == 0 ? y.chunk : 1, l == 0 && scratch.defined() ? scratch.data_ptr() : nullptr};
         }
         if (grad && !beside) lib->check(lib->attn_fwd_lists(&f, jobs, L, stream), "attn_fwd");
         else lib->check(lib->attn_fwd(&f, stream), "attn_fwd");
@@ -565,7 +565,7 @@ Tensor attend(const std::shared_ptr<Library>& lib, const Tensor& q_in, const Ten
                 void* lists = side_stream(dev);
                 hip_check(hipStreamWaitEvent(static_cast<hipStream_t>(lists), side_events(dev).ready, 0));       // (the arena is older than the selection, so this covers it too)
                 lib->check(lib->transpose_indices_multi(jobs, L, b, h, lists), "transpose_indices");
-                // (and the arena is not handed out again before the second stream is done)
+                // (and neither the arena nor the scratch is handed out again before the second stream is done)
                 hip_check(hipEventRecord(side_events(dev).done, static_cast<hipStream_t>(lists)));
                 hip_check(hipStreamWaitEvent(static_cast<hipStream_t>(stream), side_events(dev).done, 0));
             }
