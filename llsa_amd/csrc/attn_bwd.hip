@@ -1017,12 +1017,17 @@ struct GroupParams {
 // 87.5;  10 x 16384 (80) 254.6 / 250.8;  17 x 16384 at 16/12 (136) 381 / 374;  9 x 16384 at 16/32 (72) 296 / 288;  3 x 49152 at 64/32 (72) 639 / 629;  just
 // half full 4 x 16384 (32) 140 / 138.8, 12 x 16384 (96) 293.8 / 293.3, 3 x 32768 even.
 struct GroupSplit { int whole, parts; };
+// key blocks of a wave of a group that `parts` workgroups share
+__host__ __device__ inline int group_wave_blocks(int n_blocks, int parts) { return (n_blocks + kGroupWaves * parts - 1) / (kGroupWaves * parts); }
 constexpr int kGroupSlots = 2 * 256 / kXcds;
-constexpr int kGroupPartBlocks = 6;               // key blocks a part has at least
+constexpr int kGroupPartBlocks = 6;               // key blocks to a part, on the average over a group's parts, at least
 static GroupSplit group_split(int groups, int n_blocks) {
     const int rest = groups % kGroupSlots;
-    const int parts = rest == 0 ? 1 : std::min(kGroupSlots / rest, n_blocks / kGroupPartBlocks);
-    return parts < 2 ? GroupSplit{groups, 1} : GroupSplit{groups - rest, parts};
+    int parts = rest == 0 ? 1 : std::min(kGroupSlots / rest, n_blocks / kGroupPartBlocks);
+    if (parts < 2) return {groups, 1};
+    const int share = kGroupWaves * group_wave_blocks(n_blocks, parts);       // of every part but the last
+    parts = (n_blocks + share - 1) / share;                                   // (none of them empty; the shares are the same)
+    return {groups - rest, parts};
 }
 
 // UPW key blocks against the group's 16 query blocks, two query blocks per step, operands out of LDS.  `next` starts the loads of the
@@ -1121,7 +1126,7 @@ __global__ __launch_bounds__(64 * kGroupWaves, 2) void attn_kside_group_kernel(G
         }
     }
     // this wave's key blocks: a contiguous share, taken two at a time (the last alone if the share is odd)
-    const int per = (p.n_blocks + kGroupWaves * parts - 1) / (kGroupWaves * parts);
+    const int per = group_wave_blocks(p.n_blocks, parts);
     const int lo = min((part * kGroupWaves + wave) * per, p.n_blocks), hi = min(lo + per, p.n_blocks);
 
     bf16x8 bk[2][2], bv[2][2];
