@@ -573,8 +573,9 @@ extern "C" int llsa_attn_fwd_selects(int B, int H, int N, int T, int levels) {
 extern "C" int llsa_lists_ride(int B, int H, int N, const int32_t* topk, int levels) {
     if (const int rc = check_plan_query("lists_ride", B, H, N, topk, levels)) return rc;
     llsa_transpose_job jobs[LLSA_MAX_LEVELS];
-    int32_t* const some = reinterpret_cast<int32_t*>(16);     // (the plan only looks whether there is a list)
-    for (int l = 0, m = N / 16; l < levels; l++, m /= 16) jobs[l] = llsa_transpose_job{some, some, some, nullptr, nullptr, m, m, topk[l], 1};
+    int32_t* const some = reinterpret_cast<int32_t*>(16);     // (the plan only looks whether there are lists and inverse positions: of the pooled levels there are)
+    for (int l = 0, m = N / 16; l < levels; l++, m /= 16)
+        jobs[l] = llsa_transpose_job{some, some, some, nullptr, l == 0 ? nullptr : some, m, m, topk[l], 1, nullptr};
     TrJobs lists{};
     return plan_list_rows(jobs, levels, B, H, forward_width(N, two_blocks_per_wave((int64_t)B * H, N, topk, levels, true)), lists) >= 0;
 }

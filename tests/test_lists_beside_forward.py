@@ -2,6 +2,8 @@
 their own -- one range and many, rows that do not divide, repeated entries, grids of one and of two query blocks a wave, and lists too long or
 too many to ride along."""
 import ctypes as C
+import os
+import subprocess
 
 import pytest
 import torch
@@ -64,6 +66,34 @@ def test_lines_of_the_rule():
     assert not _ride(1, 1, 65536, 20, 8)                      # more than 65536 entries
     assert _ride(1, 1, 130048, 8) and not _ride(1, 1, 131072, 8, 4)      # 8128 and 8192 key blocks: their histogram takes 8160 ints of LDS at most
     assert not _ride(1, 65535, 1024, 4)                       # more rows than a grid has
+
+
+def test_the_query_plans_the_operators_jobs(tmp_path):
+    """llsa_lists_ride asks for the plan of the jobs that the operators pass: inverse positions, which double a key block's LDS, of every level but the first."""
+    emu = emu_lib().path                                      # (with the path of tests/cpu_emu)
+    import build_emu
+    (tmp_path / "ride.cpp").write_text('''
+#include "attn_fwd.hip"
+static int seen[LLSA_MAX_LEVELS];
+bool llsa::plan_transpose(const llsa_transpose_job* jobs, int n_jobs, int, int, int, TrJobs& plan) {
+    for (int i = 0; i < n_jobs; i++) seen[i] = jobs[i].inv != nullptr ? 2 : 1;
+    plan = TrJobs{};
+    return true;
+}
+extern "C" int ride(int N, const int32_t* topk, int levels, int* out) {
+    const int rc = llsa_lists_ride(1, 1, N, topk, levels);
+    for (int i = 0; i < levels; i++) out[i] = seen[i];
+    return rc;
+}
+''')
+    subprocess.run([build_emu.CLANG, "-std=c++17", "-O0", "-fPIC", "-shared", "-Wl,-Bsymbolic", "-I", os.path.join(build_emu.HERE, "include"), "-I",
+                    build_emu.CSRC, "-Wno-everything", "-ffp-contract=off", "-DLLSA_CPU_EMU_BUILD", str(tmp_path / "ride.cpp"), emu, "-o",
+                    str(tmp_path / "ride.so")], check=True)
+    lib = C.CDLL(str(tmp_path / "ride.so"))
+    for levels, N in ((1, 1024), (2, 16384), (3, 262144)):
+        out = (C.c_int * levels)()
+        assert lib.ride(N, (C.c_int32 * levels)(*[8] * levels), levels, out) == 1
+        assert list(out) == [1] + [2] * (levels - 1)
 
 
 @pytest.mark.gpu
