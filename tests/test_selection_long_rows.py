@@ -28,11 +28,14 @@ def tiles(x):
 def check(dev, n, T, BH, kind, round_scores=True):
     from llsa_amd.kernel.hip.topk import gen_sparse_indices
     pq, pk = ints(n + T, 1, BH, n, 64), ints(n + T + 1, 1, BH, n, 64)
-    if n <= 64 and kind == "few groups":
-        return
     if kind == "few groups":            # the best keys at T - 1 of the positions modulo 64
         at = torch.arange(n) % 64 < T - 1
         pk[:, :, at] = ints(n, 1, BH, int(at.sum()), 64, hi=4)
+    elif kind == "two scores":          # the larger one at the row's ends and every third key: ties on both sides of the line
+        at = torch.arange(n) % 3 == 0
+        at[0], at[-1] = False, True
+        pq[:], pk[:] = 1, 0
+        pk[:, :, at] = 1
     elif kind == "equal":
         pk[:] = pk[:, :, :1]
     elif kind == "nan":                 # rows without a number, keys without a number, a row of infinities
@@ -49,7 +52,7 @@ def check(dev, n, T, BH, kind, round_scores=True):
     assert torch.equal(out, got)
 
 
-@pytest.mark.parametrize("n,T,kind", [(16, 16, "nan"), (48, 5, "plain"), (64, 64, "equal"), (1040, 1, "plain"), (1088, 16, "few groups"), (1040, 17, "nan"), (1056, 64, "equal")])
+@pytest.mark.parametrize("n,T,kind", [(16, 16, "nan"), (48, 5, "plain"), (48, 20, "two scores"), (64, 64, "equal"), (1040, 1, "plain"), (1088, 16, "few groups"), (1040, 17, "nan"), (1056, 64, "equal")])
 def test_cpu(n, T, kind):
     with override_library_for_tests(emu_lib()):
         check(torch.device("cpu"), n, T, 1, kind)
@@ -84,11 +87,22 @@ def test_guided_tiles_gpu(N1, T, T2, BH):
     check_guided(torch.device("cuda"), N1, T, T2, BH)
 
 
+# a row a wave up to 192 T (rows of keys) or 384 T (tiles) and 16384 rows, sixteen rows a wave beyond
+SHORT = [(16, 4, 1), (48, 48, 2), (64, 1, 6), (64, 1, 7), (64, 8, 48), (64, 8, 49), (64, 64, 256), (64, 64, 257)]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("kind", ["plain", "two scores", "equal", "nan"])
+@pytest.mark.parametrize("n,T,BH", SHORT)
+def test_short_gpu(n, T, BH, kind):
+    check(torch.device("cuda"), n, T, BH, kind)
+
+
 # Rows / tiles: 16 rows a workgroup up to 256 / 400 or 560 sixteens of rows, or where they are odd; 32 up to 512 / 1536, where n is no multiple of
 # 64, or T > 32; 64 beyond
 @pytest.mark.gpu
 @pytest.mark.parametrize("kind", ["plain", "few groups", "equal", "nan"])
-@pytest.mark.parametrize("n,T,BH", [(16, 4, 1), (48, 48, 2), (64, 1, 6), (64, 1, 7), (64, 8, 48), (64, 8, 49), (64, 64, 256), (64, 64, 257), (1040, 16, 8), (2048, 32, 2), (4096, 16, 1), (1056, 16, 8), (1056, 33, 9), (2064, 8, 1), (1088, 17, 4), (1088, 16, 8),
+@pytest.mark.parametrize("n,T,BH", [(1040, 16, 8), (2048, 32, 2), (4096, 16, 1), (1056, 16, 8), (1056, 33, 9), (2064, 8, 1), (1088, 17, 4), (1088, 16, 8),
                                     (1088, 17, 8), (3072, 32, 3), (1088, 64, 8), (4096, 64, 2), (1088, 8, 6), (1088, 32, 23), (1088, 8, 23)])
 def test_gpu(n, T, BH, kind):
     check(torch.device("cuda"), n, T, BH, kind)
