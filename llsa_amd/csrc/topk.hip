@@ -326,8 +326,11 @@ __global__ __launch_bounds__(256) void topk_rank_kernel(const bf16* __restrict__
 // A workgroup is 16 RT rows, and its four waves take every fourth key tile of the row each, four tiles on their way to registers while four are worked
 // on.  What bounds it is the rate at which key tiles arrive -- each is read once per workgroup and look, hence many
 // rows a workgroup where the grid is large -- and the chain through LDS for the tiles that hold a key that passes.
-// A row whose bound lets more than kBuf keys through (ties; a period of the image that puts the best keys into few groups) has its bound
-// moved up by bisection, a look at all scores per step, at most one step per bit of a key, for no two keys of a row are equal.
+// Where a row's bound lets more than kBuf keys through (ties; a period of the image that puts the best keys into few groups), the second look ends and the workgroup
+// looks a third time with a running bound: four tiles a round, and rows whose buffers could not hold another round are cut back to little more than
+// their T best, whose least is the new bound.  No two keys of a row are equal, so behind a cut no equal score further on passes.  All scores equal, us, by a
+// bisection of the bound with a look a step / this (spread scores): 8 x 4096 rows, T = 8, 708 / 136 (95);  4 x 4096, T = 16, 384 / 80 (65);  6 x 2048, T = 8, 202 /
+// 54 (35.6);  4 x 2048, T = 32, 115 / 43 (32.7);  16 x 4096 in 64 bits, T = 32, 3770 / 312 (240).  The best keys in T - 1 of 64 groups: 4 x 4096, T = 16, 176 / 134.
 // Key: the 32-bit packed key (scores rounded to bf16, n <= kMaxPackedKeys) or the 64-bit wide key.
 // (8 x 4096 rows of 4096 keys out of tiles: 49 us, T = 32 68; out of rows 72 and 84.  Out of rows, a T-step arg-max over chunks of 512 keys per row took
 // 1480; a running threshold per row, raised whenever a buffer was full, by a wave for itself 128 and 142, with key tiles shared through LDS
@@ -341,9 +344,8 @@ template <>
 struct StreamKey<unsigned> {
     static __device__ __forceinline__ unsigned make(float s, int idx, bool) { return packed_key(s, idx); }
     static __device__ __forceinline__ unsigned long long wide(unsigned k) { return wide_key(k & 0xFFFF0000u, 0xFFFF - (int)(k & 0xFFFFu)); }
-    // the smallest and the largest key a score (given as ordered key of the score before rounding) can make
+    // the smallest key a score (given as ordered key of the score before rounding) can make
     static __device__ __forceinline__ unsigned least(unsigned score, bool) { return ordered_key(rn_bf16(key_score(score))) & 0xFFFF0000u; }
-    static __device__ __forceinline__ unsigned most(unsigned score, bool r) { return least(score, r) | 0xFFFFu; }
     // a score below this cannot make a key of at least t: one bf16 step below t's score
     static __device__ __forceinline__ unsigned score_bits(unsigned t) { return t & 0xFFFF0000u; }
 };
@@ -356,7 +358,6 @@ struct StreamKey<unsigned long long> {
     static __device__ __forceinline__ unsigned long long least(unsigned score, bool round) {
         return (unsigned long long)(round ? ordered_key(rn_bf16(key_score(score))) : score) << 32;
     }
-    static __device__ __forceinline__ unsigned long long most(unsigned score, bool round) { return least(score, round) | 0xFFFFFFFFull; }
     static __device__ __forceinline__ unsigned score_bits(unsigned long long t) { return (unsigned)(t >> 32) & 0xFFFF0000u; }
 };
 // The largest float that is certainly below (or rounds below) the score of key bits `k` (its low 16 bits are zero).
@@ -379,13 +380,18 @@ __global__ __launch_bounds__(64 * kStreamWaves) void topk_stream_kernel(const bf
     constexpr int kRows = 16 * RT, kGroups = 64 * SETS;
     constexpr bool kWide = sizeof(Key) == 8;                  // (the buffers in 64 KB of LDS)
     constexpr int kBuf = RT == 4 ? (kWide ? 96 : 128) : SETS < 4 ? 128 : (kWide && RT == 2) ? 224 : 256;
+    // where the bound is a running one: the largest T (see topk_dense), a row's keys behind a cut, key tiles a round, and a row's keys in front of a cut
+    constexpr int kMostT = SETS == 1 ? 16 : RT == 4 ? 32 : kMaxT, kKept = kMostT + kSpare;
+    constexpr int kRound = (kBuf - kKept) / 16 < W ? (kBuf - kKept) / 16 : W, kSlack = 40;
+    constexpr int kFull = kKept + 16 * kRound + kSlack < kBuf ? kKept + 16 * kRound + kSlack : kBuf;
+    static_assert(kRound >= 1 && kFull >= kKept + 16 * kRound, "the buffers hold a cut row and a round's keys");
     // one piece of LDS, for the groups' largest scores, then the rows' buffers, then what is ranked
     constexpr int kBytesGroups = kRows * (kGroups + 1) * 4, kBytesBuf = kRows * (kBuf + 1) * (int)sizeof(Key), kBytesWin = kRows * kWinStride * 8;
     constexpr int kBytes = kBytesGroups > kBytesBuf ? (kBytesGroups > kBytesWin ? kBytesGroups : kBytesWin)
                                                     : (kBytesBuf > kBytesWin ? kBytesBuf : kBytesWin);
     __shared__ unsigned long long space[(kBytes + 7) / 8];
-    __shared__ Key bound[kRows], ceiling[kRows];
-    __shared__ int cnt[kRows], n_win[RT][16], part[W][kRows];
+    __shared__ Key bound[kRows];
+    __shared__ int cnt[kRows], n_win[RT][16];
     unsigned (*const groups)[kGroups + 1] = reinterpret_cast<unsigned (*)[kGroups + 1]>(space);
     Key (*const buf)[kBuf + 1] = reinterpret_cast<Key (*)[kBuf + 1]>(space);
     unsigned long long (*const win)[16][kWinStride] = reinterpret_cast<unsigned long long (*)[16][kWinStride]>(space);
@@ -403,9 +409,20 @@ __global__ __launch_bounds__(64 * kStreamWaves) void topk_stream_kernel(const bf
         bq[rt][0] = ld16(pqb + (rt * 16 + r) * kD + quad * 8);
         bq[rt][1] = ld16(pqb + (rt * 16 + r) * kD + quad * 8 + 32);
     }
+    auto scores = [&](f32x4 (&s)[RT], const bf16x8 (&k)[2]) __attribute__((always_inline)) {
+#pragma unroll
+        for (int rt = 0; rt < RT; rt++) {
+            f32x4 z = {0.f, 0.f, 0.f, 0.f};
+            s[rt] = mfma_bf16(k[1], bq[rt][1], mfma_bf16(k[0], bq[rt][0], z));
+        }
+    };
+    auto settle = [&]() __attribute__((always_inline)) {      // LDS of this wave: what was read and written is, before what follows
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+    };
     // A look at all scores: see(s, i, tile) gets the scores of all row tiles against a key tile of this wave's, i (known at compile
     // time) = its place among the wave's tiles modulo kAhead
-    auto look = [&](auto&& see) __attribute__((always_inline)) {
+    auto look = [&](auto&& see, auto&& more) __attribute__((always_inline)) {
         struct Tiles { bf16x8 k[kAhead][2]; } ta, tb;
         auto load = [&](Tiles& o, int t) __attribute__((always_inline)) {
 #pragma unroll
@@ -420,18 +437,14 @@ __global__ __launch_bounds__(64 * kStreamWaves) void topk_stream_kernel(const bf
             for (int i = 0; i < kAhead; i++) {
                 if (t + i * W < tiles) {
                     f32x4 s[RT];
-#pragma unroll
-                    for (int rt = 0; rt < RT; rt++) {
-                        f32x4 z = {0.f, 0.f, 0.f, 0.f};
-                        s[rt] = mfma_bf16(o.k[i][1], bq[rt][1], mfma_bf16(o.k[i][0], bq[rt][0], z));
-                    }
+                    scores(s, o.k[i]);
                     see(s, i, t + i * W);
                 }
             }
         };
         constexpr int kStep = kAhead * W;
         load(ta, wave);
-        for (int t = wave; t < tiles; t += 2 * kStep) {
+        for (int t = wave; t < tiles && more(); t += 2 * kStep) {
             load(tb, t + kStep);
             work(ta, t);
             load(ta, t + 2 * kStep);
@@ -450,7 +463,7 @@ __global__ __launch_bounds__(64 * kStreamWaves) void topk_stream_kernel(const bf
         for (int rt = 0; rt < RT; rt++)
 #pragma unroll
             for (int e = 0; e < 4; e++) most[rt][i % SETS][e] = fmaxf(most[rt][i % SETS][e], s[rt][e]);
-    });
+    }, []() { return true; });
     if (tid < kRows) cnt[tid] = 0;
     if (tid < 16 * RT) n_win[tid / 16][tid % 16] = 0;
 #pragma unroll
@@ -470,10 +483,7 @@ __global__ __launch_bounds__(64 * kStreamWaves) void topk_stream_kernel(const bf
         const unsigned lo = row_bound<kGroups / 16, 1>(key, kGroups / 16, T, top, (RowShare<1>*)nullptr, turn, 0, lane);
         const unsigned t = row_threshold<kGroups / 4, 1>(key, T, lo, top, (RowShare<1>*)nullptr, turn, 0, lane, n_ge);
         // (a group without a number has the score -infinity, and below that there are keys yet: those of NaNs)
-        if (quad == 0) {
-            bound[own_rt * 16 + r] = t <= ordered_key(-INFINITY) ? (Key)1 : StreamKey<Key>::least(t, round);
-            ceiling[own_rt * 16 + r] = StreamKey<Key>::most(top, round);
-        }
+        if (quad == 0) bound[own_rt * 16 + r] = t <= ordered_key(-INFINITY) ? (Key)1 : StreamKey<Key>::least(t, round);
     }
     __syncthreads();
 
@@ -484,103 +494,101 @@ __global__ __launch_bounds__(64 * kStreamWaves) void topk_stream_kernel(const bf
         tau[rt] = t;
         low[rt] = score_floor(StreamKey<Key>::score_bits(t));
     };
-    auto collect = [&]() __attribute__((always_inline)) {
-        look([&](const f32x4 (&s)[RT], int, int tile) __attribute__((always_inline)) {
-            bool pass[RT], any = false;
+    auto take = [&](const f32x4 (&s)[RT], int tile) __attribute__((always_inline)) {
+        bool pass[RT], any = false;
 #pragma unroll
-            for (int rt = 0; rt < RT; rt++) {
-                pass[rt] = !(largest(s[rt]) < low[rt]);       // (a NaN passes: it has to be able to fill a row that has nothing better)
-                any |= pass[rt];
+        for (int rt = 0; rt < RT; rt++) {
+            pass[rt] = !(largest(s[rt]) < low[rt]);           // (a NaN passes: it has to be able to fill a row that has nothing better)
+            any |= pass[rt];
+        }
+        if (__ballot(any) == 0) return;
+#pragma unroll
+        for (int rt = 0; rt < RT; rt++) {
+            if (!pass[rt]) continue;
+            Key k[4];
+            int mine = 0;
+#pragma unroll
+            for (int e = 0; e < 4; e++) {
+                k[e] = StreamKey<Key>::make(s[rt][e], tile * 16 + 4 * quad + e, round);
+                mine += k[e] >= tau[rt] ? 1 : 0;
             }
-            if (__ballot(any) == 0) return;
+            if (mine > 0) {
+                int slot = atomicAdd(&cnt[rt * 16 + r], mine);
 #pragma unroll
-            for (int rt = 0; rt < RT; rt++) {
-                if (!pass[rt]) continue;
-                Key k[4];
-                int mine = 0;
-#pragma unroll
-                for (int e = 0; e < 4; e++) {
-                    k[e] = StreamKey<Key>::make(s[rt][e], tile * 16 + 4 * quad + e, round);
-                    mine += k[e] >= tau[rt] ? 1 : 0;
-                }
-                if (mine > 0) {
-                    int slot = atomicAdd(&cnt[rt * 16 + r], mine);
-#pragma unroll
-                    for (int e = 0; e < 4; e++)
-                        if (k[e] >= tau[rt]) buf[rt * 16 + r][min(slot++, kBuf)] = k[e];
-                }
+                for (int e = 0; e < 4; e++)
+                    if (k[e] >= tau[rt]) buf[rt * 16 + r][min(slot++, kBuf)] = k[e];
             }
-        });
+        }
     };
 #pragma unroll
     for (int rt = 0; rt < RT; rt++) set_bounds(rt, bound[rt * 16 + r]);
-    collect();
+    int counted = 0;
+    look([&](const f32x4 (&s)[RT], int, int tile) __attribute__((always_inline)) { take(s, tile); },
+         [&]() __attribute__((always_inline)) {               // (a row with more keys than its buffer holds: the rest is no help)
+             const bool none = __ballot(counted > kBuf) == 0;
+             counted = __atomic_load_n(&cnt[lane % kRows], __ATOMIC_RELAXED);      // (looked at eight tiles later)
+             return none;
+         });
     __syncthreads();
     bool over = false;
 #pragma unroll
     for (int rt = 0; rt < RT; rt++) over |= cnt[rt * 16 + r] > kBuf;
     if (__ballot(over) != 0) {                                // (the same in all waves)
-        Key lo[RT], hi[RT], mid[RT];
-        int c_lo[RT];
-#pragma unroll
-        for (int rt = 0; rt < RT; rt++) {
-            lo[rt] = tau[rt];
-            hi[rt] = ceiling[rt * 16 + r] + 1;                // (below the largest integer)
-            c_lo[rt] = cnt[rt * 16 + r];
-        }
-        for (int step = 0;; step++) {
-            bool open = false;
-#pragma unroll
-            for (int rt = 0; rt < RT; rt++) {
-                const Key half = lo[rt] + ((hi[rt] - lo[rt]) >> 1), of_score = middle_key(lo[rt], hi[rt]);
-                const bool on = c_lo[rt] > kBuf && hi[rt] - lo[rt] > 1;
-                mid[rt] = !on ? lo[rt] : (step < kScoreSteps && of_score > lo[rt] && of_score < hi[rt]) ? of_score : half;
-                open |= on;
-            }
-            if (__ballot(open) == 0) break;                   // (the same in all waves: so are the counts)
-            int c[RT];
-            float floor[RT];
-#pragma unroll
-            for (int rt = 0; rt < RT; rt++) {
-                c[rt] = 0;
-                floor[rt] = score_floor(StreamKey<Key>::score_bits(mid[rt]));
-            }
-            look([&](const f32x4 (&s)[RT], int, int tile) __attribute__((always_inline)) {
-#pragma unroll
-                for (int rt = 0; rt < RT; rt++) {
-                    if (largest(s[rt]) < floor[rt]) continue;
-#pragma unroll
-                    for (int e = 0; e < 4; e++) c[rt] += StreamKey<Key>::make(s[rt][e], tile * 16 + 4 * quad + e, round) >= mid[rt] ? 1 : 0;
-                }
-            });
-            __syncthreads();                                  // (the counts of the step before have been read)
-#pragma unroll
-            for (int rt = 0; rt < RT; rt++) {
-                c[rt] = quad_sum_i(c[rt]);
-                if (quad == 0) part[wave][rt * 16 + r] = c[rt];
-            }
-            __syncthreads();
-#pragma unroll
-            for (int rt = 0; rt < RT; rt++) {
-                int sum = 0;
-#pragma unroll
-                for (int w = 0; w < W; w++) sum += part[w][rt * 16 + r];
-                if (mid[rt] == lo[rt]) continue;              // (decided)
-                if (sum >= T) {
-                    lo[rt] = mid[rt];
-                    c_lo[rt] = sum;
-                } else {
-                    hi[rt] = mid[rt];
-                }
-            }
-        }
-        __syncthreads();
+        __syncthreads();                                      // (the counts have been read)
         if (tid < kRows) cnt[tid] = 0;
         __syncthreads();
+        bf16x8 k[2];
+        auto load = [&](int t) __attribute__((always_inline)) {
+            const bf16* p = pkb + (int64_t)min(t, tiles - 1) * 16 * kD;
+            k[0] = ld16(p + pieces.first);
+            k[1] = ld16(p + pieces.second);
+        };
+        load(wave);
+        for (int t0 = 0; t0 < tiles; t0 += kRound) {
+            if (wave < kRound && t0 + wave < tiles) {
+                f32x4 s[RT];
+                scores(s, k);
+                load(t0 + kRound + wave);
+                take(s, t0 + wave);
+            }
+            __syncthreads();
+            bool full = false;
 #pragma unroll
-        for (int rt = 0; rt < RT; rt++) set_bounds(rt, lo[rt]);
-        collect();
-        __syncthreads();
+            for (int rt = 0; rt < RT; rt++) full |= cnt[rt * 16 + r] > kFull - 16 * kRound;
+            if (__ballot(full) != 0) {                        // (the same in all waves)
+                __syncthreads();                              // (every wave has decided)
+                if (finishes) {
+                    const int row = own_rt * 16 + r, have = cnt[row];
+                    Key key[(kFull + 3) / 4], top = 0;
+#pragma unroll
+                    for (int i = 0; i < (kFull + 3) / 4; i++) {
+                        const int at = i * 4 + quad;
+                        key[i] = at < have ? buf[row][at] : (Key)0;
+                        top = key[i] > top ? key[i] : top;
+                    }
+                    top = quad_max_u(top);
+                    int turn = 0, n_ge, mine = 0;
+                    const Key t = row_threshold<(kFull + 3) / 4, 1, Key>(key, min(T, have), bound[row], top, (RowShare<1>*)nullptr, turn, 0, lane, n_ge);
+#pragma unroll
+                    for (int i = 0; i < (kFull + 3) / 4; i++) mine += key[i] >= t ? 1 : 0;
+                    settle();
+                    if (quad == 0) {
+                        cnt[row] = 0;
+                        bound[row] = t;
+                    }
+                    settle();
+                    int slot = mine > 0 ? atomicAdd(&cnt[row], mine) : 0;
+                    const Key t2 = compare_again(t, slot);
+#pragma unroll
+                    for (int i = 0; i < (kFull + 3) / 4; i++)
+                        if (key[i] >= t2) buf[row][min(slot++, kBuf)] = key[i];
+                }
+                __syncthreads();
+#pragma unroll
+                for (int rt = 0; rt < RT; rt++) set_bounds(rt, bound[rt * 16 + r]);
+            }
+            __syncthreads();                                  // (the counts have been read)
+        }
     }
 
     // ---- little more than the T best of a row's buffer, and those ranked
