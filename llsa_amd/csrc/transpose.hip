@@ -475,8 +475,8 @@ static int check_transpose_job(const int32_t* idx, const int32_t* offsets, const
 // More than 65536 entries (65536 tokens at topk 16) take as long here as the several kernels for large jobs take
 // beside the attention kernel on another stream (131072 entries: step 928 against 923 us, 196608: 672 against 664).
 constexpr int kTrLdsInts = 16 * 1024;
-static int tr_parts(int Mb, int Kb, int T, int BH, bool inverse, int lds_ints = kTrLdsInts, int histogram_ints = 2 * kTrLdsInts) {
-    const int64_t stride = tr_stride(Mb, inverse), E = (int64_t)Mb * T;
+static int tr_parts(int Mb, int Kb, int T, int BH, int sums, int lds_ints = kTrLdsInts, int histogram_ints = 2 * kTrLdsInts) {
+    const int64_t stride = tr_stride(Mb, sums), E = (int64_t)Mb * T;
     if (stride > lds_ints || Kb > histogram_ints) return 0;
     const int most_rows = (int)std::min<int64_t>(lds_ints / stride, kTrThreadsBeside);
     const int least = (Kb + most_rows - 1) / most_rows;
@@ -486,12 +486,27 @@ static int tr_parts(int Mb, int Kb, int T, int BH, bool inverse, int lds_ints = 
     return (Kb + rows - 1) / rows;                            // no empty range
 }
 
-static void add_to_plan(TrJobs& plan, const llsa_transpose_job& j, int parts) {
+// The ranges of a job and, for an inverse, after how many words of a row there is a sum (tr_stride).  An entry that adds up the words in front of its own
+// itself waits for as many LDS reads; a sum for every word doubles a key block's LDS and, where LDS decides, the ranges, each of which reads all
+// entries.  us, no sums / every word / every fourth:  1 x 1024 key blocks, lists of 16, 14.0 / 10.5 / 11.0;  6 x 1024 16.0 / 11.3 / 12.1;  6 x 2048 25.4 / 17.3 /
+// 17.3;  and where every word's would take more ranges 48 x 1024 19.5 / 26.4 / 15.9;  96 x 1024 36.2 / 41.2 / 31.0;  6 x 4096 48.0 / 46.0 / 26.0;
+// 6 x 8192, lists of 8, 117 / 186 / 92;  1 x 16384, lists of 4, 100 / 188 / 85 (every eighth 6 x 4096 28.1, 6 x 8192 92.6, 1 x 16384 81).
+struct TrRanges { int parts, sums; };
+static TrRanges tr_ranges(const llsa_transpose_job& j, int BH, int lds_ints = kTrLdsInts, int histogram_ints = 2 * kTrLdsInts) {
+    const int least = tr_parts(j.Mb, j.Kb, j.T, BH, 0, lds_ints, histogram_ints);
+    if (j.inv == nullptr) return {least, 0};
+    if (tr_parts(j.Mb, j.Kb, j.T, BH, 1, lds_ints, histogram_ints) == least) return {least, 1};
+    return {tr_parts(j.Mb, j.Kb, j.T, BH, kTrSums, lds_ints, histogram_ints), kTrSums};
+}
+
+static void add_to_plan(TrJobs& plan, const llsa_transpose_job& j, const TrRanges& ranges) {
+    const int parts = ranges.parts;
     TrJob& t = plan.job[plan.n_jobs++];
     t.idx = j.idx; t.offsets = j.offsets; t.flat = j.flat; t.work = j.work; t.inv = j.inv;
     t.Mb = j.Mb; t.Kb = j.Kb; t.T = j.T; t.chunk = j.chunk < 1 ? 1 : j.chunk;
     t.work_stride = j.work ? (int)llsa_work_list_len(j.Mb, j.Kb, j.T, t.chunk) : 0;
     t.parts = parts;
+    t.sums = ranges.sums;
     t.rows = (j.Kb + parts - 1) / parts;
     t.quads = j.T % 4 == 0 && aligned16(j.idx);
     const unsigned per = t.quads ? j.T / 4 : j.T;             // (i * ceil(2^32 / per) >> 32 is i / per while i * per < 2^32)
@@ -504,9 +519,9 @@ bool llsa::plan_transpose(const llsa_transpose_job* jobs, int n_jobs, int B, int
     for (int i = 0; i < n_jobs; i++) {
         const llsa_transpose_job& j = jobs[i];
         if (check_transpose_job(j.idx, j.offsets, j.flat, j.work, B, H, j.Mb, j.Kb, j.T, j.chunk) != 0) return false;
-        const int parts = tr_parts(j.Mb, j.Kb, j.T, B * H, j.inv != nullptr, lds_ints, lds_ints);
-        if (parts == 0) return false;
-        add_to_plan(plan, j, parts);
+        const TrRanges ranges = tr_ranges(j, B * H, lds_ints, lds_ints);
+        if (ranges.parts == 0) return false;
+        add_to_plan(plan, j, ranges);
     }
     return true;
 }
@@ -516,7 +531,7 @@ static int launch_bitmap_jobs(const TrJobs& jobs, int B, int H, bool beside, hip
     int64_t ints = 0;
     for (int i = 0; i < jobs.n_jobs; i++) {
         const TrJob& j = jobs.job[i];
-        ints = std::max<int64_t>(ints, std::max<int64_t>((int64_t)j.rows * tr_stride(j.Mb, j.inv != nullptr), j.Kb));
+        ints = std::max<int64_t>(ints, std::max<int64_t>((int64_t)j.rows * tr_stride(j.Mb, j.sums), j.Kb));
     }
     const size_t lds = sizeof(int) * (size_t)ints;
     const void* kernel = beside ? (const void*)transpose_bitmap_kernel<kTrThreadsBeside> : (const void*)transpose_bitmap_kernel<kTrThreads>;
@@ -575,7 +590,7 @@ static int transpose_general(const int32_t* idx, int32_t* offsets, int32_t* flat
 }
 
 extern "C" int llsa_transpose_one_launch(int Mb, int Kb, int T, int B, int H) {
-    return Mb > 0 && Kb > 0 && T > 0 && B > 0 && H > 0 && tr_parts(Mb, Kb, T, B * H, false) > 0;
+    return Mb > 0 && Kb > 0 && T > 0 && B > 0 && H > 0 && tr_parts(Mb, Kb, T, B * H, 0) > 0;
 }
 
 extern "C" int64_t llsa_transpose_nested_bytes(int Mb, int Kb, int T_parent, int B, int H) {
@@ -627,9 +642,10 @@ extern "C" int llsa_transpose_indices_multi(const llsa_transpose_job* jobs, int 
             several = true;
             continue;
         }
-        const int chunk = j.chunk < 1 ? 1 : j.chunk, parts = tr_parts(j.Mb, j.Kb, j.T, B * H, j.inv != nullptr);
-        if (parts > 0) {
-            add_to_plan(small, j, parts);
+        const int chunk = j.chunk < 1 ? 1 : j.chunk;
+        const TrRanges ranges = tr_ranges(j, B * H);
+        if (ranges.parts > 0) {
+            add_to_plan(small, j, ranges);
         } else {
             const int rc = transpose_general(j.idx, j.offsets, j.flat, j.work, j.inv, B, H, j.Mb, j.Kb, j.T, chunk, stream);
             if (rc != 0) return rc;

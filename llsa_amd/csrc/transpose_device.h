@@ -126,15 +126,19 @@ struct TrJob {
     int Mb, Kb, T, chunk, work_stride;
     int parts, rows;                                          // ranges per (b,h), key blocks per range
     unsigned row_magic;                                       // entry i (of four, if `quads`) belongs to query block i * row_magic >> 32
+    int sums;                                                 // see tr_stride
     int quads;                                                // T is a multiple of 4 and idx 16-byte aligned: entries are read four at a time
 };
+constexpr int kTrSums = 4;                                    // words to a sum where one for every word would cost ranges (tr_ranges)
 struct TrJobs {
     TrJob job[LLSA_MAX_LEVELS];
     int n_jobs, wgs;                                          // workgroups per (b,h): job[i].parts + 1 for each job, one after the other
 };
-// ints of LDS per key block: its row of bits, its count and then its start, and where an inverse is asked for the bits in front of every word (an entry
-// that adds up the words in front of its own itself waits for as many LDS reads: 6 x 1024 lists of 16, 20 ranges, 39.7 -> 21 us)
-__host__ __device__ inline int tr_stride(int Mb, bool inverse) { return ((Mb + 31) / 32) * (inverse ? 2 : 1) + 1; }
+// ints of LDS per key block: its row of bits, its count and then its start, and for an inverse the bits in front of every `sums`-th word (0: no inverse)
+__host__ __device__ inline int tr_stride(int Mb, int sums) {
+    const int words = (Mb + 31) / 32;
+    return words + 1 + (sums > 0 ? (words + sums - 1) / sums : 0);
+}
 
 // calls fn(key block, query block) for every entry of the (b,h), each in one thread
 template <int NT, typename Fn>
@@ -209,7 +213,7 @@ __device__ __forceinline__ void transpose_block(const TrJobs& jobs, int block, i
         return;
     }
 
-    const int words = (Mb + 31) / 32, stride = tr_stride(Mb, jb.inv != nullptr);
+    const int words = (Mb + 31) / 32, stride = tr_stride(Mb, jb.sums);
     const int lo = part * jb.rows, nr = min(jb.rows, Kb - lo);       // > 0: the host leaves no range empty
     unsigned* bm = reinterpret_cast<unsigned*>(smem);         // [nr][stride]
     for (int i = tid; i < nr * stride; i += NT) bm[i] = 0u;
@@ -249,10 +253,18 @@ __device__ __forceinline__ void transpose_block(const TrJobs& jobs, int block, i
         for (int r = tid; r < nr; r += NT) {
             unsigned* row = bm + r * stride;
             int before = 0;
+            if (jb.sums == 1) {
 #pragma unroll 4
-            for (int w = 0; w < words; w++) {
-                row[words + 1 + w] = (unsigned)before;
-                before += __popc(row[w]);
+                for (int w = 0; w < words; w++) {
+                    row[words + 1 + w] = (unsigned)before;
+                    before += __popc(row[w]);
+                }
+            } else {
+#pragma unroll 4
+                for (int w = 0; w < words; w++) {
+                    if (w % kTrSums == 0) row[words + 1 + w / kTrSums] = (unsigned)before;
+                    before += __popc(row[w]);
+                }
             }
         }
         __syncthreads();
@@ -261,7 +273,17 @@ __device__ __forceinline__ void transpose_block(const TrJobs& jobs, int block, i
             const int r = n - lo;
             if ((unsigned)r >= (unsigned)nr) return;
             const unsigned* row = bm + r * stride;
-            inv[e] = (int)row[words] + (int)row[words + 1 + (q >> 5)] + __popc(row[q >> 5] & ((1u << (q & 31)) - 1u));
+            const int w = q >> 5;
+            int pos = (int)row[words] + __popc(row[w] & ((1u << (q & 31)) - 1u));
+            if (jb.sums == 1) {
+                pos += (int)row[words + 1 + w];
+            } else {
+                const int w0 = w / kTrSums * kTrSums;
+                pos += (int)row[words + 1 + w / kTrSums];
+#pragma unroll
+                for (int i = 0; i < kTrSums - 1; i++) pos += __popc(w0 + i < w ? row[min(w0 + i, w)] : 0u);
+            }
+            inv[e] = pos;
         });
     }
     // The segments, ascending.  Eight neighbouring lanes share a row, each with an eighth of its words: the lanes count their

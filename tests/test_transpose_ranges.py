@@ -6,8 +6,9 @@ import torch
 import parity_cases as P
 from emu_util import emu_lib
 from llsa_amd._lib import override_library_for_tests
+from llsa_amd.kernel.hip.indices_transpose import transpose_indices
 
-SMALL = [(1, 2, 33, 1, 33, 4), (2, 1, 50, 5, 97, 2), (1, 1, 64, 4, 2100, 3)]
+SMALL = [(1, 2, 33, 1, 33, 4), (2, 1, 50, 5, 97, 2), (1, 1, 64, 4, 2100, 3), (1, 1, 12000, 1, 70, 64)]    # (the last: a sum for every fourth word)
 
 
 @pytest.mark.parametrize("B,H,Mb,T,Kb,chunk", SMALL)
@@ -18,6 +19,28 @@ def test_cpu(B, H, Mb, T, Kb, chunk):
 
 @pytest.mark.gpu
 @pytest.mark.parametrize("B,H,Mb,T,Kb,chunk", SMALL + [(1, 3, 4096, 16, 4096, 256), (1, 3, 4112, 16, 4112, 256), (4, 16, 1024, 64, 1024, 64),
-                                                       (1, 1, 65536, 1, 500, 64)])
+                                                       (1, 1, 65536, 1, 500, 64), (1, 6, 8192, 8, 8192, 64), (1, 48, 1024, 16, 1024, 64)])
 def test_gpu(B, H, Mb, T, Kb, chunk):
     P.check_transpose(torch.device("cuda"), B=B, H=H, Mb=Mb, T=T, Kb=Kb, chunk=chunk)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("BH,Mb,T", [(6, 8192, 8), (1, 16384, 4), (12, 4096, 8)])
+def test_inverse_costs_no_second_set_of_ranges(BH, Mb, T):
+    """Lists with their inverse positions take 1.3 to 1.6 times the time of the lists alone.  (With sums that double a key block's LDS, and so the ranges that
+    each read all entries, 3.2 to 3.6 times.)"""
+    idx = torch.randint(0, Mb, (1, BH, Mb, T), generator=torch.Generator().manual_seed(Mb)).int().cuda()
+
+    def time(inverse):
+        times = []
+        for _ in range(20):
+            a, b = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+            a.record()
+            for _ in range(10):
+                transpose_indices(idx, inverse=inverse)
+            b.record()
+            b.synchronize()
+            times.append(a.elapsed_time(b))
+        return sorted(times)[10]
+
+    assert time(True) < 2.4 * time(False)
