@@ -631,9 +631,10 @@ __global__ __launch_bounds__(64 * kStreamWaves) void topk_stream_kernel(const bf
 // smaller position wins, as it must.
 // P > 0: the parents are selected here first -- row G of the level above (N1/16 tokens, at most 16 P W) against all of its
 // keys, scores rounded to bf16, top T2 as topk_dense_kernel does it -- and written to par_out; otherwise they are read from pidx.
+// RANK: at most 64 parents, and every wave ranks them all (rank_keys).
 // (One row per wave and 512 threads a workgroup took 25 us for 768 groups of 16 rows, T = T2 = 16, and 123 us for 6144.)
 constexpr int kCascadeMaxParents = 256;           // P * W <= 16
-template <int TPW, int W, int P>
+template <int TPW, int W, int P, bool RANK>
 __global__ __launch_bounds__(64 * W) void topk_sparse_kernel(const bf16* __restrict__ pq, const bf16* __restrict__ pk,
                                                              const int* __restrict__ pidx, int* __restrict__ out, int N1, int T, int T2,
                                                              const bf16* __restrict__ pq_par, const bf16* __restrict__ pk_par,
@@ -656,7 +657,8 @@ __global__ __launch_bounds__(64 * W) void topk_sparse_kernel(const bf16* __restr
     if (tid < 16) n_win[tid] = 0;
     if (tid == 16) n_par = 0;
 
-    if constexpr (P * W == 4) {                               // at most 64 parents: every wave ranks them all (8 x 64 groups 9.9 -> 9.5 us, 48 x 64 30.6 -> 29.0)
+    if constexpr (RANK) {
+        static_assert(P * W == 4, "64 keys");
         const RankedKeys<1> ranked = rank_keys<1>(pq_par + ((int64_t)bh * N2 + G) * kD, pk_par + (int64_t)bh * N2 * kD, pieces.first, pieces.second, N2, lane);
         if (wave == 0 && ranked.rank[0] < T2) {
             const int idx = ranked.index(0, lane);
@@ -857,16 +859,23 @@ extern "C" int llsa_topk_dense_tiles(const void* pq, const void* pk_tiles, int32
 static void launch_sparse(const bf16* pq, const bf16* pk, const int* pidx, int* out, int B, int H, int N1, int T, int T2, const bf16* pq_par,
                           const bf16* pk_par, int* par_out, int tiled, hipStream_t st) {
     const dim3 grid(N1 / 16, B * H);
-#define LLSA_SPARSE_P(TPW, W, P) \
-    hipLaunchKernelGGL(HIP_KERNEL_NAME(topk_sparse_kernel<TPW, W, P>), grid, dim3(64 * W), 0, st, pq, pk, pidx, out, N1, T, T2, pq_par, pk_par, par_out, tiled)
-#define LLSA_SPARSE(TPW, W)                                    \
-    do {                                                       \
-        if (pq_par == nullptr) LLSA_SPARSE_P(TPW, W, 0);       \
-        else if (N1 / 16 <= 64) LLSA_SPARSE_P(TPW, W, 4 / W);  \
-        else LLSA_SPARSE_P(TPW, W, 16 / W);                    \
+#define LLSA_SPARSE_P(TPW, W, P, RANK) \
+    hipLaunchKernelGGL(HIP_KERNEL_NAME(topk_sparse_kernel<TPW, W, P, RANK>), grid, dim3(64 * W), 0, st, pq, pk, pidx, out, N1, T, T2, pq_par, pk_par, par_out, tiled)
+    // Up to 64 parents: ranked by every wave, the shorter chain, which out of rows costs four waves four times as many accesses as their quarters of the
+    // keys.  By groups of 16 rows, us, with quarters / ranked, rows:  topk 8/8: 64 8.9 / 8.6;  512 10.2 / 10.3;  768 11.1 / 12.2;  1152 14.1 / 16.8;  1536 15.9 /
+    // 19.0;  16/16: 64 11.8 / 10.8;  512 13.3 / 13.3;  768 14.9 / 15.3;  1536 21.0 / 24.7;  8/32: 64 15.4 / 13.5;  512 17.8 / 17.1;  768 20.7 / 20.2;  1536 28.1 / 32.0;
+    // one wave each:  8/8: 3072 20.9 / 18.2;  16/16: 35.0 / 32.2.  Tiles:  8/8: 64 8.5 / 7.6;  384 9.5 / 8.7;  1152 13.2 / 13.8;  1536 15.1 / 15.6;  3072 16.7 / 14.5;
+    // 16/16: 768 13.5 / 12.7;  1536 20.2 / 20.0;  3072 26.9 / 24.4;  8/32: 1536 26.0 / 26.0;  3072 50.6 / 43.5
+    const int64_t groups = (int64_t)N1 / 16 * B * H;
+#define LLSA_SPARSE(TPW, W)                                                                               \
+    do {                                                                                                  \
+        if (pq_par == nullptr) LLSA_SPARSE_P(TPW, W, 0, false);                                           \
+        else if (N1 / 16 <= 64 && (tiled || W < 4 || groups <= 512)) LLSA_SPARSE_P(TPW, W, 4 / W, true);  \
+        else if (N1 / 16 <= 64) LLSA_SPARSE_P(TPW, W, 4 / W, false);                                      \
+        else LLSA_SPARSE_P(TPW, W, 16 / W, false);                                                        \
     } while (0)
     // few groups: four waves each, for the shorter chain of steps; many (2 waves per SIMD): as few as hold the keys, for fewer instructions
-    const bool few = (int64_t)N1 / 16 * B * H < 2048;
+    const bool few = groups < 2048;
     if (T2 <= 4) LLSA_SPARSE(4, 1);
     else if (T2 <= 8 && few) LLSA_SPARSE(2, 4);
     else if (T2 <= 8) LLSA_SPARSE(8, 1);
