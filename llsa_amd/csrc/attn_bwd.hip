@@ -1013,14 +1013,16 @@ struct GroupParams {
 
 // Workgroups of the group-major pass over an XCD's `groups` groups.  32 CUs take two each; where that leaves a last round at most half full, the key blocks
 // of its groups are dealt out to `parts` workgroups, each with the group's tiles in LDS, and the first `whole` groups are as before.  Every key block is
-// still met by one wave, so the results are the same.  Training steps of two levels, topk 16/16, us, whole / dealt out: 1 x 16384 tokens (8 groups an XCD) 92.4 /
-// 87.5;  10 x 16384 (80) 254.6 / 250.8;  17 x 16384 at 16/12 (136) 381 / 374;  9 x 16384 at 16/32 (72) 296 / 288;  3 x 49152 at 64/32 (72) 639 / 629;  just
-// half full 4 x 16384 (32) 140 / 138.8, 12 x 16384 (96) 293.8 / 293.3, 3 x 32768 even.
+// still met by one wave, so the results are the same.  Training steps of two levels, topk 16/16, us, whole / dealt out: 1 x 16384 tokens (8 groups an XCD) 91.0 /
+// 84.8;  at 16/32 106.6 / 95.2;  10 x 16384 (80) 250.4 / 246.3;  17 x 16384 at 16/12 (136) 374.1 / 370.3;  9 x 16384 at 16/32 (72) 293.0 / 284.2;  1 x 32768 119.1 /
+// 113.7;  3 x 49152 at 64/32 (72) 635.3 / 625.3;  just half full 4 x 16384 (32) and 12 x 16384 (96) even.
 struct GroupSplit { int whole, parts; };
 // key blocks of a wave of a group that `parts` workgroups share
 __host__ __device__ inline int group_wave_blocks(int n_blocks, int parts) { return (n_blocks + kGroupWaves * parts - 1) / (kGroupWaves * parts); }
 constexpr int kGroupSlots = 2 * 256 / kXcds;
-constexpr int kGroupPartBlocks = 6;               // key blocks to a part, on the average over a group's parts, at least
+// key blocks to a part, on the average over a group's parts, at least.  3 / 4 / 6 / 8 / 12, us: 1 x 16384 84.9 / 84.9 / 84.8 / 87.3 / 90.9;  17 x 16384 at 16/12 369.8 / 369.4 /
+// 370.3 / 369.2 / 374.6;  9 x 16384 at 16/32 284.4 / 284.8 / 284.2 / 281.6 / 281.8;  3 x 49152 at 64/32 629.6 / 629.6 / 625.3 / 625.2 / 627.4
+constexpr int kGroupPartBlocks = 6;
 static GroupSplit group_split(int groups, int n_blocks) {
     const int rest = groups % kGroupSlots;
     int parts = rest == 0 ? 1 : std::min(kGroupSlots / rest, n_blocks / kGroupPartBlocks);

@@ -276,9 +276,10 @@ __device__ __forceinline__ int select_blocks(const bf16* pq_row, const bf16* key
 // one the chip waited for them: step of 12 x 16384 tokens 317 -> 309 us, of 24 x 4096 163 -> 156, of 48 x 16384 1284 -> 1264; both
 // kernels of 6 x 65536 157 -> 154, where 67 workgroups a head (66 ranges and the histogram) read all its 65536 entries each.
 // That reading is what bounds them on the largest grids: their workgroups then fill the chip by themselves for rounds, and a launch of their own, with
-// twice the LDS and so half the ranges, reads less.  Steps behind the forward / riding, us, by entries read over all workgroups (topk 16, 65536
-// tokens): 8 heads (35 M) 932 / 914;  16 (70 M) 1768 / 1759;  20 (88 M) 2257 / 2251;  24 (105 M) 2651 / 2665;  28 (123 M) 3128 / 3140;  32 (141 M)
-// 3474 / 3493, on another card 3503 / 3543.  42 x 49152, topk 20 (98 M) 3233 / 3251;  64 x 32768, topk 32 (76 M) even.
+// twice the LDS and so half the ranges, reads less.  Steps behind the forward / riding, us, by entries read over all workgroups (two levels, topk 16/16): 12 x
+// 16384 tokens 300.6 / 288.6;  24 x 16384 542.9 / 532.3;  6 x 32768 326 / 313;  65536 tokens, 2 heads 283.7 / 271.6;  6 647.6 / 642.0;  12 (53 M) 1287 / 1284;  16
+// (70 M) 1699 / 1682;  20 (88 M) 2115 / 2105;  24 (105 M) 2522 / 2505;  28 (123 M) 2944 / 2950;  32 (141 M) 3315 / 3340;  64 x 32768, 32/16 (76 M) 3973 / 3987;  42 x 49152,
+// 20/16 (98 M) 3432 / 3468;  one level, 24 x 49152 5184 / 5216.
 constexpr int kTrLdsFwd = 2 * kGroup * 2 * kTile / 2 - 32;    // ints of the kernel's LDS they work in (32 for their scratch)
 static_assert(tr_scratch_ints(256) <= 32, "the scratch of a transposing workgroup");
 constexpr int64_t kRideMaxReads = (int64_t)88 << 20;          // entries the riding workgroups may read in all

@@ -8,7 +8,7 @@
 //     backward  attn_bwd with fold_pooled = 1  (dq, dk, dv complete, rotated back and back through the qk-norm)
 //
 // Native because at the short sequences a step is bound by its host side: at B=1, H=6, N=1024 the kernels of a forward
-// take about 20 us and those of a forward + backward 70, while the same sequence issued from Python took 33 and 100 to
+// take about 13 us and those of a forward + backward 47, while the same sequence issued from Python took 33 and 100 to
 // 180 (a backward written in Python also has to win the interpreter lock on the autograd thread).
 //
 // The library's entry points are called through the table of addresses its ctypes binding (llsa_amd/_lib.py) passes in, so
@@ -247,6 +247,9 @@ struct Layout {
         // Without gradients the forward reads q and v as rows, and the pooling pass writes no tiles of them: 8 x 65536 tokens of one level 683 -> 660 us, 96 x
         // 4096 143 -> 132, 6 x 65536 of two levels 214 -> 199, 3 x 49152 193.0 -> 191.2.  But a wave then starts with rows that are further away and have to be
         // rotated, which a short pass waits for: 8 x 16384 53.4 / 54.9, 15 x 7168 57.4 / 58.9, 24 x 4096 50.8 / 51.0, 6 x 1024 16.6 / 16.8; 2 x 65536 196.2 / 193.3.
+        // With the norm and the rotation both, even up to 200000 tokens (tiles / rows, 24 x 7168 89.3 / 90.7, 12 x 16384 96.6 / 96.3, 192 x 1024 61.8 / 63.7;  without
+        // either 84.8 / 79.1, 90.3 / 83.4, 55.9 / 49.5), less beyond (96 x 4096 137.3 / 126.8);  8 heads of (B,N,H,64) views, whose rows lie 1 KB
+        // apart, with the rotation 433 / 445 at 49152 tokens, topk 64/32, 156 / 158 at 32768, 32/16.
         rows = !grad && BH * N > (int64_t(1) << 17);
         qr = take(n[1] * 2048, !rows);
         kr = take(n[1] * 2048);
@@ -518,7 +521,9 @@ Tensor attend(const std::shared_ptr<Library>& lib, const Tensor& q_in, const Ten
         // stream; the several kernels per level of the longest sequences run on a second
         // stream beside the attention kernel: the attention kernel is issued first (the GPU is waiting for it), and an
         // event recorded before it lets the second stream start as soon as the selection is done.  With few tokens over all
-        // heads the event calls cost more than the overlap saves: everything then goes to the one stream.  (One launch on the second stream
+        // heads the event calls cost more than the overlap saves: everything then goes to the one stream.  Training steps, us, behind / beside: two levels
+        // 16/16, 2 x 131072 552 / 534;  6 x 131072 1481 / 1462;  3 x 196608 1289 / 1268;  6 x 262144 even (3829 / 3827);  32/16, 3 x 65536 488 / 476;  64/32, 3 x
+        // 49152 649 / 626;  three levels, 6 x 262144, 2883 / 2876;  one level, topk 32, 6 x 65536 2247 / 2205.  (One launch on the second stream
         // gains nothing either: two levels of 131072 tokens, topk 8, behind / beside, us: 1 head 279 / 293, 2 heads 458 / 468, 6 heads
         // 1293 / 1297, 12 heads 2457 / 2449.)
         const bool beside = grad && lib->device && B * H * N >= (int64_t(1) << 17) &&

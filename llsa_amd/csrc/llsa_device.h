@@ -569,22 +569,23 @@ constexpr int kPairMaxTopk = 64;
 // ... and considered where their workgroups (four waves, a group of eight query blocks) fill the chip.  It holds three of them per CU
 // (single query blocks: four of half the work), so a last round that is mostly empty costs a whole one: at most 30 % more places than
 // groups.  And below 5/6 of a round the chip has room for all of the waves either way, and a wave of one block has half the
-// serial chain.  dQ, one / two, us (topk 16 but for 7168 and 1024 tokens):
-//   groups 384 (6 x 8192) 26.8 / 31.3;  512 (16 x 4096) 24.4 / 26.5;  640 (20 x 4096) 30.6 / 32.2
-//   728 (13 x 7168, topk 12) 37.0 / 34.8;  768 (24 x 4096) 34.7 / 34.1;  784 (14 x 7168) 39.6 / 43.6;  840 (15 x 7168) 40.8 / 45.0
-//   1024 (8 x 8192) 51.1 / 51.8;  1152 (16 x 9216) 60.8 / 63.7;  1280 (20 x 8192) 64.2 / 60.7;  1536 (24 x 8192) 78.6 / 73.2
-//   1568 (28 x 7168) 69.6 / 72.8;  2048 (16 x 16384) 101.6 / 90.8;  3072 (24 x 16384) 144.4 / 134.4
-// The forward's waves are shorter.  It gains from two as soon as the single blocks no longer fit the chip at once (512 groups), and up to a round of pairs
-// its rounds may be emptier.  Sampling, topk 8, the whole pass: 512 (8 x 8192) 43.9 / 45.2;  576 (9 x 8192) 53.9 / 52.3;  640 (10 x 8192) 53.5 / 53.0
-//   832 (13 x 8192) 62.1 / 65.9;  960 (15 x 8192) 66.7 / 68.0;  1152 (18 x 8192) 76.9 / 78.9;  1280 (20 x 8192) 81.3 / 80.8
+// serial chain.  dQ, one / two, us (topk 16 but for 7168 tokens, where it is 12):
+//   groups 384 (6 x 8192) 24.6 / 28.1;  512 (16 x 4096) 23.0 / 23.8;  640 (20 x 4096) 29.0 / 29.1
+//   728 (13 x 7168) 34.3 / 33.4;  768 (24 x 4096) 32.2 / 30.5;  784 (14 x 7168) 37.7 / 40.4;  840 (15 x 7168) 38.6 / 41.3
+//   1280 (20 x 8192) 62.0 / 57.6;  1536 (24 x 8192) 75.6 / 68.2;  two levels 1536 (12 x 16384) 68.1 / 60.8;  2048 87.3 / 80.5;  3072 140.0 / 120.5
+// (The 30 % could be more since two lists are merged in a hundred instructions: 1152 (16 x 9216) 60.6 / 59.0, the step 256.5 / 254.4;  1568 (28 x
+// 7168) 68.4 / 65.4, 278.3 / 273.8;  1024 (8 x 16384, two levels) 42.9 / 42.3.)
+// The forward's waves are shorter.  In one round of pairs, where the single blocks no longer fit the chip at once, it is two from 513 groups on, which pays
+// from about 700: sampling, the whole pass, topk 8:  512 (8 x 8192) 38.2 / 39.4;  576 43.3 / 44.6;  640 44.5 / 45.5;  544 (17 x 4096) 35.4 / 35.8;  640 36.7 /
+// 37.2;  768 (24 x 4096, topk 16) 46.1 / 45.2;  beyond a round one:  832 (13 x 8192) 53.0 / 55.9;  960 58.8 / 59.1;  1152 62.1 / 64.6;  1280 67.4 / 67.0
 // Where most of the walk is pooled blocks, which a wave of two reads once for both, two win from 512 groups on and with as much as 60 % more
 // places than groups.  Sampling, and in brackets the training step with one / two in dQ, topk 8 unless given:
-//   512 (2 x 32768, 128 pooled blocks) 97.4 / 94.7 (263.5 / 260.7);  512 (65536, 256) 147.3 / 139.5 (423.4 / 415.4), at topk 16 156.7 / 149.8 (455.9 / 448.4)
-//   512 (4 x 16384, 64) 61.1 / 60.4 (182.3 / 181.7);  640 (2 x 40960, 160) 128.6 / 125.7 (366.7 / 364.1);  960 (5 x 24576, 96) 121.7 / 118.5 (350.8 / 345.3)
-//   1024 (8 x 16384) 100.8 / 97.8 (300.2 / 295.6);  1024 (2 x 65536) 239.7 / 224.5 (749.9 / 729.6);  1664 (13 x 16384) 155.1 / 151.2 (467.0 / 461.8)
-//   but 800 (5 x 20480, 80) 102.3 / 106.7 (276.8 / 282.2);  896 (4 x 28672, 112) 125.3 / 127.7 (359.3 / 361.6)
-// With a larger topk from a full round on: 1024 (8 x 16384, topk 16) 109.1 / 107.2 (332.8 / 328.8);  960 (5 x 24576, topk 24) 154.5 / 151.7 (457.7 / 450.9)
-//   1024 (2 x 65536, topk 64) 368.7 / 358.3 (1166.0 / 1147.2);  but 512 (4 x 16384, topk 16) 65.3 / 65.8 (196.7 / 196.9);  512 (65536, topk 64) 217.3 / 221.2
+//   512 (2 x 32768, 128 pooled blocks) 73.0 / 71.5 (237.5 / 232.0);  512 (65536, 256) 118.5 / 114.0 (396.9 / 386.4), at topk 16 123.5 / 119.3 (421.0 / 412.9)
+//   640 (2 x 40960, 160) 103.0 / 103.4 (328.2 / 321.7);  960 (5 x 24576, 96) 101.7 / 98.2 (325.6 / 316.6);  1024 (2 x 65536) 207.7 / 192.5 (674.5 / 648.9)
+//   1024 (8 x 16384, 64) 84.4 / 82.7 (256.2 / 250.4);  1664 (13 x 16384) 123.8 / 121.5 (406.4 / 393.1);  but 512 (4 x 16384) 51.2 / 52.1 (159.7 / 157.5)
+//   and 800 (5 x 20480, 80) 80.9 / 84.6 (251.2 / 253.4);  896 (4 x 28672, 112) 104.7 / 106.5 (332.7 / 331.4)
+// With a larger topk from a full round on: 1024 (8 x 16384, topk 16) 91.9 / 90.4 (284.0 / 278.6);  960 (5 x 24576, topk 24) 121.3 / 118.2 (390.6 / 382.6)
+//   1024 (2 x 65536, topk 64) 280.5 / 276.0 (943.2 / 930.8);  but 512 (4 x 16384, topk 16) 55.5 / 56.3 (174.2 / 173.9);  512 (65536, topk 64) 161.5 / 166.7
 constexpr int kPairPlaces = 256 * 3;
 inline bool pairs_pay(int64_t groups, int64_t pooled_blocks, int T, bool forward) {
     const int64_t places = (groups + kPairPlaces - 1) / kPairPlaces * kPairPlaces, idle = (places - groups) * 10;
@@ -603,8 +604,10 @@ inline int64_t pooled_blocks_read(int N, const int32_t* topk, int levels) {
 inline bool two_blocks_per_wave(int64_t BH, int N, const int32_t* topk, int levels, bool forward) {
     const int64_t groups = (int64_t)N / 128 * BH, pooled = pooled_blocks_read(N, topk, levels);
     if (topk[0] > kPairMaxTopk || N % 128 != 0 || !pairs_pay(groups, pooled, topk[0], forward)) return false;
-    // Where the fine blocks are most of the walk the forward gains little from two on grids of a few rounds (topk 8, 16 pooled blocks: 17 x
-    // 4096 tokens 44.3 / 42.8, 20 x 4096 45.1 / 43.9, but 28 x 4096 52.9 / 55.8, 32 x 4096 55.8 / 57.7, 36 x 4096 62.7 / 64.9, 40 x 4096 66.2 / 66.7)
+    // Where the fine blocks are most of the walk the forward gains little from two on grids of a few rounds.  Sampling, the whole pass, topk 8, 16 pooled blocks: 28 x
+    // 4096 tokens 45.7 / 47.7, 32 x 4096 49.0 / 49.7, 36 x 4096 49.5 / 51.6, 40 x 4096 53.0 / 53.6, 64 x 4096 (2048 groups) 77.2 / 76.8;  two levels 8/8 8 x 16384 50.7 /
+    // 51.4;  16/16 12 x 16384 83.1 / 81.4, 16 x 16384 (2048) 104.9 / 101.9, 24 x 16384 149.2 / 142.8.  (At 32/16, where a fine block is named by both rows more often,
+    // two would pay from a full round on: 12 x 16384 109.6 / 103.1, its training step 361.8 / 356.9.)
     return !forward || pooled >= 4 * topk[0] || groups >= 2048;
 }
 

@@ -40,8 +40,8 @@ struct PoolParams {
 // registers every store instruction would touch 64 different cache lines with 16 or 8 bytes
 // each.  They go through LDS instead, eight rows of every block at a time and every wave by itself: 8 KB hold the half
 // tiles of the wave's eight blocks, and a store instruction writes half a tile in whole 128- or 256-byte pieces.
-// The pass is bound by memory -- loads and stores each take about as long as the whole should (19 and 15 us of 48 for
-// 2 x 6 x 16384 tokens with RoPE) -- so what counts is that waves in different phases overlap: half tiles leave LDS
+// The pass is bound by memory -- alone, loads and stores would take 19 and 15 us of its 35 for
+// 2 x 6 x 16384 tokens with RoPE -- so what counts is that waves in different phases overlap: half tiles leave LDS
 // for sixteen waves per CU, and no barrier keeps the waves of a workgroup together.
 // Units (16 bytes) of a half tile in LDS: their low index bits are XOR-ed with bits of chunk and block, so that the threads'
 // writes and the linear reads both spread evenly over the banks without padding.

@@ -472,8 +472,11 @@ static int check_transpose_job(const int32_t* idx, const int32_t* offsets, const
 // Ranges of key blocks a job is cut into for transpose_bitmap_kernel, 0: too large for it.  At least so many that a range's bitmaps take
 // at most 64 KB of LDS, and towards half the CUs over all (b,h): every range reads all entries, which is what a range's workgroup
 // spends its time on beyond about four of them (with a workgroup for every CU two levels of 12 x 16384 tokens 15.3 us, so 12).
-// More than 65536 entries (65536 tokens at topk 16) take as long here as the several kernels for large jobs take
-// beside the attention kernel on another stream (131072 entries: step 928 against 923 us, 196608: 672 against 664).
+// More than 65536 entries take longer here than lists made from those of the level above take beside the attention kernel on another stream where there are
+// many key blocks, up to 65536 the nested form takes longer or as long.  Training steps of two levels, topk 16/16, us, here / nested: 12 x 16384 tokens (16384 entries)
+// 289 / 306;  6 x 32768 313 / 359;  2 x 65536 (65536) 272 / 316;  6 x 65536 642 / 644;  16 x 65536 1697 / 1686;  32 x 65536 3329 / 3298;  2 x 131072 (131072) 564 / 534;  6 x
+// 131072 1526 / 1462;  3 x 196608 1363 / 1268.  (With few key blocks and long lists this form is the faster one beyond that line too: 3 x 65536 at 32/16, 131072
+// entries, 462 / 476;  3 x 49152 at 64/32, 196608, 617 / 626;  one level, 6 x 65536 at 32, against the counting sort 2196 / 2205.)
 constexpr int kTrLdsInts = 16 * 1024;
 static int tr_parts(int Mb, int Kb, int T, int BH, int sums, int lds_ints = kTrLdsInts, int histogram_ints = 2 * kTrLdsInts) {
     const int64_t stride = tr_stride(Mb, sums), E = (int64_t)Mb * T;

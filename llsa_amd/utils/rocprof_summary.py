@@ -21,7 +21,7 @@ os.makedirs(out, exist_ok=True)
 is_bench = wl != 'l1_infer_64k'
 bench = f'python3 bench.py --workload {wl} --no-extras --steps 5 --warmup 2' if is_bench else (
     "python3 -c \"import perf.cases as c, torch; s = c.prepare([x for x in c.listed() if x['name'] == 'l1_infer_64k'][0], 1); "
-    "[c.run(s) for _ in range(20)]; torch.cuda.synchronize()\"")
+    "[c.run(s) for _ in range(100)]; torch.cuda.synchronize()\"")
 
 def short(n):
     n = n.replace('void ', '')
@@ -47,22 +47,24 @@ cd, cdur = counters(f'{raw}/cache/p_results.db')
 with open(f'{out}/step_kernels_{wl}_sq_cache_counters.txt', 'w') as f:
     f.write(f"Wave-scheduler and cache counters per dispatch, workload {wl}: {desc}\n")
     f.write("commands (from the repository root, on the MI355X box):\n")
-    f.write(f"  rocprofv3 --pmc SQ_WAVE_CYCLES SQ_BUSY_CU_CYCLES SQ_ACTIVE_INST_VALU SQ_ACTIVE_INST_SCA SQ_ACTIVE_INST_LDS SQ_WAIT_INST_ANY SQ_VALU_MFMA_BUSY_CYCLES SQ_INSTS_VALU --kernel-trace -d prof/sq -o p -- {bench}\n")
+    f.write(f"  rocprofv3 --pmc SQ_WAVE_CYCLES SQ_BUSY_CU_CYCLES SQ_ACTIVE_INST_VALU SQ_ACTIVE_INST_SCA SQ_ACTIVE_INST_LDS SQ_WAIT_INST_ANY SQ_VALU_MFMA_BUSY_CYCLES SQ_INSTS_VALU GRBM_GUI_ACTIVE --kernel-trace -d prof/sq -o p -- {bench}\n")
     f.write(f"  rocprofv3 --pmc TCC_HIT_sum TCC_MISS_sum TCP_TOTAL_CACHE_ACCESSES_sum TCP_TCC_READ_REQ_sum SQ_LDS_BANK_CONFLICT SQ_LDS_IDX_ACTIVE --kernel-trace -d prof/cache -o p -- {bench}\n")
     f.write("averages per dispatch, summed over the chip.  WAVE_CYCLES, ACTIVE_INST_*, WAIT_INST_ANY are in units of 4 cycles per wave;\n")
     f.write("BUSY_CU_CYCLES and VALU_MFMA_BUSY_CYCLES in cycles.  mfma% = VALU_MFMA_BUSY_CYCLES / (duration x 2.4 GHz x 1024 SIMDs);\n")
     f.write("valu% = 4 x ACTIVE_INST_VALU / (same); wait% = WAIT_INST_ANY / WAVE_CYCLES; waves/CU = 4 x WAVE_CYCLES / (duration x 2.4 GHz x 256);\n")
-    f.write("ldsconf% = LDS_BANK_CONFLICT / LDS_IDX_ACTIVE, the share of the LDS's cycles that bank conflicts take.\n\n")
-    f.write(f"{'kernel':44s} {'grid':>9s} {'avg_us':>7s} {'mfma%':>6s} {'valu%':>6s} {'wait%':>6s} {'waves/CU':>8s} {'INSTS_VALU':>11s} {'INST_SCA':>10s} {'INST_LDS':>10s} {'L2hit%':>7s} {'TCP_acc':>10s} {'TCP->L2 rd':>10s} {'ldsconf%':>8s}\n")
+    f.write("ldsconf% = LDS_BANK_CONFLICT / LDS_IDX_ACTIVE, the share of the LDS's cycles that bank conflicts take; GHz = GRBM_GUI_ACTIVE / 8 dies / duration,\n")
+    f.write("the clock of kernels of 300 us and more (the counter also runs for some 8 us around a dispatch).\n\n")
+    f.write(f"{'kernel':44s} {'grid':>9s} {'avg_us':>7s} {'mfma%':>6s} {'valu%':>6s} {'wait%':>6s} {'waves/CU':>8s} {'INSTS_VALU':>11s} {'INST_SCA':>10s} {'INST_LDS':>10s} {'L2hit%':>7s} {'TCP_acc':>10s} {'TCP->L2 rd':>10s} {'ldsconf%':>8s} {'GHz':>5s}\n")
     for k in sorted(sd, key=lambda k: -sdur[k][0] * sdur[k][1]):
         s = sd[k]; c = cd.get(k, {})
         us = sdur[k][0] / 1e3
         simd_cyc = us * 1e-6 * 2.4e9 * 1024
+        ghz = f"{s['GRBM_GUI_ACTIVE'] / 8 / us / 1e3:.2f}" if us >= 300 else '-'
         hit = c.get('TCC_HIT_sum', 0); miss = c.get('TCC_MISS_sum', 0)
         f.write(f"{short(k[0])[:44]:44s} {k[1]:9d} {us:7.1f} {100*s['SQ_VALU_MFMA_BUSY_CYCLES']/simd_cyc:6.1f} {100*4*s['SQ_ACTIVE_INST_VALU']/simd_cyc:6.1f} "
                 f"{100*s['SQ_WAIT_INST_ANY']/max(s['SQ_WAVE_CYCLES'],1):6.1f} {4*s['SQ_WAVE_CYCLES']/(simd_cyc/4):8.1f} {s['SQ_INSTS_VALU']:11.3g} "
                 f"{s['SQ_ACTIVE_INST_SCA']:10.3g} {s['SQ_ACTIVE_INST_LDS']:10.3g} {100*hit/max(hit+miss,1):7.1f} {c.get('TCP_TOTAL_CACHE_ACCESSES_sum',0):10.3g} {c.get('TCP_TCC_READ_REQ_sum',0):10.3g} "
-                f"{100*c.get('SQ_LDS_BANK_CONFLICT',0)/max(c.get('SQ_LDS_IDX_ACTIVE',0),1):8.1f}\n")
+                f"{100*c.get('SQ_LDS_BANK_CONFLICT',0)/max(c.get('SQ_LDS_IDX_ACTIVE',0),1):8.1f} {ghz:>5s}\n")
 if not is_bench:
     sys.exit()
 
@@ -85,9 +87,9 @@ with open(f'{out}/step_kernels_{wl}_kernel_trace.txt', 'w') as f:
         f.write("(up to 65536 entries per (b,h) every kernel runs on the one stream: the index transposes of all levels are\n"
                 " workgroups of the forward attention kernel's launch)\n")
     else:
-        f.write("(the index transposes -- transpose_indices_kernel, tr_*_kernel, sort_segments_kernel, and transpose_bitmap_kernel for\n"
-                " the pooled levels -- run on a second stream beside the forward attention kernel: their durations overlap with it\n"
-                " and are stretched by it, so the sum exceeds the step time)\n")
+        f.write("(the index transposes -- nested_*_kernel for the fine level, transpose_bitmap_kernel for the pooled levels -- run on a\n"
+                " second stream beside the forward attention kernel: their durations overlap with it and are stretched by it, so the sum\n"
+                " exceeds the step time)\n")
 
 # ---- HBM traffic
 fd, fdur = counters(f'{raw}/fetch/p_results.db')
