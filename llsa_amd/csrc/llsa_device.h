@@ -343,7 +343,7 @@ __device__ __forceinline__ int clampi(int v, int lo, int hi) { return v < lo ? l
 // or llsa_bwd_level (fields sel, T).  Blocks of level l per (b,h): N / 16^(l+1).
 // What a wave looks up per block stays in registers.  With a loop over the levels in the kernel's arguments every block waited for a chain of scalar loads,
 // and with them for its LDS reads (they share a counter): 6 x 262144 tokens of two levels, forward 853 -> 811 us, dQ 996 -> 961; forward of 8 x 65536 of one
-// level 651 -> 627, which is less than its cycles say (these kernels run at the clock the card's power allows, 1.9 GHz and below).
+// level 651 -> 627, which is less than its cycles say (these kernels run at 1.9 to 2.1 GHz of 2.4).
 struct SharedTiles { const bf16 *k, *v; };                    // tiles of a block
 struct SharedList {
     int mine;                  // lane i: the i-th selected entry over all levels below the coarsest
