@@ -26,10 +26,12 @@
 #include <c10/hip/HIPStream.h>
 #include <hip/hip_runtime_api.h>
 
+#include <algorithm>
 #include <array>
 #include <mutex>
 #include <optional>
 #include <string>
+#include <utility>
 #include <vector>
 
 #include "../../../include/llsa_hip.h"
@@ -153,6 +155,18 @@ std::string text_of(at::IntArrayRef v) {
 bool strides_multiple(at::IntArrayRef st, int64_t m) {
     for (size_t i = 0; i + 1 < st.size(); i++)
         if (st[i] % m != 0) return false;
+    return true;
+}
+// Whether no two elements of such a tensor share memory (an expanded one's do): every dimension steps over all that the smaller steps span.
+bool own_places(const std::array<int64_t, 4>& sizes, const std::array<int64_t, 4>& st) {
+    std::array<std::pair<int64_t, int64_t>, 4> dims;          // step, entries
+    for (int i = 0; i < 4; i++) dims[i] = {sizes[i] > 1 ? st[i] : 0, sizes[i]};
+    std::sort(dims.begin(), dims.end());
+    int64_t span = 1;
+    for (const auto& [step, n] : dims) {
+        if (n > 1 && step < span) return false;
+        span += step * (n - 1);
+    }
     return true;
 }
 // last stride 1 and every row 16-byte aligned: what the kernels' 16-byte loads need
@@ -329,8 +343,8 @@ struct LlsaBackward : public Node {
         const Tensor d = as_rows(grad_out.defined() ? grad_out : at::zeros_like(out));
         const auto opts = out.options();
         const std::array<int64_t, 4> shape{B, H, N, 64};
-        auto like = [&](const std::array<int64_t, 4>& st) {  // gradients have the layout of their primals when the 8-byte stores allow it
-            return strides_multiple(st, 4) && st[3] == 1 ? at::empty_strided(shape, st, opts) : at::empty(shape, opts);
+        auto like = [&](const std::array<int64_t, 4>& st) {  // gradients have the layout of their primals when the 8-byte stores allow it and no rows meet
+            return strides_multiple(st, 4) && st[3] == 1 && own_places(shape, st) ? at::empty_strided(shape, st, opts) : at::empty(shape, opts);
         };
         Tensor dq = like(sq), dk = like(sk), dv = like(sv);
         const Tensor W = at::empty({lay->bwd_bytes}, opts.dtype(at::kByte));
