@@ -5,6 +5,7 @@ import pytest
 import torch
 
 from emu_util import emu_lib
+from gpu_time import median_us
 from llsa_amd._lib import current_lib, override_library_for_tests
 from llsa_amd.kernel.hip._common import stream_of
 
@@ -133,42 +134,23 @@ def test_rows_that_overflow_cost_one_look_more(n, T, BH, kind):
         else:
             pq, pk = (torch.randn(1, BH, n, 64, generator=torch.Generator().manual_seed(i)).bfloat16() for i in (1, 2))
         q, k, out = pq.to(dev), tiles(pk).to(dev), torch.empty(1, BH, n, T, dtype=torch.int32, device=dev)
-        times = []
-        for _ in range(20):
-            a, b = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
-            a.record()
-            for _ in range(10):
-                lib.check(lib.topk_dense_tiles(q.data_ptr(), k.data_ptr(), out.data_ptr(), 1, BH, n, T, 1, stream_of(lib, q)), "topk_dense_tiles")
-            b.record()
-            b.synchronize()
-            times.append(a.elapsed_time(b))
-        return sorted(times)[10]
+        return median_us(lambda: lib.check(lib.topk_dense_tiles(q.data_ptr(), k.data_ptr(), out.data_ptr(), 1, BH, n, T, 1, stream_of(lib, q)), "topk_dense_tiles"))
 
-    assert time(kind) < 2.8 * time("spread")
+    ratio = time(kind) / time("spread")
+    print(f"{ratio:.2f}")
+    assert ratio < 2.8
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("T", [8, 16])
-def test_cascade_out_of_rows_costs_little_more_than_its_selection(T):
-    """Out of rows four waves find a group's parents among their quarters of 64 keys: 1.2 to 1.4 times the parent-guided selection alone, 24 x 1024 rows.
-    (With every wave ranking all of them 1.45 to 1.65.)"""
+@pytest.mark.parametrize("T,most", [(8, 1.48), (16, 1.33)])
+def test_cascade_out_of_rows_costs_little_more_than_its_selection(T, most):
+    """Out of rows four waves find a group's parents among their quarters of 64 keys: 1.36 and 1.22 times the parent-guided selection alone, 24 x 1024
+    rows.  (With every wave ranking all of them 1.61 and 1.43.)"""
     from llsa_amd.kernel.hip.topk import compute_topk_indices_sparse, gen_sparse_indices, topk_cascade
     q, k, pq, pk = (torch.randn(1, 24, n, 64, generator=torch.Generator().manual_seed(n + i)).bfloat16().cuda() for n in (1024, 64) for i in (1, 2))
     par, sel = topk_cascade(pq, pk, q, k, T, T)
     assert torch.equal(par, gen_sparse_indices(pq, pk, T)) and torch.equal(sel, compute_topk_indices_sparse(q, k, par, T, T))
 
-    def time(fn):
-        times = []
-        for _ in range(30):
-            a, b = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
-            a.record()
-            for _ in range(20):
-                fn()
-            b.record()
-            b.synchronize()
-            times.append(a.elapsed_time(b))
-        return sorted(times)[10]
-
-    alone, both = time(lambda: compute_topk_indices_sparse(q, k, par, T, T)), time(lambda: topk_cascade(pq, pk, q, k, T, T))
-    print(f"T = {T}: {both / alone:.3f}")
-    assert both < 1.45 * alone
+    alone, both = median_us(lambda: compute_topk_indices_sparse(q, k, par, T, T), 20), median_us(lambda: topk_cascade(pq, pk, q, k, T, T), 20)
+    print(f"{both / alone:.2f}")
+    assert both < most * alone
